@@ -28,8 +28,8 @@
  * of the MFMA epilogues; 3: MFMA burn probe with its block-scaled shapes, per-device properties, fp8 attention forward at
  * head dims 16 / 32 / 256, a row-major fp8 B on the MFMA kernels, block-scaled products with any K that is a multiple of
  * 32 and scale rows of any pitch on the MFMA kernels; 4: mi355_gemm_splitk, a row-major B whose N is not a multiple of
- * 16 bytes inside a padded pitch on the tile kernels; 5: fp32 operands in mi355_gemm.) */
-#define MI355_ABI_VERSION 5
+ * 16 bytes inside a padded pitch on the tile kernels; 5: fp32 operands in mi355_gemm; 6: mi355_gemm_splits.) */
+#define MI355_ABI_VERSION 6
 
 #ifdef __cplusplus
 extern "C" {
@@ -137,13 +137,13 @@ int mi355_gemm_tuned(const void* A, const void* B, void* C,
                      const float* a_scale, const float* b_scale,
                      int activation, int tile, int group_m, void* stream);
 
-/* mi355_gemm with K split over `splits` workgroups per tile (0 = chosen by size: one workgroup per CU, at least sixteen
- * 64-byte K steps each, at most 32; none from half a round of 128x128 tiles on): for products of few tiles with a long K - one row of tiles against a long
+/* mi355_gemm with K split over `splits` workgroups per tile (0 = as many as mi355_gemm_splits says): for products of few
+ * tiles with a long K - one row of tiles against a long
  * weight, a small square against a long K -, where one workgroup per tile leaves most of the device idle and a few
  * K steps of loads in flight are all that hides the memory latency.  The reference's kernel has no such form
  * (python/tutorials/03-matrix-multiplication.py:241-316 gives every tile to one program); the contract is the same
  * C = act((a_scale * b_scale) * A @ B) with fp32 accumulation and one rounding, the partial sums added in split order.
- * Two launches: the tile kernel on 128x128 tiles into fp32 slices of `workspace`, then the sum and the epilogue.
+ * Two launches: the tile kernel into fp32 slices of `workspace`, then the sum and the epilogue.
  * workspace: device memory of at least splits * M * N * 4 bytes (32 * M * N * 4 always suffices for splits = 0),
  * 16-byte aligned, contents irrelevant; two calls that overlap in time need different workspaces.  fp32 operands (K-major B)
  * are split too, and sooner: their products are bound by the fp32 MFMA rate alone, so idle CUs are all that counts.  Operands that the
@@ -157,6 +157,11 @@ int mi355_gemm_splitk(const void* A, const void* B, void* C,
                       int in_dtype, int out_dtype,
                       const float* a_scale, const float* b_scale,
                       int activation, int splits, void* workspace, size_t workspace_bytes, void* stream);
+
+/* The number of splits that pay for a product of these sizes by the library's own estimate (1 = none: the plain call), at
+ * most 32 and 64 MiB of partial sums.  b_kmajor: B is K-contiguous.  Touches no device memory.
+ */
+int mi355_gemm_splits(int M, int N, int K, int in_dtype, int b_kmajor);
 
 /* mi355_gemm with a stream-K schedule: one program per CU, and the programs split ALL K steps of ALL
  * 256x256 tiles evenly, so a tile count that is not a multiple of the CU count (or smaller than it:

@@ -1353,3 +1353,40 @@ def test_fp32_operands_are_multiplied_exactly(gpu, kmajor):
         rc = lib.mi355_gemm_tuned(ta.data_ptr(), tb.data_ptr(), c.data_ptr(), 512, 768, 1024, 1024, 1, 1, 1024, 768, 1, _lib.F32, _lib.F32,
                                   None, None, _lib.ACT_NONE, tile, 8, torch.cuda.current_stream().cuda_stream)
         assert rc == 0 and bits_equal(to_np(c), ref), tile
+
+
+@pytest.mark.parametrize("tile", [8, 9, 10])   # 128x128, 128x64, 64x64
+@pytest.mark.parametrize("dtype", ["fp16", "bf16", "e4m3"])
+def test_ring_kernels_at_the_edges_of_their_ring_are_bit_exact(gpu, dtype, tile, monkeypatch):
+    # K steps of 128 bytes through four stages: K shorter than the ring, an odd and an even number of steps, a tail of one
+    # and of seven 16-byte chunks, a tail alone; one row and column, partial and whole tiles; both layouts of B; an addend
+    # row, the activation and every form of the store (16-byte, unaligned rows, strided, fp32).  Sums of small integers
+    # are exact in fp32 and below 2^8 in either 16-bit type, so every bit is determined.
+    set_knob(monkeypatch, "MI355_GEMM_TILE", str(tile))
+    set_knob(monkeypatch, "MI355_GEMM_SKINNY", "0")
+    rng = np.random.default_rng(tile)
+    el = 1 if dtype == "e4m3" else 2
+    for M, N, kbytes in [(1, 16, 16), (128, 128, 128), (130, 72, 112), (64, 136, 384), (257, 200, 512), (192, 64, 528), (100, 264, 640),
+                         (65, 128, 752), (300, 320, 1168), (129, 1000, 2048)]:
+        K = kbytes // el
+        a = rng.integers(-1, 2, size=(M, K)).astype(np.float32)
+        b = rng.integers(-1, 2, size=(K, N)).astype(np.float32)
+        row = rng.integers(-3, 4, size=(1, N)).astype(np.float32)
+        ref = a @ b
+        if dtype == "e4m3":
+            ta = torch.from_numpy(formats.encode_fp8(a, "e4m3")).to(gpu).view(torch.float8_e4m3fn)
+            tbs = [torch.from_numpy(formats.encode_fp8(np.ascontiguousarray(b.T), "e4m3")).to(gpu).view(torch.float8_e4m3fn).t()]
+        else:
+            ta = from_np(a, dtype, gpu)
+            tbs = [from_np(np.ascontiguousarray(b.T), dtype, gpu).t()] + ([from_np(b, dtype, gpu)] if N % 8 == 0 else [])
+        for tb in tbs:
+            assert bits_equal(to_np(triton_amd.matmul(ta, tb, out_dtype=torch.float32)), ref), (M, N, K, tb.stride())
+            got = to_np(triton_amd.matmul(ta, tb, out_dtype=torch.bfloat16, add=from_np(row, "fp32", gpu), activation="leaky_relu"))
+            want = ref + row
+            assert bits_equal(got, formats.round_bf16(np.where(want >= 0, want, np.float32(0.01) * want).astype(np.float32))), (M, N, K)
+            for pitch in (N + 3, N + 8):                     # rows of C on 2-byte and on 16-byte boundaries
+                cbuf = torch.full((M, pitch), 7.0, dtype=torch.float16, device=gpu)
+                rc = _lib.load().mi355_gemm(ta.data_ptr(), tb.data_ptr(), cbuf.data_ptr(), M, N, K, ta.stride(0), 1, tb.stride(0), tb.stride(1), pitch, 1,
+                                            {"fp16": _lib.F16, "bf16": _lib.BF16, "e4m3": _lib.F8E4M3}[dtype], _lib.F16, None, None, _lib.ACT_NONE,
+                                            torch.cuda.current_stream().cuda_stream)
+                assert rc == 0 and bits_equal(to_np(cbuf[:, :N].contiguous()), ref) and bool((cbuf[:, N:] == 7.0).all()), (M, N, K, pitch)

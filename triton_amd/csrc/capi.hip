@@ -126,8 +126,6 @@ int mixed_split(int M, int nn, int P) {
   return best_rows;
 }
 
-bool aligned(const void* p, size_t a) { return ((uintptr_t)p % a) == 0; }
-
 int elem_size(int dtype) {
   switch (dtype) {
     case MI355_F16: case MI355_BF16: return 2;
@@ -136,6 +134,90 @@ int elem_size(int dtype) {
     default: return 0;
   }
 }
+
+// What the ring kernels (gemm_ring.h) would take for a product of `steps` 128-byte K steps, in us: a round of one tile per
+// CU costs its prologue and epilogue plus its K steps; splits of K add the slices' way through memory and a second launch.
+// Fitted to 60 shapes from 256 to 8192 (bf16, fp16, e4m3, both layouts of B): within 15 % except where the operands' pitch
+// is not a multiple of 128 bytes (every line is then fetched in two pieces: up to 1.5 times as long, for every kernel alike).
+// One row or column of tiles against a long weight is a stream from memory: a CU gets about 30 GB/s of lines that no other CU
+// asks for (64 x 8192 x 8192 fp16, 128 tiles of 64x64: 48 us with rings of four and of eight stages alike, 35 us with two
+// splits), so that there the splits also buy bandwidth.
+struct RingPlan { int shape, splits; double us; };
+constexpr double kLaunchUs = 3.5;
+RingPlan ring_plan(int M, int N, int steps, int cus, int splits_lo, int splits_hi) {
+  const double streamed = 128.0 * steps * std::max(M, N);   // bytes of the longer operand
+  static const struct { int bm, bn; double round_us, step_us; } kShapes[3] = {{128, 128, 2.5, 0.42}, {128, 64, 1.5, 0.265}, {64, 64, 0.6, 0.165}};
+  RingPlan best{0, 1, 1e30};
+  for (int shape = 0; shape < 3; shape++) {
+    const auto& t = kShapes[shape];
+    const double step_us = (M <= t.bm || N <= t.bn) && streamed >= 64e6 ? std::max(t.step_us, (M <= t.bm ? t.bn : t.bm) * 128 / 30e3) : t.step_us;
+    const long tiles = (long)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
+    for (int splits = splits_lo; splits <= splits_hi; splits++) {
+      const int per = (steps + splits - 1) / splits;
+      const long rounds = (tiles * splits + cus - 1) / cus;
+      // (several rounds overlap a little at their ends, and keep the operands' lines moving for a sixth more per step)
+      const double n = rounds > 1 ? 0.5 * ((double)rounds + (double)tiles * splits / cus) : 1.0;
+      double us = kLaunchUs + n * (t.round_us + per * step_us * (rounds > 1 ? 1.18 : 1.0));
+      if (splits > 1) us += 2.5 + (double)splits * M * N * 8.0 / 3e6;   // (written and read again at about 3 TB/s)
+      if (us < best.us) best = {shape, splits, us};
+      if (splits > 1 && rounds > 1) break;   // (more splits only add rounds)
+    }
+  }
+  return best;
+}
+
+// The same for the kernels of 256-column tiles with `rows` rows of C each (gemm_wave128.hip: whole tiles; edges: the
+// eight-wave kernel).  A K step of a 256-row tile is bound by its 64 KiB of operands: 1.43 us with all CUs at it, a quarter
+// of that without the others' traffic.
+double tiles256_us(long tiles, int rows, int steps, int cus, bool edges, bool fp8) {
+  const long rounds = (tiles + cus - 1) / cus;
+  const double fill = rounds > 1 ? 1.0 : (double)tiles / cus;
+  const double share = rows == 256 ? 1.0 : rows == 192 ? 0.78 : 0.64;
+  return kLaunchUs + (double)rounds * share * ((edges ? 8.0 : 6.0) + (edges && !fp8 ? 1.6 : 1.43) * (0.25 + 0.75 * fill) * steps);
+}
+
+// Operands as the ring kernels want them, on top of what every tile kernel asks (16-byte chunks): 16-bit with either layout
+// of B, fp8 with a K-major one.
+bool ring_ok(int elem_bytes, bool b_kmajor) { return elem_bytes == 2 || (elem_bytes == 1 && b_kmajor); }
+
+// The streaming kernel of at most 32 rows on a side (gemm_skinny.hip: a workgroup per 32 rows of the other one, K split over
+// its four waves): 0.3 us per 128 bytes of a wave's share (0.5 where it transposes a row-major operand), or what that access
+// pattern gets from memory.  Ahead of the ring kernels where both sides are short (fp16 16 x 2048 x 2048 5.5 against 7.4 us) and
+// for fp8 (16 x 8192 x 8192 13.0 / 13.1, 16 x 2048 x 2048 4.7 / 5.0); behind them on long 16-bit weights (16 x 8192 x 8192 row
+// major 43 / 31, K-major 36 / 33, 16 x 1024 x 8192 23 / 11) and from 33 rows on (64 x 8192 x 8192 49 / 35).
+double skinny_us(int M, int N, int64_t k_bytes, int elem_bytes, bool b_kmajor) {
+  if (std::min(M, N) > 32) return 1e30;
+  const bool transposes = !b_kmajor;
+  const double bytes = (double)k_bytes * std::max(M, N);
+  return kLaunchUs + std::max((double)k_bytes / 512 * (transposes ? 0.5 : 0.3), bytes / (elem_bytes == 1 ? 7e6 : transposes ? 3.4e6 : 4.2e6));
+}
+
+// Splits of K that `mi355_gemm_splitk` takes by itself (1 = the plain call).
+int auto_splits(int M, int N, int64_t k_bytes, int in_dtype, bool b_kmajor, bool ring, int cus) {
+  if (ring) {
+    const int steps = (int)((k_bytes + 127) / 128);
+    const int most = (int)std::min<int64_t>(std::min<int64_t>(32, steps / 2), (64ll << 20) / std::max<int64_t>(1, 4ll * M * N));   // 64 MiB of partial sums
+    if (most < 2 || steps < 16) return 1;   // (below that a second launch costs more than the K steps it would save)
+    const double plain = std::min({ring_plan(M, N, steps, cus, 1, 1).us, skinny_us(M, N, k_bytes, elem_size(in_dtype), b_kmajor),
+                                   tiles256_us((long)((M + 255) / 256) * ((N + 255) / 256), 256, steps, cus, false, elem_size(in_dtype) == 1)});
+    const RingPlan split = ring_plan(M, N, steps, cus, 2, most);
+    return split.us < 0.95 * plain ? split.splits : 1;
+  }
+  // the one-barrier-per-step kernel on 128x128 tiles, 64-byte K steps: a workgroup per CU, at least sixteen K steps each, at most
+  // 32 slices; nothing to gain from half a round of tiles on or below 64 K steps
+  const int small = std::min(M, N);
+  if (small <= 32) return 1;   // (the streaming kernel)
+  const long tiles = (long)((M + 127) / 128) * ((N + 127) / 128);
+  const int ksteps = (int)((k_bytes + 63) / 64);
+  long splits = tiles * 2 > cus || ksteps < 64 ? 1 : std::min<long>(std::min<long>(cus / tiles, ksteps / 16), 32);
+  // (fp32: bound by the fp32 MFMA rate alone, 2048 cycles per K step of a 128x128 tile - whatever puts more CUs to work
+  // wins, down to eight K steps a slice; 1024^3: 74 -> 24 us)
+  if (in_dtype == MI355_F32) splits = tiles >= cus || ksteps < 16 ? 1 : std::min<long>(std::min<long>((2 * cus + tiles - 1) / tiles, ksteps / 8), 32);
+  splits = std::min<long>(splits, (64ll << 20) / std::max<int64_t>(1, 4ll * M * N));
+  return splits >= 2 ? (int)splits : 1;
+}
+
+bool aligned(const void* p, size_t a) { return ((uintptr_t)p % a) == 0; }
 
 bool copy_strides(const int64_t* src, int64_t* dst) {
   if (!src) return false;
@@ -337,47 +419,47 @@ static int gemm_impl(const void* A, const void* B, void* C, int M, int N, int K,
   if (p.num_programs > cus) p.num_programs = cus;       // (the stream-K workspace is sized for one program per CU)
   p.workspace = workspace;
   const bool skinny_allowed = tile_arg < 0 && knob(knobs().skinny, 1);  // an explicit tile means a tile kernel
-  if (skinny_allowed) {
-    // at most 64 rows on one side: stream the other operand once (X = small side, Y = streamed side).  65 .. 128 rows
-    // against a streamed side of at least 2048: two such launches, 64 rows and the rest - the tile kernels have too
-    // few tiles there (flushed do_bench, bf16, tile kernel / two launches: 2048 x 128 x 4096 50.6 / 39.1 us, 8192 x 128 x
-    // 8192 117 / 95, 128 x 8192 x 8192 124 / 102; with 256 rows the tiles win, 115 / 147).
+  const bool can_ring = ring_ok(es, b_kmajor);
+  const int ksteps128 = (p.k_bytes + 127) / 128;
+  // at most 32 rows on one side: stream the other operand once (X = small side, Y = streamed side) where that is the faster
+  // way (skinny_us), or where MI355_GEMM_SKINNY asks for it
+  if (skinny_allowed && std::min(M, N) <= 32 &&
+      (knobs().skinny != UNSET || !can_ring || skinny_us(M, N, p.k_bytes, es, b_kmajor) < ring_plan(M, N, ksteps128, cus, 1, 1).us)) {
     SkinnyArgs sk{};
     sk.K = K; sk.C = (char*)C; sk.a_scale = a_scale; sk.b_scale = b_scale;
     sk.activation = activation; sk.out_dtype = out_dtype; sk.cus = device_info().cus;
-    bool use = false, y_kmajor = false, x_kmajor = true;
-    int small = 0;
-    if (M <= 64 || (M <= 128 && N >= 2048)) {
-      sk.X = (const char*)A; sk.Y = (const char*)B; small = M; sk.L = N;
+    bool y_kmajor = true, x_kmajor = true;
+    if (M <= 32) {
+      sk.X = (const char*)A; sk.Y = (const char*)B; sk.S = M; sk.L = N;
       sk.x_pitch = p.lda; sk.y_pitch = p.ldb; sk.cs = scm; sk.cl = scn;
       sk.aux = aux; sk.aux_ss = aux_sm; sk.aux_sl = aux_sn; sk.aux_dtype = aux_dtype;
-      y_kmajor = b_kmajor; use = true;
-    } else if (N <= 64 || (N <= 128 && M >= 2048)) {
-      sk.X = (const char*)B; sk.Y = (const char*)A; small = N; sk.L = M;
+      y_kmajor = b_kmajor;
+    } else {
+      sk.X = (const char*)B; sk.Y = (const char*)A; sk.S = N; sk.L = M;
       sk.x_pitch = p.ldb; sk.y_pitch = p.lda; sk.cs = scn; sk.cl = scm;
       sk.aux = aux; sk.aux_ss = aux_sn; sk.aux_sl = aux_sm; sk.aux_dtype = aux_dtype;
-      y_kmajor = true; x_kmajor = b_kmajor; use = true;
+      x_kmajor = b_kmajor;
     }
-    if (use) {
-      SkinnyArgs part[2] = {sk, sk};
-      part[0].S = small < 64 ? small : 64;
-      part[1].S = small - part[0].S;
-      // (the second part starts 64 rows of X further: K-contiguous rows 64 pitches, S-contiguous rows 64 elements on)
-      part[1].X = sk.X + (x_kmajor ? 64 * sk.x_pitch : (int64_t)64 * es);
-      part[1].C = sk.C + 64 * sk.cs * elem_size(out_dtype);
-      if (aux) part[1].aux = (const char*)aux + 64 * sk.aux_ss * elem_size(aux_dtype);
-      const int nparts = part[1].S > 0 ? 2 : 1;
-      bool ok = true;
-      for (int i = 0; i < nparts; i++) ok = ok && gemm_skinny_ok(part[i], y_kmajor, x_kmajor, es);
-      if (ok) {
-        for (int i = 0; i < nparts; i++) {
-          const int rc = gemm_skinny_launch(part[i], in_dtype, y_kmajor, x_kmajor, stream);
-          if (rc != 0) return rc;
-        }
-        return MI355_OK;
-      }
+    if (gemm_skinny_ok(sk, y_kmajor, x_kmajor, es)) return gemm_skinny_launch(sk, in_dtype, y_kmajor, x_kmajor, stream);
+  }
+  // the ring kernels of 64 .. 128-row tiles where they are the faster ones by the two estimates above (and in place of the
+  // other 128x128 kernel wherever they take the operands)
+  int ring = -1;
+  if (can_ring) {
+    const bool by_knob = tile_arg >= 0 || knobs().tile != UNSET;
+    if (tile == 1) ring = by_knob ? 0 : ring_plan(M, N, ksteps128, cus, 1, 1).shape;
+    else if (tile >= 8 && tile <= 10) ring = tile - 8;
+    else if (!by_knob && knobs().tile_m == UNSET && knobs().mixed_rows == UNSET) {
+      const int rows = tile == 6 && p.tile_m ? p.tile_m : 256;
+      const RingPlan plan = ring_plan(M, N, ksteps128, cus, 1, 1);
+      double other = tiles256_us((long)((M + rows - 1) / rows) * ((N + 255) / 256), rows, ksteps128, cus, tile != 6, is8);
+      if (mixed_rows > 0) other *= 0.9;   // (two tile heights in one launch are chosen where they gain at least 5 %)
+      if (plan.us < other) ring = plan.shape;
     }
   }
+  if (ring >= 0)
+    return is8 ? gemm_ring8_launch(p, in_dtype == MI355_F8E5M2, ring, 1, 0, stream)
+               : gemm_ring16_launch(p, in_dtype == MI355_BF16, b_kmajor, ring, 1, 0, stream);
   if (is8 && b_kmajor && !aux && gemm8_skinny_ok(p) && skinny_allowed) return gemm8_skinny_launch(p, in_dtype == MI355_F8E5M2, stream);
   if (is8 && mixed_rows > 0) return gemm_wave128_f8_mixed_launch(p, mixed_rows, in_dtype == MI355_F8E5M2, stream);
   if (is8 && tile == 6 && (p.tile_m == 192 || p.tile_m == 128 || w128_ok)) return gemm_wave128_f8_launch(p, in_dtype == MI355_F8E5M2, b_kmajor, stream);
@@ -406,6 +488,13 @@ int mi355_gemm_tuned(const void* A, const void* B, void* C, int M, int N, int K,
                    activation, nullptr, 0, 0, 0, tile, group_m, stream_);
 }
 
+int mi355_gemm_splits(int M, int N, int K, int in_dtype, int b_kmajor) {
+  if (M <= 0 || N <= 0 || K <= 0 || in_dtype < MI355_F16 || in_dtype > MI355_F32) return 1;
+  const int es = elem_size(in_dtype);
+  return auto_splits(M, N, (int64_t)K * es, in_dtype, b_kmajor != 0, ring_ok(es, b_kmajor != 0),
+                     device_info().cus > 0 ? device_info().cus : 256);
+}
+
 int mi355_gemm_splitk(const void* A, const void* B, void* C, int M, int N, int K,
                       int64_t sam, int64_t sak, int64_t sbk, int64_t sbn, int64_t scm, int64_t scn,
                       int in_dtype, int out_dtype, const float* a_scale, const float* b_scale,
@@ -423,17 +512,10 @@ int mi355_gemm_splitk(const void* A, const void* B, void* C, int M, int N, int K
   const bool b_nmajor = !is32 && sbn == 1 && sbk % vec == 0 && sbk >= (N + vec - 1) / vec * vec && aligned(B, 16);
   const bool pitch_ok = (int64_t)sam * es < (1 << 23) && (b_kmajor ? (int64_t)sbn * es < (1 << 23) : (int64_t)sbk * es < (1 << 26));
   const int64_t k_bytes = (int64_t)K * es;
-  const int ksteps = (int)((k_bytes + 63) / 64);
+  const bool ring = ring_ok(es, b_kmajor);
+  const int step_bytes = ring ? 128 : 64, ksteps = (int)((k_bytes + step_bytes - 1) / step_bytes);
   const int cus = device_info().cus > 0 ? device_info().cus : 256;
-  if (splits == 0) {
-    // a workgroup per CU, at least sixteen K steps each, at most 32 slices to add up; nothing to gain from half a round
-    // of tiles on or below 64 K steps (measured: see ops.py::_splitk_splits)
-    const long tiles = (long)((M + 127) / 128) * ((N + 127) / 128);
-    splits = tiles * 2 > cus || ksteps < 64 ? 1 : (int)std::min<long>(std::min<long>(cus / tiles, ksteps / 16), 32);
-    // (fp32: bound by the fp32 MFMA rate alone, 2048 cycles per K step of a 128x128 tile - whatever puts more CUs to work
-    // wins, down to eight K steps a slice; 1024^3: 74 -> 24 us)
-    if (is32) splits = tiles >= cus || ksteps < 16 ? 1 : (int)std::min<long>(std::min<long>((2 * cus + tiles - 1) / tiles, ksteps / 8), 32);
-  }
+  if (splits == 0) splits = auto_splits(M, N, k_bytes, in_dtype, b_kmajor, ring, cus);
   const int per = splits >= 2 ? (ksteps + splits - 1) / splits : ksteps;
   const int used = (ksteps + per - 1) / per;   // (no split is left empty)
   if (!(a_ok && (b_kmajor || b_nmajor) && pitch_ok) || used < 2 || knob(knobs().force_strided, 0) != 0)
@@ -447,9 +529,11 @@ int mi355_gemm_splitk(const void* A, const void* B, void* C, int M, int N, int K
   p.ldb = (b_kmajor ? sbn : sbk) * es;
   p.group_m = knob(knobs().group_m, 8);
   p.workspace = (float*)workspace;
+  const int shape = ring ? ring_plan(M, N, ksteps, cus, used, used).shape : 0;
   const int rc = is32    ? gemm32_splitk_launch(p, used, per * 64, stream)
-                 : es == 1 ? gemm8_splitk_launch(p, in_dtype == MI355_F8E5M2, b_kmajor, used, per * 64, stream)
-                           : gemm16_splitk_launch(p, in_dtype == MI355_BF16, b_kmajor, used, per * 64, stream);
+                 : ring && es == 1 ? gemm_ring8_launch(p, in_dtype == MI355_F8E5M2, shape, used, per * 128, stream)
+                 : ring    ? gemm_ring16_launch(p, in_dtype == MI355_BF16, b_kmajor, shape, used, per * 128, stream)
+                           : gemm8_splitk_launch(p, in_dtype == MI355_F8E5M2, used, per * 64, stream);
   if (rc != 0) return rc;
   GemmStridedArgs out{};
   out.C = C; out.M = M; out.N = N; out.scm = scm; out.scn = scn;

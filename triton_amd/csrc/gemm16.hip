@@ -8,7 +8,7 @@ template <typename V8>
 struct Cfg16 {
   using Operand = V8;
   static constexpr int kSteps = 2, kChunks = 1;
-  static constexpr bool kRowMajorB = true, kScaled = false;
+  static constexpr bool kRowMajorB = true, kScaled = false, kRing = true;
   static constexpr int kElemBytes = 2;
   static constexpr int kStepsPerScaleDword = 1;
   // no block scales: placeholders so that generic code naming them compiles
@@ -27,15 +27,6 @@ int gemm16_launch(const GemmArgs& p, bool bf16, bool b_kmajor, int tile, hipStre
   }
   return b_kmajor ? launch_gemm_tile<Cfg16<f16x8>, true>(p, tile, stream)
                   : launch_gemm_tile<Cfg16<f16x8>, false>(p, tile, stream);
-}
-
-int gemm16_splitk_launch(const GemmArgs& p, bool bf16, bool b_kmajor, int splits, int chunk_bytes, hipStream_t stream) {
-  if (bf16) {
-    return b_kmajor ? launch_gemm_splitk<Cfg16<bf16x8>, true>(p, splits, chunk_bytes, stream)
-                    : launch_gemm_splitk<Cfg16<bf16x8>, false>(p, splits, chunk_bytes, stream);
-  }
-  return b_kmajor ? launch_gemm_splitk<Cfg16<f16x8>, true>(p, splits, chunk_bytes, stream)
-                  : launch_gemm_splitk<Cfg16<f16x8>, false>(p, splits, chunk_bytes, stream);
 }
 
 int gemm16_grouped_launch(const GroupedArgs& ga, bool bf16, int nprog, int nprog_big, hipStream_t stream) {

@@ -13,7 +13,7 @@ template <int FMT>  // 0 = e4m3fn, 1 = e5m2 (cbsz / blgp encoding of the instruc
 struct Cfg8 {
   using Operand = i32x8;
   static constexpr int kSteps = 1, kChunks = 2;
-  static constexpr bool kRowMajorB = true, kScaled = false;   // (row-major B: the one-barrier-per-step kernel only)
+  static constexpr bool kRowMajorB = true, kScaled = false, kRing = true;   // (row-major B: the one-barrier-per-step kernel only)
   static constexpr int kElemBytes = 1;
   static constexpr int kStepsPerScaleDword = 1;
   // no block scales: placeholders so that generic code naming them compiles
@@ -137,8 +137,7 @@ int gemm8_launch(const GemmArgs& p, bool e5m2, bool b_kmajor, int tile, hipStrea
   return e5m2 ? launch_gemm_tile<Cfg8<1>, true>(p, tile, stream) : launch_gemm_tile<Cfg8<0>, true>(p, tile, stream);
 }
 
-int gemm8_splitk_launch(const GemmArgs& p, bool e5m2, bool b_kmajor, int splits, int chunk_bytes, hipStream_t stream) {
-  if (b_kmajor) return e5m2 ? launch_gemm_splitk<Cfg8<1>, true>(p, splits, chunk_bytes, stream) : launch_gemm_splitk<Cfg8<0>, true>(p, splits, chunk_bytes, stream);
+int gemm8_splitk_launch(const GemmArgs& p, bool e5m2, int splits, int chunk_bytes, hipStream_t stream) {
   return e5m2 ? launch_gemm_splitk<Cfg8<1>, false>(p, splits, chunk_bytes, stream) : launch_gemm_splitk<Cfg8<0>, false>(p, splits, chunk_bytes, stream);
 }
 

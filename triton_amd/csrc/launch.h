@@ -48,7 +48,7 @@ struct GemmStridedArgs {
 
 // skinny GEMM, out[s][l] = sum_k X[s][k] * Y[l][k]
 struct SkinnyArgs {
-  const char* X;    // small operand: S <= 64 rows, K contiguous or S contiguous
+  const char* X;    // small operand: S <= 32 rows, K contiguous or S contiguous
   const char* Y;    // streamed operand: L rows, K contiguous or L contiguous
   char* C;
   int S, L, K;
@@ -109,11 +109,13 @@ int gemm_wave128_grouped_launch(const GroupedArgs& ga, bool bf16, int nprog, hip
 int gemm16_grouped_launch(const GroupedArgs& ga, bool bf16, int nprog, int nprog_big, hipStream_t stream);
 int gemm16_launch(const GemmArgs& p, bool bf16, bool b_kmajor, int tile, hipStream_t stream);
 int gemm8_launch(const GemmArgs& p, bool e5m2, bool b_kmajor, int tile, hipStream_t stream);
+// ring kernels (gemm_ring.h); shape: 0 = tiles of 128x128, 1 = 128x64, 2 = 64x64; chunk_bytes of K per split, whole 128-byte steps
+int gemm_ring16_launch(const GemmArgs& p, bool bf16, bool b_kmajor, int shape, int splits, int chunk_bytes, hipStream_t stream);
+int gemm_ring8_launch(const GemmArgs& p, bool e5m2, int shape, int splits, int chunk_bytes, hipStream_t stream);
 int gemm32_launch(const GemmArgs& p, int tile, hipStream_t stream);   // fp32 operands, K-major B; tile as for gemm16_launch
 // split-K on 128x128 tiles: `splits` chunks of `chunk_bytes` of every operand row (whole K steps of 64 bytes), fp32
 // partial tiles into p.workspace ([splits][M][N]); splitk_reduce_launch adds them up and does the epilogue
-int gemm16_splitk_launch(const GemmArgs& p, bool bf16, bool b_kmajor, int splits, int chunk_bytes, hipStream_t stream);
-int gemm8_splitk_launch(const GemmArgs& p, bool e5m2, bool b_kmajor, int splits, int chunk_bytes, hipStream_t stream);
+int gemm8_splitk_launch(const GemmArgs& p, bool e5m2, int splits, int chunk_bytes, hipStream_t stream);   // fp8 operands, row-major B
 int gemm32_splitk_launch(const GemmArgs& p, int splits, int chunk_bytes, hipStream_t stream);   // fp32 operands, K-major B
 int splitk_reduce_launch(const GemmStridedArgs& out, const float* workspace, int splits, hipStream_t stream);   // A, B, K, in_dtype of `out` unused
 bool gemm_wave128_192_ok(const GemmArgs& p, bool b_kmajor, int in_dtype, int tile_m = 192);   // the same for tiles of 192 x 256 / 128 x 256

@@ -90,38 +90,14 @@ def _scale_ptr(s, device):
     return s.data_ptr(), s
 
 
-_cu_count = {}   # device index -> compute units
-
-
-def _splitk_splits(device, M, N, k_bytes, fp32=False):
-    """Number of K splits for `matmul` (0 = none): products with less than half a round of 128x128 tiles and a long K
-    give every tile to several workgroups (`mi355_gemm_splitk`) - one workgroup per CU, at least sixteen 64-byte K steps
-    each, at most 32 slices and 64 MiB of fp32 partial sums.  Shapes with at most 64 rows on a side (and up to 128
-    against a long other side) stay with the streaming kernels."""
+def _splitk_splits(a, b, in_dt):
+    """Number of K splits for `matmul` (0 = none): products with few tiles and a long K give every tile to several
+    workgroups (`mi355_gemm_splitk`) where the library's estimate says that this pays (`mi355_gemm_splits`)."""
+    if a.shape[1] * _ELEM_BYTES[in_dt] < 2048 and in_dt != _lib.F32:   # (never pays below 16 K steps of 128 bytes)
+        return 0
     if os.environ.get("MI355_GEMM_SPLITK", "1") == "0":
         return 0
-    small, large = min(M, N), max(M, N)
-    if small <= 64 or (small <= 128 and large >= 2048):
-        return 0
-    idx = device.index if device.index is not None else torch.cuda.current_device()
-    cus = _cu_count.get(idx)
-    if cus is None:
-        cus = _cu_count[idx] = max(1, _lib.load().mi355_query(_lib.Q_CU_COUNT))
-    tiles = -(-M // 128) * -(-N // 128)
-    ksteps = -(-k_bytes // 64)
-    if fp32:
-        # bound by the fp32 MFMA rate alone: whatever puts more CUs to work wins, down to eight K steps a slice (two
-        # workgroups per CU; flushed do_bench, 1024^3: 74 -> 24 us)
-        if tiles >= cus or ksteps < 16:
-            return 0
-        splits = min(-(-2 * cus // tiles), ksteps // 8, 32, (64 << 20) // (4 * M * N))
-        return splits if splits >= 2 else 0
-    if tiles * 2 > cus or ksteps < 64:
-        return 0
-    # one workgroup per CU, at least 16 K steps each (flushed do_bench, bf16, us by number of splits - 1 / 2 / 4 / 8 / 16 /
-    # 32: 256 x 256 x 4096 51 / 34 / 24 / 20 / 19 / 23, 1024 x 1024 x 4096 52 / 38 / 30 / 36 / 49 / 71, 256 x 8192 x 8192 117 / 81 / 89 /
-    # 99 / 122 / 189, 256 x 1024 x 8192 97 / 59 / 39 / 28 / 27 / 35; 1024^3, 32 steps: 18 / 21 / 23 - not split)
-    splits = min(cus // tiles, ksteps // 16, 32, (64 << 20) // (4 * M * N))
+    splits = _lib.load().mi355_gemm_splits(a.shape[0], b.shape[1], a.shape[1], in_dt, b.stride(0) == 1)
     return splits if splits >= 2 else 0
 
 
@@ -196,7 +172,7 @@ def matmul(a, b, activation="", *, out_dtype=None, a_scale=None, b_scale=None, a
     md = hooks.enter("mi355_gemm", stream, hooks.matmul_launch_metadata, ("mi355_gemm", M, N, K_caller, _ELEM_BYTES[in_dt]))
     if (add is None and not softmax and isinstance(a, torch.Tensor) and isinstance(b, torch.Tensor)
             and (in_dt != _lib.F32 or (b.stride(0) == 1 and K % 4 == 0))):
-        splits = _splitk_splits(device, M, N, K * _ELEM_BYTES[in_dt], in_dt == _lib.F32)
+        splits = _splitk_splits(a, b, in_dt)
         if splits:
             # few tiles, long K: every tile's K range is shared out (the fp32 partial sums live in a buffer from
             # torch's caching allocator, which orders its reuse on this stream)
