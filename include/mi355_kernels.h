@@ -28,8 +28,8 @@
  * of the MFMA epilogues; 3: MFMA burn probe with its block-scaled shapes, per-device properties, fp8 attention forward at
  * head dims 16 / 32 / 256, a row-major fp8 B on the MFMA kernels, block-scaled products with any K that is a multiple of
  * 32 and scale rows of any pitch on the MFMA kernels; 4: mi355_gemm_splitk, a row-major B whose N is not a multiple of
- * 16 bytes inside a padded pitch on the tile kernels; 5: fp32 operands in mi355_gemm; 6: mi355_gemm_splits.) */
-#define MI355_ABI_VERSION 6
+ * 16 bytes inside a padded pitch on the tile kernels; 5: fp32 operands in mi355_gemm; 6: mi355_gemm_splits; 7: mi355_grouped_gemm_host.) */
+#define MI355_ABI_VERSION 7
 
 #ifdef __cplusplus
 extern "C" {
@@ -272,6 +272,15 @@ int mi355_gemm_chain(const void* A, const void* B, const void* W, void* C,
 int mi355_grouped_gemm(const void* d_a_ptrs, const void* d_b_ptrs, const void* d_c_ptrs,
                        const int32_t* d_sizes, const int32_t* d_lds, int group_size,
                        int dtype, int num_programs, void* stream);
+
+/* The same from tables in HOST memory, read before the call returns (they travel as a kernel argument, so nothing is copied
+ * to the device first): `a`, `b`, `c` are arrays of device addresses, `sizes` and `lds` as above.  One launch for up to 64
+ * problems, with tile sizes chosen per problem; problems without 16-byte rows are launched one by one.
+ * num_programs > 0 caps the workgroups of a launch.
+ */
+int mi355_grouped_gemm_host(const void* const* a, const void* const* b, void* const* c,
+                            const int32_t* sizes, const int32_t* lds, int group_size,
+                            int dtype, int num_programs, void* stream);
 
 /*
  * Block-scaled (OCP MX v1.0) GEMM: C[m,n] = sum_kb 2^(sA[m,kb]-127) 2^(sB[n,kb]-127) sum_{k in kb} A^[m,k] B^[n,k]

@@ -110,3 +110,26 @@ def test_whole_tile_groups_at_the_default_thresholds_against_closed_form(gpu, dt
         for c, r in zip(outs, ref):
             assert np.allclose(to_np(c), r, rtol=1e-2, atol=1e-2), pad
             assert np.mean(to_np(c) == r) > 0.98
+
+
+@pytest.mark.parametrize("dtype", ["fp16", "bf16"])
+@pytest.mark.parametrize("nprog", [0, 5])
+def test_host_tables_and_device_tables_agree_bit_for_bit(gpu, nprog, dtype):
+    # more problems than one table holds (64), tiles of 64 and of 128 rows next to each other, K shorter than the ring and
+    # with a tail, problems without 16-byte rows in between; the device-table entry on the same matrices, in all its forms
+    from triton_amd import _lib
+
+    rng = np.random.default_rng(70 + nprog)
+    shapes = [(17 + 31 * (i % 9), 8 * (1 + i % 7), 8 * (1 + i % 23)) for i in range(66)] + [(256, 512, 1024), (512, 256, 704), (33, 19, 7), (1, 64, 8)]
+    ga = [from_np(rng.integers(-1, 2, size=(m, k)).astype(np.float32), dtype, gpu) for m, n, k in shapes]
+    gb = [from_np(rng.integers(-1, 2, size=(k, n)).astype(np.float32), dtype, gpu) for m, n, k in shapes]
+    outs = triton_amd.group_gemm_fn(ga, gb, num_programs=nprog)
+    for a, b, c in zip(ga, gb, outs):
+        assert torch.equal(c.float(), (a.float() @ b.float()).to(c.dtype).float()), (a.shape, b.shape)
+    again = [torch.empty_like(c) for c in outs]
+    tables = [torch.tensor([t.data_ptr() for t in g], device=gpu, dtype=torch.int64) for g in (ga, gb, again)]
+    sizes = torch.tensor([v for m, n, k in shapes for v in (m, n, k)], dtype=torch.int32, device=gpu)
+    lds = torch.tensor([v for m, n, k in shapes for v in (k, n, n)], dtype=torch.int32, device=gpu)
+    rc = _lib.load().mi355_grouped_gemm(*(t.data_ptr() for t in tables), sizes.data_ptr(), lds.data_ptr(), len(shapes),
+                                        _lib.F16 if dtype == "fp16" else _lib.BF16, nprog, torch.cuda.current_stream().cuda_stream)
+    assert rc == 0 and all(torch.equal(c, d) for c, d in zip(outs, again))

@@ -24,7 +24,7 @@ Q_ABI_VERSION, Q_CU_COUNT, Q_IS_GFX950, Q_LDS_BYTES, Q_CLOCK_KHZ, Q_STREAMK_WORK
 I64x4 = c_int64 * 4
 
 # MI355_ABI_VERSION of include/mi355_kernels.h that this binding was written for
-ABI_VERSION = 6
+ABI_VERSION = 7
 
 # name -> (restype, argtypes); kept in one table so tests can check it against the header
 SIGNATURES = {
@@ -53,6 +53,7 @@ SIGNATURES = {
                                  c_int, c_int, c_void_p, c_void_p,
                                  c_void_p, c_int64, c_int64, c_int, c_int, c_int, c_void_p]),
     "mi355_grouped_gemm": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p]),
+    "mi355_grouped_gemm_host": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p]),
     "mi355_mx_gemm": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                               c_int, c_int, c_int, c_int, c_int,
                               c_int64, c_int64, c_int64, c_int64, c_int64, c_void_p]),

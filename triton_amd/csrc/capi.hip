@@ -671,6 +671,85 @@ int mi355_grouped_gemm(const void* d_a_ptrs, const void* d_b_ptrs, const void* d
   return gemm16_grouped_launch(ga, dtype == MI355_BF16, nprog, nprog_big, (hipStream_t)stream_);
 }
 
+int mi355_grouped_gemm_host(const void* const* a, const void* const* b, void* const* c,
+                            const int32_t* sizes, const int32_t* lds, int group_size,
+                            int dtype, int num_programs, void* stream_) {
+  if (!a || !b || !c || !sizes || !lds || group_size < 0 || num_programs < 0) return MI355_EINVAL;
+  if (dtype != MI355_F16 && dtype != MI355_BF16) return MI355_EDTYPE;
+  for (int i = 0; i < group_size; i++) {
+    const int32_t *s = sizes + 3 * i, *l = lds + 3 * i;
+    if (!a[i] || !b[i] || !c[i] || s[0] <= 0 || s[1] <= 0 || s[2] <= 0) return MI355_EINVAL;
+    if (l[0] < s[2] || l[1] < s[1] || l[2] < s[1]) return MI355_ESTRIDE;
+  }
+  if (!device_info().gfx950) return MI355_EDEVICE;
+  hipStream_t stream = (hipStream_t)stream_;
+  const int cus = device_info().cus > 0 ? device_info().cus : 256;
+  const bool bf16 = dtype == MI355_BF16;
+  constexpr int G = GroupedTable::kMax;
+  for (int g0 = 0; g0 < group_size; g0 += G) {
+    const int count = std::min(G, group_size - g0);
+    int order[G], n = 0;
+    double cost64[G], cost128[G], sum64 = 0, sum128 = 0, sum = 0, top64 = 0, top128 = 0, top = 0;
+    bool whole = true;
+    long tiles256 = 0;
+    for (int i = 0; i < count; i++) {
+      const int32_t *s = sizes + 3 * (g0 + i), *l = lds + 3 * (g0 + i);
+      // rows of 16-byte chunks, pitches within the kernels' lane offsets: else the product's own launch
+      if (s[2] % 8 || l[0] % 8 || l[1] % 8 || l[1] < (s[1] + 7) / 8 * 8 || !aligned(a[g0 + i], 16) || !aligned(b[g0 + i], 16) || l[0] >= (1 << 22) || l[1] >= (1 << 25)) {
+        const int rc = mi355_gemm(a[g0 + i], b[g0 + i], c[g0 + i], s[0], s[1], s[2], l[0], 1, l[1], 1, l[2], 1, dtype, dtype, nullptr, nullptr, MI355_ACT_NONE, stream_);
+        if (rc) return rc;
+        continue;
+      }
+      // us of one tile and of all, on either tile size (the figures of ring_plan with several rounds under way)
+      const int steps = (s[2] + 63) / 64;
+      const double one128 = 2.5 + 0.5 * steps, one64 = 0.6 + 0.195 * steps;
+      cost128[i] = one128 * ((s[0] + 127) / 128) * ((s[1] + 127) / 128);
+      cost64[i] = one64 * ((s[0] + 63) / 64) * ((s[1] + 63) / 64);
+      sum128 += cost128[i]; sum64 += cost64[i]; sum += std::min(cost128[i], cost64[i]);
+      top128 = std::max(top128, one128); top64 = std::max(top64, one64); top = std::max(top, cost64[i] <= cost128[i] ? one64 : one128);
+      tiles256 += (long)((s[0] + 255) / 256) * ((s[1] + 255) / 256);
+      whole = whole && s[0] % 256 == 0 && s[1] % 256 == 0 && s[2] % 128 == 0 && s[2] >= knob(knobs().grouped_wave128_min_k, 512) && l[1] % 256 == 0 &&
+              (int64_t)l[0] * 16 + s[2] * 2 < (1ll << 31) && (int64_t)s[2] * l[1] * 2 + 512 < (1ll << 31);
+      order[n++] = i;
+    }
+    if (n == 0) continue;
+    GroupedTable ga{};
+    ga.group_size = n; ga.out_dtype = dtype;
+    ga.chunk = std::max(1, knob(knobs().grouped_chunk, 4));
+    auto put = [&](int at, int i) {
+      ga.a_ptrs[at] = (uint64_t)a[g0 + i]; ga.b_ptrs[at] = (uint64_t)b[g0 + i]; ga.c_ptrs[at] = (uint64_t)c[g0 + i];
+      for (int e = 0; e < 3; e++) { ga.sizes[3 * at + e] = sizes[3 * (g0 + i) + e]; ga.lds[3 * at + e] = lds[3 * (g0 + i) + e]; }
+    };
+    int rc;
+    if (whole && knobs().grouped_wave128_min_k != 0 && tiles256 >= knob(knobs().grouped_big_min, cus)) {
+      // whole 256x256 tiles, at least one per CU: runs of them as one stream of K steps
+      for (int at = 0; at < n; at++) put(at, order[at]);
+      ga.total_tiles = (int)tiles256;
+      rc = gemm_wave128_grouped_table_launch(ga, bf16, num_programs > 0 ? std::min(num_programs, cus) : cus, stream);
+    } else {
+      // every problem on the tile size that costs it less, unless larger tiles leave CUs idle; the longest tiles first, so
+      // that the last ones to be started are short
+      const double t64 = std::max(sum64 / cus, top64), t128 = std::max(sum128 / cus, top128), tmix = std::max(sum / cus, top);
+      const int pick = t64 <= t128 && t64 <= tmix ? 64 : t128 <= tmix ? 128 : 0;
+      std::stable_sort(order, order + n, [&](int x, int y) { return sizes[3 * (g0 + x) + 2] > sizes[3 * (g0 + y) + 2]; });
+      int64_t tiles = 0;
+      for (int at = 0; at < n; at++) {
+        const int i = order[at], edge = pick ? pick : cost64[i] <= cost128[i] ? 64 : 128;
+        put(at, i);
+        ga.first_tile[at] = (int)tiles;
+        if (edge == 64) ga.small_tiles |= 1ull << at;
+        tiles += (int64_t)((ga.sizes[3 * at] + edge - 1) / edge) * ((ga.sizes[3 * at + 1] + edge - 1) / edge);
+        if (tiles > INT_MAX / 2) return MI355_ESHAPE;
+      }
+      for (int at = n; at < G; at++) ga.first_tile[at] = INT_MAX;
+      ga.total_tiles = (int)tiles;
+      rc = gemm_ring_grouped_launch(ga, bf16, num_programs > 0 ? (int)std::min<int64_t>(num_programs, tiles) : (int)tiles, stream);
+    }
+    if (rc) return rc;
+  }
+  return MI355_OK;
+}
+
 int mi355_mx_gemm(const uint8_t* A, const uint8_t* sA, const uint8_t* B, const uint8_t* sB, void* C,
                   int M, int N, int K, int fmt, int out_dtype,
                   int64_t lda, int64_t ldb, int64_t lds_a, int64_t lds_b, int64_t ldc, void* stream_) {

@@ -447,14 +447,16 @@ __global__ __launch_bounds__(256, 1) void gemm_wave128_mixed_kernel(GemmArgs p, 
 // the tiles of all problems, numbered problem after problem; a tile is one run of the stream above (its
 // loads wrap around to the tile's own first steps at the end), so consecutive tiles of a workgroup may
 // belong to different problems.  Every workgroup first reads the tables and returns unless this kernel is
-// the one that the group's shapes select (grouped_plan).
-template <typename V8>
-__global__ __launch_bounds__(256, 1) void gemm_wave128_grouped_kernel(GroupedArgs ga) {
+// the one that the group's shapes select (grouped_plan); with the tables as an argument (GroupedTable) the host has
+// selected it.
+template <typename V8, typename GA>
+__global__ __launch_bounds__(256, 1) void gemm_wave128_grouped_kernel(GA ga) {
 #if MI355_DEVICE_PASS
   extern __shared__ __attribute__((aligned(1024))) char lds_raw[];
   const unsigned lds0 = lds_addr((LDS_PTR(const void))lds_raw);
   long long total = 0;
-  if (grouped_plan(ga, &total) != 2) return;
+  if constexpr (std::is_same<GA, GroupedTable>::value) total = ga.total_tiles;
+  else if (grouped_plan(ga, &total) != 2) return;
   // The tiles of all problems, numbered problem after problem, are dealt in chunks of c consecutive tiles:
   // program w (renumbered so that the programs of one XCD are neighbours) takes the chunks w, w + nprog, ...
   // The part of a chunk inside one problem is one stream of K steps (tile after tile down a column of C
@@ -992,20 +994,24 @@ bool gemm_wave128_mixed_ok(const GemmArgs& p, bool b_kmajor, int in_dtype, int r
   return b_kmajor ? p.ldb * 8 + p.k_bytes < (1ll << 31) : (p.ldb % 512 == 0 && (int64_t)p.K * p.ldb + 512 < (1ll << 31));
 }
 
-template <typename V8>
-static int launch_wave128_grouped(const GroupedArgs& ga, int nprog, hipStream_t stream) {
+template <typename V8, typename GA>
+static int launch_wave128_grouped(const GA& ga, int nprog, hipStream_t stream) {
   constexpr int smem = 2 * 2 * 256 * 128;
   static bool attr_set = false;
   if (!attr_set) {
-    hipError_t e = hipFuncSetAttribute((const void*)gemm_wave128_grouped_kernel<V8>, hipFuncAttributeMaxDynamicSharedMemorySize, smem);
+    hipError_t e = hipFuncSetAttribute((const void*)gemm_wave128_grouped_kernel<V8, GA>, hipFuncAttributeMaxDynamicSharedMemorySize, smem);
     if (e != hipSuccess) return (int)e;
     attr_set = true;
   }
-  gemm_wave128_grouped_kernel<V8><<<dim3(nprog), dim3(256), smem, stream>>>(ga);
+  gemm_wave128_grouped_kernel<V8, GA><<<dim3(nprog), dim3(256), smem, stream>>>(ga);
   return (int)hipGetLastError();
 }
 
 int gemm_wave128_grouped_launch(const GroupedArgs& ga, bool bf16, int nprog, hipStream_t stream) {
+  return bf16 ? launch_wave128_grouped<bf16x8>(ga, nprog, stream) : launch_wave128_grouped<f16x8>(ga, nprog, stream);
+}
+
+int gemm_wave128_grouped_table_launch(const GroupedTable& ga, bool bf16, int nprog, hipStream_t stream) {
   return bf16 ? launch_wave128_grouped<bf16x8>(ga, nprog, stream) : launch_wave128_grouped<f16x8>(ga, nprog, stream);
 }
 

@@ -106,6 +106,24 @@ struct GroupedArgs {
 
 int gemm_wave128_grouped_launch(const GroupedArgs& ga, bool bf16, int nprog, hipStream_t stream);
 
+// The same tables from host memory, as a kernel argument: up to 64 problems a launch.  Names and layouts as above.
+struct GroupedTable {
+  static constexpr int kMax = 64;
+  uint64_t a_ptrs[kMax], b_ptrs[kMax], c_ptrs[kMax];
+  int sizes[kMax * 3];
+  int lds[kMax * 3];
+  int first_tile[kMax];    // ring kernel: number of the problem's first tile (past the last problem: 2^31 - 1)
+  uint64_t small_tiles;    // ring kernel: problems on tiles of 64x64, bit per problem (the others: 128x128)
+  int group_size;
+  int out_dtype;
+  int total_tiles;
+  int chunk;               // four-wave kernel
+};
+static_assert(sizeof(GroupedTable) <= 3584, "a kernel's arguments are at most 4 KiB");
+
+int gemm_wave128_grouped_table_launch(const GroupedTable& ga, bool bf16, int nprog, hipStream_t stream);   // whole 256x256 tiles, K as in grouped_plan
+int gemm_ring_grouped_launch(const GroupedTable& ga, bool bf16, int nprog, hipStream_t stream);
+
 int gemm16_grouped_launch(const GroupedArgs& ga, bool bf16, int nprog, int nprog_big, hipStream_t stream);
 int gemm16_launch(const GemmArgs& p, bool bf16, bool b_kmajor, int tile, hipStream_t stream);
 int gemm8_launch(const GemmArgs& p, bool e5m2, bool b_kmajor, int tile, hipStream_t stream);

@@ -10,8 +10,10 @@
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
 
+#include <algorithm>
 #include <stdexcept>
 #include <string>
+#include <vector>
 
 #include "../../include/mi355_kernels.h"
 
@@ -94,6 +96,37 @@ void mx_gemm(const at::Tensor& a, const at::Tensor& sa, const at::Tensor& b, con
   check(rc, "mi355_mx_gemm");
 }
 
+// [A_i @ B_i for i]: results allocated here, the tables handed over in host memory
+std::vector<at::Tensor> group_gemm(const std::vector<at::Tensor>& a, const std::vector<at::Tensor>& b, int64_t num_programs) {
+  const size_t n = a.size();
+  std::vector<at::Tensor> c;
+  if (n == 0) return c;
+  const DeviceGuard guard(a[0].device());
+  std::vector<const void*> pa(n), pb(n);
+  std::vector<void*> pc(n);
+  std::vector<int32_t> sizes(3 * n), lds(3 * n);
+  c.reserve(n);
+  size_t used = 0;
+  for (size_t i = 0; i < n; i++) {
+    on_device(a[i], 2 * (int)i); on_device(b[i], 2 * (int)i + 1);
+    TORCH_CHECK(a[i].dim() == 2 && b[i].dim() == 2, "grouped GEMM takes matrices");
+    c.push_back(at::empty({a[i].size(0), b[i].size(1)}, a[i].options()));
+    if (c[i].numel() == 0) continue;
+    if (a[i].size(1) == 0) { c[i].zero_(); continue; }
+    pa[used] = a[i].data_ptr(); pb[used] = b[i].data_ptr(); pc[used] = c[i].data_ptr();
+    int32_t *s = &sizes[3 * used], *l = &lds[3 * used];
+    s[0] = (int32_t)a[i].size(0); s[1] = (int32_t)b[i].size(1); s[2] = (int32_t)a[i].size(1);
+    // (a matrix of one row may have any row stride)
+    l[0] = (int32_t)(s[0] == 1 ? std::max<int64_t>(a[i].stride(0), s[2]) : a[i].stride(0));
+    l[1] = (int32_t)(s[2] == 1 ? std::max<int64_t>(b[i].stride(0), s[1]) : b[i].stride(0));
+    l[2] = s[1];
+    used++;
+  }
+  check(mi355_grouped_gemm_host(pa.data(), pb.data(), pc.data(), sizes.data(), lds.data(), (int)used, abi_dtype(a[0]), (int)num_programs,
+                                stream_of(a[0])), "mi355_grouped_gemm");
+  return c;
+}
+
 void strides4(const at::Tensor& t, int64_t (&s)[4]) {
   TORCH_CHECK(t.dim() == 4, "attention tensors are [Z, H, N_CTX, D]");
   for (int i = 0; i < 4; i++) s[i] = t.stride(i);
@@ -132,6 +165,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.doc() = "PyTorch-ROCm extension over the MI355X kernel library's C ABI";
   m.def("gemm", &gemm);
   m.def("mx_gemm", &mx_gemm);
+  m.def("group_gemm", &group_gemm);
   m.def("attn_fwd", &attn_fwd);
   m.def("attn_bwd", &attn_bwd);
 }

@@ -10,9 +10,9 @@ and device (the duck typing of the reference launcher, third_party/amd/backend/d
 """
 from __future__ import annotations
 
-import os
-
+import ctypes
 import math
+import os
 
 import torch
 
@@ -339,42 +339,36 @@ def matmul_persistent(a, b):
 
 def group_gemm_fn(group_A, group_B, *, num_programs: int = 0):
     """The reference's `group_gemm_fn(group_A, group_B)` (python/tutorials/08-grouped-gemm.py:143-187):
-    `[A_i @ B_i for i]` in one launch.  Builds the same five device tables (matrix addresses,
-    <M, N, K>, <lda, ldb, ldc>) and hands them to the grouped kernel; outputs have A's dtype.
-    fp16 as in the reference, or bf16.  `num_programs` is the reference's NUM_SM (0 = two per CU)."""
+    `[A_i @ B_i for i]` in one launch.  The reference copies five tables to the device first (matrix addresses,
+    <M, N, K>, <lda, ldb, ldc>); here they travel as a kernel argument; outputs have A's dtype.
+    fp16 as in the reference, or bf16.  `num_programs` is the reference's NUM_SM (0 = one per tile)."""
     assert len(group_A) == len(group_B)
     group_size = len(group_A)
     if group_size == 0:
         return []
-    device = group_A[0].device
     dt = _abi_dtype(group_A[0])
     assert dt in (_lib.F16, _lib.BF16), "grouped GEMM takes fp16 or bf16 matrices"
-    A_addrs, B_addrs, C_addrs, g_sizes, g_lds, group_C = [], [], [], [], [], []
-    for i in range(group_size):
-        A, B = group_A[i], group_B[i]
+    for i, (A, B) in enumerate(zip(group_A, group_B)):
         _check_device(2 * i, A)
         _check_device(2 * i + 1, B)
         assert A.shape[1] == B.shape[0]
         assert A.dtype == B.dtype == group_A[0].dtype, "all matrices of a group share one dtype"
         assert A.stride(1) == 1 and B.stride(1) == 1, "matrices must be row major"
-        M, K = A.shape
-        K, N = B.shape
-        C = torch.empty((M, N), device=device, dtype=A.dtype)
-        group_C.append(C)
-        A_addrs.append(A.data_ptr())
-        B_addrs.append(B.data_ptr())
-        C_addrs.append(C.data_ptr())
-        g_sizes += [M, N, K]
-        g_lds += [A.stride(0), B.stride(0), C.stride(0)]
-    # device tables, as in the reference (08:166-170)
-    d_a_ptrs = torch.tensor(A_addrs, device=device, dtype=torch.int64)
-    d_b_ptrs = torch.tensor(B_addrs, device=device, dtype=torch.int64)
-    d_c_ptrs = torch.tensor(C_addrs, device=device, dtype=torch.int64)
-    d_g_sizes = torch.tensor(g_sizes, dtype=torch.int32, device=device)
-    d_g_lds = torch.tensor(g_lds, dtype=torch.int32, device=device)
-    rc = _lib.load().mi355_grouped_gemm(d_a_ptrs.data_ptr(), d_b_ptrs.data_ptr(), d_c_ptrs.data_ptr(),
-                                        d_g_sizes.data_ptr(), d_g_lds.data_ptr(), group_size, dt,
-                                        int(num_programs), _stream())
+    ext = _lib.ext()
+    if ext is not None:
+        return ext.group_gemm(list(group_A), list(group_B), int(num_programs))
+    group_C = [torch.empty((A.shape[0], B.shape[1]), device=A.device, dtype=A.dtype) for A, B in zip(group_A, group_B)]
+    live = [i for i, C in enumerate(group_C) if C.numel() > 0 and group_A[i].shape[1] > 0]
+    for C in (group_C[i] for i in range(group_size) if i not in live):
+        C.zero_()
+    addresses = lambda group: (ctypes.c_void_p * len(live))(*(group[i].data_ptr() for i in live))   # noqa: E731
+    sizes = (ctypes.c_int32 * (3 * len(live)))(*(v for i in live for v in (*group_C[i].shape, group_A[i].shape[1])))
+    # (a matrix of one row may have any row stride)
+    lds = (ctypes.c_int32 * (3 * len(live)))(*(v for i in live for v in (
+        max(group_A[i].stride(0), group_A[i].shape[1]) if group_A[i].shape[0] == 1 else group_A[i].stride(0),
+        max(group_B[i].stride(0), group_B[i].shape[1]) if group_B[i].shape[0] == 1 else group_B[i].stride(0), group_C[i].shape[1])))
+    rc = _lib.load().mi355_grouped_gemm_host(addresses(group_A), addresses(group_B), addresses(group_C), sizes, lds, len(live),
+                                             dt, int(num_programs), _stream())
     _lib.check(rc, "mi355_grouped_gemm")
     return group_C
 
