@@ -28,8 +28,8 @@
  * of the MFMA epilogues; 3: MFMA burn probe with its block-scaled shapes, per-device properties, fp8 attention forward at
  * head dims 16 / 32 / 256, a row-major fp8 B on the MFMA kernels, block-scaled products with any K that is a multiple of
  * 32 and scale rows of any pitch on the MFMA kernels; 4: mi355_gemm_splitk, a row-major B whose N is not a multiple of
- * 16 bytes inside a padded pitch on the tile kernels; 5: fp32 operands in mi355_gemm; 6: mi355_gemm_splits; 7: mi355_grouped_gemm_host.) */
-#define MI355_ABI_VERSION 7
+ * 16 bytes inside a padded pitch on the tile kernels; 5: fp32 operands in mi355_gemm; 6: mi355_grouped_gemm_host, mi355_gemm_workspace and mi355_gemm_ws.) */
+#define MI355_ABI_VERSION 6
 
 #ifdef __cplusplus
 extern "C" {
@@ -137,7 +137,7 @@ int mi355_gemm_tuned(const void* A, const void* B, void* C,
                      const float* a_scale, const float* b_scale,
                      int activation, int tile, int group_m, void* stream);
 
-/* mi355_gemm with K split over `splits` workgroups per tile (0 = as many as mi355_gemm_splits says): for products of few
+/* mi355_gemm with K split over `splits` workgroups per tile (0 = as many as pay by the library's estimate): for products of few
  * tiles with a long K - one row of tiles against a long
  * weight, a small square against a long K -, where one workgroup per tile leaves most of the device idle and a few
  * K steps of loads in flight are all that hides the memory latency.  The reference's kernel has no such form
@@ -158,10 +158,24 @@ int mi355_gemm_splitk(const void* A, const void* B, void* C,
                       const float* a_scale, const float* b_scale,
                       int activation, int splits, void* workspace, size_t workspace_bytes, void* stream);
 
-/* The number of splits that pay for a product of these sizes by the library's own estimate (1 = none: the plain call), at
- * most 32 and 64 MiB of partial sums.  b_kmajor: B is K-contiguous.  Touches no device memory.
+/* mi355_gemm_epilogue with a workspace, for products that gain from one: operands whose rows are not whole 16-byte chunks
+ * (K or N not a multiple of the vector width, odd pitches, unaligned bases) are copied into padded rows first - one
+ * launch for both, zeros beyond K, where the reference masks its loads (python/tutorials/03-matrix-multiplication.py:297-298) -
+ * and few tiles with a long K are split as by mi355_gemm_splitk.  mi355_gemm_workspace says how many bytes such a product
+ * wants (0: none, the plain call); give mi355_gemm_ws that many, 256-byte aligned, contents irrelevant, used until the
+ * launches of the call have run.  workspace_bytes = 0 and softmax = 1 run as mi355_gemm_epilogue.
  */
-int mi355_gemm_splits(int M, int N, int K, int in_dtype, int b_kmajor);
+int64_t mi355_gemm_workspace(const void* A, const void* B, int M, int N, int K,
+                             int64_t stride_am, int64_t stride_ak, int64_t stride_bk, int64_t stride_bn, int in_dtype);
+int mi355_gemm_ws(const void* A, const void* B, void* C,
+                  int M, int N, int K,
+                  int64_t stride_am, int64_t stride_ak,
+                  int64_t stride_bk, int64_t stride_bn,
+                  int64_t stride_cm, int64_t stride_cn,
+                  int in_dtype, int out_dtype,
+                  const float* a_scale, const float* b_scale,
+                  const void* addend, int64_t stride_dm, int64_t stride_dn, int addend_dtype,
+                  int activation, int softmax, void* workspace, size_t workspace_bytes, void* stream);
 
 /* mi355_gemm with a stream-K schedule: one program per CU, and the programs split ALL K steps of ALL
  * 256x256 tiles evenly, so a tile count that is not a multiple of the CU count (or smaller than it:

@@ -1390,3 +1390,27 @@ def test_ring_kernels_at_the_edges_of_their_ring_are_bit_exact(gpu, dtype, tile,
                                             {"fp16": _lib.F16, "bf16": _lib.BF16, "e4m3": _lib.F8E4M3}[dtype], _lib.F16, None, None, _lib.ACT_NONE,
                                             torch.cuda.current_stream().cuda_stream)
                 assert rc == 0 and bits_equal(to_np(cbuf[:, :N].contiguous()), ref) and bool((cbuf[:, N:] == 7.0).all()), (M, N, K, pitch)
+
+
+@pytest.mark.parametrize("dtype", ["fp16", "bf16", "e4m3"])
+@pytest.mark.parametrize("K", [2047, 2051, 2056, 4101])   # one element short of a 128-byte line, odd, a chunk multiple, odd and split
+def test_rows_that_do_not_start_on_16_byte_boundaries_are_exact(gpu, dtype, K):
+    # the padded copies (odd K, odd N, odd pitches, bases off by one element), one operand or both, and a row-major B with
+    # good rows that is not copied although A's rows get zeros beyond K; sums of small integers below 2^24: every bit of
+    # the fp32 result is determined
+    rng = np.random.default_rng(K)
+    code = {"fp16": torch.float16, "bf16": torch.bfloat16, "e4m3": torch.float8_e4m3fn}[dtype]
+
+    def tensor(x):
+        return torch.from_numpy(x).to(gpu).to(code)
+
+    for M, N in [(300, 264), (257, 199), (1, 320), (129, 1024)]:
+        a = rng.integers(-2, 3, size=(M, K)).astype(np.float32)
+        b = rng.integers(-2, 3, size=(K, N)).astype(np.float32)
+        ref = a @ b
+        flat = tensor(np.concatenate([np.zeros(1, np.float32), a.reshape(-1)]))        # A one element behind an aligned base
+        wide = tensor(np.pad(b, ((0, 0), (1, 2 + N % 2))))                             # B inside wider rows, one column in
+        for ta in (tensor(a), flat[1:].view(M, K)):
+            for tb in (tensor(b), tensor(np.ascontiguousarray(b.T)).t(), wide[:, 1:1 + N]):
+                got = to_np(triton_amd.matmul(ta, tb, out_dtype=torch.float32))
+                assert bits_equal(got, ref), (M, N, K, tb.stride(), ta.data_ptr() % 16)

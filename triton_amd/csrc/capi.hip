@@ -53,7 +53,7 @@ const DeviceInfo& device_info() {
 constexpr int UNSET = INT_MIN;
 struct Knobs {
   int force_strided, group_m, tile, programs, skinny, grouped_big_min, grouped_wave128_min_k, grouped_chunk,
-      attn_fwd_variant, attn_programs, lean_epilogue, tile_m, rowfused_max_mk, mixed_rows;
+      attn_fwd_variant, attn_programs, lean_epilogue, tile_m, rowfused_max_mk, mixed_rows, splitk;
 };
 Knobs g_knobs;
 std::atomic<int> g_knobs_ready{0};
@@ -83,6 +83,7 @@ void load_knobs() {
   k.tile_m = read_env("MI355_GEMM_TILE_M", 0);
   k.rowfused_max_mk = read_env("MI355_ROWFUSED_MAX_MK", 0);
   k.mixed_rows = read_env("MI355_GEMM_MIXED_ROWS", 0);
+  k.splitk = read_env("MI355_GEMM_SPLITK", 0);   // 0: matmul's own route never splits K
   g_knobs = k;
   g_knobs_ready.store(1, std::memory_order_release);
 }
@@ -265,7 +266,7 @@ static int gemm_impl(const void* A, const void* B, void* C, int M, int N, int K,
                      int64_t sam, int64_t sak, int64_t sbk, int64_t sbn, int64_t scm, int64_t scn,
                      int in_dtype, int out_dtype, const float* a_scale, const float* b_scale,
                      int activation, const void* aux, int64_t aux_sm, int64_t aux_sn, int aux_dtype,
-                     int tile_arg, int group_m_arg, void* stream_, float* workspace = nullptr) {
+                     int tile_arg, int group_m_arg, void* stream_, float* workspace = nullptr, int k_rows = 0) {
   if (!A || !B || !C || M <= 0 || N <= 0 || K <= 0) return MI355_EINVAL;
   if (aux && aux_dtype != MI355_F16 && aux_dtype != MI355_BF16 && aux_dtype != MI355_F32) return MI355_EDTYPE;
   if (activation != MI355_ACT_NONE && activation != MI355_ACT_LEAKY_RELU) return MI355_EINVAL;
@@ -423,7 +424,7 @@ static int gemm_impl(const void* A, const void* B, void* C, int M, int N, int K,
   const int ksteps128 = (p.k_bytes + 127) / 128;
   // at most 32 rows on one side: stream the other operand once (X = small side, Y = streamed side) where that is the faster
   // way (skinny_us), or where MI355_GEMM_SKINNY asks for it
-  if (skinny_allowed && std::min(M, N) <= 32 &&
+  if (skinny_allowed && k_rows == 0 && std::min(M, N) <= 32 &&
       (knobs().skinny != UNSET || !can_ring || skinny_us(M, N, p.k_bytes, es, b_kmajor) < ring_plan(M, N, ksteps128, cus, 1, 1).us)) {
     SkinnyArgs sk{};
     sk.K = K; sk.C = (char*)C; sk.a_scale = a_scale; sk.b_scale = b_scale;
@@ -447,7 +448,10 @@ static int gemm_impl(const void* A, const void* B, void* C, int M, int N, int K,
   int ring = -1;
   if (can_ring) {
     const bool by_knob = tile_arg >= 0 || knobs().tile != UNSET;
-    if (tile == 1) ring = by_knob ? 0 : ring_plan(M, N, ksteps128, cus, 1, 1).shape;
+    if (k_rows > 0) {   // a row-major B that ends before A's padding does: the ring kernels know
+      ring = ring_plan(M, N, ksteps128, cus, 1, 1).shape;
+      p.K = k_rows;
+    } else if (tile == 1) ring = by_knob ? 0 : ring_plan(M, N, ksteps128, cus, 1, 1).shape;
     else if (tile >= 8 && tile <= 10) ring = tile - 8;
     else if (!by_knob && knobs().tile_m == UNSET && knobs().mixed_rows == UNSET) {
       const int rows = tile == 6 && p.tile_m ? p.tile_m : 256;
@@ -488,17 +492,11 @@ int mi355_gemm_tuned(const void* A, const void* B, void* C, int M, int N, int K,
                    activation, nullptr, 0, 0, 0, tile, group_m, stream_);
 }
 
-int mi355_gemm_splits(int M, int N, int K, int in_dtype, int b_kmajor) {
-  if (M <= 0 || N <= 0 || K <= 0 || in_dtype < MI355_F16 || in_dtype > MI355_F32) return 1;
-  const int es = elem_size(in_dtype);
-  return auto_splits(M, N, (int64_t)K * es, in_dtype, b_kmajor != 0, ring_ok(es, b_kmajor != 0),
-                     device_info().cus > 0 ? device_info().cus : 256);
-}
-
-int mi355_gemm_splitk(const void* A, const void* B, void* C, int M, int N, int K,
-                      int64_t sam, int64_t sak, int64_t sbk, int64_t sbn, int64_t scm, int64_t scn,
-                      int in_dtype, int out_dtype, const float* a_scale, const float* b_scale,
-                      int activation, int splits, void* workspace, size_t workspace_bytes, void* stream_) {
+static int splitk_impl(const void* A, const void* B, void* C, int M, int N, int K,
+                       int64_t sam, int64_t sak, int64_t sbk, int64_t sbn, int64_t scm, int64_t scn,
+                       int in_dtype, int out_dtype, const float* a_scale, const float* b_scale,
+                       int activation, const void* aux, int64_t aux_sm, int64_t aux_sn, int aux_dtype,
+                       int splits, void* workspace, size_t workspace_bytes, void* stream_, int k_rows) {
   if (!A || !B || !C || M <= 0 || N <= 0 || K <= 0 || splits < 0) return MI355_EINVAL;
   if (activation != MI355_ACT_NONE && activation != MI355_ACT_LEAKY_RELU) return MI355_EINVAL;
   if (in_dtype < MI355_F16 || in_dtype > MI355_F32) return MI355_EDTYPE;
@@ -519,12 +517,13 @@ int mi355_gemm_splitk(const void* A, const void* B, void* C, int M, int N, int K
   const int per = splits >= 2 ? (ksteps + splits - 1) / splits : ksteps;
   const int used = (ksteps + per - 1) / per;   // (no split is left empty)
   if (!(a_ok && (b_kmajor || b_nmajor) && pitch_ok) || used < 2 || knob(knobs().force_strided, 0) != 0)
-    return mi355_gemm(A, B, C, M, N, K, sam, sak, sbk, sbn, scm, scn, in_dtype, out_dtype, a_scale, b_scale, activation, stream_);
+    return gemm_impl(A, B, C, M, N, K, sam, sak, sbk, sbn, scm, scn, in_dtype, out_dtype, a_scale, b_scale, activation,
+                     aux, aux_sm, aux_sn, aux_dtype, -1, 0, stream_, nullptr, k_rows);
   if (!workspace || !aligned(workspace, 16) || workspace_bytes < (size_t)used * M * N * sizeof(float)) return MI355_EINVAL;
   hipStream_t stream = (hipStream_t)stream_;
   GemmArgs p{};
   p.A = (const char*)A; p.B = (const char*)B; p.C = (char*)C;
-  p.M = M; p.N = N; p.K = K; p.k_bytes = (int)k_bytes;
+  p.M = M; p.N = N; p.K = k_rows > 0 ? k_rows : K; p.k_bytes = (int)k_bytes;
   p.lda = sam * es;
   p.ldb = (b_kmajor ? sbn : sbk) * es;
   p.group_m = knob(knobs().group_m, 8);
@@ -538,7 +537,158 @@ int mi355_gemm_splitk(const void* A, const void* B, void* C, int M, int N, int K
   GemmStridedArgs out{};
   out.C = C; out.M = M; out.N = N; out.scm = scm; out.scn = scn;
   out.a_scale = a_scale; out.b_scale = b_scale; out.activation = activation; out.out_dtype = out_dtype;
+  out.aux = aux; out.aux_sm = aux_sm; out.aux_sn = aux_sn; out.aux_dtype = aux_dtype;
   return splitk_reduce_launch(out, (const float*)workspace, used, stream);
+}
+
+int mi355_gemm_splitk(const void* A, const void* B, void* C, int M, int N, int K,
+                      int64_t sam, int64_t sak, int64_t sbk, int64_t sbn, int64_t scm, int64_t scn,
+                      int in_dtype, int out_dtype, const float* a_scale, const float* b_scale,
+                      int activation, int splits, void* workspace, size_t workspace_bytes, void* stream_) {
+  return splitk_impl(A, B, C, M, N, K, sam, sak, sbk, sbn, scm, scn, in_dtype, out_dtype, a_scale, b_scale, activation,
+                     nullptr, 0, 0, 0, splits, workspace, workspace_bytes, stream_, 0);
+}
+
+// a row that fits one tile: product, addend, activation and softmax in ONE launch, on the fp32 accumulator,
+// one rounding at the store - what the reference's single tile does
+// (that kernel is one workgroup per 128 rows with operands of any strides, built for the small products of the
+// reference's test, where the single rounding is the point: on time the tiled GEMM plus a softmax launch wins at every
+// size - flushed caches, bf16: 32^3 10.8 against 9.3 us, 128 x 256 x 128 50 / 13, 1024 x 256 x 256 59 / 14, 8192 x 256 x 256
+// 59 / 19, 256 x 256 x 2048 237 / 33 - and takes over beyond 2^18 elements of A by default, MI355_ROWFUSED_MAX_MK)
+static bool rowfused(int M, int N, int K, int in_dtype) {
+  return N <= 256 && (in_dtype == MI355_F16 || in_dtype == MI355_BF16) && (int64_t)M * K <= (int64_t)knob(knobs().rowfused_max_mk, 1 << 18);
+}
+
+// ---- mi355_gemm_ws: how a product with a workspace runs.  Operands whose rows the MFMA kernels cannot load (rows that are not
+// whole 16-byte chunks) are first copied into rows of a padded pitch, both in one launch, zeros behind K; few tiles with a
+// long K are split.  The any-stride kernel stays where the copies would cost more than they gain.
+namespace {
+
+struct GemmRoute {
+  bool pack_a = false, pack_b = false;
+  bool kmajor = false;
+  int k = 0;                     // K as the kernels see it
+  int k_rows = 0;                // > 0: rows of a row-major B that is not copied while A's K was padded beyond them
+  int b_rows = 0;                // rows of the copy of B
+  int64_t a_pitch = 0, b_pitch = 0;   // bytes
+  int splits = 1;
+  size_t a_bytes = 0, b_bytes = 0, slice_bytes = 0;
+};
+
+size_t up(size_t v, size_t to) { return (v + to - 1) / to * to; }
+
+GemmRoute gemm_route(const void* A, const void* B, int M, int N, int K, int64_t sam, int64_t sak, int64_t sbk, int64_t sbn, int in_dtype) {
+  GemmRoute r;
+  r.k = K;
+  const int es = elem_size(in_dtype), vec = 16 / es, cus = device_info().cus > 0 ? device_info().cus : 256;
+  if (knob(knobs().force_strided, 0) != 0) return r;
+  auto split = [&](bool kmajor) {
+    if (knob(knobs().splitk, 1) == 0) return;
+    r.splits = auto_splits(M, N, (int64_t)r.k * es, in_dtype, kmajor, ring_ok(es, kmajor), cus);
+    r.slice_bytes = r.splits > 1 ? (size_t)r.splits * M * N * 4 : 0;
+  };
+  // (as in gemm_impl)
+  const bool a_ok = sak == 1 && sam % vec == 0 && sam >= K && aligned(A, 16) && K % vec == 0;
+  const bool bk_ok = sbk == 1 && sbn % vec == 0 && sbn >= K && aligned(B, 16) && K % vec == 0;
+  const bool bn_ok = es != 4 && sbn == 1 && sbk % vec == 0 && sbk >= (N + vec - 1) / vec * vec && aligned(B, 16);
+  if (a_ok && (bk_ok || bn_ok)) {
+    split(bk_ok);
+    return r;
+  }
+  if (es == 4 || sak != 1 || sam < K || (sbk == 1) == (sbn == 1)) return r;
+  r.kmajor = sbk == 1;
+  if (r.kmajor ? sbn < K : sbk < N) return r;
+  const bool b_ok = r.kmajor ? bk_ok : bn_ok;
+  // us: the copies at about 4.5 TB/s of reads and writes, then the best kernel
+  auto copy_us = [&](bool a, bool b) { return 2.0 + 2.0 * es * ((a ? (double)M * K : 0.0) + (b ? (double)N * K : 0.0)) / 4.5e6; };
+  const int steps = (int)(((int64_t)K * es + 127) / 128);
+  const double ring = ring_ok(es, r.kmajor) ? ring_plan(M, N, steps, cus, 1, 1).us : 1e30;
+  const double any = std::min(ring, tiles256_us((long)((M + 255) / 256) * ((N + 255) / 256), 256, steps, cus, true, es == 1));
+  r.pack_a = !a_ok;
+  // a row-major B with good rows only lacks the zero rows beyond K, which the ring kernels do not read
+  r.pack_b = !b_ok || (!r.kmajor && K % vec != 0 && ring + copy_us(!a_ok, false) > any + copy_us(!a_ok, true));
+  const double packed = copy_us(r.pack_a, r.pack_b) + (r.pack_b || r.kmajor || K % vec == 0 ? any : ring);
+  // (any-stride kernel: 64x64 tiles, about 1.3 us per 64 k: 1024 x 1024 x 1000 bf16 23 us, x 4100 107)
+  const long tiles = (long)((M + 63) / 64) * ((N + 63) / 64);
+  const double masked = kLaunchUs + (double)((tiles + cus - 1) / cus) * (1.0 + 1.3 * ((K + 63) / 64));
+  if (masked <= packed) {
+    r.pack_a = r.pack_b = false;
+    return r;
+  }
+  if (K % vec != 0) {
+    r.k = (int)up(K, r.pack_b || r.kmajor ? 128 / es : vec);
+    if (!r.kmajor && !r.pack_b) r.k_rows = K;
+  }
+  if (r.pack_a) {
+    r.a_pitch = (int64_t)up((size_t)r.k * es, 128);
+    r.a_bytes = up((size_t)r.a_pitch * M, 256);
+  }
+  if (r.pack_b) {
+    r.b_rows = r.kmajor ? N : r.k;
+    r.b_pitch = (int64_t)(r.kmajor ? up((size_t)r.k * es, 128) : up((size_t)N * es, 512));
+    r.b_bytes = up((size_t)r.b_pitch * r.b_rows, 256);
+  }
+  if (r.a_pitch >= (1 << 23) || r.b_pitch >= (r.kmajor ? 1 << 23 : 1 << 26)) {   // (beyond the kernels' lane offsets)
+    GemmRoute plain;
+    plain.k = K;
+    return plain;
+  }
+  split(r.kmajor);
+  return r;
+}
+
+}  // namespace
+
+int64_t mi355_gemm_workspace(const void* A, const void* B, int M, int N, int K,
+                             int64_t sam, int64_t sak, int64_t sbk, int64_t sbn, int in_dtype) {
+  if (M <= 0 || N <= 0 || K <= 0 || in_dtype < MI355_F16 || in_dtype > MI355_F32) return 0;
+  const GemmRoute r = gemm_route(A, B, M, N, K, sam, sak, sbk, sbn, in_dtype);
+  return (int64_t)(r.a_bytes + r.b_bytes + r.slice_bytes);
+}
+
+int mi355_gemm_ws(const void* A, const void* B, void* C, int M, int N, int K,
+                  int64_t sam, int64_t sak, int64_t sbk, int64_t sbn, int64_t scm, int64_t scn,
+                  int in_dtype, int out_dtype, const float* a_scale, const float* b_scale,
+                  const void* addend, int64_t sdm, int64_t sdn, int addend_dtype,
+                  int activation, int softmax, void* workspace, size_t workspace_bytes, void* stream_) {
+  if (!A || !B || !C || M <= 0 || N <= 0 || K <= 0) return MI355_EINVAL;
+  if (in_dtype < MI355_F16 || in_dtype > MI355_F32) return MI355_EDTYPE;
+  if (!device_info().gfx950) return MI355_EDEVICE;
+  if (softmax != 0 && softmax != 1) return MI355_EINVAL;
+  if (softmax && out_dtype != MI355_F16 && out_dtype != MI355_BF16 && out_dtype != MI355_F32) return MI355_EDTYPE;
+  if (workspace_bytes == 0 || (softmax && rowfused(M, N, K, in_dtype)))
+    return mi355_gemm_epilogue(A, B, C, M, N, K, sam, sak, sbk, sbn, scm, scn, in_dtype, out_dtype, a_scale, b_scale,
+                               addend, sdm, sdn, addend_dtype, activation, softmax, stream_);
+  if (addend && addend_dtype != MI355_F16 && addend_dtype != MI355_BF16 && addend_dtype != MI355_F32) return MI355_EDTYPE;
+  const GemmRoute r = gemm_route(A, B, M, N, K, sam, sak, sbk, sbn, in_dtype);
+  if (!workspace || !aligned(workspace, 256) || workspace_bytes < r.a_bytes + r.b_bytes + r.slice_bytes) return MI355_EINVAL;
+  const int es = elem_size(in_dtype);
+  char* ws = (char*)workspace;
+  RepackRows op[2];
+  int ops = 0;
+  if (r.pack_a) {
+    op[ops++] = {(const char*)A, ws, M, M, K * es, (int)up((size_t)r.k * es, 16), sam * es, r.a_pitch};
+    A = ws; sam = r.a_pitch / es;
+  }
+  if (r.pack_b) {
+    char* to = ws + r.a_bytes;
+    if (r.kmajor) op[ops++] = {(const char*)B, to, N, N, K * es, (int)up((size_t)r.k * es, 16), sbn * es, r.b_pitch};
+    else op[ops++] = {(const char*)B, to, K, r.b_rows, N * es, (int)up((size_t)N * es, 16), sbk * es, r.b_pitch};
+    B = to; (r.kmajor ? sbn : sbk) = r.b_pitch / es;
+  }
+  if (ops > 0) {
+    const int rc = repack_launch(op, ops, (hipStream_t)stream_);
+    if (rc) return rc;
+  }
+  int rc;
+  if (r.splits > 1)
+    rc = splitk_impl(A, B, C, M, N, r.k, sam, sak, sbk, sbn, scm, scn, in_dtype, out_dtype, a_scale, b_scale, activation,
+                       addend, sdm, sdn, addend_dtype, r.splits, ws + r.a_bytes + r.b_bytes, r.slice_bytes, stream_, r.k_rows);
+  else
+    rc = gemm_impl(A, B, C, M, N, r.k, sam, sak, sbk, sbn, scm, scn, in_dtype, out_dtype, a_scale, b_scale, activation,
+                   addend, sdm, sdn, addend_dtype, -1, 0, stream_, nullptr, r.k_rows);
+  if (rc || !softmax) return rc;
+  return softmax_rows_launch(C, M, N, scm, scn, out_dtype, (hipStream_t)stream_);
 }
 
 int mi355_gemm_streamk(const void* A, const void* B, void* C, int M, int N, int K,
@@ -608,14 +758,7 @@ int mi355_gemm_epilogue(const void* A, const void* B, void* C, int M, int N, int
                         int activation, int softmax, void* stream_) {
   if (softmax != 0 && softmax != 1) return MI355_EINVAL;
   if (softmax && out_dtype != MI355_F16 && out_dtype != MI355_BF16 && out_dtype != MI355_F32) return MI355_EDTYPE;
-  // a row that fits one tile: product, addend, activation and softmax in ONE launch, on the fp32 accumulator,
-  // one rounding at the store - what the reference's single tile does
-  // (that kernel is one workgroup per 128 rows with operands of any strides, built for the small products of the
-  // reference's test, where the single rounding is the point: on time the tiled GEMM plus a softmax launch wins at every
-  // size - flushed caches, bf16: 32^3 10.8 against 9.3 us, 128 x 256 x 128 50 / 13, 1024 x 256 x 256 59 / 14, 8192 x 256 x 256
-  // 59 / 19, 256 x 256 x 2048 237 / 33 - and takes over beyond 2^18 elements of A by default, MI355_ROWFUSED_MAX_MK)
-  const int64_t rowfused_max = (int64_t)knob(knobs().rowfused_max_mk, 1 << 18);
-  if (softmax && N <= 256 && (in_dtype == MI355_F16 || in_dtype == MI355_BF16) && (int64_t)M * K <= rowfused_max) {
+  if (softmax && rowfused(M, N, K, in_dtype)) {
     if (!A || !B || !C || M <= 0 || N <= 0 || K <= 0) return MI355_EINVAL;
     if (addend && addend_dtype != MI355_F16 && addend_dtype != MI355_BF16 && addend_dtype != MI355_F32) return MI355_EDTYPE;
     if (activation != MI355_ACT_NONE && activation != MI355_ACT_LEAKY_RELU) return MI355_EINVAL;

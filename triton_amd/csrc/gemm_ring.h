@@ -215,7 +215,8 @@ __device__ __forceinline__ void ring_drain_wait(int left) {
 constexpr int RING_ROW = 128;   // bytes of an operand row per K step
 
 // Tile (pm, pn) of the product p with the ring of NS stages at LDS address lds0 (NS * (BM + BN) * 128 bytes).  A has whole
-// 16-byte chunks along K and a K-major B too; a row-major B (16-bit types) has rows of whole 16-byte chunks.  Every wave's
+// 16-byte chunks along K (k_bytes of them) and a K-major B too; a row-major B (16-bit types) has rows of whole 16-byte chunks,
+// p.K of them: in the last chunk's place of A's rows there may be zeros beyond K.  Every wave's
 // fragments are in registers when the last step's MFMAs begin, so a caller that runs another tile needs one barrier first.
 template <typename E, int BM, int BN, int WN, bool B_KMAJOR, int NS>
 __device__ __forceinline__ void gemm_ring_tile(const GemmArgs& p, const int pm, const int pn, const unsigned lds0) {
@@ -360,6 +361,7 @@ __device__ __forceinline__ void gemm_ring_tile(const GemmArgs& p, const int pm, 
   if (tail) {   // (one block from the loads to their use: at a join the compiler may copy registers still in flight)
     i32x4 ta[LA], tb[LB];
     const int kfull = p.k_bytes - tail;                       // bytes of K before the tail
+    const int krows = p.K - kfull / E::kElemBytes;            // (a row-major B may end before the padded rows of A do)
     const char* kA = tileA + kfull;
     const char* kB = B_KMAJOR ? tileB + kfull : tileB + (int64_t)(kfull / 2) * p.ldb;
 #pragma unroll
@@ -367,7 +369,7 @@ __device__ __forceinline__ void gemm_ring_tile(const GemmArgs& p, const int pm, 
 #pragma unroll
     for (int q = 0; q < LB; q++) {
       if constexpr (B_KMAJOR) load16_sbase<0>(tb[q], kB, voffB[q] + q * 1024 - rowB[q] * 16 + min(rowB[q] * 16, tail - 16));
-      else load16_sbase<0>(tb[q], kB, voffB[q] + q * 1024 - (unsigned)(rowB[q] - min(rowB[q], tail / 2 - 1)) * (unsigned)p.ldb);
+      else load16_sbase<0>(tb[q], kB, voffB[q] + q * 1024 - (unsigned)(rowB[q] - min(rowB[q], krows - 1)) * (unsigned)p.ldb);
     }
     fill(true);
     const i32x4 zero = {0, 0, 0, 0};
@@ -379,7 +381,7 @@ __device__ __forceinline__ void gemm_ring_tile(const GemmArgs& p, const int pm, 
 #pragma unroll
     for (int q = 0; q < LB; q++) {
       lds_use(tb[q]);
-      const bool in = B_KMAJOR ? rowB[q] * 16 < tail : rowB[q] * 2 < tail;
+      const bool in = B_KMAJOR ? rowB[q] * 16 < tail : rowB[q] < krows;
       *(LDS_PTR(i32x4))(uintptr_t)(lds0 + A_BYTES + (wave * LB + q) * 1024 + lane * 16) = in ? tb[q] : zero;
     }
     lds_wait<0>();
@@ -463,6 +465,7 @@ __global__ __launch_bounds__(128 * WN, 1) void gemm_ring_kernel(GemmArgs p, int 
     const int z = t / tiles, k0 = z * chunk_bytes;
     t -= z * tiles;
     p.k_bytes = min(p.k_bytes - k0, chunk_bytes);   // (the host leaves no split empty)
+    p.K -= k0 / E::kElemBytes;
     p.A += k0;
     p.B += B_KMAJOR ? (int64_t)k0 : (int64_t)(k0 / E::kElemBytes) * p.ldb;
     p.C = (char*)(p.workspace + (int64_t)z * p.M * p.N);

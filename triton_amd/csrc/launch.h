@@ -168,6 +168,9 @@ int attn_bwd_pre_launch(const AttnArgs& p, bool bf16, hipStream_t stream);
 int attn_bwd_launch(const AttnArgs& p, bool bf16, hipStream_t stream);
 int gemm_rowfused_launch(const RowFusedArgs& p, bool bf16, hipStream_t stream);
 int softmax_rows_launch(void* C, int M, int N, int64_t scm, int64_t scn, int dtype, hipStream_t stream);
+// `rows` rows of `bytes` bytes, `pitch` apart, into `dst_rows` rows of `dst_bytes` (whole 16-byte chunks), zeros where the source ends
+struct RepackRows { const char* src; char* dst; int rows, dst_rows; int bytes, dst_bytes; int64_t pitch, dst_pitch; };
+int repack_launch(const RepackRows* op, int count, hipStream_t stream);   // count: 1 or 2
 int clock_probe_launch(unsigned long long* out, unsigned long long real_ticks, hipStream_t stream);
 int mfma_burn_launch(float* sink, int shape, int random_operands, int iters, int waves_per_simd, int cus, hipStream_t stream);
 int dequant_launch(const uint8_t* codes, float* out, int64_t n, int fmt, hipStream_t stream);

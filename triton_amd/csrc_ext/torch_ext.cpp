@@ -3,7 +3,7 @@
 // tensor objects (`data_ptr()`, :285-323), takes the stream the caller's framework is on
 // (python/triton/runtime/jit.py:588-589 passes torch's current stream) and launches.  Here: tensor
 // checks, sizes / strides / dtypes read off the at::Tensor, c10::hip::getCurrentHIPStream(), one C call.
-// No device code in this file and no logic beyond argument marshalling: every status of the C ABI
+// No device code in this file and no logic beyond checks, allocation and argument marshalling: every status of the C ABI
 // becomes the exception the reference raises for the same condition (RuntimeError "Triton Error [HIP]"
 // for launch failures, :258-269; ValueError for pointers the device cannot reach, :313-317).
 #include <torch/extension.h>
@@ -17,6 +17,8 @@
 
 #include "../../include/mi355_kernels.h"
 
+namespace py = pybind11;
+
 namespace {
 
 int abi_dtype(const at::Tensor& t) {
@@ -26,7 +28,7 @@ int abi_dtype(const at::Tensor& t) {
     case at::kFloat8_e4m3fn: return MI355_F8E4M3;
     case at::kFloat8_e5m2: return MI355_F8E5M2;
     case at::kFloat: return MI355_F32;
-    default: throw std::invalid_argument(std::string("unsupported dtype ") + c10::toString(t.scalar_type()));
+    default: throw py::type_error(std::string("unsupported dtype ") + c10::toString(t.scalar_type()));
   }
 }
 
@@ -57,33 +59,51 @@ const float* scale_ptr(const c10::optional<at::Tensor>& s) {
   return s->data_ptr<float>();
 }
 
-// C = act((a_scale * b_scale) * A @ B [+ D]) [row softmax]; `add` is already broadcast to [M, N] (zero strides)
-void gemm(const at::Tensor& a, const at::Tensor& b, at::Tensor& c, int64_t activation,
-          const c10::optional<at::Tensor>& a_scale, const c10::optional<at::Tensor>& b_scale,
-          const c10::optional<at::Tensor>& add, bool softmax) {
-  TORCH_CHECK(a.dim() == 2 && b.dim() == 2 && c.dim() == 2 && a.size(1) == b.size(0), "Incompatible dimensions");
-  on_device(a, 0); on_device(b, 1); on_device(c, 2);
+[[noreturn]] void fail(PyObject* type, const std::string& message) {
+  PyErr_SetString(type, message.c_str());
+  throw py::error_already_set();
+}
+
+// C = softmax_rows?(act((a_scale * b_scale) * A @ B + add)): the checks of the reference's wrapper
+// (python/tutorials/03-matrix-multiplication.py:330-348) with its exceptions, the result and the workspace from torch's
+// allocator (which orders their reuse on the current stream), one C call.  activation: MI355_ACT_*.
+at::Tensor matmul(const at::Tensor& a, const at::Tensor& b_in, int64_t activation, const c10::optional<at::ScalarType>& out_dtype,
+                  const c10::optional<at::Tensor>& a_scale, const c10::optional<at::Tensor>& b_scale,
+                  const c10::optional<at::Tensor>& add, bool softmax) {
+  at::Tensor b = b_in;
+  if (a.dim() != 2 || b.dim() != 2 || a.size(1) != b.size(0)) fail(PyExc_AssertionError, "Incompatible dimensions");
+  if (!a.is_contiguous()) fail(PyExc_AssertionError, "Matrix A must be contiguous");
+  const int in_dt = abi_dtype(a);
+  if (a.scalar_type() != b.scalar_type()) fail(PyExc_AssertionError, "Incompatible dtypes");
+  on_device(a, 0); on_device(b, 1);
   const DeviceGuard guard(a.device());
-  const int M = (int)a.size(0), K = (int)a.size(1), N = (int)b.size(1);
-  int rc;
-  if (!add.has_value() && !softmax) {
-    rc = mi355_gemm(a.data_ptr(), b.data_ptr(), c.data_ptr(), M, N, K, a.stride(0), a.stride(1), b.stride(0), b.stride(1),
-                    c.stride(0), c.stride(1), abi_dtype(a), abi_dtype(c), scale_ptr(a_scale), scale_ptr(b_scale),
-                    (int)activation, stream_of(a));
-    check(rc, "mi355_gemm");
-    return;
-  }
+  const int64_t M = a.size(0), K = a.size(1), N = b.size(1);
+  at::Tensor c = at::empty({M, N}, a.options().dtype(out_dtype.has_value() ? *out_dtype : in_dt == MI355_BF16 ? at::kBFloat16 : at::kHalf));
+  if (M == 0 || N == 0) return c;
+  if (K == 0) return c.zero_();
+  // fp32 operands run on the fp32 MFMAs with a K-major B only (the LDS transpose reads stop at 16-bit elements): a
+  // row-major B is put K-major first - one transposing copy, 1 / M of the product's work -; small products and a K
+  // that is not a multiple of four elements take the any-stride kernel of the C ABI as they are
+  if (in_dt == MI355_F32 && b.stride(0) != 1 && K % 4 == 0 && M * N * K >= (1 << 24)) b = b.t().contiguous().t();
   const void* d = nullptr;
   int64_t dsm = 0, dsn = 0;
   int ddt = 0;
+  at::Tensor wide;
   if (add.has_value()) {
-    on_device(*add, 3);
-    d = add->data_ptr(); dsm = add->stride(0); dsn = add->stride(1); ddt = abi_dtype(*add);
+    on_device(*add, 2);
+    ddt = abi_dtype(*add);
+    if (ddt != MI355_F16 && ddt != MI355_BF16 && ddt != MI355_F32) fail(PyExc_TypeError, std::string("add must be fp16, bf16 or fp32, got ") + c10::toString(add->scalar_type()));
+    wide = add->expand({M, N});   // (zero strides on broadcast axes)
+    d = wide.data_ptr(); dsm = wide.stride(0); dsn = wide.stride(1);
   }
-  rc = mi355_gemm_epilogue(a.data_ptr(), b.data_ptr(), c.data_ptr(), M, N, K, a.stride(0), a.stride(1), b.stride(0), b.stride(1),
-                           c.stride(0), c.stride(1), abi_dtype(a), abi_dtype(c), scale_ptr(a_scale), scale_ptr(b_scale),
-                           d, dsm, dsn, ddt, (int)activation, softmax ? 1 : 0, stream_of(a));
-  check(rc, "mi355_gemm_epilogue");
+  const int64_t need = mi355_gemm_workspace(a.data_ptr(), b.data_ptr(), (int)M, (int)N, (int)K, a.stride(0), a.stride(1), b.stride(0), b.stride(1), in_dt);
+  at::Tensor ws;
+  if (need > 0) ws = at::empty({need}, a.options().dtype(at::kByte));
+  const int rc = mi355_gemm_ws(a.data_ptr(), b.data_ptr(), c.data_ptr(), (int)M, (int)N, (int)K, a.stride(0), a.stride(1), b.stride(0), b.stride(1),
+                               c.stride(0), c.stride(1), in_dt, abi_dtype(c), scale_ptr(a_scale), scale_ptr(b_scale),
+                               d, dsm, dsn, ddt, (int)activation, softmax ? 1 : 0, need > 0 ? ws.data_ptr() : nullptr, (size_t)need, stream_of(a));
+  check(rc, "mi355_gemm");
+  return c;
 }
 
 void mx_gemm(const at::Tensor& a, const at::Tensor& sa, const at::Tensor& b, const at::Tensor& sb, at::Tensor& c, int64_t fmt, int64_t K) {
@@ -163,7 +183,7 @@ void attn_bwd(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, con
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.doc() = "PyTorch-ROCm extension over the MI355X kernel library's C ABI";
-  m.def("gemm", &gemm);
+  m.def("matmul", &matmul);
   m.def("mx_gemm", &mx_gemm);
   m.def("group_gemm", &group_gemm);
   m.def("attn_fwd", &attn_fwd);

@@ -90,17 +90,6 @@ def _scale_ptr(s, device):
     return s.data_ptr(), s
 
 
-def _splitk_splits(a, b, in_dt):
-    """Number of K splits for `matmul` (0 = none): products with few tiles and a long K give every tile to several
-    workgroups (`mi355_gemm_splitk`) where the library's estimate says that this pays (`mi355_gemm_splits`)."""
-    if a.shape[1] * _ELEM_BYTES[in_dt] < 2048 and in_dt != _lib.F32:   # (never pays below 16 K steps of 128 bytes)
-        return 0
-    if os.environ.get("MI355_GEMM_SPLITK", "1") == "0":
-        return 0
-    splits = _lib.load().mi355_gemm_splits(a.shape[0], b.shape[1], a.shape[1], in_dt, b.stride(0) == 1)
-    return splits if splits >= 2 else 0
-
-
 def matmul(a, b, activation="", *, out_dtype=None, a_scale=None, b_scale=None, add=None, softmax=False):
     """C = softmax_rows?(act((a_scale*b_scale) * A @ B + add)) with fp32 accumulation.
 
@@ -114,6 +103,30 @@ def matmul(a, b, activation="", *, out_dtype=None, a_scale=None, b_scale=None, a
     add-cols) and `softmax` are the fused epilogues of the reference's dot test
     (python/test/unit/language/test_core.py:3128-3141).
     """
+    act = _ACTIVATIONS.get(activation)
+    if act is None:
+        raise KeyError(f"unknown ACTIVATION {activation!r}")
+    ext = _lib.ext()
+    if ext is None or not (isinstance(a, torch.Tensor) and isinstance(b, torch.Tensor)):
+        return _matmul_ctypes(a, b, act, out_dtype, a_scale, b_scale, add, softmax)
+    if a_scale is not None:
+        a_scale = _scale_ptr(a_scale, a.device)[1]
+    if b_scale is not None:
+        b_scale = _scale_ptr(b_scale, a.device)[1]
+    if hooks.Launch.launch_enter_hook is None and hooks.Launch.launch_exit_hook is None:
+        return ext.matmul(a, b, act, out_dtype, a_scale, b_scale, add, softmax)
+    md = hooks.enter("mi355_gemm", _stream(), hooks.matmul_launch_metadata,
+                     ("mi355_gemm", a.shape[0], b.shape[1], a.shape[1], a.element_size()))
+    c = ext.matmul(a, b, act, out_dtype, a_scale, b_scale, add, softmax)
+    hooks.exit(md)
+    return c
+
+
+_ACTIVATIONS = {"": _lib.ACT_NONE, "leaky_relu": _lib.ACT_LEAKY_RELU}
+
+
+def _matmul_ctypes(a, b, act, out_dtype, a_scale, b_scale, add, softmax):
+    """`matmul` for tensors of other libraries and without the torch extension: the same checks and the same C call."""
     assert a.shape[1] == b.shape[0], "Incompatible dimensions"
     assert _is_contiguous(a), "Matrix A must be contiguous"
     in_dt = _abi_dtype(a)
@@ -121,100 +134,37 @@ def matmul(a, b, activation="", *, out_dtype=None, a_scale=None, b_scale=None, a
     _check_device(0, a)
     _check_device(1, b)
     M, K = a.shape
-    K, N = b.shape
-    K_caller = K
+    N = b.shape[1]
     if out_dtype is None:
         out_dtype = torch.bfloat16 if in_dt == _lib.BF16 else torch.float16
-    if activation not in ("", "leaky_relu"):
-        raise KeyError(f"unknown ACTIVATION {activation!r}")
     device = a.device if isinstance(a, torch.Tensor) else torch.device("cuda", torch.cuda.current_device())
     c = torch.empty((M, N), device=device, dtype=out_dtype)
     if M == 0 or N == 0:
         return c
     if K == 0:
         return c.zero_()
-    if (in_dt != _lib.F32 and (K * _ELEM_BYTES[in_dt]) % 16 != 0 and M * N * K >= 1 << 30
-            and isinstance(a, torch.Tensor) and isinstance(b, torch.Tensor)):
-        # Rows of A that are not a multiple of 16 bytes long do not start on 16-byte boundaries, which every MFMA
-        # kernel's loads need: the C ABI then runs its strided kernel (4096 x 4096 x 4100 bf16: 43 TFLOP/s).  The
-        # reference masks the K tail to zero (03:297-298); appending those zeros to K here - one copy of each
-        # operand - gives the same sums on the fast kernels (the same shape: 1000 TFLOP/s).  Below about 2^30
-        # multiply-adds the any-stride MFMA kernel is as fast or faster than the copies plus the tile kernels (flushed
-        # do_bench, bf16, that kernel / padded: 2048 x 100 x 100 12 / 27 us, 2047 x 257 x 257 16 / 32, 1024 x 1024 x 1000 23 / 23,
-        # 1024 x 1024 x 4100 107 / 70).
-        pad = -K % (16 // _ELEM_BYTES[in_dt])
-        as_bytes = (lambda t: t.view(torch.uint8)) if _ELEM_BYTES[in_dt] == 1 else (lambda t: t)
-        a = torch.nn.functional.pad(as_bytes(a), (0, pad)).view(a.dtype)
-        if b.stride(0) == 1 and b.stride(1) != 1:      # K-major B: its K axis is the contiguous one of b.t()
-            b = torch.nn.functional.pad(as_bytes(b.t()), (0, pad)).view(b.dtype).t()
-        else:
-            b = torch.nn.functional.pad(as_bytes(b), (0, 0, 0, pad)).view(b.dtype)
-        K += pad        # (the launch metadata below keeps the caller's K)
-    if (in_dt == _lib.F32 and isinstance(b, torch.Tensor) and b.stride(0) != 1 and K % 4 == 0 and M * N * K >= 1 << 24):
-        # fp32 operands run on the fp32 MFMAs with a K-major B only (the LDS transpose reads stop at 16-bit elements): a
-        # row-major B is put K-major first - one transposing copy, 1 / M of the product's work -; small products and a K
-        # that is not a multiple of four elements take the any-stride kernel of the C ABI as they are
-        b = b.t().contiguous().t()
-    vec = 16 // _ELEM_BYTES[in_dt] if in_dt != _lib.F32 else 0
-    if (vec and isinstance(b, torch.Tensor) and b.stride(1) == 1 and b.stride(0) != 1
-            and (b.stride(0) % vec != 0 or b.data_ptr() % 16 != 0) and K % vec == 0 and M * N * K >= 1 << 30):
-        # A row-major B runs on the MFMAs inside the C ABI when its rows START on 16-byte boundaries (N itself need not
-        # be a multiple: the last chunk of a row then reaches into the padding that the pitch provides).  One whose
-        # pitch is not a multiple of 16 bytes would take the any-stride kernel (8100 x 8100 x 8192 bf16: 48 TFLOP/s on
-        # the old kernel of that path): its rows are copied into a buffer with a padded pitch first - one plain copy,
-        # as the reference spends one on its fp8 case ("pre-transpose b for efficiency", 03:378-380).
-        as_bytes = (lambda t: t.view(torch.uint8)) if _ELEM_BYTES[in_dt] == 1 else (lambda t: t)
-        b = torch.nn.functional.pad(as_bytes(b), (0, -N % vec)).view(b.dtype)[:, :N]
+    if in_dt == _lib.F32 and isinstance(b, torch.Tensor) and b.stride(0) != 1 and K % 4 == 0 and M * N * K >= 1 << 24:
+        b = b.t().contiguous().t()   # (fp32 MFMAs: K-major B only)
     pa, keep_a = _scale_ptr(a_scale, device)
     pb, keep_b = _scale_ptr(b_scale, device)
-    act = _lib.ACT_LEAKY_RELU if activation == "leaky_relu" else _lib.ACT_NONE
-    stream = _stream()
-    md = hooks.enter("mi355_gemm", stream, hooks.matmul_launch_metadata, ("mi355_gemm", M, N, K_caller, _ELEM_BYTES[in_dt]))
-    if (add is None and not softmax and isinstance(a, torch.Tensor) and isinstance(b, torch.Tensor)
-            and (in_dt != _lib.F32 or (b.stride(0) == 1 and K % 4 == 0))):
-        splits = _splitk_splits(a, b, in_dt)
-        if splits:
-            # few tiles, long K: every tile's K range is shared out (the fp32 partial sums live in a buffer from
-            # torch's caching allocator, which orders its reuse on this stream)
-            ws = torch.empty(splits * M * N, dtype=torch.float32, device=device)
-            rc = _lib.load().mi355_gemm_splitk(
-                a.data_ptr(), b.data_ptr(), c.data_ptr(), M, N, K,
-                a.stride(0), a.stride(1), b.stride(0), b.stride(1), c.stride(0), c.stride(1),
-                in_dt, _TORCH_TO_ABI[out_dtype], pa, pb, act, splits, ws.data_ptr(), ws.numel() * 4, stream)
-            _lib.check(rc, "mi355_gemm_splitk")
-            hooks.exit(md)
-            return c
-    ext = _lib.ext()
-    if ext is not None and isinstance(a, torch.Tensor) and isinstance(b, torch.Tensor):
-        # the PyTorch-ROCm extension: tensors in, torch's current stream taken in C++, one C-ABI call
-        d = None
-        if add is not None:
-            if add.dtype not in (torch.float16, torch.bfloat16, torch.float32):
-                raise TypeError(f"add must be fp16, bf16 or fp32, got {add.dtype}")
-            d = torch.broadcast_to(add, (M, N))
-        ext.gemm(a, b, c, act, keep_a, keep_b, d, bool(softmax))
-        hooks.exit(md)
-        return c
-    if add is None and not softmax:
-        rc = _lib.load().mi355_gemm(
-            a.data_ptr(), b.data_ptr(), c.data_ptr(), M, N, K,
-            a.stride(0), a.stride(1), b.stride(0), b.stride(1), c.stride(0), c.stride(1),
-            in_dt, _TORCH_TO_ABI[out_dtype], pa, pb, act, stream)
-        _lib.check(rc, "mi355_gemm")
-        hooks.exit(md)
-        return c
-    d_ptr, d_sm, d_sn, d_dt = 0, 0, 0, 0
+    d_ptr, d_sm, d_sn, d_dt = None, 0, 0, 0
     if add is not None:
         _check_device(2, add)
         if add.dtype not in (torch.float16, torch.bfloat16, torch.float32):
             raise TypeError(f"add must be fp16, bf16 or fp32, got {add.dtype}")
         d = torch.broadcast_to(add, (M, N))  # zero strides on broadcast axes
         d_ptr, d_sm, d_sn, d_dt = d.data_ptr(), d.stride(0), d.stride(1), _TORCH_TO_ABI[add.dtype]
-    rc = _lib.load().mi355_gemm_epilogue(
+    lib = _lib.load()
+    stream = _stream()
+    md = hooks.enter("mi355_gemm", stream, hooks.matmul_launch_metadata, ("mi355_gemm", M, N, K, _ELEM_BYTES[in_dt]))
+    need = lib.mi355_gemm_workspace(a.data_ptr(), b.data_ptr(), M, N, K, a.stride(0), a.stride(1), b.stride(0), b.stride(1), in_dt)
+    ws = torch.empty(need, dtype=torch.uint8, device=device) if need else None
+    rc = lib.mi355_gemm_ws(
         a.data_ptr(), b.data_ptr(), c.data_ptr(), M, N, K,
         a.stride(0), a.stride(1), b.stride(0), b.stride(1), c.stride(0), c.stride(1),
-        in_dt, _TORCH_TO_ABI[out_dtype], pa, pb, d_ptr, d_sm, d_sn, d_dt, act, int(bool(softmax)), stream)
-    _lib.check(rc, "mi355_gemm_epilogue")
+        in_dt, _TORCH_TO_ABI[out_dtype], pa, pb, d_ptr, d_sm, d_sn, d_dt, act, int(bool(softmax)),
+        ws.data_ptr() if need else None, need, stream)
+    _lib.check(rc, "mi355_gemm")
     hooks.exit(md)
     return c
 
