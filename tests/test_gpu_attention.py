@@ -270,3 +270,28 @@ def test_head_dims_16_and_32_touch_only_their_own_columns(gpu, D):
         assert np.allclose(to_np(t), cf[name], atol=1e-2, rtol=1e-2), name
         assert torch.all(outs[name][..., D:] == 7.0), name       # nothing stored beyond column HEAD_DIM
     assert np.allclose(to_np(M), cf["M"], atol=2e-3, rtol=0)
+
+
+@pytest.mark.parametrize("head_dim", [64, 128])
+@pytest.mark.parametrize("n_ctx", [128, 256, 384, 1024])
+@pytest.mark.parametrize("causal", [True, False])
+def test_forward_with_groups_of_waves_along_the_keys(gpu, causal, n_ctx, head_dim, monkeypatch):
+    # 6, 7, 8: two, four and two groups whose partial results meet in LDS: fewer blocks of keys than groups, a group
+    # without any unmasked key, rows whose maximum lies in another group than the first; o and M against the fp64 closed
+    # form, with the tolerances of the other variants
+    from triton_amd import _lib
+    (q, k, v, _), (tq, tk, tv, _) = _inputs(11 + n_ctx, (1, 3, n_ctx, head_dim), "fp16", gpu)
+    k[:, :, n_ctx // 2:] *= 4.0
+    tk = from_np(k, "fp16", gpu)
+    cf = A.attn_closed_form(q, k, v, causal, 0.25)
+    I4 = _lib.I64x4
+    for variant in ("6", "7", "8"):
+        set_knob(monkeypatch, "MI355_ATTN_FWD_VARIANT", variant)
+        o = torch.full_like(tq, 7.0)
+        M = torch.full((1, 3, n_ctx), 7.0, dtype=torch.float32, device=gpu)
+        rc = _lib.load().mi355_attn_fwd(tq.data_ptr(), tk.data_ptr(), tv.data_ptr(), o.data_ptr(), M.data_ptr(),
+                                        1, 3, n_ctx, head_dim, I4(*tq.stride()), I4(*tk.stride()), I4(*tv.stride()), I4(*o.stride()),
+                                        0.25, int(causal), _lib.F16, torch.cuda.current_stream().cuda_stream)
+        assert rc == 0
+        assert np.allclose(to_np(M), cf["M"], atol=2e-3, rtol=0), variant
+        assert np.allclose(to_np(o), cf["o"], atol=1e-2, rtol=1e-2), variant

@@ -39,12 +39,21 @@ template <> struct Elem<f16x8> { using type = _Float16; };
 // never exist in memory - fragments loaded straight into registers are zero-filled, the K / V tiles in LDS are
 // zeroed once and only the chunks present are ever loaded, and only the first d_real columns of O are stored.
 // Scores, softmax and those columns of O are what a HEAD_DIM d_real kernel computes (zero columns add nothing).
-template <typename V8, int D, int QT, int NW, bool PAD = false>
+//
+// KW > 1: the workgroup's waves are KW groups that share its query rows and take every KW-th block of 64 keys each - a step
+// covers KW blocks -, and whose partial results (maximum, sum and accumulator of every row) meet in LDS at the end.  For
+// heads x rows that give fewer workgroups than CUs: a wave takes 0.7 us for a block of 64 keys (head_dim 64; MFMAs,
+// exponentials and conversions of 32 x 64 scores one after the other), so the number of blocks in a row is what such a
+// launch takes.  fp16, 16 heads x 1024 rows, head_dim 64, causal: 22.7 us in 64
+// workgroups of eight waves along the rows, 15.0 in 128 of four, 10.4 in 256 of two times two.
+template <typename V8, int D, int QT, int NW, bool PAD = false, int KW = 1>
 __global__ __launch_bounds__(NW * 64, 1) void attn_fwd_kernel(AttnArgs p) {
   using S = typename Elem<V8>::type;
-  constexpr int BM = NW * QT * 32, BN = 64;
+  constexpr int QW = NW / KW;          // waves along the query rows
+  static_assert(NW % KW == 0 && (KW == 1 || QT == 1), "whole groups of waves");
+  constexpr int BM = QW * QT * 32, BN = 64;
   constexpr int RB = D * 2;            // bytes per K/V row
-  using Tile = AttnTile<RB, BN, NW>;
+  using Tile = AttnTile<RB, BN * KW, NW>;
   constexpr int TILE = Tile::BYTES;    // bytes of one K or V tile
   constexpr int INST = Tile::INST;     // direct-load instructions per wave and tile
   constexpr int KSQ = D / 16;          // MFMA k-steps of S^T = K Q^T
@@ -66,7 +75,8 @@ __global__ __launch_bounds__(NW * 64, 1) void attn_fwd_kernel(AttnArgs p) {
   if (p.causal) qb = nqb - 1 - qb;
   const int z = hz / p.H, h = hz % p.H;
   const int m0 = qb * BM;
-  const int row0 = m0 + wave * QT * 32;  // first query row of this wave
+  const int kw = wave / QW;                   // which of a step's KW blocks of keys (wave-uniform)
+  const int row0 = m0 + (wave % QW) * QT * 32;  // first query row of this wave
 
   const char* qbase = p.q + ((int64_t)z * p.sq[0] + (int64_t)h * p.sq[1]) * 2;
   const char* kbase = p.k + ((int64_t)z * p.sk[0] + (int64_t)h * p.sk[1]) * 2;
@@ -105,8 +115,8 @@ __global__ __launch_bounds__(NW * 64, 1) void attn_fwd_kernel(AttnArgs p) {
   }
   auto issue_kv = [&](int j, int stage) {
     const unsigned kd = lds_base + stage * (2 * TILE), vd = kd + TILE;
-    const char* ksrc = kbase + (int64_t)j * BN * kpitch;
-    const char* vsrc = vbase + (int64_t)j * BN * vpitch;
+    const char* ksrc = kbase + (int64_t)j * (BN * KW) * kpitch;
+    const char* vsrc = vbase + (int64_t)j * (BN * KW) * vpitch;
 #pragma unroll
     for (int i = 0; i < INST; i++) {
       if (present[i]) {
@@ -123,11 +133,11 @@ __global__ __launch_bounds__(NW * 64, 1) void attn_fwd_kernel(AttnArgs p) {
   const unsigned lds0 = lds_addr(lds);
   unsigned ka[KSQ], va[DT][2];
 #pragma unroll
-  for (int ks = 0; ks < KSQ; ks++) ka[ks] = lds0 + rk.rowb + (rk.xk ^ (ks * 32));
+  for (int ks = 0; ks < KSQ; ks++) ka[ks] = lds0 + kw * (BN * RB) + rk.rowb + (rk.xk ^ (ks * 32));
 #pragma unroll
   for (int c = 0; c < DT; c++)
 #pragma unroll
-    for (int h2 = 0; h2 < 2; h2++) va[c][h2] = lds0 + (tv.tl ^ ((c << 6) | (h2 << 5)));
+    for (int h2 = 0; h2 < 2; h2++) va[c][h2] = lds0 + kw * (BN * RB) + (tv.tl ^ ((c << 6) | (h2 << 5)));
 
   f32x16 oacc[DT][QT];
 #pragma unroll
@@ -148,9 +158,9 @@ __global__ __launch_bounds__(NW * 64, 1) void attn_fwd_kernel(AttnArgs p) {
 
   // number of K/V steps of this block / wave
   const int kv_end_blk = p.causal ? min(p.N, m0 + BM) : p.N;
-  const int nsteps = (kv_end_blk + BN - 1) / BN;
-  const int wave_last = p.causal ? (row0 + QT * 32 - 1) / BN : nsteps - 1;  // last step with unmasked columns
-  const int wave_first_masked = p.causal ? row0 / BN : nsteps;              // first step that needs the mask
+  const int nsteps = (kv_end_blk + BN * KW - 1) / (BN * KW);
+  const int wave_last = p.causal ? (row0 + QT * 32 - 1) / BN : nsteps * KW - 1;  // last block with unmasked columns
+  const int wave_first_masked = p.causal ? row0 / BN : nsteps * KW;              // first block that needs the mask
 
   issue_kv(0, 0);
   wait_all();
@@ -164,7 +174,8 @@ __global__ __launch_bounds__(NW * 64, 1) void attn_fwd_kernel(AttnArgs p) {
     constexpr int KOFF = kStageImm ? stage * 2 * TILE : 0, VOFF = KOFF + TILE;
     const unsigned sreg = kStageImm ? 0u : (unsigned)(stage * 2 * TILE);
     if (j + 1 < nsteps) issue_kv(j + 1, stage ^ 1);
-    if (j <= wave_last && row0 < p.N) {
+    const int blk = j * KW + kw;
+    if (blk <= wave_last && row0 < p.N) {
       // ---- S^T = K Q^T : [2 kv tiles][QT q tiles]
       f32x16 s[2][QT];
 #pragma unroll
@@ -219,13 +230,13 @@ __global__ __launch_bounds__(NW * 64, 1) void attn_fwd_kernel(AttnArgs p) {
       V8 pf[QT][4];  // P^T as B operand of the second product, per 16-column k-step
 #pragma unroll
       for (int b = 0; b < QT; b++) {
-        if (j >= wave_first_masked) {
+        if (blk >= wave_first_masked) {
           const int qrow = row0 + b * 32 + l32;
 #pragma unroll
           for (int a = 0; a < 2; a++)
 #pragma unroll
             for (int r = 0; r < 16; r++) {
-              int kv = j * BN + a * 32 + (r >> 2) * 8 + g * 4 + (r & 3);
+              int kv = blk * BN + a * 32 + (r >> 2) * 8 + g * 4 + (r & 3);
               if (kv > qrow) s[a][b][r] = -INFINITY;
             }
         }
@@ -294,6 +305,43 @@ __global__ __launch_bounds__(NW * 64, 1) void attn_fwd_kernel(AttnArgs p) {
     if (j + 1 < nsteps) step(j + 1, std::integral_constant<int, 1>{});
   }
 
+  // ---- the groups' partial results into the first group's waves (the K/V stages are free)
+  if constexpr (KW > 1) {
+    constexpr int PER = DT * 16 + 2;   // floats per lane: accumulator, maximum, sum
+    LDS_PTR(float) const part = (LDS_PTR(float))(lds + QW * 32 * RB);   // (behind the rows that the epilogue stages)
+    if (kw > 0) {
+      LDS_PTR(float) to = part + ((kw - 1) * QW + wave % QW) * (PER * 64) + lane;
+#pragma unroll
+      for (int c = 0; c < DT; c++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) to[(c * 16 + r) * 64] = oacc[c][0][r];
+      to[(PER - 2) * 64] = m_i[0];
+      to[(PER - 1) * 64] = l_i[0];
+    }
+    __syncthreads();
+    if (kw > 0) return;
+    float top = m_i[0];   // (finite: the first group has the first key)
+#pragma unroll
+    for (int w = 1; w < KW; w++) top = fmaxf(top, part[((w - 1) * QW + wave) * (PER * 64) + (PER - 2) * 64 + lane]);
+    const float own = fast_exp2(m_i[0] - top);
+    l_i[0] *= own;
+#pragma unroll
+    for (int c = 0; c < DT; c++)
+#pragma unroll
+      for (int r = 0; r < 16; r++) oacc[c][0][r] *= own;
+#pragma unroll
+    for (int w = 1; w < KW; w++) {
+      LDS_PTR(float) from = part + ((w - 1) * QW + wave) * (PER * 64) + lane;
+      const float f = fast_exp2(from[(PER - 2) * 64] - top);
+      l_i[0] += f * from[(PER - 1) * 64];
+#pragma unroll
+      for (int c = 0; c < DT; c++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) oacc[c][0][r] += f * from[(c * 16 + r) * 64];
+    }
+    m_i[0] = top;
+  }
+
   // ---- epilogue: O = acc / l, M = m + log2(l)
 #pragma unroll
   for (int b = 0; b < QT; b++) {
@@ -307,7 +355,7 @@ __global__ __launch_bounds__(NW * 64, 1) void attn_fwd_kernel(AttnArgs p) {
     f32x16 ob[DT];
 #pragma unroll
     for (int c = 0; c < DT; c++) ob[c] = oacc[c][b];
-    store_rows_transposed<S, D, PAD>(ob, inv, lds0 + (wave * QT + b) * 32 * RB, obase + (int64_t)(row0 + b * 32) * opitch, opitch,
+    store_rows_transposed<S, D, PAD>(ob, inv, lds0 + ((wave % QW) * QT + b) * 32 * RB, obase + (int64_t)(row0 + b * 32) * opitch, opitch,
                             p.N - (row0 + b * 32), p.d_real, lane);
   }
 }
@@ -647,19 +695,20 @@ static int launch_fwd_stream(const AttnArgs& p, hipStream_t stream) {
   return (int)hipGetLastError();
 }
 
-template <typename V8, int D, int QT, int NW, bool PAD = false>
+template <typename V8, int D, int QT, int NW, bool PAD = false, int KW = 1>
 static int launch_fwd(const AttnArgs& p, hipStream_t stream) {
-  constexpr int BM = NW * QT * 32;
-  constexpr int smem = 2 * 2 * 64 * D * 2;
+  constexpr int BM = NW / KW * QT * 32;
+  constexpr int smem = 2 * 2 * 64 * KW * D * 2;
+  static_assert(KW == 1 || smem >= NW / KW * 32 * D * 2 + (KW - 1) * (NW / KW) * (D / 32 * 16 + 2) * 256, "the partial results fit the stages");
   static bool attr_set = false;
   if (!attr_set) {
-    hipError_t e = hipFuncSetAttribute((const void*)attn_fwd_kernel<V8, D, QT, NW, PAD>,
+    hipError_t e = hipFuncSetAttribute((const void*)attn_fwd_kernel<V8, D, QT, NW, PAD, KW>,
                                        hipFuncAttributeMaxDynamicSharedMemorySize, smem);
     if (e != hipSuccess) return (int)e;
     attr_set = true;
   }
   int nqb = (p.N + BM - 1) / BM;
-  attn_fwd_kernel<V8, D, QT, NW, PAD><<<dim3(nqb * p.Z * p.H), dim3(NW * 64), smem, stream>>>(p);
+  attn_fwd_kernel<V8, D, QT, NW, PAD, KW><<<dim3(nqb * p.Z * p.H), dim3(NW * 64), smem, stream>>>(p);
   return (int)hipGetLastError();
 }
 
@@ -667,6 +716,11 @@ template <typename V8>
 static int launch_fwd_d(const AttnArgs& p, int variant, hipStream_t stream) {
   // head dims 16 / 32: the 64-column kernels in their padding form (eight waves; persistent under the causal mask)
   if (p.d_real < p.D) return p.causal ? launch_fwd_stream<V8, 64, 8, true>(p, stream) : launch_fwd<V8, 64, 1, 8, true>(p, stream);
+  // groups of waves along the keys: 6 = 64 query rows per workgroup and two groups, 7 = 32 rows and four groups (head_dim
+  // 64: 256 keys per step, N a multiple of that), 8 = 128 rows and two groups (eight waves)
+  if (variant == 6 && p.D != 256) return p.D == 128 ? launch_fwd<V8, 128, 1, 4, false, 2>(p, stream) : launch_fwd<V8, 64, 1, 4, false, 2>(p, stream);
+  if (variant == 7 && p.D == 64 && p.N % 256 == 0) return launch_fwd<V8, 64, 1, 4, false, 4>(p, stream);
+  if (variant == 8 && p.D != 256) return p.D == 128 ? launch_fwd<V8, 128, 1, 8, false, 2>(p, stream) : launch_fwd<V8, 64, 1, 8, false, 2>(p, stream);
   if (variant == 3 && p.D != 256) return p.D == 128 ? launch_fwd_stream<V8, 128, 4>(p, stream) : launch_fwd_stream<V8, 64, 4>(p, stream);
   if (variant == 4 && p.D != 256) return p.D == 128 ? launch_fwd_stream<V8, 128, 8>(p, stream) : launch_fwd_stream<V8, 64, 8>(p, stream);
   // head_dim 256: four waves of 32 query rows, one wave per SIMD (the O accumulator alone is 128 registers)

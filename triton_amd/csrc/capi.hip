@@ -1018,6 +1018,28 @@ static bool attn_stride_ok(const int64_t* s, const void* ptr, int D) {
   return s[3] == 1 && s[2] >= D && s[2] < (1 << 24) && s[0] % 8 == 0 && s[1] % 8 == 0 && s[2] % 8 == 0 && aligned(ptr, 16);
 }
 
+// Which form of the forward: the fewer query rows there are for the CUs, the smaller a workgroup's block of rows and the more
+// of its waves go along the keys instead (us, fp16, causal / not, by form: 2 = 256 rows, 4 = its persistent form, 1 = 128
+// rows, 8 = 128 rows x 2 groups, 6 = 64 x 2, 7 = 32 x 4).
+static int attn_fwd_variant(const AttnArgs& p, int cus) {
+  const int dflt = p.causal ? 4 : 2;
+  if (p.D == 256 || p.d_real < p.D) return dflt;
+  const int64_t rows = (int64_t)p.Z * p.H * p.N;
+  // head_dim 64, 8 heads x 1024: 7 8.3 / 8.2, 6 10.3 / 10.2, 8 12.7 / 12.6, 1 15.0 / 14.6
+  if (p.D == 64 && p.N % 256 == 0 && rows <= 32ll * cus) return 7;
+  // 16 x 1024: 6 10.4 / 10.5, 7 12.1 / 15.0, 8 12.9 / 12.8; head_dim 128: 6 15.7 / 16.3, 8 18.7 / 18.5, 1 20.9 / 20.6
+  if (rows <= 64ll * cus) return 6;
+  // 16 x 2048: 8 22.4 / 24.9, 6 24.0 / 27.0, 1 26.7 / 27.5; head_dim 128: 8 32.6 / 40.1, 6 32.2 / 50.6, 1 36.9 / 41.5
+  if (rows <= 128ll * cus) return 8;
+  if (p.causal && rows <= 256ll * cus) {
+    // (few, long rows of work under the mask) 32 x 2048: 6 34.1, 8 37.1, 2 38.4, 4 40.7; 8 x 8192: 6 102, 8 101, 4 142
+    if (p.D == 64 && p.N >= 2048) return 6;
+    // head_dim 128, 8 x 8192: 8 146, 1 173, 2 189, 4 197; 32 x 2048: 2 52.3, 8 56.2, 4 56.9; 128 x 512: 2 20.7, 4 23.2
+    return p.D == 128 && p.N >= 4096 ? 8 : 2;
+  }
+  return dflt;
+}
+
 int mi355_attn_fwd(const void* q, const void* k, const void* v, void* o, float* Mlse,
                    int Z, int H, int N_CTX, int D,
                    const int64_t* sq, const int64_t* sk, const int64_t* sv, const int64_t* so,
@@ -1053,7 +1075,7 @@ int mi355_attn_fwd(const void* q, const void* k, const void* v, void* o, float* 
   // eight waves (256 query rows) per K/V stream halve the L2 -> LDS traffic.  Under the causal mask
   // their row ranges are uneven, which the persistent form (4) evens out by pairing long and short
   // query blocks per program; without a mask the one-item-per-workgroup form (2) is the faster one.
-  p.variant = knob(knobs().attn_fwd_variant, causal ? 4 : 2);
+  p.variant = knob(knobs().attn_fwd_variant, attn_fwd_variant(p, device_info().cus > 0 ? device_info().cus : 256));
   p.num_programs = knob(knobs().attn_programs, device_info().cus > 0 ? device_info().cus : 256);
   // 5: four waves of 64 query rows, 16x16x32 MFMAs, software pipelined inside the wave (head_dim 128)
   if (p.variant == 5 && attn_fwd_pipe_ok(p)) return attn_fwd_pipe_launch(p, dtype == MI355_BF16, (hipStream_t)stream_);
