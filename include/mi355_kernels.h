@@ -359,6 +359,17 @@ int mi355_attn_bwd(const void* q, const void* k, const void* v, const void* d_o,
                    float sm_scale, int causal, int dtype, void* stream);
 
 /*
+ * The same from the forward's o in place of a computed delta: the dQ kernel computes delta and writes it
+ * to `delta` (contiguous [Z,H,N_CTX]), from where the dK/dV kernel reads it.  o has the common strides too.
+ */
+int mi355_attn_bwd_o(const void* q, const void* k, const void* v, const void* o, const void* d_o,
+                     const float* Mlse, float* delta,
+                     void* dq, void* dk, void* dv,
+                     int Z, int H, int N_CTX, int D,
+                     const int64_t* stride,
+                     float sm_scale, int causal, int dtype, void* stream);
+
+/*
  * out[i] = decode(codes[i]) in fp32 for n code BYTES (MI355_DEQ_E2M1 writes 2n values), using the
  * decode routines the strided kernels use.  The formats are those of the reference type table
  * (python/triton/language/core.py:352-363) and of its up-cast emulation

@@ -295,3 +295,34 @@ def test_forward_with_groups_of_waves_along_the_keys(gpu, causal, n_ctx, head_di
         assert rc == 0
         assert np.allclose(to_np(M), cf["M"], atol=2e-3, rtol=0), variant
         assert np.allclose(to_np(o), cf["o"], atol=1e-2, rtol=1e-2), variant
+
+
+@pytest.mark.parametrize("head_dim", [64, 128])
+@pytest.mark.parametrize("n_ctx", [128, 256, 384, 1024])
+@pytest.mark.parametrize("causal", [True, False])
+def test_backward_with_groups_of_waves(gpu, causal, n_ctx, head_dim, monkeypatch):
+    # dQ groups + 16 * dK/dV groups: fewer blocks than groups, groups without any unmasked block, lengths that four groups
+    # do not divide; against the fp64 closed form with the tolerances of the plain form, and delta as the dQ kernel leaves it
+    from triton_amd import _lib
+    (q, k, v, do), (tq, tk, tv, tdo) = _inputs(23 + n_ctx, (1, 3, n_ctx, head_dim), "fp16", gpu)
+    cf = A.attn_closed_form(q, k, v, causal, 0.25, do)
+    I4 = _lib.I64x4
+    st = torch.cuda.current_stream().cuda_stream
+    o = torch.empty_like(tq)
+    M = torch.empty((1, 3, n_ctx), dtype=torch.float32, device=gpu)
+    assert _lib.load().mi355_attn_fwd(tq.data_ptr(), tk.data_ptr(), tv.data_ptr(), o.data_ptr(), M.data_ptr(), 1, 3, n_ctx, head_dim,
+                                      I4(*tq.stride()), I4(*tk.stride()), I4(*tv.stride()), I4(*o.stride()), 0.25, int(causal),
+                                      _lib.F16, st) == 0
+    want_delta = (o.double() * tdo.double()).sum(-1)
+    size = (o.double() * tdo.double()).abs().sum(-1)
+    for groups in (1 + 16, 2 + 32, 4 + 64):
+        set_knob(monkeypatch, "MI355_ATTN_BWD_GROUPS", str(groups))
+        dq, dk, dv = (torch.full_like(tq, 7.0) for _ in range(3))
+        delta = torch.full_like(M, 7.0)
+        assert _lib.load().mi355_attn_bwd_o(tq.data_ptr(), tk.data_ptr(), tv.data_ptr(), o.data_ptr(), tdo.data_ptr(), M.data_ptr(),
+                                            delta.data_ptr(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), 1, 3, n_ctx, head_dim,
+                                            I4(*tq.stride()), 0.25, int(causal), _lib.F16, st) == 0
+        # head_dim fp32 additions of terms that sum to `size`: each rounds by at most 2^-24 of it
+        assert torch.all((delta.double() - want_delta).abs() <= size * head_dim * 2.0 ** -24), groups
+        for name, t in (("dq", dq), ("dk", dk), ("dv", dv)):
+            assert np.allclose(to_np(t), cf[name], atol=1e-2, rtol=1e-2), (groups, name)

@@ -70,6 +70,9 @@ SIGNATURES = {
     "mi355_attn_bwd": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                                c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int,
                                POINTER(c_int64), c_float, c_int, c_int, c_void_p]),
+    "mi355_attn_bwd_o": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
+                                 c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int,
+                                 POINTER(c_int64), c_float, c_int, c_int, c_void_p]),
     "mi355_dequant": (c_int, [c_void_p, c_void_p, c_int64, c_int, c_void_p]),
     "mi355_clock_probe": (c_int, [c_void_p, c_int, c_void_p]),
     "mi355_mfma_burn": (c_int, [c_void_p, c_int, c_int, c_int, c_int, c_void_p]),

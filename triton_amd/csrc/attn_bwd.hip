@@ -1,5 +1,5 @@
 // Flash-attention backward for gfx950 (fp16 / bf16, head_dim 64, 128 or 256): delta = rowsum(O*dO),
-// then dK/dV with the K/V tile stationary and dQ with the Q tile stationary - the same
+// then dQ with the Q tile stationary and dK/dV with the K/V tile stationary - the same
 // atomics-free split as the reference (`_attn_bwd_preprocess`, `_attn_bwd_dkdv`, `_attn_bwd_dq`,
 // python/tutorials/06-fused-attention.py:190-204, :208-257, :261-305, driver :308-435), as
 // separate launches.
@@ -60,12 +60,22 @@ __global__ __launch_bounds__(256) void attn_bwd_pre_kernel(AttnArgs p) {
 // ---------------------------------------------------------------------------------------------
 // PAD (D = 64 only): p.d_real = 16 or 32 columns exist in memory; fragments loaded into registers are zero-filled,
 // the LDS tiles are zeroed once and only the chunks present are loaded, only the first d_real columns are stored.
-template <typename V8, int D, int QT, int NW, bool PAD = false>
+//
+// KW > 1: the waves are KW groups that share the workgroup's query rows and take every KW-th block of 64 keys each (a
+// step covers KW blocks); their sums meet in LDS at the end.  As in the forward, for launches with fewer blocks of rows
+// than CUs, which last as long as one wave's walk over the keys.  fp16, 16 heads x 1024 x 64 causal: 17.1 us in 128
+// workgroups, 12.1 in 256 of two groups (head_dim 128, backward as a whole: 51.7 -> 44.8).
+//
+// delta = rowsum(O * dO) is computed here when p.o is given (the dO fragments are in registers anyway) and written for
+// the dK/dV kernel: bf16 4 x 32 heads x 4096 x 128 causal, this kernel 866 -> 880 us and no pass of 48 us before it.
+template <typename V8, int D, int QT, int NW, bool PAD = false, int KW = 1>
 __global__ __launch_bounds__(NW * 64, 1) void attn_bwd_dq_kernel(AttnArgs p) {
   using S = typename ElemB<V8>::type;
   typedef __attribute__((ext_vector_type(4))) S S4;
-  constexpr int BM = NW * QT * 32, BN = 64, RB = D * 2, KSQ = D / 16, DT = D / 32;
-  using Tile = AttnTile<RB, BN, NW>;
+  constexpr int QW = NW / KW;          // waves along the query rows
+  static_assert(NW % KW == 0 && (KW == 1 || (QT == 1 && !PAD)), "whole groups of waves");
+  constexpr int BM = QW * QT * 32, BN = 64, RB = D * 2, KSQ = D / 16, DT = D / 32;
+  using Tile = AttnTile<RB, BN * KW, NW>;
   constexpr int TILE = Tile::BYTES;
 
   extern __shared__ __attribute__((aligned(1024))) char smem[];
@@ -81,7 +91,8 @@ __global__ __launch_bounds__(NW * 64, 1) void attn_bwd_dq_kernel(AttnArgs p) {
   int qb = pid % nqb;
   if (p.causal) qb = nqb - 1 - qb;
   const int z = hz / p.H, h = hz % p.H;
-  const int m0 = qb * BM, row0 = m0 + wave * QT * 32;
+  const int kw = KW == 1 ? 0 : wave / QW;   // which of a step's KW blocks of keys (wave-uniform)
+  const int m0 = qb * BM, row0 = m0 + (wave % QW) * QT * 32;
 
   const int64_t head_off = ((int64_t)z * p.sq[0] + (int64_t)h * p.sq[1]) * 2;
   const int64_t pitch = p.sq[2] * 2;
@@ -108,7 +119,24 @@ __global__ __launch_bounds__(NW * 64, 1) void attn_bwd_dq_kernel(AttnArgs p) {
       }
     }
     m_row[b] = p.lse[(int64_t)hz * p.N + r];
-    d_row[b] = p.delta[(int64_t)hz * p.N + r];
+    if (p.o == nullptr) {
+      d_row[b] = p.delta[(int64_t)hz * p.N + r];
+    } else {
+      const char* so = p.o + head_off + (int64_t)r * pitch + g * 16;
+      float sum = 0.f;
+#pragma unroll
+      for (int ks = 0; ks < KSQ; ks++) {
+        if (!PAD || ks * 32 + g * 16 < p.d_real * 2) {
+          const V8 of = *(const V8*)(so + ks * 32);
+          float part = 0.f;
+#pragma unroll
+          for (int e = 0; e < 8; e++) part = fmaf((float)of[e], (float)dof[b][ks][e], part);
+          sum += part;
+        }
+      }
+      d_row[b] = pair_sum(sum);
+      if (kw == 0 && g == 0 && row0 + b * 32 + l32 < p.N) const_cast<float*>(p.delta)[(int64_t)hz * p.N + r] = d_row[b];
+    }
   }
 
   // direct loads: scalar tile base + 32-bit lane offset (the host bounds the row pitch)
@@ -128,7 +156,7 @@ __global__ __launch_bounds__(NW * 64, 1) void attn_bwd_dq_kernel(AttnArgs p) {
   // work in a step) or one at a time between the MFMAs of the step before
   struct KvSrc { const char* k; const char* v; unsigned lds; };
   auto kv_src = [&](int j, int stage) {
-    const int64_t off = (int64_t)j * BN * pitch;
+    const int64_t off = (int64_t)j * (BN * KW) * pitch;
     return KvSrc{kbase + off, vbase + off, lds_base + stage * (2 * TILE)};
   };
   auto kv_load = [&](auto I_, const KvSrc& src) {
@@ -137,6 +165,13 @@ __global__ __launch_bounds__(NW * 64, 1) void attn_bwd_dq_kernel(AttnArgs p) {
       if constexpr ((I & 1) == 0) async_copy16_sbase(src.k, offKV[i], src.lds + (i * NW + wave) * 1024);
       else async_copy16_sbase(src.v, offKV[i], src.lds + TILE + (i * NW + wave) * 1024);
     }
+  };
+  constexpr int LPS = (2 * Tile::INST + 2 * KSQ - 1) / (2 * KSQ);   // loads per MFMA slot of phase 1
+  auto kv_loads = [&](auto SLOT_, const KvSrc& src) {
+    static_for<LPS>([&](auto O_) {
+      constexpr int i = decltype(SLOT_)::value * LPS + decltype(O_)::value;
+      if constexpr (i < 2 * Tile::INST) kv_load(std::integral_constant<int, i>{}, src);
+    });
   };
   auto issue_kv = [&](int j, int stage) {
     const KvSrc src = kv_src(j, stage);
@@ -150,15 +185,16 @@ __global__ __launch_bounds__(NW * 64, 1) void attn_bwd_dq_kernel(AttnArgs p) {
   // width computes its addresses per read.
   const RowRead<RB> rr(l32, g);
   const TrRead<RB> tt(i16, q4);
-  constexpr bool kPre = D <= 128;
+  // (128 keys of 256 bytes a step: the registers, but no immediates for the stage)
+  constexpr bool kPre = D <= 128, kStageImm = 4 * TILE <= 65536;
   unsigned ra[kPre ? KSQ : 1], ta[kPre ? DT : 1][2];
   if constexpr (kPre) {
 #pragma unroll
-    for (int ks = 0; ks < KSQ; ks++) ra[ks] = lds_base + rr.rowb + (rr.xk ^ (ks * 32));
+    for (int ks = 0; ks < KSQ; ks++) ra[ks] = lds_base + kw * (BN * RB) + rr.rowb + (rr.xk ^ (ks * 32));
 #pragma unroll
     for (int c = 0; c < DT; c++)
 #pragma unroll
-      for (int h2 = 0; h2 < 2; h2++) ta[c][h2] = lds_base + (tt.tl ^ ((c << 6) | (h2 << 5)));
+      for (int h2 = 0; h2 < 2; h2++) ta[c][h2] = lds_base + kw * (BN * RB) + (tt.tl ^ ((c << 6) | (h2 << 5)));
   }
 
   f32x16 dq[DT][QT];
@@ -171,9 +207,9 @@ __global__ __launch_bounds__(NW * 64, 1) void attn_bwd_dq_kernel(AttnArgs p) {
 
   const float qk_scale = p.sm_scale * 1.4426950408889634f;
   const int kv_end_blk = p.causal ? min(p.N, m0 + BM) : p.N;
-  const int nsteps = (kv_end_blk + BN - 1) / BN;
-  const int wave_last = p.causal ? (row0 + QT * 32 - 1) / BN : nsteps - 1;
-  const int wave_first_masked = p.causal ? row0 / BN : nsteps;
+  const int nsteps = (kv_end_blk + BN * KW - 1) / (BN * KW);
+  const int wave_last = p.causal ? (row0 + QT * 32 - 1) / BN : nsteps * KW - 1;  // last block with unmasked columns
+  const int wave_first_masked = p.causal ? row0 / BN : nsteps * KW;              // first block that needs the mask
 
   issue_kv(0, 0);
   wait_all();
@@ -194,16 +230,16 @@ __global__ __launch_bounds__(NW * 64, 1) void attn_bwd_dq_kernel(AttnArgs p) {
   auto step = [&](const int j, auto STAGE_, auto MASKED_) {
     constexpr int stage = decltype(STAGE_)::value;
     constexpr bool masked = decltype(MASKED_)::value;
-    constexpr int KOFF = kPre ? stage * 2 * TILE : 0, VOFF = KOFF + TILE;
-    const unsigned sbase = kPre ? 0u : lds_base + (unsigned)(stage * 2 * TILE);
+    constexpr int KOFF = kPre && kStageImm ? stage * 2 * TILE : 0, VOFF = KOFF + TILE;
+    const unsigned sbase = kPre && kStageImm ? 0u : (kPre ? 0u : lds_base) + (unsigned)(stage * 2 * TILE);
     auto row_addr = [&](auto KS_) {
       constexpr int ks = decltype(KS_)::value;
-      if constexpr (kPre) return ra[ks];
+      if constexpr (kPre) return kStageImm ? ra[ks] : ra[ks] + sbase;
       else return rr.template addr<ks>(sbase);
     };
     auto tr_addr = [&](auto C_, auto H_) {
       constexpr int c = decltype(C_)::value, h2 = decltype(H_)::value;
-      if constexpr (kPre) return ta[c][h2];
+      if constexpr (kPre) return kStageImm ? ta[c][h2] : ta[c][h2] + sbase;
       else return tt.template addr<c, h2>(sbase);
     };
     using I0 = std::integral_constant<int, 0>; using I1 = std::integral_constant<int, 1>;
@@ -228,7 +264,7 @@ __global__ __launch_bounds__(NW * 64, 1) void attn_bwd_dq_kernel(AttnArgs p) {
             else if constexpr (kind == 1) s[a][b][r] = fmaf(s[a][b][r], qk_scale, -m_row[b]);
             else if constexpr (kind == 2) s[a][b][r] = fast_exp2(s[a][b][r]);
             else if constexpr (kind == 3) {
-              const int kv = j * BN + a * 32 + (r >> 2) * 8 + g * 4 + (r & 3);
+              const int kv = (j * KW + kw) * BN + a * 32 + (r >> 2) * 8 + g * 4 + (r & 3);
               if (kv > row0 + b * 32 + l32) s[a][b][r] = 0.f;
             } else if constexpr (kind == 4) dp[a][b][r] *= s[a][b][r];
             else if constexpr (r < 8) {   // elements 2 r, 2 r + 1
@@ -276,7 +312,7 @@ __global__ __launch_bounds__(NW * 64, 1) void attn_bwd_dq_kernel(AttnArgs p) {
         for (int b = 0; b < QT; b++)
           s[a][b] = mfma32(__builtin_bit_cast(V8, kf[cur]), qf[b][ks], ks == 0 ? f32x16{} : s[a][b]);
         if constexpr (a == 0) {
-          if constexpr (!PAD && 2 * ks < 2 * Tile::INST) kv_load(std::integral_constant<int, 2 * ks < 2 * Tile::INST ? 2 * ks : 0>{}, nsrc);
+          if constexpr (!PAD) kv_loads(std::integral_constant<int, 2 * ks>{}, nsrc);
         } else {
           softmax_ops(I0{}, std::integral_constant<int, 2 * ks * XPS>{}, std::integral_constant<int, XPS>{});
         }
@@ -285,7 +321,7 @@ __global__ __launch_bounds__(NW * 64, 1) void attn_bwd_dq_kernel(AttnArgs p) {
         for (int b = 0; b < QT; b++)
           dp[a][b] = mfma32(__builtin_bit_cast(V8, vf[cur]), dof[b][ks], ks == 0 ? f32x16{} : dp[a][b]);
         if constexpr (a == 0) {
-          if constexpr (!PAD && 2 * ks + 1 < 2 * Tile::INST) kv_load(std::integral_constant<int, 2 * ks + 1 < 2 * Tile::INST ? 2 * ks + 1 : 0>{}, nsrc);
+          if constexpr (!PAD) kv_loads(std::integral_constant<int, 2 * ks + 1>{}, nsrc);
         } else {
           softmax_ops(I0{}, std::integral_constant<int, (2 * ks + 1) * XPS>{}, std::integral_constant<int, XPS>{});
           if constexpr (ks >= KSQ - 2) {
@@ -318,7 +354,7 @@ __global__ __launch_bounds__(NW * 64, 1) void attn_bwd_dq_kernel(AttnArgs p) {
     });
   };
   auto run = [&](const int j, auto STAGE_, auto MASKED_) {
-    if (j <= wave_last && row0 < p.N) step(j, STAGE_, MASKED_);
+    if (j * KW + kw <= wave_last && row0 < p.N) step(j, STAGE_, MASKED_);
     else issue_kv(min(j + 1, nsteps - 1), decltype(STAGE_)::value ^ 1);
     wait_all();
     __syncthreads();
@@ -328,7 +364,7 @@ __global__ __launch_bounds__(NW * 64, 1) void attn_bwd_dq_kernel(AttnArgs p) {
   // accumulators and copied all 64 of them back and forth at the join of every step.  (Every wave runs every
   // step's loads and barrier in either loop, so the waves of a workgroup may split at different steps.)
   using I0 = std::integral_constant<int, 0>; using I1 = std::integral_constant<int, 1>;
-  const int nplain = min(wave_first_masked, nsteps);
+  const int nplain = min((wave_first_masked - kw + KW - 1) / KW, nsteps);
   int j = 0;
   for (; j + 1 < nplain; j += 2) {
     run(j, I0{}, std::false_type{});
@@ -338,6 +374,28 @@ __global__ __launch_bounds__(NW * 64, 1) void attn_bwd_dq_kernel(AttnArgs p) {
   for (; j < nsteps; j++) {
     if (j & 1) run(j, I1{}, std::true_type{});
     else run(j, I0{}, std::true_type{});
+  }
+
+  if constexpr (KW > 1) {   // the groups' sums into the first group's waves (the K/V stages are free)
+    constexpr int PER = DT * 16;   // floats per lane
+    LDS_PTR(float) const part = (LDS_PTR(float))(lds + QW * 32 * RB);   // (behind the rows that the epilogue stages)
+    if (kw > 0) {
+      LDS_PTR(float) to = part + ((kw - 1) * QW + wave % QW) * (PER * 64) + lane;
+#pragma unroll
+      for (int c = 0; c < DT; c++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) to[(c * 16 + r) * 64] = dq[c][0][r];
+    }
+    __syncthreads();
+    if (kw > 0) return;
+#pragma unroll
+    for (int w = 1; w < KW; w++) {
+      LDS_PTR(float) from = part + ((w - 1) * QW + wave) * (PER * 64) + lane;
+#pragma unroll
+      for (int c = 0; c < DT; c++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) dq[c][0][r] += from[(c * 16 + r) * 64];
+    }
   }
 
   // dQ rows through this wave's share of the K/V stages (free: every step ends with a full wait and a barrier)
@@ -353,24 +411,31 @@ __global__ __launch_bounds__(NW * 64, 1) void attn_bwd_dq_kernel(AttnArgs p) {
   }
 }
 
+template <typename V8, int D, bool PAD = false, int KW = 1>
+static int launch_dq(const AttnArgs& p, hipStream_t stream) {
+  constexpr int QT = 1, NW = 4, BM = NW / KW * QT * 32;
+  constexpr int smem = 2 * 2 * 64 * KW * D * 2;
+  static bool attr_set = false;
+  if (!attr_set) {
+    hipError_t e = hipFuncSetAttribute((const void*)attn_bwd_dq_kernel<V8, D, QT, NW, PAD, KW>,
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, smem);
+    if (e != hipSuccess) return (int)e;
+    attr_set = true;
+  }
+  int nqb = (p.N + BM - 1) / BM;
+  attn_bwd_dq_kernel<V8, D, QT, NW, PAD, KW><<<dim3(nqb * p.Z * p.H), dim3(NW * 64), smem, stream>>>(p);
+  return (int)hipGetLastError();
+}
+
+// p.variant & 15: groups of waves along the keys (1, 2, or 4 at head_dim 64 with whole steps of 256 keys)
 template <typename V8, int D, bool PAD = false>
 static int launch_bwd_d(const AttnArgs& p, hipStream_t stream) {
-  {
-    constexpr int QT = 1, NW = 4, BM = NW * QT * 32;
-    constexpr int smem = 2 * 2 * 64 * D * 2;
-    static bool attr_set = false;
-    if (!attr_set) {
-      hipError_t e = hipFuncSetAttribute((const void*)attn_bwd_dq_kernel<V8, D, QT, NW, PAD>,
-                                         hipFuncAttributeMaxDynamicSharedMemorySize, smem);
-      if (e != hipSuccess) return (int)e;
-      attr_set = true;
-    }
-    int nqb = (p.N + BM - 1) / BM;
-    attn_bwd_dq_kernel<V8, D, QT, NW, PAD><<<dim3(nqb * p.Z * p.H), dim3(NW * 64), smem, stream>>>(p);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return (int)e;
+  if constexpr (!PAD && D <= 128) {
+    if constexpr (D == 64)
+      if ((p.variant & 15) == 4 && p.N % 256 == 0) return launch_dq<V8, D, PAD, 4>(p, stream);
+    if ((p.variant & 15) >= 2) return launch_dq<V8, D, PAD, 2>(p, stream);
   }
-  return 0;
+  return launch_dq<V8, D, PAD>(p, stream);
 }
 
 int attn_bwd_dkdv_launch(const AttnArgs& p, bool bf16, hipStream_t stream);  // attn_bwd_dkdv.hip

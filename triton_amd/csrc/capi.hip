@@ -53,7 +53,7 @@ const DeviceInfo& device_info() {
 constexpr int UNSET = INT_MIN;
 struct Knobs {
   int force_strided, group_m, tile, programs, skinny, grouped_big_min, grouped_wave128_min_k, grouped_chunk,
-      attn_fwd_variant, attn_programs, lean_epilogue, tile_m, rowfused_max_mk, mixed_rows, splitk;
+      attn_fwd_variant, attn_bwd_groups, attn_programs, lean_epilogue, tile_m, rowfused_max_mk, mixed_rows, splitk;
 };
 Knobs g_knobs;
 std::atomic<int> g_knobs_ready{0};
@@ -78,6 +78,7 @@ void load_knobs() {
   k.grouped_wave128_min_k = read_env("MI355_GROUPED_WAVE128_MIN_K", 0);
   k.grouped_chunk = read_env("MI355_GROUPED_CHUNK", 1);
   k.attn_fwd_variant = read_env("MI355_ATTN_FWD_VARIANT", 0);
+  k.attn_bwd_groups = read_env("MI355_ATTN_BWD_GROUPS", 0);   // dQ groups + 16 * dK/dV groups
   k.attn_programs = read_env("MI355_ATTN_PROGRAMS", 1);
   k.lean_epilogue = read_env("MI355_GEMM_LEAN_EPILOGUE", 0);
   k.tile_m = read_env("MI355_GEMM_TILE_M", 0);
@@ -1096,10 +1097,27 @@ int mi355_attn_bwd_preprocess(const void* o, const void* d_o, float* delta,
   return attn_bwd_pre_launch(p, dtype == MI355_BF16, (hipStream_t)stream_);
 }
 
-int mi355_attn_bwd(const void* q, const void* k, const void* v, const void* d_o,
-                   const float* Mlse, const float* delta, void* dq, void* dk, void* dv,
-                   int Z, int H, int N_CTX, int D, const int64_t* stride,
-                   float sm_scale, int causal, int dtype, void* stream_) {
+// Groups of waves of the backward kernels, dQ + 16 * dK/dV: more than one where the blocks of 128 rows leave CUs without
+// work, or under the mask where a few long walks end the launch.  In comments: the backward's us with one group each, and
+// what two (four) groups in dQ / in dK/dV change; fp16, causal.
+static int attn_bwd_variant(const AttnArgs& p, int cus) {
+  if (p.D == 256 || p.d_real < p.D) return 1 + 16;
+  const int64_t blocks = (int64_t)p.Z * p.H * p.N / 128;
+  // head_dim 64, 8 heads x 1024: 34.4, two -5.4 / -5.8, four -6.6 / -7.5; 16 x 1024: 35.2, four -2.3 / -2.2
+  if (p.D == 64 && p.N % 256 == 0 && blocks <= cus / 4) return 4 + 64;
+  // 16 x 1024: two -5.7 / -5.8; head_dim 128: 51.7, -6.9 / -8.2; 24 x 1024: 52.2, +1.1 / +0.3 (full 57.1, +8.1 / +7.6)
+  if (blocks <= cus / 2) return 2 + 32;
+  if (!p.causal || p.N < 2048) return 1 + 16;
+  // 8 x 4096: 114.9, -13.9 / -15.3; head_dim 128: 177.6, -14.9 / -16.4; 12 x 4096: 224.8, +9.0 / +6.9; full, 8 x 4096: +13 / +13
+  if (blocks <= cus) return 2 + 32;
+  // head_dim 64, 48 x 2048: 144.9, -7.0 / -0.2; 16 x 4096: 171.3, -16.7 / +7.7; 48 x 1024: 54.4, -2.0 / -0.5
+  return p.D == 64 && blocks <= 3ll * cus ? 2 + 16 : 1 + 16;
+}
+
+static int attn_bwd(const void* q, const void* k, const void* v, const void* o, const void* d_o,
+                    const float* Mlse, const float* delta, void* dq, void* dk, void* dv,
+                    int Z, int H, int N_CTX, int D, const int64_t* stride,
+                    float sm_scale, int causal, int dtype, void* stream_) {
   if (!q || !k || !v || !d_o || !Mlse || !delta || !dq || !dk || !dv) return MI355_EINVAL;
   AttnArgs p{};
   int rc = attn_common(p, Z, H, N_CTX, D, dtype);
@@ -1109,10 +1127,27 @@ int mi355_attn_bwd(const void* q, const void* k, const void* v, const void* d_o,
       !aligned(dq, 16) || !aligned(dk, 16) || !aligned(dv, 16) || !aligned(Mlse, 16) || !aligned(delta, 16))
     return MI355_ESTRIDE;
   p.q = (const char*)q; p.k = (const char*)k; p.v = (const char*)v; p.d_o = (const char*)d_o;
-  p.lse = const_cast<float*>(Mlse); p.delta = delta;
+  if (o && !aligned(o, 16)) return MI355_ESTRIDE;
+  p.o = (char*)const_cast<void*>(o); p.lse = const_cast<float*>(Mlse); p.delta = delta;
   p.dq = (char*)dq; p.dk = (char*)dk; p.dv = (char*)dv;
   p.sm_scale = sm_scale; p.causal = causal != 0;
+  p.variant = knob(knobs().attn_bwd_groups, attn_bwd_variant(p, device_info().cus > 0 ? device_info().cus : 256));
   return attn_bwd_launch(p, dtype == MI355_BF16, (hipStream_t)stream_);
+}
+
+int mi355_attn_bwd(const void* q, const void* k, const void* v, const void* d_o,
+                   const float* Mlse, const float* delta, void* dq, void* dk, void* dv,
+                   int Z, int H, int N_CTX, int D, const int64_t* stride,
+                   float sm_scale, int causal, int dtype, void* stream) {
+  return attn_bwd(q, k, v, nullptr, d_o, Mlse, delta, dq, dk, dv, Z, H, N_CTX, D, stride, sm_scale, causal, dtype, stream);
+}
+
+int mi355_attn_bwd_o(const void* q, const void* k, const void* v, const void* o, const void* d_o,
+                     const float* Mlse, float* delta, void* dq, void* dk, void* dv,
+                     int Z, int H, int N_CTX, int D, const int64_t* stride,
+                     float sm_scale, int causal, int dtype, void* stream) {
+  if (!o) return MI355_EINVAL;
+  return attn_bwd(q, k, v, o, d_o, Mlse, delta, dq, dk, dv, Z, H, N_CTX, D, stride, sm_scale, causal, dtype, stream);
 }
 
 }  // extern "C"

@@ -168,14 +168,14 @@ void attn_bwd(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, con
   on_device(q, 0); on_device(k, 1); on_device(v, 2); on_device(o, 3); on_device(d_o, 4); on_device(M, 5);
   on_device(delta, 6); on_device(dq, 7); on_device(dk, 8); on_device(dv, 9);
   const DeviceGuard guard(q.device());
-  int64_t s[4], so[4];
-  strides4(q, s); strides4(o, so);
+  int64_t s[4];
+  strides4(q, s);
+  TORCH_CHECK(o.strides() == q.strides() && d_o.strides() == q.strides(), "attention backward: q, o and do must have the same strides");
   const int Z = (int)q.size(0), H = (int)q.size(1), N = (int)q.size(2), D = (int)q.size(3);
   void* stream = stream_of(q);
-  int rc = mi355_attn_bwd_preprocess(o.data_ptr(), d_o.data_ptr(), delta.data_ptr<float>(), Z, H, N, D, so, abi_dtype(q), stream);
-  check(rc, "mi355_attn_bwd_preprocess");
-  rc = mi355_attn_bwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), d_o.data_ptr(), M.data_ptr<float>(), delta.data_ptr<float>(),
-                      dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), Z, H, N, D, s, (float)sm_scale, causal ? 1 : 0, abi_dtype(q), stream);
+  const int rc = mi355_attn_bwd_o(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), d_o.data_ptr(), M.data_ptr<float>(),
+                                  delta.data_ptr<float>(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), Z, H, N, D, s, (float)sm_scale,
+                                  causal ? 1 : 0, abi_dtype(q), stream);
   check(rc, "mi355_attn_bwd");
 }
 

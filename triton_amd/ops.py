@@ -430,12 +430,8 @@ class _attention(torch.autograd.Function):
             return dq, dk, dv, None, None
         I4 = _lib.I64x4
         lib = _lib.load()
-        rc = lib.mi355_attn_bwd_preprocess(
-            o.data_ptr(), do.data_ptr(), delta.data_ptr(), BATCH, N_HEAD, N_CTX, ctx.HEAD_DIM,
-            I4(*o.stride()), dt, _stream())
-        _lib.check(rc, "mi355_attn_bwd_preprocess")
-        rc = lib.mi355_attn_bwd(
-            q.data_ptr(), k.data_ptr(), v.data_ptr(), do.data_ptr(), M.data_ptr(), delta.data_ptr(),
+        rc = lib.mi355_attn_bwd_o(
+            q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), do.data_ptr(), M.data_ptr(), delta.data_ptr(),
             dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), BATCH, N_HEAD, N_CTX, ctx.HEAD_DIM,
             I4(*q.stride()), float(ctx.sm_scale), int(bool(ctx.causal)), dt, _stream())
         _lib.check(rc, "mi355_attn_bwd")
