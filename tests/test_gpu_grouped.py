@@ -133,3 +133,14 @@ def test_host_tables_and_device_tables_agree_bit_for_bit(gpu, nprog, dtype):
     rc = _lib.load().mi355_grouped_gemm(*(t.data_ptr() for t in tables), sizes.data_ptr(), lds.data_ptr(), len(shapes),
                                         _lib.F16 if dtype == "fp16" else _lib.BF16, nprog, torch.cuda.current_stream().cuda_stream)
     assert rc == 0 and all(torch.equal(c, d) for c, d in zip(outs, again))
+
+
+@pytest.mark.parametrize("extension", [True, False])
+def test_row_strides_beyond_32_bits_are_refused(gpu, extension, monkeypatch):
+    from triton_amd import _lib
+
+    if not extension:
+        monkeypatch.setattr(_lib, "ext", lambda: None)
+    row = torch.zeros(8, device=gpu, dtype=torch.float16).as_strided((1, 8), ((1 << 32) + 8, 1))
+    with pytest.raises(RuntimeError):
+        triton_amd.group_gemm_fn([row], [torch.zeros(8, 8, device=gpu, dtype=torch.float16)])

@@ -137,6 +137,7 @@ std::vector<at::Tensor> group_gemm(const std::vector<at::Tensor>& a, const std::
     int32_t *s = &sizes[3 * used], *l = &lds[3 * used];
     s[0] = (int32_t)a[i].size(0); s[1] = (int32_t)b[i].size(1); s[2] = (int32_t)a[i].size(1);
     // (a matrix of one row may have any row stride)
+    TORCH_CHECK(std::max({a[i].size(0), a[i].stride(0), b[i].size(0), b[i].size(1), b[i].stride(0)}) <= INT32_MAX, "sizes and row strides of a group's matrices are 32-bit");
     l[0] = (int32_t)(s[0] == 1 ? std::max<int64_t>(a[i].stride(0), s[2]) : a[i].stride(0));
     l[1] = (int32_t)(s[2] == 1 ? std::max<int64_t>(b[i].stride(0), s[1]) : b[i].stride(0));
     l[2] = s[1];

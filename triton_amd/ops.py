@@ -311,6 +311,8 @@ def group_gemm_fn(group_A, group_B, *, num_programs: int = 0):
     live = [i for i, C in enumerate(group_C) if C.numel() > 0 and group_A[i].shape[1] > 0]
     for C in (group_C[i] for i in range(group_size) if i not in live):
         C.zero_()
+    if any(max(*t.shape, t.stride(0)) >= 1 << 31 for i in live for t in (group_A[i], group_B[i])):
+        raise RuntimeError("sizes and row strides of a group's matrices are 32-bit")
     addresses = lambda group: (ctypes.c_void_p * len(live))(*(group[i].data_ptr() for i in live))   # noqa: E731
     sizes = (ctypes.c_int32 * (3 * len(live)))(*(v for i in live for v in (*group_C[i].shape, group_A[i].shape[1])))
     # (a matrix of one row may have any row stride)
