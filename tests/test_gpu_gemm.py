@@ -1414,3 +1414,19 @@ def test_rows_that_do_not_start_on_16_byte_boundaries_are_exact(gpu, dtype, K):
             for tb in (tensor(b), tensor(np.ascontiguousarray(b.T)).t(), wide[:, 1:1 + N]):
                 got = to_np(triton_amd.matmul(ta, tb, out_dtype=torch.float32))
                 assert bits_equal(got, ref), (M, N, K, tb.stride(), ta.data_ptr() % 16)
+
+
+@pytest.mark.parametrize("kmajor", [False, True])
+@pytest.mark.parametrize("M,N,K", [(4096, 4097, 1032), (4096, 4160, 1024), (4160, 4096, 1024), (4097, 4095, 1024), (4096, 4161, 1024)])
+def test_columns_or_rows_beyond_whole_tiles_in_a_call_of_their_own(gpu, M, N, K, kmajor):
+    # 1 .. 64 columns (rows) beyond a round of 256-column tiles run as a second call, 65 do not; the addend moves along with them.
+    # Whole numbers below 2^11: every sum and its fp32 output are exact
+    g = torch.Generator(device=gpu).manual_seed(M + N + K)
+    a = torch.randint(-1, 2, (M, K), device=gpu, generator=g).to(torch.bfloat16)
+    b = torch.randint(-1, 2, (N, K), device=gpu, generator=g).to(torch.bfloat16).t()
+    b = b if kmajor else b.contiguous()
+    want = a.float() @ b.float()
+    assert torch.equal(triton_amd.matmul(a, b, out_dtype=torch.float32), want)
+    for shape in ((N,), (M, 1), (M, N)):
+        add = torch.randint(-8, 9, shape, device=gpu, generator=g).to(torch.bfloat16)
+        assert torch.equal(triton_amd.matmul(a, b, out_dtype=torch.float32, add=add), want + add.float()), shape

@@ -460,6 +460,32 @@ static int gemm_impl(const void* A, const void* B, void* C, int M, int N, int K,
       double other = tiles256_us((long)((M + rows - 1) / rows) * ((N + 255) / 256), rows, ksteps128, cus, tile != 6, is8);
       if (mixed_rows > 0) other *= 0.9;   // (two tile heights in one launch are chosen where they gain at least 5 %)
       if (plan.us < other) ring = plan.shape;
+      // Up to 64 columns (or rows) beyond whole 256-column tiles: those in a call of their own where they would cost the tiles
+      // another round of CUs.  bf16, us of a call, in one / in two parts, row-major B (K-major): 4100 x 4096 x 4096 135 / 99
+      // (129 / 93), 4096 x 4128 x 4096 145 / 105 (125 / 95), 2050 x 8192 x 4096 136 / 101, 8192 x 8200 x 2048 243 / 207, 4096 x 4160 x 1024
+      // 50 / 38; edges on the other side too: 4095 x 4100 x 4100 168 / 151.  No round saved, one part: 2048 x 2052 x 4096, 6150 x 6144 x 4096.
+      const double one = std::min(plan.us, other);
+      auto parts_us = [&](int m, int n, int m2, int n2) {
+        const bool edges = m % 256 != 0 || n % 256 != 0 || p.k_bytes % 128 != 0;
+        const long tiles = (long)((m + 255) / 256) * ((n + 255) / 256);
+        return std::min(ring_plan(m, n, ksteps128, cus, 1, 1).us, tiles256_us(tiles, 256, ksteps128, cus, edges, is8)) +
+               ring_plan(m2, n2, ksteps128, cus, 1, 1).us;
+      };
+      const int rn = N % 256, rm = M % 256;
+      const double cut_n = rn > 0 && rn <= 64 && N > 256 ? parts_us(M, N - rn, M, rn) : 1e30;
+      const double cut_m = rm > 0 && rm <= 64 && M > 256 ? parts_us(M - rm, N, rm, N) : 1e30;
+      if (!workspace && std::min(cut_n, cut_m) < 0.9 * one) {
+        const bool rows = cut_m < cut_n;
+        const int m = rows ? M - rm : M, n = rows ? N : N - rn;
+        const int64_t dm = rows ? m : 0, dn = rows ? 0 : n;
+        const int rc = gemm_impl(A, B, C, m, n, K, sam, sak, sbk, sbn, scm, scn, in_dtype, out_dtype, a_scale, b_scale, activation,
+                                 aux, aux_sm, aux_sn, aux_dtype, -1, group_m_arg, stream_);
+        if (rc) return rc;
+        return gemm_impl((const char*)A + dm * sam * es, (const char*)B + dn * sbn * es, (char*)C + (dm * scm + dn * scn) * elem_size(out_dtype),
+                         M - (int)dm, N - (int)dn, K, sam, sak, sbk, sbn, scm, scn, in_dtype, out_dtype, a_scale, b_scale, activation,
+                         aux ? (const char*)aux + (dm * aux_sm + dn * aux_sn) * elem_size(aux_dtype) : nullptr, aux_sm, aux_sn, aux_dtype,
+                         -1, group_m_arg, stream_);
+      }
     }
   }
   if (ring >= 0)
