@@ -1416,6 +1416,25 @@ def test_rows_that_do_not_start_on_16_byte_boundaries_are_exact(gpu, dtype, K):
                 assert bits_equal(got, ref), (M, N, K, tb.stride(), ta.data_ptr() % 16)
 
 
+@pytest.mark.parametrize("dtype", ["fp16", "bf16"])
+@pytest.mark.parametrize("M,N,K,splits", [(512, 1024, 1017, 0), (512, 1024, 1020, 0), (512, 1024, 1023, 0), (512, 1024, 1025, 0),
+                                          (256, 256, 4089, 8), (256, 256, 4092, 8), (256, 256, 4095, 8), (256, 256, 4033, 8)])
+def test_rows_behind_a_row_major_b_stay_out_of_the_product(gpu, dtype, M, N, K, splits):
+    # only A's rows are copied, K rounded up to whole 16-byte chunks; B is used in place and ends inside the last K step:
+    # K mod 64 = 57, 60, 63 (the rounded K is whole steps) and 1 (a tail).  B is the first K rows of a matrix whose other
+    # rows are NaN.  Sums of small integers below 2^24: every bit of the fp32 result is determined
+    padded = (K + 7) // 8 * 8
+    copy = (2 * padded + 127) // 128 * 128 * M
+    need = _lib.load().mi355_gemm_workspace(1 << 20, 1 << 21, M, N, K, K, 1, N, 1, _lib.F16 if dtype == "fp16" else _lib.BF16)
+    assert need == copy + splits * 4 * M * N   # the copy of A and the slices of K, no copy of B
+    rng = np.random.default_rng(K)
+    a = rng.integers(-2, 3, size=(M, K)).astype(np.float32)
+    tall = np.full((K + 64, N), np.nan, np.float32)
+    tall[:K] = rng.integers(-2, 3, size=(K, N))
+    got = triton_amd.matmul(from_np(a, dtype, gpu), from_np(tall, dtype, gpu)[:K], out_dtype=torch.float32)
+    assert bits_equal(to_np(got), a @ tall[:K])
+
+
 @pytest.mark.parametrize("kmajor", [False, True])
 @pytest.mark.parametrize("M,N,K", [(4096, 4097, 1032), (4096, 4160, 1024), (4160, 4096, 1024), (4097, 4095, 1024), (4096, 4161, 1024)])
 def test_columns_or_rows_beyond_whole_tiles_in_a_call_of_their_own(gpu, M, N, K, kmajor):

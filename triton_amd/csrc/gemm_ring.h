@@ -16,7 +16,7 @@
 // barriers alone 20.3 us, with the fragment reads 25.5, with the loads 26.6, all 31.6 - the tiles' 537 MB from L2 at 19 TB/s
 // are the longest part; eight waves of half a tile each, or a ring twice as deep, change nothing.
 //
-// K tail (K bytes not a multiple of 128): multiplied FIRST, as step 0, from registers through LDS with zeros beyond K -
+// K tail (K bytes not a multiple of 128, or a last step that B's rows end inside): multiplied FIRST, as step 0, from registers through LDS with zeros beyond K -
 // its loads are the oldest of the prologue, so the ring fills behind them and the tail costs one ordinary step.
 #pragma once
 #include "common.h"
@@ -236,8 +236,10 @@ __device__ __forceinline__ void gemm_ring_tile(const GemmArgs& p, const int pm, 
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int wm = wave / WN, wn = wave % WN;
   const int m0 = pm * BM, n0 = pn * BN;
-  const int tail = p.k_bytes % RING_ROW;
-  const int steps = p.k_bytes / RING_ROW + (tail ? 1 : 0);
+  // (a step that a row-major B ends inside is a tail too, a whole one where A's padding fills it: B has no rows to load there)
+  const int rest = p.k_bytes % RING_ROW;
+  const int tail = !B_KMAJOR && rest == 0 && p.K * E::kElemBytes < p.k_bytes ? RING_ROW : rest;
+  const int steps = (p.k_bytes + RING_ROW - 1) / RING_ROW;
   constexpr int KROWS = RING_ROW / 2;                        // k rows of a row-major B per step
 
   auto scalar_ptr = [](const char* x) {   // (wave-uniform, but possibly read from device tables)
