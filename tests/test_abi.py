@@ -56,6 +56,20 @@ def test_strerror_and_argument_rejection_without_gpu():
     assert lib.mi355_query(12345) == -1
 
 
+def test_products_with_rows_too_far_apart_for_the_tile_kernels_copy_them():
+    # rows of B 64 MiB apart (row major) or 8 MiB (K major) are beyond the kernels' lane offsets: a B that would otherwise
+    # stay in place beside the copy of an unaligned A is copied too, as only those kernels know that its rows end before A's padding
+    lib = _lib.load()
+
+    def need(sbk, sbn, K=73, b=1 << 21):
+        return lib.mi355_gemm_workspace(1 << 20, b, 2048, 2048, K, K, 1, sbk, sbn, _lib.BF16)
+    a_copy = 256 * 2048
+    assert need(2048, 1) == need((1 << 25) - 8, 1) == a_copy
+    assert need(1 << 25, 1) == a_copy + 4096 * 128            # (B's copy has the rows of zeros beyond K)
+    assert need(1 << 40, 1) == a_copy + 4096 * 128
+    assert need(1, 1 << 22) == need(1, 80) == 2 * a_copy      # (a K-major B is always copied here: its rows are not whole chunks)
+
+
 def test_matmul_preconditions_match_reference_messages():
     a = torch.zeros(4, 8, dtype=torch.float16)
     b = torch.zeros(6, 4, dtype=torch.float16)

@@ -1435,6 +1435,19 @@ def test_rows_behind_a_row_major_b_stay_out_of_the_product(gpu, dtype, M, N, K, 
     assert bits_equal(to_np(got), a @ tall[:K])
 
 
+def test_rows_too_far_apart_for_the_tile_kernels(gpu):
+    # rows of B 64 MiB apart, behind the last one NaN; K = 73 gets padded for A (exact sums as above)
+    M = N = 2048
+    K, pitch = 73, 1 << 25
+    rng = np.random.default_rng(0)
+    a = rng.integers(-2, 3, size=(M, K)).astype(np.float32)
+    b = rng.integers(-2, 3, size=(K, N)).astype(np.float32)
+    rows = torch.empty(K + 7, pitch, dtype=torch.bfloat16, device=gpu)[:, :N]
+    rows[:K] = from_np(b, "bf16", gpu)
+    rows[K:] = float("nan")
+    assert bits_equal(to_np(triton_amd.matmul(from_np(a, "bf16", gpu), rows[:K], out_dtype=torch.float32)), a @ b)
+
+
 @pytest.mark.parametrize("kmajor", [False, True])
 @pytest.mark.parametrize("M,N,K", [(4096, 4097, 1032), (4096, 4160, 1024), (4160, 4096, 1024), (4097, 4095, 1024), (4096, 4161, 1024)])
 def test_columns_or_rows_beyond_whole_tiles_in_a_call_of_their_own(gpu, M, N, K, kmajor):

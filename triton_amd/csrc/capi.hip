@@ -290,6 +290,7 @@ static int gemm_impl(const void* A, const void* B, void* C, int M, int N, int K,
   const bool pitch_ok = (int64_t)sam * es < (1 << 23) && (b_kmajor ? (int64_t)sbn * es < (1 << 23) : (int64_t)sbk * es < (1 << 26));
   const bool fast = pitch_ok && out_ok && a_ok && (b_kmajor || b_nmajor) && knob(knobs().force_strided, 0) == 0;
 
+  if (!fast && k_rows > 0) K = k_rows;   // (the kernels of any stride have no use for A's padding, and B ends before it)
   if (!fast && is32) {
     GemmStridedArgs s{A, B, C, M, N, K, sam, sak, sbk, sbn, scm, scn, a_scale, b_scale, activation, in_dtype, out_dtype,
                       aux, aux_sm, aux_sn, aux_dtype};
@@ -625,15 +626,17 @@ GemmRoute gemm_route(const void* A, const void* B, int M, int N, int K, int64_t 
   if (es == 4 || sak != 1 || sam < K || (sbk == 1) == (sbn == 1)) return r;
   r.kmajor = sbk == 1;
   if (r.kmajor ? sbn < K : sbk < N) return r;
-  const bool b_ok = r.kmajor ? bk_ok : bn_ok;
+  // (what stays in place has rows within the kernels' lane offsets, as in gemm_impl: only their kernels know k_rows)
+  const int64_t a_most = 1 << 23, b_most = r.kmajor ? 1 << 23 : 1 << 26;
+  const bool a_stays = a_ok && sam * es < a_most, b_stays = r.kmajor ? bk_ok && sbn * es < b_most : bn_ok && sbk * es < b_most;
   // us: the copies at about 4.5 TB/s of reads and writes, then the best kernel
   auto copy_us = [&](bool a, bool b) { return 2.0 + 2.0 * es * ((a ? (double)M * K : 0.0) + (b ? (double)N * K : 0.0)) / 4.5e6; };
   const int steps = (int)(((int64_t)K * es + 127) / 128);
   const double ring = ring_ok(es, r.kmajor) ? ring_plan(M, N, steps, cus, 1, 1).us : 1e30;
   const double any = std::min(ring, tiles256_us((long)((M + 255) / 256) * ((N + 255) / 256), 256, steps, cus, true, es == 1));
-  r.pack_a = !a_ok;
+  r.pack_a = !a_stays;
   // a row-major B with good rows only lacks the zero rows beyond K, which the ring kernels do not read
-  r.pack_b = !b_ok || (!r.kmajor && K % vec != 0 && ring + copy_us(!a_ok, false) > any + copy_us(!a_ok, true));
+  r.pack_b = !b_stays || (!r.kmajor && K % vec != 0 && ring + copy_us(!a_stays, false) > any + copy_us(!a_stays, true));
   const double packed = copy_us(r.pack_a, r.pack_b) + (r.pack_b || r.kmajor || K % vec == 0 ? any : ring);
   // (any-stride kernel: 64x64 tiles, about 1.3 us per 64 k: 1024 x 1024 x 1000 bf16 23 us, x 4100 107)
   const long tiles = (long)((M + 63) / 64) * ((N + 63) / 64);
@@ -655,7 +658,7 @@ GemmRoute gemm_route(const void* A, const void* B, int M, int N, int K, int64_t 
     r.b_pitch = (int64_t)(r.kmajor ? up((size_t)r.k * es, 128) : up((size_t)N * es, 512));
     r.b_bytes = up((size_t)r.b_pitch * r.b_rows, 256);
   }
-  if (r.a_pitch >= (1 << 23) || r.b_pitch >= (r.kmajor ? 1 << 23 : 1 << 26)) {   // (beyond the kernels' lane offsets)
+  if (r.a_pitch >= a_most || r.b_pitch >= b_most) {   // (beyond the kernels' lane offsets)
     GemmRoute plain;
     plain.k = K;
     return plain;
