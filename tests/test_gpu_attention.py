@@ -298,6 +298,35 @@ def test_forward_with_groups_of_waves_along_the_keys(gpu, causal, n_ctx, head_di
 
 
 @pytest.mark.parametrize("head_dim", [64, 128])
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("key", [float("-inf"), -65504.0])
+def test_forward_with_keys_masked_through_their_scores(gpu, key, causal, head_dim, monkeypatch):
+    # whole blocks of 64 keys whose scores are -inf (or the lowest that fp16 keys give), among them the first block of the
+    # second, third and fourth group of waves: weight 0, as in the forms without groups (2, 4); block 0 keeps some keys
+    from triton_amd import _lib
+    n_ctx = 512
+    (q, k, v, _), _ = _inputs(5, (1, 3, n_ctx, head_dim), "fp16", gpu)
+    q[..., 0] = 1.0
+    for block in (1, 2, 3, 5, 7):
+        k[:, :, block * 64:block * 64 + 64, 0] = key
+    k[:, :, 32:64, 0] = key
+    k[:, 1, 256:320, 0] = key     # (one head: nothing left behind block 0 but block 6)
+    cf = A.attn_closed_form(q, k, v, causal, 0.25)
+    assert np.isfinite(cf["o"]).all()
+    tq, tk, tv = (from_np(x, "fp16", gpu) for x in (q, k, v))
+    I4 = _lib.I64x4
+    for variant in ("2", "4", "6", "7", "8"):
+        set_knob(monkeypatch, "MI355_ATTN_FWD_VARIANT", variant)
+        o = torch.full_like(tq, 7.0)
+        M = torch.full((1, 3, n_ctx), 7.0, dtype=torch.float32, device=gpu)
+        assert _lib.load().mi355_attn_fwd(tq.data_ptr(), tk.data_ptr(), tv.data_ptr(), o.data_ptr(), M.data_ptr(), 1, 3, n_ctx, head_dim,
+                                          I4(*tq.stride()), I4(*tk.stride()), I4(*tv.stride()), I4(*o.stride()),
+                                          0.25, int(causal), _lib.F16, torch.cuda.current_stream().cuda_stream) == 0
+        assert np.allclose(to_np(M), cf["M"], atol=2e-3, rtol=0), variant
+        assert np.allclose(to_np(o), cf["o"], atol=1e-2, rtol=1e-2), variant
+
+
+@pytest.mark.parametrize("head_dim", [64, 128])
 @pytest.mark.parametrize("n_ctx", [128, 256, 384, 1024])
 @pytest.mark.parametrize("causal", [True, False])
 def test_backward_with_groups_of_waves(gpu, causal, n_ctx, head_dim, monkeypatch):

@@ -156,6 +156,11 @@ __global__ __launch_bounds__(NW * 64, 1) void attn_fwd_kernel(AttnArgs p) {
   // so P stays below 2^RESCALE_LOG2 and the result O = acc / l, M = m + log2(l) is unchanged.
   constexpr float RESCALE_LOG2 = 8.f;
 
+  // What is subtracted from a row's scores for the maximum m.  A group behind the first can meet keys whose scores are all
+  // -inf before any other: they get 0 there as behind a finite maximum, not exp2(-inf + inf).  (Such a first block of a row
+  // makes it NaN in every form.)
+  auto subtracted = [&](float m) { return KW > 1 && kw > 0 && m == -INFINITY ? 0.f : m; };
+
   // number of K/V steps of this block / wave
   const int kv_end_blk = p.causal ? min(p.N, m0 + BM) : p.N;
   const int nsteps = (kv_end_blk + BN * KW - 1) / (BN * KW);
@@ -248,7 +253,7 @@ __global__ __launch_bounds__(NW * 64, 1) void attn_fwd_kernel(AttnArgs p) {
         mx = pair_max(mx);
         const float m_new = fmaxf(m_i[b], mx * qk_scale);
         if (__builtin_amdgcn_ballot_w64(m_new > m_i[b] + RESCALE_LOG2) != 0) {
-          const float alpha = fast_exp2(m_i[b] - m_new);
+          const float alpha = fast_exp2(m_i[b] - subtracted(m_new));
           l_i[b] *= alpha;
           m_i[b] = m_new;
 #pragma unroll
@@ -256,7 +261,7 @@ __global__ __launch_bounds__(NW * 64, 1) void attn_fwd_kernel(AttnArgs p) {
 #pragma unroll
             for (int r = 0; r < 16; r++) oacc[c][b][r] *= alpha;
         }
-        const float m_cur = m_i[b];
+        const float m_cur = subtracted(m_i[b]);
         float rs = 0.f;
 #pragma unroll
         for (int a = 0; a < 2; a++)
@@ -320,7 +325,7 @@ __global__ __launch_bounds__(NW * 64, 1) void attn_fwd_kernel(AttnArgs p) {
     }
     __syncthreads();
     if (kw > 0) return;
-    float top = m_i[0];   // (finite: the first group has the first key)
+    float top = m_i[0];   // (the first group has the first key: where it is -inf, the group's sum is NaN and the row with it)
 #pragma unroll
     for (int w = 1; w < KW; w++) top = fmaxf(top, part[((w - 1) * QW + wave) * (PER * 64) + (PER - 2) * 64 + lane]);
     const float own = fast_exp2(m_i[0] - top);
