@@ -666,6 +666,34 @@ def test_skinny_16bit_kernel_is_bit_exact_on_integers(gpu, monkeypatch, dtype, s
             assert bits_equal(to_np(triton_amd.matmul(t8a, t8b, out_dtype=torch.float32)), ref), (fmt, shape)
 
 
+@pytest.mark.parametrize("dtype", ["fp16", "bf16", "e4m3"])
+@pytest.mark.parametrize("forced", [False, True])
+@pytest.mark.parametrize("M,N,K", [(33, 64, 4096), (48, 96, 96), (49, 96, 96), (49, 2048, 4160), (64, 64, 8192), (64, 32, 64),
+                                   (2048, 64, 4096), (96, 33, 4096), (160, 50, 192), (40, 64, 16384), (1, 1000, 256), (4, 33, 2048)])
+def test_streaming_kernel_up_to_64_rows_is_bit_exact(gpu, monkeypatch, dtype, forced, M, N, K):
+    # 33 .. 64 rows of A or columns of B next to a K-contiguous long operand, by the size rule and wherever the streaming
+    # kernel can run (MI355_GEMM_SKINNY=1): K bytes of whole lines and of an odd number of 64-byte pieces, more and at most 48
+    # rows, waves without a share of K; fp8 with up to four rows and columns that are not blocks of 32.  K is not split
+    # (MI355_GEMM_SPLITK=0).  Exact integer sums
+    set_knob(monkeypatch, "MI355_GEMM_SPLITK", "0")
+    if forced:
+        set_knob(monkeypatch, "MI355_GEMM_SKINNY", "1")
+    rng = np.random.default_rng(M + 3 * N + 7 * K)
+    a = rng.integers(-2, 3, size=(M, K)).astype(np.float32)
+    b = rng.integers(-2, 3, size=(K, N)).astype(np.float32)
+    z = rng.integers(-4, 5, size=(M, N)).astype(np.float32)
+    if dtype == "e4m3":
+        put = lambda x: torch.from_numpy(formats.encode_fp8(np.ascontiguousarray(x), dtype)).to(gpu).view(torch.float8_e4m3fn)   # noqa: E731
+    else:
+        put = lambda x: from_np(x, dtype, gpu)   # noqa: E731
+    ta = put(a)
+    for tb in (put(b), put(b.T).t()):
+        assert bits_equal(to_np(triton_amd.matmul(ta, tb, out_dtype=torch.float32)), a @ b), tb.stride()
+        got = triton_amd.matmul(ta, tb, "leaky_relu", out_dtype=torch.float32, add=torch.from_numpy(z).to(gpu))
+        want = a @ b + z
+        assert bits_equal(to_np(got), np.where(want >= 0, want, want * np.float32(0.01))), tb.stride()
+
+
 @pytest.mark.parametrize("dtype", ["fp16", "bf16"])
 def test_skinny_16bit_decode_shapes_against_closed_form(gpu, dtype):
     # M = 16 and 64 against N = K = 4096, and the transposed 4096 x 64: random data, output in the

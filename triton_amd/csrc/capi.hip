@@ -182,33 +182,64 @@ double tiles256_us(long tiles, int rows, int steps, int cus, bool edges, bool fp
 // of B, fp8 with a K-major one.
 bool ring_ok(int elem_bytes, bool b_kmajor) { return elem_bytes == 2 || (elem_bytes == 1 && b_kmajor); }
 
-// The streaming kernel of at most 32 rows on a side (gemm_skinny.hip: a workgroup per 32 rows of the other one, K split over
-// its four waves): 0.3 us per 128 bytes of a wave's share (0.5 where it transposes a row-major operand), or what that access
-// pattern gets from memory.  Ahead of the ring kernels where both sides are short (fp16 16 x 2048 x 2048 5.5 against 7.4 us) and
-// for fp8 (16 x 8192 x 8192 13.0 / 13.1, 16 x 2048 x 2048 4.7 / 5.0); behind them on long 16-bit weights (16 x 8192 x 8192 row
-// major 43 / 31, K-major 36 / 33, 16 x 1024 x 8192 23 / 11) and from 33 rows on (64 x 8192 x 8192 49 / 35).
-double skinny_us(int M, int N, int64_t k_bytes, int elem_bytes, bool b_kmajor) {
-  if (std::min(M, N) > 32) return 1e30;
-  const bool transposes = !b_kmajor;
-  const double bytes = (double)k_bytes * std::max(M, N);
-  return kLaunchUs + std::max((double)k_bytes / 512 * (transposes ? 0.5 : 0.3), bytes / (elem_bytes == 1 ? 7e6 : transposes ? 3.4e6 : 4.2e6));
+// Whether the streaming kernel (gemm_skinny.hip: a workgroup per 32 rows of the long operand, K split over its four waves)
+// takes a product of at most 64 rows on a side ahead of the ring kernels.  Measured over rows 1 .. 64, long sides of 1024 ..
+// 32768, K of 512 .. 16384, fp16 and e4m3, all layouts, weights from memory and from cache; ring / streaming, us:
+//   * a K-contiguous long operand: as long as its workgroups are one round of CUs (16 x 8192 x 2048 fp16 12.0 / 10.0, 16 x
+//     12288 x 2048 12 / 16.5), from 2048 bytes of K on (16 x 4096 x 512 fp16 4.6 / 4.6; below, the ring up to 15 % ahead) - for
+//     the columns of C with any K (4096 x 16 x 512 e4m3 even, x 1024 1.07 times as long in the ring).  33 .. 40 rows: from 8192
+//     bytes of K on (33 x 2048 x 8192 fp16 33.3 / 29.9, e4m3 18.9 / 17.6; x 4096 e4m3 even; 48 rows: ring 34.7 / 36.5); 49 .. 64
+//     rows of 16 bits, whose own form moves whole lines: the same (64 x 2048 x 8192 37.0 / 30.6, 8192 x 64 x 8192 42.4 / 38.1, x 2048
+//     even - with the weight in memory; from cache the ring is up to 30 % ahead there), fp8: ring (64 x 4096 x 8192 0.88)
+//   * a row-major long operand: up to 32 rows, three quarters of a round (16 x 2048 x 2048 fp16 8.1 / 6.3 from cache, even from
+//     memory; 16 x 8192 x 8192 39 / 43)
+bool streams(int M, int N, int64_t k_bytes, int elem_bytes, bool b_kmajor, int cus) {
+  const bool cols = M > 64;
+  const int S = cols ? N : M, L = cols ? M : N;
+  const bool y_kmajor = cols || b_kmajor;
+  if (!gemm_skinny_sizes_ok(S, L, k_bytes, y_kmajor, cols ? b_kmajor : true, elem_bytes)) return false;
+  if (!y_kmajor) return L <= 24 * cus;
+  if (L > 32 * cus) return false;
+  if (S <= 32) return cols || k_bytes >= 2048;
+  return k_bytes >= 8192 && (S <= 40 || (elem_bytes == 2 && S > 48));
+}
+
+// fp8 and up to four rows against a long side that is not whole blocks of 32: the kernel that streams straight into registers
+// (gemm8.hip; 1 x 2056 x 2048 5.4 / 5.0, 1 x 1000 x 4096 7.6 / 7.2, 8 x 2056 x 2048 even, 16 x 8200 x 2048 the ring 15 % ahead)
+bool streams8(int M, int N, int64_t k_bytes, int elem_bytes, bool b_kmajor, int cus) {
+  return elem_bytes == 1 && b_kmajor && M <= 4 && N % 32 != 0 && N <= 32 * cus && k_bytes % 256 == 0;
+}
+
+// us of a product that `streams` says yes to: within 15 % with K-contiguous operands, 30 % with a row-major long one (a weight
+// from cache that much faster, from memory slower)
+double stream_us(int M, int N, int64_t k_bytes, bool b_kmajor, int cus) {
+  const double steps = (double)k_bytes / 128, fill = (double)std::max(M, N) / (32.0 * cus);
+  if (M <= 64 && !b_kmajor) return 2.5 + steps * std::max(0.2, 0.33 * fill);
+  const int rows = std::min(M, N);
+  if (rows > 32) return 5.0 + steps * std::max(0.17, 0.24 * fill);
+  return 3.5 + steps * (rows > 16 ? std::max(0.136, 0.21 * fill) : std::max(0.105, 0.18 * fill));
 }
 
 // Splits of K that `mi355_gemm_splitk` takes by itself (1 = the plain call).
 int auto_splits(int M, int N, int64_t k_bytes, int in_dtype, bool b_kmajor, bool ring, int cus) {
   if (ring) {
     const int steps = (int)((k_bytes + 127) / 128);
-    const int most = (int)std::min<int64_t>(std::min<int64_t>(32, steps / 2), (64ll << 20) / std::max<int64_t>(1, 4ll * M * N));   // 64 MiB of partial sums
-    if (most < 2 || steps < 16) return 1;   // (below that a second launch costs more than the K steps it would save)
-    const double plain = std::min({ring_plan(M, N, steps, cus, 1, 1).us, skinny_us(M, N, k_bytes, elem_size(in_dtype), b_kmajor),
-                                   tiles256_us((long)((M + 255) / 256) * ((N + 255) / 256), 256, steps, cus, false, elem_size(in_dtype) == 1)});
+    // (up to 64 rows or columns: nothing to gain from 32 K steps - 64 x 2048 x 2048 fp16 8.4 us, in the best splits 9.6, 1 x
+    // 1000 x 4096 e4m3 7.6 / 10.2; 64 x 2048 x 4096 18.0 / 12.1 - or in slices of fewer than eight)
+    const bool few = std::min(M, N) <= 64, stream = streams(M, N, k_bytes, elem_size(in_dtype), b_kmajor, cus);
+    const int most = (int)std::min<int64_t>(std::min<int64_t>(32, steps / (few ? 8 : 2)), (64ll << 20) / std::max<int64_t>(1, 4ll * M * N));   // 64 MiB of partial sums
+    if (most < 2 || steps < (few ? 48 : 16)) return 1;   // (below that a second launch costs more than the K steps it would save)
+    const double plain = stream ? stream_us(M, N, k_bytes, b_kmajor, cus)
+                                : std::min(ring_plan(M, N, steps, cus, 1, 1).us,
+                                           tiles256_us((long)((M + 255) / 256) * ((N + 255) / 256), 256, steps, cus, false, elem_size(in_dtype) == 1));
     const RingPlan split = ring_plan(M, N, steps, cus, 2, most);
-    return split.us < 0.95 * plain ? split.splits : 1;
+    // (columns that are not groups of four are added up one by one: 8192 x 33 x 8192 e4m3 19.0 us, in two slices 22.1)
+    return split.us + (few && N % 4 != 0 ? 1.5 : 0.0) < (stream ? 0.85 : 0.95) * plain ? split.splits : 1;
   }
   // the one-barrier-per-step kernel on 128x128 tiles, 64-byte K steps: a workgroup per CU, at least sixteen K steps each, at most
   // 32 slices; nothing to gain from half a round of tiles on or below 64 K steps
   const int small = std::min(M, N);
-  if (small <= 32) return 1;   // (the streaming kernel)
+  if (small <= 32) return 1;
   const long tiles = (long)((M + 127) / 128) * ((N + 127) / 128);
   const int ksteps = (int)((k_bytes + 63) / 64);
   long splits = tiles * 2 > cus || ksteps < 64 ? 1 : std::min<long>(std::min<long>(cus / tiles, ksteps / 16), 32);
@@ -424,15 +455,15 @@ static int gemm_impl(const void* A, const void* B, void* C, int M, int N, int K,
   const bool skinny_allowed = tile_arg < 0 && knob(knobs().skinny, 1);  // an explicit tile means a tile kernel
   const bool can_ring = ring_ok(es, b_kmajor);
   const int ksteps128 = (p.k_bytes + 127) / 128;
-  // at most 32 rows on one side: stream the other operand once (X = small side, Y = streamed side) where that is the faster
-  // way (skinny_us), or where MI355_GEMM_SKINNY asks for it
-  if (skinny_allowed && k_rows == 0 && std::min(M, N) <= 32 &&
-      (knobs().skinny != UNSET || !can_ring || skinny_us(M, N, p.k_bytes, es, b_kmajor) < ring_plan(M, N, ksteps128, cus, 1, 1).us)) {
+  // at most 64 rows on one side: stream the other operand once (X = small side, Y = streamed side) where that is the faster
+  // way, or where MI355_GEMM_SKINNY asks for it
+  if (skinny_allowed && k_rows == 0 &&
+      (knobs().skinny != UNSET || streams(M, N, p.k_bytes, es, b_kmajor, cus) || streams8(M, N, p.k_bytes, es, b_kmajor, cus))) {
     SkinnyArgs sk{};
     sk.K = K; sk.C = (char*)C; sk.a_scale = a_scale; sk.b_scale = b_scale;
     sk.activation = activation; sk.out_dtype = out_dtype; sk.cus = device_info().cus;
     bool y_kmajor = true, x_kmajor = true;
-    if (M <= 32) {
+    if (M <= 64) {
       sk.X = (const char*)A; sk.Y = (const char*)B; sk.S = M; sk.L = N;
       sk.x_pitch = p.lda; sk.y_pitch = p.ldb; sk.cs = scm; sk.cl = scn;
       sk.aux = aux; sk.aux_ss = aux_sm; sk.aux_sl = aux_sn; sk.aux_dtype = aux_dtype;
@@ -444,6 +475,7 @@ static int gemm_impl(const void* A, const void* B, void* C, int M, int N, int K,
       x_kmajor = b_kmajor;
     }
     if (gemm_skinny_ok(sk, y_kmajor, x_kmajor, es)) return gemm_skinny_launch(sk, in_dtype, y_kmajor, x_kmajor, stream);
+    if (is8 && b_kmajor && !aux && gemm8_skinny_ok(p)) return gemm8_skinny_launch(p, in_dtype == MI355_F8E5M2, stream);
   }
   // the ring kernels of 64 .. 128-row tiles where they are the faster ones by the two estimates above (and in place of the
   // other 128x128 kernel wherever they take the operands)
@@ -492,7 +524,6 @@ static int gemm_impl(const void* A, const void* B, void* C, int M, int N, int K,
   if (ring >= 0)
     return is8 ? gemm_ring8_launch(p, in_dtype == MI355_F8E5M2, ring, 1, 0, stream)
                : gemm_ring16_launch(p, in_dtype == MI355_BF16, b_kmajor, ring, 1, 0, stream);
-  if (is8 && b_kmajor && !aux && gemm8_skinny_ok(p) && skinny_allowed) return gemm8_skinny_launch(p, in_dtype == MI355_F8E5M2, stream);
   if (is8 && mixed_rows > 0) return gemm_wave128_f8_mixed_launch(p, mixed_rows, in_dtype == MI355_F8E5M2, stream);
   if (is8 && tile == 6 && (p.tile_m == 192 || p.tile_m == 128 || w128_ok)) return gemm_wave128_f8_launch(p, in_dtype == MI355_F8E5M2, b_kmajor, stream);
   if (is8) return gemm8_launch(p, in_dtype == MI355_F8E5M2, b_kmajor, tile, stream);

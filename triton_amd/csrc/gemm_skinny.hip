@@ -1,9 +1,9 @@
-// Skinny GEMM (fp16 / bf16, and fp8 with both operands K-contiguous): one side of the product has at most 32 rows (decode-style M = 1..32,
-// or N <= 32), so the work is reading the other operand once from HBM
+// Skinny GEMM (fp16 / bf16, and fp8 with both operands K-contiguous): one side of the product has at most 64 rows (decode-style M = 1..64,
+// or N <= 64), so the work is reading the other operand once from HBM
 // (shapes of python/test/regression/test_performance.py:36-44; kernel contract of
 // python/tutorials/03-matrix-multiplication.py:241-316).
 //
-// Written for out[s][l] = sum_k X[s][k] * Y[l][k]: X the small operand (S <= 32 rows), Y the
+// Written for out[s][l] = sum_k X[s][k] * Y[l][k]: X the small operand (S <= 64 rows), Y the
 // streamed one (L rows).  The host maps (A, B) or (B^T, A^T) onto (X, Y).
 //   * one workgroup per 32 rows of Y, its waves split K into contiguous ranges and meet in LDS at
 //     the end - no tile reuse to organise, what matters is bytes in flight: every wave keeps
@@ -13,7 +13,7 @@
 //     private to the wave (no barriers in the loop) and come back transposed (ds_read_b64_tr_b16);
 //   * X is re-read by every workgroup from L2, prefetched with the same depth through the same
 //     ring: read back row-wise when K is contiguous, transposed when S is (the row-major B of a
-//     product with N = 32).
+//     product with N = 32 or 64).
 #include "common.h"
 #include "launch.h"
 #include "formats.h"
@@ -45,17 +45,24 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(SkinnyArgs p) {
   constexpr int LT = YM == 4 ? 2 : 1;   // 32-column tiles of the output per wave
   constexpr int TT = LT * ST;           // accumulator tiles per wave: [LT][ST]
   static_assert(!F8 || (!Y_LDS && YM != 4 && XM == 2), "fp8: both operands K-contiguous, X through LDS");
+  static_assert(XM != 3 || (NS % 2 == 0 && YM != 4), "pair tiles: a stage's parity is its slot's");
   constexpr int PD = NS - 1;          // stages in flight
   constexpr int LPS = (YM == 4 ? 4 : 2) + 2 * ST;   // vector-memory operations per stage: 2 (4) of Y, 2 per 32 rows of X
   // X: 0 = K contiguous, straight into registers (32-byte pieces of 32 rows per instruction: slower,
   //        kept for comparison); 1 = S contiguous, through LDS with a transposed read;
   //    2 = K contiguous, through LDS (64-byte pieces of 16 rows per instruction);
+  //    3 = K contiguous, through LDS in whole 128-byte lines (8 rows per instruction): pair tiles of [32 ST s][128
+  //        bytes of k] in a ring of their own, loaded like the pair tiles of YM 3 - first half of the rows with the odd
+  //        stage before the pair, second half with its even stage (needs K bytes a multiple of 128; not for fp8)
   constexpr bool X_LDS = XM != 0;
   static_assert(!((Y_LDS || YM == 4) && XM == 1), "one operand at most is transposed through LDS");
   constexpr int XROW = 64 * ST;       // bytes of one k row of an S-contiguous X tile: S = 32 ST
   constexpr int YSLOT = (YM == 1 || YM == 2) ? 2048 : YM == 4 ? 4096 : 0;   // [32 k][32 l] 16-bit, [32 l][64 bytes of k], or [32 k][64 l]
   constexpr int ND = 4, YPAIR = 4096;            // YM == 3: ring of ND tiles [32 l][128 bytes of k] behind the stage ring
   constexpr int XSLOT = (XM == 1 || XM == 2) ? 2048 * ST : 0;   // [32 k][32 ST s] or [32 ST s][32 k]
+  constexpr int XPAIR = 4096 * ST;               // XM == 3: [32 ST s][128 bytes of k]
+  constexpr int XND = (YM == 3 && ST == 2) ? 3 : 4;   // pair tiles of X in its ring (three where four do not fit next to Y's; a tile is dead
+                                                     // before the loads that re-use its place are issued from three on)
   constexpr int SLOT = YSLOT + XSLOT;            // bytes of one stage in LDS
   static_assert(PD * LPS < 64, "vmcnt has 6 bits");
   extern __shared__ __attribute__((aligned(1024))) char smem[];
@@ -68,7 +75,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(SkinnyArgs p) {
   const int l0 = xcd_remap(blockIdx.x, gridDim.x) * (32 * LT);
 
   const int nstages = p.K / (F8 ? 64 : 32);
-  const int per = YM == 3 ? (((nstages + NW - 1) / NW + 1) & ~1) : (nstages + NW - 1) / NW;   // (pair tiles: whole pairs of stages)
+  const int per = (YM == 3 || XM == 3) ? (((nstages + NW - 1) / NW + 1) & ~1) : (nstages + NW - 1) / NW;   // (pair tiles: whole pairs of stages)
   const int j_lo = wave * per, j_hi = min(nstages, j_lo + per);
 
   f32x16 acc[TT];
@@ -128,6 +135,18 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(SkinnyArgs p) {
   unsigned yrd3[2];
 #pragma unroll
   for (int ks = 0; ks < 2; ks++) yrd3[ks] = yring + l32 * 128 + ((((F8 ? 2 * g + ks : 2 * ks + g)) ^ ((l32 >> 1) & 7)) << 4);
+  // XM == 3: the same for X; instruction i of a pair (0 .. 4 ST - 1) moves rows 8 i .. 8 i + 7 (rows beyond S fetch
+  // row S - 1 into their place)
+  const unsigned xring = lds_addr(lds) + NW * (NS * SLOT) + (YM == 3 ? NW * (ND * YPAIR) : 0) + wave * (XND * XPAIR);
+  unsigned xdma3[XM == 3 ? 4 * ST : 1];
+  unsigned xrd3[2];
+  if constexpr (XM == 3) {
+#pragma unroll
+    for (int i = 0; i < 4 * ST; i++)
+      xdma3[i] = (unsigned)min(8 * i + (lane >> 3), p.S - 1) * (unsigned)p.x_pitch + (((lane & 7) ^ (4 * (i & 1) + (lane >> 4))) << 4);
+#pragma unroll
+    for (int ks = 0; ks < 2; ks++) xrd3[ks] = xring + l32 * 128 + (((2 * ks + g) ^ ((l32 >> 1) & 7)) << 4);
+  }
   // YM == 4: load instruction i of a stage moves k rows 8 i .. 8 i + 7 of 128 bytes (64 l); in the rows with bit 1 of
   // k set the two 64-byte halves change places (chunk c at position c ^ 4), so that the four k rows of a transposed
   // read - 128 bytes apart - lie in four different quarters of the banks.  Lane of a read: k row 8 g + i16 / 4 (+ 4,
@@ -167,6 +186,16 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(SkinnyArgs p) {
 #pragma unroll
       for (int i = 0; i < 2 * ST; i++)
         async_copy16_sbase(xsrc + (int64_t)i * (16 / ST) * p.x_pitch, xdma, ring + sl * SLOT + YSLOT + i * 1024);
+    } else if constexpr (XM == 3) {
+      // odd stage: first half of the rows of the NEXT pair (the last pair again where there is none); even: second half of its own
+      const int d = min((j + 1) >> 1, (j_hi >> 1) - 1), half = (j & 1) ^ 1;
+      const char* xsrc = p.X + (int64_t)d * 128;
+      const unsigned dst = xring + (d % XND) * XPAIR + half * (2 * ST * 1024);
+      static_for<2 * ST>([&](auto I_) {
+        constexpr int i = decltype(I_)::value;
+        if (half) async_copy16_sbase(xsrc, xdma3[2 * ST + i], dst + i * 1024);
+        else async_copy16_sbase(xsrc, xdma3[i], dst + i * 1024);
+      });
     } else if constexpr (XM == 2) {
       const char* xsrc = p.X + (int64_t)j * 64;
 #pragma unroll
@@ -244,7 +273,25 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(SkinnyArgs p) {
       yf[1] = yr[sl][1];
     }
     V8 xf[2][ST];
-    if constexpr (XM == 2) {
+    if constexpr (XM == 3) {
+      const unsigned xb = (unsigned)((j >> 1) % XND) * XPAIR;
+      i32x4 xv[2][ST];
+      static_for<2>([&](auto KS_) {
+        constexpr int ks = decltype(KS_)::value;
+        static_for<ST>([&](auto T_) {
+          constexpr int t = decltype(T_)::value;
+          xv[ks][t] = lds_read_b128<t * 4096>((xrd3[ks] ^ ((sl & 1) * 64u)) + xb);
+        });
+      });
+      lds_wait<0>();
+#pragma unroll
+      for (int ks = 0; ks < 2; ks++)
+#pragma unroll
+        for (int t = 0; t < ST; t++) {
+          lds_use(xv[ks][t]);
+          xf[ks][t] = __builtin_bit_cast(V8, xv[ks][t]);
+        }
+    } else if constexpr (XM == 2) {
       i32x4 xv[2][ST];
       static_for<2>([&](auto KS_) {
         constexpr int ks = decltype(KS_)::value;
@@ -319,6 +366,13 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(SkinnyArgs p) {
       async_copy16_sbase(src, ydma3[0], dst);
       async_copy16_sbase(src + 8 * p.y_pitch, ydma3[1], dst + 1024);
     }
+    if constexpr (XM == 3) {
+      // first half of the rows of the first pair
+      const int d = j_lo >> 1;
+      const char* xsrc = p.X + (int64_t)d * 128;
+      const unsigned dst = xring + (d % XND) * XPAIR;
+      static_for<2 * ST>([&](auto I_) { async_copy16_sbase(xsrc, xdma3[decltype(I_)::value], dst + decltype(I_)::value * 1024); });
+    }
     static_for<PD>([&](auto S_) { issue(min(j_lo + decltype(S_)::value, j_hi - 1), S_); });
     for (int j = j_lo; j < j_hi; j += NS) {
       static_for<NS>([&](auto U_) {
@@ -377,7 +431,8 @@ static int launch_skinny(const SkinnyArgs& p, hipStream_t stream) {
   // (YM 4, 64 columns per workgroup: half as many workgroups, so eight waves each split K eight ways)
   constexpr int NW = YM == 4 ? 8 : 4, NS = YM == 4 ? 3 : 4;
   constexpr int LT = YM == 4 ? 2 : 1;
-  constexpr int ring = NW * NS * ((YM == 1 || YM == 2 ? 2048 : YM == 4 ? 4096 : 0) + (XM == 1 || XM == 2 ? 2048 * ST : 0)) + (YM == 3 ? NW * 4 * 4096 : 0), red = NW * LT * ST * 16 * 64 * 4;
+  constexpr int ring = NW * NS * ((YM == 1 || YM == 2 ? 2048 : YM == 4 ? 4096 : 0) + (XM == 1 || XM == 2 ? 2048 * ST : 0)) + (YM == 3 ? NW * 4 * 4096 : 0) +
+                       (XM == 3 ? NW * ((YM == 3 && ST == 2) ? 3 : 4) * 4096 * ST : 0), red = NW * LT * ST * 16 * 64 * 4;
   static_assert(ring <= 160 * 1024, "LDS of one CU");
   constexpr int smem = ring > red ? ring : red;
   static bool attr_set = false;
@@ -391,15 +446,17 @@ static int launch_skinny(const SkinnyArgs& p, hipStream_t stream) {
   return (int)hipGetLastError();
 }
 
-// S <= 32, whole 32-row blocks of Y and whole 64-byte stages; pitches in bytes, 16-byte aligned rows,
-// small enough that 64 rows of X / 32 rows of Y are reached with 32-bit offsets.  An S-contiguous
-// X (x_kmajor false) needs S = 32 and a K-contiguous Y.  elem_bytes = 2 or 1 (fp8: both
-// operands K-contiguous).
-bool gemm_skinny_ok(const SkinnyArgs& p, bool y_kmajor, bool x_kmajor, int elem_bytes) {
-  if (!x_kmajor && (!y_kmajor || p.S != 32)) return false;
+// S <= 64 (32 next to an L-contiguous Y), whole 32-row blocks of Y and whole 64-byte stages; an S-contiguous
+// X (x_kmajor false) needs S = 32 or 64 and a K-contiguous Y.  elem_bytes = 2 or 1 (fp8: both operands K-contiguous).
+bool gemm_skinny_sizes_ok(int S, int L, int64_t k_bytes, bool y_kmajor, bool x_kmajor, int elem_bytes) {
+  if (!x_kmajor && (!y_kmajor || (S != 32 && S != 64))) return false;
   if (elem_bytes == 1 && !(x_kmajor && y_kmajor)) return false;
-  const int64_t kb = (int64_t)p.K * elem_bytes;
-  return p.S >= 1 && p.S <= 32 && p.L >= 32 && p.L % 32 == 0 && kb >= 64 && kb % 64 == 0 &&
+  return S >= 1 && S <= (y_kmajor ? 64 : 32) && L >= 32 && L % 32 == 0 && k_bytes >= 64 && k_bytes % 64 == 0;
+}
+
+// Pitches in bytes: 16-byte aligned rows, small enough that 64 rows of X / 32 rows of Y are reached with 32-bit offsets.
+bool gemm_skinny_ok(const SkinnyArgs& p, bool y_kmajor, bool x_kmajor, int elem_bytes) {
+  return gemm_skinny_sizes_ok(p.S, p.L, (int64_t)p.K * elem_bytes, y_kmajor, x_kmajor, elem_bytes) &&
          p.x_pitch % 16 == 0 && p.y_pitch % 16 == 0 && p.x_pitch < (1 << 25) && p.y_pitch < (1 << 26);
 }
 
@@ -416,6 +473,12 @@ template <typename E, int XM, int ST>
 static int launch_skinny_yk(const SkinnyArgs& p, int elem_bytes, hipStream_t stream) {
   if constexpr (YK == 3) {
     if (((int64_t)p.K * elem_bytes) % 128 == 0) {
+      // (49 .. 64 K-contiguous rows of X: whole lines for X too, in a ring of three pair tiles next to Y's four; 16-bit.
+      // 64 x 8192 x 8192 with a K-contiguous weight 32.0 -> 30.0 us, 8192 x 64 x 8192 30.1 -> 28.2; but 48 rows 26.0 -> 27.5.
+      // With at most 32 rows whole lines for X measured +-0 and -1.2 %: 64-byte pieces)
+      if constexpr (XM == 2 && ST == 2 && !E::kF8) {
+        if (p.S > 48) return launch_skinny<E, 3, 3, ST>(p, stream);
+      }
       return launch_skinny<E, 3, XM, ST>(p, stream);
     }
     return launch_skinny<E, 2, XM, ST>(p, stream);
@@ -427,8 +490,9 @@ static int launch_skinny_yk(const SkinnyArgs& p, int elem_bytes, hipStream_t str
 template <typename V8>
 static int launch_skinny_v(const SkinnyArgs& p, bool y_kmajor, bool x_kmajor, hipStream_t stream) {
   using E = Skinny16<V8>;
-  if (!x_kmajor) return launch_skinny_yk<E, 1, 1>(p, 2, stream);
-  if (y_kmajor) return launch_skinny_yk<E, 2, 1>(p, 2, stream);
+  const bool two = p.S > 32;
+  if (!x_kmajor) return two ? launch_skinny_yk<E, 1, 2>(p, 2, stream) : launch_skinny_yk<E, 1, 1>(p, 2, stream);
+  if (y_kmajor) return two ? launch_skinny_yk<E, 2, 2>(p, 2, stream) : launch_skinny_yk<E, 2, 1>(p, 2, stream);
   // an L-contiguous Y: whole lines (64 columns per workgroup) where L is a multiple of 64
   // (enough columns that 64 per workgroup still
   // give every compute unit one - 16 x 16384 x 8192 5250 -> 6050 GB/s, but 16 x 8192 x 8192, 128 workgroups, 4685 -> 4580)
@@ -438,8 +502,9 @@ static int launch_skinny_v(const SkinnyArgs& p, bool y_kmajor, bool x_kmajor, hi
 
 // kind: 0 fp16, 1 bf16, 2 fp8 e4m3fn, 3 fp8 e5m2 (the dtype codes of the C ABI)
 int gemm_skinny_launch(const SkinnyArgs& p, int kind, bool y_kmajor, bool x_kmajor, hipStream_t stream) {
-  if (kind == 2) return launch_skinny_yk<Skinny8<0>, 2, 1>(p, 1, stream);
-  if (kind == 3) return launch_skinny_yk<Skinny8<1>, 2, 1>(p, 1, stream);
+  const bool two = p.S > 32;
+  if (kind == 2) return two ? launch_skinny_yk<Skinny8<0>, 2, 2>(p, 1, stream) : launch_skinny_yk<Skinny8<0>, 2, 1>(p, 1, stream);
+  if (kind == 3) return two ? launch_skinny_yk<Skinny8<1>, 2, 2>(p, 1, stream) : launch_skinny_yk<Skinny8<1>, 2, 1>(p, 1, stream);
   return kind == 1 ? launch_skinny_v<bf16x8>(p, y_kmajor, x_kmajor, stream) : launch_skinny_v<f16x8>(p, y_kmajor, x_kmajor, stream);
 }
 

@@ -48,7 +48,7 @@ struct GemmStridedArgs {
 
 // skinny GEMM, out[s][l] = sum_k X[s][k] * Y[l][k]
 struct SkinnyArgs {
-  const char* X;    // small operand: S <= 32 rows, K contiguous or S contiguous
+  const char* X;    // small operand: S <= 64 rows, K contiguous or S contiguous
   const char* Y;    // streamed operand: L rows, K contiguous or L contiguous
   char* C;
   int S, L, K;
@@ -155,6 +155,7 @@ bool gemm_wave128_mxfp8_ok(const GemmArgs& p);
 int gemm_wave128_mxfp8_launch(const GemmArgs& p, hipStream_t stream);
 bool gemm8_skinny_ok(const GemmArgs& p);  // M <= 32, K a multiple of 256
 int gemm8_skinny_launch(const GemmArgs& p, bool e5m2, hipStream_t stream);
+bool gemm_skinny_sizes_ok(int S, int L, int64_t k_bytes, bool y_kmajor, bool x_kmajor, int elem_bytes);
 bool gemm_skinny_ok(const SkinnyArgs& p, bool y_kmajor, bool x_kmajor, int elem_bytes);
 int gemm_skinny_launch(const SkinnyArgs& p, int kind, bool y_kmajor, bool x_kmajor, hipStream_t stream);
 int gemm_strided_launch(const GemmStridedArgs& p, hipStream_t stream);   // fp32 FMAs, one thread per 4 x 4 outputs (a second implementation for tests)
