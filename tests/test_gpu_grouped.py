@@ -144,3 +144,20 @@ def test_row_strides_beyond_32_bits_are_refused(gpu, extension, monkeypatch):
     row = torch.zeros(8, device=gpu, dtype=torch.float16).as_strided((1, 8), ((1 << 32) + 8, 1))
     with pytest.raises(RuntimeError):
         triton_amd.group_gemm_fn([row], [torch.zeros(8, 8, device=gpu, dtype=torch.float16)])
+
+
+@pytest.mark.parametrize("dtype", ["fp16", "bf16"])
+@pytest.mark.parametrize("extension", [True, False])
+def test_rows_of_a_and_b_may_overlap(gpu, extension, dtype, monkeypatch):
+    # one row repeated (row stride 0) and windows shifted by less than a row, in A and in B, next to an ordinary problem;
+    # exact sums of small integers
+    from triton_amd import _lib
+
+    if not extension:
+        monkeypatch.setattr(_lib, "ext", lambda: None)
+    rng = np.random.default_rng(3)
+    ints = lambda *shape: from_np(rng.integers(-2, 3, size=shape).astype(np.float32), dtype, gpu)   # noqa: E731
+    a = [ints(1, 64).expand(96, 64), ints(96, 64), ints(1024).as_strided((96, 64), (8, 1)), ints(72, 64), ints(96, 64), ints(1, 8).expand(1, 8)]
+    b = [ints(64, 80), ints(1, 80).expand(64, 80), ints(64, 80), ints(1024).as_strided((64, 80), (8, 1)), ints(64, 80), ints(1, 72).expand(8, 72)]
+    for x, y, c in zip(a, b, triton_amd.group_gemm_fn(a, b)):
+        assert torch.equal(c.float(), x.float() @ y.float())

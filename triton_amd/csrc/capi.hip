@@ -883,7 +883,7 @@ int mi355_grouped_gemm_host(const void* const* a, const void* const* b, void* co
   for (int i = 0; i < group_size; i++) {
     const int32_t *s = sizes + 3 * i, *l = lds + 3 * i;
     if (!a[i] || !b[i] || !c[i] || s[0] <= 0 || s[1] <= 0 || s[2] <= 0) return MI355_EINVAL;
-    if (l[0] < s[2] || l[1] < s[1] || l[2] < s[1]) return MI355_ESTRIDE;
+    if (l[2] < s[1]) return MI355_ESTRIDE;   // (rows of C must not overlap; those of A and B may)
   }
   if (!device_info().gfx950) return MI355_EDEVICE;
   hipStream_t stream = (hipStream_t)stream_;
@@ -898,8 +898,8 @@ int mi355_grouped_gemm_host(const void* const* a, const void* const* b, void* co
     long tiles256 = 0;
     for (int i = 0; i < count; i++) {
       const int32_t *s = sizes + 3 * (g0 + i), *l = lds + 3 * (g0 + i);
-      // rows of 16-byte chunks, pitches within the kernels' lane offsets: else the product's own launch
-      if (s[2] % 8 || l[0] % 8 || l[1] % 8 || l[1] < (s[1] + 7) / 8 * 8 || !aligned(a[g0 + i], 16) || !aligned(b[g0 + i], 16) || l[0] >= (1 << 22) || l[1] >= (1 << 25)) {
+      // rows of 16-byte chunks that do not overlap, pitches within the kernels' lane offsets: else the product's own launch
+      if (s[2] % 8 || l[0] % 8 || l[0] < s[2] || l[1] % 8 || l[1] < (s[1] + 7) / 8 * 8 || !aligned(a[g0 + i], 16) || !aligned(b[g0 + i], 16) || l[0] >= (1 << 22) || l[1] >= (1 << 25)) {
         const int rc = mi355_gemm(a[g0 + i], b[g0 + i], c[g0 + i], s[0], s[1], s[2], l[0], 1, l[1], 1, l[2], 1, dtype, dtype, nullptr, nullptr, MI355_ACT_NONE, stream_);
         if (rc) return rc;
         continue;
