@@ -161,3 +161,20 @@ def test_rows_of_a_and_b_may_overlap(gpu, extension, dtype, monkeypatch):
     b = [ints(64, 80), ints(1, 80).expand(64, 80), ints(64, 80), ints(1024).as_strided((64, 80), (8, 1)), ints(64, 80), ints(1, 72).expand(8, 72)]
     for x, y, c in zip(a, b, triton_amd.group_gemm_fn(a, b)):
         assert torch.equal(c.float(), x.float() @ y.float())
+
+
+@pytest.mark.parametrize("dtype", ["fp16", "bf16"])
+@pytest.mark.parametrize("every", [1, 2, 40])
+def test_problems_without_16_byte_rows_share_a_launch(gpu, dtype, every):
+    # 70 problems (a table holds 64), all of them, every other one and two (one in each table) without 16-byte rows: odd sizes, a
+    # base that is not aligned, one row, one column, K = 1, several tiles; exact sums of small integers
+    rng = np.random.default_rng(every)
+    odd = [(37, 19, 7), (1, 1, 1), (130, 65, 33), (1, 200, 250), (200, 1, 70), (64, 64, 65), (65, 130, 8)]
+    ga, gb = [], []
+    for i in range(70):
+        m, n, k = odd[(i // every) % len(odd)] if i % every == 0 else (16 + 8 * (i % 9), 8 * (1 + i % 7), 64)
+        x, y = (from_np(rng.integers(-2, 3, size=s).astype(np.float32), dtype, gpu) for s in ((m, k), (k * n + 1,)))
+        ga.append(x)
+        gb.append((y[1:] if i % every == 0 else y[:-1]).view(k, n))
+    for x, y, c in zip(ga, gb, triton_amd.group_gemm_fn(ga, gb)):
+        assert torch.equal(c.float(), (x.float() @ y.float()).to(c.dtype).float()), (x.shape, y.shape)

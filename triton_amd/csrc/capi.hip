@@ -892,16 +892,15 @@ int mi355_grouped_gemm_host(const void* const* a, const void* const* b, void* co
   constexpr int G = GroupedTable::kMax;
   for (int g0 = 0; g0 < group_size; g0 += G) {
     const int count = std::min(G, group_size - g0);
-    int order[G], n = 0;
+    int order[G], n = 0, odd[G], nodd = 0;
     double cost64[G], cost128[G], sum64 = 0, sum128 = 0, sum = 0, top64 = 0, top128 = 0, top = 0;
     bool whole = true;
     long tiles256 = 0;
     for (int i = 0; i < count; i++) {
       const int32_t *s = sizes + 3 * (g0 + i), *l = lds + 3 * (g0 + i);
-      // rows of 16-byte chunks that do not overlap, pitches within the kernels' lane offsets: else the product's own launch
+      // rows of 16-byte chunks that do not overlap, pitches within the kernels' lane offsets: else the kernel of any strides
       if (s[2] % 8 || l[0] % 8 || l[0] < s[2] || l[1] % 8 || l[1] < (s[1] + 7) / 8 * 8 || !aligned(a[g0 + i], 16) || !aligned(b[g0 + i], 16) || l[0] >= (1 << 22) || l[1] >= (1 << 25)) {
-        const int rc = mi355_gemm(a[g0 + i], b[g0 + i], c[g0 + i], s[0], s[1], s[2], l[0], 1, l[1], 1, l[2], 1, dtype, dtype, nullptr, nullptr, MI355_ACT_NONE, stream_);
-        if (rc) return rc;
+        odd[nodd++] = i;
         continue;
       }
       // us of one tile and of all, on either tile size (the figures of ring_plan with several rounds under way)
@@ -916,15 +915,36 @@ int mi355_grouped_gemm_host(const void* const* a, const void* const* b, void* co
               (int64_t)l[0] * 16 + s[2] * 2 < (1ll << 31) && (int64_t)s[2] * l[1] * 2 + 512 < (1ll << 31);
       order[n++] = i;
     }
-    if (n == 0) continue;
     GroupedTable ga{};
-    ga.group_size = n; ga.out_dtype = dtype;
-    ga.chunk = std::max(1, knob(knobs().grouped_chunk, 4));
     auto put = [&](int at, int i) {
       ga.a_ptrs[at] = (uint64_t)a[g0 + i]; ga.b_ptrs[at] = (uint64_t)b[g0 + i]; ga.c_ptrs[at] = (uint64_t)c[g0 + i];
       for (int e = 0; e < 3; e++) { ga.sizes[3 * at + e] = sizes[3 * (g0 + i) + e]; ga.lds[3 * at + e] = lds[3 * (g0 + i) + e]; }
     };
     int rc;
+    if (nodd > 0) {
+      int64_t tiles = 0;
+      for (int at = 0; at < nodd; at++) {
+        put(at, odd[at]);
+        ga.first_tile[at] = (int)std::min<int64_t>(tiles, INT_MAX);
+        tiles += (int64_t)((ga.sizes[3 * at] + 63) / 64) * ((ga.sizes[3 * at + 1] + 63) / 64);
+      }
+      for (int at = nodd; at < G; at++) ga.first_tile[at] = INT_MAX;
+      if (nodd > 1 && tiles <= INT_MAX / 2) {
+        ga.group_size = nodd; ga.out_dtype = dtype; ga.total_tiles = (int)tiles;
+        rc = gemm_masked_grouped_launch(ga, bf16, stream);
+        if (rc) return rc;
+      } else {
+        for (int at = 0; at < nodd; at++) {
+          const int32_t *s = sizes + 3 * (g0 + odd[at]), *l = lds + 3 * (g0 + odd[at]);
+          rc = mi355_gemm(a[g0 + odd[at]], b[g0 + odd[at]], c[g0 + odd[at]], s[0], s[1], s[2], l[0], 1, l[1], 1, l[2], 1, dtype, dtype, nullptr, nullptr, MI355_ACT_NONE, stream_);
+          if (rc) return rc;
+        }
+      }
+    }
+    if (n == 0) continue;
+    ga = GroupedTable{};
+    ga.group_size = n; ga.out_dtype = dtype;
+    ga.chunk = std::max(1, knob(knobs().grouped_chunk, 4));
     if (whole && knobs().grouped_wave128_min_k != 0 && tiles256 >= knob(knobs().grouped_big_min, cus)) {
       // whole 256x256 tiles, at least one per CU: runs of them as one stream of K steps
       for (int at = 0; at < n; at++) put(at, order[at]);

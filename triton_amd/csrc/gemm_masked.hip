@@ -74,15 +74,16 @@ __device__ __forceinline__ void store_out(void* p, int64_t idx, int dtype, float
   }
 }
 
+// Tile number `tile` of a product, row after row of tiles; once per workgroup.
 template <int IN>
-__global__ __launch_bounds__(256) void gemm_masked_kernel(GemmStridedArgs p) {
+__device__ __forceinline__ void masked_tile(const GemmStridedArgs& p, const unsigned tile) {
   using V8 = std::conditional_t<IN == 1, bf16x8, f16x8>;
   __shared__ __attribute__((aligned(16))) uint16_t sa[2][MBM * PITCH];
   __shared__ __attribute__((aligned(16))) uint16_t sb[2][MBN * PITCH];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave >> 1, wn = wave & 1, l32 = lane & 31, g = lane >> 5;
   const int nbn = (p.N + MBN - 1) / MBN;   // (a one-dimensional grid: either count of tiles may exceed 65535)
-  const int m0 = (int)(blockIdx.x / nbn) * MBM, n0 = (int)(blockIdx.x % nbn) * MBN;
+  const int m0 = (int)(tile / nbn) * MBM, n0 = (int)(tile % nbn) * MBN;
   const bool b_rows_contiguous = p.sbn == 1 && p.sbk != 1;   // row-major B: fetch along n, store transposed
 
   // A and a B with any other layout: thread -> row tid / 4, elements 8 (tid % 4) .. + 7 and 32 further of the K step;
@@ -171,6 +172,25 @@ __global__ __launch_bounds__(256) void gemm_masked_kernel(GemmStridedArgs p) {
   }
 }
 
+template <int IN>
+__global__ __launch_bounds__(256) void gemm_masked_kernel(GemmStridedArgs p) { masked_tile<IN>(p, blockIdx.x); }
+
+// The problems of a group that the tile kernels do not take, a workgroup per tile of any of them.  Bound by the launches
+// where it stands in for one of each problem: 100 problems of 37 x 19 x 7 636 us a call one by one and 184 together, of 16 x
+// 250 x 250 886 and 189 (two launches of 64 and 36, the host's checks of the tensors are what is left).
+template <int IN>
+__global__ __launch_bounds__(256) void gemm_masked_grouped_kernel(GroupedTable ga) {
+  // one table entry per lane: the problem of a tile is a comparison away
+  const int t = (int)blockIdx.x, first = ga.first_tile[threadIdx.x & 63];
+  const int gi = __builtin_amdgcn_readfirstlane((int)__popcll(__ballot(first <= t)) - 1);
+  GemmStridedArgs p{};
+  p.A = (const void*)ga.a_ptrs[gi]; p.B = (const void*)ga.b_ptrs[gi]; p.C = (void*)ga.c_ptrs[gi];
+  p.M = ga.sizes[gi * 3]; p.N = ga.sizes[gi * 3 + 1]; p.K = ga.sizes[gi * 3 + 2];
+  p.sam = ga.lds[gi * 3]; p.sak = 1; p.sbk = ga.lds[gi * 3 + 1]; p.sbn = 1; p.scm = ga.lds[gi * 3 + 2]; p.scn = 1;
+  p.in_dtype = IN; p.out_dtype = ga.out_dtype;
+  masked_tile<IN>(p, (unsigned)(t - ga.first_tile[gi]));
+}
+
 }  // namespace
 
 int gemm_masked_launch(const GemmStridedArgs& p, hipStream_t stream) {
@@ -183,6 +203,12 @@ int gemm_masked_launch(const GemmStridedArgs& p, hipStream_t stream) {
     case 2: hipLaunchKernelGGL(gemm_masked_kernel<2>, grid, dim3(256), 0, stream, p); break;
     default: hipLaunchKernelGGL(gemm_masked_kernel<3>, grid, dim3(256), 0, stream, p); break;
   }
+  return (int)hipGetLastError();
+}
+
+int gemm_masked_grouped_launch(const GroupedTable& ga, bool bf16, hipStream_t stream) {
+  if (bf16) gemm_masked_grouped_kernel<1><<<dim3(ga.total_tiles), dim3(256), 0, stream>>>(ga);
+  else gemm_masked_grouped_kernel<0><<<dim3(ga.total_tiles), dim3(256), 0, stream>>>(ga);
   return (int)hipGetLastError();
 }
 

@@ -112,7 +112,7 @@ struct GroupedTable {
   uint64_t a_ptrs[kMax], b_ptrs[kMax], c_ptrs[kMax];
   int sizes[kMax * 3];
   int lds[kMax * 3];
-  int first_tile[kMax];    // ring kernel: number of the problem's first tile (past the last problem: 2^31 - 1)
+  int first_tile[kMax];    // ring and masked kernels: number of the problem's first tile (past the last problem: 2^31 - 1)
   uint64_t small_tiles;    // ring kernel: problems on tiles of 64x64, bit per problem (the others: 128x128)
   int group_size;
   int out_dtype;
@@ -123,6 +123,7 @@ static_assert(sizeof(GroupedTable) <= 3584, "a kernel's arguments are at most 4 
 
 int gemm_wave128_grouped_table_launch(const GroupedTable& ga, bool bf16, int nprog, hipStream_t stream);   // whole 256x256 tiles, K as in grouped_plan
 int gemm_ring_grouped_launch(const GroupedTable& ga, bool bf16, int nprog, hipStream_t stream);
+int gemm_masked_grouped_launch(const GroupedTable& ga, bool bf16, hipStream_t stream);   // tiles of 64x64, any row strides
 
 int gemm16_grouped_launch(const GroupedArgs& ga, bool bf16, int nprog, int nprog_big, hipStream_t stream);
 int gemm16_launch(const GemmArgs& p, bool bf16, bool b_kmajor, int tile, hipStream_t stream);
