@@ -178,3 +178,22 @@ def test_problems_without_16_byte_rows_share_a_launch(gpu, dtype, every):
         gb.append((y[1:] if i % every == 0 else y[:-1]).view(k, n))
     for x, y, c in zip(ga, gb, triton_amd.group_gemm_fn(ga, gb)):
         assert torch.equal(c.float(), (x.float() @ y.float()).to(c.dtype).float()), (x.shape, y.shape)
+
+
+def test_matrices_of_other_libraries(gpu):
+    # whatever has data_ptr(), dtype, shape, stride(i) and device, next to a tensor of torch's and alone
+    class Foreign:
+        def __init__(self, t):
+            self.t, self.dtype, self.shape, self.device = t, t.dtype, tuple(t.shape), t.device
+
+        def data_ptr(self):
+            return self.t.data_ptr()
+
+        def stride(self, i):
+            return self.t.stride(i)
+
+    rng = np.random.default_rng(8)
+    a, b = ([from_np(rng.integers(-2, 3, size=(64, 64)).astype(np.float32), "fp16", gpu) for _ in range(2)] for _ in range(2))
+    want = [x.float() @ y.float() for x, y in zip(a, b)]
+    for ga, gb in (([Foreign(a[0]), a[1]], [b[0], b[1]]), ([Foreign(x) for x in a], [Foreign(y) for y in b])):
+        assert all(torch.equal(c.float(), w) for c, w in zip(triton_amd.group_gemm_fn(ga, gb), want))

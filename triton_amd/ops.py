@@ -305,7 +305,7 @@ def group_gemm_fn(group_A, group_B, *, num_programs: int = 0):
         assert A.dtype == B.dtype == group_A[0].dtype, "all matrices of a group share one dtype"
         assert A.stride(1) == 1 and B.stride(1) == 1, "matrices must be row major"
     ext = _lib.ext()
-    if ext is not None:
+    if ext is not None and all(isinstance(t, torch.Tensor) for t in (*group_A, *group_B)):
         return ext.group_gemm(list(group_A), list(group_B), int(num_programs))
     group_C = [torch.empty((A.shape[0], B.shape[1]), device=A.device, dtype=A.dtype) for A, B in zip(group_A, group_B)]
     live = [i for i, C in enumerate(group_C) if C.numel() > 0 and group_A[i].shape[1] > 0]
