@@ -59,6 +59,27 @@ def test_fp8_record_counts_flops8(gpu):
     assert seen[0]["flops8"] == 2.0 * 64 ** 3 and seen[0]["bytes"] == 2 * 64 * 64
 
 
+@pytest.mark.parametrize("extension", [True, False])
+def test_hooks_see_launches_only(gpu, extension, monkeypatch):
+    # an empty result, an empty sum and refused operands launch nothing: no record, and no enter hook without its exit hook
+    if not extension:
+        monkeypatch.setattr(_lib, "ext", lambda: None)
+    seen = []
+    monkeypatch.setattr(hooks.Launch, "launch_enter_hook", seen.append)
+    new = lambda *shape, dtype=torch.float16, device=gpu: torch.ones(*shape, device=device, dtype=dtype)   # noqa: E731
+    assert triton_amd.matmul(new(0, 8), new(8, 4)).shape == (0, 4)
+    assert triton_amd.matmul(new(4, 8), new(8, 0)).shape == (4, 0)
+    assert not triton_amd.matmul(new(4, 0), new(0, 4)).any()
+    for a, b, error in ((new(4, 8), new(4, 8), AssertionError), (new(8, 4).t(), new(8, 4), AssertionError),
+                        (new(4, 8), new(8, 4, dtype=torch.bfloat16), AssertionError), (new(4, 8, dtype=torch.int32), new(8, 4, dtype=torch.int32), TypeError),
+                        (new(4, 8, device="cpu"), new(8, 4), ValueError)):
+        with pytest.raises(error):
+            triton_amd.matmul(a, b)
+    assert seen == []
+    triton_amd.matmul(new(4, 8), new(8, 4))
+    assert len(seen) == 1
+
+
 def test_memory_leak(gpu):
     # the reference's test, with matmul as the kernel: 100 launches may not grow the heap by 30 kB
     a = torch.randn(64, 64, device=gpu, dtype=torch.float16)

@@ -113,13 +113,20 @@ def matmul(a, b, activation="", *, out_dtype=None, a_scale=None, b_scale=None, a
         a_scale = _scale_ptr(a_scale, a.device)[1]
     if b_scale is not None:
         b_scale = _scale_ptr(b_scale, a.device)[1]
-    if hooks.Launch.launch_enter_hook is None and hooks.Launch.launch_exit_hook is None:
+    hooked = hooks.Launch.launch_enter_hook is not None or hooks.Launch.launch_exit_hook is not None
+    if not hooked or not _launches(a, b):
         return ext.matmul(a, b, act, out_dtype, a_scale, b_scale, add, softmax)
     md = hooks.enter("mi355_gemm", _stream(), hooks.matmul_launch_metadata,
                      ("mi355_gemm", a.shape[0], b.shape[1], a.shape[1], a.element_size()))
     c = ext.matmul(a, b, act, out_dtype, a_scale, b_scale, add, softmax)
     hooks.exit(md)
     return c
+
+
+def _launches(a, b):
+    """Whether the product of two tensors launches a kernel: an empty one and operands that are refused do not reach the hooks."""
+    return (a.dim() == 2 and b.dim() == 2 and a.shape[1] == b.shape[0] and a.is_contiguous() and a.dtype == b.dtype and
+            a.dtype in _TORCH_TO_ABI and a.is_cuda and b.is_cuda and min(*a.shape, b.shape[1]) > 0)
 
 
 _ACTIVATIONS = {"": _lib.ACT_NONE, "leaky_relu": _lib.ACT_LEAKY_RELU}
