@@ -74,9 +74,29 @@ __device__ __forceinline__ void store_out(void* p, int64_t idx, int dtype, float
   }
 }
 
-// Tile number `tile` of a product, row after row of tiles; once per workgroup.
-template <int IN>
-__device__ __forceinline__ void masked_tile(const GemmStridedArgs& p, const unsigned tile) {
+// The problem of the group that this workgroup has a tile of, and that tile's number (one table entry per lane: the problem
+// is a comparison away).
+__device__ __forceinline__ GemmStridedArgs problem_of(const GroupedTable& ga, unsigned& tile) {
+  const int first = ga.first_tile[threadIdx.x & 63];
+  const int gi = __builtin_amdgcn_readfirstlane((int)__popcll(__ballot(first <= (int)tile)) - 1);
+  GemmStridedArgs p{};
+  p.A = (const void*)ga.a_ptrs[gi]; p.B = (const void*)ga.b_ptrs[gi]; p.C = (void*)ga.c_ptrs[gi];
+  p.M = ga.sizes[gi * 3]; p.N = ga.sizes[gi * 3 + 1]; p.K = ga.sizes[gi * 3 + 2];
+  p.sam = ga.lds[gi * 3]; p.sak = 1; p.sbk = ga.lds[gi * 3 + 1]; p.sbn = 1; p.scm = ga.lds[gi * 3 + 2]; p.scn = 1;
+  p.in_dtype = p.out_dtype = ga.out_dtype;
+  tile -= (unsigned)ga.first_tile[gi];
+  return p;
+}
+__device__ __forceinline__ const GemmStridedArgs& problem_of(const GemmStridedArgs& p, unsigned&) { return p; }
+
+// Args: GemmStridedArgs, a workgroup per tile, or GroupedTable, a workgroup per tile of any of the problems of a group that the
+// tile kernels do not take.  Bound by the launches where it stands in for one of each problem: 100 problems of 37 x 19 x 7
+// 636 us a call one by one and 184 together, of 16 x 250 x 250 886 and 189 (two launches of 64 and 36, the host's checks of the
+// tensors are what is left).
+template <int IN, typename Args = GemmStridedArgs>
+__global__ __launch_bounds__(256) void gemm_masked_kernel(Args args) {
+  unsigned tile = blockIdx.x;
+  const GemmStridedArgs& p = problem_of(args, tile);
   using V8 = std::conditional_t<IN == 1, bf16x8, f16x8>;
   __shared__ __attribute__((aligned(16))) uint16_t sa[2][MBM * PITCH];
   __shared__ __attribute__((aligned(16))) uint16_t sb[2][MBN * PITCH];
@@ -172,25 +192,6 @@ __device__ __forceinline__ void masked_tile(const GemmStridedArgs& p, const unsi
   }
 }
 
-template <int IN>
-__global__ __launch_bounds__(256) void gemm_masked_kernel(GemmStridedArgs p) { masked_tile<IN>(p, blockIdx.x); }
-
-// The problems of a group that the tile kernels do not take, a workgroup per tile of any of them.  Bound by the launches
-// where it stands in for one of each problem: 100 problems of 37 x 19 x 7 636 us a call one by one and 184 together, of 16 x
-// 250 x 250 886 and 189 (two launches of 64 and 36, the host's checks of the tensors are what is left).
-template <int IN>
-__global__ __launch_bounds__(256) void gemm_masked_grouped_kernel(GroupedTable ga) {
-  // one table entry per lane: the problem of a tile is a comparison away
-  const int t = (int)blockIdx.x, first = ga.first_tile[threadIdx.x & 63];
-  const int gi = __builtin_amdgcn_readfirstlane((int)__popcll(__ballot(first <= t)) - 1);
-  GemmStridedArgs p{};
-  p.A = (const void*)ga.a_ptrs[gi]; p.B = (const void*)ga.b_ptrs[gi]; p.C = (void*)ga.c_ptrs[gi];
-  p.M = ga.sizes[gi * 3]; p.N = ga.sizes[gi * 3 + 1]; p.K = ga.sizes[gi * 3 + 2];
-  p.sam = ga.lds[gi * 3]; p.sak = 1; p.sbk = ga.lds[gi * 3 + 1]; p.sbn = 1; p.scm = ga.lds[gi * 3 + 2]; p.scn = 1;
-  p.in_dtype = IN; p.out_dtype = ga.out_dtype;
-  masked_tile<IN>(p, (unsigned)(t - ga.first_tile[gi]));
-}
-
 }  // namespace
 
 int gemm_masked_launch(const GemmStridedArgs& p, hipStream_t stream) {
@@ -207,8 +208,8 @@ int gemm_masked_launch(const GemmStridedArgs& p, hipStream_t stream) {
 }
 
 int gemm_masked_grouped_launch(const GroupedTable& ga, bool bf16, hipStream_t stream) {
-  if (bf16) gemm_masked_grouped_kernel<1><<<dim3(ga.total_tiles), dim3(256), 0, stream>>>(ga);
-  else gemm_masked_grouped_kernel<0><<<dim3(ga.total_tiles), dim3(256), 0, stream>>>(ga);
+  if (bf16) gemm_masked_kernel<1, GroupedTable><<<dim3(ga.total_tiles), dim3(256), 0, stream>>>(ga);
+  else gemm_masked_kernel<0, GroupedTable><<<dim3(ga.total_tiles), dim3(256), 0, stream>>>(ga);
   return (int)hipGetLastError();
 }
 
