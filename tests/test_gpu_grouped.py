@@ -18,6 +18,19 @@ def _run(gpu, ga, gb, dtype, **kw):
     return [to_np(c) for c in triton_amd.group_gemm_fn(ta, tb, **kw)]
 
 
+def _run_device_tables(gpu, ta, tb, dtype, nprog=0):
+    """The same through mi355_grouped_gemm, whose five tables live on the device."""
+    from triton_amd import _lib
+
+    tc = [torch.full((a.shape[0], b.shape[1]), 7.0, dtype=a.dtype, device=gpu) for a, b in zip(ta, tb)]
+    pointers = [torch.tensor([t.data_ptr() for t in g], device=gpu, dtype=torch.int64) for g in (ta, tb, tc)]
+    sizes = torch.tensor([v for a, b in zip(ta, tb) for v in (a.shape[0], b.shape[1], a.shape[1])], dtype=torch.int32, device=gpu)
+    lds = torch.tensor([v for a, b, c in zip(ta, tb, tc) for v in (a.stride(0), b.stride(0), c.stride(0))], dtype=torch.int32, device=gpu)
+    assert _lib.load().mi355_grouped_gemm(*(t.data_ptr() for t in pointers), sizes.data_ptr(), lds.data_ptr(), len(ta),
+                                          _lib.F16 if dtype == "fp16" else _lib.BF16, nprog, torch.cuda.current_stream().cuda_stream) == 0
+    return tc
+
+
 @pytest.mark.parametrize("dtype", ["fp16", "bf16"])
 def test_reference_example_sizes(gpu, dtype):
     # 08:190-205: square problems 1024, 512, 256, 128 of uniform [0, 1) values
@@ -36,9 +49,9 @@ def test_reference_example_sizes(gpu, dtype):
 @pytest.mark.parametrize("big_min", [None, 1])
 @pytest.mark.parametrize("nprog", [0, 1, 7, 100])
 def test_ragged_problems_are_bit_exact_on_integers(gpu, nprog, big_min, monkeypatch):
-    # partial tiles, a single row, K tails (K % 32 != 0), and problems without 16-byte rows; once with
-    # the tile size the library picks for this group (128x128: fewer 256x256 tiles than CUs) and once
-    # with the 256x256 form forced (MI355_GROUPED_BIG_MIN=1)
+    # partial tiles, a single row, K tails (K % 32 != 0), and problems without 16-byte rows: tables in host memory (ring and
+    # any-stride kernels, whatever MI355_GROUPED_BIG_MIN says of a group that is not whole 256x256 tiles) and on the device, there
+    # with the tile size that is picked for this group (128x128: fewer 256x256 tiles than CUs) and with the 256x256 form (=1)
     if big_min is not None:
         set_knob(monkeypatch, "MI355_GROUPED_BIG_MIN", str(big_min))
     rng = np.random.default_rng(nprog)
@@ -50,6 +63,9 @@ def test_ragged_problems_are_bit_exact_on_integers(gpu, nprog, big_min, monkeypa
         outs = _run(gpu, ga, gb, dtype, num_programs=nprog)
         for c, r in zip(outs, ref):
             assert bits_equal(c, r)   # integer results below 2^11 are exact in fp16 and bf16
+        ta, tb = ([from_np(x, dtype, gpu) for x in g] for g in (ga, gb))
+        for c, r in zip(_run_device_tables(gpu, ta, tb, dtype, nprog), ref):
+            assert bits_equal(to_np(c), r)
 
 
 def test_strided_rows_and_empty_group(gpu):
@@ -67,8 +83,8 @@ def test_strided_rows_and_empty_group(gpu):
 @pytest.mark.parametrize("chunk", [4, 1, 3])
 @pytest.mark.parametrize("nprog", [0, 7, 100])
 def test_groups_of_whole_256_tiles(gpu, nprog, chunk, monkeypatch):
-    # every problem whole 256x256 tiles and K % 128 == 0: the four-wave 16x16-MFMA kernel takes the group
-    # (thresholds lowered so that 20 tiles and K = 128 are enough); exact sums of small integers, rounded
+    # every problem whole 256x256 tiles and K % 128 == 0: the four-wave 16x16-MFMA kernel takes the group, behind either
+    # kind of table (thresholds lowered so that 20 tiles and K = 128 are enough); exact sums of small integers, rounded
     # once; K from one pair of stages up to several, M != N, problems of one tile between larger ones
     set_knob(monkeypatch, "MI355_GROUPED_BIG_MIN", "1")
     set_knob(monkeypatch, "MI355_GROUPED_WAVE128_MIN_K", "128")
@@ -84,17 +100,23 @@ def test_groups_of_whole_256_tiles(gpu, nprog, chunk, monkeypatch):
         outs = _run(gpu, ga, gb, dtype, num_programs=nprog)
         for c, r in zip(outs, ref):
             assert bits_equal(c, formats.round_to(r, dtype))   # (K = 1024 reaches beyond bf16's exact integers)
-    # the same group through the eight-wave kernels
+        ta, tb = ([from_np(x, dtype, gpu) for x in g] for g in (ga, gb))
+        for c, r in zip(_run_device_tables(gpu, ta, tb, dtype, nprog), ref):
+            assert bits_equal(to_np(c), formats.round_to(r, dtype))
+    # the same group without that kernel: the ring kernels behind a host table, the eight-wave ones behind the device's
     set_knob(monkeypatch, "MI355_GROUPED_WAVE128_MIN_K", "0")
     for c, r in zip(_run(gpu, ga, gb, "fp16", num_programs=nprog), ref):
         assert bits_equal(c, r)
+    ta, tb = ([from_np(x, "fp16", gpu) for x in g] for g in (ga, gb))
+    for c, r in zip(_run_device_tables(gpu, ta, tb, "fp16", nprog), ref):
+        assert bits_equal(to_np(c), r)
 
 
 @pytest.mark.parametrize("dtype", ["fp16", "bf16"])
 def test_whole_tile_groups_at_the_default_thresholds_against_closed_form(gpu, dtype):
     # 256 tiles of 256x256 with K = 2048 select the four-wave kernel without any knob: N(0,1) operands, padded
     # rows of A and C-sized B pitch of 512-byte multiples in the second problem.  A B pitch that is no such
-    # multiple (third case) sends the group to the eight-wave kernels.
+    # multiple (third case) sends the group to the ring kernels (tables on the device: the eight-wave ones).
     rng = np.random.default_rng(5)
     mk = lambda shape: formats.round_to(rng.standard_normal(shape).astype(np.float32), dtype)
     a = [mk((2048, 2048)) for _ in range(4)]
@@ -106,19 +128,17 @@ def test_whole_tile_groups_at_the_default_thresholds_against_closed_form(gpu, dt
     for pad in (0, 256, 8):
         if pad:
             tb[1] = from_np(np.pad(b[1], ((0, 0), (pad, 0))), dtype, gpu)[:, pad:]
-        outs = triton_amd.group_gemm_fn(ta, tb)
-        for c, r in zip(outs, ref):
-            assert np.allclose(to_np(c), r, rtol=1e-2, atol=1e-2), pad
-            assert np.mean(to_np(c) == r) > 0.98
+        for outs in (triton_amd.group_gemm_fn(ta, tb), _run_device_tables(gpu, ta, tb, dtype)):
+            for c, r in zip(outs, ref):
+                assert np.allclose(to_np(c), r, rtol=1e-2, atol=1e-2), pad
+                assert np.mean(to_np(c) == r) > 0.98
 
 
 @pytest.mark.parametrize("dtype", ["fp16", "bf16"])
 @pytest.mark.parametrize("nprog", [0, 5])
 def test_host_tables_and_device_tables_agree_bit_for_bit(gpu, nprog, dtype):
     # more problems than one table holds (64), tiles of 64 and of 128 rows next to each other, K shorter than the ring and
-    # with a tail, problems without 16-byte rows in between; the device-table entry on the same matrices, in all its forms
-    from triton_amd import _lib
-
+    # with a tail, problems without 16-byte rows in between; the device-table entry on the same matrices (its 128x128 form)
     rng = np.random.default_rng(70 + nprog)
     shapes = [(17 + 31 * (i % 9), 8 * (1 + i % 7), 8 * (1 + i % 23)) for i in range(66)] + [(256, 512, 1024), (512, 256, 704), (33, 19, 7), (1, 64, 8)]
     ga = [from_np(rng.integers(-1, 2, size=(m, k)).astype(np.float32), dtype, gpu) for m, n, k in shapes]
@@ -126,13 +146,7 @@ def test_host_tables_and_device_tables_agree_bit_for_bit(gpu, nprog, dtype):
     outs = triton_amd.group_gemm_fn(ga, gb, num_programs=nprog)
     for a, b, c in zip(ga, gb, outs):
         assert torch.equal(c.float(), (a.float() @ b.float()).to(c.dtype).float()), (a.shape, b.shape)
-    again = [torch.empty_like(c) for c in outs]
-    tables = [torch.tensor([t.data_ptr() for t in g], device=gpu, dtype=torch.int64) for g in (ga, gb, again)]
-    sizes = torch.tensor([v for m, n, k in shapes for v in (m, n, k)], dtype=torch.int32, device=gpu)
-    lds = torch.tensor([v for m, n, k in shapes for v in (k, n, n)], dtype=torch.int32, device=gpu)
-    rc = _lib.load().mi355_grouped_gemm(*(t.data_ptr() for t in tables), sizes.data_ptr(), lds.data_ptr(), len(shapes),
-                                        _lib.F16 if dtype == "fp16" else _lib.BF16, nprog, torch.cuda.current_stream().cuda_stream)
-    assert rc == 0 and all(torch.equal(c, d) for c, d in zip(outs, again))
+    assert all(torch.equal(c, d) for c, d in zip(outs, _run_device_tables(gpu, ga, gb, dtype, nprog)))
 
 
 @pytest.mark.parametrize("extension", [True, False])
