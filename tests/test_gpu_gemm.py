@@ -641,11 +641,9 @@ def test_decode_shape_m16(gpu):
                                    (2048, 100, 256)])
 def test_skinny_16bit_kernel_is_bit_exact_on_integers(gpu, monkeypatch, dtype, shape):
     # at most 64 rows on one side (shapes of python/test/regression/test_performance.py:36-44): the
-    # streaming kernel (K split over the waves of a workgroup) for row-major and K-major B; M > 64
-    # with N <= 64 takes it with the operands swapped (a row-major B then needs N = 32 or 64; the
-    # other cases here fall through to the tile kernels); 65 .. 128 rows against at least 2048 on the other
-    # side run as two launches, 64 rows and the rest.  Every partial sum is an exact integer,
-    # so the result does not depend on how K is split.
+    # streaming kernel (K split over the waves of a workgroup) or the ring kernels, as the size rule has it, for row-major and
+    # K-major B; M > 64 with N <= 64 takes the former with the operands swapped (a row-major B then needs N = 32 or 64); 65 ..
+    # 128 rows: ring kernels.  Every partial sum is an exact integer, so the result does not depend on how K is split.
     M, N, K = shape
     rng = np.random.default_rng(M + 3 * N + 7 * K)
     a = rng.integers(-2, 3, size=(M, K)).astype(np.float32)
@@ -811,9 +809,9 @@ def test_row_major_fp8_b_under_every_tile_choice_with_addend_activation_and_fp8_
                                    (1024, 32, 256), (100, 2048, 64), (2048, 128, 64)])
 def test_fused_epilogues_of_the_reference_dot_test(gpu, dtype, shape):
     # add-matrix / add-rows / add-cols / softmax / chain-dot (python/test/unit/language/test_core.py:3128-3145)
-    # through mi355_gemm_epilogue: MFMA tile kernels, the any-stride kernel (100, 70, 50) and four skinny
-    # shapes (the streaming kernels add the addend in their own epilogue; the second one runs with the
-    # operands swapped, the last two as two launches of 64 rows and the rest).  Integer data: bit-exact.
+    # through the product's epilogues: MFMA tile kernels, the any-stride kernel (100, 70, 50) and four shapes of few
+    # rows or columns (the streaming kernel, which adds the addend in its own epilogue, and the ring kernels).  Integer data:
+    # bit-exact.
     M, N, K = shape
     rng = np.random.default_rng(M + N + K)
     a = rng.integers(-2, 3, size=(M, K)).astype(np.float32)
@@ -1198,11 +1196,9 @@ def test_c_rows_of_8_and_16_byte_alignment_through_the_c_abi(gpu, shape, pad):
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", ["fp16", "bf16"])
 @pytest.mark.parametrize("shape", [(16, 16384, 512), (7, 32768, 192), (32, 16448, 96), (1, 16384, 2048)])
-def test_skinny_kernel_with_64_columns_per_workgroup_is_bit_exact(gpu, dtype, shape):
-    # a row-major B wide enough that 64 columns per workgroup still cover the compute units (N / 64 >= 256): the
-    # form of the streaming kernel that fetches whole 128-byte lines of B - two column tiles per wave, eight waves
-    # splitting K, k rows with bit 1 set stored with their halves swapped.  Exact integer sums (K from 3 to 64
-    # stages, so some waves get none), every M class, an epilogue with the addend; N = 16448 has 257 workgroups.
+def test_few_rows_against_a_wide_row_major_b_are_bit_exact(gpu, dtype, shape):
+    # a row-major B with more columns than one round of the streaming kernel's workgroups: the ring kernels on 64-column tiles,
+    # several rounds of them.  Exact integer sums, every class of M, an epilogue with the addend; N = 16448 has 257 tiles.
     M, N, K = shape
     rng = np.random.default_rng(M + N + K)
     a = rng.integers(-2, 3, size=(M, K)).astype(np.float32)

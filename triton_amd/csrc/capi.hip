@@ -217,7 +217,7 @@ double stream_us(int M, int N, int64_t k_bytes, bool b_kmajor, int cus) {
   if (M <= 64 && !b_kmajor) return 2.5 + steps * std::max(0.2, 0.33 * fill);
   const int rows = std::min(M, N);
   if (rows > 32) return 5.0 + steps * std::max(0.17, 0.24 * fill);
-  return 3.5 + steps * (rows > 16 ? std::max(0.136, 0.21 * fill) : std::max(0.105, 0.18 * fill));
+  return rows > 16 ? 3.9 + steps * std::max(0.152, 0.235 * fill) : 3.5 + steps * std::max(0.105, 0.18 * fill);
 }
 
 // Splits of K that `mi355_gemm_splitk` takes by itself (1 = the plain call).
@@ -461,7 +461,7 @@ static int gemm_impl(const void* A, const void* B, void* C, int M, int N, int K,
       (knobs().skinny != UNSET || streams(M, N, p.k_bytes, es, b_kmajor, cus) || streams8(M, N, p.k_bytes, es, b_kmajor, cus))) {
     SkinnyArgs sk{};
     sk.K = K; sk.C = (char*)C; sk.a_scale = a_scale; sk.b_scale = b_scale;
-    sk.activation = activation; sk.out_dtype = out_dtype; sk.cus = device_info().cus;
+    sk.activation = activation; sk.out_dtype = out_dtype;
     bool y_kmajor = true, x_kmajor = true;
     if (M <= 64) {
       sk.X = (const char*)A; sk.Y = (const char*)B; sk.S = M; sk.L = N;

@@ -199,16 +199,10 @@ __device__ __forceinline__ void ring_pin(f32x4& c) {
 template <int NS, int L>
 __device__ __forceinline__ void ring_drain_wait(int left) {
 #if MI355_DEVICE_PASS
-  static_assert(NS == 4 || NS == 8, "ladders for these depths");
-  if constexpr (NS == 8)
-    asm volatile("s_cmp_lt_i32 %0, 8\n\ts_cbranch_scc1 ring_seven_%=\n\ts_waitcnt vmcnt(%1)\n\ts_branch ring_done_%=\n"
-                 "ring_seven_%=:\n\ts_cmp_lt_i32 %0, 6\n\ts_cbranch_scc1 ring_five_%=\n\ts_waitcnt vmcnt(%2)\n\ts_branch ring_done_%=\n"
-                 "ring_five_%=:\n\ts_cmp_lt_i32 %0, 4\n\ts_cbranch_scc1 ring_all_%=\n\ts_waitcnt vmcnt(%3)\n\ts_branch ring_done_%=\n"
-                 "ring_all_%=:\n\ts_waitcnt vmcnt(0)\nring_done_%=:" :: "s"(left), "i"(6 * L), "i"(4 * L), "i"(2 * L) : "memory", "scc");
-  else
-    asm volatile("s_cmp_lt_i32 %0, 4\n\ts_cbranch_scc1 ring_three_%=\n\ts_waitcnt vmcnt(%1)\n\ts_branch ring_done_%=\n"
-                 "ring_three_%=:\n\ts_cmp_lt_i32 %0, 3\n\ts_cbranch_scc1 ring_all_%=\n\ts_waitcnt vmcnt(%2)\n\ts_branch ring_done_%=\n"
-                 "ring_all_%=:\n\ts_waitcnt vmcnt(0)\nring_done_%=:" :: "s"(left), "i"(2 * L), "i"(L) : "memory", "scc");
+  static_assert(NS == 4, "the ladder of this depth");
+  asm volatile("s_cmp_lt_i32 %0, 4\n\ts_cbranch_scc1 ring_three_%=\n\ts_waitcnt vmcnt(%1)\n\ts_branch ring_done_%=\n"
+               "ring_three_%=:\n\ts_cmp_lt_i32 %0, 3\n\ts_cbranch_scc1 ring_all_%=\n\ts_waitcnt vmcnt(%2)\n\ts_branch ring_done_%=\n"
+               "ring_all_%=:\n\ts_waitcnt vmcnt(0)\nring_done_%=:" :: "s"(left), "i"(2 * L), "i"(L) : "memory", "scc");
 #endif
 }
 
