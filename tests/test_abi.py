@@ -70,6 +70,19 @@ def test_products_with_rows_too_far_apart_for_the_tile_kernels_copy_them():
     assert need(1, 1 << 22) == need(1, 80) == 2 * a_copy      # (a K-major B is always copied here: its rows are not whole chunks)
 
 
+def _workspace(M, N, K, dtype, kmajor=True, ldb=None):
+    """Bytes that matmul asks for (256 CUs, aligned operands): copies of unaligned rows and slices of a split K."""
+    b = (1, ldb or K) if kmajor else (ldb or N, 1)
+    return _lib.load().mi355_gemm_workspace(1 << 20, 1 << 21, M, N, K, K, 1, *b, dtype)
+
+
+def test_fp32_products_are_split_where_that_shortens_the_fullest_cu():
+    # tiles of 128x128 per CU times K steps per slice: no split of few steps or of nearly a round of tiles, remainders taken account of
+    for M, N, K, slices in ((2048, 1920, 256, 0), (2048, 1920, 2048, 0), (1536, 1536, 512, 0), (1536, 1536, 1024, 3), (1024, 1024, 1024, 4),
+                            (1024, 1408, 4096, 8), (512, 512, 8192, 16)):
+        assert _workspace(M, N, K, _lib.F32) == slices * 4 * M * N, (M, N, K)
+
+
 def test_matmul_preconditions_match_reference_messages():
     a = torch.zeros(4, 8, dtype=torch.float16)
     b = torch.zeros(6, 4, dtype=torch.float16)

@@ -243,9 +243,16 @@ int auto_splits(int M, int N, int64_t k_bytes, int in_dtype, bool b_kmajor, bool
   const long tiles = (long)((M + 127) / 128) * ((N + 127) / 128);
   const int ksteps = (int)((k_bytes + 63) / 64);
   long splits = tiles * 2 > cus || ksteps < 64 ? 1 : std::min<long>(std::min<long>(cus / tiles, ksteps / 16), 32);
-  // (fp32: bound by the fp32 MFMA rate alone, 2048 cycles per K step of a 128x128 tile - whatever puts more CUs to work
-  // wins, down to eight K steps a slice; 1024^3: 74 -> 24 us)
-  if (in_dtype == MI355_F32) splits = tiles >= cus || ksteps < 16 ? 1 : std::min<long>(std::min<long>((2 * cus + tiles - 1) / tiles, ksteps / 8), 32);
+  if (in_dtype == MI355_F32) {
+    // bound by the fp32 MFMA rate alone: a CU takes 1.05 us for a K step of every 128x128 tile that it has, so what counts is how
+    // many that is on the fullest CU; the slices' way through memory and the second launch come on top.  (A workgroup or two for every
+    // CU, whatever the remainder, was up to 1.6 times as long as the unsplit product: 2048 x 1920 x 256 40.7 us for 25.8; 1024 x 1408 x
+    // 4096 in six slices 149, in five 121, unsplit 271)
+    auto us = [&](long s) { return (double)((tiles * s + cus - 1) / cus) * ((ksteps + s - 1) / s) * 1.05 + (s > 1 ? 5.0 + (double)s * M * N * 8.0 / 6e6 : 0.0); };
+    splits = 1;
+    for (long s = 2; tiles < cus && s <= std::min<long>(32, ksteps / 8); s++)
+      if (us(s) < us(splits)) splits = s;
+  }
   splits = std::min<long>(splits, (64ll << 20) / std::max<int64_t>(1, 4ll * M * N));
   return splits >= 2 ? (int)splits : 1;
 }
