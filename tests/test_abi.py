@@ -83,6 +83,14 @@ def test_fp32_products_are_split_where_that_shortens_the_fullest_cu():
         assert _workspace(M, N, K, _lib.F32) == slices * 4 * M * N, (M, N, K)
 
 
+def test_rows_are_not_copied_for_a_single_short_step():
+    # K below 48 with rows of C that are no whole groups of four: the kernel of any strides (B's rows are not 16-byte chunks)
+    assert _workspace(4024, 5214, 16, _lib.F8E4M3, False, 5230) == 0
+    assert _workspace(5246, 2775, 30, _lib.F16, False) == 0
+    assert _workspace(5248, 1792, 28, _lib.F8E4M3, False) > 0
+    assert _workspace(2084, 2092, 63, _lib.F8E4M3, False) > 0
+
+
 def test_matmul_preconditions_match_reference_messages():
     a = torch.zeros(4, 8, dtype=torch.float16)
     b = torch.zeros(6, 4, dtype=torch.float16)

@@ -643,7 +643,7 @@ struct GemmRoute {
 
 size_t up(size_t v, size_t to) { return (v + to - 1) / to * to; }
 
-GemmRoute gemm_route(const void* A, const void* B, int M, int N, int K, int64_t sam, int64_t sak, int64_t sbk, int64_t sbn, int in_dtype) {
+GemmRoute gemm_route(const void* A, const void* B, int M, int N, int K, int64_t sam, int64_t sak, int64_t sbk, int64_t sbn, int in_dtype, bool addend) {
   GemmRoute r;
   r.k = K;
   const int es = elem_size(in_dtype), vec = 16 / es, cus = device_info().cus > 0 ? device_info().cus : 256;
@@ -664,6 +664,10 @@ GemmRoute gemm_route(const void* A, const void* B, int M, int N, int K, int64_t 
   if (es == 4 || sak != 1 || sam < K || (sbk == 1) == (sbn == 1)) return r;
   r.kmajor = sbk == 1;
   if (r.kmajor ? sbn < K : sbk < N) return r;
+  // K is a single step of the any-stride kernel, and rows of C that are no whole groups of four or an addend make the tile kernels'
+  // epilogues slow: the copies do not pay (us, that kernel / padded copies: 4024 x 5214 x 16 e4m3 49 / 78, 5246 x 2775 x 30 fp16 31 / 53, 520 x
+  // 3873 x 32 8.7 / 11.6, 5164 x 2532 x 24 26 / 22 but 35 / 45 with an addend; whole groups of four: 5248 x 1792 x 28 e4m3 27 / 15)
+  if (K < 48 && (int64_t)M * N * K < 1 << 30 && (N % 4 != 0 || addend)) return r;
   // (what stays in place has rows within the kernels' lane offsets, as in gemm_impl: only their kernels know k_rows)
   const int64_t a_most = 1 << 23, b_most = r.kmajor ? 1 << 23 : 1 << 26;
   const bool a_stays = a_ok && sam * es < a_most, b_stays = r.kmajor ? bk_ok && sbn * es < b_most : bn_ok && sbk * es < b_most;
@@ -710,7 +714,7 @@ GemmRoute gemm_route(const void* A, const void* B, int M, int N, int K, int64_t 
 int64_t mi355_gemm_workspace(const void* A, const void* B, int M, int N, int K,
                              int64_t sam, int64_t sak, int64_t sbk, int64_t sbn, int in_dtype) {
   if (M <= 0 || N <= 0 || K <= 0 || in_dtype < MI355_F16 || in_dtype > MI355_F32) return 0;
-  const GemmRoute r = gemm_route(A, B, M, N, K, sam, sak, sbk, sbn, in_dtype);
+  const GemmRoute r = gemm_route(A, B, M, N, K, sam, sak, sbk, sbn, in_dtype, false);
   return (int64_t)(r.a_bytes + r.b_bytes + r.slice_bytes);
 }
 
@@ -728,7 +732,7 @@ int mi355_gemm_ws(const void* A, const void* B, void* C, int M, int N, int K,
     return mi355_gemm_epilogue(A, B, C, M, N, K, sam, sak, sbk, sbn, scm, scn, in_dtype, out_dtype, a_scale, b_scale,
                                addend, sdm, sdn, addend_dtype, activation, softmax, stream_);
   if (addend && addend_dtype != MI355_F16 && addend_dtype != MI355_BF16 && addend_dtype != MI355_F32) return MI355_EDTYPE;
-  const GemmRoute r = gemm_route(A, B, M, N, K, sam, sak, sbk, sbn, in_dtype);
+  const GemmRoute r = gemm_route(A, B, M, N, K, sam, sak, sbk, sbn, in_dtype, addend != nullptr);   // (with an addend no more than without)
   if (!workspace || !aligned(workspace, 256) || workspace_bytes < r.a_bytes + r.b_bytes + r.slice_bytes) return MI355_EINVAL;
   const int es = elem_size(in_dtype);
   char* ws = (char*)workspace;
