@@ -91,6 +91,11 @@ def test_rows_are_not_copied_for_a_single_short_step():
     assert _workspace(2084, 2092, 63, _lib.F8E4M3, False) > 0
 
 
+def test_few_rows_are_split_where_that_pays_for_the_second_launch():
+    for M, N, K, slices in ((16, 320, 4704, 0), (64, 2048, 2048, 0), (16, 8192, 8192, 0), (64, 8192, 8192, 2), (32, 4096, 4096, 4)):
+        assert _workspace(M, N, K, _lib.F16) == slices * 4 * M * N, (M, N, K)
+
+
 def test_matmul_preconditions_match_reference_messages():
     a = torch.zeros(4, 8, dtype=torch.float16)
     b = torch.zeros(6, 4, dtype=torch.float16)

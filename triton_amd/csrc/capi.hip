@@ -233,8 +233,10 @@ int auto_splits(int M, int N, int64_t k_bytes, int in_dtype, bool b_kmajor, bool
                                 : std::min(ring_plan(M, N, steps, cus, 1, 1).us,
                                            tiles256_us((long)((M + 255) / 256) * ((N + 255) / 256), 256, steps, cus, false, elem_size(in_dtype) == 1));
     const RingPlan split = ring_plan(M, N, steps, cus, 2, most);
-    // (columns that are not groups of four are added up one by one: 8192 x 33 x 8192 e4m3 19.0 us, in two slices 22.1)
-    return split.us + (few && N % 4 != 0 ? 1.5 : 0.0) < (stream ? 0.85 : 0.95) * plain ? split.splits : 1;
+    // (columns that are not groups of four are added up one by one: 8192 x 33 x 8192 e4m3 19.0 us, in two slices 22.1;
+    // and the few workgroups that add up many slices take 0.4 us for each: 16 x 320 x 4704 fp16 9.1 us, in nine slices 10.2)
+    const double sums = few ? (N % 4 != 0 ? 1.5 : 0.0) + 0.4 * std::max(0, split.splits - 4) : 0.0;
+    return split.us + sums < (stream ? 0.8 : 0.95) * plain ? split.splits : 1;
   }
   // the one-barrier-per-step kernel on 128x128 tiles, 64-byte K steps: a workgroup per CU, at least sixteen K steps each, at most
   // 32 slices; nothing to gain from half a round of tiles on or below 64 K steps
