@@ -1472,6 +1472,26 @@ def test_rows_too_far_apart_for_the_tile_kernels(gpu):
     assert bits_equal(to_np(triton_amd.matmul(from_np(a, "bf16", gpu), rows[:K], out_dtype=torch.float32)), a @ b)
 
 
+@pytest.mark.parametrize("dtype", ["fp16", "bf16", "e4m3"])
+@pytest.mark.parametrize("M,N,K", [(2176, 2176, 64), (2176, 2176, 192), (2150, 2168, 40), (1664, 4100, 16), (1536, 1536, 128), (3456, 3584, 96)])
+def test_short_k_on_two_128x128_tiles_per_cu(gpu, dtype, M, N, K):
+    # more 128x128 tiles than CUs and at most 384 bytes of K, whole tiles from half as many on: the kernel of one barrier per 64-byte step;
+    # with an addend the ring kernels.  K of one chunk, of a step and a chunk, of whole steps; exact sums
+    rng = np.random.default_rng(M + K)
+    a = rng.integers(-2, 3, size=(M, K)).astype(np.float32)
+    b = rng.integers(-2, 3, size=(K, N)).astype(np.float32)
+    if dtype == "e4m3":
+        K8 = (K + 15) // 16 * 16   # (rows of whole 16-byte chunks)
+        a, b = np.pad(a, ((0, 0), (0, K8 - K))), np.pad(b, ((0, K8 - K), (0, 0)))
+        put = lambda x: torch.from_numpy(formats.encode_fp8(np.ascontiguousarray(x), dtype)).to(gpu).view(torch.float8_e4m3fn)   # noqa: E731
+    else:
+        put = lambda x: from_np(x, dtype, gpu)   # noqa: E731
+    ref, ta, row = a @ b, put(a), torch.arange(N, device=gpu, dtype=torch.float32)
+    for tb in (put(b), put(b.T).t()):
+        assert bits_equal(to_np(triton_amd.matmul(ta, tb, out_dtype=torch.float32)), ref), tb.stride()
+        assert bits_equal(to_np(triton_amd.matmul(ta, tb, out_dtype=torch.float32, add=row)), ref + np.arange(N, dtype=np.float32)), tb.stride()
+
+
 @pytest.mark.parametrize("kmajor", [False, True])
 @pytest.mark.parametrize("M,N,K", [(4096, 4097, 1032), (4096, 4160, 1024), (4160, 4096, 1024), (4097, 4095, 1024), (4096, 4161, 1024)])
 def test_columns_or_rows_beyond_whole_tiles_in_a_call_of_their_own(gpu, M, N, K, kmajor):

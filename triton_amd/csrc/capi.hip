@@ -178,6 +178,18 @@ double tiles256_us(long tiles, int rows, int steps, int cus, bool edges, bool fp
   return kLaunchUs + (double)rounds * share * ((edges ? 8.0 : 6.0) + (edges && !fp8 ? 1.6 : 1.43) * (0.25 + 0.75 * fill) * steps);
 }
 
+// Products of a short K whose 128x128 tiles are more than the CUs: the kernel of one barrier per 64-byte step on those tiles, two
+// workgroups on a CU where a ring leaves room for one.  Measured over 16 .. 1280 tiles and K bytes of 16 .. 2048, this kernel / ring or
+// 256x256 tiles, us: 2688 x 2688 x 64 fp16 8.2 / 11.5, x 192 11.5 / 13.2, x 256 12.4 / 13.0; e4m3 x 384 10.6 / 12.6, x 512 12.3 / 12.7; row-major B, x 256
+// 12.0 / 13.6; edges cost it more (2659 x 2656 x 64 9.4 / 11.4, x 192 12.2 / 13.0).  Up to half as many tiles, whole ones only (1792 x 1920 x 64 6.0 / 7.1, 1763 x 1888
+// 1.06).  Not where one round of 256x256 tiles fills the CUs (3840 x 4096 x 16 1.1).
+bool short_k(int M, int N, int k_bytes, bool b_kmajor, int cus) {
+  const long tiles = (long)((M + 127) / 128) * ((N + 127) / 128), tiles256 = (long)((M + 255) / 256) * ((N + 255) / 256);
+  if (tiles256 <= cus && tiles256 * 10 >= cus * 9) return false;
+  if (tiles > cus) return k_bytes <= (!b_kmajor && tiles * 4 <= cus * 7 ? 512 : 384);
+  return M % 128 == 0 && N % 128 == 0 && k_bytes <= 256 && tiles * 2 > cus;
+}
+
 // Operands as the ring kernels want them, on top of what every tile kernel asks (16-byte chunks): 16-bit with either layout
 // of B, fp8 with a K-major one.
 bool ring_ok(int elem_bytes, bool b_kmajor) { return elem_bytes == 2 || (elem_bytes == 1 && b_kmajor); }
@@ -487,15 +499,17 @@ static int gemm_impl(const void* A, const void* B, void* C, int M, int N, int K,
     if (is8 && b_kmajor && !aux && gemm8_skinny_ok(p)) return gemm8_skinny_launch(p, in_dtype == MI355_F8E5M2, stream);
   }
   // the ring kernels of 64 .. 128-row tiles where they are the faster ones by the two estimates above (and in place of the
-  // other 128x128 kernel wherever they take the operands)
+  // other 128x128 kernel but for the short K above)
   int ring = -1;
   if (can_ring) {
     const bool by_knob = tile_arg >= 0 || knobs().tile != UNSET;
     if (k_rows > 0) {   // a row-major B that ends before A's padding does: the ring kernels know
       ring = ring_plan(M, N, ksteps128, cus, 1, 1).shape;
       p.K = k_rows;
-    } else if (tile == 1) ring = by_knob ? 0 : ring_plan(M, N, ksteps128, cus, 1, 1).shape;
+    } else if (!by_knob && tile != 6 && !aux && p.c_vec_ok && short_k(M, N, p.k_bytes, b_kmajor, cus)) tile = 1;   // (its addends and odd rows of C cost more)
+    else if (tile == 1) ring = by_knob ? 0 : ring_plan(M, N, ksteps128, cus, 1, 1).shape;
     else if (tile >= 8 && tile <= 10) ring = tile - 8;
+    else if (tile == 11) tile = 1;   // the one-barrier-per-step kernel on 128x128 tiles
     else if (!by_knob && knobs().tile_m == UNSET && knobs().mixed_rows == UNSET) {
       const int rows = tile == 6 && p.tile_m ? p.tile_m : 256;
       const RingPlan plan = ring_plan(M, N, ksteps128, cus, 1, 1);

@@ -8,7 +8,7 @@ template <typename V8>
 struct Cfg16 {
   using Operand = V8;
   static constexpr int kSteps = 2, kChunks = 1;
-  static constexpr bool kRowMajorB = true, kScaled = false, kRing = true;
+  static constexpr bool kRowMajorB = true, kScaled = false;
   static constexpr int kElemBytes = 2;
   static constexpr int kStepsPerScaleDword = 1;
   // no block scales: placeholders so that generic code naming them compiles

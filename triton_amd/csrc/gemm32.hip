@@ -12,7 +12,7 @@ namespace mi355 {
 struct Cfg32 {
   using Operand = f32x4;
   static constexpr int kSteps = 2, kChunks = 1;
-  static constexpr bool kRowMajorB = false, kScaled = false, kRing = false;
+  static constexpr bool kRowMajorB = false, kScaled = false;
   static constexpr int kElemBytes = 4;
   static constexpr int kStepsPerScaleDword = 1;
   __device__ static int scale_dword_offset(int) { return 0; }

@@ -13,7 +13,7 @@ template <int FMT>  // 0 = e4m3fn, 1 = e5m2 (cbsz / blgp encoding of the instruc
 struct Cfg8 {
   using Operand = i32x8;
   static constexpr int kSteps = 1, kChunks = 2;
-  static constexpr bool kRowMajorB = true, kScaled = false, kRing = true;   // (row-major B: the one-barrier-per-step kernel only)
+  static constexpr bool kRowMajorB = true, kScaled = false;   // (row-major B: the one-barrier-per-step kernel only)
   static constexpr int kElemBytes = 1;
   static constexpr int kStepsPerScaleDword = 1;
   // no block scales: placeholders so that generic code naming them compiles

@@ -27,7 +27,6 @@
 //                     one-barrier-per-step form)
 //   kElemBytes        bytes per element of a row-major B (2 or 1; unused without kRowMajorB)
 //   kScaled           block-scaled: per-row e8m0 scales ride along (MX)
-//   kRing             the ring kernels (gemm_ring.h) take this type's products on tiles of 128 rows and fewer
 //   Operand           register type of one MFMA operand
 //   mma<ks>(...)      the MFMA itself
 #pragma once
@@ -1544,9 +1543,7 @@ static int launch_gemm_tile(const GemmArgs& p, int tile, hipStream_t stream) {
     if (tile >= 3 && whole) return launch_gemm_w4<Cfg, 4, B_KMAJOR, 4>(p, stream);
   }
   if (tile >= 3) tile = 2;
-  if constexpr (!Cfg::kRing) {   // (the ring kernels of gemm_ring.h have the smaller tiles of the other types)
-    if (tile == 1) return launch_gemm<Cfg, 128, 128, 2, 2, B_KMAJOR, 4>(p, stream);
-  }
+  if (tile == 1) return launch_gemm<Cfg, 128, 128, 2, 2, B_KMAJOR, 4>(p, stream);
   if (tile == 0 && p.k_bytes % (RBK * Cfg::kStepsPerScaleDword) == 0) return launch_gemm_pp<Cfg, 256, 256, B_KMAJOR, 4>(p, stream);
   return launch_gemm<Cfg, 256, 256, 2, 4, B_KMAJOR, 4>(p, stream);
 }
