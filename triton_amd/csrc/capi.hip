@@ -1138,7 +1138,8 @@ static int attn_fwd_variant(const AttnArgs& p, int cus) {
   // 16 x 1024: 6 10.4 / 10.5, 7 12.1 / 15.0, 8 12.9 / 12.8; head_dim 128: 6 15.7 / 16.3, 8 18.7 / 18.5, 1 20.9 / 20.6
   if (rows <= 64ll * cus) return 6;
   // 16 x 2048: 8 22.4 / 24.9, 6 24.0 / 27.0, 1 26.7 / 27.5; head_dim 128: 8 32.6 / 40.1, 6 32.2 / 50.6, 1 36.9 / 41.5
-  if (rows <= 128ll * cus) return 8;
+  // (two blocks of keys are not worth the groups' meeting: 256 x 128, no mask, head_dim 128: 8 10.2, 2 8.8; causal 8 ahead)
+  if (rows <= 128ll * cus && (p.causal || p.N > 128)) return 8;
   if (p.causal && rows <= 256ll * cus) {
     // (few, long rows of work under the mask) 32 x 2048: 6 34.1, 8 37.1, 2 38.4, 4 40.7; 8 x 8192: 6 102, 8 101, 4 142
     if (p.D == 64 && p.N >= 2048) return 6;
