@@ -942,16 +942,16 @@ int mi355_grouped_gemm_host(const void* const* a, const void* const* b, void* co
               (int64_t)l[0] * 16 + s[2] * 2 < (1ll << 31) && (int64_t)s[2] * l[1] * 2 + 512 < (1ll << 31);
       order[n++] = i;
     }
-    GroupedTable ga{};
-    auto put = [&](int at, int i) {
+    auto put = [&](GroupedTable& ga, int at, int i) {
       ga.a_ptrs[at] = (uint64_t)a[g0 + i]; ga.b_ptrs[at] = (uint64_t)b[g0 + i]; ga.c_ptrs[at] = (uint64_t)c[g0 + i];
       for (int e = 0; e < 3; e++) { ga.sizes[3 * at + e] = sizes[3 * (g0 + i) + e]; ga.lds[3 * at + e] = lds[3 * (g0 + i) + e]; }
     };
     int rc;
     if (nodd > 0) {
+      GroupedTable ga{};
       int64_t tiles = 0;
       for (int at = 0; at < nodd; at++) {
-        put(at, odd[at]);
+        put(ga, at, odd[at]);
         ga.first_tile[at] = (int)std::min<int64_t>(tiles, INT_MAX);
         tiles += (int64_t)((ga.sizes[3 * at] + 63) / 64) * ((ga.sizes[3 * at + 1] + 63) / 64);
       }
@@ -969,12 +969,12 @@ int mi355_grouped_gemm_host(const void* const* a, const void* const* b, void* co
       }
     }
     if (n == 0) continue;
-    ga = GroupedTable{};
+    GroupedTable ga{};
     ga.group_size = n; ga.out_dtype = dtype;
     ga.chunk = std::max(1, knob(knobs().grouped_chunk, 4));
     if (whole && knobs().grouped_wave128_min_k != 0 && tiles256 >= knob(knobs().grouped_big_min, cus)) {
       // whole 256x256 tiles, at least one per CU: runs of them as one stream of K steps
-      for (int at = 0; at < n; at++) put(at, order[at]);
+      for (int at = 0; at < n; at++) put(ga, at, order[at]);
       ga.total_tiles = (int)tiles256;
       rc = gemm_wave128_grouped_table_launch(ga, bf16, num_programs > 0 ? std::min(num_programs, cus) : cus, stream);
     } else {
@@ -986,7 +986,7 @@ int mi355_grouped_gemm_host(const void* const* a, const void* const* b, void* co
       int64_t tiles = 0;
       for (int at = 0; at < n; at++) {
         const int i = order[at], edge = pick ? pick : cost64[i] <= cost128[i] ? 64 : 128;
-        put(at, i);
+        put(ga, at, i);
         ga.first_tile[at] = (int)tiles;
         if (edge == 64) ga.small_tiles |= 1ull << at;
         tiles += (int64_t)((ga.sizes[3 * at] + edge - 1) / edge) * ((ga.sizes[3 * at + 1] + edge - 1) / edge);

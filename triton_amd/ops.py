@@ -312,8 +312,12 @@ def group_gemm_fn(group_A, group_B, *, num_programs: int = 0):
         assert A.dtype == B.dtype == group_A[0].dtype, "all matrices of a group share one dtype"
         assert A.stride(1) == 1 and B.stride(1) == 1, "matrices must be row major"
     ext = _lib.ext()
-    if ext is not None and all(isinstance(t, torch.Tensor) for t in (*group_A, *group_B)):
-        return ext.group_gemm(list(group_A), list(group_B), int(num_programs))
+    if ext is not None:
+        try:
+            return ext.group_gemm(list(group_A), list(group_B), int(num_programs))
+        except TypeError:   # (matrices of other libraries; looking at each one's type first costs a call more than a microsecond)
+            if all(isinstance(t, torch.Tensor) for t in (*group_A, *group_B)):
+                raise
     group_C = [torch.empty((A.shape[0], B.shape[1]), device=A.device, dtype=A.dtype) for A, B in zip(group_A, group_B)]
     live = [i for i, C in enumerate(group_C) if C.numel() > 0 and group_A[i].shape[1] > 0]
     for C in (group_C[i] for i in range(group_size) if i not in live):
