@@ -1506,3 +1506,60 @@ def test_columns_or_rows_beyond_whole_tiles_in_a_call_of_their_own(gpu, M, N, K,
     for shape in ((N,), (M, 1), (M, N)):
         add = torch.randint(-8, 9, shape, device=gpu, generator=g).to(torch.bfloat16)
         assert torch.equal(triton_amd.matmul(a, b, out_dtype=torch.float32, add=add), want + add.float()), shape
+
+
+@pytest.mark.parametrize("programs", [3, 256])
+@pytest.mark.parametrize("kmajor", [False, True])
+@pytest.mark.parametrize("dtype", ["fp16", "bf16", "e4m3"])
+def test_four_wave_kernels_on_tiles_moved_back_from_the_edges_are_bit_exact(gpu, monkeypatch, dtype, kmajor, programs):
+    # sizes that are no whole tiles: the last tiles lie partly over their neighbours, and with a row-major B the last columns
+    # of a tile may be padding.  One tile, one row or column more, a chunk more, odd rows of C, a K tail, every tile height;
+    # bias row, addend matrix, activation, fp32 / fp8 output.  Whole numbers: exact in every order
+    set_knob(monkeypatch, "MI355_GEMM_TILE", "6")
+    set_knob(monkeypatch, "MI355_GEMM_PROGRAMS", str(programs))
+    if dtype == "e4m3" and not kmajor:
+        pytest.skip("a row-major fp8 B of these sizes runs another kernel")
+    tdt = {"fp16": torch.float16, "bf16": torch.bfloat16, "e4m3": torch.float8_e4m3fn}[dtype]
+    out = torch.float16 if dtype != "bf16" else torch.bfloat16
+    g = torch.Generator(device=gpu).manual_seed(len(dtype) + kmajor)
+
+    def ints(*shape, top=2):
+        return torch.randint(-top, top + 1, shape, device=gpu, generator=g)
+
+    for M, N, K in ((256, 256, 256), (257, 256, 256), (256, 257, 512), (264, 264, 256), (511, 513, 256), (300, 1003, 640), (513, 519, 256 + 48)):
+        pitch = -(-N // 16) * 16
+        a = ints(M, K).to(tdt)
+        b = ints(N, K).to(tdt)
+        if kmajor:
+            tb = b.t()
+        else:
+            tb = torch.full((K, pitch), float("nan"), device=gpu, dtype=tdt)[:, :N]   # (what the padding holds is nobody's business)
+            tb.copy_(b.t())
+        want = a.float() @ b.t().float()
+        bias, addend = ints(N, top=8).to(out), ints(M, N, top=8).to(torch.float32)
+        assert torch.equal(triton_amd.matmul(a, tb, out_dtype=out).float(), want.to(out).float()), (M, N, K)
+        assert torch.equal(triton_amd.matmul(a, tb, out_dtype=torch.float32), want), (M, N, K)
+        assert torch.equal(triton_amd.matmul(a, tb, out_dtype=out, add=bias).float(), (want + bias.float()).to(out).float()), (M, N, K)
+        assert torch.equal(triton_amd.matmul(a, tb, out_dtype=torch.float32, add=addend), want + addend), (M, N, K)
+        got = triton_amd.matmul(a, tb, "leaky_relu", out_dtype=out, add=bias[:1].reshape(1, 1).expand(M, 1)).float()
+        ref = torch.nn.functional.leaky_relu(want + bias[0].float(), 0.01)
+        assert torch.allclose(got, ref, rtol=2 ** -8, atol=1e-3), (M, N, K)   # (0.01 x and the result rounded once each)
+    for rows in ("192", "128"):
+        set_knob(monkeypatch, "MI355_GEMM_TILE_M", rows)
+        for M, N, K in ((192, 256, 256), (200, 264, 512), (449, 520, 256)):
+            a, b = ints(M, K).to(tdt), ints(N, K).to(tdt)
+            tb = b.t() if kmajor else b.t().contiguous()
+            assert torch.equal(triton_amd.matmul(a, tb, out_dtype=out).float(), (a.float() @ b.t().float()).to(out).float()), (M, N, K, rows)
+
+
+def test_an_addend_that_is_c_is_added_once(gpu):
+    # in place through the C ABI: tiles that lie over their neighbours would add it twice
+    M, N, K = 5001, 5000, 256
+    g = torch.Generator(device=gpu).manual_seed(3)
+    a = torch.randint(-2, 3, (M, K), device=gpu, generator=g).to(torch.bfloat16)
+    b = torch.randint(-2, 3, (N, K), device=gpu, generator=g).to(torch.bfloat16)
+    c = torch.randint(-8, 9, (M, N), device=gpu, generator=g).to(torch.float32)
+    want = a.float() @ b.t().float() + c
+    rc = _lib.load().mi355_gemm_epilogue(a.data_ptr(), b.data_ptr(), c.data_ptr(), M, N, K, K, 1, 1, K, N, 1, _lib.BF16, _lib.F32, None, None,
+                                         c.data_ptr(), N, 1, _lib.F32, _lib.ACT_NONE, 0, torch.cuda.current_stream().cuda_stream)
+    assert rc == 0 and torch.equal(c, want)

@@ -4,6 +4,7 @@
 // launch on the caller's stream out, an integer status back.
 #include <algorithm>
 #include <cmath>
+#include <utility>
 #include <hip/hip_runtime.h>
 #include <stdlib.h>
 #include <string.h>
@@ -168,8 +169,8 @@ RingPlan ring_plan(int M, int N, int steps, int cus, int splits_lo, int splits_h
   return best;
 }
 
-// The same for the kernels of 256-column tiles with `rows` rows of C each (gemm_wave128.hip: whole tiles; edges: the
-// eight-wave kernel).  A K step of a 256-row tile is bound by its 64 KiB of operands: 1.43 us with all CUs at it, a quarter
+// The same for the kernels of 256-column tiles with `rows` rows of C each (gemm_wave128.hip; edges: the eight-wave kernel, for
+// what that one does not take).  A K step of a 256-row tile is bound by its 64 KiB of operands: 1.43 us with all CUs at it, a quarter
 // of that without the others' traffic.
 double tiles256_us(long tiles, int rows, int steps, int cus, bool edges, bool fp8) {
   const long rounds = (tiles + cus - 1) / cus;
@@ -269,6 +270,18 @@ int auto_splits(int M, int N, int64_t k_bytes, int in_dtype, bool b_kmajor, bool
   }
   splits = std::min<long>(splits, (64ll << 20) / std::max<int64_t>(1, 4ll * M * N));
   return splits >= 2 ? (int)splits : 1;
+}
+
+// Whether an addend's elements lie among C's (a call that adds in place).
+bool addend_in_c(const GemmArgs& p) {
+  if (!p.aux) return false;
+  auto span = [&](const void* at, int64_t sm, int64_t sn, int dtype) {   // (strides of either sign)
+    const int64_t m = (p.M - 1) * sm, n = (p.N - 1) * sn;
+    const char* first = (const char*)at + (std::min<int64_t>(m, 0) + std::min<int64_t>(n, 0)) * elem_size(dtype);
+    return std::pair<const char*, const char*>(first, (const char*)at + (std::max<int64_t>(m, 0) + std::max<int64_t>(n, 0) + 1) * elem_size(dtype));
+  };
+  const auto c = span(p.C, p.ldc, p.scn, p.out_dtype), d = span(p.aux, p.aux_sm, p.aux_sn, p.aux_dtype);
+  return d.first < c.second && c.first < d.second;
 }
 
 bool aligned(const void* p, size_t a) { return ((uintptr_t)p % a) == 0; }
@@ -398,19 +411,21 @@ static int gemm_impl(const void* A, const void* B, void* C, int M, int N, int K,
   // (an epilogue addend: instantiations of their own)
   // (fp8 from three quarters of a round: at 144 tiles the eight-wave kernel is 4-7 % ahead - 3072^3 1520 vs
   // 1450, 3072x3072x8192 2040 vs 1890 TFLOP/s -, at 196 tiles the four-wave one by 2 %, at 225 by 13 %)
-  const bool w128_ok = is8 ? gemm_wave128_f8_ok(p, b_kmajor) : gemm_wave128_ok(p, b_kmajor, in_dtype);
+  // (partial tiles are whole ones moved back over their neighbours: an addend that is C itself must be read only once)
+  const bool once = (M % 256 != 0 || N % 256 != 0) && addend_in_c(p);
+  const bool w128_ok = !once && (is8 ? gemm_wave128_f8_ok(p, b_kmajor) : gemm_wave128_ok(p, b_kmajor));
   if (tiles256 * (is8 ? 4 : 2) >= cus * (is8 ? 3 : 1) && w128_ok) tile = 6;
   tile = tile_arg >= 0 ? tile_arg : knob(knobs().tile, tile);
   // 16-bit products whose 256 x 256 tiles fill the last round of CUs badly (or whose M is a multiple of 192 only): the
   // same kernel on tiles of 192 x 256 where those use the CUs better (3072^3: 192 tiles instead of 144 for 256 CUs)
   if (!is8 && tile_arg < 0 && (knobs().tile == UNSET || knobs().tile_m == 192) && gemm_wave128_192_ok(p, b_kmajor, in_dtype)) {
     auto fill = [&](long t) { return t <= 0 ? 0.0 : (double)t / (double)(((t + cus - 1) / cus) * cus); };
-    const long tiles192 = (long)(M / 192) * (N / 256);
+    const long tiles192 = (long)((M + 191) / 192) * ((N + 255) / 256);
     const int want = knob(knobs().tile_m, 0);
     // (below half a round of 256-row tiles the 128-row tiles further down may fill better still: 3072 x 2048 x 4096 bf16,
     // 128 tiles of 192 rows 734 TFLOP/s, 192 tiles of 128 rows 815)
-    const long tiles128 = (long)(M / 128) * (N / 256);
-    const bool rather128 = tile == 1 && M % 128 == 0 && tiles128 <= cus && fill(tiles128) > fill(tiles192) &&
+    const long tiles128 = (long)((M + 127) / 128) * ((N + 255) / 256);
+    const bool rather128 = tile == 1 && tiles128 <= cus && fill(tiles128) > fill(tiles192) &&
                            gemm_wave128_192_ok(p, b_kmajor, in_dtype, 128);
     if (want == 192 || (want == 0 && !rather128 && tiles192 * 2 >= cus && (tile != 6 || fill(tiles192) > fill(tiles256) + 0.08))) {
       tile = 6;
@@ -424,7 +439,7 @@ static int gemm_impl(const void* A, const void* B, void* C, int M, int N, int K,
   // 4096 (420 / 560) 2185 / 1995
   if (is8 && tile_arg < 0 && (knobs().tile == UNSET || knobs().tile_m == 192) && gemm_wave128_f8_192_ok(p, b_kmajor)) {
     auto fill = [&](long t) { return t <= 0 ? 0.0 : (double)t / (double)(((t + cus - 1) / cus) * cus); };
-    const long tiles192 = (long)(M / 192) * (N / 256);
+    const long tiles192 = (long)((M + 191) / 192) * ((N + 255) / 256);
     const int want = knob(knobs().tile_m, 0);
     if (want == 192 || (want == 0 && tiles192 * 4 >= cus * 3 && (tile != 6 || fill(tiles192) > fill(tiles256) + 0.08))) {
       tile = 6;
@@ -436,7 +451,7 @@ static int gemm_impl(const void* A, const void* B, void* C, int M, int N, int K,
   // 2048 x 8192, 144 tiles: 650 -> 692; at half a round the 128 x 128 tiles stay ahead, 2048 x 2048 x 4096: 627 vs 569)
   if (!is8 && tile_arg < 0 && (knobs().tile == UNSET || knobs().tile_m == 128) && p.tile_m == 0 &&
       gemm_wave128_192_ok(p, b_kmajor, in_dtype, 128)) {
-    const long tiles128 = (long)(M / 128) * (N / 256);
+    const long tiles128 = (long)((M + 127) / 128) * ((N + 255) / 256);
     const int want = knob(knobs().tile_m, 0);
     if (want == 128 || (want == 0 && tile == 1 && tiles128 * 16 >= cus * 9 && tiles128 <= cus)) {
       tile = 6;
@@ -446,7 +461,7 @@ static int gemm_impl(const void* A, const void* B, void* C, int M, int N, int K,
   // fp8 likewise (measured: see the design notes' table of shapes)
   if (is8 && tile_arg < 0 && (knobs().tile == UNSET || knobs().tile_m == 128) && p.tile_m == 0 &&
       gemm_wave128_f8_192_ok(p, b_kmajor, 128)) {
-    const long tiles128 = (long)(M / 128) * (N / 256);
+    const long tiles128 = (long)((M + 127) / 128) * ((N + 255) / 256);
     const int want = knob(knobs().tile_m, 0);
     if (want == 128 || (want == 0 && tile == 1 && tiles128 * 16 >= cus * 9 && tiles128 <= cus)) {
       tile = 6;
@@ -522,7 +537,7 @@ static int gemm_impl(const void* A, const void* B, void* C, int M, int N, int K,
       // 50 / 38; edges on the other side too: 4095 x 4100 x 4100 168 / 151.  No round saved, one part: 2048 x 2052 x 4096, 6150 x 6144 x 4096.
       const double one = std::min(plan.us, other);
       auto parts_us = [&](int m, int n, int m2, int n2) {
-        const bool edges = m % 256 != 0 || n % 256 != 0 || p.k_bytes % 128 != 0;
+        const bool edges = tile != 6 || m < 256 || n < 256;
         const long tiles = (long)((m + 255) / 256) * ((n + 255) / 256);
         return std::min(ring_plan(m, n, ksteps128, cus, 1, 1).us, tiles256_us(tiles, 256, ksteps128, cus, edges, is8)) +
                ring_plan(m2, n2, ksteps128, cus, 1, 1).us;
@@ -553,7 +568,7 @@ static int gemm_impl(const void* A, const void* B, void* C, int M, int N, int K,
   // 6: four waves, 128x128 of C per wave from 16x16x32 MFMAs (whole tiles)
   // (a tile height of 192 / 128 rows was set above only after gemm_wave128_192_ok had accepted the shape for it)
   if (mixed_rows > 0 && !is8) return gemm_wave128_mixed_launch(p, mixed_rows, in_dtype == MI355_BF16, b_kmajor, stream);
-  if (tile == 6 && (p.tile_m == 192 || p.tile_m == 128 || gemm_wave128_ok(p, b_kmajor, in_dtype))) return gemm_wave128_launch(p, in_dtype == MI355_BF16, b_kmajor, stream);
+  if (tile == 6 && (p.tile_m == 192 || p.tile_m == 128 || w128_ok)) return gemm_wave128_launch(p, in_dtype == MI355_BF16, b_kmajor, stream);
   return gemm16_launch(p, in_dtype == MI355_BF16, b_kmajor, tile, stream);
 }
 
@@ -691,7 +706,8 @@ GemmRoute gemm_route(const void* A, const void* B, int M, int N, int K, int64_t 
   auto copy_us = [&](bool a, bool b) { return 2.0 + 2.0 * es * ((a ? (double)M * K : 0.0) + (b ? (double)N * K : 0.0)) / 4.5e6; };
   const int steps = (int)(((int64_t)K * es + 127) / 128);
   const double ring = ring_ok(es, r.kmajor) ? ring_plan(M, N, steps, cus, 1, 1).us : 1e30;
-  const double any = std::min(ring, tiles256_us((long)((M + 255) / 256) * ((N + 255) / 256), 256, steps, cus, true, es == 1));
+  const long tiles256 = (long)((M + 255) / 256) * ((N + 255) / 256);
+  const double any = std::min(ring, tiles256_us(tiles256, 256, steps, cus, M < 256 || N < 256, es == 1));
   r.pack_a = !a_stays;
   // a row-major B with good rows only lacks the zero rows beyond K, which the ring kernels do not read
   r.pack_b = !b_stays || (!r.kmajor && K % vec != 0 && ring + copy_us(!a_stays, false) > any + copy_us(!a_stays, true));
@@ -704,7 +720,9 @@ GemmRoute gemm_route(const void* A, const void* B, int M, int N, int K, int64_t 
     return r;
   }
   if (K % vec != 0) {
-    r.k = (int)up(K, r.pack_b || r.kmajor ? 128 / es : vec);
+    // (whole pairs of 128-byte K steps where the 256 x 256 tiles are at least half a round: no tail behind their loop)
+    const int to = tiles256 * 2 >= cus && (int64_t)K * es >= 1024 ? 256 : 128;
+    r.k = (int)up(K, r.pack_b || r.kmajor ? to / es : vec);
     if (!r.kmajor && !r.pack_b) r.k_rows = K;
   }
   if (r.pack_a) {
@@ -1051,7 +1069,7 @@ int mi355_mx_gemm(const uint8_t* A, const uint8_t* sA, const uint8_t* B, const u
   // 360 / 491, 644 / 856, 627 / 754, 1072 / 1244, 947 / 1120; beyond one round they lose (3072^3, 288 tiles: MXFP4 2084 for
   // the 192-row tiles / 1555, 4096^3 3209 / 2834)
   if ((knobs().tile == UNSET || knobs().tile_m == 128) && gemm_wave128_mx_192_ok(p, fmt == MI355_MXFP4 ? 512 : 1024, 128)) {
-    const long tiles128 = (long)(M / 128) * (N / 256);
+    const long tiles128 = (long)((M + 127) / 128) * ((N + 255) / 256);
     const int want = knob(knobs().tile_m, 0);
     if (want == 128 || (want == 0 && tiles128 >= 16 && tiles128 <= cus)) {
       tile = 6;
@@ -1064,7 +1082,7 @@ int mi355_mx_gemm(const uint8_t* A, const uint8_t* sA, const uint8_t* B, const u
   // 1945 / 2345, 519 / 630; not taken where they fill worse (3840 x 3840 x 4096: 3080 / 2230)
   if ((knobs().tile == UNSET || knobs().tile_m == 192) && p.tile_m == 0 && gemm_wave128_mx_192_ok(p, fmt == MI355_MXFP4 ? 512 : 1024)) {
     auto fill = [&](long t) { return t <= 0 ? 0.0 : (double)t / (double)(((t + cus - 1) / cus) * cus); };
-    const long tiles192 = (long)(M / 192) * (N / 256);
+    const long tiles192 = (long)((M + 191) / 192) * ((N + 255) / 256);
     const int want = knob(knobs().tile_m, 0);
     const bool enough192 = tiles192 * 2 >= cus || (tiles192 >= 16 && p.k_bytes >= 1024);
     if (want == 192 || (want == 0 && enough192 && (tile != 6 || fill(tiles192) > fill(tiles256) * 1.1))) {

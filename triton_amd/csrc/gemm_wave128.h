@@ -65,77 +65,141 @@ static inline int wave128_grid(int tiles, int cap) {
   return (tiles + rounds - 1) / rounds;
 }
 
-// AuxT: element type of the addend of the fused epilogues (void = none).  With an addend the kernels are
-// separate instantiations: its arguments cost the plain kernels scalar registers that they need for their
-// load bases.  `aux_vec`: the four addend elements of a lane are consecutive and aligned (one load).
-template <int MT, int NT, typename AuxT>
-__device__ __forceinline__ void gemm_epilogue16_impl(f32x4 (&acc)[MT][NT], const GemmArgs& p, int mrow0, int ncol0, int l16, int kg) {
-  constexpr bool AUX = !std::is_void<AuxT>::value;
-  using AuxE = std::conditional_t<AUX, AuxT, float>;
-  typedef AuxE Aux4 __attribute__((ext_vector_type(4)));
+// Exchange between the lane pairs (kg, kg ^ 1): see gemm_epilogue16_lean.
+__device__ __forceinline__ void swap16(int& a, int& b) {
+#if MI355_DEVICE_PASS
+  asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(a), "+v"(b));
+#endif
+}
+
+// Scales, addend, activation and any N, one row of 16x16 tiles at a time, every option behind one uniform branch per row.
+// ANY = false: C in a 16-bit type with unit column stride, the addend (if any) a row of N consecutive values - a bias, read
+// once for all rows of the lane (rows_epilogue).  C leaves as 16 bytes per lane (gemm_epilogue16_lean) whatever its alignment:
+// the memory pipeline splits what it has to.  ANY = true: every output type, strides and addend that the C ABI takes.
+// Columns from p.N on are left out; they can only be the last seven of the wave's 128, the padding that a tile of a
+// row-major B may end in, so that only the last columns are looked at.
+template <int MT, int NT, bool ANY>
+__device__ __forceinline__ void gemm_epilogue16(f32x4 (&acc)[MT][NT], const GemmArgs& p, int mrow0, int ncol0, int l16, int kg) {
+  static_assert(NT % 2 == 0, "pairs of 16-column tiles");
   float alpha = 1.f;
   if (p.a_scale) alpha *= *p.a_scale;
   if (p.b_scale) alpha *= *p.b_scale;
-  const bool leaky = p.activation == 1;
-  const bool aux_vec = AUX && p.aux_sn == 1 && p.aux_sm % 4 == 0 && (uintptr_t)p.aux % 16 == 0;
+  // columns of the lane's four that exist, for tile j
+  auto columns = [&](auto J_) { return decltype(J_)::value == NT - 1 ? min(p.N - (ncol0 + decltype(J_)::value * 16 + kg * 4), 4) : 4; };
+  // r += the addend at `off` (its row's first element)
+  auto add_row = [&](f32x4 (&r)[NT], int64_t off) {
+    auto typed = [&](auto* aux) {
+      using AuxT = std::remove_const_t<std::remove_pointer_t<decltype(aux)>>;
+      typedef AuxT Aux4 __attribute__((ext_vector_type(4), aligned(sizeof(AuxT))));
+      auto* const at = aux + off + (int64_t)(ncol0 + kg * 4) * p.aux_sn;
+      if (!ANY || p.aux_sn == 1) {
+        static_for<NT>([&](auto J_) {
+          constexpr int j = decltype(J_)::value;
+          const int count = columns(J_);
+          if (j < NT - 1 || count == 4) {
+            const Aux4 t = *(const Aux4*)(at + j * 16);
+#pragma unroll
+            for (int e = 0; e < 4; e++) r[j][e] += (float)t[e];
+          } else {
+#pragma unroll
+            for (int e = 0; e < 3; e++)
+              if (e < count) r[j][e] += (float)at[j * 16 + e];
+          }
+        });
+      } else {
+        static_for<NT>([&](auto J_) {
+          constexpr int j = decltype(J_)::value;
+          const int count = columns(J_);
+#pragma unroll
+          for (int e = 0; e < 4; e++)
+            if (j < NT - 1 || e < count) r[j][e] += (float)at[(j * 16 + e) * p.aux_sn];
+        });
+      }
+    };
+    if (p.aux_dtype == 4) typed((const float*)p.aux);
+    else if (p.aux_dtype == 1) typed((const __bf16*)p.aux);
+    else typed((const _Float16*)p.aux);
+  };
+  f32x4 bias[ANY ? 1 : NT];
+  if constexpr (!ANY) {
+    static_for<NT>([&](auto J_) { bias[decltype(J_)::value] = f32x4{0.f, 0.f, 0.f, 0.f}; });
+    if (p.aux) add_row(bias, 0);
+  }
   static_for<MT>([&](auto I_) {
     constexpr int i = decltype(I_)::value;
     const int m = mrow0 + i * 16 + l16;
-    static_for<NT>([&](auto J_) {
-      constexpr int j = decltype(J_)::value;
-      const int n = ncol0 + j * 16 + kg * 4;
-      float v[4];
-#pragma unroll
-      for (int e = 0; e < 4; e++) v[e] = acc[i][j][e] * alpha;
-      if constexpr (AUX) {
-        const AuxE* ax = (const AuxE*)p.aux + (int64_t)m * p.aux_sm + (int64_t)n * p.aux_sn;
-        if (aux_vec) {
-          const Aux4 t = *(const Aux4*)ax;
-#pragma unroll
-          for (int e = 0; e < 4; e++) v[e] += (float)t[e];
-        } else {
-#pragma unroll
-          for (int e = 0; e < 4; e++) v[e] += (float)ax[e * p.aux_sn];
-        }
-      }
-      if (leaky) {
+    f32x4 r[NT];
+    static_for<NT>([&](auto J_) { r[decltype(J_)::value] = acc[i][decltype(J_)::value] * alpha; });
+    if (p.aux) {
+      if constexpr (ANY) add_row(r, (int64_t)m * p.aux_sm);
+      else static_for<NT>([&](auto J_) { r[decltype(J_)::value] += bias[decltype(J_)::value]; });
+    }
+    if (p.activation == 1)
+      static_for<NT>([&](auto J_) {
+        f32x4& v = r[decltype(J_)::value];
 #pragma unroll
         for (int e = 0; e < 4; e++) v[e] = v[e] >= 0.f ? v[e] : 0.01f * v[e];
-      }
-      if (p.out_dtype == 2 || p.out_dtype == 3) {
-        store4_fp8(p.C, (int64_t)m * p.ldc + (int64_t)n * p.scn, p.scn, p.out_dtype, v, p.c_vec_ok, 4);
-      } else if (p.out_dtype == 4) {
-        float* c = (float*)p.C + (int64_t)m * p.ldc + (int64_t)n * p.scn;
-        if (p.c_vec_ok) *(f32x4*)c = f32x4{v[0], v[1], v[2], v[3]};
-        else {
+      });
+    if (!ANY || ((p.out_dtype == 0 || p.out_dtype == 1) && p.scn == 1)) {
+      int h[NT][2];   // the row in C's type, two columns a register
+      auto round = [&](auto x) {
+        using OutT = decltype(x);
+        typedef OutT Out2 __attribute__((ext_vector_type(2)));
+        static_for<NT>([&](auto J_) {
+          constexpr int j = decltype(J_)::value;
+          h[j][0] = __builtin_bit_cast(int, Out2{(OutT)r[j][0], (OutT)r[j][1]});
+          h[j][1] = __builtin_bit_cast(int, Out2{(OutT)r[j][2], (OutT)r[j][3]});
+        });
+      };
+      if (p.out_dtype == 1) round((__bf16)0.f);
+      else round((_Float16)0.f);
+      typedef int Chunk __attribute__((ext_vector_type(4), aligned(2)));
+      const int col = ncol0 + 4 * (kg & 2) + 16 * (kg & 1);
+      short* const row = (short*)p.C + (int64_t)m * p.ldc + col;
+      static_for<NT / 2>([&](auto J_) {
+        constexpr int j = 2 * decltype(J_)::value;
+        swap16(h[j][0], h[j + 1][0]);
+        swap16(h[j][1], h[j + 1][1]);
+        const int w[4] = {h[j][0], h[j][1], h[j + 1][0], h[j + 1][1]};
+        const int count = p.N - (col + j * 16);
+        if (j < NT - 2 || count >= 8) {
+          *(Chunk*)(row + j * 16) = Chunk{w[0], w[1], w[2], w[3]};
+        } else {
 #pragma unroll
-          for (int e = 0; e < 4; e++) c[e * p.scn] = v[e];
+          for (int e = 0; e < 7; e++)
+            if (e < count) row[j * 16 + e] = (short)(w[e / 2] >> (16 * (e & 1)));
         }
-      } else if (p.out_dtype == 1) {
-        __bf16* c = (__bf16*)p.C + (int64_t)m * p.ldc + (int64_t)n * p.scn;
-        if (p.c_vec_ok) *(bf16x4*)c = bf16x4{(__bf16)v[0], (__bf16)v[1], (__bf16)v[2], (__bf16)v[3]};
-        else {
+      });
+      return;
+    }
+    if constexpr (ANY)
+      static_for<NT>([&](auto J_) {
+        constexpr int j = decltype(J_)::value;
+        const int n = ncol0 + j * 16 + kg * 4, count = columns(J_);
+        const int64_t at = (int64_t)m * p.ldc + (int64_t)n * p.scn;
+        const float v[4] = {r[j][0], r[j][1], r[j][2], r[j][3]};
+        if (p.out_dtype == 2 || p.out_dtype == 3) {
+          if (count > 0) store4_fp8(p.C, at, p.scn, p.out_dtype, v, p.c_vec_ok && n % 4 == 0, count);
+        } else if (p.out_dtype == 4) {
+          typedef float Four __attribute__((ext_vector_type(4), aligned(4)));
+          if (p.scn == 1 && count == 4) *(Four*)((float*)p.C + at) = r[j];
+          else {
 #pragma unroll
-          for (int e = 0; e < 4; e++) c[e * p.scn] = (__bf16)v[e];
-        }
-      } else {
-        _Float16* c = (_Float16*)p.C + (int64_t)m * p.ldc + (int64_t)n * p.scn;
-        if (p.c_vec_ok) *(f16x4*)c = f16x4{(_Float16)v[0], (_Float16)v[1], (_Float16)v[2], (_Float16)v[3]};
-        else {
+            for (int e = 0; e < 4; e++)
+              if (e < count) ((float*)p.C)[at + e * p.scn] = v[e];
+          }
+        } else {
 #pragma unroll
-          for (int e = 0; e < 4; e++) c[e * p.scn] = (_Float16)v[e];
+          for (int e = 0; e < 4; e++)
+            if (e < count) ((short*)p.C)[at + e * p.scn] = p.out_dtype == 1 ? __builtin_bit_cast(short, (__bf16)v[e]) : __builtin_bit_cast(short, (_Float16)v[e]);
         }
-      }
-    });
+      });
   });
 }
 
-template <int MT, int NT, bool AUX = false>
-__device__ __forceinline__ void gemm_epilogue16(f32x4 (&acc)[MT][NT], const GemmArgs& p, int mrow0, int ncol0, int l16, int kg) {
-  if constexpr (!AUX) gemm_epilogue16_impl<MT, NT, void>(acc, p, mrow0, ncol0, l16, kg);
-  else if (p.aux_dtype == 4) gemm_epilogue16_impl<MT, NT, float>(acc, p, mrow0, ncol0, l16, kg);
-  else if (p.aux_dtype == 1) gemm_epilogue16_impl<MT, NT, __bf16>(acc, p, mrow0, ncol0, l16, kg);
-  else gemm_epilogue16_impl<MT, NT, _Float16>(acc, p, mrow0, ncol0, l16, kg);
+// Whether the problem is one for gemm_epilogue16<ANY = false>.
+static inline bool rows_epilogue(const GemmArgs& p) {
+  return (p.out_dtype == 0 || p.out_dtype == 1) && p.scn == 1 && (!p.aux || (p.aux_sm == 0 && p.aux_sn == 1));
 }
 
 // The same for a plain C = A @ B in the operands' own 16-bit type with unit column stride (the grouped GEMM).
@@ -169,11 +233,6 @@ __device__ __forceinline__ void gemm_epilogue16_plain(f32x4 (&acc)[MT][NT], cons
 // (v_permlane16_swap: the odd 16-lane rows of its first register with the even rows of its second): the even lane
 // then holds 8 consecutive columns of the first tile and the odd lane 8 of the second - 16 bytes per lane, half the
 // requests and half the store instructions (rows need 16-byte alignment: lean_epilogue_type).
-__device__ __forceinline__ void swap16(int& a, int& b) {
-#if MI355_DEVICE_PASS
-  asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(a), "+v"(b));
-#endif
-}
 template <int MT, int NT, typename OutT>
 __device__ __forceinline__ void gemm_epilogue16_lean(f32x4 (&acc)[MT][NT], const GemmArgs& p, int mrow0, int ncol0, int l16, int kg) {
   static_assert(NT % 2 == 0 && sizeof(OutT) == 2, "pairs of 16-column tiles of a 16-bit type");
@@ -201,7 +260,7 @@ __device__ __forceinline__ void gemm_epilogue16_lean(f32x4 (&acc)[MT][NT], const
 }
 // 0 = the problem needs the general epilogue; else the C ABI code + 1 of the 16-bit output type the lean one writes
 static inline int lean_epilogue_type(const GemmArgs& p) {
-  if (!p.lean_ok || p.aux || p.activation != 0 || p.scn != 1 || !p.c_vec_ok || p.ldc % 8 != 0) return 0;
+  if (!p.lean_ok || p.aux || p.activation != 0 || p.scn != 1 || !p.c_vec_ok || p.ldc % 8 != 0 || p.N % 8 != 0) return 0;
   return p.out_dtype == 0 ? 1 : p.out_dtype == 1 ? 2 : 0;
 }
 

@@ -41,9 +41,9 @@ __device__ __forceinline__ void mfma16(f16x8 a, f16x8 b, f32x4& c) {
 }
 
 // The tiles `tile`, `tile + tile_step`, ... (< `tile_stop`, by default M/256 * N/256) of one problem, computed by the calling workgroup
-// with the 128 KiB of LDS at `lds0`.  XCD: pass the tile numbers through the per-XCD remap first.  EPI: 0 = scales,
-// activation, any output type; 1 = C has the type of the operands, no scales, no activation; 2 = 0 plus the addend;
-// 3 = the lean epilogue (gemm_epilogue16_lean) with C in the operands' type.
+// with the 128 KiB of LDS at `lds0`.  XCD: pass the tile numbers through the per-XCD remap first.  EPI: 0 = every
+// epilogue of the C ABI; 1 = C has the type of the operands, no scales, no activation; 2 = C in a 16-bit type with a bias row
+// at most (rows_epilogue), any N; 3 = the lean epilogue (gemm_epilogue16_lean) with C in the operands' type.
 // TAIL: K bytes need not be a multiple of 256; what is left behind the last pair of K steps (16 .. 240 bytes of
 // every operand row) is multiplied after the K loop, 64 bytes at a time, through a 32 KiB LDS buffer of its own
 // behind the two stages (which by then hold the next tile's first steps): plain loads with a zero fill, one
@@ -66,13 +66,23 @@ __device__ __forceinline__ void gemm_wave128_tiles(const GemmArgs& p, int tile, 
   const int wm = wave >> 1, wn = wave & 1;
   const int l16 = lane & 15, kg = lane >> 4;
 
-  const int num_m = p.M / BM, num_n = p.N / BN;
+  // Sizes that are no whole tiles: the last tile of a row or column ends where the matrix does and covers part of its
+  // neighbour once more (the same sums in the same order: both write the same bits), so that no load and no row needs a
+  // bound.  A row-major B is fetched in 16-byte chunks: there the last tile begins at one, and the epilogue leaves out the
+  // up to seven columns of padding that it then ends in.
+  // (Edges ran the eight-wave kernel, with bounds on every load and an epilogue of single elements, us: 3001 x 5003 x 1024 bf16
+  // with a bias row 83 -> 39, 6420 x 6701 x 844 240 -> 106, 3738 x 7135 x 455 fp16 112 -> 61, 4095 x 4100 x 4100 bf16 162 -> 140;
+  // a bias row on whole tiles, 4096^3 fp16 129 -> 108, is the epilogue alone.)
+  const int num_m = (p.M + BM - 1) / BM, num_n = (p.N + BN - 1) / BN;
+  const int last_m0 = p.M - BM, last_n0 = (B_KMAJOR ? p.N : (p.N + 7) & ~7) - BN;
   const int ntiles = num_m * num_n;
   const int tend = tile_stop < 0 ? ntiles : tile_stop;   // the walk ends before this tile
   // The tiles are computed as ONE stream of K steps: the loads of the last two steps of a tile already
   // fetch the first two K steps of the next one, so its first fragments are in registers when the finished
   // tile is stored.
   auto tile_at = [&](int t, int& tm, int& tn) { grouped_tile(XCD ? xcd_remap(t, ntiles) : t, num_m, num_n, p.group_m, tm, tn); };
+  auto row_of = [&](int tm) { return min(tm * BM, last_m0); };
+  auto col_of = [&](int tn) { return min(tn * BN, last_n0); };
   int pm, pn;
   tile_at(tile, pm, pn);
   const int nk = TAIL ? (p.k_bytes / (2 * ROWB)) * 2 : p.k_bytes / ROWB;   // K steps of the pipelined loop (an even number)
@@ -98,16 +108,15 @@ __device__ __forceinline__ void gemm_wave128_tiles(const GemmArgs& p, int tile, 
   // column group (n / 16) ^ 2 (k & 3) ^ ((k >> 3) & 1) of its row: a transpose read is served two 16-lane
   // groups at a time - four consecutive k rows each, eight rows apart, the same 16 columns - and this
   // spreads those 8 x 32 bytes over all banks.  With k = 16 wave + 2 j + i / 32 the XOR terms are
-  // 4 (j & 1) + 2 (i / 32) and (j >> 2) & 1 (which needs a pitch that is a multiple of 512 bytes).
+  // 4 (j & 1) + 2 (i / 32) and (j >> 2) & 1.
 #pragma unroll
   for (int q = 0; q < 8; q++) {
     if constexpr (B_KMAJOR) {
       const unsigned chunk = dslot ^ (((q & 1) * 4 + (lane >> 4)) & 7);
       voffB[q] = (drow + 8 * q) * (unsigned)p.ldb + chunk * 16 - (unsigned)ioff_of(q);
     } else {
-      const unsigned pg = (lane & 31) >> 1, half = lane & 1;
-      const unsigned v0 = (lane >> 5) * (unsigned)p.ldb + ((pg ^ (2 * (lane >> 5))) * 32) + half * 16;
-      voffB[q] = (v0 ^ ((4 * (q & 1) + ((q >> 2) & 1)) * 32)) + 2 * q * (unsigned)p.ldb - (unsigned)ioff_of(q);
+      const unsigned group = ((lane & 31) >> 1) ^ (2 * (lane >> 5)) ^ (4 * (q & 1) + ((q >> 2) & 1));
+      voffB[q] = (2 * q + (lane >> 5)) * (unsigned)p.ldb + group * 32 + (lane & 1) * 16 - (unsigned)ioff_of(q);
     }
   }
   // scalar bases of the K step the loads are fetching (two K steps ahead of the MFMAs)
@@ -138,13 +147,13 @@ __device__ __forceinline__ void gemm_wave128_tiles(const GemmArgs& p, int tile, 
     voffPB = B_KMAJOR ? (lane & 7) * (unsigned)p.ldb : ((lane & 7) >> 2) * (unsigned)p.ldb + (lane & 3) * 128;
   }
   auto set_fill_tile = [&](int fm, int fn) {
-    fA = scalar_ptr(p.A + ((int64_t)fm * BM + wave * (BM / 4)) * p.lda);
-    fB = scalar_ptr(B_KMAJOR ? p.B + ((int64_t)fn * BN + wave * 64) * p.ldb
-                             : p.B + (int64_t)fn * BN * 2 + (int64_t)(wave * 16) * p.ldb);
+    const int64_t m0 = row_of(fm), n0 = col_of(fn);
+    fA = scalar_ptr(p.A + (m0 + wave * (BM / 4)) * p.lda);
+    fB = scalar_ptr(B_KMAJOR ? p.B + (n0 + wave * 64) * p.ldb : p.B + n0 * 2 + (int64_t)(wave * 16) * p.ldb);
     if constexpr (PF) {
-      pA = scalar_ptr(p.A + ((int64_t)fm * BM + (fn & 3) * (BM / 4) + wave * (BM / 16)) * p.lda);
-      pB = scalar_ptr(B_KMAJOR ? p.B + ((int64_t)fn * BN + (fm & 7) * 32 + wave * 8) * p.ldb
-                               : p.B + (int64_t)fn * BN * 2 + (int64_t)((fm & 7) * 8 + wave * 2) * p.ldb);
+      pA = scalar_ptr(p.A + (m0 + (fn & 3) * (BM / 4) + wave * (BM / 16)) * p.lda);
+      pB = scalar_ptr(B_KMAJOR ? p.B + (n0 + (fm & 7) * 32 + wave * 8) * p.ldb
+                               : p.B + n0 * 2 + (int64_t)((fm & 7) * 8 + wave * 2) * p.ldb);
     }
   };
   set_fill_tile(pm, pn);
@@ -315,7 +324,8 @@ __device__ __forceinline__ void gemm_wave128_tiles(const GemmArgs& p, int tile, 
     if constexpr (TAIL) {
       const int k_main = nk * ROWB, tail = p.k_bytes - k_main;   // bytes per row: done, and left (a multiple of 16)
       const unsigned tailA = lds0 + 2 * STAGE, tailB = tailA + BM * 64;
-      const char* const tA = p.A + (int64_t)pm * BM * p.lda + k_main;
+      const int n0 = col_of(pn);
+      const char* const tA = p.A + (int64_t)row_of(pm) * p.lda + k_main;
       for (int h = 0; h * 64 < tail; h++) {
         // this half-step's 64 bytes of the 256 A rows and of the 256 B rows (K-major B) or its 32 k rows of 512
         // bytes (row-major B, in the column-group order of the stages): 1024 + 1024 chunks of 16 bytes, four
@@ -332,12 +342,12 @@ __device__ __forceinline__ void gemm_wave128_tiles(const GemmArgs& p, int tile, 
           vb[i] = i32x4{0, 0, 0, 0};
           if constexpr (B_KMAJOR) {
             const int row = id >> 2, kb = h * 64 + (id & 3) * 16;
-            if (kb < tail) vb[i] = *(const i32x4*)(p.B + ((int64_t)pn * BN + row) * p.ldb + k_main + kb);
+            if (kb < tail) vb[i] = *(const i32x4*)(p.B + (int64_t)(n0 + row) * p.ldb + k_main + kb);
           } else {
             const int kr = id >> 5, pc = id & 31;
             const int k = k_main / 2 + h * 32 + kr;
             const int lg = (pc >> 1) ^ (2 * (kr & 3)) ^ ((kr >> 3) & 1);
-            if (k < p.K) vb[i] = *(const i32x4*)(p.B + (int64_t)k * p.ldb + (int64_t)pn * BN * 2 + lg * 32 + (pc & 1) * 16);
+            if (k < p.K) vb[i] = *(const i32x4*)(p.B + (int64_t)k * p.ldb + (int64_t)n0 * 2 + lg * 32 + (pc & 1) * 16);
           }
         }
 #pragma unroll
@@ -382,7 +392,7 @@ __device__ __forceinline__ void gemm_wave128_tiles(const GemmArgs& p, int tile, 
     // (the tile and lane coordinates pass through an empty assembly statement so that none of the
     // epilogue's address arithmetic is hoisted out of the tile loop, where it would occupy - and spill -
     // registers throughout the K loop)
-    int em = pm * BM + wm * (BM / 2), en = pn * BN + wn * 128, el = l16, ek = kg;
+    int em = row_of(pm) + wm * (BM / 2), en = col_of(pn) + wn * 128, el = l16, ek = kg;
     asm volatile("" : "+s"(em), "+s"(en), "+v"(el), "+v"(ek));
     using OwnT = std::conditional_t<std::is_same<V8, bf16x8>::value, __bf16, _Float16>;
     if constexpr (EPI == 1) {
@@ -391,7 +401,7 @@ __device__ __forceinline__ void gemm_wave128_tiles(const GemmArgs& p, int tile, 
       if (p.c_vec_ok && p.ldc % 8 == 0) gemm_epilogue16_lean<MT, NT, OwnT>(acc, p, em, en, el, ek);
       else gemm_epilogue16_plain<MT, NT, OwnT>(acc, p, em, en, el, ek);
     } else if constexpr (EPI == 3) gemm_epilogue16_lean<MT, NT, OwnT>(acc, p, em, en, el, ek);
-    else gemm_epilogue16<MT, NT, EPI == 2>(acc, p, em, en, el, ek);
+    else gemm_epilogue16<MT, NT, EPI == 0>(acc, p, em, en, el, ek);
     tile += tile_step;
     if (tile >= tend) break;
     tile_at(tile, pm, pn);
@@ -532,7 +542,7 @@ __device__ __forceinline__ void mfma16_f8(const i32x8& a, const i32x8& b, f32x4&
 #endif
 }
 
-// EPI: 0 = general epilogue, 2 = with the addend, 3 / 4 = lean epilogue writing fp16 / bf16
+// EPI: 0 = every epilogue of the C ABI, 2 = C in a 16-bit type with a bias row at most (rows_epilogue), 3 / 4 = lean epilogue writing fp16 / bf16
 // TAIL: K bytes need not be a multiple of 256 (of 16 still): the main loop does the whole pairs of K steps, and what is
 // left of each row (16 .. 240 bytes, the same for every tile) follows as one or two K steps whose fragments every lane
 // loads straight from global memory - the same two chunks per 128-byte step as from LDS, zeros beyond K, the masked
@@ -566,8 +576,13 @@ __device__ __forceinline__ void gemm_wave128_f8_tiles(const GemmArgs& p, int til
   const int wm = wave >> 1, wn = wave & 1;
   const int l16 = lane & 15, kg = lane >> 4;
 
-  const int num_m = p.M / BM, num_n = p.N / BN;
+  // (sizes that are no whole tiles: the last tile of a row or column ends where the matrix does, as in the 16-bit kernel;
+  // e4m3 4983 x 2048 x 4864 57.5 us on the eight-wave kernel, 44.2 here, 8192 x 4480 x 7168 257 / 212)
+  const int num_m = (p.M + BM - 1) / BM, num_n = (p.N + BN - 1) / BN;
+  const int last_m0 = p.M - BM, last_n0 = (B_KMAJOR ? p.N : (p.N + 15) & ~15) - BN;
   const int ntiles = num_m * num_n;
+  auto row_of = [&](int tm) { return min(tm * BM, last_m0); };
+  auto col_of = [&](int tn) { return min(tn * BN, last_n0); };
   int pm, pn;   // (the tiles are computed as one stream of K steps)
   grouped_tile(xcd_remap(tile, ntiles), num_m, num_n, p.group_m, pm, pn);
   const int nk = TAIL ? p.k_bytes / (2 * ROWB) * 2 : p.k_bytes / ROWB;
@@ -604,12 +619,13 @@ __device__ __forceinline__ void gemm_wave128_f8_tiles(const GemmArgs& p, int til
   const unsigned voffPA = (lane % (BM / 16)) * (unsigned)p.lda;
   const unsigned voffPB = B_KMAJOR ? (lane & 7) * (unsigned)p.ldb : ((lane & 7) >> 1) * (unsigned)p.ldb + (lane & 1) * 128;
   auto set_fill_tile = [&](int fm, int fn) {
-    fA = p.A + ((int64_t)fm * BM + wave * (BM / 4)) * p.lda;
-    fB = B_KMAJOR ? p.B + ((int64_t)fn * BN + wave * 64) * p.ldb : p.B + (int64_t)fn * BN + (int64_t)(wave * 32) * p.ldb;
+    const int64_t m0 = row_of(fm), n0 = col_of(fn);
+    fA = p.A + (m0 + wave * (BM / 4)) * p.lda;
+    fB = B_KMAJOR ? p.B + (n0 + wave * 64) * p.ldb : p.B + n0 + (int64_t)(wave * 32) * p.ldb;
     if constexpr (PF) {
-      pA = p.A + ((int64_t)fm * BM + (fn & 3) * (BM / 4) + wave * (BM / 16)) * p.lda;
-      pB = B_KMAJOR ? p.B + ((int64_t)fn * BN + (fm & 7) * 32 + wave * 8) * p.ldb
-                    : p.B + (int64_t)fn * BN + (int64_t)((fm & 7) * 16 + wave * 4) * p.ldb;
+      pA = p.A + (m0 + (fn & 3) * (BM / 4) + wave * (BM / 16)) * p.lda;
+      pB = B_KMAJOR ? p.B + (n0 + (fm & 7) * 32 + wave * 8) * p.ldb
+                    : p.B + n0 + (int64_t)((fm & 7) * 16 + wave * 4) * p.ldb;
     }
   };
   set_fill_tile(pm, pn);
@@ -758,7 +774,7 @@ __device__ __forceinline__ void gemm_wave128_f8_tiles(const GemmArgs& p, int til
     if constexpr (TAIL) {
       // (free here: a1 and the B set 1 - the last step read the next tile's first fragments into a0 and the B set 0)
       const int k_main = nk * ROWB, tail = p.k_bytes - k_main;
-      int tm = pm * BM + wm * 128, tn = pn * BN + wn * 128, tl = l16, tk = kg;
+      int tm = row_of(pm) + wm * 128, tn = col_of(pn) + wn * 128, tl = l16, tk = kg;
       asm volatile("" : "+s"(tm), "+s"(tn), "+v"(tl), "+v"(tk));   // (keeps this address arithmetic out of the K loop)
       // a scalar base per fragment and one 32-bit lane offset per operand (gemm_wave128_f8_ok bounds 128 rows plus K)
       const char* const tA = p.A + (int64_t)tm * p.lda + k_main;
@@ -793,11 +809,11 @@ __device__ __forceinline__ void gemm_wave128_f8_tiles(const GemmArgs& p, int til
       }
     }
     mfma_drain(acc);
-    int em = pm * BM + wm * (BM / 2), en = pn * BN + wn * 128, el = l16, ek = kg;
+    int em = row_of(pm) + wm * (BM / 2), en = col_of(pn) + wn * 128, el = l16, ek = kg;
     asm volatile("" : "+s"(em), "+s"(en), "+v"(el), "+v"(ek));   // (keeps the epilogue's address arithmetic out of the K loop)
     if constexpr (EPI == 3) gemm_epilogue16_lean<MT, NT, _Float16>(acc, p, em, en, el, ek);
     else if constexpr (EPI == 4) gemm_epilogue16_lean<MT, NT, __bf16>(acc, p, em, en, el, ek);
-    else gemm_epilogue16<MT, NT, EPI == 2>(acc, p, em, en, el, ek);
+    else gemm_epilogue16<MT, NT, EPI == 0>(acc, p, em, en, el, ek);
     tile += tile_step;
     if (tile >= ntiles) break;
     grouped_tile(xcd_remap(tile, ntiles), num_m, num_n, p.group_m, pm, pn);
@@ -876,7 +892,7 @@ static int launch_wave128_f8(const GemmArgs& p, hipStream_t stream) {
     if (e != hipSuccess) return (int)e;
     attr_set = true;
   }
-  const int tiles = (p.M / BM) * (p.N / 256);
+  const int tiles = ((p.M + BM - 1) / BM) * ((p.N + 255) / 256);
   const int grid = wave128_grid(tiles, p.num_programs);
   gemm_wave128_f8_kernel<FMT, EPI, TAIL, B_KMAJOR, BM><<<dim3(grid), dim3(256), smem, stream>>>(p);
   return (int)hipGetLastError();
@@ -891,63 +907,61 @@ int gemm_wave128_f8_launch(const GemmArgs& p, bool e5m2, bool b_kmajor, hipStrea
     if (lean_epilogue_type(p) == 1) return e5m2 ? launch_wave128_f8<1, 3, false, true, 128>(p, stream) : launch_wave128_f8<0, 3, false, true, 128>(p, stream);
     return e5m2 ? launch_wave128_f8<1, 4, false, true, 128>(p, stream) : launch_wave128_f8<0, 4, false, true, 128>(p, stream);
   }
-  if (!b_kmajor) {   // (gemm_wave128_f8_ok: whole pairs of K steps, no addend)
+  if (!b_kmajor) {   // (gemm_wave128_f8_ok: whole pairs of K steps)
     const int lean = lean_epilogue_type(p);
     if (lean == 1) return e5m2 ? launch_wave128_f8<1, 3, false, false>(p, stream) : launch_wave128_f8<0, 3, false, false>(p, stream);
     if (lean == 2) return e5m2 ? launch_wave128_f8<1, 4, false, false>(p, stream) : launch_wave128_f8<0, 4, false, false>(p, stream);
     return e5m2 ? launch_wave128_f8<1, 0, false, false>(p, stream) : launch_wave128_f8<0, 0, false, false>(p, stream);
   }
-  if (p.k_bytes % 256 != 0) {   // (gemm_wave128_f8_ok: no addend then)
+  if (p.k_bytes % 256 != 0) {
     const int lean = lean_epilogue_type(p);
     if (lean == 1) return e5m2 ? launch_wave128_f8<1, 3, true>(p, stream) : launch_wave128_f8<0, 3, true>(p, stream);
     if (lean == 2) return e5m2 ? launch_wave128_f8<1, 4, true>(p, stream) : launch_wave128_f8<0, 4, true>(p, stream);
+    if (rows_epilogue(p)) return e5m2 ? launch_wave128_f8<1, 2, true>(p, stream) : launch_wave128_f8<0, 2, true>(p, stream);
     return e5m2 ? launch_wave128_f8<1, 0, true>(p, stream) : launch_wave128_f8<0, 0, true>(p, stream);
   }
-  if (p.aux) return e5m2 ? launch_wave128_f8<1, 2>(p, stream) : launch_wave128_f8<0, 2>(p, stream);
   const int lean = lean_epilogue_type(p);
   if (lean == 1) return e5m2 ? launch_wave128_f8<1, 3>(p, stream) : launch_wave128_f8<0, 3>(p, stream);
   if (lean == 2) return e5m2 ? launch_wave128_f8<1, 4>(p, stream) : launch_wave128_f8<0, 4>(p, stream);
+  if (rows_epilogue(p)) return e5m2 ? launch_wave128_f8<1, 2>(p, stream) : launch_wave128_f8<0, 2>(p, stream);
   return e5m2 ? launch_wave128_f8<1, 0>(p, stream) : launch_wave128_f8<0, 0>(p, stream);
 }
 
-// fp8: whole tiles, at least one pair of 128-byte K steps; with a K-major B, what is left behind the last pair is the
-// TAIL form's, which exists without the addend
+// fp8: a whole tile at least, a pair of 128-byte K steps; with a K-major B, what is left behind the last pair is the TAIL form's
+// (whole tiles only: its steps cost so much that the smaller tiles are ahead where edges come on top, 5056 x 6400 x 1152 51 us
+// for 43, 7579 x 3328 x 1408 51 for 45)
 bool gemm_wave128_f8_ok(const GemmArgs& p, bool b_kmajor) {
-  if (!(p.M % 256 == 0 && p.N % 256 == 0 && p.k_bytes % 16 == 0 && p.k_bytes >= 256)) return false;
-  if (p.k_bytes % 256 != 0 && p.aux) return false;
+  if (!(p.M >= 256 && p.N >= 256 && p.k_bytes % 16 == 0 && p.k_bytes >= 256)) return false;
+  if (p.k_bytes % 256 != 0 && (p.M % 256 != 0 || p.N % 256 != 0)) return false;
   if (p.lda * 8 + p.k_bytes >= (1ll << 31)) return false;
   if (b_kmajor) return p.ldb * 8 + p.k_bytes < (1ll << 31);
-  // row-major B: whole pairs of K steps, no addend; 32 rows plus a tile row within 32-bit lane offsets
-  return p.k_bytes % 256 == 0 && !p.aux && p.ldb % 16 == 0 && p.ldb * 32 + 256 < (1ll << 32);
+  // row-major B: whole pairs of K steps; 32 rows plus a tile row within 32-bit lane offsets
+  return p.k_bytes % 256 == 0 && p.ldb % 16 == 0 && p.ldb * 32 + 256 < (1ll << 32);
 }
 
-// fp8 on tiles of 192 x 256 (128 x 256): M a multiple of 192 (128), K-major B, whole pairs of K steps, a 16-bit C through
+// fp8 on tiles of 192 x 256 (128 x 256): K-major B, whole pairs of K steps, a 16-bit C through
 // the lean epilogue
 bool gemm_wave128_f8_192_ok(const GemmArgs& p, bool b_kmajor, int tile_m) {
-  if (!(b_kmajor && p.M % tile_m == 0 && p.N % 256 == 0 && p.k_bytes % 256 == 0 && p.k_bytes >= 256)) return false;
+  if (!(b_kmajor && p.M >= tile_m && p.N >= 256 && p.k_bytes % 256 == 0 && p.k_bytes >= 256)) return false;
   if (lean_epilogue_type(p) == 0) return false;
   return p.lda * 8 + p.k_bytes < (1ll << 31) && p.ldb * 8 + p.k_bytes < (1ll << 31);
 }
 
-bool gemm_wave128_ok(const GemmArgs& p, bool b_kmajor, int in_dtype) {
-  // whole tiles, at least one pair of 128-byte K steps (what is left behind the last pair: the TAIL form, which
-  // exists for 16-bit operands with the lean epilogue - C in the operands' type - only), 32-bit lane offsets
-  if (!(p.M % 256 == 0 && p.N % 256 == 0 && p.k_bytes % 16 == 0 && p.k_bytes >= 256)) return false;
-  if (p.k_bytes % 256 != 0 && !((in_dtype == 0 || in_dtype == 1) && lean_epilogue_type(p) == in_dtype + 1)) return false;
+bool gemm_wave128_ok(const GemmArgs& p, bool b_kmajor) {
+  // a whole tile at least, a pair of 128-byte K steps (what is left behind the last pair: the TAIL form), 32-bit lane offsets
+  if (!(p.M >= 256 && p.N >= 256 && p.k_bytes % 16 == 0 && p.k_bytes >= 256)) return false;
   if (p.lda * 8 + p.k_bytes >= (1ll << 31)) return false;
-  // (row-major B: the per-load XOR of the column group acts on the whole lane offset, so the row term
-  // in it - a multiple of the pitch - must leave the bits of the 512-byte tile row alone)
-  return b_kmajor ? p.ldb * 8 + p.k_bytes < (1ll << 31) : (p.ldb % 512 == 0 && (int64_t)p.K * p.ldb + 512 < (1ll << 31));
+  return b_kmajor ? p.ldb * 8 + p.k_bytes < (1ll << 31) : (int64_t)p.K * p.ldb + 512 < (1ll << 31);
 }
 
-// The 192 x 256 tiles: M a multiple of 192, whole pairs of K steps, C in the operands' type through the lean epilogue
+// The 192 x 256 tiles: whole pairs of K steps, C in the operands' type through the lean epilogue
 // (the one instantiation per type and B layout).  Worth it where the 256 x 256 tiles leave CUs idle in the last round:
 // 3072^3 has 144 of those for 256 CUs and 192 of these.
 bool gemm_wave128_192_ok(const GemmArgs& p, bool b_kmajor, int in_dtype, int tile_m) {
-  if (!(p.M % tile_m == 0 && p.N % 256 == 0 && p.k_bytes % 256 == 0 && p.k_bytes >= 256)) return false;
+  if (!(p.M >= tile_m && p.N >= 256 && p.k_bytes % 256 == 0 && p.k_bytes >= 256)) return false;
   if (!((in_dtype == 0 || in_dtype == 1) && lean_epilogue_type(p) == in_dtype + 1)) return false;
   if (p.lda * 8 + p.k_bytes >= (1ll << 31)) return false;
-  return b_kmajor ? p.ldb * 8 + p.k_bytes < (1ll << 31) : (p.ldb % 512 == 0 && (int64_t)p.K * p.ldb + 512 < (1ll << 31));
+  return b_kmajor ? p.ldb * 8 + p.k_bytes < (1ll << 31) : (int64_t)p.K * p.ldb + 512 < (1ll << 31);
 }
 
 template <typename V8, bool B_KMAJOR, int EPI, bool TAIL = false, int BM = 256>
@@ -959,7 +973,7 @@ static int launch_wave128(const GemmArgs& p, hipStream_t stream) {
     if (e != hipSuccess) return (int)e;
     attr_set = true;
   }
-  const int tiles = (p.M / BM) * (p.N / 256);
+  const int tiles = ((p.M + BM - 1) / BM) * ((p.N + 255) / 256);
   const int grid = wave128_grid(tiles, p.num_programs);
   gemm_wave128_kernel<V8, B_KMAJOR, EPI, TAIL, BM><<<dim3(grid), dim3(256), smem, stream>>>(p);
   return (int)hipGetLastError();
@@ -991,7 +1005,7 @@ bool gemm_wave128_mixed_ok(const GemmArgs& p, bool b_kmajor, int in_dtype, int r
   if (!(p.N % 256 == 0 && p.k_bytes % 256 == 0 && p.k_bytes >= 256)) return false;
   if (!((in_dtype == 0 || in_dtype == 1) && lean_epilogue_type(p) == in_dtype + 1)) return false;
   if (p.lda * 8 + p.k_bytes >= (1ll << 31)) return false;
-  return b_kmajor ? p.ldb * 8 + p.k_bytes < (1ll << 31) : (p.ldb % 512 == 0 && (int64_t)p.K * p.ldb + 512 < (1ll << 31));
+  return b_kmajor ? p.ldb * 8 + p.k_bytes < (1ll << 31) : (int64_t)p.K * p.ldb + 512 < (1ll << 31);
 }
 
 template <typename V8, typename GA>
@@ -1021,10 +1035,13 @@ static int gemm_wave128_launch_typed(const GemmArgs& p, bool b_kmajor, bool own_
     return b_kmajor ? launch_wave128<V8, true, 3, false, 192>(p, stream) : launch_wave128<V8, false, 3, false, 192>(p, stream);
   if (p.tile_m == 128)
     return b_kmajor ? launch_wave128<V8, true, 3, false, 128>(p, stream) : launch_wave128<V8, false, 3, false, 128>(p, stream);
-  if (p.k_bytes % 256 != 0)   // (gemm_wave128_ok: the lean epilogue then)
-    return b_kmajor ? launch_wave128<V8, true, 3, true>(p, stream) : launch_wave128<V8, false, 3, true>(p, stream);
-  if (p.aux) return b_kmajor ? launch_wave128<V8, true, 2>(p, stream) : launch_wave128<V8, false, 2>(p, stream);
+  if (p.k_bytes % 256 != 0) {
+    if (own_type_lean) return b_kmajor ? launch_wave128<V8, true, 3, true>(p, stream) : launch_wave128<V8, false, 3, true>(p, stream);
+    if (rows_epilogue(p)) return b_kmajor ? launch_wave128<V8, true, 2, true>(p, stream) : launch_wave128<V8, false, 2, true>(p, stream);
+    return b_kmajor ? launch_wave128<V8, true, 0, true>(p, stream) : launch_wave128<V8, false, 0, true>(p, stream);
+  }
   if (own_type_lean) return b_kmajor ? launch_wave128<V8, true, 3>(p, stream) : launch_wave128<V8, false, 3>(p, stream);
+  if (rows_epilogue(p)) return b_kmajor ? launch_wave128<V8, true, 2>(p, stream) : launch_wave128<V8, false, 2>(p, stream);
   return b_kmajor ? launch_wave128<V8, true, 0>(p, stream) : launch_wave128<V8, false, 0>(p, stream);
 }
 

@@ -324,7 +324,7 @@ __device__ __forceinline__ void gemm_wave128_mxfp8_tiles(const GemmArgs& p, int 
     asm volatile("" : "+s"(em), "+s"(en), "+v"(el), "+v"(ek));   // (keeps the epilogue's address arithmetic out of the K loop)
     if constexpr (EPI == 3) gemm_epilogue16_lean<MT, NT, _Float16>(acc, p, em, en, el, ek);
     else if constexpr (EPI == 4) gemm_epilogue16_lean<MT, NT, __bf16>(acc, p, em, en, el, ek);
-    else gemm_epilogue16<MT, NT>(acc, p, em, en, el, ek);
+    else gemm_epilogue16<MT, NT, true>(acc, p, em, en, el, ek);
     tile += tile_step;
     if (tile >= ntiles) break;
     grouped_tile(xcd_remap(tile, ntiles), num_m, num_n, p.group_m, pm, pn);
@@ -722,7 +722,7 @@ __device__ __forceinline__ void gemm_wave128_mxfp4_tiles(const GemmArgs& p, int 
     asm volatile("" : "+s"(em), "+s"(en), "+v"(el), "+v"(ek));   // (keeps the epilogue's address arithmetic out of the K loop)
     if constexpr (EPI == 3) gemm_epilogue16_lean<MT, NT, _Float16>(acc, p, em, en, el, ek);
     else if constexpr (EPI == 4) gemm_epilogue16_lean<MT, NT, __bf16>(acc, p, em, en, el, ek);
-    else gemm_epilogue16<MT, NT>(acc, p, em, en, el, ek);
+    else gemm_epilogue16<MT, NT, true>(acc, p, em, en, el, ek);
     tile += tile_step;
     if (tile >= ntiles) break;
     grouped_tile(xcd_remap(tile, ntiles), num_m, num_n, p.group_m, pm, pn);

@@ -137,7 +137,7 @@ int gemm8_splitk_launch(const GemmArgs& p, bool e5m2, int splits, int chunk_byte
 int gemm32_splitk_launch(const GemmArgs& p, int splits, int chunk_bytes, hipStream_t stream);   // fp32 operands, K-major B
 int splitk_reduce_launch(const GemmStridedArgs& out, const float* workspace, int splits, hipStream_t stream);   // A, B, K, in_dtype of `out` unused
 bool gemm_wave128_192_ok(const GemmArgs& p, bool b_kmajor, int in_dtype, int tile_m = 192);   // the same for tiles of 192 x 256 / 128 x 256
-bool gemm_wave128_ok(const GemmArgs& p, bool b_kmajor, int in_dtype);
+bool gemm_wave128_ok(const GemmArgs& p, bool b_kmajor);   // 16-bit operands: sizes from one tile on
 bool gemm_wave128_f8_ok(const GemmArgs& p, bool b_kmajor);
 bool gemm_wave128_mixed_ok(const GemmArgs& p, bool b_kmajor, int in_dtype, int rows256);   // rows256 rows on 256-row tiles, the rest on 192-row tiles
 int gemm_wave128_mixed_launch(const GemmArgs& p, int rows256, bool bf16, bool b_kmajor, hipStream_t stream);
