@@ -28,8 +28,8 @@
  * of the MFMA epilogues; 3: MFMA burn probe with its block-scaled shapes, per-device properties, fp8 attention forward at
  * head dims 16 / 32 / 256, a row-major fp8 B on the MFMA kernels, block-scaled products with any K that is a multiple of
  * 32 and scale rows of any pitch on the MFMA kernels; 4: mi355_gemm_splitk, a row-major B whose N is not a multiple of
- * 16 bytes inside a padded pitch on the tile kernels; 5: fp32 operands in mi355_gemm; 6: mi355_grouped_gemm_host, mi355_gemm_workspace and mi355_gemm_ws.) */
-#define MI355_ABI_VERSION 6
+ * 16 bytes inside a padded pitch on the tile kernels; 5: fp32 operands in mi355_gemm; 6: mi355_grouped_gemm_host, mi355_gemm_workspace and mi355_gemm_ws; 7: mi355_mx_gemm_ws and mi355_mx_gemm_workspace.) */
+#define MI355_ABI_VERSION 7
 
 #ifdef __cplusplus
 extern "C" {
@@ -310,6 +310,15 @@ int mi355_mx_gemm(const uint8_t* A, const uint8_t* sA, const uint8_t* B, const u
                   int M, int N, int K, int fmt, int out_dtype,
                   int64_t lda, int64_t ldb, int64_t lds_a, int64_t lds_b, int64_t ldc,
                   void* stream);
+
+/* The same with a workspace of the caller's (device memory, 16-byte aligned, its own for every call under way): products of
+ * few tiles and a long K are then split along K, the fp32 slices being added in split order.  The size that a product wants,
+ * in bytes, comes from mi355_mx_gemm_workspace (0: none); with workspace_bytes 0 the call is mi355_mx_gemm. */
+int64_t mi355_mx_gemm_workspace(int M, int N, int K, int fmt);
+int mi355_mx_gemm_ws(const uint8_t* A, const uint8_t* sA, const uint8_t* B, const uint8_t* sB, void* C,
+                     int M, int N, int K, int fmt, int out_dtype,
+                     int64_t lda, int64_t ldb, int64_t lds_a, int64_t lds_b, int64_t ldc,
+                     void* workspace, size_t workspace_bytes, void* stream);
 
 /*
  * Flash-attention forward: O = softmax(Q K^T * sm_scale [+ causal mask]) V per (z, h); also writes

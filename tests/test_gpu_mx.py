@@ -305,3 +305,32 @@ def test_random_shapes_through_the_default_dispatch_are_bit_exact(gpu, fmt):
         got = to_np(triton_amd.mx_matmul(t(a), t(sa), t(b), t(sb), fmt, out_dtype=out))
         name = {torch.float32: "fp32", torch.bfloat16: "bf16", torch.float16: "fp16"}[out]
         assert bits_equal(got, formats.round_to(ref32, name)), (fmt, case, M, N, K, name)
+
+
+@pytest.mark.parametrize("tile", [8, 9, 10, None])   # 128x128, 128x64, 64x64, the default dispatch (splits of K where few tiles have a long K)
+@pytest.mark.parametrize("fmt", ["mxfp4", "mxfp8"])
+def test_ring_kernels_at_the_edges_of_their_ring_are_bit_exact(gpu, monkeypatch, fmt, tile):
+    # the block-scaled ring kernels: one K step, fewer than the ring is deep, more; an MXFP4 K that ends in half a step; rows and
+    # columns below, at and past a tile.  NaN codes and scales behind every operand's rows: nobody may use them.  Exact sums
+    if tile is not None:
+        set_knob(monkeypatch, "MI355_GEMM_TILE", str(tile))
+    rng = np.random.default_rng(100 + (tile or 0))
+    for M, N, K in ((128, 128, 128), (64, 64, 256), (65, 130, 384), (1, 7, 512), (200, 300, 1152), (257, 129, 640), (16, 1024, 4096), (300, 500, 4224)):
+        fp4 = fmt == "mxfp4"
+        if fp4:
+            a, sa, b, sb = _operands(rng, M, N, K, fmt, lo=126, hi=129)
+        else:
+            a, b = (formats.encode_fp8(rng.integers(-2, 3, size=(rows, K)).astype(np.float32), "e4m3") for rows in (M, N))
+            sa, sb = (rng.integers(126, 129, size=(rows, K // 32)).astype(np.uint8) for rows in (M, N))
+        ref = mx.mx_matmul(a, sa, b, sb, fmt, out_dtype="fp32")
+
+        def padded(x, rows, columns, fill):
+            wide = np.full((x.shape[0] + rows, x.shape[1] + columns), fill, dtype=np.uint8)
+            wide[: x.shape[0], : x.shape[1]] = x
+            return torch.from_numpy(wide).to(gpu)[: x.shape[0], : x.shape[1]]
+
+        for extra in (0, 16):
+            ops = [padded(x, 1, extra, 0xFF if scale or not fp4 else 0x77) for x, scale in ((a, False), (sa, True), (b, False), (sb, True))]
+            got = triton_amd.mx_matmul(*ops, fmt, out_dtype=torch.float32)
+            assert bits_equal(to_np(got), ref), (M, N, K, extra)
+        assert bits_equal(_run(gpu, a, sa, b, sb, fmt, torch.bfloat16), formats.round_bf16(ref)), (M, N, K)

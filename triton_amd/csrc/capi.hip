@@ -147,13 +147,13 @@ int elem_size(int dtype) {
 // splits), so that there the splits also buy bandwidth.
 struct RingPlan { int shape, splits; double us; };
 constexpr double kLaunchUs = 3.5;
-RingPlan ring_plan(int M, int N, int steps, int cus, int splits_lo, int splits_hi) {
+RingPlan ring_plan(int M, int N, int steps, int cus, int splits_lo, int splits_hi, double step_share = 1.0) {
   const double streamed = 128.0 * steps * std::max(M, N);   // bytes of the longer operand
   static const struct { int bm, bn; double round_us, step_us; } kShapes[3] = {{128, 128, 2.5, 0.42}, {128, 64, 1.5, 0.265}, {64, 64, 0.6, 0.165}};
   RingPlan best{0, 1, 1e30};
   for (int shape = 0; shape < 3; shape++) {
     const auto& t = kShapes[shape];
-    const double step_us = (M <= t.bm || N <= t.bn) && streamed >= 64e6 ? std::max(t.step_us, (M <= t.bm ? t.bn : t.bm) * 128 / 30e3) : t.step_us;
+    const double step_us = (M <= t.bm || N <= t.bn) && streamed >= 64e6 ? std::max(t.step_us, (M <= t.bm ? t.bn : t.bm) * 128 / 30e3) : t.step_us * step_share;
     const long tiles = (long)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
     for (int splits = splits_lo; splits <= splits_hi; splits++) {
       const int per = (steps + splits - 1) / splits;
@@ -1019,9 +1019,28 @@ int mi355_grouped_gemm_host(const void* const* a, const void* const* b, void* co
   return MI355_OK;
 }
 
-int mi355_mx_gemm(const uint8_t* A, const uint8_t* sA, const uint8_t* B, const uint8_t* sB, void* C,
-                  int M, int N, int K, int fmt, int out_dtype,
-                  int64_t lda, int64_t ldb, int64_t lds_a, int64_t lds_b, int64_t ldc, void* stream_) {
+// A K step of the block-scaled ring kernels takes 1.3 times the others' (1024 x 4096 x 4096, 128x128 tiles: e4m3 18.3 us, MXFP8
+// 23.7; 4096^3 MXFP8 90, MXFP4 59, half as many steps).
+constexpr double kMxStep = 1.3;
+
+// Splits of K of a block-scaled product that has a workspace (1 = none), as auto_splits for the other ring kernels.
+static int mx_splits(int M, int N, int64_t k_bytes, int cus) {
+  const int steps = (int)((k_bytes + 127) / 128);
+  const int most = (int)std::min<int64_t>(std::min<int64_t>(32, steps / 2), (64ll << 20) / std::max<int64_t>(1, 4ll * M * N));
+  if (knob(knobs().splitk, 1) == 0 || most < 2 || steps < 16) return 1;
+  const RingPlan split = ring_plan(M, N, steps, cus, 2, most, kMxStep);
+  return split.us < 0.95 * ring_plan(M, N, steps, cus, 1, 1, kMxStep).us ? split.splits : 1;
+}
+
+int64_t mi355_mx_gemm_workspace(int M, int N, int K, int fmt) {
+  if (M <= 0 || N <= 0 || K <= 0 || K % 128 != 0 || (fmt != MI355_MXFP4 && fmt != MI355_MXFP8)) return 0;
+  const int splits = mx_splits(M, N, fmt == MI355_MXFP4 ? K / 2 : K, device_info().cus > 0 ? device_info().cus : 256);
+  return splits > 1 ? (int64_t)splits * M * N * 4 : 0;
+}
+
+static int mx_impl(const uint8_t* A, const uint8_t* sA, const uint8_t* B, const uint8_t* sB, void* C,
+                   int M, int N, int K, int fmt, int out_dtype,
+                   int64_t lda, int64_t ldb, int64_t lds_a, int64_t lds_b, int64_t ldc, void* workspace, size_t workspace_bytes, void* stream_) {
   if (!A || !sA || !B || !sB || !C || M <= 0 || N <= 0 || K <= 0) return MI355_EINVAL;
   if (fmt != MI355_MXFP4 && fmt != MI355_MXFP8) return MI355_EINVAL;
   if (out_dtype != MI355_F16 && out_dtype != MI355_BF16 && out_dtype != MI355_F32) return MI355_EDTYPE;
@@ -1091,6 +1110,43 @@ int mi355_mx_gemm(const uint8_t* A, const uint8_t* sA, const uint8_t* B, const u
     }
   }
   p.num_programs = knob(knobs().programs, cus);
+  // the ring kernels of 64 .. 128-row tiles, split along K where there is a workspace, where they are the faster ones by the
+  // estimates of the other products (MXFP4 steps hold twice the elements in the same bytes, which are what bounds both).  us, the
+  // 128x128 kernel of one barrier per step / ring: MXFP8 567 x 1280 x 5888 73 / 18, 2304 x 1536 x 4480 64 / 26, 256 x 3968 x 3840 42 /
+  // 9, MXFP4 192 x 1152 x 5120 38 / 7, 1024 x 1920 x 5632 39 / 14; the four-wave kernels on few tiles / ring: MXFP4 1024 x 4096 x 4096
+  // 18.6 / 15.1, MXFP8 31.5 / 23.7, 512 x 8192 x 8192 56 / 41; these stay ahead from about a round of their tiles on (2048 x 4096 x 4096
+  // MXFP4 23.6 / 29.8, MXFP8 34 / 45)
+  const bool ring_takes = K % 128 == 0 && lds_a % 4 == 0 && lds_b % 4 == 0 && aligned(sA, 4) && aligned(sB, 4) && lds_a < (1 << 24) && lds_b < (1 << 24);
+  if (ring_takes && knobs().tile_m == UNSET && knobs().mixed_rows == UNSET) {
+    const int steps = (p.k_bytes + 127) / 128, group_bytes = fmt == MI355_MXFP4 ? 512 : 1024;
+    int shape = -1, splits = 1;
+    if (knobs().tile != UNSET) {
+      if (knobs().tile >= 8 && knobs().tile <= 10) shape = knobs().tile - 8;
+    } else {
+      if (workspace) splits = mx_splits(M, N, p.k_bytes, cus);
+      const RingPlan plan = ring_plan(M, N, steps, cus, splits, splits, kMxStep);
+      double other = 1e30;
+      // (the eight-wave kernel on 256 x 256 tiles, for what the four-wave ones do not take)
+      if (tile != 6 && tiles256 * 2 >= cus && p.k_bytes % 128 == 0) other = 1.12 * tiles256_us(tiles256, 256, steps, cus, true, true);
+      if (tile == 6) {
+        const int rows = p.tile_m ? p.tile_m : 256, tail = (p.k_bytes % group_bytes + 127) / 128;
+        other = tiles256_us((long)((M + rows - 1) / rows) * ((N + 255) / 256), rows, steps - tail + tail * (fmt == MI355_MXFP4 ? 9 : 21), cus, false, true);
+      }
+      if (plan.us < other) shape = plan.shape;
+      else splits = 1;
+    }
+    if (shape >= 0) {
+      const int per = (steps + splits - 1) / splits, used = (steps + per - 1) / per;
+      if (used < 2) return gemm_ring_mx_launch(p, fmt == MI355_MXFP4, shape, 1, 0, (hipStream_t)stream_);
+      if (!aligned(workspace, 16) || workspace_bytes < (size_t)used * M * N * sizeof(float)) return MI355_EINVAL;
+      p.workspace = (float*)workspace;
+      const int rc = gemm_ring_mx_launch(p, fmt == MI355_MXFP4, shape, used, per * 128, (hipStream_t)stream_);
+      if (rc) return rc;
+      GemmStridedArgs out{};
+      out.C = C; out.M = M; out.N = N; out.scm = ldc; out.scn = 1; out.out_dtype = out_dtype;
+      return splitk_reduce_launch(out, (const float*)workspace, used, (hipStream_t)stream_);
+    }
+  }
   // and on both tile heights in one launch, as for the 16-bit and fp8 products
   if (knobs().tile == UNSET && knobs().tile_m == UNSET && N % 256 == 0) {
     const int want = knob(knobs().mixed_rows, -1), group = fmt == MI355_MXFP4 ? 512 : 1024;
@@ -1101,6 +1157,18 @@ int mi355_mx_gemm(const uint8_t* A, const uint8_t* sA, const uint8_t* B, const u
   }
   tile = knob(knobs().tile, tile);
   return mx_gemm_launch(p, fmt, tile, (hipStream_t)stream_);
+}
+
+int mi355_mx_gemm(const uint8_t* A, const uint8_t* sA, const uint8_t* B, const uint8_t* sB, void* C,
+                  int M, int N, int K, int fmt, int out_dtype,
+                  int64_t lda, int64_t ldb, int64_t lds_a, int64_t lds_b, int64_t ldc, void* stream_) {
+  return mx_impl(A, sA, B, sB, C, M, N, K, fmt, out_dtype, lda, ldb, lds_a, lds_b, ldc, nullptr, 0, stream_);
+}
+
+int mi355_mx_gemm_ws(const uint8_t* A, const uint8_t* sA, const uint8_t* B, const uint8_t* sB, void* C,
+                     int M, int N, int K, int fmt, int out_dtype,
+                     int64_t lda, int64_t ldb, int64_t lds_a, int64_t lds_b, int64_t ldc, void* workspace, size_t workspace_bytes, void* stream_) {
+  return mx_impl(A, sA, B, sB, C, M, N, K, fmt, out_dtype, lda, ldb, lds_a, lds_b, ldc, workspace_bytes ? workspace : nullptr, workspace_bytes, stream_);
 }
 
 int mi355_clock_probe(uint64_t* ticks, int duration_us, void* stream_) {

@@ -150,6 +150,26 @@ __device__ __forceinline__ void async_copy4_asm(const void* gsrc, unsigned lds_w
 #endif
 }
 
+// The same with a wave-uniform 64-bit base and a 32-bit lane offset (async_copy16_sbase, SETTLE as there).
+template <bool SETTLE = false>
+__device__ __forceinline__ void async_copy4_sbase(const void* sbase, unsigned lane_off, unsigned lds_wave_base) {
+#if MI355_DEVICE_PASS
+  if constexpr (SETTLE)
+    asm volatile("s_nop 4\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1"
+                 :: "v"(lane_off), "s"(sbase), "s"(lds_wave_base) : "memory");
+  else
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1"
+                 :: "v"(lane_off), "s"(sbase), "s"(lds_wave_base) : "memory");
+#endif
+}
+
+// 4 bytes per lane into a register, like load16_sbase.
+__device__ __forceinline__ void load4_sbase(int& dst, const void* sbase, unsigned lane_off) {
+#if MI355_DEVICE_PASS
+  asm volatile("global_load_dword %0, %1, %2" : "=v"(dst) : "v"(lane_off), "s"(sbase));
+#endif
+}
+
 // 2^x by the hardware transcendental unit (denormal results flush to zero, as the reference
 // allows on AMD: python/tutorials/06-fused-attention.py:452-454 `allow_flush_denorm`).
 __device__ __forceinline__ float fast_exp2(float x) {

@@ -29,7 +29,7 @@ namespace mi355 {
 // copied all of them once per pair of steps.
 template <typename V8>
 struct Ring16 {
-  static constexpr int kElemBytes = 2;
+  static constexpr int kElemBytes = 2, kSubSteps = 2, kScaleDwords = 0;
   using Operand = V8;
   __device__ static void mma(const bf16x8& a, const bf16x8& b, f32x4& c) {
 #if MI355_DEVICE_PASS
@@ -44,12 +44,41 @@ struct Ring16 {
 };
 template <int FMT>   // 0 = e4m3fn, 1 = e5m2
 struct Ring8 {
-  static constexpr int kElemBytes = 1;
+  static constexpr int kElemBytes = 1, kSubSteps = 1, kScaleDwords = 0;
   using Operand = i32x8;
   __device__ static void mma(const i32x8& a, const i32x8& b, f32x4& c) {
 #if MI355_DEVICE_PASS
     if constexpr (FMT == 0) asm volatile("v_mfma_f32_16x16x128_f8f6f4 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
     else asm volatile("v_mfma_f32_16x16x128_f8f6f4 %0, %1, %2, %0 cbsz:1 blgp:1" : "+a"(c) : "v"(a), "v"(b));
+#endif
+  }
+};
+
+// Block-scaled elements (OCP MX: one e8m0 scale for every 32 of K): kScaleDwords dwords of scales per row and K step travel
+// through the stages behind the operands.  MXFP8: a lane's two chunks, kg and 4 + kg, are halves of the blocks that the
+// instruction takes them for, and the lane supplies the scale of block kg (see gemm_wave128_mx.hip).  MXFP4: a chunk is a
+// block; lane kg takes block 2 kg in the first sub-step and 2 kg + 1 in the second, so that one 16-bit read fetches both
+// scales and the sub-step's instruction names its byte.
+struct RingMx8 {
+  static constexpr int kElemBytes = 1, kSubSteps = 1, kScaleDwords = 1, kBlockBytes = 32;
+  using Operand = i32x8;
+  template <int KS>
+  __device__ static void mma(const i32x8& a, const i32x8& b, f32x4& c, int sa, int sb) {
+#if MI355_DEVICE_PASS
+    asm volatile("v_mfma_scale_f32_16x16x128_f8f6f4 %0, %1, %2, %0, %3, %4 op_sel_hi:[0,0,0]" : "+a"(c) : "v"(a), "v"(b), "v"(sa), "v"(sb));
+#endif
+  }
+};
+struct RingMx4 {
+  static constexpr int kElemBytes = 1, kSubSteps = 2, kScaleDwords = 2, kBlockBytes = 16;
+  using Operand = i32x4;
+  template <int KS>
+  __device__ static void mma(const i32x4& a, const i32x4& b, f32x4& c, int sa, int sb) {
+#if MI355_DEVICE_PASS
+    if constexpr (KS == 0)
+      asm volatile("v_mfma_scale_f32_16x16x128_f8f6f4 %0, %1, %2, %0, %3, %4 op_sel_hi:[0,0,0] cbsz:4 blgp:4" : "+a"(c) : "v"(a), "v"(b), "v"(sa), "v"(sb));
+    else
+      asm volatile("v_mfma_scale_f32_16x16x128_f8f6f4 %0, %1, %2, %0, %3, %4 op_sel:[1,1,0] op_sel_hi:[0,0,0] cbsz:4 blgp:4" : "+a"(c) : "v"(a), "v"(b), "v"(sa), "v"(sb));
 #endif
   }
 };
@@ -207,24 +236,29 @@ __device__ __forceinline__ void ring_drain_wait(int left) {
 }
 
 constexpr int RING_ROW = 128;   // bytes of an operand row per K step
+template <typename E, int BM, int BN>
+constexpr int ring_stage_bytes() { return (BM + BN) * (RING_ROW + 4 * E::kScaleDwords); }
 
 // Tile (pm, pn) of the product p with the ring of NS stages at LDS address lds0 (NS * (BM + BN) * 128 bytes).  A has whole
 // 16-byte chunks along K (k_bytes of them) and a K-major B too; a row-major B (16-bit types) has rows of whole 16-byte chunks,
-// p.K of them: in the last chunk's place of A's rows there may be zeros beyond K.  Every wave's
+// p.K of them: in the last chunk's place of A's rows there may be zeros beyond K.  Block-scaled: both operands K-major, K a
+// multiple of 128 elements, scale rows that begin on dwords.  Every wave's
 // fragments are in registers when the last step's MFMAs begin, so a caller that runs another tile needs one barrier first.
 template <typename E, int BM, int BN, int WN, bool B_KMAJOR, int NS>
 __device__ __forceinline__ void gemm_ring_tile(const GemmArgs& p, const int pm, const int pn, const unsigned lds0) {
 #if MI355_DEVICE_PASS
-  constexpr bool FP8 = E::kElemBytes == 1;
-  static_assert(B_KMAJOR || !FP8, "row-major B: 16-bit types");
+  using Op = typename E::Operand;
+  constexpr bool WIDE = sizeof(Op) == 32;                  // a fragment is two chunks of a row, else one for each sub-step
+  constexpr int SD = E::kScaleDwords;
+  constexpr bool MX = SD > 0;
+  static_assert(B_KMAJOR || E::kElemBytes == 2, "row-major B: 16-bit types");
   static_assert((BM == 64 || BM == 128) && (BN == 64 || BN == 128), "tile sizes");
   constexpr int NW = 2 * WN, TM = BM / 2, TN = BN / WN, MT = TM / 16, NT = TN / 16;
-  constexpr int A_BYTES = BM * RING_ROW, STAGE = (BM + BN) * RING_ROW;
-  constexpr int LA = BM / 8 / NW, LB = BN / 8 / NW, L = LA + LB;   // direct loads per wave and step: 1 KiB each
-  constexpr int KS = FP8 ? 1 : 2, NMFMA = KS * MT * NT;
-  constexpr int NR = 2 * MT + (B_KMAJOR ? 2 : 4) * NT;     // LDS reads per wave and step
+  constexpr int A_BYTES = BM * RING_ROW, S_BYTES = (BM + BN) * RING_ROW, STAGE = ring_stage_bytes<E, BM, BN>();
+  constexpr int BLOCKS = (BM + BN) / 64, LS = (BLOCKS * SD + NW - 1) / NW;   // scales: loads of one dword of 64 rows
+  constexpr int LA = BM / 8 / NW, LB = BN / 8 / NW, L = LA + LB + LS;   // direct loads per wave and step: 1 KiB each, then the scales
+  constexpr int KS = E::kSubSteps, NMFMA = KS * MT * NT;
   static_assert(NS * L < 64, "vmcnt has six bits");
-  using Op = typename E::Operand;
 
   const int lane = threadIdx.x & 63, l16 = lane & 15, kg = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
@@ -249,19 +283,20 @@ __device__ __forceinline__ void gemm_ring_tile(const GemmArgs& p, const int pm, 
   // clamped onto the last valid ones.  The lane offsets carry 4096 (taken off the base) so that none is negative once
   // the instruction offset, which moves the LDS side, is taken back out of the global side.
   auto xor_of = [](int k) { return BN == 128 ? ((k & 3) << 1) ^ ((k >> 3) & 1) : (((k >> 1) & 1) << 1) ^ ((k >> 3) & 1); };
+  auto chunk_of = [](int c) { return MX && KS == 2 ? 2 * (c & 3) + (c >> 2) : c; };   // the chunk of the row in the place of chunk c
   unsigned voffA[LA], voffB[LB];
   int chunkA[LA], rowB[LB];   // for the tail: the lane's chunk of A (and of a K-major B), the lane's k row of a row-major B
 #pragma unroll
   for (int q = 0; q < LA; q++) {
     const int r = (wave * LA + q) * 8 + (lane >> 3);
-    chunkA[q] = (lane & 7) ^ ((r >> 1) & 7);
+    chunkA[q] = chunk_of((lane & 7) ^ ((r >> 1) & 7));
     voffA[q] = (unsigned)min(r, p.M - 1 - m0) * (unsigned)p.lda + chunkA[q] * 16 + 4096u - q * 1024;
   }
 #pragma unroll
   for (int q = 0; q < LB; q++) {
     if constexpr (B_KMAJOR) {
       const int r = (wave * LB + q) * 8 + (lane >> 3);
-      rowB[q] = (lane & 7) ^ ((r >> 1) & 7);
+      rowB[q] = chunk_of((lane & 7) ^ ((r >> 1) & 7));
       voffB[q] = (unsigned)min(r, p.N - 1 - n0) * (unsigned)p.ldb + rowB[q] * 16 + 4096u - q * 1024;
     } else {
       constexpr int CPR = BN / 8, RPI = 64 / CPR;   // 16-byte chunks per k row, k rows per instruction
@@ -277,8 +312,37 @@ __device__ __forceinline__ void gemm_ring_tile(const GemmArgs& p, const int pm, 
   const char* tileB = scalar_ptr((B_KMAJOR ? p.B + (int64_t)n0 * p.ldb : p.B + (int64_t)n0 * 2) - 4096);
   const char* fA = tail ? tileA - RING_ROW : tileA;   // the K step being requested (step s, or s - 1 behind a tail)
   const char* fB = tail ? tileB - stepB : tileB;
+  // scales: dword d of the 64 rows of block b (those of A, then those of B) at S_BYTES + 256 (b SD + d); waves without a share of
+  // their own repeat another's, so that every wave counts the same loads
+  const char* fS[LS > 0 ? LS : 1];
+  unsigned voffS[LS > 0 ? LS : 1], slotS[LS > 0 ? LS : 1];
+  auto scale_rows = [&](int b) {   // the lane's row of block b: address of the operand's scales, rows, pitch
+    const bool a = b < BM / 64;
+    const int r = (a ? b : b - BM / 64) * 64 + lane;
+    return a ? (unsigned)min(r, p.M - 1 - m0) * (unsigned)p.lds_a : (unsigned)min(r, p.N - 1 - n0) * (unsigned)p.lds_b;
+  };
+  auto scale_base = [&](int b) {
+    return scalar_ptr((const char*)(b < BM / 64 ? p.sA + (int64_t)m0 * p.lds_a : p.sB + (int64_t)n0 * p.lds_b));
+  };
+  if constexpr (MX) {
+#pragma unroll
+    for (int l = 0; l < LS; l++) {
+      const int at = (wave * LS + l) % (BLOCKS * SD), b = at / SD, d = at % SD;
+      fS[l] = scale_base(b) - (tail ? 4 * SD : 0);
+      voffS[l] = scale_rows(b) + 4 * d;
+      slotS[l] = S_BYTES + at * 256;
+    }
+  }
+  auto advance = [&]() {
+    fA += RING_ROW;
+    fB += stepB;
+#pragma unroll
+    for (int l = 0; l < LS; l++) fS[l] += 4 * SD;
+  };
   auto issue = [&](auto Q_, unsigned stage_base, auto SETTLE_) {   // (SETTLE in the prologue: scalar registers may just have been restored)
     constexpr int q = decltype(Q_)::value;
+    if constexpr (q >= LA + LB) async_copy4_sbase<decltype(SETTLE_)::value>(fS[q - LA - LB], voffS[q - LA - LB], stage_base + slotS[q - LA - LB]);
+    else
     if constexpr (q < LA) async_copy16_sbase_off<q * 1024, q == 0, decltype(SETTLE_)::value>(fA, voffA[q], stage_base + wave * (LA * 1024));
     else async_copy16_sbase_off<(q - LA) * 1024, q == LA, decltype(SETTLE_)::value>(fB, voffB[q - LA], stage_base + A_BYTES + wave * (LB * 1024));
   };
@@ -299,14 +363,28 @@ __device__ __forceinline__ void gemm_ring_tile(const GemmArgs& p, const int pm, 
       for (int t = 0; t < NT; t++) adrB[t] = lds0 + A_BYTES + k * (BN * 2) + (((wn * NT + t) ^ xor_of(k)) * 32) + (l16 & 3) * 8;
     }
   }
-  struct Frags { Op a[KS][MT]; Op b[KS][NT]; };
+  // scale byte x of row R at 256 (R / 64 SD + x / 4) + 4 (R % 64) + x % 4 (16 rows of a tile stay in one block of 64)
+  auto scale_at = [&](int row) {
+    const int x = KS == 2 ? 2 * kg : kg;
+    return lds0 + S_BYTES + ((row >> 6) * SD + (x >> 2)) * 256 + (row & 63) * 4 + (x & 3);
+  };
+  const unsigned adrSA = scale_at(wm * TM + l16), adrSB = scale_at(BM + wn * TN + l16);
+  struct Frags { Op a[KS][MT]; Op b[KS][NT]; int sa[MX ? MT : 1]; int sb[MX ? NT : 1]; };
   Frags f[2];
-  // read number R of a step: the fragments of A first, then those of B
+  // read number R of a step: the fragments of A first, then those of B, then the scales
   auto read_frag = [&](auto R_, unsigned so, Frags& dst) {
     constexpr int r = decltype(R_)::value;
-    if constexpr (r < KS * MT) {
+    if constexpr (r >= KS * (MT + NT)) {
+      constexpr int t = r - KS * (MT + NT);
+      auto read = [&](auto T_, unsigned adr) {
+        if constexpr (KS == 2) return lds_read_u16<decltype(T_)::value * 64>(adr);
+        else return lds_read_u8<decltype(T_)::value * 64>(adr);
+      };
+      if constexpr (t < MT) dst.sa[t] = read(std::integral_constant<int, t>{}, adrSA + so);
+      else dst.sb[t - MT] = read(std::integral_constant<int, t - MT>{}, adrSB + so);
+    } else if constexpr (r < KS * MT) {
       constexpr int ks = r / MT, t = r % MT;
-      if constexpr (FP8) {
+      if constexpr (WIDE) {
         const i32x4 lo = lds_read_b128<t * 16 * RING_ROW>(adrA[0] + so), hi = lds_read_b128<t * 16 * RING_ROW>(adrA[1] + so);
         dst.a[0][t] = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
       } else {
@@ -314,7 +392,7 @@ __device__ __forceinline__ void gemm_ring_tile(const GemmArgs& p, const int pm, 
       }
     } else {
       constexpr int ks = (r - KS * MT) / NT, t = (r - KS * MT) % NT;
-      if constexpr (FP8) {
+      if constexpr (WIDE) {
         const i32x4 lo = lds_read_b128<t * 16 * RING_ROW>(adrB[0] + so), hi = lds_read_b128<t * 16 * RING_ROW>(adrB[1] + so);
         dst.b[0][t] = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
       } else if constexpr (B_KMAJOR) {
@@ -326,13 +404,17 @@ __device__ __forceinline__ void gemm_ring_tile(const GemmArgs& p, const int pm, 
       }
     }
   };
-  constexpr int NFRAG = KS * (MT + NT);
+  constexpr int NFRAG = KS * (MT + NT) + (MX ? MT + NT : 0);
   auto pin = [&](Frags& x) {
     static_for<KS>([&](auto S_) {
       constexpr int s = decltype(S_)::value;
       static_for<MT>([&](auto T_) { lds_use(x.a[s][decltype(T_)::value]); });
       static_for<NT>([&](auto T_) { lds_use(x.b[s][decltype(T_)::value]); });
     });
+    if constexpr (MX) {
+      static_for<MT>([&](auto T_) { lds_use(x.sa[decltype(T_)::value]); });
+      static_for<NT>([&](auto T_) { lds_use(x.sb[decltype(T_)::value]); });
+    }
   };
 
   f32x4 acc[MT][NT];
@@ -349,8 +431,7 @@ __device__ __forceinline__ void gemm_ring_tile(const GemmArgs& p, const int pm, 
 #pragma unroll
     for (int s = 0; s < NS; s++) {
       if (s < steps && !(s == 0 && skip0)) static_for<L>([&](auto Q_) { issue(Q_, lds0 + s * STAGE, std::true_type{}); });
-      fA += RING_ROW;
-      fB += stepB;
+      advance();
     }
     if (steps >= NS) wait_vmcnt<(NS - 1) * L>(); else wait_vmcnt<0>();   // (all but the youngest NS - 1 steps)
   };
@@ -367,6 +448,9 @@ __device__ __forceinline__ void gemm_ring_tile(const GemmArgs& p, const int pm, 
       if constexpr (B_KMAJOR) load16_sbase<0>(tb[q], kB, voffB[q] + q * 1024 - rowB[q] * 16 + min(rowB[q] * 16, tail - 16));
       else load16_sbase<0>(tb[q], kB, voffB[q] + q * 1024 - (unsigned)(rowB[q] - min(rowB[q], krows - 1)) * (unsigned)p.ldb);
     }
+    int ts = 0;   // (block-scaled: K is a multiple of 128 elements, so an MXFP4 tail is four blocks - one dword of scales - and there is no other)
+    const int bs = wave % BLOCKS;
+    if constexpr (MX) load4_sbase(ts, scale_base(bs) + kfull / RING_ROW * 4 * SD, scale_rows(bs));
     fill(true);
     const i32x4 zero = {0, 0, 0, 0};
 #pragma unroll
@@ -379,6 +463,12 @@ __device__ __forceinline__ void gemm_ring_tile(const GemmArgs& p, const int pm, 
       lds_use(tb[q]);
       const bool in = B_KMAJOR ? rowB[q] * 16 < tail : rowB[q] < krows;
       *(LDS_PTR(i32x4))(uintptr_t)(lds0 + A_BYTES + (wave * LB + q) * 1024 + lane * 16) = in ? tb[q] : zero;
+    }
+    if constexpr (MX) {
+      lds_use(ts);
+#pragma unroll
+      for (int d = 0; d < SD; d++)   // (2^0 beyond K: multiplies zeros)
+        *(LDS_PTR(int))(uintptr_t)(lds0 + S_BYTES + (bs * SD + d) * 256 + lane * 4) = d == 0 ? ts : 0x7f7f7f7f;
     }
     lds_wait<0>();
   } else {
@@ -405,7 +495,8 @@ __device__ __forceinline__ void gemm_ring_tile(const GemmArgs& p, const int pm, 
     block_barrier();
     static_for<NMFMA>([&](auto N_) {
       constexpr int n = decltype(N_)::value, ks = n / (MT * NT), i = (n / NT) % MT, j = n % NT;
-      E::mma(f[P].b[ks][j], f[P].a[ks][i], acc[i][j]);
+      if constexpr (MX) E::template mma<ks>(f[P].b[ks][j], f[P].a[ks][i], acc[i][j], f[P].sb[j], f[P].sa[i]);
+      else E::mma(f[P].b[ks][j], f[P].a[ks][i], acc[i][j]);
       // The reads over the first three quarters of the MFMAs, so that the last ones have returned by the end of the step; the
       // loads over all of them (behind each other they would wait for the memory pipeline, and the MFMAs behind them).
       constexpr int RS = NMFMA * 3 / 4;
@@ -417,8 +508,7 @@ __device__ __forceinline__ void gemm_ring_tile(const GemmArgs& p, const int pm, 
     });
     lds_wait<0>();
     pin(f[P ^ 1]);
-    fA += RING_ROW;
-    fB += stepB;
+    advance();
     cur = next;
     s++;
   };
@@ -464,6 +554,7 @@ __global__ __launch_bounds__(128 * WN, 1) void gemm_ring_kernel(GemmArgs p, int 
     p.K -= k0 / E::kElemBytes;
     p.A += k0;
     p.B += B_KMAJOR ? (int64_t)k0 : (int64_t)(k0 / E::kElemBytes) * p.ldb;
+    if constexpr (E::kScaleDwords > 0) { p.sA += k0 / E::kBlockBytes; p.sB += k0 / E::kBlockBytes; }
     p.C = (char*)(p.workspace + (int64_t)z * p.M * p.N);
     p.ldc = p.N; p.scn = 1; p.out_dtype = 4;        // fp32 partial sums, dense rows (the workspace is 16-byte aligned)
     p.c_vec_ok = p.N % 4 == 0;
@@ -476,7 +567,7 @@ __global__ __launch_bounds__(128 * WN, 1) void gemm_ring_kernel(GemmArgs p, int 
 
 template <typename E, int BM, int BN, int WN, bool B_KMAJOR, int NS>
 static int launch_gemm_ring(const GemmArgs& p, int splits, int chunk_bytes, hipStream_t stream) {
-  constexpr int smem = NS * (BM + BN) * RING_ROW;
+  constexpr int smem = NS * ring_stage_bytes<E, BM, BN>();
   static_assert(smem <= 160 * 1024, "LDS ring does not fit");
   static bool attr_set = false;  // benign race: setting the attribute twice is harmless
   if (!attr_set) {

@@ -131,6 +131,7 @@ int gemm8_launch(const GemmArgs& p, bool e5m2, bool b_kmajor, int tile, hipStrea
 int gemm_ring16_launch(const GemmArgs& p, bool bf16, bool b_kmajor, int shape, int splits, int chunk_bytes, hipStream_t stream);
 int gemm_ring8_launch(const GemmArgs& p, bool e5m2, int shape, int splits, int chunk_bytes, hipStream_t stream);
 int gemm32_launch(const GemmArgs& p, int tile, hipStream_t stream);   // fp32 operands, K-major B; tile as for gemm16_launch
+int gemm_ring_mx_launch(const GemmArgs& p, bool fp4, int shape, int splits, int chunk_bytes, hipStream_t stream);   // K a multiple of 128, scale rows on dwords
 // split-K on 128x128 tiles: `splits` chunks of `chunk_bytes` of every operand row (whole K steps of 64 bytes), fp32
 // partial tiles into p.workspace ([splits][M][N]); splitk_reduce_launch adds them up and does the epilogue
 int gemm8_splitk_launch(const GemmArgs& p, bool e5m2, int splits, int chunk_bytes, hipStream_t stream);   // fp8 operands, row-major B

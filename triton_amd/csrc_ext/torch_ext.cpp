@@ -110,9 +110,13 @@ void mx_gemm(const at::Tensor& a, const at::Tensor& sa, const at::Tensor& b, con
   on_device(a, 0); on_device(sa, 1); on_device(b, 2); on_device(sb, 3); on_device(c, 4);
   TORCH_CHECK(a.dim() == 2 && b.dim() == 2 && sa.dim() == 2 && sb.dim() == 2 && c.dim() == 2, "MX operands, scales and result are matrices");
   const DeviceGuard guard(a.device());
-  const int rc = mi355_mx_gemm((const uint8_t*)a.data_ptr(), (const uint8_t*)sa.data_ptr(), (const uint8_t*)b.data_ptr(),
-                               (const uint8_t*)sb.data_ptr(), c.data_ptr(), (int)a.size(0), (int)b.size(0), (int)K, (int)fmt,
-                               abi_dtype(c), a.stride(0), b.stride(0), sa.stride(0), sb.stride(0), c.stride(0), stream_of(a));
+  const int64_t need = mi355_mx_gemm_workspace((int)a.size(0), (int)b.size(0), (int)K, (int)fmt);
+  at::Tensor ws;
+  if (need > 0) ws = at::empty({need}, c.options().dtype(at::kByte));
+  const int rc = mi355_mx_gemm_ws((const uint8_t*)a.data_ptr(), (const uint8_t*)sa.data_ptr(), (const uint8_t*)b.data_ptr(),
+                                  (const uint8_t*)sb.data_ptr(), c.data_ptr(), (int)a.size(0), (int)b.size(0), (int)K, (int)fmt,
+                                  abi_dtype(c), a.stride(0), b.stride(0), sa.stride(0), sb.stride(0), c.stride(0),
+                                  need > 0 ? ws.data_ptr() : nullptr, (size_t)need, stream_of(a));
   check(rc, "mi355_mx_gemm");
 }
 

@@ -359,10 +359,14 @@ def mx_matmul(a_packed, a_scale, b_packed, b_scale, fmt="mxfp4", out_dtype=torch
     if ext is not None:
         ext.mx_gemm(a_packed, a_scale, b_packed, b_scale, c, f, K)
         return c
-    rc = _lib.load().mi355_mx_gemm(
+    lib = _lib.load()
+    need = lib.mi355_mx_gemm_workspace(M, N, K, f)
+    ws = torch.empty(need, dtype=torch.uint8, device=c.device) if need > 0 else None
+    rc = lib.mi355_mx_gemm_ws(
         a_packed.data_ptr(), a_scale.data_ptr(), b_packed.data_ptr(), b_scale.data_ptr(), c.data_ptr(),
         M, N, K, f, _TORCH_TO_ABI[out_dtype],
-        a_packed.stride(0), b_packed.stride(0), a_scale.stride(0), b_scale.stride(0), c.stride(0), _stream())
+        a_packed.stride(0), b_packed.stride(0), a_scale.stride(0), b_scale.stride(0), c.stride(0),
+        None if ws is None else ws.data_ptr(), need, _stream())
     _lib.check(rc, "mi355_mx_gemm")
     return c
 
