@@ -720,8 +720,8 @@ GemmRoute gemm_route(const void* A, const void* B, int M, int N, int K, int64_t 
     return r;
   }
   if (K % vec != 0) {
-    // (whole pairs of 128-byte K steps where the 256 x 256 tiles are at least half a round: no tail behind their loop)
-    const int to = tiles256 * 2 >= cus && (int64_t)K * es >= 1024 ? 256 : 128;
+    // (whole pairs of 128-byte K steps where there are several rounds of 256 x 256 tiles, whose kernel then walks them as one stream)
+    const int to = tiles256 > cus && (int64_t)K * es >= 1024 ? 256 : 128;
     r.k = (int)up(K, r.pack_b || r.kmajor ? to / es : vec);
     if (!r.kmajor && !r.pack_b) r.k_rows = K;
   }
@@ -1064,30 +1064,18 @@ static int mx_impl(const uint8_t* A, const uint8_t* sA, const uint8_t* B, const 
   int tile = (tiles256 * 2 >= cus) ? (tiles256 % cus == 0 ? 5 : 4) : 1;
   // MXFP4 with whole 256x256 tiles, K at least 1024 and at least half a round of tiles: four waves of
   // scaled 16x16x128 MFMAs (8192^3: 4000-4050 vs 3340-3640 TFLOP/s for the persistent eight-wave kernel)
-  // K beyond the last whole group of K steps (four 128-byte steps for MXFP4, eight for MXFP8) is those kernels' tail
-  // form, whose steps are not pipelined: one costs about 3.5 (MXFP4) / 7 (MXFP8) steps of the main loop (8192 x 8192 x
-  // 8704: MXFP4 3890 vs 3540 TFLOP/s for the eight-wave kernel, MXFP8 2110 vs 2100; x 4608: 3230 vs 3280 and 1740 vs
-  // 2040).  It is chosen where the tail is short against the main loop - and wherever the eight-wave kernels cannot take
-  // the product at all (K bytes not a multiple of 64: 8192 x 8192 x 8224 ran the one-thread-per-output kernel, 700 ms).
-  auto tail_pays = [&](int group_bytes, int cost) {
-    const int tail = p.k_bytes % group_bytes;
-    if (tail == 0) return true;
-    const bool eight_wave_runs = p.k_bytes % 64 == 0 && lds_a % 4 == 0 && lds_b % 4 == 0 && aligned(sA, 4) && aligned(sB, 4);
-    return !eight_wave_runs || (int64_t)((tail + 127) / 128) * cost <= (int64_t)(p.k_bytes - tail) / 128;
-  };
-  // (below half a round of tiles the four-wave kernels still win where K is long - flushed do_bench, four-wave / 128 x 128
-  // tiles: MXFP4 2048 x 2048 x 4096 1010 / 745 TFLOP/s, 1024 x 1024 x 4096 240 / 198, MXFP8 2048 x 2048 x 4096 636 / 407,
-  // 1536 x 1536 x 2048 278 / 219 - and lose where it is short: MXFP4 2048 x 2048 x 1024 427 / 504, 1024^3 117 / 139)
+  const int group = fmt == MI355_MXFP4 ? 512 : 1024;   // bytes of a row in a group of K steps of their streaming forms
+  // (below half a round of tiles too where K is long, next to the ring kernels below)
   const bool enough = tiles256 * 2 >= cus || (tiles256 >= 16 && p.k_bytes >= 1024);
-  if (fmt == MI355_MXFP4 && enough && gemm_wave128_mxfp4_ok(p) && tail_pays(512, 9)) tile = 6;
+  if (fmt == MI355_MXFP4 && enough && gemm_wave128_mxfp4_ok(p)) tile = 6;
   // (MXFP8 likewise: 2530-2570 vs 2110-2240)
-  if (fmt == MI355_MXFP8 && enough && gemm_wave128_mxfp8_ok(p) && tail_pays(1024, 21)) tile = 6;
+  if (fmt == MI355_MXFP8 && enough && gemm_wave128_mxfp8_ok(p)) tile = 6;
   // the same kernels on tiles of 128 x 256 wherever those fit one round of CUs (from 16 on): flushed do_bench, best of
   // the other forms / 128-row tiles, MXFP4: 1024^3 141 / 162 TFLOP/s, 2048 x 2048 x 1024 503 / 600, 2048 x 2048 x 4096 1012 /
   // 1309, 1536 x 2048 x 8192 1071 / 1216, 3072 x 2048 x 4096 1661 / 1854, 2304 x 2048 x 8192 1606 / 1795; MXFP8: 92 / 127,
   // 360 / 491, 644 / 856, 627 / 754, 1072 / 1244, 947 / 1120; beyond one round they lose (3072^3, 288 tiles: MXFP4 2084 for
   // the 192-row tiles / 1555, 4096^3 3209 / 2834)
-  if ((knobs().tile == UNSET || knobs().tile_m == 128) && gemm_wave128_mx_192_ok(p, fmt == MI355_MXFP4 ? 512 : 1024, 128)) {
+  if ((knobs().tile == UNSET || knobs().tile_m == 128) && gemm_wave128_mx_192_ok(p, group, 128)) {
     const long tiles128 = (long)((M + 127) / 128) * ((N + 255) / 256);
     const int want = knob(knobs().tile_m, 0);
     if (want == 128 || (want == 0 && tiles128 >= 16 && tiles128 <= cus)) {
@@ -1099,7 +1087,7 @@ static int mx_impl(const uint8_t* A, const uint8_t* sA, const uint8_t* B, const 
   // do_bench, 256-row choice / 192-row tiles, MXFP4: 3072^3 1750 / 2100 TFLOP/s, 4608 x 4096 x 4096 2475 / 2885, 6144^3
   // 3725 / 3970, 1536 x 8192 x 8192 3205 / 3780, 1536 x 2048 x 8192 880 / 1080; MXFP8: 1255 / 1420, 1480 / 1830, 2275 / 2520,
   // 1945 / 2345, 519 / 630; not taken where they fill worse (3840 x 3840 x 4096: 3080 / 2230)
-  if ((knobs().tile == UNSET || knobs().tile_m == 192) && p.tile_m == 0 && gemm_wave128_mx_192_ok(p, fmt == MI355_MXFP4 ? 512 : 1024)) {
+  if ((knobs().tile == UNSET || knobs().tile_m == 192) && p.tile_m == 0 && gemm_wave128_mx_192_ok(p, group)) {
     auto fill = [&](long t) { return t <= 0 ? 0.0 : (double)t / (double)(((t + cus - 1) / cus) * cus); };
     const long tiles192 = (long)((M + 191) / 192) * ((N + 255) / 256);
     const int want = knob(knobs().tile_m, 0);
@@ -1118,7 +1106,7 @@ static int mx_impl(const uint8_t* A, const uint8_t* sA, const uint8_t* B, const 
   // MXFP4 23.6 / 29.8, MXFP8 34 / 45)
   const bool ring_takes = K % 128 == 0 && lds_a % 4 == 0 && lds_b % 4 == 0 && aligned(sA, 4) && aligned(sB, 4) && lds_a < (1 << 24) && lds_b < (1 << 24);
   if (ring_takes && knobs().tile_m == UNSET && knobs().mixed_rows == UNSET) {
-    const int steps = (p.k_bytes + 127) / 128, group_bytes = fmt == MI355_MXFP4 ? 512 : 1024;
+    const int steps = (p.k_bytes + 127) / 128;
     int shape = -1, splits = 1;
     if (knobs().tile != UNSET) {
       if (knobs().tile >= 8 && knobs().tile <= 10) shape = knobs().tile - 8;
@@ -1126,11 +1114,13 @@ static int mx_impl(const uint8_t* A, const uint8_t* sA, const uint8_t* B, const 
       if (workspace) splits = mx_splits(M, N, p.k_bytes, cus);
       const RingPlan plan = ring_plan(M, N, steps, cus, splits, splits, kMxStep);
       double other = 1e30;
-      // (the eight-wave kernel on 256 x 256 tiles, for what the four-wave ones do not take)
-      if (tile != 6 && tiles256 * 2 >= cus && p.k_bytes % 128 == 0) other = 1.12 * tiles256_us(tiles256, 256, steps, cus, true, true);
       if (tile == 6) {
-        const int rows = p.tile_m ? p.tile_m : 256, tail = (p.k_bytes % group_bytes + 127) / 128;
-        other = tiles256_us((long)((M + rows - 1) / rows) * ((N + 255) / 256), rows, steps - tail + tail * (fmt == MI355_MXFP4 ? 9 : 21), cus, false, true);
+        // (within 15 % of: 4096 x 4096 x 1024 .. 4224 MXFP8 23 .. 58 us, MXFP4 18 .. 45; unlike the 16-bit kernels hardly shorter where
+        // they leave CUs idle: 4096 x 1664 x 1408 MXFP8, 112 tiles, 24.7 us - ring 16.5 -, 3072 x 3072 x 3200, 144 tiles, 42 - ring 51)
+        const int rows = p.tile_m ? p.tile_m : 256;
+        const long tiles = (long)((M + rows - 1) / rows) * ((N + 255) / 256), rounds = (tiles + cus - 1) / cus;
+        const double fill = rounds > 1 ? 1.0 : (double)tiles / cus, share = rows == 256 ? 1.0 : rows == 192 ? 0.78 : 0.64;
+        other = kLaunchUs + (double)rounds * share * (8.0 + 1.5 * steps * (0.7 + 0.3 * fill));
       }
       if (plan.us < other) shape = plan.shape;
       else splits = 1;
@@ -1149,7 +1139,7 @@ static int mx_impl(const uint8_t* A, const uint8_t* sA, const uint8_t* B, const 
   }
   // and on both tile heights in one launch, as for the 16-bit and fp8 products
   if (knobs().tile == UNSET && knobs().tile_m == UNSET && N % 256 == 0) {
-    const int want = knob(knobs().mixed_rows, -1), group = fmt == MI355_MXFP4 ? 512 : 1024;
+    const int want = knob(knobs().mixed_rows, -1);
     int rows = 0;
     if (want > 0) rows = want;
     else if (want < 0 && tile == 6 && p.tile_m == 0 && tiles256 > cus) rows = mixed_split(M, N / 256, cus);

@@ -51,6 +51,73 @@ __device__ __forceinline__ void mfma_drain(f32x4 (&acc)[MT][8]) {
   for (int i = 0; i < MT; i++) mfma_drain_row(acc[i]);
 }
 
+// Rows that are no whole number of 128-byte K steps (the ANYK forms): what is left of them, `rest` bytes, is multiplied FIRST, as
+// step 0, from registers through LDS with zeros beyond K - its loads are the oldest of the prologue, so the second stage
+// fills behind them and the step runs like any other.  Those forms take one tile per workgroup, and an odd number of
+// steps ends with one more step behind the loop.  (A tail multiplied behind the loop, without overlap, cost three to seven steps, a
+// group of scales more than a step: us, with that / so: bf16 8192 x 8192 x 8176 K-major 893 / 794, e4m3 8192 x 8192 x 1664 120 / 110; against the
+// eight-wave kernel: 4096 x 4096 x 1088 fp16 with a bias row 75 / 38, MXFP8 6400 x 7936 x 8064 915 / 377, MXFP4 5376 x 5376 x 6912 212 / 112.)
+// L loads of 8 rows each, 16 bytes a lane, in the order of the direct loads (PERM: chunks of MXFP4 rows, see there).
+template <bool PERM>
+__device__ __forceinline__ int head_chunk(int q, int lane) {
+  const int s = (lane & 7) ^ (((q & 1) * 4 + (lane >> 4)) & 7);
+  return PERM ? 2 * (s & 3) + (s >> 2) : s;
+}
+template <int L, bool PERM = false>
+__device__ __forceinline__ void head_load(i32x4 (&t)[L], const char* src, unsigned pitch, int lane, int rest) {
+#pragma unroll
+  for (int q = 0; q < L; q++) load16_sbase<0>(t[q], src, ((lane >> 3) + 8 * q) * pitch + min(head_chunk<PERM>(q, lane) * 16, rest - 16));
+}
+template <int L, bool PERM = false>
+__device__ __forceinline__ void head_store(i32x4 (&t)[L], unsigned dst, int lane, int rest) {
+  const i32x4 zero = {0, 0, 0, 0};
+#pragma unroll
+  for (int q = 0; q < L; q++) {
+    lds_use(t[q]);
+    *(LDS_PTR(i32x4))(uintptr_t)(dst + q * 1024 + lane * 16) = head_chunk<PERM>(q, lane) * 16 < rest ? t[q] : zero;
+  }
+}
+
+// The e8m0 scales of the block-scaled kernels lie in LDS as 16 bytes a row - a group of G K steps -, A's row r at 16 r and B's
+// behind 256 of those, in two slots.  Scale rows that begin on 16 bytes and a K of whole groups are fetched 16 bytes a lane; the
+// ANYK forms, whose rows begin on dwords, fetch a dword a lane, 16 rows an instruction: a quarter of the wave's rows in
+// each of four steps (G = 2: two quarters in each of two), in the G steps between the last read of the slot and the first of the
+// next.  (A dword of 64 rows an instruction, one for each operand and step, made the loop 12 to 19 % longer: 64 lines to look
+// up instead of 16.)  `bytes`: what a row holds, in whole dwords; the lanes behind it fetch the last one again.
+template <int ROWS, int Q0, int QN, bool SETTLE>
+__device__ __forceinline__ void scale_quarters(const char* sa, const char* sb, unsigned pitch_a, unsigned pitch_b, int q, int at, int bytes, unsigned slot, int wave, int lane) {
+#pragma unroll
+  for (int i = Q0; i < Q0 + QN; i++) {
+    const int row = 16 * (q + i) + (lane >> 2);
+    const unsigned in_row = min(at + 4 * (lane & 3), bytes - 4);
+    if (ROWS == 64 || row < ROWS) async_copy4_sbase<SETTLE>(sa, (unsigned)min(row, ROWS - 1) * pitch_a + in_row, slot + (wave * ROWS + 16 * (q + i)) * 16);
+    async_copy4_sbase<SETTLE>(sb, (unsigned)row * pitch_b + in_row, slot + 4096 + (wave * 64 + 16 * (q + i)) * 16);
+  }
+}
+// The first step of `blocks` scale blocks (see head_load), through registers: dword d of the wave's rows, 2^0 behind the last block.
+template <int SD>
+__device__ __forceinline__ void head_scale_load(int (&t)[2][SD], const char* sa, const char* sb, unsigned off_a, unsigned off_b, int blocks) {
+#pragma unroll
+  for (int d = 0; d < SD; d++) {   // (no dword without a block of the row)
+    const unsigned at = 4 * min(d, (blocks - 1) / 4);
+    load4_sbase(t[0][d], sa, off_a + at);
+    load4_sbase(t[1][d], sb, off_b + at);
+  }
+}
+template <int SD>
+__device__ __forceinline__ void head_scale_store(int (&t)[2][SD], unsigned slot, int wave, int lane, int blocks) {
+#pragma unroll
+  for (int d = 0; d < SD; d++) {
+    const int n = blocks - 4 * d;
+    const unsigned mask = n >= 4 ? ~0u : n <= 0 ? 0u : (1u << (8 * n)) - 1u;
+#pragma unroll
+    for (int o = 0; o < 2; o++) {
+      lds_use(t[o][d]);
+      *(LDS_PTR(int))(uintptr_t)(slot + o * 4096 + (wave * 64 + lane) * 16 + 4 * d) = (int)(((unsigned)t[o][d] & mask) | (0x7f7f7f7fu & ~mask));
+    }
+  }
+}
+
 // Workgroups for `tiles` tiles on at most `cap` CUs.  More tiles than CUs need r = ceil(tiles / cap) rounds
 // however they are dealt: ceil(tiles / r) programs walk r tiles each (the last ones r - 1) as one stream of K
 // steps, without the restart that a fresh workgroup per tile pays, and the CUs left without a program leave

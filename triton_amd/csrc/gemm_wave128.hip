@@ -44,17 +44,14 @@ __device__ __forceinline__ void mfma16(f16x8 a, f16x8 b, f32x4& c) {
 // with the 128 KiB of LDS at `lds0`.  XCD: pass the tile numbers through the per-XCD remap first.  EPI: 0 = every
 // epilogue of the C ABI; 1 = C has the type of the operands, no scales, no activation; 2 = C in a 16-bit type with a bias row
 // at most (rows_epilogue), any N; 3 = the lean epilogue (gemm_epilogue16_lean) with C in the operands' type.
-// TAIL: K bytes need not be a multiple of 256; what is left behind the last pair of K steps (16 .. 240 bytes of
-// every operand row) is multiplied after the K loop, 64 bytes at a time, through a 32 KiB LDS buffer of its own
-// behind the two stages (which by then hold the next tile's first steps): plain loads with a zero fill, one
-// un-pipelined sub-step each - a per-tile cost of a few microseconds that only products with such a K pay
-// (the reference's own uneven-K shape 8192 x 8192 x 8176, python/test/regression/test_performance.py:46).
-template <typename V8, bool B_KMAJOR, bool XCD, int EPI = 0, bool TAIL = false, int BM = 256>
+// ANYK: any K of whole 16-byte chunks, one tile (see head_load); a row-major B may end inside the last step (its p.K rows)
+// where A's padding fills it.  (The reference's own uneven-K shape: 8192 x 8192 x 8176, python/test/regression/test_performance.py:46.)
+template <typename V8, bool B_KMAJOR, bool XCD, int EPI = 0, bool ANYK = false, int BM = 256>
 __device__ __forceinline__ void gemm_wave128_tiles(const GemmArgs& p, int tile, const int tile_step, const unsigned lds0, const int tile_stop = -1) {
 #if MI355_DEVICE_PASS
   // BM = 192: tiles of 192 x 256 (96 x 128 per wave) for problems whose 256 x 256 tiles would leave a quarter or more of
   // the CUs idle - only the A side changes: six direct loads per wave and K step instead of eight, six fragments
-  static_assert((BM == 256 || BM == 192 || BM == 128) && !(TAIL && BM != 256), "tile heights");
+  static_assert((BM == 256 || BM == 192 || BM == 128) && !(ANYK && BM != 256), "tile heights");
   constexpr int BN = 256, ROWB = 128;
   constexpr int A_BYTES = BM * ROWB, STAGE = A_BYTES + BN * ROWB;  // 64 KiB (56 KiB)
   constexpr int MT = BM / 32, NT = 8, KS = 2;                       // 16x16 tiles per wave, 16x16x32 sub-steps per stage
@@ -85,8 +82,10 @@ __device__ __forceinline__ void gemm_wave128_tiles(const GemmArgs& p, int tile, 
   auto col_of = [&](int tn) { return min(tn * BN, last_n0); };
   int pm, pn;
   tile_at(tile, pm, pn);
-  const int nk = TAIL ? (p.k_bytes / (2 * ROWB)) * 2 : p.k_bytes / ROWB;   // K steps of the pipelined loop (an even number)
-  int nk_last = nk;   // the same number, but opaque: see mfma_retire
+  const int part = p.k_bytes % ROWB;   // (ANYK) bytes of the first step of a K that is no whole number of them
+  const int head = !ANYK ? 0 : part > 0 ? part : !B_KMAJOR && p.K * 2 < p.k_bytes ? ROWB : 0;
+  const int nk = ANYK ? (p.k_bytes + ROWB - 1) / ROWB : p.k_bytes / ROWB;   // K steps (an even number without ANYK)
+  int nk_last = nk & ~1;   // the steps of the loop, but opaque: see mfma_retire
   asm volatile("" : "+s"(nk_last));
 
   // ---- direct loads: instruction q = 8 * wave + j moves rows 8 q .. 8 q + 7 of a tile; the swizzle of
@@ -129,7 +128,7 @@ __device__ __forceinline__ void gemm_wave128_tiles(const GemmArgs& p, int tile, 
     const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
     return (const char*)(((uint64_t)hi << 32) | lo);
   };
-  // L2 prefetch (dense kernels without a K tail, whose buffer has the LDS this needs): the two LDS stages let a load
+  // L2 prefetch (dense kernels): the two LDS stages let a load
   // run at most one K step ahead of its use, about a microsecond - enough for operands that the last-level cache
   // holds, not for a first touch in HBM (after the reference's cache flush between timed calls every line is one).
   // So PFD K steps ahead of the loads each wave touches a few lines of the step to come: the 32 tiles that run on
@@ -137,7 +136,7 @@ __device__ __forceinline__ void gemm_wave128_tiles(const GemmArgs& p, int tile, 
   // eight, and the programs split a panel's lines among themselves by their tile coordinates (tile column & 3 picks
   // the quarter of the A rows, tile row & 7 the eighth of the B rows), the four waves split that share again.  One
   // lane per 128-byte line, 16 + 8 lines per wave and K step.
-  constexpr bool PF = XCD && !TAIL && MI355_W128_PREFETCH;
+  constexpr bool PF = XCD && MI355_W128_PREFETCH;
   constexpr int PFD = MI355_W128_PREFETCH_DISTANCE;
   const char* pA = nullptr;
   const char* pB = nullptr;
@@ -223,7 +222,7 @@ __device__ __forceinline__ void gemm_wave128_tiles(const GemmArgs& p, int tile, 
   zero_acc();
 
   // ---- prologue: both stages requested, first fragments of stage 0 read
-  static_for<NLOADS>([&](auto L_) { issue(std::integral_constant<int, load_of(decltype(L_)::value)>{}, fA, fB, lds0, std::true_type{}); });
+  auto second_stage = [&]() {
   static_for<NLOADS>([&](auto L_) { issue(std::integral_constant<int, load_of(decltype(L_)::value)>{}, fA + ROWB, fB + kstepB, lds0 + STAGE, std::true_type{}); });
   fA += 2 * ROWB;
   fB += 2 * (int64_t)kstepB;
@@ -239,6 +238,43 @@ __device__ __forceinline__ void gemm_wave128_tiles(const GemmArgs& p, int tile, 
     pB += 2 * (int64_t)kstepB;
   }
   wait_vmcnt<NLOADS + (PF ? 4 : 0)>();
+  };
+  if (ANYK && head) {   // (one block from the loads to their use: at a join the compiler may copy registers still in flight)
+    const int k_main = p.k_bytes - head;
+    const int krows = p.K - k_main / 2;   // rows of a row-major B in this step
+    i32x4 ta[LA], tb[8];
+    head_load(ta, fA + k_main, (unsigned)p.lda, lane, head);
+    if constexpr (B_KMAJOR) {
+      head_load(tb, fB + k_main, (unsigned)p.ldb, lane, head);
+    } else {
+      const char* const kB = scalar_ptr(p.B + (int64_t)col_of(pn) * 2 + (int64_t)(k_main / 2) * p.ldb);
+#pragma unroll
+      for (int q = 0; q < 8; q++) {
+        const int k = wave * 16 + 2 * q + (lane >> 5);
+        const unsigned in_row = voffB[q] + (unsigned)ioff_of(q) - (2 * q + (lane >> 5)) * (unsigned)p.ldb;
+        load16_sbase<0>(tb[q], kB, (unsigned)min(k, krows - 1) * (unsigned)p.ldb + in_row);
+      }
+    }
+    fA -= ROWB;   // (step s is now the bytes from 128 (s - 1) on)
+    fB -= kstepB;
+    if constexpr (PF) { pA -= ROWB; pB -= kstepB; }
+    second_stage();
+    head_store(ta, lds0 + wave * (LA * 1024), lane, head);
+    if constexpr (B_KMAJOR) {
+      head_store(tb, lds0 + A_BYTES + wave * 8192, lane, head);
+    } else {
+      const i32x4 zero = {0, 0, 0, 0};
+#pragma unroll
+      for (int q = 0; q < 8; q++) {
+        lds_use(tb[q]);
+        *(LDS_PTR(i32x4))(uintptr_t)(lds0 + A_BYTES + wave * 8192 + q * 1024 + lane * 16) = wave * 16 + 2 * q + (lane >> 5) < krows ? tb[q] : zero;
+      }
+    }
+    lds_wait<0>();
+  } else {
+    static_for<NLOADS>([&](auto L_) { issue(std::integral_constant<int, load_of(decltype(L_)::value)>{}, fA, fB, lds0, std::true_type{}); });
+    second_stage();
+  }
   block_barrier();
   using Z = std::integral_constant<int, 0>;
   static_for<NRD>([&](auto OP_) { read_one(OP_, Z{}, Z{}, f[0]); });
@@ -316,71 +352,14 @@ __device__ __forceinline__ void gemm_wave128_tiles(const GemmArgs& p, int tile, 
     // wait for ALL outstanding loads, a full drain in every step (-6 to -12 %).  One full wait per tile in front of
     // the loop tells it that its reloads have landed; the stores of the epilogue are all that this waits for.
     if constexpr (PF) wait_all();
-    for (int kt = 0; kt < nk; kt += 2) {
+    for (int kt = 0; kt < (ANYK ? nk & ~1 : nk); kt += 2) {
       stage(I0{}, touch_a(), touch_b()); advance();
       stage(I1{}, touch_a(), touch_b()); advance();
       if (kt + 2 >= nk_last) mfma_retire();
     }
-    if constexpr (TAIL) {
-      const int k_main = nk * ROWB, tail = p.k_bytes - k_main;   // bytes per row: done, and left (a multiple of 16)
-      const unsigned tailA = lds0 + 2 * STAGE, tailB = tailA + BM * 64;
-      const int n0 = col_of(pn);
-      const char* const tA = p.A + (int64_t)row_of(pm) * p.lda + k_main;
-      for (int h = 0; h * 64 < tail; h++) {
-        // this half-step's 64 bytes of the 256 A rows and of the 256 B rows (K-major B) or its 32 k rows of 512
-        // bytes (row-major B, in the column-group order of the stages): 1024 + 1024 chunks of 16 bytes, four
-        // each per thread, zeros beyond K
-        i32x4 va[4], vb[4];
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-          const int id = tid + 256 * i;
-          {
-            const int row = id >> 2, kb = h * 64 + (id & 3) * 16;
-            va[i] = i32x4{0, 0, 0, 0};
-            if (kb < tail) va[i] = *(const i32x4*)(tA + (int64_t)row * p.lda + kb);
-          }
-          vb[i] = i32x4{0, 0, 0, 0};
-          if constexpr (B_KMAJOR) {
-            const int row = id >> 2, kb = h * 64 + (id & 3) * 16;
-            if (kb < tail) vb[i] = *(const i32x4*)(p.B + (int64_t)(n0 + row) * p.ldb + k_main + kb);
-          } else {
-            const int kr = id >> 5, pc = id & 31;
-            const int k = k_main / 2 + h * 32 + kr;
-            const int lg = (pc >> 1) ^ (2 * (kr & 3)) ^ ((kr >> 3) & 1);
-            if (k < p.K) vb[i] = *(const i32x4*)(p.B + (int64_t)k * p.ldb + (int64_t)n0 * 2 + lg * 32 + (pc & 1) * 16);
-          }
-        }
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-          const int id = tid + 256 * i;
-          *(LDS_PTR(i32x4))(uintptr_t)(tailA + id * 16) = va[i];     // A: row id / 4 at 64 (id / 4), chunk id % 4
-          *(LDS_PTR(i32x4))(uintptr_t)(tailB + id * 16) = vb[i];     // B: the same, or k row id / 32, chunk id % 32
-        }
-        lds_wait<0>();
-        block_barrier();
-        static_for<MT>([&](auto T_) {
-          constexpr int t = decltype(T_)::value;
-          f[1].a[t] = __builtin_bit_cast(V8, lds_read_b128<t * 16 * 64>(tailA + (wm * 128 + l16) * 64 + kg * 16));
-        });
-        static_for<NT>([&](auto T_) {
-          constexpr int t = decltype(T_)::value;
-          if constexpr (B_KMAJOR) {
-            f[1].b[t] = __builtin_bit_cast(V8, lds_read_b128<t * 16 * 64>(tailB + (wn * 128 + l16) * 64 + kg * 16));
-          } else {
-            const unsigned ad = adrB[t] - (lds0 + A_BYTES) + tailB;
-            s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LDS_PTR(s16x4))(uintptr_t)ad);
-            s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LDS_PTR(s16x4))(uintptr_t)(ad + 4 * BN * 2));
-            f[1].b[t] = __builtin_bit_cast(V8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-          }
-        });
-        lds_wait<0>();
-        pin(f[1]);
-        block_barrier();   // every wave holds its fragments: the buffer may be overwritten
-        static_for<NM>([&](auto N_) {
-          constexpr int n = decltype(N_)::value, i = n / NT, j = n % NT;
-          mfma16(f[1].b[j], f[1].a[i], acc[i][j]);
-        });
-      }
+    if (ANYK && (nk & 1)) {
+      substep(I0{}, I0{}, T{}, F{}, nullptr, nullptr);
+      substep(I0{}, I1{}, F{}, F{}, nullptr, nullptr);
       mfma_retire();
     }
     // The next tile's first fragments were requested by reads the compiler cannot see: have them landed
@@ -412,11 +391,11 @@ __device__ __forceinline__ void gemm_wave128_tiles(const GemmArgs& p, int tile, 
 }
 
 // Workgroup b computes the tiles b, b + gridDim.x, ... (the grid: wave128_grid).
-template <typename V8, bool B_KMAJOR, int EPI, bool TAIL = false, int BM = 256>
+template <typename V8, bool B_KMAJOR, int EPI, bool ANYK = false, int BM = 256>
 __global__ __launch_bounds__(256, 1) void gemm_wave128_kernel(GemmArgs p) {
 #if MI355_DEVICE_PASS
   extern __shared__ __attribute__((aligned(1024))) char lds_raw[];
-  gemm_wave128_tiles<V8, B_KMAJOR, true, EPI, TAIL, BM>(p, blockIdx.x, gridDim.x, lds_addr((LDS_PTR(const void))lds_raw));
+  gemm_wave128_tiles<V8, B_KMAJOR, true, EPI, ANYK, BM>(p, blockIdx.x, gridDim.x, lds_addr((LDS_PTR(const void))lds_raw));
 #endif
 }
 
@@ -523,17 +502,6 @@ __global__ __launch_bounds__(256, 1) void gemm_wave128_grouped_kernel(GA ga) {
 // places the two halves directly in the eight-register operand and waits for each fragment just
 // before its first use); the direct global->LDS loads stay invisible to its bookkeeping.
 // ---------------------------------------------------------------------------------------------
-// The tail's fragments come from ordinary loads and moves that the compiler schedules; the MFMAs that read them are
-// assembly it cannot see into: everything that writes these registers has completed behind this statement (the values
-// pass through it) and two idle cycles separate the last such write from the first MFMA.
-template <int NA, int NB>
-__device__ __forceinline__ void settle_operands(i32x8 (&a)[NA], i32x8 (&b)[NB]) {
-#if MI355_DEVICE_PASS
-  static_assert(NA == 4 && NB == 8, "four A fragments and the first four of the B set");
-  asm volatile("s_nop 1" : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]), "+v"(b[0]), "+v"(b[1]), "+v"(b[2]), "+v"(b[3]));
-#endif
-}
-
 template <int FMT>
 __device__ __forceinline__ void mfma16_f8(const i32x8& a, const i32x8& b, f32x4& c) {
 #if MI355_DEVICE_PASS
@@ -543,11 +511,7 @@ __device__ __forceinline__ void mfma16_f8(const i32x8& a, const i32x8& b, f32x4&
 }
 
 // EPI: 0 = every epilogue of the C ABI, 2 = C in a 16-bit type with a bias row at most (rows_epilogue), 3 / 4 = lean epilogue writing fp16 / bf16
-// TAIL: K bytes need not be a multiple of 256 (of 16 still): the main loop does the whole pairs of K steps, and what is
-// left of each row (16 .. 240 bytes, the same for every tile) follows as one or two K steps whose fragments every lane
-// loads straight from global memory - the same two chunks per 128-byte step as from LDS, zeros beyond K, the masked
-// tail of the reference's loop (python/tutorials/03-matrix-multiplication.py:297-298) - into the fragment registers
-// that the pipeline has free at that point (it already holds the next tile's first B and A fragments in the others).
+// ANYK: any K of whole 16-byte chunks, one tile (see head_load); K-major B.
 // B_KMAJOR = false: B is row-major [K, N].  Its stage holds the K step's 128 k rows of 256 bytes (wave w loads the rows
 // 32 w .. 32 w + 31, four per load); the 16-byte chunk c of row k lives in chunk c ^ g(k), g(k) = (k & 7) | 8 ((k >> 4) & 1),
 // and a B fragment is four 8-bit transpose reads (ds_read_b64_tr_b8: within 16 lanes, lane 2 r + h addresses the bytes
@@ -560,10 +524,10 @@ __device__ __forceinline__ void mfma16_f8(const i32x8& a, const i32x8& b, f32x4&
 // wave: 64 x 128, four A fragments; twelve loads for the sixteen MFMAs of a half step), for products with too few
 // 256 x 256 tiles for this kernel.
 // The calling workgroup computes the tiles `tile`, `tile + tile_step`, ... of the problem with the LDS at `lds_raw`.
-template <int FMT, int EPI, bool TAIL = false, bool B_KMAJOR = true, int BM = 256>
+template <int FMT, int EPI, bool ANYK = false, bool B_KMAJOR = true, int BM = 256>
 __device__ __forceinline__ void gemm_wave128_f8_tiles(const GemmArgs& p, int tile, const int tile_step, LDS_PTR(char) const lds_raw) {
-  static_assert(BM == 256 || ((BM == 192 || BM == 128) && !TAIL && (EPI == 3 || EPI == 4)), "192- and 128-row tiles: lean epilogue, no K tail");
-  static_assert(B_KMAJOR || !TAIL, "the K tail loads K-contiguous fragments");
+  static_assert(BM == 256 || ((BM == 192 || BM == 128) && !ANYK && (EPI == 3 || EPI == 4)), "192- and 128-row tiles: lean epilogue, no K tail");
+  static_assert(B_KMAJOR || !ANYK, "a K of any length: K-contiguous rows");
 #if MI355_DEVICE_PASS
   constexpr int BN = 256, ROWB = 128;
   constexpr int A_BYTES = BM * ROWB, STAGE = A_BYTES + BN * ROWB;  // 64 KiB (56 KiB)
@@ -585,8 +549,9 @@ __device__ __forceinline__ void gemm_wave128_f8_tiles(const GemmArgs& p, int til
   auto col_of = [&](int tn) { return min(tn * BN, last_n0); };
   int pm, pn;   // (the tiles are computed as one stream of K steps)
   grouped_tile(xcd_remap(tile, ntiles), num_m, num_n, p.group_m, pm, pn);
-  const int nk = TAIL ? p.k_bytes / (2 * ROWB) * 2 : p.k_bytes / ROWB;
-  int nk_last = nk;   // the same number, but opaque: see mfma_retire
+  const int head = ANYK ? p.k_bytes % ROWB : 0;   // bytes of the first step of a K that is no whole number of them
+  const int nk = (p.k_bytes + ROWB - 1) / ROWB;   // K steps (an even number without ANYK)
+  int nk_last = nk & ~1;   // the steps of the loop, but opaque: see mfma_retire
   asm volatile("" : "+s"(nk_last));
 
   // ---- direct loads, exactly as in the 16-bit kernel (the tiles are the same bytes): a lane offset per load,
@@ -688,7 +653,7 @@ __device__ __forceinline__ void gemm_wave128_f8_tiles(const GemmArgs& p, int til
   zero_acc();
 
   // ---- prologue: both stages requested, B and the first four A fragments of stage 0 read
-  static_for<NLOADS>([&](auto L_) { issue(std::integral_constant<int, load_of(decltype(L_)::value)>{}, fA, fB, lds0, std::true_type{}); });
+  auto second_stage = [&]() {
   static_for<NLOADS>([&](auto L_) { issue(std::integral_constant<int, load_of(decltype(L_)::value)>{}, fA + ROWB, fB + kstepB, lds0 + STAGE, std::true_type{}); });
   fA += 2 * ROWB;
   fB += 2 * kstepB;
@@ -704,6 +669,22 @@ __device__ __forceinline__ void gemm_wave128_f8_tiles(const GemmArgs& p, int til
     pB += 2 * kstepB;
   }
   wait_vmcnt<NLOADS + (PF ? 4 : 0)>();
+  };
+  if (ANYK && head) {   // (one block from the loads to their use: at a join the compiler may copy registers still in flight)
+    i32x4 ta[LA], tb[8];
+    head_load(ta, fA + p.k_bytes - head, (unsigned)p.lda, lane, head);
+    head_load(tb, fB + p.k_bytes - head, (unsigned)p.ldb, lane, head);
+    fA -= ROWB;   // (step s is now the bytes from 128 (s - 1) on)
+    fB -= ROWB;
+    if constexpr (PF) { pA -= ROWB; pB -= ROWB; }
+    second_stage();
+    head_store(ta, lds0 + wave * (LA * 1024), lane, head);
+    head_store(tb, lds0 + A_BYTES + wave * 8192, lane, head);
+    lds_wait<0>();
+  } else {
+    static_for<NLOADS>([&](auto L_) { issue(std::integral_constant<int, load_of(decltype(L_)::value)>{}, fA, fB, lds0, std::true_type{}); });
+    second_stage();
+  }
   block_barrier();
   static_for<NT>([&](auto T_) { b[0][decltype(T_)::value] = read_b(T_, std::integral_constant<int, 0>{}); });
 #pragma unroll
@@ -766,47 +747,14 @@ __device__ __forceinline__ void gemm_wave128_f8_tiles(const GemmArgs& p, int til
   if (nk == 2) { fk = 1; advance(); }
   while (true) {
     if constexpr (PF) wait_all();   // (once per tile: tells the compiler that its own loads have landed, see the 16-bit kernel)
-    for (int kt = 0; kt < nk; kt += 2) {
+    for (int kt = 0; kt < (ANYK ? nk & ~1 : nk); kt += 2) {
       step(I0{}, I0{}, touch_a(), touch_b()); advance();
       step(I1{}, I1{}, touch_a(), touch_b()); advance();
       if (kt + 2 >= nk_last) mfma_retire();
     }
-    if constexpr (TAIL) {
-      // (free here: a1 and the B set 1 - the last step read the next tile's first fragments into a0 and the B set 0)
-      const int k_main = nk * ROWB, tail = p.k_bytes - k_main;
-      int tm = row_of(pm) + wm * 128, tn = col_of(pn) + wn * 128, tl = l16, tk = kg;
-      asm volatile("" : "+s"(tm), "+s"(tn), "+v"(tl), "+v"(tk));   // (keeps this address arithmetic out of the K loop)
-      // a scalar base per fragment and one 32-bit lane offset per operand (gemm_wave128_f8_ok bounds 128 rows plus K)
-      const char* const tA = p.A + (int64_t)tm * p.lda + k_main;
-      const char* const tB = p.B + (int64_t)tn * p.ldb + k_main;
-      const unsigned offA = (unsigned)tl * (unsigned)p.lda + tk * 16, offB = (unsigned)tl * (unsigned)p.ldb + tk * 16;
-      for (int h = 0; h * ROWB < tail; h++) {
-        const bool lo_ok = h * ROWB + tk * 16 < tail, hi_ok = h * ROWB + 64 + tk * 16 < tail;
-        auto frag = [&](const char* src, unsigned off) {
-          i32x4 lo = {0, 0, 0, 0}, hi = {0, 0, 0, 0};
-          if (lo_ok) lo = *(const i32x4*)(src + h * ROWB + (uint64_t)off);
-          if (hi_ok) hi = *(const i32x4*)(src + h * ROWB + 64 + (uint64_t)off);
-          return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-        };
-        // (a quarter of the wave's tile at a time - four B and four A fragments: with all eight B fragments at once the
-        // compiler spills lane offsets of the K loop across the tail and reloads them in front of the loop, behind
-        // the wait there, so that their first use inside the loop would drain every load, in every step)
-        static_for<4>([&](auto Q_) {
-          constexpr int bh = decltype(Q_)::value / 2, ah = decltype(Q_)::value % 2;
-          if constexpr (ah == 0) {
-#pragma unroll
-            for (int t = 0; t < MH; t++) b[1][t] = frag(tB + (int64_t)(bh * MH + t) * 16 * p.ldb, offB);
-          }
-#pragma unroll
-          for (int t = 0; t < MH; t++) a1[t] = frag(tA + (int64_t)(ah * MH + t) * 16 * p.lda, offA);
-          settle_operands(a1, b[1]);
-          static_for<MH * MH>([&](auto N_) {
-            constexpr int n = decltype(N_)::value, i = n / MH, j = n % MH;
-            mfma16_f8<FMT>(b[1][j], a1[i], acc[ah * MH + i][bh * MH + j]);
-          });
-        });
-        mfma_retire();   // (inside the loop's block, like the main loop's: see mfma_retire)
-      }
+    if (ANYK && (nk & 1)) {
+      step(I0{}, I0{}, touch_a(), touch_b());
+      mfma_retire();
     }
     mfma_drain(acc);
     int em = row_of(pm) + wm * (BM / 2), en = col_of(pn) + wn * 128, el = l16, ek = kg;
@@ -824,11 +772,11 @@ __device__ __forceinline__ void gemm_wave128_f8_tiles(const GemmArgs& p, int til
 }
 
 // Workgroup b computes the tiles b, b + gridDim.x, ... (the grid: wave128_grid).
-template <int FMT, int EPI, bool TAIL = false, bool B_KMAJOR = true, int BM = 256>
+template <int FMT, int EPI, bool ANYK = false, bool B_KMAJOR = true, int BM = 256>
 __global__ __launch_bounds__(256, 1) void gemm_wave128_f8_kernel(GemmArgs p) {
 #if MI355_DEVICE_PASS
   extern __shared__ __attribute__((aligned(1024))) char lds_raw[];
-  gemm_wave128_f8_tiles<FMT, EPI, TAIL, B_KMAJOR, BM>(p, blockIdx.x, gridDim.x, (LDS_PTR(char))lds_raw);
+  gemm_wave128_f8_tiles<FMT, EPI, ANYK, B_KMAJOR, BM>(p, blockIdx.x, gridDim.x, (LDS_PTR(char))lds_raw);
 #endif
 }
 
@@ -883,18 +831,18 @@ bool gemm_wave128_f8_mixed_ok(const GemmArgs& p, bool b_kmajor, int rows256) {
   return p.lda * 8 + p.k_bytes < (1ll << 31) && p.ldb * 8 + p.k_bytes < (1ll << 31);
 }
 
-template <int FMT, int EPI, bool TAIL = false, bool B_KMAJOR = true, int BM = 256>
+template <int FMT, int EPI, bool ANYK = false, bool B_KMAJOR = true, int BM = 256>
 static int launch_wave128_f8(const GemmArgs& p, hipStream_t stream) {
   constexpr int smem = 2 * (BM + 256) * 128 + 1024;   // (two stages and the 1 KiB that the L2 touches land in)
   static bool attr_set = false;
   if (!attr_set) {
-    hipError_t e = hipFuncSetAttribute((const void*)gemm_wave128_f8_kernel<FMT, EPI, TAIL, B_KMAJOR, BM>, hipFuncAttributeMaxDynamicSharedMemorySize, smem);
+    hipError_t e = hipFuncSetAttribute((const void*)gemm_wave128_f8_kernel<FMT, EPI, ANYK, B_KMAJOR, BM>, hipFuncAttributeMaxDynamicSharedMemorySize, smem);
     if (e != hipSuccess) return (int)e;
     attr_set = true;
   }
   const int tiles = ((p.M + BM - 1) / BM) * ((p.N + 255) / 256);
-  const int grid = wave128_grid(tiles, p.num_programs);
-  gemm_wave128_f8_kernel<FMT, EPI, TAIL, B_KMAJOR, BM><<<dim3(grid), dim3(256), smem, stream>>>(p);
+  const int grid = ANYK ? tiles : wave128_grid(tiles, p.num_programs);
+  gemm_wave128_f8_kernel<FMT, EPI, ANYK, B_KMAJOR, BM><<<dim3(grid), dim3(256), smem, stream>>>(p);
   return (int)hipGetLastError();
 }
 
@@ -927,12 +875,9 @@ int gemm_wave128_f8_launch(const GemmArgs& p, bool e5m2, bool b_kmajor, hipStrea
   return e5m2 ? launch_wave128_f8<1, 0>(p, stream) : launch_wave128_f8<0, 0>(p, stream);
 }
 
-// fp8: a whole tile at least, a pair of 128-byte K steps; with a K-major B, what is left behind the last pair is the TAIL form's
-// (whole tiles only: its steps cost so much that the smaller tiles are ahead where edges come on top, 5056 x 6400 x 1152 51 us
-// for 43, 7579 x 3328 x 1408 51 for 45)
+// fp8: a whole tile at least, a pair of 128-byte K steps, a K-major B unless K is whole pairs of them
 bool gemm_wave128_f8_ok(const GemmArgs& p, bool b_kmajor) {
   if (!(p.M >= 256 && p.N >= 256 && p.k_bytes % 16 == 0 && p.k_bytes >= 256)) return false;
-  if (p.k_bytes % 256 != 0 && (p.M % 256 != 0 || p.N % 256 != 0)) return false;
   if (p.lda * 8 + p.k_bytes >= (1ll << 31)) return false;
   if (b_kmajor) return p.ldb * 8 + p.k_bytes < (1ll << 31);
   // row-major B: whole pairs of K steps; 32 rows plus a tile row within 32-bit lane offsets
@@ -948,7 +893,7 @@ bool gemm_wave128_f8_192_ok(const GemmArgs& p, bool b_kmajor, int tile_m) {
 }
 
 bool gemm_wave128_ok(const GemmArgs& p, bool b_kmajor) {
-  // a whole tile at least, a pair of 128-byte K steps (what is left behind the last pair: the TAIL form), 32-bit lane offsets
+  // a whole tile at least, a pair of 128-byte K steps, 32-bit lane offsets
   if (!(p.M >= 256 && p.N >= 256 && p.k_bytes % 16 == 0 && p.k_bytes >= 256)) return false;
   if (p.lda * 8 + p.k_bytes >= (1ll << 31)) return false;
   return b_kmajor ? p.ldb * 8 + p.k_bytes < (1ll << 31) : (int64_t)p.K * p.ldb + 512 < (1ll << 31);
@@ -964,18 +909,18 @@ bool gemm_wave128_192_ok(const GemmArgs& p, bool b_kmajor, int in_dtype, int til
   return b_kmajor ? p.ldb * 8 + p.k_bytes < (1ll << 31) : (int64_t)p.K * p.ldb + 512 < (1ll << 31);
 }
 
-template <typename V8, bool B_KMAJOR, int EPI, bool TAIL = false, int BM = 256>
+template <typename V8, bool B_KMAJOR, int EPI, bool ANYK = false, int BM = 256>
 static int launch_wave128(const GemmArgs& p, hipStream_t stream) {
-  constexpr int smem = 2 * (BM + 256) * 128 + (TAIL ? 2 * 256 * 64 : 1024);   // (with the tail buffer: all 160 KiB of the CU; without: 1 KiB that the L2 touches land in)
+  constexpr int smem = 2 * (BM + 256) * 128 + 1024;   // (two stages and the 1 KiB that the L2 touches land in)
   static bool attr_set = false;
   if (!attr_set) {
-    hipError_t e = hipFuncSetAttribute((const void*)gemm_wave128_kernel<V8, B_KMAJOR, EPI, TAIL, BM>, hipFuncAttributeMaxDynamicSharedMemorySize, smem);
+    hipError_t e = hipFuncSetAttribute((const void*)gemm_wave128_kernel<V8, B_KMAJOR, EPI, ANYK, BM>, hipFuncAttributeMaxDynamicSharedMemorySize, smem);
     if (e != hipSuccess) return (int)e;
     attr_set = true;
   }
   const int tiles = ((p.M + BM - 1) / BM) * ((p.N + 255) / 256);
-  const int grid = wave128_grid(tiles, p.num_programs);
-  gemm_wave128_kernel<V8, B_KMAJOR, EPI, TAIL, BM><<<dim3(grid), dim3(256), smem, stream>>>(p);
+  const int grid = ANYK ? tiles : wave128_grid(tiles, p.num_programs);
+  gemm_wave128_kernel<V8, B_KMAJOR, EPI, ANYK, BM><<<dim3(grid), dim3(256), smem, stream>>>(p);
   return (int)hipGetLastError();
 }
 
@@ -1035,7 +980,7 @@ static int gemm_wave128_launch_typed(const GemmArgs& p, bool b_kmajor, bool own_
     return b_kmajor ? launch_wave128<V8, true, 3, false, 192>(p, stream) : launch_wave128<V8, false, 3, false, 192>(p, stream);
   if (p.tile_m == 128)
     return b_kmajor ? launch_wave128<V8, true, 3, false, 128>(p, stream) : launch_wave128<V8, false, 3, false, 128>(p, stream);
-  if (p.k_bytes % 256 != 0) {
+  if (p.k_bytes % 256 != 0 || (!b_kmajor && p.K * 2 < p.k_bytes)) {
     if (own_type_lean) return b_kmajor ? launch_wave128<V8, true, 3, true>(p, stream) : launch_wave128<V8, false, 3, true>(p, stream);
     if (rows_epilogue(p)) return b_kmajor ? launch_wave128<V8, true, 2, true>(p, stream) : launch_wave128<V8, false, 2, true>(p, stream);
     return b_kmajor ? launch_wave128<V8, true, 0, true>(p, stream) : launch_wave128<V8, false, 0, true>(p, stream);

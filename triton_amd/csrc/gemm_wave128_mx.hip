@@ -3,6 +3,7 @@
 // 64 KiB LDS stages filled by direct global->LDS loads with fixed scalar bases - with scaled 16x16x128 f8f6f4
 // MFMAs and the e8m0 block scales travelling through a small LDS ring of their own.
 #include "gemm_wave128.h"
+#include <algorithm>
 
 namespace mi355 {
 
@@ -13,27 +14,6 @@ __device__ __forceinline__ void mfma16_mxfp8(const i32x8& a, const i32x8& b, f32
                : "+a"(c) : "v"(a), "v"(b), "v"(sa), "v"(sb));
 #endif
 }
-// The tails' fragments and scales come from ordinary loads and moves that the compiler schedules; the MFMAs that read
-// them are assembly it cannot see into: everything that writes these registers has completed behind this statement (the
-// values pass through it) and two idle cycles separate the last such write from the first MFMA.
-template <typename R>
-__device__ __forceinline__ void settle_one(R& r) {
-#if MI355_DEVICE_PASS
-  asm volatile("" : "+v"(r));
-#endif
-}
-template <typename... R>
-__device__ __forceinline__ void settle_pass(R&... r) {
-  (settle_one(r), ...);
-}
-template <typename... R>
-__device__ __forceinline__ void settle_tail(R&... r) {
-#if MI355_DEVICE_PASS
-  settle_pass(r...);
-  asm volatile("s_nop 1" ::: "memory");
-  settle_pass(r...);
-#endif
-}
 #ifndef MXFP8_CHUNK
 #define MXFP8_CHUNK(kg, c) ((kg) + 4 * (c))
 #endif
@@ -42,20 +22,18 @@ __device__ __forceinline__ void settle_tail(R&... r) {
 // 128 elements = four scale blocks, the scales travel 16 bytes per row (four K steps) per direct load into a
 // two-slot LDS ring like those of the MXFP4 kernel below.
 // EPI: 0 = general epilogue, 3 / 4 = lean epilogue (gemm_epilogue16_lean) writing fp16 / bf16
-// TAIL: K need not be a multiple of 1024 (of 32 still, the scale block): the main loop does the whole groups of eight K
-// steps, and what is left of each row (32 .. 992 bytes, the same for every tile) follows in K steps whose fragments and
-// scale bytes every lane loads straight from global memory - zeros (and the scale 1) beyond K - into the registers that
-// the pipeline has free at that point, a quarter of the wave's tile at a time.
+// ANYK: any K of whole scale blocks, scale rows that begin on dwords, one tile (see head_load, scale_quarters).
 // BM = 192: tiles of 192 x 256, as in the MXFP4 kernel below.
-template <int EPI, bool TAIL = false, int BM = 256>
+template <int EPI, bool ANYK = false, int BM = 256>
 __device__ __forceinline__ void gemm_wave128_mxfp8_tiles(const GemmArgs& p, int tile, const int tile_step, LDS_PTR(char) const lds_raw) {
-  static_assert(BM == 256 || ((BM == 192 || BM == 128) && !TAIL && (EPI == 3 || EPI == 4)), "192- and 128-row tiles: lean epilogue, no K tail");
+  static_assert(BM == 256 || ((BM == 192 || BM == 128) && !ANYK && (EPI == 3 || EPI == 4)), "192- and 128-row tiles: lean epilogue, no K tail");
 #if MI355_DEVICE_PASS
   constexpr int BN = 256, ROWB = 128;
   constexpr int A_BYTES = BM * ROWB, STAGE = A_BYTES + BN * ROWB;  // 64 KiB (56 KiB)
   constexpr int MT = BM / 32, NT = 8, MH = MT / 2;
   constexpr int LA = BM / 32, NLOADS = LA + 8;                      // direct loads per wave and K step: A, then B
   constexpr int SC_BASE = 2 * STAGE, SC_SLOT = (256 + BN) * 16;     // scale ring behind the two stages (A part: room for 256 rows)
+  constexpr int SD = 1, G = 4, BLOCK = 32;                          // dwords of scales per K step, steps of a group, bytes of a block
   const unsigned lds0 = lds_addr((LDS_PTR(const void))lds_raw);
 
   const int tid = threadIdx.x, lane = tid & 63;
@@ -63,12 +41,17 @@ __device__ __forceinline__ void gemm_wave128_mxfp8_tiles(const GemmArgs& p, int 
   const int wm = wave >> 1, wn = wave & 1;
   const int l16 = lane & 15, kg = lane >> 4;
 
-  const int num_m = p.M / BM, num_n = p.N / BN;
+  // (sizes that are no whole tiles: the last tile of a row or column ends where the matrix does, as in the 16-bit kernel)
+  const int num_m = (p.M + BM - 1) / BM, num_n = (p.N + BN - 1) / BN;
+  const int last_m0 = p.M - BM, last_n0 = p.N - BN;
   const int ntiles = num_m * num_n;
+  auto row_of = [&](int tm) { return min(tm * BM, last_m0); };
+  auto col_of = [&](int tn) { return min(tn * BN, last_n0); };
   int pm, pn;   // (the tiles tile, tile + tile_step, ... are computed as one stream of K steps)
   grouped_tile(xcd_remap(tile, ntiles), num_m, num_n, p.group_m, pm, pn);
-  const int nk = TAIL ? p.k_bytes / (8 * ROWB) * 8 : p.k_bytes / ROWB;
-  int nk_last = nk;   // the same number, but opaque: see mfma_retire
+  const int head = ANYK ? p.k_bytes % ROWB : 0;   // bytes of the first step of a K that is no whole number of them
+  const int nk = (p.k_bytes + ROWB - 1) / ROWB;   // K steps (whole groups without ANYK)
+  int nk_last = ANYK ? nk & ~1 : nk;   // the steps of the loop, but opaque: see mfma_retire
   asm volatile("" : "+s"(nk_last));
 
   // ---- direct loads, exactly as in the 16-bit kernel (the tiles are the same bytes)
@@ -94,16 +77,17 @@ __device__ __forceinline__ void gemm_wave128_mxfp8_tiles(const GemmArgs& p, int 
   const char* pA = nullptr;
   const char* pB = nullptr;
   const unsigned voffPA = (lane % (BM / 16)) * (unsigned)p.lda, voffPB = (lane & 7) * (unsigned)p.ldb;
-  const unsigned touch_lds = lds0 + SC_BASE + 2 * SC_SLOT + wave * 256;
+  const unsigned touch_lds = lds0 + SC_BASE + (ANYK ? 3 : 2) * SC_SLOT + wave * 256;
   auto set_fill_tile = [&](int fm, int fn) {
-    fA = p.A + ((int64_t)fm * BM + wave * (BM / 4)) * p.lda;
-    fB = p.B + ((int64_t)fn * BN + wave * 64) * p.ldb;
+    const int64_t m0 = row_of(fm), n0 = col_of(fn);
+    fA = p.A + (m0 + wave * (BM / 4)) * p.lda;
+    fB = p.B + (n0 + wave * 64) * p.ldb;
     if constexpr (PF) {
-      pA = p.A + ((int64_t)fm * BM + (fn & 3) * (BM / 4) + wave * (BM / 16)) * p.lda;
-      pB = p.B + ((int64_t)fn * BN + (fm & 7) * 32 + wave * 8) * p.ldb;
+      pA = p.A + (m0 + (fn & 3) * (BM / 4) + wave * (BM / 16)) * p.lda;
+      pB = p.B + (n0 + (fm & 7) * 32 + wave * 8) * p.ldb;
     }
-    gSA = (const char*)p.sA + ((int64_t)fm * BM + wave * (BM / 4)) * p.lds_a;
-    gSB = (const char*)p.sB + ((int64_t)fn * BN + wave * 64) * p.lds_b;
+    gSA = (const char*)p.sA + (m0 + wave * (BM / 4)) * p.lds_a;
+    gSB = (const char*)p.sB + (n0 + wave * 64) * p.lds_b;
   };
   set_fill_tile(pm, pn);
   auto load_of = [](int slot) constexpr { return slot < LA ? slot : 8 + slot - LA; };   // load slot -> j (A: 0 .. LA-1, B: 8 .. 15)
@@ -127,10 +111,10 @@ __device__ __forceinline__ void gemm_wave128_mxfp8_tiles(const GemmArgs& p, int 
   const unsigned adrSA = lds0 + SC_BASE + (wm * (BM / 2) + l16) * 16 + kg;
   const unsigned adrSB = lds0 + SC_BASE + 256 * 16 + (wn * 128 + l16) * 16 + kg;
   int sa[2][MT], sb[2][NT];
-  auto read_scale = [&](auto OP_, auto SET_, auto OFF_) {   // OFF: slot * SC_SLOT + (K step & 3) * 4
+  auto read_scale = [&](auto OP_, auto SET_, auto OFF_, unsigned so) {   // OFF: slot * SC_SLOT + (K step & 3) * 4
     constexpr int op = decltype(OP_)::value, set = decltype(SET_)::value, off = decltype(OFF_)::value;
-    if constexpr (op < MT) sa[set][op] = lds_read_u8<off + op * 256>(adrSA);
-    else sb[set][op - MT] = lds_read_u8<off + (op - MT) * 256>(adrSB);
+    if constexpr (op < MT) sa[set][op] = lds_read_u8<off + op * 256>(adrSA + so);
+    else sb[set][op - MT] = lds_read_u8<off + (op - MT) * 256>(adrSB + so);
   };
   auto pin_scales = [&](auto SET_) {
     constexpr int set = decltype(SET_)::value;
@@ -170,8 +154,15 @@ __device__ __forceinline__ void gemm_wave128_mxfp8_tiles(const GemmArgs& p, int 
   zero_acc();
 
   // ---- prologue: both stages requested, B and the first four A fragments of stage 0 read
-  issue_scales(0, std::true_type{});
-  static_for<NLOADS>([&](auto L_) { issue(std::integral_constant<int, load_of(decltype(L_)::value)>{}, fA, fB, lds0, std::true_type{}); });
+  // ANYK: `x` counts the K steps that the scale groups do (a head has its scales in a third slot); in the second half of step x go
+  // out the quarters of group (x + 1) / G + 1 whose turn it is
+  const int sbytes = (p.k_bytes / BLOCK + 3) & ~3;
+  auto scale_turn = [&](int x) {
+    const int g = (x + 1) / G + 1;
+    scale_quarters<BM / 4, 0, 4 / G, false>(gSA, gSB, (unsigned)p.lds_a, (unsigned)p.lds_b, (x + 1) % G * (4 / G), g * 16, sbytes, lds0 + SC_BASE + (g & 1) * SC_SLOT, wave, lane);
+  };
+  auto scale_offset = [&](int x) { return (unsigned)((x / G & 1) * SC_SLOT + x % G * (4 * SD)); };
+  auto second_stage = [&]() {
   static_for<NLOADS>([&](auto L_) { issue(std::integral_constant<int, load_of(decltype(L_)::value)>{}, fA + ROWB, fB + ROWB, lds0 + STAGE, std::true_type{}); });
   fA += 2 * ROWB;
   fB += 2 * ROWB;
@@ -187,8 +178,35 @@ __device__ __forceinline__ void gemm_wave128_mxfp8_tiles(const GemmArgs& p, int 
     pB += 2 * ROWB;
   }
   wait_vmcnt<NLOADS + (PF ? 4 : 0)>();
+  };
+  if (ANYK && head) {   // (one block from the loads to their use: at a join the compiler may copy registers still in flight)
+    const int k_main = p.k_bytes - head, blocks = (head + BLOCK - 1) / BLOCK;
+    i32x4 ta[LA], tb[8];
+    int ts[2][SD];
+    head_load<LA>(ta, fA + k_main, (unsigned)p.lda, lane, head);
+    head_load<8>(tb, fB + k_main, (unsigned)p.ldb, lane, head);
+    head_scale_load<SD>(ts, gSA + k_main / BLOCK, gSB + k_main / BLOCK, voffSA, voffSB, blocks);
+    scale_quarters<BM / 4, 0, 4, true>(gSA, gSB, (unsigned)p.lds_a, (unsigned)p.lds_b, 0, 0, sbytes, lds0 + SC_BASE, wave, lane);
+    fA -= ROWB;   // (step s is now the bytes from 128 (s - 1) on)
+    fB -= ROWB;
+    if constexpr (PF) { pA -= ROWB; pB -= ROWB; }
+    second_stage();
+    head_store<LA>(ta, lds0 + wave * (LA * 1024), lane, head);
+    head_store<8>(tb, lds0 + A_BYTES + wave * 8192, lane, head);
+    head_scale_store<SD>(ts, lds0 + SC_BASE + 2 * SC_SLOT, wave, lane, blocks);
+    lds_wait<0>();
+  } else {
+    if constexpr (ANYK) {
+      scale_quarters<BM / 4, 0, 4, true>(gSA, gSB, (unsigned)p.lds_a, (unsigned)p.lds_b, 0, 0, sbytes, lds0 + SC_BASE, wave, lane);
+      scale_turn(-1);
+    } else {
+      issue_scales(0, std::true_type{});
+    }
+    static_for<NLOADS>([&](auto L_) { issue(std::integral_constant<int, load_of(decltype(L_)::value)>{}, fA, fB, lds0, std::true_type{}); });
+    second_stage();
+  }
   block_barrier();
-  static_for<MT + NT>([&](auto OP_) { read_scale(OP_, std::integral_constant<int, 0>{}, std::integral_constant<int, 0>{}); });
+  static_for<MT + NT>([&](auto OP_) { read_scale(OP_, std::integral_constant<int, 0>{}, std::integral_constant<int, 0>{}, ANYK && head ? 2u * SC_SLOT : 0u); });
   lds_wait<0>();
   pin_scales(std::integral_constant<int, 0>{});
 #pragma unroll
@@ -198,9 +216,10 @@ __device__ __forceinline__ void gemm_wave128_mxfp8_tiles(const GemmArgs& p, int 
 
   // K step U (0..7 within a group of eight: stage and register sets U & 1, scale slot U >> 2); its loads fetch
   // K step `fk` of the fill tile.
-  auto step = [&](auto U_, int fk) {
+  auto step = [&](auto U_, int fk, int x) {   // x (ANYK): the step among those of the scale groups
     constexpr int U = decltype(U_)::value, P = U & 1, cur = U & 1, nxt = cur ^ 1, UN = (U + 1) & 7;
     constexpr int so = P * STAGE, sn = (P ^ 1) * STAGE;
+    const unsigned scales = ANYK ? scale_offset(x + 1) : 0u;   // (of the next step)
     static_for<MH * NT>([&](auto N_) {
       constexpr int n = decltype(N_)::value, i = n / NT, j = n % NT;
       mfma16_mxfp8(b[cur][j], a0[i], acc[i][j], sb[cur][j], sa[cur][i]);
@@ -217,16 +236,17 @@ __device__ __forceinline__ void gemm_wave128_mxfp8_tiles(const GemmArgs& p, int 
       if constexpr (n >= NT && n < NT + MH) a0[n - NT] = read_frag(fragA, sn + (n - NT) * 16 * ROWB);
       // (the next step's scales: one read per two MFMAs, or - 192-row tiles, 14 reads for 24 MFMAs - one per MFMA)
       constexpr int HALF = MH * NT, NSC = MT + NT, EXTRA = NLOADS > HALF / 2 ? NLOADS - HALF / 2 : 0;
-      using OffNext = std::integral_constant<int, (UN >> 2) * SC_SLOT + (UN & 3) * 4>;
+      using OffNext = std::integral_constant<int, ANYK ? 0 : (UN >> 2) * SC_SLOT + (UN & 3) * 4>;
       if constexpr (HALF >= 2 * NSC) {
-        if constexpr (n % 2 == 0) read_scale(std::integral_constant<int, n / 2>{}, std::integral_constant<int, nxt>{}, OffNext{});
+        if constexpr (n % 2 == 0) read_scale(std::integral_constant<int, n / 2>{}, std::integral_constant<int, nxt>{}, OffNext{}, scales);
       } else {
-        if constexpr (n < NSC) read_scale(std::integral_constant<int, n>{}, std::integral_constant<int, nxt>{}, OffNext{});
+        if constexpr (n < NSC) read_scale(std::integral_constant<int, n>{}, std::integral_constant<int, nxt>{}, OffNext{}, scales);
       }
       // (the scales of the K steps fk .. fk + 3 are requested in the third step of every four, into the slot whose
       // last reader was the read for the step before this one)
       // (between the last A load and the first B load, which sets M0 for its group again)
-      if constexpr ((U & 3) == 2 && n == 2 * LA) issue_scales(fk >> 2, std::false_type{});
+      if constexpr (!ANYK && (U & 3) == 2 && n == 2 * LA) issue_scales(fk >> 2, std::false_type{});
+      if constexpr (ANYK && n == 2 * LA) scale_turn(x);
       // (one load per two MFMAs; the 192-row tile has 14 loads for its 24 MFMAs, the 128-row tile 12 for 16: from MFMA R
       // on every MFMA is followed by one.  The loads stay in slot order - A, then B - because only the first of each
       // operand sets M0.)
@@ -259,68 +279,28 @@ __device__ __forceinline__ void gemm_wave128_mxfp8_tiles(const GemmArgs& p, int 
       set_fill_tile(fm, fn);
     }
   };
+  if (ANYK && nk == 2) { fk = 1; advance(); }
   while (true) {
     if constexpr (PF) wait_all();   // (once per tile: tells the compiler that its own loads have landed, see the 16-bit kernel)
-    for (int kt = 0; kt < nk; kt += 8) {
-      static_for<8>([&](auto U_) { step(U_, fk); advance(); });
-      if (kt + 8 >= nk_last) mfma_retire();
-    }
-    if constexpr (TAIL) {
-      // (free here: a1, the B set 1 and the scale set 1 - the last step read the next tile's first fragments and scales
-      // into the others)
-      const int k_main = nk * ROWB, tail = p.k_bytes - k_main;
-      int tm = pm * BM + wm * 128, tn = pn * BN + wn * 128, tl = l16, tk = kg;
-      asm volatile("" : "+s"(tm), "+s"(tn), "+v"(tl), "+v"(tk));   // (keeps this address arithmetic out of the K loop)
-      // a scalar base per fragment and one 32-bit lane offset per operand (gemm_wave128_mxfp8_ok bounds them)
-      const char* const tA = p.A + (int64_t)tm * p.lda + k_main;
-      const char* const tB = p.B + (int64_t)tn * p.ldb + k_main;
-      const uint8_t* const tSA = p.sA + (int64_t)tm * p.lds_a + k_main / 32;
-      const uint8_t* const tSB = p.sB + (int64_t)tn * p.lds_b + k_main / 32;
-      unsigned offA = (unsigned)tl * (unsigned)p.lda + tk * 16, offB = (unsigned)tl * (unsigned)p.ldb + tk * 16;
-      unsigned offSA = (unsigned)tl * (unsigned)p.lds_a + tk, offSB = (unsigned)tl * (unsigned)p.lds_b + tk;
-      for (int h = 0; h * ROWB < tail; h++) {
-        // chunk tk (low registers) and chunk 4 + tk (high registers) of the step; the scale of its block tk
-        const bool lo_ok = h * ROWB + tk * 16 < tail, hi_ok = h * ROWB + 64 + tk * 16 < tail, sc_ok = h * ROWB + tk * 32 < tail;
-        auto frag = [&](const char* src, unsigned off) {
-          i32x4 lo = {0, 0, 0, 0}, hi = {0, 0, 0, 0};
-          if (lo_ok) lo = *(const i32x4*)(src + h * ROWB + (uint64_t)off);
-          if (hi_ok) hi = *(const i32x4*)(src + h * ROWB + 64 + (uint64_t)off);
-          return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-        };
-        auto scale = [&](const uint8_t* src, unsigned off) {
-          int v = 127;   // (2^0: multiplies zeros)
-          if (sc_ok) v = src[h * 4 + (uint64_t)off];
-          return v;
-        };
-        static_for<4>([&](auto Q_) {
-          constexpr int bh = decltype(Q_)::value / 2, ah = decltype(Q_)::value % 2;
-          // (the offsets pass through an assembly statement, which stays behind the MFMAs of the quarter before: the
-          // compiler cannot start this quarter's loads earlier and so needs no second set of registers for them)
-          asm volatile("" : "+v"(offA), "+v"(offB), "+v"(offSA), "+v"(offSB));
-          if constexpr (ah == 0) {
-#pragma unroll
-            for (int t = 0; t < MH; t++) {
-              b[1][t] = frag(tB + (int64_t)(bh * MH + t) * 16 * p.ldb, offB);
-              sb[1][t] = scale(tSB + (int64_t)(bh * MH + t) * 16 * p.lds_b, offSB);
-            }
-          }
-#pragma unroll
-          for (int t = 0; t < MH; t++) {
-            a1[t] = frag(tA + (int64_t)(ah * MH + t) * 16 * p.lda, offA);
-            sa[1][t] = scale(tSA + (int64_t)(ah * MH + t) * 16 * p.lds_a, offSA);
-          }
-          settle_tail(a1[0], a1[1], a1[2], a1[3], b[1][0], b[1][1], b[1][2], b[1][3],
-                      sa[1][0], sa[1][1], sa[1][2], sa[1][3], sb[1][0], sb[1][1], sb[1][2], sb[1][3]);
-          static_for<MH * MH>([&](auto N_) {
-            constexpr int n = decltype(N_)::value, i = n / MH, j = n % MH;
-            mfma16_mxfp8(b[1][j], a1[i], acc[ah * MH + i][bh * MH + j], sb[1][j], sa[1][i]);
-          });
-        });
-        mfma_retire();   // (inside the loop's block, like the main loop's: see mfma_retire)
+    if constexpr (ANYK) {
+      const int x0 = head ? -1 : 0;
+      for (int kt = 0; kt < (nk & ~1); kt += 2) {
+        step(I0{}, fk, kt + x0); advance();
+        step(I1{}, fk, kt + 1 + x0); advance();
+        if (kt + 2 >= nk_last) mfma_retire();
+      }
+      if (nk & 1) {
+        step(I0{}, fk, nk - 1 + x0);
+        mfma_retire();
+      }
+    } else {
+      for (int kt = 0; kt < nk; kt += 8) {
+        static_for<8>([&](auto U_) { step(U_, fk, 0); advance(); });
+        if (kt + 8 >= nk_last) mfma_retire();
       }
     }
     mfma_drain(acc);
-    int em = pm * BM + wm * (BM / 2), en = pn * BN + wn * 128, el = l16, ek = kg;
+    int em = row_of(pm) + wm * (BM / 2), en = col_of(pn) + wn * 128, el = l16, ek = kg;
     asm volatile("" : "+s"(em), "+s"(en), "+v"(el), "+v"(ek));   // (keeps the epilogue's address arithmetic out of the K loop)
     if constexpr (EPI == 3) gemm_epilogue16_lean<MT, NT, _Float16>(acc, p, em, en, el, ek);
     else if constexpr (EPI == 4) gemm_epilogue16_lean<MT, NT, __bf16>(acc, p, em, en, el, ek);
@@ -335,11 +315,11 @@ __device__ __forceinline__ void gemm_wave128_mxfp8_tiles(const GemmArgs& p, int 
 }
 
 // Workgroup b computes the tiles b, b + gridDim.x, ... (the grid: wave128_grid).
-template <int EPI, bool TAIL = false, int BM = 256>
+template <int EPI, bool ANYK = false, int BM = 256>
 __global__ __launch_bounds__(256, 1) void gemm_wave128_mxfp8_kernel(GemmArgs p) {
 #if MI355_DEVICE_PASS
   extern __shared__ __attribute__((aligned(1024))) char lds_raw[];
-  gemm_wave128_mxfp8_tiles<EPI, TAIL, BM>(p, blockIdx.x, gridDim.x, (LDS_PTR(char))lds_raw);
+  gemm_wave128_mxfp8_tiles<EPI, ANYK, BM>(p, blockIdx.x, gridDim.x, (LDS_PTR(char))lds_raw);
 #endif
 }
 
@@ -382,27 +362,31 @@ static int launch_wave128_mxfp8_mixed(const GemmArgs& p, int rows256, hipStream_
   return (int)hipGetLastError();
 }
 
-bool gemm_wave128_mxfp8_ok(const GemmArgs& p) {
-  // whole tiles, at least one group of eight K steps (K >= 1024; what is left behind the last group: the TAIL form),
-  // scale rows that a 16-byte load can fetch
-  return p.M % 256 == 0 && p.N % 256 == 0 && p.k_bytes % 32 == 0 && p.k_bytes >= 1024 &&
-         p.lda * 8 + p.k_bytes < (1ll << 31) && p.ldb * 8 + p.k_bytes < (1ll << 31) &&
-         p.lds_a % 16 == 0 && p.lds_b % 16 == 0 && ((uintptr_t)p.sA | (uintptr_t)p.sB) % 16 == 0 &&
-         p.lds_a * 64 + p.k_bytes / 32 < (1ll << 31) && p.lds_b * 64 + p.k_bytes / 32 < (1ll << 31);
+// a whole tile at least, a pair of 128-byte K steps, 32-bit lane offsets, scale rows that begin on dwords
+static bool mx_sizes_ok(const GemmArgs& p) {
+  return p.M >= 256 && p.N >= 256 && p.k_bytes >= 256 && p.lda * 8 + p.k_bytes < (1ll << 31) && p.ldb * 8 + p.k_bytes < (1ll << 31) &&
+         p.lds_a % 4 == 0 && p.lds_b % 4 == 0 && ((uintptr_t)p.sA | (uintptr_t)p.sB) % 4 == 0 &&
+         p.lds_a * 64 + p.k_bytes / 16 < (1ll << 31) && p.lds_b * 64 + p.k_bytes / 16 < (1ll << 31);
+}
+// scale rows that a 16-byte load can fetch and a K of whole groups of steps: the streaming forms
+static bool mx_whole_groups(const GemmArgs& p, int group_bytes) {
+  return p.k_bytes % group_bytes == 0 && p.lds_a % 16 == 0 && p.lds_b % 16 == 0 && ((uintptr_t)p.sA | (uintptr_t)p.sB) % 16 == 0;
 }
 
-template <int EPI, bool TAIL = false, int BM = 256>
+bool gemm_wave128_mxfp8_ok(const GemmArgs& p) { return mx_sizes_ok(p) && p.k_bytes % 32 == 0; }
+
+template <int EPI, bool ANYK = false, int BM = 256>
 static int launch_wave128_mxfp8(const GemmArgs& p, hipStream_t stream) {
-  constexpr int smem = 2 * (BM + 256) * 128 + 2 * 512 * 16 + 1024;   // (stages, scale ring and the 1 KiB that the L2 touches land in)
+  constexpr int smem = 2 * (BM + 256) * 128 + (ANYK ? 3 : 2) * 512 * 16 + 1024;   // (stages, scale ring and the 1 KiB that the L2 touches land in)
   static bool attr_set = false;
   if (!attr_set) {
-    hipError_t e = hipFuncSetAttribute((const void*)gemm_wave128_mxfp8_kernel<EPI, TAIL, BM>, hipFuncAttributeMaxDynamicSharedMemorySize, smem);
+    hipError_t e = hipFuncSetAttribute((const void*)gemm_wave128_mxfp8_kernel<EPI, ANYK, BM>, hipFuncAttributeMaxDynamicSharedMemorySize, smem);
     if (e != hipSuccess) return (int)e;
     attr_set = true;
   }
-  const int tiles = (p.M / BM) * (p.N / 256);
-  const int grid = wave128_grid(tiles, p.num_programs);
-  gemm_wave128_mxfp8_kernel<EPI, TAIL, BM><<<dim3(grid), dim3(256), smem, stream>>>(p);
+  const int tiles = ((p.M + BM - 1) / BM) * ((p.N + 255) / 256);
+  const int grid = ANYK ? tiles : wave128_grid(tiles, p.num_programs);
+  gemm_wave128_mxfp8_kernel<EPI, ANYK, BM><<<dim3(grid), dim3(256), smem, stream>>>(p);
   return (int)hipGetLastError();
 }
 
@@ -412,7 +396,7 @@ int gemm_wave128_mxfp8_launch(const GemmArgs& p, hipStream_t stream) {
     return lean == 1 ? launch_wave128_mxfp8<3, false, 192>(p, stream) : launch_wave128_mxfp8<4, false, 192>(p, stream);
   if (p.tile_m == 128)
     return lean == 1 ? launch_wave128_mxfp8<3, false, 128>(p, stream) : launch_wave128_mxfp8<4, false, 128>(p, stream);
-  if (p.k_bytes % 1024 != 0)
+  if (!mx_whole_groups(p, 1024))
     return lean == 1 ? launch_wave128_mxfp8<3, true>(p, stream) : lean == 2 ? launch_wave128_mxfp8<4, true>(p, stream) : launch_wave128_mxfp8<0, true>(p, stream);
   return lean == 1 ? launch_wave128_mxfp8<3>(p, stream) : lean == 2 ? launch_wave128_mxfp8<4>(p, stream) : launch_wave128_mxfp8<0>(p, stream);
 }
@@ -442,19 +426,17 @@ __device__ __forceinline__ void mfma16_mxfp4(const i32x4& a, const i32x4& b, f32
 }
 
 // EPI: 0 = general epilogue, 3 / 4 = lean epilogue (gemm_epilogue16_lean) writing fp16 / bf16
-// TAIL: K need not be a multiple of 1024 (of 32 still, the scale block): the main loop does the whole groups of four K
-// steps, and what is left of each row (16 .. 496 bytes, the same for every tile) follows in K steps whose fragments and
-// scale bytes every lane loads straight from global memory - zeros (and the scale 1) beyond K - into the fragment and
-// scale registers that the pipeline has free at that point.
+// ANYK: any K of whole scale blocks, scale rows that begin on dwords, one tile (see head_load, scale_quarters).
 // BM = 192: tiles of 192 x 256 (a wave: 96 x 128, six A fragments, 48 of the tile's A rows and scale rows to fetch), for
 // products whose 256 x 256 tiles fill the last round of CUs badly; lean epilogue, K steps in whole groups.
-template <int EPI, bool TAIL = false, int BM = 256>
+template <int EPI, bool ANYK = false, int BM = 256>
 __device__ __forceinline__ void gemm_wave128_mxfp4_tiles(const GemmArgs& p, int tile, const int tile_step, LDS_PTR(char) const lds_raw) {
-  static_assert(BM == 256 || ((BM == 192 || BM == 128) && !TAIL && (EPI == 3 || EPI == 4)), "192- and 128-row tiles: lean epilogue, no K tail");
+  static_assert(BM == 256 || ((BM == 192 || BM == 128) && !ANYK && (EPI == 3 || EPI == 4)), "192- and 128-row tiles: lean epilogue, no K tail");
 #if MI355_DEVICE_PASS
   constexpr int BN = 256, ROWB = 128;
   constexpr int A_BYTES = BM * ROWB, STAGE = A_BYTES + BN * ROWB;  // 64 KiB (56 KiB)
   constexpr int SC_BASE = 2 * STAGE, SC_SLOT = (256 + BN) * 16;     // scale ring behind the two stages (A part: room for 256 rows)
+  constexpr int SD = 2, G = 2, BLOCK = 16;                          // dwords of scales per K step, steps of a group, bytes of a block
   constexpr int MT = BM / 32, NT = 8, KS = 2, NM = MT * NT, NRD = MT + NT;
   constexpr int LA = BM / 32, NLOADS = LA + 8;                      // direct loads per wave and K step: A, then B
   constexpr int EVERY = NM / 16;                                    // MFMAs per load slot: 4 (64 MFMAs) or 3 (48)
@@ -465,12 +447,17 @@ __device__ __forceinline__ void gemm_wave128_mxfp4_tiles(const GemmArgs& p, int 
   const int wm = wave >> 1, wn = wave & 1;
   const int l16 = lane & 15, kg = lane >> 4;
 
-  const int num_m = p.M / BM, num_n = p.N / BN;
+  // (sizes that are no whole tiles: the last tile of a row or column ends where the matrix does, as in the 16-bit kernel)
+  const int num_m = (p.M + BM - 1) / BM, num_n = (p.N + BN - 1) / BN;
+  const int last_m0 = p.M - BM, last_n0 = p.N - BN;
   const int ntiles = num_m * num_n;
+  auto row_of = [&](int tm) { return min(tm * BM, last_m0); };
+  auto col_of = [&](int tn) { return min(tn * BN, last_n0); };
   int pm, pn;   // (the tiles tile, tile + tile_step, ... are computed as one stream of K steps)
   grouped_tile(xcd_remap(tile, ntiles), num_m, num_n, p.group_m, pm, pn);
-  const int nk = TAIL ? p.k_bytes / (4 * ROWB) * 4 : p.k_bytes / ROWB;
-  int nk_last = nk;   // the same number, but opaque: see mfma_retire
+  const int head = ANYK ? p.k_bytes % ROWB : 0;   // bytes of the first step of a K that is no whole number of them
+  const int nk = (p.k_bytes + ROWB - 1) / ROWB;   // K steps (whole groups without ANYK)
+  int nk_last = ANYK ? nk & ~1 : nk;   // the steps of the loop, but opaque: see mfma_retire
   asm volatile("" : "+s"(nk_last));
 
   // ---- operand loads, as in the 16-bit kernel
@@ -499,16 +486,17 @@ __device__ __forceinline__ void gemm_wave128_mxfp4_tiles(const GemmArgs& p, int 
   const char* pA = nullptr;
   const char* pB = nullptr;
   const unsigned voffPA = (lane % (BM / 16)) * (unsigned)p.lda, voffPB = (lane & 7) * (unsigned)p.ldb;
-  const unsigned touch_lds = lds0 + SC_BASE + 2 * SC_SLOT + wave * 256;
+  const unsigned touch_lds = lds0 + SC_BASE + (ANYK ? 3 : 2) * SC_SLOT + wave * 256;
   auto set_fill_tile = [&](int fm, int fn) {
-    fA = p.A + ((int64_t)fm * BM + wave * (BM / 4)) * p.lda;
-    fB = p.B + ((int64_t)fn * BN + wave * 64) * p.ldb;
+    const int64_t m0 = row_of(fm), n0 = col_of(fn);
+    fA = p.A + (m0 + wave * (BM / 4)) * p.lda;
+    fB = p.B + (n0 + wave * 64) * p.ldb;
     if constexpr (PF) {
-      pA = p.A + ((int64_t)fm * BM + (fn & 3) * (BM / 4) + wave * (BM / 16)) * p.lda;
-      pB = p.B + ((int64_t)fn * BN + (fm & 7) * 32 + wave * 8) * p.ldb;
+      pA = p.A + (m0 + (fn & 3) * (BM / 4) + wave * (BM / 16)) * p.lda;
+      pB = p.B + (n0 + (fm & 7) * 32 + wave * 8) * p.ldb;
     }
-    gSA = (const char*)p.sA + ((int64_t)fm * BM + wave * (BM / 4)) * p.lds_a;
-    gSB = (const char*)p.sB + ((int64_t)fn * BN + wave * 64) * p.lds_b;
+    gSA = (const char*)p.sA + (m0 + wave * (BM / 4)) * p.lds_a;
+    gSB = (const char*)p.sB + (n0 + wave * 64) * p.lds_b;
   };
   set_fill_tile(pm, pn);
   auto load_of = [](int slot) constexpr { return slot < LA ? slot : 8 + slot - LA; };   // load slot -> j (A: 0 .. LA-1, B: 8 .. 15)
@@ -556,10 +544,10 @@ __device__ __forceinline__ void gemm_wave128_mxfp4_tiles(const GemmArgs& p, int 
   const unsigned adrSA = lds0 + SC_BASE + (wm * (BM / 2) + l16) * 16 + 2 * kg;
   const unsigned adrSB = lds0 + SC_BASE + 256 * 16 + (wn * 128 + l16) * 16 + 2 * kg;
   int sa[2][MT], sb[2][NT];
-  auto read_scale = [&](auto OP_, auto SET_, auto OFF_) {   // OFF: slot * SC_SLOT + (K step & 1) * 8
+  auto read_scale = [&](auto OP_, auto SET_, auto OFF_, unsigned so) {   // OFF: slot * SC_SLOT + (K step & 1) * 8
     constexpr int op = decltype(OP_)::value, set = decltype(SET_)::value, off = decltype(OFF_)::value;
-    if constexpr (op < MT) sa[set][op] = lds_read_u16<off + op * 256>(adrSA);
-    else sb[set][op - MT] = lds_read_u16<off + (op - MT) * 256>(adrSB);
+    if constexpr (op < MT) sa[set][op] = lds_read_u16<off + op * 256>(adrSA + so);
+    else sb[set][op - MT] = lds_read_u16<off + (op - MT) * 256>(adrSB + so);
   };
   auto pin_scales = [&](auto SET_) {
     constexpr int set = decltype(SET_)::value;
@@ -579,8 +567,15 @@ __device__ __forceinline__ void gemm_wave128_mxfp4_tiles(const GemmArgs& p, int 
   // ---- prologue
   using I0 = std::integral_constant<int, 0>; using I1 = std::integral_constant<int, 1>;
   using T = std::true_type; using F = std::false_type;
-  issue_scales(0, std::true_type{});
-  static_for<NLOADS>([&](auto L_) { issue(std::integral_constant<int, load_of(decltype(L_)::value)>{}, fA, fB, lds0, std::true_type{}); });
+  // ANYK: `x` counts the K steps that the scale groups do (a head has its scales in a third slot); in the second half of step x go
+  // out the quarters of group (x + 1) / G + 1 whose turn it is
+  const int sbytes = (p.k_bytes / BLOCK + 3) & ~3;
+  auto scale_turn = [&](int x) {
+    const int g = (x + 1) / G + 1;
+    scale_quarters<BM / 4, 0, 4 / G, false>(gSA, gSB, (unsigned)p.lds_a, (unsigned)p.lds_b, (x + 1) % G * (4 / G), g * 16, sbytes, lds0 + SC_BASE + (g & 1) * SC_SLOT, wave, lane);
+  };
+  auto scale_offset = [&](int x) { return (unsigned)((x / G & 1) * SC_SLOT + x % G * (4 * SD)); };
+  auto second_stage = [&]() {
   static_for<NLOADS>([&](auto L_) { issue(std::integral_constant<int, load_of(decltype(L_)::value)>{}, fA + ROWB, fB + ROWB, lds0 + STAGE, std::true_type{}); });
   fA += 2 * ROWB;
   fB += 2 * ROWB;
@@ -596,16 +591,44 @@ __device__ __forceinline__ void gemm_wave128_mxfp4_tiles(const GemmArgs& p, int 
     pB += 2 * ROWB;
   }
   wait_vmcnt<NLOADS + (PF ? 4 : 0)>();
+  };
+  if (ANYK && head) {   // (one block from the loads to their use: at a join the compiler may copy registers still in flight)
+    const int k_main = p.k_bytes - head, blocks = (head + BLOCK - 1) / BLOCK;
+    i32x4 ta[LA], tb[8];
+    int ts[2][SD];
+    head_load<LA, true>(ta, fA + k_main, (unsigned)p.lda, lane, head);
+    head_load<8, true>(tb, fB + k_main, (unsigned)p.ldb, lane, head);
+    head_scale_load<SD>(ts, gSA + k_main / BLOCK, gSB + k_main / BLOCK, voffSA, voffSB, blocks);
+    scale_quarters<BM / 4, 0, 4, true>(gSA, gSB, (unsigned)p.lds_a, (unsigned)p.lds_b, 0, 0, sbytes, lds0 + SC_BASE, wave, lane);
+    fA -= ROWB;   // (step s is now the bytes from 128 (s - 1) on)
+    fB -= ROWB;
+    if constexpr (PF) { pA -= ROWB; pB -= ROWB; }
+    second_stage();
+    head_store<LA, true>(ta, lds0 + wave * (LA * 1024), lane, head);
+    head_store<8, true>(tb, lds0 + A_BYTES + wave * 8192, lane, head);
+    head_scale_store<SD>(ts, lds0 + SC_BASE + 2 * SC_SLOT, wave, lane, blocks);
+    lds_wait<0>();
+  } else {
+    if constexpr (ANYK) {
+      scale_quarters<BM / 4, 0, 4, true>(gSA, gSB, (unsigned)p.lds_a, (unsigned)p.lds_b, 0, 0, sbytes, lds0 + SC_BASE, wave, lane);
+      scale_turn(-1);
+    } else {
+      issue_scales(0, std::true_type{});
+    }
+    static_for<NLOADS>([&](auto L_) { issue(std::integral_constant<int, load_of(decltype(L_)::value)>{}, fA, fB, lds0, std::true_type{}); });
+    second_stage();
+  }
   block_barrier();
   static_for<NRD>([&](auto OP_) { read_one(OP_, I0{}, I0{}, f[0]); });
-  static_for<NRD>([&](auto OP_) { read_scale(OP_, I0{}, I0{}); });
+  static_for<NRD>([&](auto OP_) { read_scale(OP_, I0{}, I0{}, ANYK && head ? 2u * SC_SLOT : 0u); });
   lds_wait<0>();
   pin_scales(I0{});
 
   // K step U (0..3 within a group of four: stage U & 1, scale slot U >> 1)
-  auto step = [&](auto U_, int fk) {   // fk: the K step (of the fill tile) that this step's loads fetch
+  auto step = [&](auto U_, int fk, int x) {   // fk: the K step (of the fill tile) that this step's loads fetch; x (ANYK): the step among those of the scale groups
     constexpr int U = decltype(U_)::value, P = U & 1, UN = (U + 1) & 3;
-    using OffNext = std::integral_constant<int, (UN >> 1) * SC_SLOT + (UN & 1) * 8>;
+    using OffNext = std::integral_constant<int, ANYK ? 0 : (UN >> 1) * SC_SLOT + (UN & 1) * 8>;
+    const unsigned scales = ANYK ? scale_offset(x + 1) : 0u;   // (of the next step)
     // sub-step 0 (blocks 2 kg); meanwhile the fragments of sub-step 1
     static_for<NM>([&](auto N_) {
       constexpr int n = decltype(N_)::value, i = n / NT, j = n % NT;
@@ -622,12 +645,13 @@ __device__ __forceinline__ void gemm_wave128_mxfp4_tiles(const GemmArgs& p, int 
       constexpr int n = decltype(N_)::value, i = n / NT, j = n % NT;
       mfma16_mxfp4<1>(f[1].b[j], f[1].a[i], acc[i][j], sb[P][j], sa[P][i]);
       if constexpr (n % 2 == 0 && n / 2 < NRD) read_one(std::integral_constant<int, n / 2>{}, std::integral_constant<int, P ^ 1>{}, I0{}, f[0]);
-      if constexpr (n % 2 == 1 && n / 2 < NRD) read_scale(std::integral_constant<int, n / 2>{}, std::integral_constant<int, P ^ 1>{}, OffNext{});
+      if constexpr (n % 2 == 1 && n / 2 < NRD) read_scale(std::integral_constant<int, n / 2>{}, std::integral_constant<int, P ^ 1>{}, OffNext{}, scales);
       if constexpr (n % EVERY == 1 && n / EVERY < NLOADS) issue(std::integral_constant<int, load_of(n / EVERY)>{}, fA, fB, lds0 + P * STAGE, std::false_type{});   // one per 64 (48) cycles
       // (the scales of the K steps fk, fk + 1 are requested in the even steps, into the slot that the pair
       // two steps back used: its last readers were the reads of that pair's second step, in its sub-step 0)
       // (after the last operand load: the eight loads of an operand share the M0 value that the first one sets)
-      if constexpr (P == 0 && n == NM - 2) issue_scales(fk >> 1, std::false_type{});
+      if constexpr (!ANYK && P == 0 && n == NM - 2) issue_scales(fk >> 1, std::false_type{});
+      if constexpr (ANYK && n == NM - 2) scale_turn(x);
       if constexpr (n % 2 == 1) __builtin_amdgcn_sched_barrier(0);
     });
     if constexpr (PF) {
@@ -658,67 +682,31 @@ __device__ __forceinline__ void gemm_wave128_mxfp4_tiles(const GemmArgs& p, int 
       set_fill_tile(fm, fn);
     }
   };
+  if (ANYK && nk == 2) { fk = 1; advance(); }
   while (true) {
     if constexpr (PF) wait_all();   // (once per tile: tells the compiler that its own loads have landed, see the 16-bit kernel)
-    for (int kt = 0; kt < nk; kt += 4) {
-      step(I0{}, fk); advance();
-      step(I1{}, fk); advance();
-      step(I2{}, fk); advance();
-      step(I3{}, fk); advance();
-      if (kt + 4 >= nk_last) mfma_retire();
-    }
-    if constexpr (TAIL) {
-      // (free here: the fragment set 1 and the scale set 1 - the last step read the next tile's first fragments and
-      // scales into the sets 0)
-      const int k_main = nk * ROWB, tail = p.k_bytes - k_main;
-      int tm = pm * BM + wm * 128, tn = pn * BN + wn * 128, tl = l16, tk = kg;
-      asm volatile("" : "+s"(tm), "+s"(tn), "+v"(tl), "+v"(tk));   // (keeps this address arithmetic out of the K loop)
-      // a scalar base per fragment and one 32-bit lane offset per operand (gemm_wave128_mxfp4_ok bounds them)
-      const char* const tA = p.A + (int64_t)tm * p.lda + k_main;
-      const char* const tB = p.B + (int64_t)tn * p.ldb + k_main;
-      const uint8_t* const tSA = p.sA + (int64_t)tm * p.lds_a + k_main / 16;
-      const uint8_t* const tSB = p.sB + (int64_t)tn * p.lds_b + k_main / 16;
-      const unsigned offA = (unsigned)tl * (unsigned)p.lda + tk * 32, offB = (unsigned)tl * (unsigned)p.ldb + tk * 32;
-      const unsigned offSA = (unsigned)tl * (unsigned)p.lds_a + tk * 2, offSB = (unsigned)tl * (unsigned)p.lds_b + tk * 2;
-      for (int h = 0; h * ROWB < tail; h++) {
-        // the blocks 2 tk (sub-step 0) and 2 tk + 1 (sub-step 1) of the step; their scales in bytes 0 and 1
-        const bool ok0 = h * ROWB + tk * 32 < tail, ok1 = h * ROWB + tk * 32 + 16 < tail;
-        auto scale = [&](const uint8_t* src, unsigned off) {
-          int v0 = 127, v1 = 127;   // (2^0: multiplies zeros)
-          if (ok0) v0 = src[h * 8 + (uint64_t)off];
-          if (ok1) v1 = src[h * 8 + 1 + (uint64_t)off];
-          return v0 | (v1 << 8);
-        };
-#pragma unroll
-        for (int t = 0; t < MT; t++) sa[1][t] = scale(tSA + (int64_t)t * 16 * p.lds_a, offSA);
-#pragma unroll
-        for (int t = 0; t < NT; t++) sb[1][t] = scale(tSB + (int64_t)t * 16 * p.lds_b, offSB);
-        static_for<KS>([&](auto KS_) {
-          constexpr int ks = decltype(KS_)::value;
-          const bool ok = ks == 0 ? ok0 : ok1;
-          auto frag = [&](const char* src, unsigned off) {
-            i32x4 v = {0, 0, 0, 0};
-            if (ok) v = *(const i32x4*)(src + h * ROWB + ks * 16 + (uint64_t)off);
-            return v;
-          };
-#pragma unroll
-          for (int t = 0; t < MT; t++) f[1].a[t] = frag(tA + (int64_t)t * 16 * p.lda, offA);
-#pragma unroll
-          for (int t = 0; t < NT; t++) f[1].b[t] = frag(tB + (int64_t)t * 16 * p.ldb, offB);
-          settle_pass(sa[1][0], sa[1][1], sa[1][2], sa[1][3], sa[1][4], sa[1][5], sa[1][6], sa[1][7],
-                      sb[1][0], sb[1][1], sb[1][2], sb[1][3], sb[1][4], sb[1][5], sb[1][6], sb[1][7]);
-          settle_tail(f[1].a[0], f[1].a[1], f[1].a[2], f[1].a[3], f[1].a[4], f[1].a[5], f[1].a[6], f[1].a[7],
-                      f[1].b[0], f[1].b[1], f[1].b[2], f[1].b[3], f[1].b[4], f[1].b[5], f[1].b[6], f[1].b[7]);
-          static_for<NM>([&](auto N_) {
-            constexpr int n = decltype(N_)::value, i = n / NT, j = n % NT;
-            mfma16_mxfp4<ks>(f[1].b[j], f[1].a[i], acc[i][j], sb[1][j], sa[1][i]);
-          });
-        });
-        mfma_retire();   // (inside the loop's block, like the main loop's: see mfma_retire)
+    if constexpr (ANYK) {
+      const int x0 = head ? -1 : 0;
+      for (int kt = 0; kt < (nk & ~1); kt += 2) {
+        step(I0{}, fk, kt + x0); advance();
+        step(I1{}, fk, kt + 1 + x0); advance();
+        if (kt + 2 >= nk_last) mfma_retire();
+      }
+      if (nk & 1) {
+        step(I0{}, fk, nk - 1 + x0);
+        mfma_retire();
+      }
+    } else {
+      for (int kt = 0; kt < nk; kt += 4) {
+        step(I0{}, fk, 0); advance();
+        step(I1{}, fk, 0); advance();
+        step(I2{}, fk, 0); advance();
+        step(I3{}, fk, 0); advance();
+        if (kt + 4 >= nk_last) mfma_retire();
       }
     }
     mfma_drain(acc);
-    int em = pm * BM + wm * (BM / 2), en = pn * BN + wn * 128, el = l16, ek = kg;
+    int em = row_of(pm) + wm * (BM / 2), en = col_of(pn) + wn * 128, el = l16, ek = kg;
     asm volatile("" : "+s"(em), "+s"(en), "+v"(el), "+v"(ek));   // (keeps the epilogue's address arithmetic out of the K loop)
     if constexpr (EPI == 3) gemm_epilogue16_lean<MT, NT, _Float16>(acc, p, em, en, el, ek);
     else if constexpr (EPI == 4) gemm_epilogue16_lean<MT, NT, __bf16>(acc, p, em, en, el, ek);
@@ -733,11 +721,11 @@ __device__ __forceinline__ void gemm_wave128_mxfp4_tiles(const GemmArgs& p, int 
 }
 
 // Workgroup b computes the tiles b, b + gridDim.x, ... (the grid: wave128_grid).
-template <int EPI, bool TAIL = false, int BM = 256>
+template <int EPI, bool ANYK = false, int BM = 256>
 __global__ __launch_bounds__(256, 1) void gemm_wave128_mxfp4_kernel(GemmArgs p) {
 #if MI355_DEVICE_PASS
   extern __shared__ __attribute__((aligned(1024))) char lds_raw[];
-  gemm_wave128_mxfp4_tiles<EPI, TAIL, BM>(p, blockIdx.x, gridDim.x, (LDS_PTR(char))lds_raw);
+  gemm_wave128_mxfp4_tiles<EPI, ANYK, BM>(p, blockIdx.x, gridDim.x, (LDS_PTR(char))lds_raw);
 #endif
 }
 
@@ -789,42 +777,32 @@ int gemm_wave128_mx_mixed_launch(const GemmArgs& p, int fmt, int rows256, hipStr
 
 // the first `rows256` rows on 256-row tiles and the rest on 192-row tiles, under the conditions of the 192-row tiles
 bool gemm_wave128_mx_mixed_ok(const GemmArgs& p, int group_bytes, int rows256) {
-  if (!(rows256 > 0 && rows256 < p.M && rows256 % 256 == 0 && (p.M - rows256) % 192 == 0)) return false;
-  GemmArgs q = p;
-  q.M = 768;   // (a multiple of both tile heights: the other conditions of gemm_wave128_mx_192_ok)
-  return gemm_wave128_mx_192_ok(q, group_bytes, 192);
+  if (!(rows256 > 0 && rows256 < p.M && rows256 % 256 == 0 && (p.M - rows256) % 192 == 0 && p.N % 256 == 0)) return false;
+  return gemm_wave128_mx_192_ok(p, group_bytes, 192);
 }
 
-// the block-scaled forms on tiles of 192 x 256: M a multiple of 192, whole groups of K steps (`group_bytes` of a row: 512
-// for MXFP4, 1024 for MXFP8), a 16-bit C through the lean epilogue
+// the block-scaled forms on tiles of 192 x 256 or 128 x 256: whole groups of K steps (`group_bytes` of a row: 512 for MXFP4, 1024
+// for MXFP8), a 16-bit C through the lean epilogue
 bool gemm_wave128_mx_192_ok(const GemmArgs& p, int group_bytes, int tile_m) {
-  return p.M % tile_m == 0 && p.N % 256 == 0 && p.k_bytes % group_bytes == 0 && p.k_bytes >= group_bytes && lean_epilogue_type(p) != 0 &&
-         p.lda * 8 + p.k_bytes < (1ll << 31) && p.ldb * 8 + p.k_bytes < (1ll << 31) &&
-         p.lds_a % 16 == 0 && p.lds_b % 16 == 0 && ((uintptr_t)p.sA | (uintptr_t)p.sB) % 16 == 0 &&
-         p.lds_a * 64 + p.k_bytes / 16 < (1ll << 31) && p.lds_b * 64 + p.k_bytes / 16 < (1ll << 31);
+  GemmArgs q = p;
+  q.M = p.M >= tile_m ? std::max(p.M, 256) : 0;
+  return mx_sizes_ok(q) && mx_whole_groups(p, group_bytes) && lean_epilogue_type(p) != 0;
 }
 
-bool gemm_wave128_mxfp4_ok(const GemmArgs& p) {
-  // whole tiles, at least one group of four K steps (K >= 1024 elements; what is left behind the last group: the TAIL
-  // form), scale rows that a 16-byte load can fetch
-  return p.M % 256 == 0 && p.N % 256 == 0 && p.k_bytes % 16 == 0 && p.k_bytes >= 512 &&
-         p.lda * 8 + p.k_bytes < (1ll << 31) && p.ldb * 8 + p.k_bytes < (1ll << 31) &&
-         p.lds_a % 16 == 0 && p.lds_b % 16 == 0 && ((uintptr_t)p.sA | (uintptr_t)p.sB) % 16 == 0 &&
-         p.lds_a * 64 + p.k_bytes / 16 < (1ll << 31) && p.lds_b * 64 + p.k_bytes / 16 < (1ll << 31);
-}
+bool gemm_wave128_mxfp4_ok(const GemmArgs& p) { return mx_sizes_ok(p) && p.k_bytes % 16 == 0; }
 
-template <int EPI, bool TAIL = false, int BM = 256>
+template <int EPI, bool ANYK = false, int BM = 256>
 static int launch_wave128_mxfp4(const GemmArgs& p, hipStream_t stream) {
-  constexpr int smem = 2 * (BM + 256) * 128 + 2 * 512 * 16 + 1024;   // (stages, scale ring and the 1 KiB that the L2 touches land in)
+  constexpr int smem = 2 * (BM + 256) * 128 + (ANYK ? 3 : 2) * 512 * 16 + 1024;   // (stages, scale ring and the 1 KiB that the L2 touches land in)
   static bool attr_set = false;
   if (!attr_set) {
-    hipError_t e = hipFuncSetAttribute((const void*)gemm_wave128_mxfp4_kernel<EPI, TAIL, BM>, hipFuncAttributeMaxDynamicSharedMemorySize, smem);
+    hipError_t e = hipFuncSetAttribute((const void*)gemm_wave128_mxfp4_kernel<EPI, ANYK, BM>, hipFuncAttributeMaxDynamicSharedMemorySize, smem);
     if (e != hipSuccess) return (int)e;
     attr_set = true;
   }
-  const int tiles = (p.M / BM) * (p.N / 256);
-  const int grid = wave128_grid(tiles, p.num_programs);
-  gemm_wave128_mxfp4_kernel<EPI, TAIL, BM><<<dim3(grid), dim3(256), smem, stream>>>(p);
+  const int tiles = ((p.M + BM - 1) / BM) * ((p.N + 255) / 256);
+  const int grid = ANYK ? tiles : wave128_grid(tiles, p.num_programs);
+  gemm_wave128_mxfp4_kernel<EPI, ANYK, BM><<<dim3(grid), dim3(256), smem, stream>>>(p);
   return (int)hipGetLastError();
 }
 
@@ -834,7 +812,7 @@ int gemm_wave128_mxfp4_launch(const GemmArgs& p, hipStream_t stream) {
     return lean == 1 ? launch_wave128_mxfp4<3, false, 192>(p, stream) : launch_wave128_mxfp4<4, false, 192>(p, stream);
   if (p.tile_m == 128)
     return lean == 1 ? launch_wave128_mxfp4<3, false, 128>(p, stream) : launch_wave128_mxfp4<4, false, 128>(p, stream);
-  if (p.k_bytes % 512 != 0)
+  if (!mx_whole_groups(p, 512))
     return lean == 1 ? launch_wave128_mxfp4<3, true>(p, stream) : lean == 2 ? launch_wave128_mxfp4<4, true>(p, stream) : launch_wave128_mxfp4<0, true>(p, stream);
   return lean == 1 ? launch_wave128_mxfp4<3>(p, stream) : lean == 2 ? launch_wave128_mxfp4<4>(p, stream) : launch_wave128_mxfp4<0>(p, stream);
 }
