@@ -355,3 +355,75 @@ def test_backward_with_groups_of_waves(gpu, causal, n_ctx, head_dim, monkeypatch
         assert torch.all((delta.double() - want_delta).abs() <= size * head_dim * 2.0 ** -24), groups
         for name, t in (("dq", dq), ("dk", dk), ("dv", dv)):
             assert np.allclose(to_np(t), cf[name], atol=1e-2, rtol=1e-2), (groups, name)
+
+
+def _qkv(gpu, n=256, d=64, dtype=torch.float16, seed=0):
+    g = torch.Generator(device=gpu).manual_seed(seed)
+    return [torch.randn(1, 2, n, d, device=gpu, generator=g).to(dtype).requires_grad_() for _ in range(3)]
+
+
+def test_native_autograd_node_gives_the_python_function_s_bits(gpu):
+    # the same launches on the same tensors: equal results with and without gradients, for permuted inputs, for a subset of
+    # inputs that need gradients, in several backward passes and under hooks on the saved tensors
+    from triton_amd import ops
+
+    for d, dtype in ((64, torch.float16), (128, torch.bfloat16), (32, torch.bfloat16)):
+        q, k, v = _qkv(gpu, d=d, dtype=dtype)
+        do = torch.randn(q.shape, device=gpu).to(dtype)
+        want = ops._attention.apply(q, k, v, True, 0.125)
+        want_grads = torch.autograd.grad(want, (q, k, v), do)
+        packed = []
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: packed.append(t.shape) or t.clone(), lambda t: t):
+            got = triton_amd.attention(q, k, v, True, 0.125)
+        assert len(packed) == 5 and "PythonFunction" not in type(got.grad_fn).__name__
+        for _ in range(2):
+            grads = torch.autograd.grad(got, (q, k, v), do, retain_graph=True)
+            assert torch.equal(got, want) and all(torch.equal(a, b) for a, b in zip(grads, want_grads))
+        only = triton_amd.attention(q.detach(), k, v.detach(), True, 0.125)
+        only.backward(do)
+        assert torch.equal(k.grad, want_grads[1]) and q.grad is None
+        with torch.no_grad():
+            assert torch.equal(triton_amd.attention(q, k, v, True, 0.125), want)
+        assert not triton_amd.attention(q.detach(), k.detach(), v.detach(), True, 0.125).requires_grad
+        o = torch.utils.checkpoint.checkpoint(triton_amd.attention, q, k, v, True, 0.125, use_reentrant=False)
+        assert all(torch.equal(a, b) for a, b in zip(torch.autograd.grad(o, (q, k, v), do), want_grads))
+
+
+def test_calls_that_the_native_autograd_node_refuses_fail_as_before(gpu):
+    from triton_amd import hooks, ops
+
+    q, k, v = _qkv(gpu)
+    o = triton_amd.attention(q, k, v, False, 0.125)
+    with pytest.raises(AssertionError):   # (from the engine's thread)
+        o.backward(torch.randn(1, 2, 64, 256, device=gpu).half().transpose(2, 3))
+    q2, k2, v2 = _qkv(gpu, n=192)
+    with pytest.raises(ValueError, match="shape"):
+        triton_amd.attention(q2, k2, v2, False, 0.125)
+    with pytest.raises(AssertionError):
+        triton_amd.attention(q, k[..., :32], v, False, 0.125)
+    with pytest.raises(AssertionError):
+        triton_amd.attention(q, k.bfloat16(), v, False, 0.125)
+    with pytest.raises(TypeError):
+        triton_amd.attention(q.double(), k.double(), v.double(), False, 0.125)
+    with pytest.raises(ValueError):
+        triton_amd.attention(q.cpu(), k.cpu(), v.cpu(), False, 0.125)
+    f8 = [t.detach().to(torch.float8_e5m2) for t in (q, k, v)]
+    with pytest.raises(AssertionError):   # (V not transposed in memory)
+        triton_amd.attention(*f8, False, 0.125)
+    # what looks inside a call still sees the Python function: launch hooks, functorch, tensor subclasses
+    seen = []
+    hooks.Launch.launch_enter_hook = lambda md: seen.append(md.get()["name"])
+    try:
+        triton_amd.attention(q, k, v, False, 0.125)
+    finally:
+        hooks.Launch.launch_enter_hook = None
+    assert len(seen) == 1 and "mi355_attn_fwd" in seen[0]
+    for call in (lambda f: torch.func.vmap(lambda a: f(a, k, v, False, 0.125))(q.detach()[None]),
+                 lambda f: torch.func.jvp(lambda a: f(a, k, v, False, 0.125), (q.detach(),), (torch.ones_like(q),))):
+        errors = []
+        for f in (ops._attention.apply, triton_amd.attention):
+            with pytest.raises(RuntimeError) as e:
+                call(f)
+            errors.append(str(e.value))
+        assert errors[0] == errors[1]
+    assert triton_amd.attention(q.detach(), torch.nn.Parameter(k.detach()), v.detach(), False, 0.125).grad_fn.next_functions[1][0] is not None

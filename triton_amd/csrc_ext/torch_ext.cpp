@@ -184,6 +184,52 @@ void attn_bwd(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, con
   check(rc, "mi355_attn_bwd");
 }
 
+// `attention` with its autograd node in native code: the same saved tensors, launches and checks as `_attention` of ops.py, which
+// stays for everything else (tensor subclasses, tracing, functorch, forward-mode differentiation, hooks around launches) and
+// for every call that it refuses.  us for a forward and backward pass of [1, 16, 1024, 64] fp16, of which the kernels are 38: 91
+// through the Python function, 49 here (a forward alone 13.5 / 7.5).
+[[noreturn]] void assertion(const char* message) {   // (thrown from the engine's own threads too: what PythonEngine expects there)
+  py::gil_scoped_acquire gil;
+  PyErr_SetString(PyExc_AssertionError, message);
+  python_error e;
+  e.persist();
+  throw e;
+}
+
+struct Attention : torch::autograd::Function<Attention> {
+  static at::Tensor forward(torch::autograd::AutogradContext* ctx, const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, double sm_scale, bool causal) {
+    at::Tensor o = at::empty_like(q), M = at::empty({q.size(0), q.size(1), q.size(2)}, q.options().dtype(at::kFloat));
+    attn_fwd(q, k, v, o, M, sm_scale, causal);
+    ctx->save_for_backward({q, k, v, o, M});
+    ctx->saved_data["sm_scale"] = sm_scale;
+    ctx->saved_data["causal"] = causal;
+    return o;
+  }
+  static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx, torch::autograd::variable_list grads) {
+    const auto saved = ctx->get_saved_variables();
+    const at::Tensor &q = saved[0], &k = saved[1], &v = saved[2], &o = saved[3], &M = saved[4], &d_o = grads[0];
+    if (!d_o.is_contiguous()) assertion("");
+    if (q.strides() != k.strides() || q.strides() != v.strides() || q.strides() != o.strides() || q.strides() != d_o.strides()) assertion("");
+    if (q.size(2) % 128 != 0) assertion("");
+    at::Tensor dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(v), delta = at::empty_like(M);
+    attn_bwd(q, k, v, o, d_o, M, delta, dq, dk, dv, ctx->saved_data["sm_scale"].toDouble(), ctx->saved_data["causal"].toBool());
+    return {dq, dk, dv, at::Tensor(), at::Tensor()};
+  }
+};
+
+c10::optional<at::Tensor> attention(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, double sm_scale, bool causal) {
+  const auto type = q.scalar_type();
+  const bool is8 = type == at::kFloat8_e4m3fn || type == at::kFloat8_e5m2;
+  if (q.dim() != 4 || k.dim() != 4 || v.dim() != 4 || k.scalar_type() != type || v.scalar_type() != type || !q.is_cuda() || !k.is_cuda() || !v.is_cuda()) return c10::nullopt;
+  const int64_t D = q.size(3);
+  if ((type != at::kHalf && type != at::kBFloat16 && !is8) || k.size(3) != D || v.size(3) != D || (D != 16 && D != 32 && D != 64 && D != 128 && D != 256)) return c10::nullopt;
+  if (is8 && (v.stride(2) != 1 || q.requires_grad() || k.requires_grad() || v.requires_grad())) return c10::nullopt;
+  if (at::GradMode::is_enabled() && (q.requires_grad() || k.requires_grad() || v.requires_grad())) return Attention::apply(q, k, v, sm_scale, causal);
+  at::Tensor o = at::empty_like(q), M = at::empty({q.size(0), q.size(1), q.size(2)}, q.options().dtype(at::kFloat));
+  attn_fwd(q, k, v, o, M, sm_scale, causal);
+  return o;
+}
+
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
@@ -193,4 +239,5 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("group_gemm", &group_gemm);
   m.def("attn_fwd", &attn_fwd);
   m.def("attn_bwd", &attn_bwd);
+  m.def("attention", &attention);
 }

@@ -15,6 +15,7 @@ import math
 import os
 
 import torch
+from torch.autograd import forward_ad
 
 from . import _lib, hooks
 
@@ -462,7 +463,25 @@ def attention(q, k, v, causal, sm_scale):
     and 32 (06:447): those run the 64-column kernels in a form that pads with zeros on the fly - the rows are
     loaded as they are (32 or 64 bytes), the missing columns never exist in memory, and only the first
     HEAD_DIM columns of every output and gradient are stored - so no padded copies are made."""
+    ext = _lib.ext()
+    if ext is not None and _plain_call(q, k, v, sm_scale):
+        o = ext.attention(q, k, v, float(sm_scale), bool(causal))   # (None: a call that the function below refuses)
+        if o is not None:
+            return o
     return _attention.apply(q, k, v, causal, sm_scale)
+
+
+def _plain_call(q, k, v, sm_scale):
+    """Whether nobody but autograd looks at a call: no tensor subclasses, modes, tracing, functorch transforms, dual numbers or
+    hooks around launches, which are all `_attention`'s."""
+    return (type(q) in _PLAIN and type(k) in _PLAIN and type(v) in _PLAIN and type(sm_scale) in (float, int) and
+            hooks.Launch.launch_enter_hook is None and hooks.Launch.launch_exit_hook is None and
+            not torch.compiler.is_compiling() and torch._C._get_tracing_state() is None and
+            torch._C._functorch.peek_interpreter_stack() is None and forward_ad._current_level < 0 and
+            torch._C._len_torch_function_stack() == 0 and torch._C._len_torch_dispatch_stack() == 0)
+
+
+_PLAIN = (torch.Tensor, torch.nn.Parameter)
 
 
 def default_sm_scale(head_dim: int) -> float:
