@@ -169,14 +169,24 @@ RingPlan ring_plan(int M, int N, int steps, int cus, int splits_lo, int splits_h
   return best;
 }
 
+// The same plan against kernels of other tiles: what one split's rounds take (195 products of up to 2800 tiles and 4 .. 64 steps: within 6 %
+// rms).  The estimates above, up to a fifth longer for several rounds, are for the choice among the rings and splits that they were fitted to.
+double ring_rounds_us(int M, int N, int steps, int cus, int shape) {
+  static const struct { int bm, bn; double round_us, step_us, whole; } kShapes[3] = {{128, 128, 3.4, 0.365, 0.86}, {128, 64, 2.2, 0.25, 0.91}, {64, 64, 1.1, 0.158, 0.7}};
+  const auto& t = kShapes[shape];
+  const long tiles = (long)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn), rounds = (tiles + cus - 1) / cus;
+  return 1.2 + (rounds > 1 ? t.whole * rounds + (1.0 - t.whole) * tiles / cus : 1.0) * (t.round_us + steps * t.step_us * (rounds > 1 ? 1.0 : 1.04));
+}
+
 // The same for the kernels of 256-column tiles with `rows` rows of C each (gemm_wave128.hip; edges: the eight-wave kernel, for
-// what that one does not take).  A K step of a 256-row tile is bound by its 64 KiB of operands: 1.43 us with all CUs at it, a quarter
-// of that without the others' traffic.
+// what that one does not take).  A K step of a 256-row tile is bound by its 64 KiB of operands and by power: with idle CUs it is
+// somewhat shorter, and several rounds are dealt evenly, so that an unfilled last round is spread over all of them.  180 products
+// of 64 .. 768 tiles and 8 .. 128 steps, bf16 in both layouts and e4m3: within 3 % rms, 11 % at most.
 double tiles256_us(long tiles, int rows, int steps, int cus, bool edges, bool fp8) {
   const long rounds = (tiles + cus - 1) / cus;
-  const double fill = rounds > 1 ? 1.0 : (double)tiles / cus;
-  const double share = rows == 256 ? 1.0 : rows == 192 ? 0.78 : 0.64;
-  return kLaunchUs + (double)rounds * share * ((edges ? 8.0 : 6.0) + (edges && !fp8 ? 1.6 : 1.43) * (0.25 + 0.75 * fill) * steps);
+  const double fill = (double)tiles / (double)(rounds * cus), busy = rounds > 1 ? 0.48 + 0.52 * fill : 0.62 + 0.38 * fill;
+  const double share = rows == 256 ? 1.0 : rows == 192 ? 0.78 : 0.64, step = (fp8 ? 1.28 : 1.34) * (edges ? fp8 ? 1.0 : 1.12 : 1.0);
+  return 3.2 + (double)rounds * share * ((edges ? 10.0 : 8.0) + step * busy * steps);
 }
 
 // Products of a short K whose 128x128 tiles are more than the CUs: the kernel of one barrier per 64-byte step on those tiles, two
@@ -528,27 +538,38 @@ static int gemm_impl(const void* A, const void* B, void* C, int M, int N, int K,
     else if (!by_knob && knobs().tile_m == UNSET && knobs().mixed_rows == UNSET) {
       const int rows = tile == 6 && p.tile_m ? p.tile_m : 256;
       const RingPlan plan = ring_plan(M, N, ksteps128, cus, 1, 1);
+      const double plan_us = tile == 6 ? ring_rounds_us(M, N, ksteps128, cus, plan.shape) : plan.us;
       double other = tiles256_us((long)((M + rows - 1) / rows) * ((N + 255) / 256), rows, ksteps128, cus, tile != 6, is8);
       if (mixed_rows > 0) other *= 0.9;   // (two tile heights in one launch are chosen where they gain at least 5 %)
-      if (plan.us < other) ring = plan.shape;
-      // Up to 64 columns (or rows) beyond whole 256-column tiles: those in a call of their own where they would cost the tiles
-      // another round of CUs.  bf16, us of a call, in one / in two parts, row-major B (K-major): 4100 x 4096 x 4096 135 / 99
-      // (129 / 93), 4096 x 4128 x 4096 145 / 105 (125 / 95), 2050 x 8192 x 4096 136 / 101, 8192 x 8200 x 2048 243 / 207, 4096 x 4160 x 1024
-      // 50 / 38; edges on the other side too: 4095 x 4100 x 4100 168 / 151.  No round saved, one part: 2048 x 2052 x 4096, 6150 x 6144 x 4096.
-      const double one = std::min(plan.us, other);
-      auto parts_us = [&](int m, int n, int m2, int n2) {
-        const bool edges = tile != 6 || m < 256 || n < 256;
-        const long tiles = (long)((m + 255) / 256) * ((n + 255) / 256);
-        return std::min(ring_plan(m, n, ksteps128, cus, 1, 1).us, tiles256_us(tiles, 256, ksteps128, cus, edges, is8)) +
-               ring_plan(m2, n2, ksteps128, cus, 1, 1).us;
+      if (plan_us < (tile == 6 ? 0.92 : 1.0) * other) ring = plan.shape;   // (pitches move the rings by up to 15 %: 1664 x 6912 x 2112 bf16, 702 tiles, 53 us for the estimate's 47)
+      // A product that needs part of one more round of 256 x 256 tiles in two calls: rows (or columns) for whole rounds of those, the
+      // rest on whatever is best for it.  us of a call, in one / in two parts: e4m3 6707 x 2944 x 3968 78 / 69, fp16 6016 x 2880 x
+      // 7232 255 / 209; up to 64 columns or rows beyond whole tiles likewise, bf16 4100 x 4096 x 4096 135 / 99 (K-major B 129 / 93),
+      // 2050 x 8192 x 4096 136 / 101, 4096 x 4160 x 1024 50 / 38.  No round saved, one part: 2048 x 2052 x 4096, 6150 x 6144 x 4096.
+      const double one = std::min(plan_us, other);
+      auto best_us = [&](int m, int n) {
+        const RingPlan ring = ring_plan(m, n, ksteps128, cus, 1, 1);
+        const double ring_us = tile == 6 ? ring_rounds_us(m, n, ksteps128, cus, ring.shape) : ring.us;
+        if (tile == 6 && (m < 256 || n < 256)) return ring_us;
+        return std::min(ring_us, tiles256_us((long)((m + 255) / 256) * ((n + 255) / 256), 256, ksteps128, cus, tile != 6, is8));
       };
-      const int rn = N % 256, rm = M % 256;
-      const double cut_n = rn > 0 && rn <= 64 && N > 256 ? parts_us(M, N - rn, M, rn) : 1e30;
-      const double cut_m = rm > 0 && rm <= 64 && M > 256 ? parts_us(M - rm, N, rm, N) : 1e30;
-      if (!workspace && std::min(cut_n, cut_m) < 0.9 * one) {
-        const bool rows = cut_m < cut_n;
-        const int m = rows ? M - rm : M, n = rows ? N : N - rn;
-        const int64_t dm = rows ? m : 0, dn = rows ? 0 : n;
+      double cut_us = 1e30;
+      int m = M, n = N;   // the first part
+      auto cut = [&](int m1, int n1) {
+        if (m1 <= 0 || n1 <= 0 || (m1 >= M && n1 >= N)) return;
+        const double us = best_us(m1, n1) + (m1 < M ? best_us(M - m1, N) : best_us(M, N - n1));
+        if (us < cut_us) { cut_us = us; m = m1; n = n1; }
+      };
+      const int rn = N % 256, rm = M % 256, nn = (N + 255) / 256, mm = (M + 255) / 256;
+      if (rn > 0 && rn <= 64 && N > 256) cut(M, N - rn);
+      if (rm > 0 && rm <= 64 && M > 256) cut(M - rm, N);
+      if (tile == 6 && tiles256 > cus) {
+        const int slots = (int)(tiles256 / cus) * cus;
+        cut(std::min(M, slots / nn * 256), N);
+        cut(M, std::min(N, slots / mm * 256));
+      }
+      if (!workspace && cut_us < 0.92 * one) {
+        const int64_t dm = m < M ? m : 0, dn = m < M ? 0 : n;
         const int rc = gemm_impl(A, B, C, m, n, K, sam, sak, sbk, sbn, scm, scn, in_dtype, out_dtype, a_scale, b_scale, activation,
                                  aux, aux_sm, aux_sn, aux_dtype, -1, group_m_arg, stream_);
         if (rc) return rc;
