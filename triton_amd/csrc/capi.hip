@@ -1238,10 +1238,24 @@ static int attn_fwd_variant(const AttnArgs& p, int cus) {
   // (two blocks of keys are not worth the groups' meeting: 256 x 128, no mask, head_dim 128: 8 10.2, 2 8.8; causal 8 ahead)
   if (rows <= 128ll * cus && (p.causal || p.N > 128)) return 8;
   if (p.causal && rows <= 256ll * cus) {
-    // (few, long rows of work under the mask) 32 x 2048: 6 34.1, 8 37.1, 2 38.4, 4 40.7; 8 x 8192: 6 102, 8 101, 4 142
-    if (p.D == 64 && p.N >= 2048) return 6;
+    // (few, long rows of work under the mask) 32 x 2048: 6 34.1, 8 37.1, 2 38.4, 4 40.7; 8 x 8192: 6 102, 8 101, 4 142; 36 x 1152: 6
+    // 18.0, 8 19.6, 2 20.8; 27 x 1280: 6 18.1, 8 21.3, 2 24.6
+    if (p.D == 64 && p.N >= 1152) return 6;
     // head_dim 128, 8 x 8192: 8 146, 1 173, 2 189, 4 197; 32 x 2048: 2 52.3, 8 56.2, 4 56.9; 128 x 512: 2 20.7, 4 23.2
     return p.D == 128 && p.N >= 4096 ? 8 : 2;
+  }
+  if (p.causal) {
+    // The persistent form deals pairs of a long and a short block of 256 rows, every pair the same work, in whole rounds of CUs: it is
+    // the fastest where the pairs fill those (128 x 1024 of head_dim 128, 256 pairs: 4 48, 1 58, 2 58, 8 64) and up to twice as
+    // long where they do not.  us, 8 / 1 / 2 / 4, head_dim 64: 15 x 4992 77 / 103 / 113 / 163, 24 x 2816 42 / 45 / 50 / 71, 75 x 1664 49 / 46
+    // / 49 / 82, 20 x 7680 213 / 219 / 226 / 330, 90 x 1152 34 / 33 / 28 / 39; head_dim 128: 20 x 3328 86 / 77 / 92 / 139, 27 x 3456 102 / 119 / 122 /
+    // 125, 36 x 5632 327 / 341 / 332 / 459, 105 x 2432 203 / 190 / 195 / 243, 100 x 3584 413 / 378 / 360 / 413.  (70 shapes: within 2 % of the
+    // best in the geometric mean, 12 % at most; the pairs everywhere 34 and 20 %, up to 2.1 times as long.)
+    const int64_t heads = (int64_t)p.Z * p.H, nb = (p.N + 255) / 256, pairs = heads * ((nb + 1) / 2);
+    const double dealt = (double)((pairs + cus - 1) / cus * (nb + 1)) * 65536.0 * cus, work = 0.5 * (double)heads * p.N * (p.N + 256.0);
+    if (dealt < 1.04 * work) return 4;
+    if (p.D == 64) return p.N <= 1280 ? 2 : 8;
+    return p.N <= 2600 ? 1 : rows < 560ll * cus ? 8 : 2;
   }
   return dflt;
 }
@@ -1312,6 +1326,8 @@ static int attn_bwd_variant(const AttnArgs& p, int cus) {
   if (p.D == 64 && p.N % 256 == 0 && blocks <= cus / 4) return 4 + 64;
   // 16 x 1024: two -5.7 / -5.8; head_dim 128: 51.7, -6.9 / -8.2; 24 x 1024: 52.2, +1.1 / +0.3 (full 57.1, +8.1 / +7.6)
   if (blocks <= cus / 2) return 2 + 32;
+  // 15 x 1280: 41.3, both -5.9; head_dim 128, 15 x 1152: 55.2, -4.8 (49 x 384: +2.3)
+  if (p.causal && p.N >= 1024 && blocks * 5 <= cus * 3ll) return 2 + 32;
   if (!p.causal || p.N < 2048) return 1 + 16;
   // 8 x 4096: 114.9, -13.9 / -15.3; head_dim 128: 177.6, -14.9 / -16.4; 12 x 4096: 224.8, +9.0 / +6.9; full, 8 x 4096: +13 / +13
   if (blocks <= cus) return 2 + 32;
