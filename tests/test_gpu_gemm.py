@@ -1563,3 +1563,23 @@ def test_an_addend_that_is_c_is_added_once(gpu):
     rc = _lib.load().mi355_gemm_epilogue(a.data_ptr(), b.data_ptr(), c.data_ptr(), M, N, K, K, 1, 1, K, N, 1, _lib.BF16, _lib.F32, None, None,
                                          c.data_ptr(), N, 1, _lib.F32, _lib.ACT_NONE, 0, torch.cuda.current_stream().cuda_stream)
     assert rc == 0 and torch.equal(c, want)
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "e4m3"])
+@pytest.mark.parametrize("M,N,K", [(5696, 832, 1032), (700, 6496, 2048), (4095, 4104, 2048), (4608, 4352, 1280), (6656, 2944, 2064)])
+def test_a_part_of_a_round_of_tiles_in_a_call_of_its_own(gpu, dtype, M, N, K):
+    # whole rounds of 128x128 or 256x256 tiles in one call, the rest in a second one, split along K where there is a workspace; rows
+    # and columns as the cut; the addend moves along.  Whole numbers below 2^12: exact
+    tdt = {"bf16": torch.bfloat16, "e4m3": torch.float8_e4m3fn}[dtype]
+    g = torch.Generator(device=gpu).manual_seed(M + N + K)
+    a = torch.randint(-1, 2, (M, K), device=gpu, generator=g).to(tdt)
+    b = torch.randint(-1, 2, (N, K), device=gpu, generator=g).to(tdt).t()
+    want = a.float() @ b.float()
+    for tb in (b, b.contiguous()) if dtype == "bf16" else (b,):
+        assert torch.equal(triton_amd.matmul(a, tb, out_dtype=torch.float32), want)
+        for shape in ((N,), (M, 1), (M, N)):
+            add = torch.randint(-8, 9, shape, device=gpu, generator=g).to(torch.bfloat16)
+            assert torch.equal(triton_amd.matmul(a, tb, out_dtype=torch.float32, add=add), want + add.float()), shape
+        row = torch.randint(-8, 9, (N,), device=gpu, generator=g).to(torch.bfloat16)
+        got = triton_amd.matmul(a, tb, out_dtype=torch.bfloat16, add=row)
+        assert torch.equal(got, (want + row.float()).to(torch.bfloat16))

@@ -189,6 +189,43 @@ double tiles256_us(long tiles, int rows, int steps, int cus, bool edges, bool fp
   return 3.2 + (double)rounds * share * ((edges ? 10.0 : 8.0) + step * busy * steps);
 }
 
+// A product that needs part of one more round of tiles, in two calls: rows (or columns) for whole rounds of CUs - of 256 x 256 tiles,
+// or of 128x128 ring tiles where those are what it runs on -, the rest on whatever is best for it; and up to 64 columns or rows beyond
+// whole 256-column tiles likewise.  `tile` as in gemm_impl (1: ring kernels only, 6: four-wave kernels; else the eight-wave one),
+// `ring` the ring shape that one call would take or -1.  us of a call, in one / in two parts: e4m3 6707 x 2944 x 3968 78 / 69, fp16 6016
+// x 2880 x 7232 255 / 209, bf16 4100 x 4096 x 4096 135 / 99 (K-major B 129 / 93), 2050 x 8192 x 4096 136 / 101, 4096 x 4160 x 1024 50 / 38; on ring
+// tiles bf16 5696 x 832 x 3456 48.1 / 41.8, fp16 2048 x 2560 x 2048 35.8 / 31.5.  No round saved, one part: 2048 x 2052 x 4096, 6150 x 6144 x 4096.
+struct Cut { int m, n; double us; };   // sizes of the first part
+Cut best_cut(int M, int N, int steps, int cus, int tile, int ring, bool is8) {
+  const bool rounds = tile == 6 || tile == 1;
+  auto best_us = [&](int m, int n) {
+    const RingPlan plan = ring_plan(m, n, steps, cus, 1, 1);
+    const double ring_us = rounds ? ring_rounds_us(m, n, steps, cus, plan.shape) : plan.us;
+    if (tile == 1 || (tile == 6 && (m < 256 || n < 256))) return ring_us;
+    return std::min(ring_us, tiles256_us((long)((m + 255) / 256) * ((n + 255) / 256), 256, steps, cus, tile != 6, is8));
+  };
+  Cut best{M, N, 1e30};
+  auto cut = [&](int m, int n) {
+    if (m <= 0 || n <= 0 || (m >= M && n >= N)) return;
+    const double us = best_us(m, n) + (m < M ? best_us(M - m, N) : best_us(M, N - n));
+    if (us < best.us) best = {m, n, us};
+  };
+  auto whole_rounds = [&](int edge) {
+    const int nn = (N + edge - 1) / edge, mm = (M + edge - 1) / edge;
+    const long tiles = (long)nn * mm;
+    if (tiles <= cus) return;
+    const int slots = (int)(tiles / cus) * cus;
+    cut(std::min(M, slots / nn * edge), N);
+    cut(M, std::min(N, slots / mm * edge));
+  };
+  const int rn = N % 256, rm = M % 256;
+  if (tile != 1 && rn > 0 && rn <= 64 && N > 256) cut(M, N - rn);
+  if (tile != 1 && rm > 0 && rm <= 64 && M > 256) cut(M - rm, N);
+  if (tile == 6) whole_rounds(256);
+  if (ring == 0 && rounds) whole_rounds(128);
+  return best;
+}
+
 // Products of a short K whose 128x128 tiles are more than the CUs: the kernel of one barrier per 64-byte step on those tiles, two
 // workgroups on a CU where a ring leaves room for one.  Measured over 16 .. 1280 tiles and K bytes of 16 .. 2048, this kernel / ring or
 // 256x256 tiles, us: 2688 x 2688 x 64 fp16 8.2 / 11.5, x 192 11.5 / 13.2, x 256 12.4 / 13.0; e4m3 x 384 10.6 / 12.6, x 512 12.3 / 12.7; row-major B, x 256
@@ -338,11 +375,18 @@ const char* mi355_strerror(int code) {
   return "unknown error";
 }
 
+static int splitk_impl(const void* A, const void* B, void* C, int M, int N, int K,
+                       int64_t sam, int64_t sak, int64_t sbk, int64_t sbn, int64_t scm, int64_t scn,
+                       int in_dtype, int out_dtype, const float* a_scale, const float* b_scale,
+                       int activation, const void* aux, int64_t aux_sm, int64_t aux_sn, int aux_dtype,
+                       int splits, void* workspace, size_t workspace_bytes, void* stream_, int k_rows);
+
+// `workspace`: stream-K's.  `spare`: room for the slices of a second part that is split along K (see best_cut), or none.
 static int gemm_impl(const void* A, const void* B, void* C, int M, int N, int K,
                      int64_t sam, int64_t sak, int64_t sbk, int64_t sbn, int64_t scm, int64_t scn,
                      int in_dtype, int out_dtype, const float* a_scale, const float* b_scale,
                      int activation, const void* aux, int64_t aux_sm, int64_t aux_sn, int aux_dtype,
-                     int tile_arg, int group_m_arg, void* stream_, float* workspace = nullptr, int k_rows = 0) {
+                     int tile_arg, int group_m_arg, void* stream_, float* workspace = nullptr, int k_rows = 0, void* spare = nullptr, size_t spare_bytes = 0) {
   if (!A || !B || !C || M <= 0 || N <= 0 || K <= 0) return MI355_EINVAL;
   if (aux && aux_dtype != MI355_F16 && aux_dtype != MI355_BF16 && aux_dtype != MI355_F32) return MI355_EDTYPE;
   if (activation != MI355_ACT_NONE && activation != MI355_ACT_LEAKY_RELU) return MI355_EINVAL;
@@ -532,51 +576,33 @@ static int gemm_impl(const void* A, const void* B, void* C, int M, int N, int K,
       ring = ring_plan(M, N, ksteps128, cus, 1, 1).shape;
       p.K = k_rows;
     } else if (!by_knob && tile != 6 && !aux && p.c_vec_ok && short_k(M, N, p.k_bytes, b_kmajor, cus)) tile = 1;   // (its addends and odd rows of C cost more)
-    else if (tile == 1) ring = by_knob ? 0 : ring_plan(M, N, ksteps128, cus, 1, 1).shape;
+    else if (tile == 1 && by_knob) ring = 0;
     else if (tile >= 8 && tile <= 10) ring = tile - 8;
     else if (tile == 11) tile = 1;   // the one-barrier-per-step kernel on 128x128 tiles
-    else if (!by_knob && knobs().tile_m == UNSET && knobs().mixed_rows == UNSET) {
+    else if (tile == 1 || (!by_knob && knobs().tile_m == UNSET && knobs().mixed_rows == UNSET)) {
       const int rows = tile == 6 && p.tile_m ? p.tile_m : 256;
       const RingPlan plan = ring_plan(M, N, ksteps128, cus, 1, 1);
-      const double plan_us = tile == 6 ? ring_rounds_us(M, N, ksteps128, cus, plan.shape) : plan.us;
-      double other = tiles256_us((long)((M + rows - 1) / rows) * ((N + 255) / 256), rows, ksteps128, cus, tile != 6, is8);
+      const bool rounds = tile == 6 || tile == 1;
+      const double plan_us = rounds ? ring_rounds_us(M, N, ksteps128, cus, plan.shape) : plan.us;
+      double other = tile == 1 ? 1e30 : tiles256_us((long)((M + rows - 1) / rows) * ((N + 255) / 256), rows, ksteps128, cus, tile != 6, is8);
       if (mixed_rows > 0) other *= 0.9;   // (two tile heights in one launch are chosen where they gain at least 5 %)
       if (plan_us < (tile == 6 ? 0.92 : 1.0) * other) ring = plan.shape;   // (pitches move the rings by up to 15 %: 1664 x 6912 x 2112 bf16, 702 tiles, 53 us for the estimate's 47)
-      // A product that needs part of one more round of 256 x 256 tiles in two calls: rows (or columns) for whole rounds of those, the
-      // rest on whatever is best for it.  us of a call, in one / in two parts: e4m3 6707 x 2944 x 3968 78 / 69, fp16 6016 x 2880 x
-      // 7232 255 / 209; up to 64 columns or rows beyond whole tiles likewise, bf16 4100 x 4096 x 4096 135 / 99 (K-major B 129 / 93),
-      // 2050 x 8192 x 4096 136 / 101, 4096 x 4160 x 1024 50 / 38.  No round saved, one part: 2048 x 2052 x 4096, 6150 x 6144 x 4096.
-      const double one = std::min(plan_us, other);
-      auto best_us = [&](int m, int n) {
-        const RingPlan ring = ring_plan(m, n, ksteps128, cus, 1, 1);
-        const double ring_us = tile == 6 ? ring_rounds_us(m, n, ksteps128, cus, ring.shape) : ring.us;
-        if (tile == 6 && (m < 256 || n < 256)) return ring_us;
-        return std::min(ring_us, tiles256_us((long)((m + 255) / 256) * ((n + 255) / 256), 256, ksteps128, cus, tile != 6, is8));
-      };
-      double cut_us = 1e30;
-      int m = M, n = N;   // the first part
-      auto cut = [&](int m1, int n1) {
-        if (m1 <= 0 || n1 <= 0 || (m1 >= M && n1 >= N)) return;
-        const double us = best_us(m1, n1) + (m1 < M ? best_us(M - m1, N) : best_us(M, N - n1));
-        if (us < cut_us) { cut_us = us; m = m1; n = n1; }
-      };
-      const int rn = N % 256, rm = M % 256, nn = (N + 255) / 256, mm = (M + 255) / 256;
-      if (rn > 0 && rn <= 64 && N > 256) cut(M, N - rn);
-      if (rm > 0 && rm <= 64 && M > 256) cut(M - rm, N);
-      if (tile == 6 && tiles256 > cus) {
-        const int slots = (int)(tiles256 / cus) * cus;
-        cut(std::min(M, slots / nn * 256), N);
-        cut(M, std::min(N, slots / mm * 256));
-      }
-      if (!workspace && cut_us < 0.92 * one) {
+      const Cut cut = best_cut(M, N, ksteps128, cus, tile, ring, is8);
+      if (!workspace && cut.us < (tile == 1 ? 0.88 : 0.92) * std::min(plan_us, other)) {
+        const int m = cut.m, n = cut.n;
         const int64_t dm = m < M ? m : 0, dn = m < M ? 0 : n;
         const int rc = gemm_impl(A, B, C, m, n, K, sam, sak, sbk, sbn, scm, scn, in_dtype, out_dtype, a_scale, b_scale, activation,
                                  aux, aux_sm, aux_sn, aux_dtype, -1, group_m_arg, stream_);
         if (rc) return rc;
-        return gemm_impl((const char*)A + dm * sam * es, (const char*)B + dn * sbn * es, (char*)C + (dm * scm + dn * scn) * elem_size(out_dtype),
-                         M - (int)dm, N - (int)dn, K, sam, sak, sbk, sbn, scm, scn, in_dtype, out_dtype, a_scale, b_scale, activation,
-                         aux ? (const char*)aux + (dm * aux_sm + dn * aux_sn) * elem_size(aux_dtype) : nullptr, aux_sm, aux_sn, aux_dtype,
-                         -1, group_m_arg, stream_);
+        const int m2 = M - (int)dm, n2 = N - (int)dn;
+        A = (const char*)A + dm * sam * es; B = (const char*)B + dn * sbn * es; C = (char*)C + (dm * scm + dn * scn) * elem_size(out_dtype);
+        if (aux) aux = (const char*)aux + (dm * aux_sm + dn * aux_sn) * elem_size(aux_dtype);
+        const int splits = spare_bytes > 0 ? auto_splits(m2, n2, p.k_bytes, in_dtype, b_kmajor, true, cus) : 1;
+        if (splits > 1 && (size_t)splits * m2 * n2 * 4 <= spare_bytes)
+          return splitk_impl(A, B, C, m2, n2, K, sam, sak, sbk, sbn, scm, scn, in_dtype, out_dtype, a_scale, b_scale, activation,
+                             aux, aux_sm, aux_sn, aux_dtype, splits, spare, spare_bytes, stream_, 0);
+        return gemm_impl(A, B, C, m2, n2, K, sam, sak, sbk, sbn, scm, scn, in_dtype, out_dtype, a_scale, b_scale, activation,
+                         aux, aux_sm, aux_sn, aux_dtype, -1, group_m_arg, stream_);
       }
     }
   }
@@ -690,7 +716,7 @@ struct GemmRoute {
   int b_rows = 0;                // rows of the copy of B
   int64_t a_pitch = 0, b_pitch = 0;   // bytes
   int splits = 1;
-  size_t a_bytes = 0, b_bytes = 0, slice_bytes = 0;
+  size_t a_bytes = 0, b_bytes = 0, slice_bytes = 0;   // (slices of the whole product, or of a second part of it)
 };
 
 size_t up(size_t v, size_t to) { return (v + to - 1) / to * to; }
@@ -702,8 +728,21 @@ GemmRoute gemm_route(const void* A, const void* B, int M, int N, int K, int64_t 
   if (knob(knobs().force_strided, 0) != 0) return r;
   auto split = [&](bool kmajor) {
     if (knob(knobs().splitk, 1) == 0) return;
-    r.splits = auto_splits(M, N, (int64_t)r.k * es, in_dtype, kmajor, ring_ok(es, kmajor), cus);
+    const int64_t k_bytes = (int64_t)r.k * es;
+    r.splits = auto_splits(M, N, k_bytes, in_dtype, kmajor, ring_ok(es, kmajor), cus);
     r.slice_bytes = r.splits > 1 ? (size_t)r.splits * M * N * 4 : 0;
+    if (r.splits > 1 || r.k_rows > 0 || !ring_ok(es, kmajor) || k_bytes < 2048) return;
+    // room for the slices of what best_cut leaves to a second call (gemm_impl decides again: without the room that part is not split)
+    const long tiles256 = (long)((M + 255) / 256) * ((N + 255) / 256);
+    const int steps = (int)((k_bytes + 127) / 128), tile = M >= 256 && N >= 256 && tiles256 * (es == 1 ? 4 : 2) >= cus * (es == 1 ? 3 : 1) ? 6 : 1;
+    if ((long)((M + 127) / 128) * ((N + 127) / 128) <= cus) return;
+    const RingPlan plan = ring_plan(M, N, steps, cus, 1, 1);
+    const double plan_us = ring_rounds_us(M, N, steps, cus, plan.shape), other = tile == 6 ? tiles256_us(tiles256, 256, steps, cus, false, es == 1) : 1e30;
+    const Cut cut = best_cut(M, N, steps, cus, tile, plan_us < 0.92 * other ? plan.shape : -1, es == 1);
+    if (cut.us > std::min(plan_us, other)) return;
+    const int m2 = cut.m < M ? M - cut.m : M, n2 = cut.m < M ? N : N - cut.n, splits = auto_splits(m2, n2, k_bytes, in_dtype, kmajor, true, cus);
+    const size_t bytes = splits > 1 ? (size_t)splits * m2 * n2 * 4 : 0;
+    if (bytes <= (16u << 20)) r.slice_bytes = bytes;
   };
   // (as in gemm_impl)
   const bool a_ok = sak == 1 && sam % vec == 0 && sam >= K && aligned(A, 16) && K % vec == 0;
@@ -813,7 +852,7 @@ int mi355_gemm_ws(const void* A, const void* B, void* C, int M, int N, int K,
                        addend, sdm, sdn, addend_dtype, r.splits, ws + r.a_bytes + r.b_bytes, r.slice_bytes, stream_, r.k_rows);
   else
     rc = gemm_impl(A, B, C, M, N, r.k, sam, sak, sbk, sbn, scm, scn, in_dtype, out_dtype, a_scale, b_scale, activation,
-                   addend, sdm, sdn, addend_dtype, -1, 0, stream_, nullptr, r.k_rows);
+                   addend, sdm, sdn, addend_dtype, -1, 0, stream_, nullptr, r.k_rows, ws + r.a_bytes + r.b_bytes, r.slice_bytes);
   if (rc || !softmax) return rc;
   return softmax_rows_launch(C, M, N, scm, scn, out_dtype, (hipStream_t)stream_);
 }
