@@ -1379,7 +1379,7 @@ def test_fp32_operands_are_multiplied_exactly(gpu, kmajor):
         assert rc == 0 and bits_equal(to_np(c), ref), tile
 
 
-@pytest.mark.parametrize("tile", [8, 9, 10])   # 128x128, 128x64, 64x64
+@pytest.mark.parametrize("tile", [8, 9, 10, 12])   # 128x128, 128x64, 64x64, 64x32 with a ring of eight (K-major B)
 @pytest.mark.parametrize("dtype", ["fp16", "bf16", "e4m3"])
 def test_ring_kernels_at_the_edges_of_their_ring_are_bit_exact(gpu, dtype, tile, monkeypatch):
     # K steps of 128 bytes through four stages: K shorter than the ring, an odd and an even number of steps, a tail of one
@@ -1391,7 +1391,7 @@ def test_ring_kernels_at_the_edges_of_their_ring_are_bit_exact(gpu, dtype, tile,
     rng = np.random.default_rng(tile)
     el = 1 if dtype == "e4m3" else 2
     for M, N, kbytes in [(1, 16, 16), (128, 128, 128), (130, 72, 112), (64, 136, 384), (257, 200, 512), (192, 64, 528), (100, 264, 640),
-                         (65, 128, 752), (300, 320, 1168), (129, 1000, 2048)]:
+                         (65, 128, 752), (300, 320, 1168), (129, 1000, 2048)] + ([(33, 31, 896), (64, 40, 1040)] if tile == 12 else []):
         K = kbytes // el
         a = rng.integers(-1, 2, size=(M, K)).astype(np.float32)
         b = rng.integers(-1, 2, size=(K, N)).astype(np.float32)
@@ -1509,16 +1509,13 @@ def test_columns_or_rows_beyond_whole_tiles_in_a_call_of_their_own(gpu, M, N, K,
 
 
 @pytest.mark.parametrize("programs", [3, 256])
-@pytest.mark.parametrize("kmajor", [False, True])
-@pytest.mark.parametrize("dtype", ["fp16", "bf16", "e4m3"])
+@pytest.mark.parametrize("dtype,kmajor", [("fp16", False), ("fp16", True), ("bf16", False), ("bf16", True), ("e4m3", True)])
 def test_four_wave_kernels_on_tiles_moved_back_from_the_edges_are_bit_exact(gpu, monkeypatch, dtype, kmajor, programs):
     # sizes that are no whole tiles: the last tiles lie partly over their neighbours, and with a row-major B the last columns
     # of a tile may be padding.  One tile, one row or column more, a chunk more, odd rows of C, a K tail, every tile height;
     # bias row, addend matrix, activation, fp32 / fp8 output.  Whole numbers: exact in every order
     set_knob(monkeypatch, "MI355_GEMM_TILE", "6")
     set_knob(monkeypatch, "MI355_GEMM_PROGRAMS", str(programs))
-    if dtype == "e4m3" and not kmajor:
-        pytest.skip("a row-major fp8 B of these sizes runs another kernel")
     tdt = {"fp16": torch.float16, "bf16": torch.bfloat16, "e4m3": torch.float8_e4m3fn}[dtype]
     out = torch.float16 if dtype != "bf16" else torch.bfloat16
     g = torch.Generator(device=gpu).manual_seed(len(dtype) + kmajor)

@@ -145,9 +145,18 @@ int elem_size(int dtype) {
 // One row or column of tiles against a long weight is a stream from memory: a CU gets about 30 GB/s of lines that no other CU
 // asks for (64 x 8192 x 8192 fp16, 128 tiles of 64x64: 48 us with rings of four and of eight stages alike, 35 us with two
 // splits), so that there the splits also buy bandwidth.
-struct RingPlan { int shape, splits; double us; };
+struct RingPlan { int shape, splits; double us; };   // shape: 0 = tiles of 128x128, 1 = 128x64, 2 = 64x64, 3 = 64x32
+
+// Ring tiles of 64x32, eight steps deep, for up to 64 rows next to a K-major weight: twice the workgroups of 64x64 tiles without a
+// split and its second launch, one round of CUs.  Measured over 16 .. 64 rows, 1024 .. 16384 columns, K bytes of 2048 .. 16384, fp16 and
+// e4m3, weights from memory, us, the best of the other rings, splits and the streaming kernel / these tiles: e4m3 33 x 8192 x 8192 18.2 /
+// 13.7, 64 x 8192 x 8192 18.6 / 16.8, 48 x 4096 x 4096 8.3 / 6.9, 24 x 6016 x 5376 8.6 / 8.2; fp16 24 x 4096 x 4096 11.1 / 9.5, 33 x 6016 x 5376 22.0 /
+// 15.5, 48 x 3000 x 2304 8.4 / 7.1; beyond one round behind (64 x 12288 x 4096 27 / 33).  A row-major weight's 64-byte pieces are no
+// faster on them (fp16 64 x 8192 x 8192 34.5 / 45).
+bool thin_ok(int M, int N, int64_t k_bytes, bool b_kmajor, int cus) { return b_kmajor && M <= 64 && (N + 31) / 32 <= cus && k_bytes > 2048; }
+
 constexpr double kLaunchUs = 3.5;
-RingPlan ring_plan(int M, int N, int steps, int cus, int splits_lo, int splits_hi, double step_share = 1.0) {
+RingPlan ring_plan(int M, int N, int steps, int cus, int splits_lo, int splits_hi, double step_share = 1.0, bool thin = false) {
   const double streamed = 128.0 * steps * std::max(M, N);   // bytes of the longer operand
   static const struct { int bm, bn; double round_us, step_us; } kShapes[3] = {{128, 128, 2.5, 0.42}, {128, 64, 1.5, 0.265}, {64, 64, 0.6, 0.165}};
   RingPlan best{0, 1, 1e30};
@@ -165,6 +174,17 @@ RingPlan ring_plan(int M, int N, int steps, int cus, int splits_lo, int splits_h
       if (us < best.us) best = {shape, splits, us};
       if (splits > 1 && rounds > 1) break;   // (more splits only add rounds)
     }
+  }
+  // 64x32 tiles (thin_ok): a step is latency, or the weight's way - from memory where it is larger than the last-level cache keeps next
+  // to others (fp16, 24 rows, 128 tiles: 4096 x 4096, 33 MB, 9.4 us, 4096 x 8192, 67 MB, 20.0 - two splits of 64x64 tiles 16.2)
+  const long tiles = (N + 31) / 32;
+  const bool far = N * 128.0 * steps > 48e6;
+  for (int splits = splits_lo; thin && splits <= splits_hi && tiles * splits <= cus; splits++) {
+    const int per = (steps + splits - 1) / splits;
+    const double rows = std::max(M - 16, 0);
+    double us = 3.2 + per * std::max(far ? 0.13 + 1.4e-3 * std::max(M - 24, 0) : 0.095 + 4.5e-4 * rows, 7.1e-4 * tiles * splits + 6e-4 * rows);
+    if (splits > 1) us += 2.5 + (double)splits * M * N * 8.0 / 3e6;
+    if (us < best.us) best = {3, splits, us};
   }
   return best;
 }
@@ -255,6 +275,9 @@ bool ring_ok(int elem_bytes, bool b_kmajor) { return elem_bytes == 2 || (elem_by
 //     memory; 16 x 8192 x 8192 39 / 43)
 bool streams(int M, int N, int64_t k_bytes, int elem_bytes, bool b_kmajor, int cus) {
   const bool cols = M > 64;
+  // (64x32 ring tiles: above 16 rows, and below from 70 % of a round of CUs on - 16 x 8192 x 8192 fp16 33.6 / 29.0, e4m3 13.7 / 13.2; 16 x
+  // 4096 x 8192 e4m3 8.8 / 9.3)
+  if (!cols && thin_ok(M, N, k_bytes, b_kmajor, cus) && (M > 16 || (N + 31) / 32 * 10 > cus * 7)) return false;
   const int S = cols ? N : M, L = cols ? M : N;
   const bool y_kmajor = cols || b_kmajor;
   if (!gemm_skinny_sizes_ok(S, L, k_bytes, y_kmajor, cols ? b_kmajor : true, elem_bytes)) return false;
@@ -289,10 +312,11 @@ int auto_splits(int M, int N, int64_t k_bytes, int in_dtype, bool b_kmajor, bool
     const bool few = std::min(M, N) <= 64, stream = streams(M, N, k_bytes, elem_size(in_dtype), b_kmajor, cus);
     const int most = (int)std::min<int64_t>(std::min<int64_t>(32, steps / (few ? 8 : 2)), (64ll << 20) / std::max<int64_t>(1, 4ll * M * N));   // 64 MiB of partial sums
     if (most < 2 || steps < (few ? 48 : 16)) return 1;   // (below that a second launch costs more than the K steps it would save)
+    const bool thin = !stream && thin_ok(M, N, k_bytes, b_kmajor, cus);
     const double plain = stream ? stream_us(M, N, k_bytes, b_kmajor, cus)
-                                : std::min(ring_plan(M, N, steps, cus, 1, 1).us,
+                                : std::min(ring_plan(M, N, steps, cus, 1, 1, 1.0, thin).us,
                                            tiles256_us((long)((M + 255) / 256) * ((N + 255) / 256), 256, steps, cus, false, elem_size(in_dtype) == 1));
-    const RingPlan split = ring_plan(M, N, steps, cus, 2, most);
+    const RingPlan split = ring_plan(M, N, steps, cus, 2, most, 1.0, thin);
     // (columns that are not groups of four are added up one by one: 8192 x 33 x 8192 e4m3 19.0 us, in two slices 22.1;
     // and the few workgroups that add up many slices take 0.4 us for each: 16 x 320 x 4704 fp16 9.1 us, in nine slices 10.2)
     const double sums = few ? (N % 4 != 0 ? 1.5 : 0.0) + 0.4 * std::max(0, split.splits - 4) : 0.0;
@@ -578,11 +602,12 @@ static int gemm_impl(const void* A, const void* B, void* C, int M, int N, int K,
     } else if (!by_knob && tile != 6 && !aux && p.c_vec_ok && short_k(M, N, p.k_bytes, b_kmajor, cus)) tile = 1;   // (its addends and odd rows of C cost more)
     else if (tile == 1 && by_knob) ring = 0;
     else if (tile >= 8 && tile <= 10) ring = tile - 8;
+    else if (tile == 12 && b_kmajor) ring = 3;
     else if (tile == 11) tile = 1;   // the one-barrier-per-step kernel on 128x128 tiles
     else if (tile == 1 || (!by_knob && knobs().tile_m == UNSET && knobs().mixed_rows == UNSET)) {
       const int rows = tile == 6 && p.tile_m ? p.tile_m : 256;
-      const RingPlan plan = ring_plan(M, N, ksteps128, cus, 1, 1);
-      const bool rounds = tile == 6 || tile == 1;
+      const RingPlan plan = ring_plan(M, N, ksteps128, cus, 1, 1, 1.0, thin_ok(M, N, p.k_bytes, b_kmajor, cus));
+      const bool rounds = (tile == 6 || tile == 1) && plan.shape < 3;
       const double plan_us = rounds ? ring_rounds_us(M, N, ksteps128, cus, plan.shape) : plan.us;
       double other = tile == 1 ? 1e30 : tiles256_us((long)((M + rows - 1) / rows) * ((N + 255) / 256), rows, ksteps128, cus, tile != 6, is8);
       if (mixed_rows > 0) other *= 0.9;   // (two tile heights in one launch are chosen where they gain at least 5 %)
@@ -672,7 +697,7 @@ static int splitk_impl(const void* A, const void* B, void* C, int M, int N, int 
   p.ldb = (b_kmajor ? sbn : sbk) * es;
   p.group_m = knob(knobs().group_m, 8);
   p.workspace = (float*)workspace;
-  const int shape = ring ? ring_plan(M, N, ksteps, cus, used, used).shape : 0;
+  const int shape = ring ? ring_plan(M, N, ksteps, cus, used, used, 1.0, thin_ok(M, N, k_bytes, b_kmajor, cus)).shape : 0;
   const int rc = is32    ? gemm32_splitk_launch(p, used, per * 64, stream)
                  : ring && es == 1 ? gemm_ring8_launch(p, in_dtype == MI355_F8E5M2, shape, used, per * 128, stream)
                  : ring    ? gemm_ring16_launch(p, in_dtype == MI355_BF16, b_kmajor, shape, used, per * 128, stream)

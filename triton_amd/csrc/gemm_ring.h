@@ -12,6 +12,10 @@
 // before: bf16 1024 x 4096 x 4096 31.6 / 40.3 / 47.6, 45.6; 2048^3 18.9 / 23.6 / 26.6, 24.7; 1024^3 9.9 / 7.7 / 6.2, 13.5; fp16
 // 512^3 6.8 / 5.1 / 4.3, 8.3; e4m3 1024 x 4096 x 4096 18.3 / 23.8 / 25.6, 24.3; 384 x 256 x 6784 fp16 39.0 / 31.3 / 21.4, 66.1.)
 //
+// Tiles of 64x32 are for up to 64 rows next to a K-major B, where the loads of one workgroup per CU are all there is: 12 KB
+// a step, eight steps deep, 96 KB requested.  Against the better of 64x64 tiles, those split along K and the streaming kernel,
+// us, weights from memory: e4m3 33 x 8192 x 8192 18.2 -> 13.7, fp16 33 x 6016 x 5376 22.0 -> 15.5.
+//
 // What is left at one 128 x 128 tile per CU (bf16, 1024 x 4096 x 4096, copies of the kernel with parts taken out): MFMAs and
 // barriers alone 20.3 us, with the fragment reads 25.5, with the loads 26.6, all 31.6 - the tiles' 537 MB from L2 at 19 TB/s
 // are the longest part; eight waves of half a tile each, or a ring twice as deep, change nothing.
@@ -144,11 +148,11 @@ __device__ __forceinline__ void ring_epilogue(f32x4 (&acc)[MT][NT], const GemmAr
   const bool inside = mrow0 + MT * 16 <= p.M && ncol0 + NT * 16 <= p.N;
   auto store16 = [&](auto* c0) {
     using OutT = std::remove_pointer_t<decltype(c0)>;
+    (void)inside;
     typedef OutT Out2 __attribute__((ext_vector_type(2)));
     typedef OutT Out4 __attribute__((ext_vector_type(4), aligned(2)));
-    if (inside && p.c_vec_ok && p.ldc % 8 == 0) {
+    if constexpr (NT % 2 == 0) if (inside && p.c_vec_ok && p.ldc % 8 == 0) {
       // two neighbouring tiles exchanged between lane pairs (kg, kg ^ 1): 16 bytes per lane (see gemm_epilogue16_lean)
-      static_assert(NT % 2 == 0, "pairs of 16-column tiles");
       const int col = ncol0 + 4 * (kg & 2) + 16 * (kg & 1);
       static_for<MT>([&](auto I_) {
         constexpr int i = decltype(I_)::value;
@@ -228,10 +232,16 @@ __device__ __forceinline__ void ring_pin(f32x4& c) {
 template <int NS, int L>
 __device__ __forceinline__ void ring_drain_wait(int left) {
 #if MI355_DEVICE_PASS
-  static_assert(NS == 4, "the ladder of this depth");
-  asm volatile("s_cmp_lt_i32 %0, 4\n\ts_cbranch_scc1 ring_three_%=\n\ts_waitcnt vmcnt(%1)\n\ts_branch ring_done_%=\n"
-               "ring_three_%=:\n\ts_cmp_lt_i32 %0, 3\n\ts_cbranch_scc1 ring_all_%=\n\ts_waitcnt vmcnt(%2)\n\ts_branch ring_done_%=\n"
-               "ring_all_%=:\n\ts_waitcnt vmcnt(0)\nring_done_%=:" :: "s"(left), "i"(2 * L), "i"(L) : "memory", "scc");
+  static_assert(NS == 4 || NS == 8, "the ladders of these depths");
+  if constexpr (NS == 4)
+    asm volatile("s_cmp_lt_i32 %0, 4\n\ts_cbranch_scc1 ring_three_%=\n\ts_waitcnt vmcnt(%1)\n\ts_branch ring_done_%=\n"
+                 "ring_three_%=:\n\ts_cmp_lt_i32 %0, 3\n\ts_cbranch_scc1 ring_all_%=\n\ts_waitcnt vmcnt(%2)\n\ts_branch ring_done_%=\n"
+                 "ring_all_%=:\n\ts_waitcnt vmcnt(0)\nring_done_%=:" :: "s"(left), "i"(2 * L), "i"(L) : "memory", "scc");
+  else   // (seven and five steps to go wait for one step more than they have to)
+    asm volatile("s_cmp_lt_i32 %0, 6\n\ts_cbranch_scc1 ring_five_%=\n\ts_waitcnt vmcnt(%3)\n\ts_branch ring_done_%=\n"
+                 "ring_five_%=:\n\ts_cmp_lt_i32 %0, 4\n\ts_cbranch_scc1 ring_three_%=\n\ts_waitcnt vmcnt(%1)\n\ts_branch ring_done_%=\n"
+                 "ring_three_%=:\n\ts_cmp_lt_i32 %0, 3\n\ts_cbranch_scc1 ring_all_%=\n\ts_waitcnt vmcnt(%2)\n\ts_branch ring_done_%=\n"
+                 "ring_all_%=:\n\ts_waitcnt vmcnt(0)\nring_done_%=:" :: "s"(left), "i"(2 * L), "i"(L), "i"(4 * L) : "memory", "scc");
 #endif
 }
 
@@ -251,8 +261,8 @@ __device__ __forceinline__ void gemm_ring_tile(const GemmArgs& p, const int pm, 
   constexpr bool WIDE = sizeof(Op) == 32;                  // a fragment is two chunks of a row, else one for each sub-step
   constexpr int SD = E::kScaleDwords;
   constexpr bool MX = SD > 0;
-  static_assert(B_KMAJOR || E::kElemBytes == 2, "row-major B: 16-bit types");
-  static_assert((BM == 64 || BM == 128) && (BN == 64 || BN == 128), "tile sizes");
+  static_assert(B_KMAJOR || (E::kElemBytes == 2 && BN >= 64), "row-major B: 16-bit types, pieces of 128 bytes and more");
+  static_assert((BM == 64 || BM == 128) && (BN == 32 || BN == 64 || BN == 128), "tile sizes");
   constexpr int NW = 2 * WN, TM = BM / 2, TN = BN / WN, MT = TM / 16, NT = TN / 16;
   constexpr int A_BYTES = BM * RING_ROW, S_BYTES = (BM + BN) * RING_ROW, STAGE = ring_stage_bytes<E, BM, BN>();
   constexpr int BLOCKS = (BM + BN) / 64, LS = (BLOCKS * SD + NW - 1) / NW;   // scales: loads of one dword of 64 rows
