@@ -119,9 +119,8 @@ int mi355_gemm(const void* A, const void* B, void* C,
  * 5 = the eight-wave pipelined kernel as persistent programs (one per CU, MI355_GEMM_PROGRAMS
  * overrides) that walk their tiles as one stream of K steps, the schedule of
  * python/tutorials/09-persistent-matmul.py:141-190, 6 = four waves of 128x128 from 16x16x32
- * (fp8: 16x16x128) MFMAs on 256x256 tiles (whole tiles, K at least 128 elements - fp8: at least 256 bytes, any multiple of 16 with a
- * K-major B, a multiple of 256 with a row-major one -, a row-major 16-bit B with a pitch that is a multiple of 512 bytes; the
- * heuristic's choice for such products from
+ * (fp8: 16x16x128) MFMAs on 256x256 tiles (M and N at least 256, K at least 256 bytes and any multiple of 16, a multiple of 256 for a row-major
+ * fp8 B; the heuristic's choice for such products from
  * 128 tiles on, fp8 from 192; with more tiles than MI355_GEMM_PROGRAMS, default the CU count, its programs
  * take ceil(tiles / programs) tiles each as one stream of K steps)
  * (a kernel that does not exist for the dtype or shape falls back to the nearest one).  group_m: the

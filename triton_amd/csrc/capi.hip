@@ -182,7 +182,7 @@ RingPlan ring_plan(int M, int N, int steps, int cus, int splits_lo, int splits_h
   for (int splits = splits_lo; thin && splits <= splits_hi && tiles * splits <= cus; splits++) {
     const int per = (steps + splits - 1) / splits;
     const double rows = std::max(M - 16, 0);
-    double us = 3.2 + per * std::max(far ? 0.13 + 1.4e-3 * std::max(M - 24, 0) : 0.095 + 4.5e-4 * rows, 7.1e-4 * tiles * splits + 6e-4 * rows);
+    double us = 3.2 + per * std::max(far ? 0.15 + 1.4e-3 * std::max(M - 24, 0) : 0.095 + 4.5e-4 * rows, far ? 7.6e-4 * tiles * splits + 1.05e-3 * rows : 7.1e-4 * tiles * splits + 6e-4 * rows);
     if (splits > 1) us += 2.5 + (double)splits * M * N * 8.0 / 3e6;
     if (us < best.us) best = {3, splits, us};
   }
@@ -273,11 +273,11 @@ bool ring_ok(int elem_bytes, bool b_kmajor) { return elem_bytes == 2 || (elem_by
 //     even - with the weight in memory; from cache the ring is up to 30 % ahead there), fp8: ring (64 x 4096 x 8192 0.88)
 //   * a row-major long operand: up to 32 rows, three quarters of a round (16 x 2048 x 2048 fp16 8.1 / 6.3 from cache, even from
 //     memory; 16 x 8192 x 8192 39 / 43)
-bool streams(int M, int N, int64_t k_bytes, int elem_bytes, bool b_kmajor, int cus) {
+bool streams(int M, int N, int64_t k_bytes, int elem_bytes, bool b_kmajor, int cus, bool thin = true) {
   const bool cols = M > 64;
   // (64x32 ring tiles: above 16 rows, and below from 70 % of a round of CUs on - 16 x 8192 x 8192 fp16 33.6 / 29.0, e4m3 13.7 / 13.2; 16 x
   // 4096 x 8192 e4m3 8.8 / 9.3)
-  if (!cols && thin_ok(M, N, k_bytes, b_kmajor, cus) && (M > 16 || (N + 31) / 32 * 10 > cus * 7)) return false;
+  if (!cols && thin && thin_ok(M, N, k_bytes, b_kmajor, cus) && (M > 16 || (N + 31) / 32 * 10 > cus * 7)) return false;
   const int S = cols ? N : M, L = cols ? M : N;
   const bool y_kmajor = cols || b_kmajor;
   if (!gemm_skinny_sizes_ok(S, L, k_bytes, y_kmajor, cols ? b_kmajor : true, elem_bytes)) return false;
@@ -303,16 +303,16 @@ double stream_us(int M, int N, int64_t k_bytes, bool b_kmajor, int cus) {
   return rows > 16 ? 3.9 + steps * std::max(0.152, 0.235 * fill) : 3.5 + steps * std::max(0.105, 0.18 * fill);
 }
 
-// Splits of K that `mi355_gemm_splitk` takes by itself (1 = the plain call).
-int auto_splits(int M, int N, int64_t k_bytes, int in_dtype, bool b_kmajor, bool ring, int cus) {
+// Splits of K that `mi355_gemm_splitk` takes by itself (1 = the plain call).  thin_too = false: without the 64x32 ring tiles.
+int auto_splits(int M, int N, int64_t k_bytes, int in_dtype, bool b_kmajor, bool ring, int cus, bool thin_too = true) {
   if (ring) {
     const int steps = (int)((k_bytes + 127) / 128);
     // (up to 64 rows or columns: nothing to gain from 32 K steps - 64 x 2048 x 2048 fp16 8.4 us, in the best splits 9.6, 1 x
     // 1000 x 4096 e4m3 7.6 / 10.2; 64 x 2048 x 4096 18.0 / 12.1 - or in slices of fewer than eight)
-    const bool few = std::min(M, N) <= 64, stream = streams(M, N, k_bytes, elem_size(in_dtype), b_kmajor, cus);
+    const bool few = std::min(M, N) <= 64, stream = streams(M, N, k_bytes, elem_size(in_dtype), b_kmajor, cus, thin_too);
     const int most = (int)std::min<int64_t>(std::min<int64_t>(32, steps / (few ? 8 : 2)), (64ll << 20) / std::max<int64_t>(1, 4ll * M * N));   // 64 MiB of partial sums
     if (most < 2 || steps < (few ? 48 : 16)) return 1;   // (below that a second launch costs more than the K steps it would save)
-    const bool thin = !stream && thin_ok(M, N, k_bytes, b_kmajor, cus);
+    const bool thin = !stream && thin_too && thin_ok(M, N, k_bytes, b_kmajor, cus);
     const double plain = stream ? stream_us(M, N, k_bytes, b_kmajor, cus)
                                 : std::min(ring_plan(M, N, steps, cus, 1, 1, 1.0, thin).us,
                                            tiles256_us((long)((M + 255) / 256) * ((N + 255) / 256), 256, steps, cus, false, elem_size(in_dtype) == 1));
@@ -320,7 +320,9 @@ int auto_splits(int M, int N, int64_t k_bytes, int in_dtype, bool b_kmajor, bool
     // (columns that are not groups of four are added up one by one: 8192 x 33 x 8192 e4m3 19.0 us, in two slices 22.1;
     // and the few workgroups that add up many slices take 0.4 us for each: 16 x 320 x 4704 fp16 9.1 us, in nine slices 10.2)
     const double sums = few ? (N % 4 != 0 ? 1.5 : 0.0) + 0.4 * std::max(0, split.splits - 4) : 0.0;
-    return split.us + sums < (stream ? 0.8 : 0.95) * plain ? split.splits : 1;
+    // (next to 64x32 tiles: a weight from memory at 5.8 TB/s at best - 16 x 8192 x 8192 fp16, two splits, 25 us by their steps, measured 32)
+    const double least = thin && 128.0 * steps * N >= 64e6 ? kLaunchUs + 2.5 + 128.0 * steps * N / 5.8e6 + (double)split.splits * M * N * 8.0 / 3e6 : 0.0;
+    return std::max(split.us, least) + sums < (stream ? 0.8 : 0.95) * plain ? split.splits : 1;
   }
   // the one-barrier-per-step kernel on 128x128 tiles, 64-byte K steps: a workgroup per CU, at least sixteen K steps each, at most
   // 32 slices; nothing to gain from half a round of tiles on or below 64 K steps
@@ -637,7 +639,7 @@ static int gemm_impl(const void* A, const void* B, void* C, int M, int N, int K,
   if (is8 && mixed_rows > 0) return gemm_wave128_f8_mixed_launch(p, mixed_rows, in_dtype == MI355_F8E5M2, stream);
   if (is8 && tile == 6 && (p.tile_m == 192 || p.tile_m == 128 || w128_ok)) return gemm_wave128_f8_launch(p, in_dtype == MI355_F8E5M2, b_kmajor, stream);
   if (is8) return gemm8_launch(p, in_dtype == MI355_F8E5M2, b_kmajor, tile, stream);
-  // 6: four waves, 128x128 of C per wave from 16x16x32 MFMAs (whole tiles)
+  // 6: four waves, 128x128 of C per wave from 16x16x32 MFMAs
   // (a tile height of 192 / 128 rows was set above only after gemm_wave128_192_ok had accepted the shape for it)
   if (mixed_rows > 0 && !is8) return gemm_wave128_mixed_launch(p, mixed_rows, in_dtype == MI355_BF16, b_kmajor, stream);
   if (tile == 6 && (p.tile_m == 192 || p.tile_m == 128 || w128_ok)) return gemm_wave128_launch(p, in_dtype == MI355_BF16, b_kmajor, stream);
@@ -756,6 +758,10 @@ GemmRoute gemm_route(const void* A, const void* B, int M, int N, int K, int64_t 
     const int64_t k_bytes = (int64_t)r.k * es;
     r.splits = auto_splits(M, N, k_bytes, in_dtype, kmajor, ring_ok(es, kmajor), cus);
     r.slice_bytes = r.splits > 1 ? (size_t)r.splits * M * N * 4 : 0;
+    if (ring_ok(es, kmajor) && thin_ok(M, N, k_bytes, kmajor, cus)) {   // (the bytes stay at least those of a split on other tiles)
+      const int others = auto_splits(M, N, k_bytes, in_dtype, kmajor, true, cus, false);
+      if (others > 1) r.slice_bytes = std::max(r.slice_bytes, (size_t)others * M * N * 4);
+    }
     if (r.splits > 1 || r.k_rows > 0 || !ring_ok(es, kmajor) || k_bytes < 2048) return;
     // room for the slices of what best_cut leaves to a second call (gemm_impl decides again: without the room that part is not split)
     const long tiles256 = (long)((M + 255) / 256) * ((N + 255) / 256);
