@@ -1580,3 +1580,27 @@ def test_a_part_of_a_round_of_tiles_in_a_call_of_its_own(gpu, dtype, M, N, K):
         row = torch.randint(-8, 9, (N,), device=gpu, generator=g).to(torch.bfloat16)
         got = triton_amd.matmul(a, tb, out_dtype=torch.bfloat16, add=row)
         assert torch.equal(got, (want + row.float()).to(torch.bfloat16))
+
+
+@pytest.mark.parametrize("M,N,kbytes", [(17, 1000, 2064), (64, 8192, 2176), (33, 8161, 2304), (16, 8192, 4096), (16, 5760, 2176), (64, 8200, 2176), (24, 4096, 8192)])
+@pytest.mark.parametrize("dtype", ["bf16", "e4m3"])
+def test_few_rows_next_to_a_k_major_weight_at_the_edges_of_their_tiles(gpu, dtype, M, N, kbytes):
+    # sizes around the rule for the 64x32 ring tiles: the first K beyond it, a whole round of CUs and just beyond one, partial
+    # last tiles, 16 rows on either side of the streaming kernel, a K that other tiles split.  Sums of at most 2^13 products of -1 .. 1 are
+    # whole numbers below 2^24: exact in fp32, with the workspace and without.
+    rng = np.random.default_rng(M + N)
+    K = kbytes // (1 if dtype == "e4m3" else 2)
+    a = rng.integers(-1, 2, size=(M, K)).astype(np.float32)
+    b = rng.integers(-1, 2, size=(N, K)).astype(np.float32)
+    row = rng.integers(-3, 4, size=(1, N)).astype(np.float32)
+    ref = a @ b.T
+    if dtype == "e4m3":
+        ta, tb = (torch.from_numpy(formats.encode_fp8(x, "e4m3")).to(gpu).view(torch.float8_e4m3fn) for x in (a, b))
+    else:
+        ta, tb = from_np(a, dtype, gpu), from_np(b, dtype, gpu)
+    assert bits_equal(to_np(triton_amd.matmul(ta, tb.t(), out_dtype=torch.float32)), ref)
+    assert bits_equal(to_np(triton_amd.matmul(ta, tb.t(), out_dtype=torch.float32, add=from_np(row, "fp32", gpu))), ref + row)
+    c = torch.empty(M, N, dtype=torch.float32, device=gpu)
+    rc = _lib.load().mi355_gemm(ta.data_ptr(), tb.data_ptr(), c.data_ptr(), M, N, K, K, 1, 1, K, N, 1, _lib.F8E4M3 if dtype == "e4m3" else _lib.BF16,
+                                _lib.F32, None, None, _lib.ACT_NONE, torch.cuda.current_stream().cuda_stream)
+    assert rc == 0 and bits_equal(to_np(c), ref)
