@@ -263,7 +263,8 @@ bool short_k(int M, int N, int k_bytes, bool b_kmajor, int cus) {
 bool ring_ok(int elem_bytes, bool b_kmajor) { return elem_bytes == 2 || (elem_bytes == 1 && b_kmajor); }
 
 // Whether the streaming kernel (gemm_skinny.hip: a workgroup per 32 rows of the long operand, K split over its four waves)
-// takes a product of at most 64 rows on a side ahead of the ring kernels.  Measured over rows 1 .. 64, long sides of 1024 ..
+// takes a product of at most 64 rows on a side ahead of the ring kernels (17 .. 64 rows of C next to a K-major weight are the 64x32 ring
+// tiles', `thin`: the figures of 33 rows and more below hold for the columns of C, and for what those tiles are compared with).  Measured over rows 1 .. 64, long sides of 1024 ..
 // 32768, K of 512 .. 16384, fp16 and e4m3, all layouts, weights from memory and from cache; ring / streaming, us:
 //   * a K-contiguous long operand: as long as its workgroups are one round of CUs (16 x 8192 x 2048 fp16 12.0 / 10.0, 16 x
 //     12288 x 2048 12 / 16.5), from 2048 bytes of K on (16 x 4096 x 512 fp16 4.6 / 4.6; below, the ring up to 15 % ahead) - for
