@@ -1509,14 +1509,14 @@ def test_columns_or_rows_beyond_whole_tiles_in_a_call_of_their_own(gpu, M, N, K,
 
 
 @pytest.mark.parametrize("programs", [3, 256])
-@pytest.mark.parametrize("dtype,kmajor", [("fp16", False), ("fp16", True), ("bf16", False), ("bf16", True), ("e4m3", True)])
+@pytest.mark.parametrize("dtype,kmajor", [("fp16", False), ("fp16", True), ("bf16", False), ("bf16", True), ("e4m3", True), ("e4m3", False), ("e5m2", False)])
 def test_four_wave_kernels_on_tiles_moved_back_from_the_edges_are_bit_exact(gpu, monkeypatch, dtype, kmajor, programs):
     # sizes that are no whole tiles: the last tiles lie partly over their neighbours, and with a row-major B the last columns
     # of a tile may be padding.  One tile, one row or column more, a chunk more, odd rows of C, a K tail, every tile height;
     # bias row, addend matrix, activation, fp32 / fp8 output.  Whole numbers: exact in every order
     set_knob(monkeypatch, "MI355_GEMM_TILE", "6")
     set_knob(monkeypatch, "MI355_GEMM_PROGRAMS", str(programs))
-    tdt = {"fp16": torch.float16, "bf16": torch.bfloat16, "e4m3": torch.float8_e4m3fn}[dtype]
+    tdt = {"fp16": torch.float16, "bf16": torch.bfloat16, "e4m3": torch.float8_e4m3fn, "e5m2": torch.float8_e5m2}[dtype]
     out = torch.float16 if dtype != "bf16" else torch.bfloat16
     g = torch.Generator(device=gpu).manual_seed(len(dtype) + kmajor)
 
@@ -1547,6 +1547,41 @@ def test_four_wave_kernels_on_tiles_moved_back_from_the_edges_are_bit_exact(gpu,
             a, b = ints(M, K).to(tdt), ints(N, K).to(tdt)
             tb = b.t() if kmajor else b.t().contiguous()
             assert torch.equal(triton_amd.matmul(a, tb, out_dtype=out).float(), (a.float() @ b.t().float()).to(out).float()), (M, N, K, rows)
+
+
+@pytest.mark.parametrize("out", ["fp16", "bf16"])
+@pytest.mark.parametrize("fmt", ["e4m3", "e5m2"])
+def test_tiles_that_end_in_a_row_major_fp8_b_s_padding_store_no_column_behind_c(gpu, monkeypatch, fmt, out):
+    # a row-major fp8 B is fetched in chunks of 16 columns: the last tile of an N that is no multiple of 16 ends in up to 15 columns that
+    # C does not have - the first ones of its next row where C is dense, and behind the last row nobody's.  The padding of B
+    # holds NaN codes, C lies in a larger buffer; the four-wave kernel forced, then the sizes that take it by themselves.  Whole
+    # numbers: exact
+    lib, stream = _lib.load(), torch.cuda.current_stream().cuda_stream
+    tdt = torch.float8_e4m3fn if fmt == "e4m3" else torch.float8_e5m2
+    odt, abi_out = {"fp16": (torch.float16, _lib.F16), "bf16": (torch.bfloat16, _lib.BF16)}[out]
+    abi_in = _lib.F8E4M3 if fmt == "e4m3" else _lib.F8E5M2
+    g = torch.Generator(device=gpu).manual_seed(7)
+    for M, N, K, forced in ((256, 264, 256, True), (300, 257, 256, True), (257, 271, 512, True), (511, 520, 256, True), (4096, 4104, 1024, False), (4096, 4088, 1024, False)):
+        if forced:
+            set_knob(monkeypatch, "MI355_GEMM_TILE", "6")
+        else:
+            monkeypatch.delenv("MI355_GEMM_TILE", raising=False)
+            lib.mi355_refresh_env()
+        a = torch.randint(-2, 3, (M, K), device=gpu, generator=g).to(tdt)
+        b = torch.randint(-2, 3, (K, N), device=gpu, generator=g).to(tdt)
+        want = (a.float() @ b.float()).to(odt)
+        assert torch.equal(triton_amd.matmul(a, b, out_dtype=odt), want), (M, N, K)
+        for b_pitch in (-(-N // 16) * 16, -(-N // 16) * 16 + 48):
+            wide = torch.full((K, b_pitch), 0x7F, device=gpu, dtype=torch.uint8)
+            wide[:, :N] = b.view(torch.uint8)
+            for ldc in (N, -(-N // 8) * 8 + 8):
+                for row in (None, torch.randint(-8, 9, (N,), device=gpu, generator=g).to(odt)):
+                    c = torch.full((M + 2, ldc), -7.0, device=gpu, dtype=odt)
+                    expect = c.clone()
+                    expect[:M, :N] = want if row is None else (a.float() @ b.float() + row.float()).to(odt)
+                    rc = lib.mi355_gemm_epilogue(a.data_ptr(), wide.data_ptr(), c.data_ptr(), M, N, K, K, 1, b_pitch, 1, ldc, 1, abi_in, abi_out, None, None,
+                                                 None if row is None else row.data_ptr(), 0, 1, abi_out, _lib.ACT_NONE, 0, stream)
+                    assert rc == 0 and torch.equal(c, expect), (M, N, K, b_pitch, ldc, row is None)
 
 
 def test_an_addend_that_is_c_is_added_once(gpu):

@@ -143,8 +143,8 @@ __device__ __forceinline__ void swap16(int& a, int& b) {
 // ANY = false: C in a 16-bit type with unit column stride, the addend (if any) a row of N consecutive values - a bias, read
 // once for all rows of the lane (rows_epilogue).  C leaves as 16 bytes per lane (gemm_epilogue16_lean) whatever its alignment:
 // the memory pipeline splits what it has to.  ANY = true: every output type, strides and addend that the C ABI takes.
-// Columns from p.N on are left out; they can only be the last seven of the wave's 128, the padding that a tile of a
-// row-major B may end in, so that only the last columns are looked at.
+// Columns from p.N on are left out; they can only be the last seven (16-bit operands) or fifteen (fp8) of the wave's 128, the
+// padding of a 16-byte chunk that a tile of a row-major B may end in, so that only the last 16 columns are looked at.
 template <int MT, int NT, bool ANY>
 __device__ __forceinline__ void gemm_epilogue16(f32x4 (&acc)[MT][NT], const GemmArgs& p, int mrow0, int ncol0, int l16, int kg) {
   static_assert(NT % 2 == 0, "pairs of 16-column tiles");

@@ -856,9 +856,12 @@ int gemm_wave128_f8_launch(const GemmArgs& p, bool e5m2, bool b_kmajor, hipStrea
     return e5m2 ? launch_wave128_f8<1, 4, false, true, 128>(p, stream) : launch_wave128_f8<0, 4, false, true, 128>(p, stream);
   }
   if (!b_kmajor) {   // (gemm_wave128_f8_ok: whole pairs of K steps)
-    const int lean = lean_epilogue_type(p);
+    // The last column of tiles ends at whole 16-byte chunks of B's rows, that is at whole sixteens of columns: the lean epilogue, which
+    // stores every column of its tile, only where C has them all (N = 8 mod 16 passes lean_epilogue_type, enough for 16-bit operands)
+    const int lean = p.N % 16 == 0 ? lean_epilogue_type(p) : 0;
     if (lean == 1) return e5m2 ? launch_wave128_f8<1, 3, false, false>(p, stream) : launch_wave128_f8<0, 3, false, false>(p, stream);
     if (lean == 2) return e5m2 ? launch_wave128_f8<1, 4, false, false>(p, stream) : launch_wave128_f8<0, 4, false, false>(p, stream);
+    if (rows_epilogue(p)) return e5m2 ? launch_wave128_f8<1, 2, false, false>(p, stream) : launch_wave128_f8<0, 2, false, false>(p, stream);
     return e5m2 ? launch_wave128_f8<1, 0, false, false>(p, stream) : launch_wave128_f8<0, 0, false, false>(p, stream);
   }
   if (p.k_bytes % 256 != 0) {
