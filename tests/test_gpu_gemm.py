@@ -1549,6 +1549,23 @@ def test_four_wave_kernels_on_tiles_moved_back_from_the_edges_are_bit_exact(gpu,
             assert torch.equal(triton_amd.matmul(a, tb, out_dtype=out).float(), (a.float() @ b.t().float()).to(out).float()), (M, N, K, rows)
 
 
+@pytest.mark.parametrize("dtype", ["fp16", "bf16"])
+@pytest.mark.parametrize("K", [136, 160, 184, 200, 248, 264])
+def test_few_k_steps_with_a_remainder_next_to_a_row_major_b_are_bit_exact(gpu, monkeypatch, dtype, K):
+    # three, four and five K steps of which the first is a remainder: the fill cursor of the four-wave kernel wraps while the lines that
+    # it touches ahead still have to lie among B's rows, whatever the tile's row (eight of them share a panel of B).  B is the last of
+    # its allocation's rows.  Whole numbers: exact
+    set_knob(monkeypatch, "MI355_GEMM_TILE", "6")
+    tdt = {"fp16": torch.float16, "bf16": torch.bfloat16}[dtype]
+    g = torch.Generator(device=gpu).manual_seed(K)
+    M, N = 2049, 4104
+    a = torch.randint(-2, 3, (M, K), device=gpu, generator=g).to(tdt)
+    b = torch.randint(-2, 3, (4096, N), device=gpu, generator=g).to(tdt)[4096 - K:]
+    want = a.float() @ b.float()
+    assert torch.equal(triton_amd.matmul(a, b, out_dtype=tdt), want.to(tdt))
+    assert torch.equal(triton_amd.matmul(a, b, out_dtype=torch.float32), want)
+
+
 @pytest.mark.parametrize("out", ["fp16", "bf16"])
 @pytest.mark.parametrize("fmt", ["e4m3", "e5m2"])
 def test_tiles_that_end_in_a_row_major_fp8_b_s_padding_store_no_column_behind_c(gpu, monkeypatch, fmt, out):

@@ -342,6 +342,9 @@ __device__ __forceinline__ void gemm_wave128_tiles(const GemmArgs& p, int tile, 
       int fm, fn;
       tile_at(ftile, fm, fn);
       set_fill_tile(fm, fn);
+      // (behind a head, step s is 128 bytes back: from the tile's own start a touch of the last step of three or four would lie up to 63
+      // rows behind a row-major B; the loads themselves fetch the first two whole steps)
+      if constexpr (PF && ANYK && !B_KMAJOR) { if (head) pB -= kstepB; }
     }
   };
   if (nk == 2) { fk = 1; advance(); }   // (two steps per tile: the prologue fetched both, the cursor is on the next tile)
