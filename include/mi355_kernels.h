@@ -312,7 +312,7 @@ int mi355_mx_gemm(const uint8_t* A, const uint8_t* sA, const uint8_t* B, const u
 
 /* The same with a workspace of the caller's (device memory, 16-byte aligned, its own for every call under way): products of
  * few tiles and a long K are then split along K, the fp32 slices being added in split order.  The size that a product wants,
- * in bytes, comes from mi355_mx_gemm_workspace (0: none); with workspace_bytes 0 the call is mi355_mx_gemm. */
+ * in bytes, comes from mi355_mx_gemm_workspace (0: none); with less than that, or a null pointer, the call is mi355_mx_gemm. */
 int64_t mi355_mx_gemm_workspace(int M, int N, int K, int fmt);
 int mi355_mx_gemm_ws(const uint8_t* A, const uint8_t* sA, const uint8_t* B, const uint8_t* sB, void* C,
                      int M, int N, int K, int fmt, int out_dtype,

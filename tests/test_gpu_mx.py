@@ -6,6 +6,7 @@ import pytest
 import torch
 
 import triton_amd
+from triton_amd import _lib
 from oracle import formats, mx
 from util import bits_equal, report_error, to_np, set_knob
 
@@ -334,3 +335,25 @@ def test_ring_kernels_at_the_edges_of_their_ring_are_bit_exact(gpu, monkeypatch,
             got = triton_amd.mx_matmul(*ops, fmt, out_dtype=torch.float32)
             assert bits_equal(to_np(got), ref), (M, N, K, extra)
         assert bits_equal(_run(gpu, a, sa, b, sb, fmt, torch.bfloat16), formats.round_bf16(ref)), (M, N, K)
+
+
+@pytest.mark.parametrize("fmt", ["mxfp4", "mxfp8"])
+def test_less_workspace_than_a_split_wants_means_the_plain_call(gpu, fmt):
+    # through the C ABI: no room, a byte less than asked for (left as it was), all of it, and a null pointer.  Exact sums
+    lib, stream = _lib.load(), torch.cuda.current_stream().cuda_stream
+    M, N, K = 64, 512, 8192
+    a, sa, b, sb = _operands(np.random.default_rng(5), M, N, K, "mxfp4", lo=126, hi=129)
+    if fmt == "mxfp8":
+        a, b = (formats.encode_fp8(np.random.default_rng(rows).integers(-2, 3, size=(rows, K)).astype(np.float32), "e4m3") for rows in (M, N))
+    ref = mx.mx_matmul(a, sa, b, sb, fmt, out_dtype="fp32")
+    ta, tsa, tb, tsb = (torch.from_numpy(x).to(gpu) for x in (a, sa, b, sb))
+    need = lib.mi355_mx_gemm_workspace(M, N, K, _lib.MXFP4 if fmt == "mxfp4" else _lib.MXFP8)
+    assert need > 0
+    for size, null in ((need, False), (need - 1, False), (16, False), (0, False), (need, True)):
+        ws = torch.full((need,), 0xA5, device=gpu, dtype=torch.uint8)
+        c = torch.empty(M, N, device=gpu, dtype=torch.float32)
+        rc = lib.mi355_mx_gemm_ws(ta.data_ptr(), tsa.data_ptr(), tb.data_ptr(), tsb.data_ptr(), c.data_ptr(), M, N, K,
+                                  _lib.MXFP4 if fmt == "mxfp4" else _lib.MXFP8, _lib.F32, ta.stride(0), tb.stride(0), tsa.stride(0), tsb.stride(0), N,
+                                  None if null else ws.data_ptr(), size, stream)
+        assert rc == 0 and bits_equal(to_np(c), ref), (size, null)
+        assert bool((ws == 0xA5).all()) == (size < need or null), (size, null)
