@@ -60,13 +60,11 @@ def test_mxfp4_exact_sums_are_bitwise(gpu, shape):
 @pytest.mark.parametrize("programs", [3, 256])
 @pytest.mark.parametrize("fmt", ["mxfp4", "mxfp8"])
 def test_four_wave_kernels_k_tails_are_bit_exact(gpu, monkeypatch, fmt, programs):
-    # K not a multiple of 1024 in the four-wave kernels: what is left behind the last whole group of K steps follows in
-    # steps whose fragments and scale bytes come straight from global memory, zeros beyond K.  Every class of tail
-    # (one block, part of a step, whole steps, all but one block), one and several tiles per program (the tail runs
-    # while the stages and half of the registers hold the next tile's first steps), each epilogue (fp32: general;
-    # bf16, fp16: lean).  Exact data (fp4 values, or small integers as e4m3, with scales 1/2, 1, 2: every partial sum
-    # is exact in fp32), so the results carry the oracle's bits.  The scale rows are slices of wider ones: the
-    # 16-byte scale loads of these kernels need a pitch that is a multiple of 16.
+    # K that is no whole number of scale groups in the four-wave kernels: what is left of the last 128-byte step of a row is multiplied
+    # first, with zeros - and scales of 1 - beyond K.  Every class of remainder (one block, part of a step, whole steps, all but
+    # one block; one tile per workgroup, whatever the number of programs) and each epilogue (fp32: general; bf16, fp16: lean).
+    # Exact data (fp4 values, or small integers as e4m3, with scales 1/2, 1, 2: every partial sum is exact in fp32), so the
+    # results carry the oracle's bits.  The scale rows are slices of wider ones, NaN behind K.
     set_knob(monkeypatch, "MI355_GEMM_TILE", "6")
     set_knob(monkeypatch, "MI355_GEMM_PROGRAMS", programs)
     rng = np.random.default_rng(programs + len(fmt))
@@ -82,7 +80,7 @@ def test_four_wave_kernels_k_tails_are_bit_exact(gpu, monkeypatch, fmt, programs
             sb = rng.integers(126, 129, size=(N, K // 32)).astype(np.uint8)
         ref32 = mx.mx_matmul(a, sa, b, sb, fmt, out_dtype="fp32")
         pitch = -(-(K // 32) // 16) * 16
-        wa = torch.full((M, pitch), 0xFF, dtype=torch.uint8, device=gpu)      # (NaN scales beyond K: never read)
+        wa = torch.full((M, pitch), 0xFF, dtype=torch.uint8, device=gpu)      # (NaN scales beyond K: read in whole dwords, never used)
         wb = torch.full((N, pitch), 0xFF, dtype=torch.uint8, device=gpu)
         wa[:, :K // 32] = t(sa)
         wb[:, :K // 32] = t(sb)
@@ -92,6 +90,51 @@ def test_four_wave_kernels_k_tails_are_bit_exact(gpu, monkeypatch, fmt, programs
         for out, rnd in ((torch.float32, lambda x: x), (torch.bfloat16, formats.round_bf16), (torch.float16, lambda x: x.astype(np.float16).astype(np.float32))):
             got = to_np(triton_amd.mx_matmul(ta, wa[:, :K // 32], tb, wb[:, :K // 32], fmt, out_dtype=out))
             assert bits_equal(got, rnd(ref32)), (fmt, K, programs, out)
+
+
+@pytest.mark.parametrize("programs", [3, 256])
+@pytest.mark.parametrize("fmt", ["mxfp4", "mxfp8"])
+def test_four_wave_kernels_on_tiles_moved_back_from_the_edges_are_bit_exact(gpu, monkeypatch, fmt, programs):
+    # M and N of no whole tiles, at every way the scales travel: rows of a pitch that is 4 mod 16 (a dword a lane) or whole 16 bytes, K
+    # of two, three, five and nine 128-byte steps, with a remainder before them and without, and of whole scale groups (several tiles
+    # as one stream for 3 programs); tiles of 192 and 128 rows.  Data as above, NaN scales behind K and behind the rows
+    set_knob(monkeypatch, "MI355_GEMM_TILE", "6")
+    set_knob(monkeypatch, "MI355_GEMM_PROGRAMS", str(programs))
+    rng = np.random.default_rng(programs + len(fmt))
+    per_byte = 2 if fmt == "mxfp4" else 1
+    group = 512 if fmt == "mxfp4" else 1024
+
+    def check(M, N, kbytes, pitch_mod):
+        K = kbytes * per_byte
+        if fmt == "mxfp4":
+            a, sa, b, sb = _operands(rng, M, N, K, fmt, lo=126, hi=129)
+        else:
+            a, b = (formats.encode_fp8(rng.integers(-4, 5, size=(rows, K)).astype(np.float32), "e4m3") for rows in (M, N))
+            sa, sb = (rng.integers(126, 129, size=(rows, K // 32)).astype(np.uint8) for rows in (M, N))
+        ref = mx.mx_matmul(a, sa, b, sb, fmt, out_dtype="fp32")
+        pitch = K // 32
+        while pitch % 16 != pitch_mod:
+            pitch += 1
+
+        def scales(x):
+            wide = np.full((x.shape[0] + 1, pitch), 0xFF, dtype=np.uint8)
+            wide[:-1, : x.shape[1]] = x
+            return torch.from_numpy(wide).to(gpu)[:-1, : x.shape[1]]
+
+        ta, tb = torch.from_numpy(a).to(gpu), torch.from_numpy(b).to(gpu)
+        for out, rnd in ((torch.float32, lambda x: x), (torch.bfloat16, formats.round_bf16)):
+            got = to_np(triton_amd.mx_matmul(ta, scales(sa), tb, scales(sb), fmt, out_dtype=out))
+            assert bits_equal(got, rnd(ref)), (M, N, K, pitch, out)
+
+    for M, N in ((257, 300), (511, 513), (264, 520)):
+        for kbytes in (256, 256 + (16 if fmt == "mxfp4" else 32), 384, 640, 1152):
+            check(M, N, kbytes, 4)
+        for kbytes in (384, group, 3 * group):
+            check(M, N, kbytes, 0)
+    for rows in ("192", "128"):
+        set_knob(monkeypatch, "MI355_GEMM_TILE_M", rows)
+        for M, N in ((192, 256), (200, 264), (449, 520)):
+            check(M, N, 2 * group, 0)
 
 
 @pytest.mark.parametrize("programs", [3, 256])
@@ -280,8 +323,8 @@ def test_mxfp8_with_freshly_uploaded_operands_is_bit_exact_every_time(gpu, monke
 
 @pytest.mark.parametrize("fmt", ["mxfp4", "mxfp8"])
 def test_random_shapes_through_the_default_dispatch_are_bit_exact(gpu, fmt):
-    # Whatever kernel the size heuristics pick (four-wave tiles of three heights, two heights in one launch, their K
-    # tails, the eight-wave kernels, partial tiles): exact data - fp4 values or small integers as e4m3, scales 1/2, 1,
+    # Whatever kernel the size heuristics pick (four-wave tiles of three heights, two heights in one launch, any K,
+    # partial tiles, the ring and the eight-wave kernels): exact data - fp4 values or small integers as e4m3, scales 1/2, 1,
     # 2 - make every partial sum exact in fp32, so the results carry the oracle's bits.  Seeded shapes around the
     # thresholds of the heuristics.
     rng = np.random.default_rng({"mxfp4": 11, "mxfp8": 12}[fmt])
