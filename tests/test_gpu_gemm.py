@@ -1601,6 +1601,24 @@ def test_tiles_that_end_in_a_row_major_fp8_b_s_padding_store_no_column_behind_c(
                     assert rc == 0 and torch.equal(c, expect), (M, N, K, b_pitch, ldc, row is None)
 
 
+def test_sums_of_slices_beyond_2_31_groups_of_columns(gpu):
+    # 92736 x 92736 in two slices of the caller's, 69 GB: 2.15e9 groups of four columns.  Whole numbers: exact; rows from all over C
+    M = N = 92736
+    K = 128
+    g = torch.Generator(device=gpu).manual_seed(31)
+    a = torch.randint(-2, 3, (M, K), device=gpu, generator=g).half()
+    b = torch.randint(-2, 3, (N, K), device=gpu, generator=g).half()
+    ws = torch.empty(2 * M * N, dtype=torch.float32, device=gpu)
+    c = torch.full((M, N), float("nan"), dtype=torch.float16, device=gpu)
+    rc = _lib.load().mi355_gemm_splitk(a.data_ptr(), b.data_ptr(), c.data_ptr(), M, N, K, K, 1, 1, K, N, 1, _lib.F16, _lib.F16, None, None, _lib.ACT_NONE,
+                                       2, ws.data_ptr(), ws.numel() * 4, torch.cuda.current_stream().cuda_stream)
+    assert rc == 0
+    for first in (*range(0, M - 64, 4999), M - 64):
+        assert torch.equal(c[first:first + 64], (a[first:first + 64].float() @ b.float().t()).half()), first
+    del ws, c
+    torch.cuda.empty_cache()
+
+
 def test_an_addend_that_is_c_is_added_once(gpu):
     # in place through the C ABI: tiles that lie over their neighbours would add it twice
     M, N, K = 5001, 5000, 256

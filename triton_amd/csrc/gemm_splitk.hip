@@ -87,7 +87,7 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(GemmStridedArgs p, c
 
 int splitk_reduce_launch(const GemmStridedArgs& out, const float* workspace, int splits, hipStream_t stream) {
   const int64_t groups = ((int64_t)out.N + 3) / 4, threads = (int64_t)out.M * groups;
-  if (threads <= 0 || threads > 0x7fffffffll) return -1;   // (the slices are 64 MiB at most by the library's own choice; a caller's: 8 TB)
+  if (threads <= 0 || threads > 0xffffff00ll) return -1;   // (the launch's own limit, and the index's: 128 GiB of a caller's slices; the library's are 64 MiB at most)
   splitk_reduce_kernel<<<dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, stream>>>(out, workspace, splits, (unsigned)groups, (unsigned)threads);
   return (int)hipGetLastError();
 }
