@@ -44,8 +44,8 @@ __device__ __forceinline__ void mfma16(f16x8 a, f16x8 b, f32x4& c) {
 // with the 128 KiB of LDS at `lds0`.  XCD: pass the tile numbers through the per-XCD remap first.  EPI: 0 = every
 // epilogue of the C ABI; 1 = C has the type of the operands, no scales, no activation; 2 = C in a 16-bit type with a bias row
 // at most (rows_epilogue), any N; 3 = the lean epilogue (gemm_epilogue16_lean) with C in the operands' type.
-// ANYK: any K of whole 16-byte chunks, one tile (see head_load); a row-major B may end inside the last step (its p.K rows)
-// where A's padding fills it.  (The reference's own uneven-K shape: 8192 x 8192 x 8176, python/test/regression/test_performance.py:46.)
+// ANYK: any K of whole 16-byte chunks, one tile (see head_load).  (The reference's own uneven-K shape: 8192 x 8192 x 8176,
+// python/test/regression/test_performance.py:46.)
 template <typename V8, bool B_KMAJOR, bool XCD, int EPI = 0, bool ANYK = false, int BM = 256>
 __device__ __forceinline__ void gemm_wave128_tiles(const GemmArgs& p, int tile, const int tile_step, const unsigned lds0, const int tile_stop = -1) {
 #if MI355_DEVICE_PASS
@@ -82,8 +82,7 @@ __device__ __forceinline__ void gemm_wave128_tiles(const GemmArgs& p, int tile, 
   auto col_of = [&](int tn) { return min(tn * BN, last_n0); };
   int pm, pn;
   tile_at(tile, pm, pn);
-  const int part = p.k_bytes % ROWB;   // (ANYK) bytes of the first step of a K that is no whole number of them
-  const int head = !ANYK ? 0 : part > 0 ? part : !B_KMAJOR && p.K * 2 < p.k_bytes ? ROWB : 0;
+  const int head = ANYK ? p.k_bytes % ROWB : 0;   // bytes of the first step of a K that is no whole number of them
   const int nk = ANYK ? (p.k_bytes + ROWB - 1) / ROWB : p.k_bytes / ROWB;   // K steps (an even number without ANYK)
   int nk_last = nk & ~1;   // the steps of the loop, but opaque: see mfma_retire
   asm volatile("" : "+s"(nk_last));
@@ -241,7 +240,7 @@ __device__ __forceinline__ void gemm_wave128_tiles(const GemmArgs& p, int tile, 
   };
   if (ANYK && head) {   // (one block from the loads to their use: at a join the compiler may copy registers still in flight)
     const int k_main = p.k_bytes - head;
-    const int krows = p.K - k_main / 2;   // rows of a row-major B in this step
+    const int krows = head / 2;   // rows of a row-major B in this step
     i32x4 ta[LA], tb[8];
     head_load(ta, fA + k_main, (unsigned)p.lda, lane, head);
     if constexpr (B_KMAJOR) {
@@ -986,7 +985,7 @@ static int gemm_wave128_launch_typed(const GemmArgs& p, bool b_kmajor, bool own_
     return b_kmajor ? launch_wave128<V8, true, 3, false, 192>(p, stream) : launch_wave128<V8, false, 3, false, 192>(p, stream);
   if (p.tile_m == 128)
     return b_kmajor ? launch_wave128<V8, true, 3, false, 128>(p, stream) : launch_wave128<V8, false, 3, false, 128>(p, stream);
-  if (p.k_bytes % 256 != 0 || (!b_kmajor && p.K * 2 < p.k_bytes)) {
+  if (p.k_bytes % 256 != 0) {
     if (own_type_lean) return b_kmajor ? launch_wave128<V8, true, 3, true>(p, stream) : launch_wave128<V8, false, 3, true>(p, stream);
     if (rows_epilogue(p)) return b_kmajor ? launch_wave128<V8, true, 2, true>(p, stream) : launch_wave128<V8, false, 2, true>(p, stream);
     return b_kmajor ? launch_wave128<V8, true, 0, true>(p, stream) : launch_wave128<V8, false, 0, true>(p, stream);
