@@ -1674,3 +1674,26 @@ def test_few_rows_next_to_a_k_major_weight_at_the_edges_of_their_tiles(gpu, dtyp
     rc = _lib.load().mi355_gemm(ta.data_ptr(), tb.data_ptr(), c.data_ptr(), M, N, K, K, 1, 1, K, N, 1, _lib.F8E4M3 if dtype == "e4m3" else _lib.BF16,
                                 _lib.F32, None, None, _lib.ACT_NONE, torch.cuda.current_stream().cuda_stream)
     assert rc == 0 and bits_equal(to_np(c), ref)
+
+
+@pytest.mark.parametrize("dtype,kmajor,sizes", [
+    ("bf16", False, [(1344, 6080, 6400), (4992, 896, 5632), (2816, 1536, 3584), (688, 5984, 4800), (5568, 768, 3072), (1264, 3392, 4304)]),
+    ("bf16", True, [(704, 6272, 4736), (2304, 2048, 5632), (5136, 800, 4224), (1536, 2752, 4672), (1664, 2688, 3968), (4352, 1024, 3328)]),
+    ("e4m3", True, [(6640, 632, 5888), (6528, 2560, 7744), (5632, 768, 7168)])])
+def test_whoever_is_told_to_bring_a_workspace_finds_sums_in_it(gpu, dtype, kmajor, sizes):
+    # `mi355_gemm_workspace` and the call decide by one rule whether a product is cut and its second part split along K (aligned
+    # operands: no padded copies).  Among the sizes some whose only call is the faster way.  Whole numbers: exact
+    lib, stream = _lib.load(), torch.cuda.current_stream().cuda_stream
+    tdt, abi = (torch.bfloat16, _lib.BF16) if dtype == "bf16" else (torch.float8_e4m3fn, _lib.F8E4M3)
+    for M, N, K in sizes:
+        strides = (K, 1, *((1, K) if kmajor else (N, 1)))
+        need = lib.mi355_gemm_workspace(1 << 20, 1 << 21, M, N, K, *strides, abi)
+        g = torch.Generator(device=gpu).manual_seed(M)
+        a, b = (torch.randint(-1, 2, (rows, K), device=gpu, generator=g).to(tdt) for rows in (M, N))
+        tb = b if kmajor else b.t().contiguous()
+        ws = torch.full((need // 4 + 64,), float("nan"), device=gpu)
+        c = torch.empty(M, N, device=gpu, dtype=torch.bfloat16)
+        rc = lib.mi355_gemm_ws(a.data_ptr(), tb.data_ptr(), c.data_ptr(), M, N, K, *strides, N, 1, abi, _lib.BF16, None, None,
+                               None, 0, 0, 0, _lib.ACT_NONE, 0, ws.data_ptr(), need, stream)
+        assert rc == 0 and torch.equal(c, (a.float() @ b.float().t()).bfloat16()), (M, N, K)
+        assert not ws[:need // 4].isnan().any() and ws[need // 4:].isnan().all(), (M, N, K, need)

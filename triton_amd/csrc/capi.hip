@@ -358,6 +358,133 @@ bool addend_in_c(const GemmArgs& p) {
   return d.first < c.second && c.first < d.second;
 }
 
+// Which tile kernel a product runs on (not fp32's); `tile_arg` as in gemm_impl.
+struct TileChoice { int tile = 1, tile_m = 0; bool w128_ok = false; };   // tile_m: 0, or 192 / 128 rows of a four-wave tile
+TileChoice tile_choice(const GemmArgs& p, int in_dtype, bool b_kmajor, int tile_arg, int cus) {
+  const int M = p.M, N = p.N;
+  const bool is8 = elem_size(in_dtype) == 1;
+  const long tiles256 = (long)((M + 255) / 256) * ((N + 255) / 256);
+  TileChoice c;
+  // large problems run the software-pipelined 8-wave kernel
+  // (5 = the persistent form of the pipelined kernel; it falls back to 4 for edge tiles or a K tail)
+  // persistent only when every program gets the same number of tiles: with a remainder the hardware's
+  // dynamic dispatch of one workgroup per tile balances better (6144^3: 1011 vs 942 TFLOP/s)
+  c.tile = (tiles256 * 2 >= cus) ? (tiles256 % cus == 0 ? 5 : 4) : 1;
+  // 16-bit operands, from 256 rows and columns and at least half a round of tiles on: four waves of
+  // 16x16x32 MFMAs (at 8192^3 bf16 +5 % over the persistent form with a row-major
+  // B, +14 % with a K-major B; at 3072^3, 144 tiles, 790 vs 660 TFLOP/s for the 128x128 tiles)
+  // (fp8, K-major B: 16x16x128 MFMAs, 8192^3 e4m3 2790-2810 vs 2570-2600 TFLOP/s)
+  // (fp8 from three quarters of a round: at 144 tiles the eight-wave kernel is 4-7 % ahead - 3072^3 1520 vs
+  // 1450, 3072x3072x8192 2040 vs 1890 TFLOP/s -, at 196 tiles the four-wave one by 2 %, at 225 by 13 %)
+  // (partial tiles are whole ones moved back over their neighbours: an addend that is C itself must be read only once)
+  const bool once = (M % 256 != 0 || N % 256 != 0) && addend_in_c(p);
+  c.w128_ok = !once && (is8 ? gemm_wave128_f8_ok(p, b_kmajor) : gemm_wave128_ok(p, b_kmajor));
+  if (tiles256 * (is8 ? 4 : 2) >= cus * (is8 ? 3 : 1) && c.w128_ok) c.tile = 6;
+  c.tile = tile_arg >= 0 ? tile_arg : knob(knobs().tile, c.tile);
+  // 16-bit products whose 256 x 256 tiles fill the last round of CUs badly (or whose M is a multiple of 192 only): the
+  // same kernel on tiles of 192 x 256 where those use the CUs better (3072^3: 192 tiles instead of 144 for 256 CUs)
+  if (!is8 && tile_arg < 0 && (knobs().tile == UNSET || knobs().tile_m == 192) && gemm_wave128_192_ok(p, b_kmajor, in_dtype)) {
+    auto fill = [&](long t) { return t <= 0 ? 0.0 : (double)t / (double)(((t + cus - 1) / cus) * cus); };
+    const long tiles192 = (long)((M + 191) / 192) * ((N + 255) / 256);
+    const int want = knob(knobs().tile_m, 0);
+    // (below half a round of 256-row tiles the 128-row tiles further down may fill better still: 3072 x 2048 x 4096 bf16,
+    // 128 tiles of 192 rows 734 TFLOP/s, 192 tiles of 128 rows 815)
+    const long tiles128 = (long)((M + 127) / 128) * ((N + 255) / 256);
+    const bool rather128 = c.tile == 1 && tiles128 <= cus && fill(tiles128) > fill(tiles192) &&
+                           gemm_wave128_192_ok(p, b_kmajor, in_dtype, 128);
+    if (want == 192 || (want == 0 && !rather128 && tiles192 * 2 >= cus && (c.tile != 6 || fill(tiles192) > fill(tiles256) + 0.08))) {
+      c.tile = 6;
+      c.tile_m = 192;
+    }
+  }
+  // fp8 likewise (K-major B, 16-bit C), from three quarters of a round of the 192-row tiles on.  Flushed do_bench, e4m3,
+  // 256-row choice / 192-row tiles: 3072^3 (144 / 192 tiles) 1100 / 1565 TFLOP/s, 3072 x 3072 x 8192 1365 / 2145, 2304 x
+  // 4096 x 4096 1220 / 1785, 4608 x 4096 x 4096 (288 / 384) 1600 / 2070, 6144^3 (576 / 768) 2510 / 2805, 1536 x 8192 x 8192
+  // (192 / 256) 2100 / 2680; not taken where they fill worse: 3840 x 3840 x 4096 (225 / 300) 2270 / 1530, 5376 x 5120 x
+  // 4096 (420 / 560) 2185 / 1995
+  if (is8 && tile_arg < 0 && (knobs().tile == UNSET || knobs().tile_m == 192) && gemm_wave128_f8_192_ok(p, b_kmajor)) {
+    auto fill = [&](long t) { return t <= 0 ? 0.0 : (double)t / (double)(((t + cus - 1) / cus) * cus); };
+    const long tiles192 = (long)((M + 191) / 192) * ((N + 255) / 256);
+    const int want = knob(knobs().tile_m, 0);
+    if (want == 192 || (want == 0 && tiles192 * 4 >= cus * 3 && (c.tile != 6 || fill(tiles192) > fill(tiles256) + 0.08))) {
+      c.tile = 6;
+      c.tile_m = 192;
+    }
+  }
+  // and on tiles of 128 x 256 where the 256 x 256 tiles are too few for their kernel (less than half a round) but these
+  // fill more than half of one round (2560^3: 100 and 200 tiles; 716 -> 825 TFLOP/s against the 128 x 128 tiles; 2304 x
+  // 2048 x 8192, 144 tiles: 650 -> 692; at half a round the 128 x 128 tiles stay ahead, 2048 x 2048 x 4096: 627 vs 569)
+  if (!is8 && tile_arg < 0 && (knobs().tile == UNSET || knobs().tile_m == 128) && c.tile_m == 0 &&
+      gemm_wave128_192_ok(p, b_kmajor, in_dtype, 128)) {
+    const long tiles128 = (long)((M + 127) / 128) * ((N + 255) / 256);
+    const int want = knob(knobs().tile_m, 0);
+    if (want == 128 || (want == 0 && c.tile == 1 && tiles128 * 16 >= cus * 9 && tiles128 <= cus)) {
+      c.tile = 6;
+      c.tile_m = 128;
+    }
+  }
+  // fp8 likewise (measured: see the design notes' table of shapes)
+  if (is8 && tile_arg < 0 && (knobs().tile == UNSET || knobs().tile_m == 128) && c.tile_m == 0 &&
+      gemm_wave128_f8_192_ok(p, b_kmajor, 128)) {
+    const long tiles128 = (long)((M + 127) / 128) * ((N + 255) / 256);
+    const int want = knob(knobs().tile_m, 0);
+    if (want == 128 || (want == 0 && c.tile == 1 && tiles128 * 16 >= cus * 9 && tiles128 <= cus)) {
+      c.tile = 6;
+      c.tile_m = 128;
+    }
+  }
+  return c;
+}
+
+// 16-bit and fp8 products of more than one round of tiles whose last round is badly filled: the upper rows on 256-row
+// tiles and the lower ones on 192-row tiles in ONE launch, split by mixed_split.  MI355_GEMM_MIXED_ROWS forces the rows
+// of the 256-row part (0 = never).
+int mixed_choice(const GemmArgs& p, const TileChoice& c, int in_dtype, bool b_kmajor, int cus) {
+  const int M = p.M, N = p.N;
+  const long tiles256 = (long)((M + 255) / 256) * ((N + 255) / 256);
+  const bool is8 = elem_size(in_dtype) == 1;
+  auto mixed_ok = [&](int rows256) {
+    return is8 ? gemm_wave128_f8_mixed_ok(p, b_kmajor, rows256) : gemm_wave128_mixed_ok(p, b_kmajor, in_dtype, rows256);
+  };
+  if (knobs().tile == UNSET && knobs().tile_m == UNSET && N % 256 == 0) {
+    const int want = knob(knobs().mixed_rows, -1);
+    if (want > 0) {
+      if (mixed_ok(want)) return want;
+    } else if (want < 0 && c.tile == 6 && c.tile_m == 0 && tiles256 > cus && M % 256 == 0) {
+      const int rows = mixed_split(M, N / 256, cus);
+      if (rows > 0 && mixed_ok(rows)) return rows;
+    }
+  }
+  return 0;
+}
+
+// Whether a product goes to a ring kernel (`ring`: its shape, else -1; in place of the other 128x128 kernel but for the short K
+// of short_k) and whether it is worth two calls (`cut`, us 1e30: one).  The one place that decides: for the call, and for the room that
+// the second part of a cut product is given (gemm_route).
+struct PartChoice { int tile, ring; Cut cut; };
+PartChoice part_choice(const GemmArgs& p, const TileChoice& c, int es, bool b_kmajor, bool by_knob, int mixed_rows, int cus) {
+  const int M = p.M, N = p.N, steps = (p.k_bytes + 127) / 128, tile = c.tile;
+  const bool is8 = es == 1;
+  PartChoice r{tile, -1, {M, N, 1e30}};
+  if (!by_knob && tile != 6 && !p.aux && p.c_vec_ok && short_k(M, N, p.k_bytes, b_kmajor, cus)) r.tile = 1;   // (its addends and odd rows of C cost more)
+  else if (tile == 1 && by_knob) r.ring = 0;
+  else if (tile >= 8 && tile <= 10) r.ring = tile - 8;
+  else if (tile == 12 && b_kmajor) r.ring = 3;
+  else if (tile == 11) r.tile = 1;   // the one-barrier-per-step kernel on 128x128 tiles
+  else if (tile == 1 || (!by_knob && knobs().tile_m == UNSET && knobs().mixed_rows == UNSET)) {
+    const int rows = tile == 6 && c.tile_m ? c.tile_m : 256;
+    const RingPlan plan = ring_plan(M, N, steps, cus, 1, 1, 1.0, thin_ok(M, N, p.k_bytes, b_kmajor, cus));
+    const bool rounds = (tile == 6 || tile == 1) && plan.shape < 3;
+    const double plan_us = rounds ? ring_rounds_us(M, N, steps, cus, plan.shape) : plan.us;
+    double other = tile == 1 ? 1e30 : tiles256_us((long)((M + rows - 1) / rows) * ((N + 255) / 256), rows, steps, cus, tile != 6, is8);
+    if (mixed_rows > 0) other *= 0.9;   // (two tile heights in one launch are chosen where they gain at least 5 %)
+    if (plan_us < (tile == 6 ? 0.92 : 1.0) * other) r.ring = plan.shape;   // (pitches move the rings by up to 15 %: 1664 x 6912 x 2112 bf16, 702 tiles, 53 us for the estimate's 47)
+    const Cut cut = best_cut(M, N, steps, cus, tile, r.ring, is8);
+    if (cut.us < (tile == 1 ? 0.88 : 0.92) * std::min(plan_us, other)) r.cut = cut;
+  }
+  return r;
+}
+
 bool aligned(const void* p, size_t a) { return ((uintptr_t)p % a) == 0; }
 
 bool copy_strides(const int64_t* src, int64_t* dst) {
@@ -480,92 +607,10 @@ static int gemm_impl(const void* A, const void* B, void* C, int M, int N, int K,
     const int t32 = tile_arg >= 0 ? tile_arg : knob(knobs().tile, large ? (tiles256 % cus == 0 ? 5 : 4) : 1);
     return gemm32_launch(p, t32 == 6 || t32 == 7 ? 4 : t32, stream);   // (the four-wave 16x16 kernels and stream-K have no fp32 form)
   }
-  // large problems run the software-pipelined 8-wave kernel
-  // (5 = the persistent form of the pipelined kernel; it falls back to 4 for edge tiles or a K tail)
-  // persistent only when every program gets the same number of tiles: with a remainder the hardware's
-  // dynamic dispatch of one workgroup per tile balances better (6144^3: 1011 vs 942 TFLOP/s)
-  int tile = (tiles256 * 2 >= cus) ? (tiles256 % cus == 0 ? 5 : 4) : 1;
-  // 16-bit operands, whole 256x256 tiles and K steps, at least half a round of tiles: four waves of
-  // 16x16x32 MFMAs, one workgroup per tile (at 8192^3 bf16 +5 % over the persistent form with a row-major
-  // B, +14 % with a K-major B; at 3072^3, 144 tiles, 790 vs 660 TFLOP/s for the 128x128 tiles)
-  // (fp8, K-major B: 16x16x128 MFMAs, 8192^3 e4m3 2790-2810 vs 2570-2600 TFLOP/s)
-  // (an epilogue addend: instantiations of their own)
-  // (fp8 from three quarters of a round: at 144 tiles the eight-wave kernel is 4-7 % ahead - 3072^3 1520 vs
-  // 1450, 3072x3072x8192 2040 vs 1890 TFLOP/s -, at 196 tiles the four-wave one by 2 %, at 225 by 13 %)
-  // (partial tiles are whole ones moved back over their neighbours: an addend that is C itself must be read only once)
-  const bool once = (M % 256 != 0 || N % 256 != 0) && addend_in_c(p);
-  const bool w128_ok = !once && (is8 ? gemm_wave128_f8_ok(p, b_kmajor) : gemm_wave128_ok(p, b_kmajor));
-  if (tiles256 * (is8 ? 4 : 2) >= cus * (is8 ? 3 : 1) && w128_ok) tile = 6;
-  tile = tile_arg >= 0 ? tile_arg : knob(knobs().tile, tile);
-  // 16-bit products whose 256 x 256 tiles fill the last round of CUs badly (or whose M is a multiple of 192 only): the
-  // same kernel on tiles of 192 x 256 where those use the CUs better (3072^3: 192 tiles instead of 144 for 256 CUs)
-  if (!is8 && tile_arg < 0 && (knobs().tile == UNSET || knobs().tile_m == 192) && gemm_wave128_192_ok(p, b_kmajor, in_dtype)) {
-    auto fill = [&](long t) { return t <= 0 ? 0.0 : (double)t / (double)(((t + cus - 1) / cus) * cus); };
-    const long tiles192 = (long)((M + 191) / 192) * ((N + 255) / 256);
-    const int want = knob(knobs().tile_m, 0);
-    // (below half a round of 256-row tiles the 128-row tiles further down may fill better still: 3072 x 2048 x 4096 bf16,
-    // 128 tiles of 192 rows 734 TFLOP/s, 192 tiles of 128 rows 815)
-    const long tiles128 = (long)((M + 127) / 128) * ((N + 255) / 256);
-    const bool rather128 = tile == 1 && tiles128 <= cus && fill(tiles128) > fill(tiles192) &&
-                           gemm_wave128_192_ok(p, b_kmajor, in_dtype, 128);
-    if (want == 192 || (want == 0 && !rather128 && tiles192 * 2 >= cus && (tile != 6 || fill(tiles192) > fill(tiles256) + 0.08))) {
-      tile = 6;
-      p.tile_m = 192;
-    }
-  }
-  // fp8 likewise (K-major B, 16-bit C), from three quarters of a round of the 192-row tiles on.  Flushed do_bench, e4m3,
-  // 256-row choice / 192-row tiles: 3072^3 (144 / 192 tiles) 1100 / 1565 TFLOP/s, 3072 x 3072 x 8192 1365 / 2145, 2304 x
-  // 4096 x 4096 1220 / 1785, 4608 x 4096 x 4096 (288 / 384) 1600 / 2070, 6144^3 (576 / 768) 2510 / 2805, 1536 x 8192 x 8192
-  // (192 / 256) 2100 / 2680; not taken where they fill worse: 3840 x 3840 x 4096 (225 / 300) 2270 / 1530, 5376 x 5120 x
-  // 4096 (420 / 560) 2185 / 1995
-  if (is8 && tile_arg < 0 && (knobs().tile == UNSET || knobs().tile_m == 192) && gemm_wave128_f8_192_ok(p, b_kmajor)) {
-    auto fill = [&](long t) { return t <= 0 ? 0.0 : (double)t / (double)(((t + cus - 1) / cus) * cus); };
-    const long tiles192 = (long)((M + 191) / 192) * ((N + 255) / 256);
-    const int want = knob(knobs().tile_m, 0);
-    if (want == 192 || (want == 0 && tiles192 * 4 >= cus * 3 && (tile != 6 || fill(tiles192) > fill(tiles256) + 0.08))) {
-      tile = 6;
-      p.tile_m = 192;
-    }
-  }
-  // and on tiles of 128 x 256 where the 256 x 256 tiles are too few for their kernel (less than half a round) but these
-  // fill more than half of one round (2560^3: 100 and 200 tiles; 716 -> 825 TFLOP/s against the 128 x 128 tiles; 2304 x
-  // 2048 x 8192, 144 tiles: 650 -> 692; at half a round the 128 x 128 tiles stay ahead, 2048 x 2048 x 4096: 627 vs 569)
-  if (!is8 && tile_arg < 0 && (knobs().tile == UNSET || knobs().tile_m == 128) && p.tile_m == 0 &&
-      gemm_wave128_192_ok(p, b_kmajor, in_dtype, 128)) {
-    const long tiles128 = (long)((M + 127) / 128) * ((N + 255) / 256);
-    const int want = knob(knobs().tile_m, 0);
-    if (want == 128 || (want == 0 && tile == 1 && tiles128 * 16 >= cus * 9 && tiles128 <= cus)) {
-      tile = 6;
-      p.tile_m = 128;
-    }
-  }
-  // fp8 likewise (measured: see the design notes' table of shapes)
-  if (is8 && tile_arg < 0 && (knobs().tile == UNSET || knobs().tile_m == 128) && p.tile_m == 0 &&
-      gemm_wave128_f8_192_ok(p, b_kmajor, 128)) {
-    const long tiles128 = (long)((M + 127) / 128) * ((N + 255) / 256);
-    const int want = knob(knobs().tile_m, 0);
-    if (want == 128 || (want == 0 && tile == 1 && tiles128 * 16 >= cus * 9 && tiles128 <= cus)) {
-      tile = 6;
-      p.tile_m = 128;
-    }
-  }
-  // 16-bit and fp8 products of more than one round of tiles whose last round is badly filled: the upper rows on 256-row
-  // tiles and the lower ones on 192-row tiles in ONE launch, split by mixed_split.  MI355_GEMM_MIXED_ROWS forces the rows
-  // of the 256-row part (0 = never).
-  int mixed_rows = 0;
-  auto mixed_ok = [&](int rows256) {
-    return is8 ? gemm_wave128_f8_mixed_ok(p, b_kmajor, rows256) : gemm_wave128_mixed_ok(p, b_kmajor, in_dtype, rows256);
-  };
-  if (tile_arg < 0 && knobs().tile == UNSET && knobs().tile_m == UNSET && N % 256 == 0) {
-    const int want = knob(knobs().mixed_rows, -1);
-    const int nn = N / 256, P = cus;
-    if (want > 0) {
-      if (mixed_ok(want)) mixed_rows = want;
-    } else if (want < 0 && tile == 6 && p.tile_m == 0 && tiles256 > cus && M % 256 == 0) {
-      const int rows = mixed_split(M, nn, P);
-      if (rows > 0 && mixed_ok(rows)) mixed_rows = rows;
-    }
-  }
+  const TileChoice choice = tile_choice(p, in_dtype, b_kmajor, tile_arg, cus);
+  int tile = choice.tile;
+  p.tile_m = choice.tile_m;
+  const int mixed_rows = tile_arg < 0 ? mixed_choice(p, choice, in_dtype, b_kmajor, cus) : 0;
   p.num_programs = knob(knobs().programs, cus);  // persistent and stream-K forms (tile 5 / 7): one workgroup per CU
   if (p.num_programs > cus) p.num_programs = cus;       // (the stream-K workspace is sized for one program per CU)
   p.workspace = workspace;
@@ -594,30 +639,18 @@ static int gemm_impl(const void* A, const void* B, void* C, int M, int N, int K,
     if (gemm_skinny_ok(sk, y_kmajor, x_kmajor, es)) return gemm_skinny_launch(sk, in_dtype, y_kmajor, x_kmajor, stream);
     if (is8 && b_kmajor && !aux && gemm8_skinny_ok(p)) return gemm8_skinny_launch(p, in_dtype == MI355_F8E5M2, stream);
   }
-  // the ring kernels of 64 .. 128-row tiles where they are the faster ones by the two estimates above (and in place of the
-  // other 128x128 kernel but for the short K above)
+  // the ring kernels of 64 .. 128-row tiles, and products in two calls
   int ring = -1;
   if (can_ring) {
-    const bool by_knob = tile_arg >= 0 || knobs().tile != UNSET;
     if (k_rows > 0) {   // a row-major B that ends before A's padding does: the ring kernels know
       ring = ring_plan(M, N, ksteps128, cus, 1, 1).shape;
       p.K = k_rows;
-    } else if (!by_knob && tile != 6 && !aux && p.c_vec_ok && short_k(M, N, p.k_bytes, b_kmajor, cus)) tile = 1;   // (its addends and odd rows of C cost more)
-    else if (tile == 1 && by_knob) ring = 0;
-    else if (tile >= 8 && tile <= 10) ring = tile - 8;
-    else if (tile == 12 && b_kmajor) ring = 3;
-    else if (tile == 11) tile = 1;   // the one-barrier-per-step kernel on 128x128 tiles
-    else if (tile == 1 || (!by_knob && knobs().tile_m == UNSET && knobs().mixed_rows == UNSET)) {
-      const int rows = tile == 6 && p.tile_m ? p.tile_m : 256;
-      const RingPlan plan = ring_plan(M, N, ksteps128, cus, 1, 1, 1.0, thin_ok(M, N, p.k_bytes, b_kmajor, cus));
-      const bool rounds = (tile == 6 || tile == 1) && plan.shape < 3;
-      const double plan_us = rounds ? ring_rounds_us(M, N, ksteps128, cus, plan.shape) : plan.us;
-      double other = tile == 1 ? 1e30 : tiles256_us((long)((M + rows - 1) / rows) * ((N + 255) / 256), rows, ksteps128, cus, tile != 6, is8);
-      if (mixed_rows > 0) other *= 0.9;   // (two tile heights in one launch are chosen where they gain at least 5 %)
-      if (plan_us < (tile == 6 ? 0.92 : 1.0) * other) ring = plan.shape;   // (pitches move the rings by up to 15 %: 1664 x 6912 x 2112 bf16, 702 tiles, 53 us for the estimate's 47)
-      const Cut cut = best_cut(M, N, ksteps128, cus, tile, ring, is8);
-      if (!workspace && cut.us < (tile == 1 ? 0.88 : 0.92) * std::min(plan_us, other)) {
-        const int m = cut.m, n = cut.n;
+    } else {
+      const PartChoice parts = part_choice(p, choice, es, b_kmajor, tile_arg >= 0 || knobs().tile != UNSET, mixed_rows, cus);
+      tile = parts.tile;
+      ring = parts.ring;
+      if (!workspace && parts.cut.us < 1e30) {
+        const int m = parts.cut.m, n = parts.cut.n;
         const int64_t dm = m < M ? m : 0, dn = m < M ? 0 : n;
         const int rc = gemm_impl(A, B, C, m, n, K, sam, sak, sbk, sbn, scm, scn, in_dtype, out_dtype, a_scale, b_scale, activation,
                                  aux, aux_sm, aux_sn, aux_dtype, -1, group_m_arg, stream_);
@@ -638,12 +671,12 @@ static int gemm_impl(const void* A, const void* B, void* C, int M, int N, int K,
     return is8 ? gemm_ring8_launch(p, in_dtype == MI355_F8E5M2, ring, 1, 0, stream)
                : gemm_ring16_launch(p, in_dtype == MI355_BF16, b_kmajor, ring, 1, 0, stream);
   if (is8 && mixed_rows > 0) return gemm_wave128_f8_mixed_launch(p, mixed_rows, in_dtype == MI355_F8E5M2, stream);
-  if (is8 && tile == 6 && (p.tile_m == 192 || p.tile_m == 128 || w128_ok)) return gemm_wave128_f8_launch(p, in_dtype == MI355_F8E5M2, b_kmajor, stream);
+  if (is8 && tile == 6 && (p.tile_m == 192 || p.tile_m == 128 || choice.w128_ok)) return gemm_wave128_f8_launch(p, in_dtype == MI355_F8E5M2, b_kmajor, stream);
   if (is8) return gemm8_launch(p, in_dtype == MI355_F8E5M2, b_kmajor, tile, stream);
   // 6: four waves, 128x128 of C per wave from 16x16x32 MFMAs
   // (a tile height of 192 / 128 rows was set above only after gemm_wave128_192_ok had accepted the shape for it)
   if (mixed_rows > 0 && !is8) return gemm_wave128_mixed_launch(p, mixed_rows, in_dtype == MI355_BF16, b_kmajor, stream);
-  if (tile == 6 && (p.tile_m == 192 || p.tile_m == 128 || w128_ok)) return gemm_wave128_launch(p, in_dtype == MI355_BF16, b_kmajor, stream);
+  if (tile == 6 && (p.tile_m == 192 || p.tile_m == 128 || choice.w128_ok)) return gemm_wave128_launch(p, in_dtype == MI355_BF16, b_kmajor, stream);
   return gemm16_launch(p, in_dtype == MI355_BF16, b_kmajor, tile, stream);
 }
 
@@ -763,15 +796,22 @@ GemmRoute gemm_route(const void* A, const void* B, int M, int N, int K, int64_t 
       const int others = auto_splits(M, N, k_bytes, in_dtype, kmajor, true, cus, false);
       if (others > 1) r.slice_bytes = std::max(r.slice_bytes, (size_t)others * M * N * 4);
     }
-    if (r.splits > 1 || r.k_rows > 0 || !ring_ok(es, kmajor) || k_bytes < 2048) return;
-    // room for the slices of what best_cut leaves to a second call (gemm_impl decides again: without the room that part is not split)
-    const long tiles256 = (long)((M + 255) / 256) * ((N + 255) / 256);
-    const int steps = (int)((k_bytes + 127) / 128), tile = M >= 256 && N >= 256 && tiles256 * (es == 1 ? 4 : 2) >= cus * (es == 1 ? 3 : 1) ? 6 : 1;
-    if ((long)((M + 127) / 128) * ((N + 127) / 128) <= cus) return;
-    const RingPlan plan = ring_plan(M, N, steps, cus, 1, 1);
-    const double plan_us = ring_rounds_us(M, N, steps, cus, plan.shape), other = tile == 6 ? tiles256_us(tiles256, 256, steps, cus, false, es == 1) : 1e30;
-    const Cut cut = best_cut(M, N, steps, cus, tile, plan_us < 0.92 * other ? plan.shape : -1, es == 1);
-    if (cut.us > std::min(plan_us, other)) return;
+    if (r.splits > 1 || r.k_rows > 0 || !ring_ok(es, kmajor) || k_bytes < 2048 || (long)((M + 127) / 128) * ((N + 127) / 128) <= cus) return;
+    // Room for the slices of what a cut leaves to a second call, by gemm_impl's own rule for a dense C of a 16-bit type without an addend
+    // (what this function is told).  For another C the rule may differ: then the room is not used, or that part is not split.
+    GemmArgs p{};
+    p.A = (const char*)A; p.B = (const char*)B;
+    p.M = M; p.N = N; p.K = r.k; p.k_bytes = (int)k_bytes;
+    p.lda = r.pack_a ? r.a_pitch : sam * es;
+    p.ldb = r.pack_b ? r.b_pitch : (kmajor ? sbn : sbk) * es;
+    p.ldc = N; p.scn = 1; p.out_dtype = in_dtype == MI355_BF16 ? MI355_BF16 : MI355_F16;
+    p.c_vec_ok = N % 4 == 0; p.lean_ok = knob(knobs().lean_epilogue, 1);
+    const TileChoice c = tile_choice(p, in_dtype, kmajor, -1, cus);
+    PartChoice parts = part_choice(p, c, es, kmajor, knobs().tile != UNSET, 0, cus);
+    if (parts.cut.us < 1e30)   // (two tile heights only make one call shorter: looked at where a cut is left without them)
+      if (const int rows = mixed_choice(p, c, in_dtype, kmajor, cus)) parts = part_choice(p, c, es, kmajor, knobs().tile != UNSET, rows, cus);
+    const Cut cut = parts.cut;
+    if (cut.us >= 1e30) return;
     const int m2 = cut.m < M ? M - cut.m : M, n2 = cut.m < M ? N : N - cut.n, splits = auto_splits(m2, n2, k_bytes, in_dtype, kmajor, true, cus);
     const size_t bytes = splits > 1 ? (size_t)splits * m2 * n2 * 4 : 0;
     if (bytes <= (16u << 20)) r.slice_bytes = bytes;
