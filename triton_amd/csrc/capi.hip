@@ -423,7 +423,7 @@ TileChoice tile_choice(const GemmArgs& p, int in_dtype, bool b_kmajor, int tile_
       c.tile_m = 128;
     }
   }
-  // fp8 likewise (measured: see the design notes' table of shapes)
+  // fp8 likewise, where the same part of a round is filled
   if (is8 && tile_arg < 0 && (knobs().tile == UNSET || knobs().tile_m == 128) && c.tile_m == 0 &&
       gemm_wave128_f8_192_ok(p, b_kmajor, 128)) {
     const long tiles128 = (long)((M + 127) / 128) * ((N + 255) / 256);
@@ -1194,7 +1194,7 @@ static int mx_impl(const uint8_t* A, const uint8_t* sA, const uint8_t* B, const 
   const int cus = device_info().cus > 0 ? device_info().cus : 256;
   const long tiles256 = (long)((M + 255) / 256) * ((N + 255) / 256);
   int tile = (tiles256 * 2 >= cus) ? (tiles256 % cus == 0 ? 5 : 4) : 1;
-  // MXFP4 with whole 256x256 tiles, K at least 1024 and at least half a round of tiles: four waves of
+  // MXFP4 from 256 rows and columns, 256 bytes of K and half a round of tiles on: four waves of
   // scaled 16x16x128 MFMAs (8192^3: 4000-4050 vs 3340-3640 TFLOP/s for the persistent eight-wave kernel)
   const int group = fmt == MI355_MXFP4 ? 512 : 1024;   // bytes of a row in a group of K steps of their streaming forms
   // (below half a round of tiles too where K is long, next to the ring kernels below)

@@ -290,8 +290,8 @@ __device__ __forceinline__ void gemm_epilogue16_plain(f32x4 (&acc)[MT][NT], cons
 
 // The common case as an epilogue of its own: C in a 16-bit type with unit column stride and aligned rows, the
 // product scaled by the per-tensor scales (1 without), no activation, no addend.  The general epilogue above decides
-// output type, activation and store form at run time inside its 64 unrolled tiles, which makes it 70 KiB of code -
-// more than the instruction cache holds, fetched anew at the end of every tile (and from memory when the kernel
+// output type, activation and store form at run time inside its 64 unrolled tiles: kernels of 132 - 140 KB with it (70 KiB of 81 when
+// the figures here were taken) against 22 - 27 without, more than the instruction cache holds, fetched anew at the end of every tile (and from memory when the kernel
 // starts on cold caches): same call, 8192^3 bf16 1425 -> 1457 TFLOP/s back to back and 1352 -> 1397 with flushed
 // caches, 4096^3 1201 -> 1301 and 1011 -> 1205.  Kernels take it as a separate instantiation, chosen on the host.
 // A lane holds 4 consecutive columns of a 16-column tile (8 bytes of C), so stores straight from the registers are 64
