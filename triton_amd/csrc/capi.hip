@@ -1336,6 +1336,23 @@ static bool attn_stride_ok(const int64_t* s, const void* ptr, int D) {
   return s[3] == 1 && s[2] >= D && s[2] < (1 << 24) && s[0] % 8 == 0 && s[1] % 8 == 0 && s[2] % 8 == 0 && aligned(ptr, 16);
 }
 
+// Steps of 64 keys that the busiest program of the causal persistent form walks: blocks of 256 rows dealt one after the other to
+// `programs`, whole rounds of heads long-to-short and short-to-long in turn (attn_fwd_stream_kernel).
+static int64_t stream_busiest(int64_t heads, int N, int programs) {
+  constexpr int kMost = 1024;
+  const int nb = (N + 255) / 256, G = (int)std::min<int64_t>(std::min(programs, kMost), heads * nb), per_round = std::max(1, G / nb);
+  int64_t steps[kMost] = {};
+  int at = 0;
+  for (int64_t h = 0; h < heads; h++) {
+    const bool up = ((h / per_round) & 1) != 0;
+    for (int j = 0; j < nb; j++) {
+      steps[at] += (std::min(N, ((up ? j : nb - 1 - j) + 1) * 256) + 63) / 64;
+      if (++at == G) at = 0;
+    }
+  }
+  return *std::max_element(steps, steps + G);
+}
+
 // Which form of the forward: the fewer query rows there are for the CUs, the smaller a workgroup's block of rows and the more
 // of its waves go along the keys instead (us, fp16, causal / not, by form: 2 = 256 rows, 4 = its persistent form, 1 = 128
 // rows, 8 = 128 rows x 2 groups, 6 = 64 x 2, 7 = 32 x 4).
@@ -1358,16 +1375,28 @@ static int attn_fwd_variant(const AttnArgs& p, int cus) {
     return p.D == 128 && p.N >= 4096 ? 8 : 2;
   }
   if (p.causal) {
-    // The persistent form deals pairs of a long and a short block of 256 rows, every pair the same work, in whole rounds of CUs: it is
-    // the fastest where the pairs fill those (128 x 1024 of head_dim 128, 256 pairs: 4 48, 1 58, 2 58, 8 64) and up to twice as
-    // long where they do not.  us, 8 / 1 / 2 / 4, head_dim 64: 15 x 4992 77 / 103 / 113 / 163, 24 x 2816 42 / 45 / 50 / 71, 75 x 1664 49 / 46
-    // / 49 / 82, 20 x 7680 213 / 219 / 226 / 330, 90 x 1152 34 / 33 / 28 / 39; head_dim 128: 20 x 3328 86 / 77 / 92 / 139, 27 x 3456 102 / 119 / 122 /
-    // 125, 36 x 5632 327 / 341 / 332 / 459, 105 x 2432 203 / 190 / 195 / 243, 100 x 3584 413 / 378 / 360 / 413.  (70 shapes: within 2 % of the
-    // best in the geometric mean, 12 % at most; the pairs everywhere 34 and 20 %, up to 2.1 times as long.)
-    const int64_t heads = (int64_t)p.Z * p.H, nb = (p.N + 255) / 256, pairs = heads * ((nb + 1) / 2);
-    const double dealt = (double)((pairs + cus - 1) / cus * (nb + 1)) * 65536.0 * cus, work = 0.5 * (double)heads * p.N * (p.N + 256.0);
-    if (dealt < 1.04 * work) return 4;
-    if (p.D == 64) return p.N <= 1280 ? 2 : 8;
+    // The persistent form is the fastest where its programs get the same work: `dealt`, the busiest program's share against an even one.
+    // us, 8 / 1 / 2 / 4, head_dim 64: 64 x 2048 (dealt 1.00) 62 / 67 / 64 / 51, 15 x 8192 (1.07) 205 / 208 / 240 / 173, 22 x 5888 (1.14) 143 / 154 / 149
+    // / 134, 102 x 1280 (1.17) 41 / 34 / 36 / 39, 15 x 4992 (3.2) 77 / 103 / 113 / 163; head_dim 128: 116 x 1024 (1.10) 67 / 56 / 59 / 50, 35 x 3584
+    // (1.32) 155 / 162 / 158 / 139, 48 x 2048 (1.33) 74 / 74 / 78 / 80, 44 x 1536 (3.0) 51 / 44 / 46 / 77.  With more than two rounds of blocks the
+    // other forms even out too: head_dim 64 176 x 1920 (1.23) 121 / 120 / 132 / 136, 128 512 x 768 (1.17) 176 / 126 / 130 / 134.  Below 1024
+    // (512) rows a head it is behind at an even deal as well: 512 x 512 44 / 38 / 37 / 41, head_dim 128 512 x 256 41 / 27 / 29 / 30.
+    // (518 shapes: within 1.9 % of the best form in the geometric mean; the four that are 3 - 5 % behind this one lie next to the bounds.)
+    const int64_t heads = (int64_t)p.Z * p.H;
+    if (p.N >= (p.D == 64 ? 1024 : 512)) {
+      const double work = 0.5 * (double)heads * p.N * (p.N + 256.0);
+      const double dealt = (double)stream_busiest(heads, p.N, cus) * 64 * 256 * cus / work;
+      const bool many = heads * ((p.N + 255) / 256) > 2ll * cus;
+      if (dealt < (p.D == 64 ? many ? 1.08 : 1.16 : many ? 1.16 : 1.33)) return 4;
+    }
+    // head_dim 64: 256 x 512 (whole rounds of blocks) 24 / 22 / 21 / 23, 110 x 768 22 / 19 / 23 / 30, 160 x 896 34 / 29 / 38 / 45, 72 x 1024 23 / 29 / 33 /
+    // 30, 92 x 1152 34 / 32 / 27 / 39, 24 x 2816 42 / 45 / 50 / 71; head_dim 128: 20 x
+    // 3328 86 / 77 / 92 / 139, 105 x 2432 203 / 190 / 195 / 243, 36 x 5632 327 / 341 / 332 / 459, 100 x 3584 413 / 378 / 360 / 413
+    if (p.D == 64) {
+      const int64_t blocks = heads * ((p.N + 255) / 256), rounds = (blocks + cus - 1) / cus;
+      if (p.N <= 1024) return p.N <= 768 && blocks * 100 > rounds * cus * 78 ? 2 : 1;
+      return p.N <= 1280 ? 2 : 8;
+    }
     return p.N <= 2600 ? 1 : rows < 560ll * cus ? 8 : 2;
   }
   return dflt;
