@@ -430,7 +430,8 @@ def test_calls_that_the_native_autograd_node_refuses_fail_as_before(gpu):
 
 
 @pytest.mark.parametrize("Z,H,N,D", [(3, 30, 1152, 64), (2, 12, 2816, 64), (5, 4, 3328, 128), (7, 15, 1152, 128), (6, 12, 2688, 128), (1, 32, 2304, 64),
-                                     (3, 24, 1024, 64), (4, 40, 896, 64), (7, 29, 512, 64), (2, 30, 2048, 64), (4, 29, 1024, 128), (6, 8, 2048, 128)])
+                                     (3, 24, 1024, 64), (4, 40, 896, 64), (7, 29, 512, 64), (2, 30, 2048, 64), (4, 29, 1024, 128), (6, 8, 2048, 128),
+                                     (4, 65, 1024, 64), (2, 65, 2048, 64), (3, 60, 768, 128)])
 def test_causal_blocks_that_do_not_fill_whole_rounds_of_cus(gpu, monkeypatch, Z, H, N, D):
     # shapes for every form that the rule takes where the dealt blocks leave CUs idle, and on either side of it, against those: P rounded to 16
     # bits against another running maximum, sums in another order (twice the type's unit of 2^-11 in the norm; seen 3e-4)

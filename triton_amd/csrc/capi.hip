@@ -1397,19 +1397,22 @@ static int attn_fwd_variant(const AttnArgs& p, int cus) {
     // (1.32) 155 / 162 / 158 / 139, 48 x 2048 (1.33) 74 / 74 / 78 / 80, 44 x 1536 (3.0) 51 / 44 / 46 / 77.  With more than two rounds of blocks the
     // other forms even out too: head_dim 64 176 x 1920 (1.23) 121 / 120 / 132 / 136, 128 512 x 768 (1.17) 176 / 126 / 130 / 134.  Below 1024
     // (512) rows a head it is behind at an even deal as well: 512 x 512 44 / 38 / 37 / 41, head_dim 128 512 x 256 41 / 27 / 29 / 30.
-    // (518 shapes: within 1.9 % of the best form in the geometric mean; the four that are 3 - 5 % behind this one lie next to the bounds.)
-    const int64_t heads = (int64_t)p.Z * p.H;
-    if (p.N >= (p.D == 64 ? 1024 : 512)) {
+    // It is no longer the fastest, however even the deal, of head_dim 64 from four rounds on (1024 x 1280 (1.07) 343 / 303 / 315 / 396, 661 x
+    // 1536 (1.07) 318 / 288 / 299 / 350, 256 x 2048 (1.00) 194 / 191 / 212 / 204, 128 x 4096 (1.00) 344 / 350 / 358 / 359) and of 128 for heads of three or five
+    // blocks (443 x 768 (1.16) 154 / 110 / 111 / 125, 727 x 1280 (1.10), 1 / 4, 8 % apart; 332 x 2048 (1.14) 525 / 438 / 473 / 431).
+    // (682 shapes of 512 .. 12288 rows and 1 to 20 rounds: within 2.6 % of the best form at head_dim 64, 0.7 % at 128, in the geometric mean.)
+    const int64_t heads = (int64_t)p.Z * p.H, nb = (p.N + 255) / 256, blocks = heads * nb;
+    const bool many = blocks > 2ll * cus, others = p.D == 64 ? blocks > 4ll * cus : many && (nb == 3 || nb == 5);
+    if (p.N >= (p.D == 64 ? 1024 : 512) && !others) {
       const double work = 0.5 * (double)heads * p.N * (p.N + 256.0);
       const double dealt = (double)stream_busiest(heads, p.N, cus) * 64 * 256 * cus / work;
-      const bool many = heads * ((p.N + 255) / 256) > 2ll * cus;
       if (dealt < (p.D == 64 ? many ? 1.08 : 1.16 : many ? 1.16 : 1.33)) return 4;
     }
     // head_dim 64: 256 x 512 (whole rounds of blocks) 24 / 22 / 21 / 23, 110 x 768 22 / 19 / 23 / 30, 160 x 896 34 / 29 / 38 / 45, 72 x 1024 23 / 29 / 33 /
     // 30, 92 x 1152 34 / 32 / 27 / 39, 24 x 2816 42 / 45 / 50 / 71; head_dim 128: 20 x
     // 3328 86 / 77 / 92 / 139, 105 x 2432 203 / 190 / 195 / 243, 36 x 5632 327 / 341 / 332 / 459, 100 x 3584 413 / 378 / 360 / 413
     if (p.D == 64) {
-      const int64_t blocks = heads * ((p.N + 255) / 256), rounds = (blocks + cus - 1) / cus;
+      const int64_t rounds = (blocks + cus - 1) / cus;
       if (p.N <= 1024) return p.N <= 768 && blocks * 100 > rounds * cus * 78 ? 2 : 1;
       return p.N <= 1280 ? 2 : 8;
     }
