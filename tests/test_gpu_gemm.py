@@ -1022,6 +1022,16 @@ def test_row_major_fp8_b_with_n_not_a_multiple_of_16_in_a_padded_pitch(gpu, fmt,
         assert got.shape == (M, N) and bits_equal(to_np(got), ref), bb.stride()
 
 
+@pytest.mark.parametrize("fmt,tdt", [("e4m3", torch.float8_e4m3fn), ("e5m2", torch.float8_e5m2)])
+@pytest.mark.parametrize("M,N,K", [(7, 1687, 721), (104, 2496, 776), (300, 130, 65), (300, 130, 63), (129, 260, 255), (257, 100, 257), (1, 204, 650)])
+def test_small_fp8_products_with_a_row_major_b_and_rows_of_odd_bytes_are_exact(gpu, fmt, tdt, M, N, K):
+    # either side of the sizes from which such operands are copied to rows that the tile kernels can load.  Whole numbers below 2^13
+    rng = np.random.default_rng(M + N + K)
+    a, b = rng.integers(-3, 4, size=(M, K)).astype(np.float32), rng.integers(-3, 4, size=(K, N)).astype(np.float32)
+    ta, tb = (torch.from_numpy(formats.encode_fp8(x, fmt)).to(gpu).view(tdt) for x in (a, b))
+    assert bits_equal(to_np(triton_amd.matmul(ta, tb, out_dtype=torch.float32)), a @ b)
+
+
 @pytest.mark.parametrize("case", ["bf16 row-major B", "fp16 K-major B", "fp8"])
 def test_k_not_a_multiple_of_16_bytes_takes_the_fast_kernels_through_zero_padding(gpu, case):
     # rows that are not 16-byte multiples cannot be loaded by the MFMA kernels; the wrapper appends the zeros that the

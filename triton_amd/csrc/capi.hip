@@ -839,14 +839,21 @@ GemmRoute gemm_route(const void* A, const void* B, int M, int N, int K, int64_t 
   const int steps = (int)(((int64_t)K * es + 127) / 128);
   const double ring = ring_ok(es, r.kmajor) ? ring_plan(M, N, steps, cus, 1, 1).us : 1e30;
   const long tiles256 = (long)((M + 255) / 256) * ((N + 255) / 256);
-  const double any = std::min(ring, tiles256_us(tiles256, 256, steps, cus, M < 256 || N < 256, es == 1));
+  // (fp8 next to a row-major B, which no ring kernel takes: the 128x128 kernel of one barrier per 64-byte step, and what its copies take
+  // beyond the 2 us below.  104 x 2496 x 776 e4m3 any-stride kernel / copies 39 / 14 us, 240 x 100 x 648 e5m2 18.5 / 13, 272 x 550 x 226 11.3 / 11;
+  // with less K the any-stride kernel stays: e5m2 198 x 707 x 154 9.1 / 11.4, 732 x 3038 x 54 9.3 / 14.5, e4m3 2303 x 674 x 49 10.2 / 13.2)
+  const long rounds128 = ((long)((M + 127) / 128) * ((N + 127) / 128) + cus - 1) / cus;
+  const bool one_barrier = !ring_ok(es, r.kmajor) && K >= (in_dtype == MI355_F8E4M3 ? 65 : 256);
+  const double other = one_barrier ? 5.3 + 0.34 * (double)rounds128 * ((K + 63) / 64) : ring;
+  const double any = std::min(other, tiles256_us(tiles256, 256, steps, cus, M < 256 || N < 256, es == 1));
   r.pack_a = !a_stays;
   // a row-major B with good rows only lacks the zero rows beyond K, which the ring kernels do not read
   r.pack_b = !b_stays || (!r.kmajor && K % vec != 0 && ring + copy_us(!a_stays, false) > any + copy_us(!a_stays, true));
   const double packed = copy_us(r.pack_a, r.pack_b) + (r.pack_b || r.kmajor || K % vec == 0 ? any : ring);
-  // (any-stride kernel: 64x64 tiles, about 1.3 us per 64 k: 1024 x 1024 x 1000 bf16 23 us, x 4100 107)
+  // (any-stride kernel: 64x64 tiles, about 1.3 us per 64 k: 1024 x 1024 x 1000 bf16 23 us, x 4100 107; e4m3, row-major B 2.8: 3 x 1442 x 2161 98)
   const long tiles = (long)((M + 63) / 64) * ((N + 63) / 64);
-  const double masked = kLaunchUs + (double)((tiles + cus - 1) / cus) * (1.0 + 1.3 * ((K + 63) / 64));
+  const double step64 = in_dtype == MI355_F8E4M3 && !r.kmajor && K > 64 ? 2.8 : 1.3;
+  const double masked = kLaunchUs + (double)((tiles + cus - 1) / cus) * (1.0 + step64 * ((K + 63) / 64));
   if (masked <= packed) {
     r.pack_a = r.pack_b = false;
     return r;
