@@ -1483,10 +1483,12 @@ def test_rows_too_far_apart_for_the_tile_kernels(gpu):
 
 
 @pytest.mark.parametrize("dtype", ["fp16", "bf16", "e4m3"])
-@pytest.mark.parametrize("M,N,K", [(2176, 2176, 64), (2176, 2176, 192), (2150, 2168, 40), (1664, 4100, 16), (1536, 1536, 128), (3456, 3584, 96)])
+@pytest.mark.parametrize("M,N,K", [(2176, 2176, 64), (2176, 2176, 192), (2150, 2168, 40), (1664, 4100, 16), (1536, 1536, 128), (3456, 3584, 96),
+                                   (4224, 1408, 128), (2432, 2440, 152), (1216, 7488, 128)])
 def test_short_k_on_two_128x128_tiles_per_cu(gpu, dtype, M, N, K):
     # more 128x128 tiles than CUs and at most 384 bytes of K, whole tiles from half as many on: the kernel of one barrier per 64-byte step;
-    # with an addend the ring kernels.  K of one chunk, of a step and a chunk, of whole steps; exact sums
+    # with an addend the ring kernels.  K of one chunk, of a step and a chunk, of whole steps; exact sums.  The last three have 16-bit results
+    # that four-wave kernels with tiles moved back could take, which one of them does
     rng = np.random.default_rng(M + K)
     a = rng.integers(-2, 3, size=(M, K)).astype(np.float32)
     b = rng.integers(-2, 3, size=(K, N)).astype(np.float32)
@@ -1500,6 +1502,7 @@ def test_short_k_on_two_128x128_tiles_per_cu(gpu, dtype, M, N, K):
     for tb in (put(b), put(b.T).t()):
         assert bits_equal(to_np(triton_amd.matmul(ta, tb, out_dtype=torch.float32)), ref), tb.stride()
         assert bits_equal(to_np(triton_amd.matmul(ta, tb, out_dtype=torch.float32, add=row)), ref + np.arange(N, dtype=np.float32)), tb.stride()
+        assert bits_equal(to_np(triton_amd.matmul(ta, tb, out_dtype=torch.float16)), ref), tb.stride()   # (whole numbers below 2^10)
 
 
 @pytest.mark.parametrize("kmajor", [False, True])

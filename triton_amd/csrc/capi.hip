@@ -466,7 +466,13 @@ PartChoice part_choice(const GemmArgs& p, const TileChoice& c, int es, bool b_km
   const int M = p.M, N = p.N, steps = (p.k_bytes + 127) / 128, tile = c.tile;
   const bool is8 = es == 1;
   PartChoice r{tile, -1, {M, N, 1e30}};
-  if (!by_knob && tile != 6 && !p.aux && p.c_vec_ok && short_k(M, N, p.k_bytes, b_kmajor, cus)) r.tile = 1;   // (its addends and odd rows of C cost more)
+  // (partial four-wave tiles pay for a prologue and edges over a short K: fp16 K-major 4224 x 1408 x 128 9.1 / 7.7 us, 6640 x 5448 x 144 40 / 37, e4m3 4240 x 4224 x
+  // 152 25.8 / 22; row-major B 7256 x 4688 x 192 37 / 32; not where 256-row tiles fill more than half of their one round: fp16 1216 x 7488 x 128 11.4 / 12.6, K-major
+  // 2464 x 5376 x 168 17.2 / 18.6, e4m3 4152 x 3212 x 320 15.6 / 18.7; nor with an activation: 3104 x 5456 x 152 23.2 / 28.8)
+  const long tiles256 = (long)((M + 255) / 256) * ((N + 255) / 256);
+  const bool partial = knobs().tile_m == UNSET && knobs().mixed_rows == UNSET && (M % (c.tile_m ? c.tile_m : 256) != 0 || N % 256 != 0) &&
+                       p.activation == MI355_ACT_NONE && (tiles256 > cus || tiles256 * 2 <= cus) && p.k_bytes <= (tiles256 > cus || !b_kmajor ? 384 : 320);
+  if (!by_knob && (tile != 6 || partial) && !p.aux && p.c_vec_ok && short_k(M, N, p.k_bytes, b_kmajor, cus)) r.tile = 1;   // (its addends and odd rows of C cost more)
   else if (tile == 1 && by_knob) r.ring = 0;
   else if (tile >= 8 && tile <= 10) r.ring = tile - 8;
   else if (tile == 12 && b_kmajor) r.ring = 3;
