@@ -1665,11 +1665,12 @@ def test_a_part_of_a_round_of_tiles_in_a_call_of_its_own(gpu, dtype, M, N, K):
         assert torch.equal(got, (want + row.float()).to(torch.bfloat16))
 
 
-@pytest.mark.parametrize("M,N,kbytes", [(17, 1000, 2064), (64, 8192, 2176), (33, 8161, 2304), (16, 8192, 4096), (16, 5760, 2176), (64, 8200, 2176), (24, 4096, 8192)])
+@pytest.mark.parametrize("M,N,kbytes", [(17, 1000, 2064), (64, 8192, 2176), (33, 8161, 2304), (16, 8192, 4096), (16, 5760, 2176), (64, 8200, 2176), (24, 4096, 8192),
+                                        (8, 7008, 8192), (9, 7008, 8192), (12, 6016, 8192), (13, 6016, 8192), (1, 7905, 8192)])
 @pytest.mark.parametrize("dtype", ["bf16", "e4m3"])
 def test_few_rows_next_to_a_k_major_weight_at_the_edges_of_their_tiles(gpu, dtype, M, N, kbytes):
     # sizes around the rule for the 64x32 ring tiles: the first K beyond it, a whole round of CUs and just beyond one, partial
-    # last tiles, 16 rows on either side of the streaming kernel, a K that other tiles split.  Sums of at most 2^13 products of -1 .. 1 are
+    # last tiles, 16 rows on either side of the streaming kernel, a K that other tiles split, up to eight (fp8: twelve) rows that stream.  Sums of at most 2^13 products of -1 .. 1 are
     # whole numbers below 2^24: exact in fp32, with the workspace and without.
     rng = np.random.default_rng(M + N)
     K = kbytes // (1 if dtype == "e4m3" else 2)
