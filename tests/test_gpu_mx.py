@@ -381,6 +381,22 @@ def test_ring_kernels_at_the_edges_of_their_ring_are_bit_exact(gpu, monkeypatch,
 
 
 @pytest.mark.parametrize("fmt", ["mxfp4", "mxfp8"])
+@pytest.mark.parametrize("M,N,K", [(1024, 5888, 128), (2050, 2564, 256), (3328, 2816, 128), (4096, 4096, 128), (4793, 2304, 384), (4793, 2300, 128), (5120, 4608, 512)])
+def test_few_k_steps_and_more_than_a_round_of_tiles_are_bit_exact(gpu, fmt, M, N, K):
+    # each kernel that the rule takes: 128x128 tiles of one barrier per step, eight waves with whole columns and partial rows (one and two rounds of
+    # programs), the ring for partial columns, MXFP8 of several rounds ahead of the four-wave kernel.  Exact sums
+    rng = np.random.default_rng(M + N + K)
+    if fmt == "mxfp4":
+        a, sa, b, sb = _operands(rng, M, N, K, fmt, lo=126, hi=129)
+    else:
+        a, b = (formats.encode_fp8(rng.integers(-2, 3, size=(rows, K)).astype(np.float32), "e4m3") for rows in (M, N))
+        sa, sb = (rng.integers(126, 129, size=(rows, K // 32)).astype(np.uint8) for rows in (M, N))
+    ref = mx.mx_matmul(a, sa, b, sb, fmt, out_dtype="fp32")
+    assert bits_equal(_run(gpu, a, sa, b, sb, fmt, torch.float32), ref)
+    assert bits_equal(_run(gpu, a, sa, b, sb, fmt, torch.bfloat16), formats.round_bf16(ref))
+
+
+@pytest.mark.parametrize("fmt", ["mxfp4", "mxfp8"])
 def test_less_workspace_than_a_split_wants_means_the_plain_call(gpu, fmt):
     # through the C ABI: no room, a byte less than asked for (left as it was), all of it, and a null pointer.  Exact sums
     lib, stream = _lib.load(), torch.cuda.current_stream().cuda_stream

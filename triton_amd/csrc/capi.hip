@@ -1246,6 +1246,20 @@ static int mx_impl(const uint8_t* A, const uint8_t* sA, const uint8_t* B, const 
       p.tile_m = 192;
     }
   }
+  // Few K steps and more than a round of tiles: the kernels without a ring's prologue, 128x128 tiles of one barrier per step below half a round of
+  // 256x256 tiles and the eight-wave kernel from there on where its columns are whole.  us, ring / these, MXFP4: 1024 x 5888 x 128 10.5 / 8.1, 4352 x 1600 x 256
+  // 11.4 / 9.2, 4608 x 3328 x 128 17.9 / 10.6, 4800 x 7168 x 128 36.4 / 23.2, 7680 x 7936 x 384 69 / 44; MXFP8 3608 x 1720 x 128 10.3 / 8.7, 2368 x 5376 x 128 17.3 / 11.8; partial
+  // columns: MXFP4 4608 x 3264 x 256 17.8 / 21.5, MXFP8 2240 x 4160 x 128 13.2 / 15.4; odd rows of C 5924 x 2670 x 128 21 / 67.  MXFP8 of several rounds ahead of the four-wave
+  // kernel too: 6144 x 6656 x 512 48.6 / 40.7, 5632 x 4608 x 256 28.4 / 24.7, not of one and a bit: 4608 x 4096 x 256 22 / 24.
+  bool few_steps = false;
+  if (knobs().tile == UNSET && knobs().tile_m == UNSET && knobs().mixed_rows == UNSET && K % 128 == 0 && p.c_vec_ok) {
+    if (tile == 1) few_steps = p.k_bytes <= 256 && (long)((M + 127) / 128) * ((N + 127) / 128) > cus;
+    else if (tile != 6) few_steps = p.k_bytes <= 192 && N % 256 == 0;
+    else if (fmt == MI355_MXFP8 && p.tile_m == 0 && p.k_bytes <= 512 && N % 256 == 0 && tiles256 * 5 > 7 * cus) {
+      few_steps = true;
+      tile = tiles256 % cus == 0 ? 5 : 4;
+    }
+  }
   p.num_programs = knob(knobs().programs, cus);
   // the ring kernels of 64 .. 128-row tiles, split along K where there is a workspace, where they are the faster ones by the
   // estimates of the other products (MXFP4 steps hold twice the elements in the same bytes, which are what bounds both).  us, the
@@ -1254,7 +1268,7 @@ static int mx_impl(const uint8_t* A, const uint8_t* sA, const uint8_t* B, const 
   // 18.6 / 15.1, MXFP8 31.5 / 23.7, 512 x 8192 x 8192 56 / 41; these stay ahead from about a round of their tiles on (2048 x 4096 x 4096
   // MXFP4 23.6 / 29.8, MXFP8 34 / 45)
   const bool ring_takes = K % 128 == 0 && lds_a % 4 == 0 && lds_b % 4 == 0 && aligned(sA, 4) && aligned(sB, 4) && lds_a < (1 << 24) && lds_b < (1 << 24);
-  if (ring_takes && knobs().tile_m == UNSET && knobs().mixed_rows == UNSET) {
+  if (ring_takes && !few_steps && knobs().tile_m == UNSET && knobs().mixed_rows == UNSET) {
     const int steps = (p.k_bytes + 127) / 128;
     int shape = -1, splits = 1;
     if (knobs().tile != UNSET) {
