@@ -278,10 +278,11 @@ bool streams(int M, int N, int64_t k_bytes, int elem_bytes, bool b_kmajor, int c
   const bool cols = M > 64;
   // (64x32 ring tiles: above 16 rows, and below from 70 % of a round of CUs on - 16 x 8192 x 8192 fp16 33.6 / 29.0, e4m3 13.7 / 13.2; 16 x
   // 4096 x 8192 e4m3 8.8 / 9.3)
-  // (but not up to eight rows, fp8 twelve, next to a weight of 44 MB (47) and more, which is memory's to bound: 1 x 6016 x 24832 fp16 33.1 / 28.1, 4 x 6144 x 10496 bf16
-  // 16.4 / 14.1, 8 x 7008 x 4096 17.1 / 13.0, 12 x 7424 x 7168 e5m2 13.1 / 10.9; now and then behind: 8 x 6656 x 8192 25.1 / 27.7; smaller ones 6.2 / 6.6.  fp8 to 9000 bytes of
-  // K: 4 x 6912 x 11520 13.9 / 14.6)
-  const bool far = elem_bytes == 2 ? M <= 8 && (double)N * k_bytes >= 44e6 : M <= 12 && (double)N * k_bytes >= 47e6 && k_bytes < 9000;
+  // (but not next to a weight of 44 MB (fp8: 47) and more, which is memory's to bound: 1 x 6016 x 24832 fp16 33.1 / 28.1, 4 x 6144 x 10496 bf16 16.4 / 14.1, 8 x
+  // 7008 x 4096 17.1 / 13.0, 12 x 7424 x 7168 e5m2 13.1 / 10.9; smaller ones 6.2 / 6.6; fp8 to 9000 bytes of K: 4 x 6912 x 11520 13.9 / 14.6.  More than eight (twelve) rows
+  // only up to 64 MiB: 16 x 7680 x 4096 fp16 18.3 / 14.5, x 6272 e5m2 12.5 / 10.8.  Now and then behind: 8 x 6656 x 8192 bf16 25.1 / 27.7; from cache 3 %)
+  const double weight = (double)N * k_bytes;
+  const bool far = (elem_bytes == 2 ? weight >= 44e6 : weight >= 47e6 && k_bytes < 9000) && (M <= (elem_bytes == 2 ? 8 : 12) || weight < 64.0 * (1 << 20));
   if (!cols && thin && thin_ok(M, N, k_bytes, b_kmajor, cus) && (M > 16 || ((N + 31) / 32 * 10 > cus * 7 && !far))) return false;
   const int S = cols ? N : M, L = cols ? M : N;
   const bool y_kmajor = cols || b_kmajor;
