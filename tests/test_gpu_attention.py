@@ -442,3 +442,33 @@ def test_causal_blocks_that_do_not_fill_whole_rounds_of_cus(gpu, monkeypatch, Z,
     want = triton_amd.attention(q, k, v, True, D ** -0.5).float()
     assert torch.isfinite(got).all() and (got - want).norm() <= 2 ** -10 * want.norm()
     assert (got - want).abs().max() <= 2 ** -7 * want.abs().max()
+
+
+@pytest.mark.parametrize("dtype", ["fp16", "e5m2"])
+@pytest.mark.parametrize("H,N,D", [(81, 512, 64),      # every head by length, heads that eight XCDs do not share evenly
+                                   (3, 11264, 64),     # fewer heads than XCDs
+                                   (27, 8192, 64),     # heads of an XCD one by one, then by length
+                                   (40, 896, 128),
+                                   (65, 512, 256)])    # (one block of 128 rows more than a round of CUs: dealt)
+def test_dealt_causal_blocks_are_every_block_once(gpu, monkeypatch, dtype, H, N, D):
+    # a head by itself has at most 256 blocks and is not dealt: the same kernel with the same bits, head by head
+    set_knob(monkeypatch, "MI355_ATTN_FWD_VARIANT", "1")
+    set_knob(monkeypatch, "MI355_ATTN_BWD_GROUPS", str(1 + 16))
+    g = torch.Generator(device=gpu).manual_seed(N)
+    q, k, v, do = (torch.randn(1, H, N, D, device=gpu, generator=g).half() for _ in range(4))
+    if dtype == "e5m2":
+        q, k, v = (t.to(torch.float8_e5m2) for t in (q, k, v))
+        v = v.view(torch.uint8).permute(0, 1, 3, 2).contiguous().permute(0, 1, 3, 2).view(torch.float8_e5m2)
+
+    def call(h):
+        ts = [t[:, h] for t in (q, k, v)]
+        if dtype == "e5m2":
+            return [triton_amd.attention(*ts, True, D ** -0.5).view(torch.uint8)]
+        ts = [t.contiguous().requires_grad_() for t in ts]
+        o = triton_amd.attention(*ts, True, D ** -0.5)
+        return [o, *torch.autograd.grad(o, ts, do[:, h].contiguous())]
+
+    whole = call(slice(0, H))
+    for h in range(H):
+        for a, b in zip(whole, call(slice(h, h + 1))):
+            assert torch.equal(a[:, h:h + 1], b), h

@@ -86,11 +86,9 @@ __global__ __launch_bounds__(NW * 64, 1) void attn_bwd_dq_kernel(AttnArgs p) {
   const int l32 = lane & 31, g = lane >> 5, i16 = lane & 15, q4 = lane >> 4;
 
   const int nqb = (p.N + BM - 1) / BM;
-  int pid = xcd_remap(blockIdx.x, nqb * p.Z * p.H);
-  const int hz = pid / nqb;
-  int qb = pid % nqb;
-  if (p.causal) qb = nqb - 1 - qb;
-  const int z = hz / p.H, h = hz % p.H;
+  int hz, z, h, qb;
+  attn_block(p, nqb, hz, z, h, qb);
+  if (p.causal) qb = nqb - 1 - qb;   // longest first
   const int kw = KW == 1 ? 0 : wave / QW;   // which of a step's KW blocks of keys (wave-uniform)
   const int m0 = qb * BM, row0 = m0 + (wave % QW) * QT * 32;
 
@@ -423,7 +421,7 @@ static int launch_dq(const AttnArgs& p, hipStream_t stream) {
     attr_set = true;
   }
   int nqb = (p.N + BM - 1) / BM;
-  attn_bwd_dq_kernel<V8, D, QT, NW, PAD, KW><<<dim3(nqb * p.Z * p.H), dim3(NW * 64), smem, stream>>>(p);
+  attn_bwd_dq_kernel<V8, D, QT, NW, PAD, KW><<<dim3(nqb * p.Z * p.H), dim3(NW * 64), smem, stream>>>(deal_blocks(p, nqb));
   return (int)hipGetLastError();
 }
 

@@ -96,10 +96,8 @@ __global__ __launch_bounds__(NW * 64, 1) void attn_bwd_dkdv_kernel(AttnArgs p) {
   const int l32 = lane & 31, g = lane >> 5, i16 = lane & 15, q4 = lane >> 4;
 
   const int nkb = (p.N + BN - 1) / BN;
-  int pid = xcd_remap(blockIdx.x, nkb * p.Z * p.H);
-  const int hz = pid / nkb;
-  const int kbk = pid % nkb;  // causal: low key blocks have the most work, ascending order = longest first
-  const int z = hz / p.H, h = hz % p.H;
+  int hz, z, h, kbk;   // (under the mask the low key blocks have the most work)
+  attn_block(p, nkb, hz, z, h, kbk);
   const int kw = KW == 1 ? 0 : wave / QW;   // which of a stage's tiles (wave-uniform)
   const int n0 = kbk * BN, nrow0 = n0 + (wave % QW) * 32;
 
@@ -648,7 +646,7 @@ static int launch_dkdv(const AttnArgs& p, hipStream_t stream) {
     attr_set = true;
   }
   int nkb = (p.N + BN - 1) / BN;
-  attn_bwd_dkdv_kernel<V8, D, NW, PAD, KW><<<dim3(nkb * p.Z * p.H), dim3(NW * 64), smem, stream>>>(p);
+  attn_bwd_dkdv_kernel<V8, D, NW, PAD, KW><<<dim3(nkb * p.Z * p.H), dim3(NW * 64), smem, stream>>>(deal_blocks(p, nkb));
   return (int)hipGetLastError();
 }
 

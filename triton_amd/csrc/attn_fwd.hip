@@ -69,11 +69,9 @@ __global__ __launch_bounds__(NW * 64, 1) void attn_fwd_kernel(AttnArgs p) {
   // block -> (head, query block): consecutive logical ids (same XCD) walk the query blocks of
   // one head; causal blocks in descending order of work
   const int nqb = (p.N + BM - 1) / BM;
-  int pid = xcd_remap(blockIdx.x, nqb * p.Z * p.H);
-  const int hz = pid / nqb;
-  int qb = pid % nqb;
-  if (p.causal) qb = nqb - 1 - qb;
-  const int z = hz / p.H, h = hz % p.H;
+  int hz, z, h, qb;
+  attn_block(p, nqb, hz, z, h, qb);
+  if (p.causal) qb = nqb - 1 - qb;   // longest first
   const int m0 = qb * BM;
   const int kw = wave / QW;                   // which of a step's KW blocks of keys (wave-uniform)
   const int row0 = m0 + (wave % QW) * QT * 32;  // first query row of this wave
@@ -713,7 +711,7 @@ static int launch_fwd(const AttnArgs& p, hipStream_t stream) {
     attr_set = true;
   }
   int nqb = (p.N + BM - 1) / BM;
-  attn_fwd_kernel<V8, D, QT, NW, PAD, KW><<<dim3(nqb * p.Z * p.H), dim3(NW * 64), smem, stream>>>(p);
+  attn_fwd_kernel<V8, D, QT, NW, PAD, KW><<<dim3(nqb * p.Z * p.H), dim3(NW * 64), smem, stream>>>(deal_blocks(p, nqb));
   return (int)hipGetLastError();
 }
 

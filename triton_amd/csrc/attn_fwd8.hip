@@ -54,11 +54,9 @@ __global__ __launch_bounds__(NW * 64, NW == 4 && D <= 128 ? 2 : 1) void attn_fwd
   const int l32 = lane & 31, g = lane >> 5;
 
   const int nqb = (p.N + BM - 1) / BM;
-  int pid = xcd_remap(blockIdx.x, nqb * p.Z * p.H);
-  const int hz = pid / nqb;
-  int qb = pid % nqb;
-  if (p.causal) qb = nqb - 1 - qb;
-  const int z = hz / p.H, h = hz % p.H;
+  int hz, z, h, qb;
+  attn_block(p, nqb, hz, z, h, qb);
+  if (p.causal) qb = nqb - 1 - qb;   // longest first
   const int m0 = qb * BM, row0 = m0 + wave * 32;
 
   const char* qbase = p.q + (int64_t)z * p.sq[0] + (int64_t)h * p.sq[1];
@@ -300,7 +298,7 @@ static int launch_fwd8(const AttnArgs& p, hipStream_t stream) {
     attr_set = true;
   }
   const int nqb = (p.N + BM - 1) / BM;
-  attn_fwd8_kernel<FMT, D, NW, PAD><<<dim3(nqb * p.Z * p.H), dim3(NW * 64), smem, stream>>>(p);
+  attn_fwd8_kernel<FMT, D, NW, PAD><<<dim3(nqb * p.Z * p.H), dim3(NW * 64), smem, stream>>>(deal_blocks(p, nqb));
   return (int)hipGetLastError();
 }
 

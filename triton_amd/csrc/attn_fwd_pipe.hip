@@ -232,11 +232,9 @@ __global__ __launch_bounds__(256, 1) void attn_fwd_pipe_kernel(AttnArgs p) {
   const int l32 = lane & 31, g = lane >> 5, i16 = lane & 15, q4 = lane >> 4;
 
   const int nqb = p.N / BM;
-  int pid = xcd_remap(blockIdx.x, nqb * p.Z * p.H);
-  const int hz = pid / nqb;
-  int qb = pid % nqb;
-  if (p.causal) qb = nqb - 1 - qb;       // longest first
-  const int z = hz / p.H, h = hz % p.H;
+  int hz, z, h, qb;
+  attn_block(p, nqb, hz, z, h, qb);
+  if (p.causal) qb = nqb - 1 - qb;   // longest first
   const int m0 = qb * BM;
   const int row0 = m0 + wave * 64;       // first query row of this wave
 
@@ -749,7 +747,7 @@ static int launch_fwd_pipe(const AttnArgs& p, hipStream_t stream) {
     attr_set = true;
   }
   const int nqb = p.N / BM;
-  attn_fwd_pipe_kernel<S, BF><<<dim3(nqb * p.Z * p.H), dim3(256), smem, stream>>>(p);
+  attn_fwd_pipe_kernel<S, BF><<<dim3(nqb * p.Z * p.H), dim3(256), smem, stream>>>(deal_blocks(p, nqb));
   return (int)hipGetLastError();
 }
 

@@ -13,6 +13,7 @@
 // half-sweep) select different 64-byte groups, so the 32 lanes cover all banks once.
 #pragma once
 #include "common.h"
+#include "launch.h"
 
 namespace mi355 {
 
@@ -61,6 +62,25 @@ struct AttnTile {
     return base + off(pitch, wave, lane, i);
   }
 };
+
+// This workgroup's head (z, h; hz = z * H + h) and block of rows among its `nblk`: `rank` counts from the longest where the
+// launch is dealt by length (deal_blocks).
+__device__ __forceinline__ void attn_block(const AttnArgs& p, int nblk, int& hz, int& z, int& h, int& rank) {
+  const int bid = blockIdx.x;
+  if (bid < p.head_blocks) {
+    hz = div_by(xcd_remap(bid, p.head_blocks), nblk, p.mul_blk, rank);
+  } else {
+    int i;
+    rank = div_by(bid - p.head_blocks, p.by_length, p.mul_len, i);
+    // block rank * by_length + i runs on XCD (..) % 8: turned by (rank * by_length) % 8, all but the last few heads of a rank stay on one
+    if (p.by_length >= 8) {
+      i += rank * p.by_length & 7;
+      if (i >= p.by_length) i -= p.by_length;
+    }
+    hz = p.Z * p.H - p.by_length + i;
+  }
+  z = div_by(hz, p.H, p.mul_h, h);
+}
 
 // Zero the `bytes` of LDS at `base` with all `nthreads` threads of the workgroup (padded tiles: the chunks that no
 // load ever writes must read as zeros); the caller synchronises afterwards.

@@ -1414,43 +1414,38 @@ static int attn_fwd_variant(const AttnArgs& p, int cus) {
   if (rows <= 64ll * cus) return 6;
   // 16 x 2048: 8 22.4 / 24.9, 6 24.0 / 27.0, 1 26.7 / 27.5; head_dim 128: 8 32.6 / 40.1, 6 32.2 / 50.6, 1 36.9 / 41.5
   // (two blocks of keys are not worth the groups' meeting: 256 x 128, no mask, head_dim 128: 8 10.2, 2 8.8; causal 8 ahead)
-  if (rows <= 128ll * cus && (p.causal || p.N > 128)) return 8;
-  if (p.causal && rows <= 256ll * cus) {
-    // (few, long rows of work under the mask) 32 x 2048: 6 34.1, 8 37.1, 2 38.4, 4 40.7; 8 x 8192: 6 102, 8 101, 4 142; 36 x 1152: 6
-    // 18.0, 8 19.6, 2 20.8; 27 x 1280: 6 18.1, 8 21.3, 2 24.6
-    if (p.D == 64 && p.N >= 1152) return 6;
-    // head_dim 128, 8 x 8192: 8 146, 1 173, 2 189, 4 197; 32 x 2048: 2 52.3, 8 56.2, 4 56.9; 128 x 512: 2 20.7, 4 23.2
-    return p.D == 128 && p.N >= 4096 ? 8 : 2;
+  if (!p.causal) return rows <= 128ll * cus && p.N > 128 ? 8 : dflt;
+  // Under the mask, with the blocks dealt by length (deal_blocks).  us, 6 / 8 / 1 / 2 / 4:
+  if (p.D == 64) {
+    // short rows: 48 x 640 9.4 / 10.3 / 11.1 / 12.6 / 14.6, 77 x 512 14.3 / 11.0 / 10.9 / 13.1 / 14.8, 256 x 512 26.6 / 21.9 / 18.9 / 19.1 / 22.7
+    if (p.N < 1024) return rows <= 128ll * cus ? 6 : 1;
+    // 14 x 2688 26.1 / 29.8 / 34.2 / 44.6 / 48.0, 24 x 2048 25.7 / 25.8 / 28.8 / 37.3 / 39.8, 25 x 2304 35.2 / 32.3 / 34.2 / 41.3 / 44.3
+    // 16 x 3200 35.4 / 37.0 / 40.9 / 53.3 / 57.0
+    if (rows <= (p.N >= 2560 ? 200ll : 192ll) * cus) return 6;
+    // 24 x 5632 145 / 127 / 136 / 148 / 239, 64 x 2048 57.1 / 48.0 / 49.4 / 52.8 / 51.8; 66 x 1024 24.0 / 21.6 / 21.4 / 23.1 / 30.0, 128 x 1024
+    // 37.2 / 29.3 / 28.4 / 29.8 / 32.1; 64 x 4096 199 / 170 / 177 / 161 / 180, 174 x 1152 66.1 / 52.5 / 48.6 / 51.0 / 66.6
+    if (p.N < 1536) return 1;
+    return rows <= 640ll * cus ? 8 : 2;
   }
-  if (p.causal) {
-    // The persistent form is the fastest where its programs get the same work: `dealt`, the busiest program's share against an even one.
-    // us, 8 / 1 / 2 / 4, head_dim 64: 64 x 2048 (dealt 1.00) 62 / 67 / 64 / 51, 15 x 8192 (1.07) 205 / 208 / 240 / 173, 22 x 5888 (1.14) 143 / 154 / 149
-    // / 134, 102 x 1280 (1.17) 41 / 34 / 36 / 39, 15 x 4992 (3.2) 77 / 103 / 113 / 163; head_dim 128: 116 x 1024 (1.10) 67 / 56 / 59 / 50, 35 x 3584
-    // (1.32) 155 / 162 / 158 / 139, 48 x 2048 (1.33) 74 / 74 / 78 / 80, 44 x 1536 (3.0) 51 / 44 / 46 / 77.  With more than two rounds of blocks the
-    // other forms even out too: head_dim 64 176 x 1920 (1.23) 121 / 120 / 132 / 136, 128 512 x 768 (1.17) 176 / 126 / 130 / 134.  Below 1024
-    // (512) rows a head it is behind at an even deal as well: 512 x 512 44 / 38 / 37 / 41, head_dim 128 512 x 256 41 / 27 / 29 / 30.
-    // It is no longer the fastest, however even the deal, of head_dim 64 from four rounds on (1024 x 1280 (1.07) 343 / 303 / 315 / 396, 661 x
-    // 1536 (1.07) 318 / 288 / 299 / 350, 256 x 2048 (1.00) 194 / 191 / 212 / 204, 128 x 4096 (1.00) 344 / 350 / 358 / 359) and of 128 for heads of three or five
-    // blocks (443 x 768 (1.16) 154 / 110 / 111 / 125, 727 x 1280 (1.10), 1 / 4, 8 % apart; 332 x 2048 (1.14) 525 / 438 / 473 / 431).
-    // (682 shapes of 512 .. 12288 rows and 1 to 20 rounds: within 2.6 % of the best form at head_dim 64, 0.7 % at 128, in the geometric mean.)
-    const int64_t heads = (int64_t)p.Z * p.H, nb = (p.N + 255) / 256, blocks = heads * nb;
-    const bool many = blocks > 2ll * cus, others = p.D == 64 ? blocks > 4ll * cus : many && (nb == 3 || nb == 5);
-    if (p.N >= (p.D == 64 ? 1024 : 512) && !others) {
-      const double work = 0.5 * (double)heads * p.N * (p.N + 256.0);
-      const double dealt = (double)stream_busiest(heads, p.N, cus) * 64 * 256 * cus / work;
-      if (dealt < (p.D == 64 ? many ? 1.08 : 1.16 : many ? 1.16 : 1.33)) return 4;
-    }
-    // head_dim 64: 256 x 512 (whole rounds of blocks) 24 / 22 / 21 / 23, 110 x 768 22 / 19 / 23 / 30, 160 x 896 34 / 29 / 38 / 45, 72 x 1024 23 / 29 / 33 /
-    // 30, 92 x 1152 34 / 32 / 27 / 39, 24 x 2816 42 / 45 / 50 / 71; head_dim 128: 20 x
-    // 3328 86 / 77 / 92 / 139, 105 x 2432 203 / 190 / 195 / 243, 36 x 5632 327 / 341 / 332 / 459, 100 x 3584 413 / 378 / 360 / 413
-    if (p.D == 64) {
-      const int64_t rounds = (blocks + cus - 1) / cus;
-      if (p.N <= 1024) return p.N <= 768 && blocks * 100 > rounds * cus * 78 ? 2 : 1;
-      return p.N <= 1280 ? 2 : 8;
-    }
-    return p.N <= 2600 ? 1 : rows < 560ll * cus ? 8 : 2;
+  // 24 x 896 15.4 / 17.1 / 18.8 / 21.6 / 24.8, 16 x 1536 20.7 / 24.4 / 28.4 / 36.8 / 40.8; 30 x 768 16.5 / 15.7 / 17.0 / 21.7 / 25.0
+  if (rows <= 96ll * cus && p.N >= 896) return 6;
+  // 76 x 384 15.0 / 11.6 / 11.3 / 11.5 / 14.4, 52 x 512 16.5 / 12.9 / 13.0 / 16.6 / 19.7, 51 x 640 23.2 / 15.6 / 16.8 / 17.1 / 20.2; 88 x 640 31.4 /
+  // 23.7 / 20.8 / 23.5 / 33.1, 256 x 256 29.2 / 20.6 / 14.8 / 15.7 / 17.5; one round of blocks of 256 rows, 105 x 384 24.7 / 19.4 / 15.0 / 13.1 / 15.3,
+  // 125 x 512 39.3 / 26.1 / 21.4 / 20.7 / 22.0
+  const int64_t heads = (int64_t)p.Z * p.H, nb = (p.N + 255) / 256, blocks = heads * nb, blocks128 = heads * ((p.N + 127) / 128);
+  if (p.N <= 640) return blocks128 <= cus ? (p.N >= 512 ? 8 : 1) : p.N > 256 && blocks <= cus ? 2 : 1;
+  // 32 x 2048 60.8 / 44.4 / 47.9 / 52.4 / 56.4, 10 x 4736 92.8 / 74.2 / 88.3 / 98.7 / 106
+  if (rows <= 256ll * cus) return 8;
+  // 16 x 5248 168 / 139 / 135 / 143 / 175, 30 x 2944 116 / 88.7 / 78.5 / 80.1 / 110; 20 x 5632 237 / 178 / 181 / 166 / 236, 39 x 2560 161 / 92 / 84 / 75 / 112
+  if (rows <= 360ll * cus) return 1;
+  // The persistent form where its programs get the same work (`dealt`: the busiest program's share against an even one) over
+  // many rounds: 256 x 1024 161 / 118 / 98.0 / 99.9 / 96.1, 128 x 4096 879 / 658 / 584 / 579 / 567; 64 x 4096 411 / 307 / 286 / 272 / 277
+  if (blocks >= 4ll * cus) {
+    const double work = 0.5 * (double)heads * p.N * (p.N + 256.0);
+    const double dealt = (double)stream_busiest(heads, p.N, cus) * 64 * 256 * cus / work;
+    if (dealt < 1.02) return 4;
   }
-  return dflt;
+  return 2;
 }
 
 int mi355_attn_fwd(const void* q, const void* k, const void* v, void* o, float* Mlse,
@@ -1516,16 +1511,17 @@ static int attn_bwd_variant(const AttnArgs& p, int cus) {
   if (p.D == 256 || p.d_real < p.D) return 1 + 16;
   const int64_t blocks = (int64_t)p.Z * p.H * p.N / 128;
   // head_dim 64, 8 heads x 1024: 34.4, two -5.4 / -5.8, four -6.6 / -7.5; 16 x 1024: 35.2, four -2.3 / -2.2
-  if (p.D == 64 && p.N % 256 == 0 && blocks <= cus / 4) return 4 + 64;
+  // (6 x 1536: two 29.7, four 25.6; 10 x 1536: 30.5, 35.1)
+  if (p.D == 64 && p.N % 256 == 0 && blocks <= (p.causal && p.N >= 1280 ? cus * 5 / 16 : cus / 4)) return 4 + 64;
   // 16 x 1024: two -5.7 / -5.8; head_dim 128: 51.7, -6.9 / -8.2; 24 x 1024: 52.2, +1.1 / +0.3 (full 57.1, +8.1 / +7.6)
   if (blocks <= cus / 2) return 2 + 32;
-  // 15 x 1280: 41.3, both -5.9; head_dim 128, 15 x 1152: 55.2, -4.8 (49 x 384: +2.3)
-  if (p.causal && p.N >= 1024 && blocks * 5 <= cus * 3ll) return 2 + 32;
-  if (!p.causal || p.N < 2048) return 1 + 16;
-  // 8 x 4096: 114.9, -13.9 / -15.3; head_dim 128: 177.6, -14.9 / -16.4; 12 x 4096: 224.8, +9.0 / +6.9; full, 8 x 4096: +13 / +13
-  if (blocks <= cus) return 2 + 32;
-  // head_dim 64, 48 x 2048: 144.9, -7.0 / -0.2; 16 x 4096: 171.3, -16.7 / +7.7; 48 x 1024: 54.4, -2.0 / -0.5
-  return p.D == 64 && blocks <= 3ll * cus ? 2 + 16 : 1 + 16;
+  // Under the mask (blocks dealt by length, deal_blocks) also where one round of CUs is nearly full, since half as many rows a
+  // block even out better: one / two groups in both, 24 x 768 29.4 / 22.3, 28 x 1024 36.2 / 33.8, 8 x 3968 108 / 80.2, 12 x 3328
+  // 96.4 / 85.3, 58 x 512 23.5 / 26.1, 19 x 2432 77.9 / 82.6; head_dim 128: 12 x 1664 73.8 / 53.9, 4 x 6528 248 / 175, 24 x 1152 58.4 /
+  // 55.6, 48 x 384 29.0 / 33.1, 12 x 3712 169 / 176
+  if (!p.causal) return 1 + 16;
+  if (p.N >= (p.D == 64 ? 768 : 1024) && blocks <= cus) return 2 + 32;
+  return p.D == 64 && p.N >= 2560 && blocks * 4 <= cus * 5ll ? 2 + 32 : 1 + 16;
 }
 
 static int attn_bwd(const void* q, const void* k, const void* v, const void* o, const void* d_o,

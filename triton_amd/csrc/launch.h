@@ -77,17 +77,57 @@ struct RowFusedArgs {
   const void* aux; int64_t aux_sm, aux_sn; int aux_dtype;   // addend as in GemmArgs
 };
 
+// n / d and what remains for 0 <= n < 2^31, with mul = (2^32 - 1) / d from the host: the product's high word is at most one short.
+__host__ __device__ inline int div_by(int n, int d, unsigned mul, int& remainder) {
+  int q = (int)(((uint64_t)(unsigned)n * mul) >> 32), r = n - q * d;
+  if (r >= d) { q++; r -= d; }
+  remainder = r;
+  return q;
+}
+
+// (256 bytes: two cache lines.  The arguments come from host memory at the start of every launch, a third line of them was
+// 0.2 us on launches of 6.)
 struct AttnArgs {
   const char* q; const char* k; const char* v; char* o; float* lse;
   const char* d_o; const float* delta; char* dq; char* dk; char* dv;
-  int Z, H, N, D;
-  int64_t sq[4], sk[4], sv[4], so[4];  // element strides
+  int Z, H, N;
   float sm_scale;
-  int causal;
-  int variant;  // tiling variant (tuning knob)
+  int64_t sq[4], sk[4], sv[4], so[4];  // element strides
   int num_programs;  // persistent forward: CUs to fill (0 = one workgroup per item)
-  int d_real;   // head dims 16 / 32: columns present in memory (D is then 64: the kernels pad with zeros on the fly)
+  int16_t causal;
+  int16_t variant;  // tiling variant (tuning knob)
+  int16_t D;
+  int16_t d_real;   // head dims 16 / 32: columns present in memory (D is then 64: the kernels pad with zeros on the fly)
+  // blocks of rows -> heads (attn_block of attn_tiles.h), set by deal_blocks
+  int head_blocks;  // blocks of the heads that go one by one
+  int by_length;    // heads behind them, dealt by length
+  unsigned mul_blk, mul_len, mul_h;   // (2^32 - 1) / a head's blocks, by_length, H
 };
+static_assert(sizeof(AttnArgs) <= 256, "two cache lines");
+
+// A launch of `nblk` blocks of rows for every head.  Under the mask the blocks of a head are of different lengths.  Most heads
+// still go one by one, each XCD through heads of its own, so that the blocks that run together share one head's rows in
+// their L2; the last ones go by length over all of them, the longest first, so that the launch ends with short blocks on
+// every CU and no XCD is left with more than another.  That part is four rounds of an XCD's 32 CUs and the heads that
+// eight XCDs do not share evenly.  us, forward and backward, heads in turn / the last two by length / four rounds / all:
+// bf16 10 x 6400 x 128 622 / 496 / 495 / 495 (a head and a quarter for each XCD in turn), fp16 24 x 3072 x 128 336 / 299
+// / 307 / 306, bf16 32 x 4096 x 64 378 / 377 / 347 / 347, 256 x 512 x 128 196 / 195 / 176 / 176, 128 x 4096 x 128 2366 /
+// 2356 / 2353 / 2420 (16 heads at a time in an XCD's L2).  Launches of one block a CU have nothing to even out and keep
+// their heads together (forward, 27 x 1024 x 128 19.1 / - / - / 20.7).
+inline AttnArgs deal_blocks(AttnArgs p, int nblk) {
+  const int64_t heads = (int64_t)p.Z * p.H, blocks = heads * nblk;
+  int64_t one_by_one = heads;
+  if (p.causal && blocks > 256) {
+    const int64_t tail = (128 + nblk - 1) / nblk;
+    one_by_one = heads / 8 > tail ? (heads / 8 - tail) * 8 : 0;
+  }
+  p.head_blocks = (int)(one_by_one * nblk);
+  p.by_length = (int)(heads - one_by_one);
+  p.mul_blk = 0xffffffffu / (unsigned)nblk;
+  p.mul_len = p.by_length > 0 ? 0xffffffffu / (unsigned)p.by_length : 0;
+  p.mul_h = 0xffffffffu / (unsigned)p.H;
+  return p;
+}
 
 // Device-side tables of a grouped GEMM (layout of python/tutorials/08-grouped-gemm.py:66-77).
 struct GroupedArgs {
