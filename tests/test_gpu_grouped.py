@@ -211,3 +211,46 @@ def test_matrices_of_other_libraries(gpu):
     want = [x.float() @ y.float() for x, y in zip(a, b)]
     for ga, gb in (([Foreign(a[0]), a[1]], [b[0], b[1]]), ([Foreign(x) for x in a], [Foreign(y) for y in b])):
         assert all(torch.equal(c.float(), w) for c, w in zip(triton_amd.group_gemm_fn(ga, gb), want))
+
+
+def test_groups_checked_in_native_code_are_the_python_function_s(gpu, monkeypatch):
+    # lists and tuples of plain tensors go past the Python function's checks: the same bits as through them, and everything else -
+    # modes, subclasses, refusals - is still the Python function's
+    from torch.overrides import TorchFunctionMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+    from triton_amd import _lib
+    g = torch.Generator(device=gpu).manual_seed(5)
+    shapes = [(33, 64, 40), (1, 8, 1), (256, 128, 512), (0, 16, 8), (5, 7, 0)]
+    a = [torch.randn(m, k, device=gpu, generator=g).half() for m, n, k in shapes]
+    b = [torch.randn(k, n, device=gpu, generator=g).half() for m, n, k in shapes]
+    ext = _lib.ext()
+    want = ext.group_gemm(a, b, 0)
+    for got in (triton_amd.group_gemm_fn(a, b), triton_amd.group_gemm_fn(tuple(a), tuple(b)), ext.group_gemm_plain(a, b, 0)):
+        assert isinstance(got, list) and all(torch.equal(x, y) and x.dtype == y.dtype and not x.requires_grad for x, y in zip(got, want))
+    with torch.inference_mode():
+        assert all(x.is_inference() for x in triton_amd.group_gemm_fn(a, b))
+
+    class Sub(torch.Tensor):
+        pass
+
+    refused = [([a[0].as_subclass(Sub)], [b[0]]), ([a[0]], [b[0].bfloat16()]), ([a[0]], [b[1]]), ([a[0].t()], [b[0].t()]), ([a[0].cpu()], [b[0]]),
+               ([a[0].float()], [b[0].float()]), ([a[0][0]], [b[0]]), ([None], [b[0]]), (a[:2], b[:1]), ([], []), (iter(a), iter(b))]
+    assert all(ext.group_gemm_plain(*r, 0) is None for r in refused)
+
+    class Functions(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    class Dispatch(TorchDispatchMode):
+        seen = 0
+
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            Dispatch.seen += 1
+            return func(*args, **(kwargs or {}))
+
+    for mode in (Functions(), Dispatch()):
+        with mode:
+            assert ext.group_gemm_plain(a, b, 0) is None
+    with Dispatch():
+        triton_amd.matmul(a[0], b[0])
+    assert Dispatch.seen > 0

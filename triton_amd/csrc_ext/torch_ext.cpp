@@ -7,6 +7,9 @@
 // becomes the exception the reference raises for the same condition (RuntimeError "Triton Error [HIP]"
 // for launch failures, :258-269; ValueError for pointers the device cannot reach, :313-317).
 #include <torch/extension.h>
+#include <torch/csrc/autograd/python_variable.h>
+#include <ATen/PythonTorchFunctionTLS.h>
+#include <ATen/hip/EmptyTensor.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
 
@@ -52,6 +55,20 @@ using DeviceGuard = c10::DeviceGuard;
 
 void* stream_of(const at::Tensor& t) { return (void*)c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
 
+// Whether nobody stands between a call and the device: no dispatch mode, functorch level or tracer is on.
+bool plain_dispatch() {
+  return (c10::impl::tls_local_dispatch_key_set().included_ - c10::default_included_set).empty();
+}
+
+// A result or workspace on the device of `like`.  Straight from the device's allocator where plain_dispatch(): the way through the
+// dispatcher is host time of its own for every tensor of calls whose kernels run for 4 us.
+at::Tensor fresh(at::IntArrayRef sizes, at::ScalarType type, const at::Tensor& like) {
+  if (plain_dispatch() && like.layout() == at::kStrided) return at::detail::empty_cuda(sizes, type, like.device(), c10::nullopt);
+  return at::empty(sizes, like.options().dtype(type));
+}
+
+at::Tensor fresh_like(const at::Tensor& t) { return t.is_contiguous() ? fresh(t.sizes(), t.scalar_type(), t) : at::empty_like(t); }
+
 const float* scale_ptr(const c10::optional<at::Tensor>& s) {
   if (!s.has_value()) return nullptr;
   TORCH_CHECK(s->scalar_type() == at::kFloat && s->numel() == 1, "scales are one fp32 value per tensor");
@@ -78,7 +95,7 @@ at::Tensor matmul(const at::Tensor& a, const at::Tensor& b_in, int64_t activatio
   on_device(a, 0); on_device(b, 1);
   const DeviceGuard guard(a.device());
   const int64_t M = a.size(0), K = a.size(1), N = b.size(1);
-  at::Tensor c = at::empty({M, N}, a.options().dtype(out_dtype.has_value() ? *out_dtype : in_dt == MI355_BF16 ? at::kBFloat16 : at::kHalf));
+  at::Tensor c = fresh({M, N}, out_dtype.has_value() ? *out_dtype : in_dt == MI355_BF16 ? at::kBFloat16 : at::kHalf, a);
   if (M == 0 || N == 0) return c;
   if (K == 0) return c.zero_();
   // fp32 operands run on the fp32 MFMAs with a K-major B only (the LDS transpose reads stop at 16-bit elements): a
@@ -98,7 +115,7 @@ at::Tensor matmul(const at::Tensor& a, const at::Tensor& b_in, int64_t activatio
   }
   const int64_t need = mi355_gemm_workspace(a.data_ptr(), b.data_ptr(), (int)M, (int)N, (int)K, a.stride(0), a.stride(1), b.stride(0), b.stride(1), in_dt);
   at::Tensor ws;
-  if (need > 0) ws = at::empty({need}, a.options().dtype(at::kByte));
+  if (need > 0) ws = fresh({need}, at::kByte, a);
   const int rc = mi355_gemm_ws(a.data_ptr(), b.data_ptr(), c.data_ptr(), (int)M, (int)N, (int)K, a.stride(0), a.stride(1), b.stride(0), b.stride(1),
                                c.stride(0), c.stride(1), in_dt, abi_dtype(c), scale_ptr(a_scale), scale_ptr(b_scale),
                                d, dsm, dsn, ddt, (int)activation, softmax ? 1 : 0, need > 0 ? ws.data_ptr() : nullptr, (size_t)need, stream_of(a));
@@ -112,7 +129,7 @@ void mx_gemm(const at::Tensor& a, const at::Tensor& sa, const at::Tensor& b, con
   const DeviceGuard guard(a.device());
   const int64_t need = mi355_mx_gemm_workspace((int)a.size(0), (int)b.size(0), (int)K, (int)fmt);
   at::Tensor ws;
-  if (need > 0) ws = at::empty({need}, c.options().dtype(at::kByte));
+  if (need > 0) ws = fresh({need}, at::kByte, c);
   const int rc = mi355_mx_gemm_ws((const uint8_t*)a.data_ptr(), (const uint8_t*)sa.data_ptr(), (const uint8_t*)b.data_ptr(),
                                   (const uint8_t*)sb.data_ptr(), c.data_ptr(), (int)a.size(0), (int)b.size(0), (int)K, (int)fmt,
                                   abi_dtype(c), a.stride(0), b.stride(0), sa.stride(0), sb.stride(0), c.stride(0),
@@ -134,7 +151,7 @@ std::vector<at::Tensor> group_gemm(const std::vector<at::Tensor>& a, const std::
   for (size_t i = 0; i < n; i++) {
     on_device(a[i], 2 * (int)i); on_device(b[i], 2 * (int)i + 1);
     TORCH_CHECK(a[i].dim() == 2 && b[i].dim() == 2, "grouped GEMM takes matrices");
-    c.push_back(at::empty({a[i].size(0), b[i].size(1)}, a[i].options()));
+    c.push_back(fresh({a[i].size(0), b[i].size(1)}, a[i].scalar_type(), a[i]));
     if (c[i].numel() == 0) continue;
     if (a[i].size(1) == 0) { c[i].zero_(); continue; }
     pa[used] = a[i].data_ptr(); pb[used] = b[i].data_ptr(); pc[used] = c[i].data_ptr();
@@ -150,6 +167,31 @@ std::vector<at::Tensor> group_gemm(const std::vector<at::Tensor>& a, const std::
   check(mi355_grouped_gemm_host(pa.data(), pb.data(), pc.data(), sizes.data(), lds.data(), (int)used, abi_dtype(a[0]), (int)num_programs,
                                 stream_of(a[0])), "mi355_grouped_gemm");
   return c;
+}
+
+// group_gemm of two lists or tuples of plain tensors that it takes: the checks of `group_gemm_fn` without a Python object for every
+// shape and stride (us, four products / thirteen of 18 .. 1306 rows: 11.6 / 27.3 with the checks in Python, 8.5 / 13.0).  None: a call that the
+// Python function looks at itself - other types, modes around it, whatever it refuses.
+py::object group_gemm_plain(const py::object& group_a, const py::object& group_b, int64_t num_programs) {
+  auto sequence = [](const py::object& o) { return PyList_CheckExact(o.ptr()) || PyTuple_CheckExact(o.ptr()); };
+  if (!sequence(group_a) || !sequence(group_b) || !plain_dispatch() || at::impl::torch_function_mode_enabled()) return py::none();
+  const Py_ssize_t n = PySequence_Fast_GET_SIZE(group_a.ptr());
+  if (n == 0 || PySequence_Fast_GET_SIZE(group_b.ptr()) != n) return py::none();
+  std::vector<at::Tensor> a, b;
+  a.reserve(n);
+  b.reserve(n);
+  for (Py_ssize_t i = 0; i < n; i++) {
+    PyObject *oa = PySequence_Fast_GET_ITEM(group_a.ptr(), i), *ob = PySequence_Fast_GET_ITEM(group_b.ptr(), i);
+    if (!THPVariable_CheckExact(oa) || !THPVariable_CheckExact(ob)) return py::none();
+    a.push_back(THPVariable_Unpack(oa));
+    b.push_back(THPVariable_Unpack(ob));
+    const at::Tensor &x = a[i], &y = b[i];
+    if (x.layout() != at::kStrided || y.layout() != at::kStrided || !x.is_cuda() || !y.is_cuda() || x.dim() != 2 || y.dim() != 2 ||
+        x.scalar_type() != a[0].scalar_type() || y.scalar_type() != a[0].scalar_type() || x.size(1) != y.size(0) || x.stride(1) != 1 || y.stride(1) != 1)
+      return py::none();
+  }
+  if (a[0].scalar_type() != at::kHalf && a[0].scalar_type() != at::kBFloat16) return py::none();
+  return py::cast(group_gemm(a, b, num_programs));
 }
 
 void strides4(const at::Tensor& t, int64_t (&s)[4]) {
@@ -199,7 +241,7 @@ void attn_bwd(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, con
 
 struct Attention : torch::autograd::Function<Attention> {
   static at::Tensor forward(torch::autograd::AutogradContext* ctx, const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, double sm_scale, bool causal) {
-    at::Tensor o = at::empty_like(q), M = at::empty({q.size(0), q.size(1), q.size(2)}, q.options().dtype(at::kFloat));
+    at::Tensor o = fresh_like(q), M = fresh({q.size(0), q.size(1), q.size(2)}, at::kFloat, q);
     attn_fwd(q, k, v, o, M, sm_scale, causal);
     ctx->save_for_backward({q, k, v, o, M});
     ctx->saved_data["sm_scale"] = sm_scale;
@@ -212,7 +254,7 @@ struct Attention : torch::autograd::Function<Attention> {
     if (!d_o.is_contiguous()) assertion("");
     if (q.strides() != k.strides() || q.strides() != v.strides() || q.strides() != o.strides() || q.strides() != d_o.strides()) assertion("");
     if (q.size(2) % 128 != 0) assertion("");
-    at::Tensor dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(v), delta = at::empty_like(M);
+    at::Tensor dq = fresh_like(q), dk = fresh_like(k), dv = fresh_like(v), delta = fresh_like(M);
     attn_bwd(q, k, v, o, d_o, M, delta, dq, dk, dv, ctx->saved_data["sm_scale"].toDouble(), ctx->saved_data["causal"].toBool());
     return {dq, dk, dv, at::Tensor(), at::Tensor()};
   }
@@ -226,7 +268,7 @@ c10::optional<at::Tensor> attention(const at::Tensor& q, const at::Tensor& k, co
   if ((type != at::kHalf && type != at::kBFloat16 && !is8) || k.size(3) != D || v.size(3) != D || (D != 16 && D != 32 && D != 64 && D != 128 && D != 256)) return c10::nullopt;
   if (is8 && (v.stride(2) != 1 || q.requires_grad() || k.requires_grad() || v.requires_grad())) return c10::nullopt;
   if (at::GradMode::is_enabled() && (q.requires_grad() || k.requires_grad() || v.requires_grad())) return Attention::apply(q, k, v, sm_scale, causal);
-  at::Tensor o = at::empty_like(q), M = at::empty({q.size(0), q.size(1), q.size(2)}, q.options().dtype(at::kFloat));
+  at::Tensor o = fresh_like(q), M = fresh({q.size(0), q.size(1), q.size(2)}, at::kFloat, q);
   attn_fwd(q, k, v, o, M, sm_scale, causal);
   return o;
 }
@@ -238,6 +280,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("matmul", &matmul);
   m.def("mx_gemm", &mx_gemm);
   m.def("group_gemm", &group_gemm);
+  m.def("group_gemm_plain", &group_gemm_plain);
   m.def("attn_fwd", &attn_fwd);
   m.def("attn_bwd", &attn_bwd);
   m.def("attention", &attention);

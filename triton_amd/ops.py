@@ -304,6 +304,11 @@ def group_gemm_fn(group_A, group_B, *, num_programs: int = 0):
     group_size = len(group_A)
     if group_size == 0:
         return []
+    ext = _lib.ext()
+    if ext is not None:
+        group_C = ext.group_gemm_plain(group_A, group_B, int(num_programs))   # (None: a call that the rest of this function looks at)
+        if group_C is not None:
+            return group_C
     dt = _abi_dtype(group_A[0])
     assert dt in (_lib.F16, _lib.BF16), "grouped GEMM takes fp16 or bf16 matrices"
     for i, (A, B) in enumerate(zip(group_A, group_B)):
@@ -312,7 +317,6 @@ def group_gemm_fn(group_A, group_B, *, num_programs: int = 0):
         assert A.shape[1] == B.shape[0]
         assert A.dtype == B.dtype == group_A[0].dtype, "all matrices of a group share one dtype"
         assert A.stride(1) == 1 and B.stride(1) == 1, "matrices must be row major"
-    ext = _lib.ext()
     if ext is not None:
         try:
             return ext.group_gemm(list(group_A), list(group_B), int(num_programs))
