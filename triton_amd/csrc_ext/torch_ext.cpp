@@ -67,7 +67,15 @@ at::Tensor fresh(at::IntArrayRef sizes, at::ScalarType type, const at::Tensor& l
   return at::empty(sizes, like.options().dtype(type));
 }
 
-at::Tensor fresh_like(const at::Tensor& t) { return t.is_contiguous() ? fresh(t.sizes(), t.scalar_type(), t) : at::empty_like(t); }
+// (a dimension of one element may have any stride in a contiguous tensor: the backward compares strides, so that these are kept too)
+at::Tensor fresh_like(const at::Tensor& t) {
+  int64_t dense = 1;
+  for (int64_t d = t.dim() - 1; d >= 0; d--) {
+    if (t.stride(d) != dense) return at::empty_like(t);
+    dense *= t.size(d);
+  }
+  return fresh(t.sizes(), t.scalar_type(), t);
+}
 
 const float* scale_ptr(const c10::optional<at::Tensor>& s) {
   if (!s.has_value()) return nullptr;
