@@ -1711,3 +1711,53 @@ def test_whoever_is_told_to_bring_a_workspace_finds_sums_in_it(gpu, dtype, kmajo
                                None, 0, 0, 0, _lib.ACT_NONE, 0, ws.data_ptr(), need, stream)
         assert rc == 0 and torch.equal(c, (a.float() @ b.float().t()).bfloat16()), (M, N, K)
         assert not ws[:need // 4].isnan().any() and ws[need // 4:].isnan().all(), (M, N, K, need)
+
+
+@pytest.mark.parametrize("tile", [None, 6, 8, 9, 10])
+@pytest.mark.parametrize("kmajor", [False, True])
+@pytest.mark.parametrize("M,N,K,pad,at", [
+    (300, 258, 130, 0, 0), (256, 256, 8, 0, 2), (129, 10, 70, 2, 0), (67, 8, 64, 2, 2), (257, 262, 192, 0, 4), (384, 266, 1028, 0, 0), (513, 500, 1090, 6, 2),
+    (260, 300, 4102, 0, 0), (40, 1002, 2054, 0, 2), (1030, 1030, 318, 2, 0), (64, 254, 62, 0, 0)])
+def test_rows_of_whole_dwords_are_read_in_place(gpu, monkeypatch, tile, kmajor, M, N, K, pad, at):
+    # rows that begin on dwords (pitch 2 mod 8 elements, bases 4 bytes off), a K and an N that end at every dword of a 16-byte chunk, tiles' edges, fewer
+    # than eight columns in a last tile, splits of K.  NaN between the rows and around the operands: what is read there must not count.  Whole numbers: exact
+    g = torch.Generator(device=gpu).manual_seed(M + N + K)
+
+    def operand(rows, cols):
+        pitch = cols + pad + cols % 2
+        room = torch.full((at + rows * pitch + 8,), float("nan"), device=gpu, dtype=torch.bfloat16)
+        x = room[at:at + rows * pitch].view(rows, pitch)[:, :cols]
+        return x.copy_(torch.randint(-1, 2, (rows, cols), device=gpu, generator=g))
+
+    a, b = operand(M, K), operand(N, K) if kmajor else operand(K, N)
+    bt = b.t() if kmajor else b
+    want = a.float() @ bt.float()
+    if tile is not None:
+        set_knob(monkeypatch, "MI355_GEMM_TILE", tile)
+    lib, stream = _lib.load(), torch.cuda.current_stream().cuda_stream
+    strides = (a.stride(0), 1, bt.stride(0), bt.stride(1))
+    need = lib.mi355_gemm_workspace(a.data_ptr(), b.data_ptr(), M, N, K, *strides, _lib.BF16)
+    ws = torch.full((need // 4 + 64,), float("nan"), device=gpu)
+    row = torch.randint(-8, 9, (N,), device=gpu, generator=g).to(torch.bfloat16)
+    for size in (0, need):
+        for add in (None, row):
+            c = torch.full((M, N), float("nan"), device=gpu)
+            rc = lib.mi355_gemm_ws(a.data_ptr(), b.data_ptr(), c.data_ptr(), M, N, K, *strides, N, 1, _lib.BF16, _lib.F32, None, None,
+                                   None if add is None else add.data_ptr(), 0, 1, _lib.BF16, _lib.ACT_NONE, 0, ws.data_ptr() if size else None, size, stream)
+            assert rc == 0 and torch.equal(c, want if add is None else want + row.float()), (size, add is None)
+    for splits, size in ((2, 0), (2, 8 * M * N)):   # (without room for the slices: the plain call)
+        ws = torch.full((2 * M * N,), float("nan"), device=gpu)
+        c = torch.full((M, N), float("nan"), device=gpu)
+        rc = lib.mi355_gemm_splitk(a.data_ptr(), b.data_ptr(), c.data_ptr(), M, N, K, *strides, N, 1, _lib.BF16, _lib.F32, None, None, _lib.ACT_NONE, splits,
+                                   ws.data_ptr() if size else None, size, stream)
+        assert rc == 0 and torch.equal(c, want), size
+
+
+@pytest.mark.parametrize("M,N,K", [(4095, 4100, 4100), (2050, 8192, 4098), (4100, 4098, 2050), (1025, 1027, 1030), (1024, 1030, 1027)])
+@pytest.mark.parametrize("kmajor", [False, True])
+def test_large_products_of_rows_on_dwords(gpu, M, N, K, kmajor):
+    # what the default does with them: one call or two (four columns in a call of their own), one operand copied where only its rows are odd
+    g = torch.Generator(device=gpu).manual_seed(M + N + K)
+    a, b = (torch.randint(-1, 2, shape, device=gpu, generator=g).to(torch.bfloat16) for shape in ((M, K), (N, K) if kmajor else (K, N)))
+    b = b.t() if kmajor else b
+    assert torch.equal(triton_amd.matmul(a, b, out_dtype=torch.float32), a.float() @ b.float())

@@ -498,6 +498,35 @@ PartChoice part_choice(const GemmArgs& p, const TileChoice& c, int es, bool b_km
 
 bool aligned(const void* p, size_t a) { return ((uintptr_t)p % a) == 0; }
 
+// 16-bit operands whose rows begin on dwords and are whole ones: what the ring and the four-wave kernels take where the rows are not whole
+// 16-byte chunks.  (Eight elements at least: the chunk that a row ends inside is read as the row's last 16 bytes.  `behind`: where those reach
+// in front of N columns of a row-major B there are others.)
+struct DwordRows { bool a, bk, bn; };
+DwordRows dword_rows(const void* A, const void* B, int M, int N, int K, int64_t sam, int64_t sak, int64_t sbk, int64_t sbn, int es, bool behind) {
+  if (es != 2) return {false, false, false};
+  const bool k = K % 2 == 0 && K >= 8;
+  return {k && sak == 1 && sam % 2 == 0 && sam >= K && aligned(A, 4), k && sbk == 1 && sbn % 2 == 0 && sbn >= K && aligned(B, 4),
+          sbn == 1 && ((sbk != 1 && sbk % 2 == 0 && N % 2 == 0 && (N >= 8 || behind) && sbk >= N && aligned(B, 4)) ||
+                       (sbk % 8 == 0 && sbk >= (N + 7) / 8 * 8 && aligned(B, 16)))};
+}
+
+// us of the any-stride kernel: 64x64 tiles, about 1.3 us per 64 k (1024 x 1024 x 1000 bf16 23 us, x 4100 107; e4m3, row-major B 2.8: 3 x 1442 x 2161 98)
+double any_stride_us(int M, int N, int K, int cus, double step64 = 1.3) {
+  const long tiles = (long)((M + 63) / 64) * ((N + 63) / 64);
+  return kLaunchUs + (double)((tiles + cus - 1) / cus) * (1.0 + step64 * ((K + 63) / 64));
+}
+
+// Whether a 16-bit product stays on that kernel whatever its operands' rows: K is a single step of it, and rows of C that are no whole groups
+// of four or an addend make the tile kernels' epilogues slow (see gemm_route), or its rounds are shorter.
+bool short_for_any_stride(int M, int N, int K, bool addend) { return K < 48 && (int64_t)M * N * K < 1 << 30 && (N % 4 != 0 || addend); }
+
+bool any_stride_ahead(int M, int N, int K, bool addend, int cus) {
+  if (short_for_any_stride(M, N, K, addend)) return true;
+  const int steps = (K + 63) / 64;
+  const double tiles = std::min(ring_plan(M, N, steps, cus, 1, 1).us, tiles256_us((long)((M + 255) / 256) * ((N + 255) / 256), 256, steps, cus, M < 256 || N < 256, false));
+  return any_stride_us(M, N, K, cus) <= tiles;
+}
+
 bool copy_strides(const int64_t* src, int64_t* dst) {
   if (!src) return false;
   for (int i = 0; i < 4; i++) dst[i] = src[i];
@@ -544,14 +573,15 @@ static int splitk_impl(const void* A, const void* B, void* C, int M, int N, int 
                        int64_t sam, int64_t sak, int64_t sbk, int64_t sbn, int64_t scm, int64_t scn,
                        int in_dtype, int out_dtype, const float* a_scale, const float* b_scale,
                        int activation, const void* aux, int64_t aux_sm, int64_t aux_sn, int aux_dtype,
-                       int splits, void* workspace, size_t workspace_bytes, void* stream_, int k_rows);
+                       int splits, void* workspace, size_t workspace_bytes, void* stream_, int k_rows, bool behind = false);
 
-// `workspace`: stream-K's.  `spare`: room for the slices of a second part that is split along K (see best_cut), or none.
+// `workspace`: stream-K's.  `spare`: room for the slices of a second part that is split along K (see best_cut), or none.  `behind`: eight columns of
+// B at least lie in front of these (see dword_rows).
 static int gemm_impl(const void* A, const void* B, void* C, int M, int N, int K,
                      int64_t sam, int64_t sak, int64_t sbk, int64_t sbn, int64_t scm, int64_t scn,
                      int in_dtype, int out_dtype, const float* a_scale, const float* b_scale,
                      int activation, const void* aux, int64_t aux_sm, int64_t aux_sn, int aux_dtype,
-                     int tile_arg, int group_m_arg, void* stream_, float* workspace = nullptr, int k_rows = 0, void* spare = nullptr, size_t spare_bytes = 0) {
+                     int tile_arg, int group_m_arg, void* stream_, float* workspace = nullptr, int k_rows = 0, void* spare = nullptr, size_t spare_bytes = 0, bool behind = false) {
   if (!A || !B || !C || M <= 0 || N <= 0 || K <= 0) return MI355_EINVAL;
   if (aux && aux_dtype != MI355_F16 && aux_dtype != MI355_BF16 && aux_dtype != MI355_F32) return MI355_EDTYPE;
   if (activation != MI355_ACT_NONE && activation != MI355_ACT_LEAKY_RELU) return MI355_EINVAL;
@@ -566,13 +596,18 @@ static int gemm_impl(const void* A, const void* B, void* C, int M, int N, int K,
 
   const bool out_ok = true;   // every output type of the ABI has a store in the MFMA epilogues (fp8: hardware conversion, saturating)
   const bool a_ok = sak == 1 && sam % vec == 0 && sam >= K && aligned(A, 16) && K % vec == 0;
-  const bool b_kmajor = sbk == 1 && sbn % vec == 0 && sbn >= K && aligned(B, 16);
+  const bool b_kmajor16 = sbk == 1 && sbn % vec == 0 && sbn >= K && aligned(B, 16);
   // (a row-major B: rows of whole 16-byte chunks - N itself need not be one: the last chunk of a row then reaches into
   // the padding that the pitch provides, and the columns beyond N are never stored)
   const bool b_nmajor = !is32 && sbn == 1 && sbk % vec == 0 && sbk >= (N + vec - 1) / vec * vec && aligned(B, 16);
+  // Rows of 16-bit elements that begin on dwords: the ring and the four-wave kernels' (`loose`), where no kernel of 16-byte chunks takes the operands
+  const bool chunks = a_ok && (b_kmajor16 || b_nmajor);
+  const DwordRows rows = dword_rows(A, B, M, N, K, sam, sak, sbk, sbn, es, behind);
+  const bool loose = !chunks && rows.a && (rows.bk || rows.bn) && (k_rows > 0 || !any_stride_ahead(M, N, K, aux != nullptr, device_info().cus > 0 ? device_info().cus : 256));
+  const bool b_kmajor = loose ? rows.bk : b_kmajor16;
   // the tile copies address 256 rows of an operand with 32-bit byte offsets from a 64-bit tile base
   const bool pitch_ok = (int64_t)sam * es < (1 << 23) && (b_kmajor ? (int64_t)sbn * es < (1 << 23) : (int64_t)sbk * es < (1 << 26));
-  const bool fast = pitch_ok && out_ok && a_ok && (b_kmajor || b_nmajor) && knob(knobs().force_strided, 0) == 0;
+  const bool fast = pitch_ok && out_ok && (chunks || loose) && knob(knobs().force_strided, 0) == 0;
 
   if (!fast && k_rows > 0) K = k_rows;   // (the kernels of any stride have no use for A's padding, and B ends before it)
   if (!fast && is32) {
@@ -630,7 +665,7 @@ static int gemm_impl(const void* A, const void* B, void* C, int M, int N, int K,
   const int ksteps128 = (p.k_bytes + 127) / 128;
   // at most 64 rows on one side: stream the other operand once (X = small side, Y = streamed side) where that is the faster
   // way, or where MI355_GEMM_SKINNY asks for it
-  if (skinny_allowed && k_rows == 0 &&
+  if (skinny_allowed && k_rows == 0 && !loose &&
       (knobs().skinny != UNSET || streams(M, N, p.k_bytes, es, b_kmajor, cus) || streams8(M, N, p.k_bytes, es, b_kmajor, cus))) {
     SkinnyArgs sk{};
     sk.K = K; sk.C = (char*)C; sk.a_scale = a_scale; sk.b_scale = b_scale;
@@ -672,11 +707,12 @@ static int gemm_impl(const void* A, const void* B, void* C, int M, int N, int K,
         const int splits = spare_bytes > 0 ? auto_splits(m2, n2, p.k_bytes, in_dtype, b_kmajor, true, cus) : 1;
         if (splits > 1 && (size_t)splits * m2 * n2 * 4 <= spare_bytes)
           return splitk_impl(A, B, C, m2, n2, K, sam, sak, sbk, sbn, scm, scn, in_dtype, out_dtype, a_scale, b_scale, activation,
-                             aux, aux_sm, aux_sn, aux_dtype, splits, spare, spare_bytes, stream_, 0);
+                             aux, aux_sm, aux_sn, aux_dtype, splits, spare, spare_bytes, stream_, 0, dn >= 8);
         return gemm_impl(A, B, C, m2, n2, K, sam, sak, sbk, sbn, scm, scn, in_dtype, out_dtype, a_scale, b_scale, activation,
-                         aux, aux_sm, aux_sn, aux_dtype, -1, group_m_arg, stream_);
+                         aux, aux_sm, aux_sn, aux_dtype, -1, group_m_arg, stream_, nullptr, 0, nullptr, 0, dn >= 8);
       }
     }
+    if (loose && ring < 0 && mixed_rows == 0 && !(tile == 6 && (p.tile_m != 0 || choice.w128_ok))) ring = ring_plan(M, N, ksteps128, cus, 1, 1).shape;
   }
   if (ring >= 0)
     return is8 ? gemm_ring8_launch(p, in_dtype == MI355_F8E5M2, ring, 1, 0, stream)
@@ -712,7 +748,7 @@ static int splitk_impl(const void* A, const void* B, void* C, int M, int N, int 
                        int64_t sam, int64_t sak, int64_t sbk, int64_t sbn, int64_t scm, int64_t scn,
                        int in_dtype, int out_dtype, const float* a_scale, const float* b_scale,
                        int activation, const void* aux, int64_t aux_sm, int64_t aux_sn, int aux_dtype,
-                       int splits, void* workspace, size_t workspace_bytes, void* stream_, int k_rows) {
+                       int splits, void* workspace, size_t workspace_bytes, void* stream_, int k_rows, bool behind) {
   if (!A || !B || !C || M <= 0 || N <= 0 || K <= 0 || splits < 0) return MI355_EINVAL;
   if (activation != MI355_ACT_NONE && activation != MI355_ACT_LEAKY_RELU) return MI355_EINVAL;
   if (in_dtype < MI355_F16 || in_dtype > MI355_F32) return MI355_EDTYPE;
@@ -721,9 +757,13 @@ static int splitk_impl(const void* A, const void* B, void* C, int M, int N, int 
   const int es = elem_size(in_dtype), vec = 16 / es;
   // what the tile kernels ask of the operands (as in mi355_gemm); anything else, or nothing to split: the plain call
   const bool a_ok = sak == 1 && sam % vec == 0 && sam >= K && aligned(A, 16) && K % vec == 0;
-  const bool b_kmajor = sbk == 1 && sbn % vec == 0 && sbn >= K && aligned(B, 16);
+  const bool b_kmajor16 = sbk == 1 && sbn % vec == 0 && sbn >= K && aligned(B, 16);
   const bool is32 = in_dtype == MI355_F32;   // (fp32 operands: the fp32 MFMAs, K-major B only)
   const bool b_nmajor = !is32 && sbn == 1 && sbk % vec == 0 && sbk >= (N + vec - 1) / vec * vec && aligned(B, 16);
+  const bool chunks = a_ok && (b_kmajor16 || b_nmajor);
+  const DwordRows rows = dword_rows(A, B, M, N, K, sam, sak, sbk, sbn, es, behind);
+  const bool loose = !chunks && rows.a && (rows.bk || rows.bn);
+  const bool b_kmajor = loose ? rows.bk : b_kmajor16;
   const bool pitch_ok = (int64_t)sam * es < (1 << 23) && (b_kmajor ? (int64_t)sbn * es < (1 << 23) : (int64_t)sbk * es < (1 << 26));
   const int64_t k_bytes = (int64_t)K * es;
   const bool ring = ring_ok(es, b_kmajor);
@@ -732,10 +772,12 @@ static int splitk_impl(const void* A, const void* B, void* C, int M, int N, int 
   if (splits == 0) splits = auto_splits(M, N, k_bytes, in_dtype, b_kmajor, ring, cus);
   const int per = splits >= 2 ? (ksteps + splits - 1) / splits : ksteps;
   const int used = (ksteps + per - 1) / per;   // (no split is left empty)
-  if (!(a_ok && (b_kmajor || b_nmajor) && pitch_ok) || used < 2 || knob(knobs().force_strided, 0) != 0)
+  // (dword rows need no room for slices to be taken: a call without it is the plain one)
+  const bool room = workspace && aligned(workspace, 16) && used >= 2 && workspace_bytes >= (size_t)used * M * N * sizeof(float);
+  if (!(pitch_ok && (chunks || (loose && room))) || used < 2 || knob(knobs().force_strided, 0) != 0)
     return gemm_impl(A, B, C, M, N, K, sam, sak, sbk, sbn, scm, scn, in_dtype, out_dtype, a_scale, b_scale, activation,
-                     aux, aux_sm, aux_sn, aux_dtype, -1, 0, stream_, nullptr, k_rows);
-  if (!workspace || !aligned(workspace, 16) || workspace_bytes < (size_t)used * M * N * sizeof(float)) return MI355_EINVAL;
+                     aux, aux_sm, aux_sn, aux_dtype, -1, 0, stream_, nullptr, k_rows, nullptr, 0, behind);
+  if (!room) return MI355_EINVAL;
   hipStream_t stream = (hipStream_t)stream_;
   GemmArgs p{};
   p.A = (const char*)A; p.B = (const char*)B; p.C = (char*)C;
@@ -841,10 +883,14 @@ GemmRoute gemm_route(const void* A, const void* B, int M, int N, int K, int64_t 
   // K is a single step of the any-stride kernel, and rows of C that are no whole groups of four or an addend make the tile kernels'
   // epilogues slow: the copies do not pay (us, that kernel / padded copies: 4024 x 5214 x 16 e4m3 49 / 78, 5246 x 2775 x 30 fp16 31 / 53, 520 x
   // 3873 x 32 8.7 / 11.6, 5164 x 2532 x 24 26 / 22 but 35 / 45 with an addend; whole groups of four: 5248 x 1792 x 28 e4m3 27 / 15)
-  if (K < 48 && (int64_t)M * N * K < 1 << 30 && (N % 4 != 0 || addend)) return r;
+  if (short_for_any_stride(M, N, K, addend)) return r;
   // (what stays in place has rows within the kernels' lane offsets, as in gemm_impl: only their kernels know k_rows)
   const int64_t a_most = 1 << 23, b_most = r.kmajor ? 1 << 23 : 1 << 26;
-  const bool a_stays = a_ok && sam * es < a_most, b_stays = r.kmajor ? bk_ok && sbn * es < b_most : bn_ok && sbk * es < b_most;
+  // (16-bit rows of whole dwords stay too, `loose`, but for what the rows between 128-byte lines cost the kernels where that is more than the copies do)
+  const DwordRows rows = dword_rows(A, B, M, N, K, sam, sak, sbk, sbn, es, false);
+  // (next to a row-major B of whole chunks A alone is copied, with K rounded up, which B's rows need not be)
+  const bool round_a = !r.kmajor && bn_ok && K % vec != 0;
+  const bool a_line = (a_ok || (rows.a && !round_a)) && sam * es < a_most, b_line = r.kmajor ? (bk_ok || rows.bk) && sbn * es < b_most : (bn_ok || rows.bn) && sbk * es < b_most;
   // us: the copies at about 4.5 TB/s of reads and writes, then the best kernel
   auto copy_us = [&](bool a, bool b) { return 2.0 + 2.0 * es * ((a ? (double)M * K : 0.0) + (b ? (double)N * K : 0.0)) / 4.5e6; };
   const int steps = (int)(((int64_t)K * es + 127) / 128);
@@ -857,19 +903,45 @@ GemmRoute gemm_route(const void* A, const void* B, int M, int N, int K, int64_t 
   const bool one_barrier = !ring_ok(es, r.kmajor) && K >= (in_dtype == MI355_F8E4M3 ? 65 : 256);
   const double other = one_barrier ? 5.3 + 0.34 * (double)rounds128 * ((K + 63) / 64) : ring;
   const double any = std::min(other, tiles256_us(tiles256, 256, steps, cus, M < 256 || N < 256, es == 1));
+  // What rows that do not begin on 128-byte lines add to a kernel's time, a line being fetched in two pieces, against the copies: 70 drawn products of
+  // such rows either way, and these in the probe of both, bf16, us, pitch a multiple of 128 bytes / 4 bytes more: 256x256 tiles, row-major B 4096^3 103 / 109, 8192^3
+  // 747 / 790, K-major 101 / 112, 721 / 830; ring tiles 1024^3 8.1 / 8.3, 2048^3 18.6 / 24.4, 1024 x 4096 x 4096 32 / 39.  Ring tiles: 0.4 of a step for each
+  // operand, so that a short K stays (copied / in place: 684 x 1113 x 1554 15.4 / 8.3, 2732 x 426 x 972 15.3 / 9.7, 1349 x 5067 x 276 26 / 21) and a long one is copied
+  // (1282 x 604 x 6798 31.2 / 34.3, 3246 x 818 x 4286 41.4 / 45.9).  256-row tiles: 0.08 of their time, K-major 0.11 (5506 x 7021 x 2926 219 / 242, 2472 x 4042 x 1030
+  // 40.1 / 36.3), and a K that is not whole pairs of steps runs on no others (1581 x 7168 x 5428 146 / 169).
+  const bool loose_a = a_line && !a_ok, loose_b = b_line && !(r.kmajor ? bk_ok : bn_ok);
+  bool loose = false;
+  if (loose_a || loose_b) {
+    const bool launch = !a_line || !b_line;   // (a copy is needed in any case)
+    const double copies = (launch ? 0.0 : 5.0) + 2.0 * es * ((loose_a ? (double)M * K : 0.0) + (loose_b ? (double)N * K : 0.0)) / 6.2e6;
+    double lines;
+    if (any == ring) {
+      const int s = auto_splits(M, N, (int64_t)K * es, in_dtype, r.kmajor, true, cus), shape = ring_plan(M, N, steps, cus, s, s).shape;
+      const int bm = shape == 2 ? 64 : 128, bn = shape == 0 ? 128 : 64;
+      const double rounds = std::max(1.0, (double)((M + bm - 1) / bm) * ((N + bn - 1) / bn) * s / cus);
+      lines = (loose_a + loose_b) * 0.4 * (shape == 0 ? 0.42 : shape == 1 ? 0.265 : 0.165) * ((steps + s - 1) / s) * rounds;
+    } else {
+      const double here = M >= 256 && N >= 256 ? std::min(any, best_cut(M, N, steps, cus, 6, -1, false).us) : any;
+      double other_rows = here;
+      if (K * es % 256 != 0)
+        for (int h : {192, 128}) other_rows = std::min(other_rows, tiles256_us((long)((M + h - 1) / h) * ((N + 255) / 256), h, steps, cus, false, false));
+      lines = (loose_a + loose_b) * (r.kmajor ? 0.11 : 0.08) * here + here - other_rows;
+    }
+    loose = lines <= copies;
+  }
+  const bool a_stays = a_line && (loose || !loose_a), b_stays = b_line && (loose || !loose_b);
   r.pack_a = !a_stays;
   // a row-major B with good rows only lacks the zero rows beyond K, which the ring kernels do not read
-  r.pack_b = !b_stays || (!r.kmajor && K % vec != 0 && ring + copy_us(!a_stays, false) > any + copy_us(!a_stays, true));
-  const double packed = copy_us(r.pack_a, r.pack_b) + (r.pack_b || r.kmajor || K % vec == 0 ? any : ring);
-  // (any-stride kernel: 64x64 tiles, about 1.3 us per 64 k: 1024 x 1024 x 1000 bf16 23 us, x 4100 107; e4m3, row-major B 2.8: 3 x 1442 x 2161 98)
-  const long tiles = (long)((M + 63) / 64) * ((N + 63) / 64);
-  const double step64 = in_dtype == MI355_F8E4M3 && !r.kmajor && K > 64 ? 2.8 : 1.3;
-  const double masked = kLaunchUs + (double)((tiles + cus - 1) / cus) * (1.0 + step64 * ((K + 63) / 64));
+  const bool even = es == 2 && K % 2 == 0 && K >= 8 && !round_a;   // (K as it is will do for dword rows, next to copies too)
+  const bool short_b = !r.kmajor && K % vec != 0 && !even;
+  r.pack_b = !b_stays || (short_b && ring + copy_us(!a_stays, false) > any + copy_us(!a_stays, true));
+  const double packed = (r.pack_a || r.pack_b ? copy_us(r.pack_a, r.pack_b) : 0.0) + (r.pack_b || !short_b ? any : ring);
+  const double masked = any_stride_us(M, N, K, cus, in_dtype == MI355_F8E4M3 && !r.kmajor && K > 64 ? 2.8 : 1.3);
   if (masked <= packed) {
     r.pack_a = r.pack_b = false;
     return r;
   }
-  if (K % vec != 0) {
+  if (K % vec != 0 && !(even && !(r.pack_a && r.pack_b))) {
     // (whole pairs of 128-byte K steps where there are several rounds of 256 x 256 tiles, whose kernel then walks them as one stream)
     const int to = tiles256 > cus && (int64_t)K * es >= 1024 ? 256 : 128;
     r.k = (int)up(K, r.pack_b || r.kmajor ? to / es : vec);

@@ -103,6 +103,11 @@ __device__ __forceinline__ void async_copy16_sbase_off(const void* sbase, unsign
 #endif
 }
 
+// The 16 bytes of v moved down by s bytes (0 .. 15, the same for the whole wave), zeros behind them.
+__device__ __forceinline__ i32x4 bytes_down(i32x4 v, int s) {
+  return __builtin_bit_cast(i32x4, __builtin_bit_cast(unsigned __int128, v) >> (8 * s));
+}
+
 // A touch of one dword per lane, lanes 0 .. NLANES-1 only, at (wave-uniform 64-bit base + 32-bit lane offset),
 // landing in 256 bytes of LDS that nobody reads: brings those lanes' cache lines into the L2 ahead of the loads that
 // want them.  Counts in vmcnt like any load; sets M0 like the copies above (SETM0) or uses the value a preceding

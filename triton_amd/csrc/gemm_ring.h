@@ -250,8 +250,10 @@ template <typename E, int BM, int BN>
 constexpr int ring_stage_bytes() { return (BM + BN) * (RING_ROW + 4 * E::kScaleDwords); }
 
 // Tile (pm, pn) of the product p with the ring of NS stages at LDS address lds0 (NS * (BM + BN) * 128 bytes).  A has whole
-// 16-byte chunks along K (k_bytes of them) and a K-major B too; a row-major B (16-bit types) has rows of whole 16-byte chunks,
-// p.K of them: in the last chunk's place of A's rows there may be zeros beyond K.  Block-scaled: both operands K-major, K a
+// 16-byte chunks along K (k_bytes in all) and a K-major B too; a row-major B (16-bit types) has p.K rows of whole 16-byte chunks: in
+// the last chunk's place of A's rows there may be zeros beyond K.  16-bit types: dwords instead of chunks will do (8 elements at least),
+// for the rows' begin as for their length - a direct load moves 16 bytes from any dword on, as fast as from rows of 16-byte but not 128-byte
+// pitch (bf16 2048^3, rows of 2048 / 2056 / 2050 elements 18.6 / 24.5 / 24.4 us, 1024^3 8.1 / 8.2 / 8.3).  Block-scaled: both operands K-major, K a
 // multiple of 128 elements, scale rows that begin on dwords.  Every wave's
 // fragments are in registers when the last step's MFMAs begin, so a caller that runs another tile needs one barrier first.
 template <typename E, int BM, int BN, int WN, bool B_KMAJOR, int NS>
@@ -275,8 +277,10 @@ __device__ __forceinline__ void gemm_ring_tile(const GemmArgs& p, const int pm, 
   const int wm = wave / WN, wn = wave % WN;
   const int m0 = pm * BM, n0 = pn * BN;
   // (a step that a row-major B ends inside is a tail too, a whole one where A's padding fills it: B has no rows to load there)
+  // (and so is one that holds the last row of a row-major B whose rows end inside a chunk: nothing may be read behind that row)
   const int rest = p.k_bytes % RING_ROW;
-  const int tail = !B_KMAJOR && rest == 0 && p.K * E::kElemBytes < p.k_bytes ? RING_ROW : rest;
+  const bool open_rows = !B_KMAJOR && p.N % 8 != 0 && ((p.ldb | (int64_t)(uintptr_t)p.B) & 15) != 0;
+  const int tail = !B_KMAJOR && rest == 0 && (open_rows || p.K * E::kElemBytes < p.k_bytes) ? RING_ROW : rest;
   const int steps = (p.k_bytes + RING_ROW - 1) / RING_ROW;
   constexpr int KROWS = RING_ROW / 2;                        // k rows of a row-major B per step
 
@@ -449,6 +453,16 @@ __device__ __forceinline__ void gemm_ring_tile(const GemmArgs& p, const int pm, 
     i32x4 ta[LA], tb[LB];
     const int kfull = p.k_bytes - tail;                       // bytes of K before the tail
     const int krows = p.K - kfull / E::kElemBytes;            // (a row-major B may end before the padded rows of A do)
+    // The chunk that a row ends inside is read as the row's last 16 bytes and moved down: of K-contiguous rows at k_bytes, of rows of a
+    // row-major B at N (past_row: bytes that the lane's chunk of load q reaches beyond).
+    auto cut_chunk = [&](i32x4 v, int chunk) { return MX || E::kElemBytes != 2 || chunk * 16 + 16 <= tail ? v : bytes_down(v, -tail & 15); };
+    auto past_row = [&](int q) {
+      if (!open_rows) return 0;
+      constexpr int CPR = BN / 8, RPI = 64 / CPR;
+      const int pc = lane % CPR, k = (wave * LB + q) * RPI + lane / CPR;
+      const int chunk = min((((pc >> 1) ^ xor_of(k)) << 1) | (pc & 1), (p.N + 7) / 8 - 1 - n0 / 8);
+      return max(0, (n0 + chunk * 8 + 8 - p.N) * 2);
+    };
     const char* kA = tileA + kfull;
     const char* kB = B_KMAJOR ? tileB + kfull : tileB + (int64_t)(kfull / 2) * p.ldb;
 #pragma unroll
@@ -456,7 +470,7 @@ __device__ __forceinline__ void gemm_ring_tile(const GemmArgs& p, const int pm, 
 #pragma unroll
     for (int q = 0; q < LB; q++) {
       if constexpr (B_KMAJOR) load16_sbase<0>(tb[q], kB, voffB[q] + q * 1024 - rowB[q] * 16 + min(rowB[q] * 16, tail - 16));
-      else load16_sbase<0>(tb[q], kB, voffB[q] + q * 1024 - (unsigned)(rowB[q] - min(rowB[q], krows - 1)) * (unsigned)p.ldb);
+      else load16_sbase<0>(tb[q], kB, voffB[q] + q * 1024 - (unsigned)(rowB[q] - min(rowB[q], krows - 1)) * (unsigned)p.ldb - (unsigned)past_row(q));
     }
     int ts = 0;   // (block-scaled: K is a multiple of 128 elements, so an MXFP4 tail is four blocks - one dword of scales - and there is no other)
     const int bs = wave % BLOCKS;
@@ -466,12 +480,14 @@ __device__ __forceinline__ void gemm_ring_tile(const GemmArgs& p, const int pm, 
 #pragma unroll
     for (int q = 0; q < LA; q++) {
       lds_use(ta[q]);
-      *(LDS_PTR(i32x4))(uintptr_t)(lds0 + (wave * LA + q) * 1024 + lane * 16) = chunkA[q] * 16 < tail ? ta[q] : zero;
+      *(LDS_PTR(i32x4))(uintptr_t)(lds0 + (wave * LA + q) * 1024 + lane * 16) = chunkA[q] * 16 < tail ? cut_chunk(ta[q], chunkA[q]) : zero;
     }
 #pragma unroll
     for (int q = 0; q < LB; q++) {
       lds_use(tb[q]);
       const bool in = B_KMAJOR ? rowB[q] * 16 < tail : rowB[q] < krows;
+      if constexpr (B_KMAJOR) tb[q] = cut_chunk(tb[q], rowB[q]);
+      else if (past_row(q) > 0) tb[q] = bytes_down(tb[q], -2 * p.N & 15);
       *(LDS_PTR(i32x4))(uintptr_t)(lds0 + A_BYTES + (wave * LB + q) * 1024 + lane * 16) = in ? tb[q] : zero;
     }
     if constexpr (MX) {

@@ -63,18 +63,22 @@ __device__ __forceinline__ int head_chunk(int q, int lane) {
   const int s = (lane & 7) ^ (((q & 1) * 4 + (lane >> 4)) & 7);
   return PERM ? 2 * (s & 3) + (s >> 2) : s;
 }
+// BYTES: `rest` need not be whole chunks.  The chunk that a row ends inside is read as the row's last 16 bytes and moved down, so
+// that nothing behind the row is read (the rows have 16 bytes at least).
 template <int L, bool PERM = false>
 __device__ __forceinline__ void head_load(i32x4 (&t)[L], const char* src, unsigned pitch, int lane, int rest) {
-#pragma unroll
-  for (int q = 0; q < L; q++) load16_sbase<0>(t[q], src, ((lane >> 3) + 8 * q) * pitch + min(head_chunk<PERM>(q, lane) * 16, rest - 16));
+#pragma unroll   // (16 taken off the base: no lane offset is negative)
+  for (int q = 0; q < L; q++) load16_sbase<0>(t[q], src - 16, ((lane >> 3) + 8 * q) * pitch + min(head_chunk<PERM>(q, lane) * 16 + 16, rest));
 }
-template <int L, bool PERM = false>
+template <int L, bool PERM = false, bool BYTES = false>
 __device__ __forceinline__ void head_store(i32x4 (&t)[L], unsigned dst, int lane, int rest) {
   const i32x4 zero = {0, 0, 0, 0};
 #pragma unroll
   for (int q = 0; q < L; q++) {
+    const int at = head_chunk<PERM>(q, lane) * 16;
     lds_use(t[q]);
-    *(LDS_PTR(i32x4))(uintptr_t)(dst + q * 1024 + lane * 16) = head_chunk<PERM>(q, lane) * 16 < rest ? t[q] : zero;
+    const i32x4 whole = !BYTES || at + 16 <= rest ? t[q] : bytes_down(t[q], -rest & 15);
+    *(LDS_PTR(i32x4))(uintptr_t)(dst + q * 1024 + lane * 16) = at < rest ? whole : zero;
   }
 }
 

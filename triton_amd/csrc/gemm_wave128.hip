@@ -44,7 +44,7 @@ __device__ __forceinline__ void mfma16(f16x8 a, f16x8 b, f32x4& c) {
 // with the 128 KiB of LDS at `lds0`.  XCD: pass the tile numbers through the per-XCD remap first.  EPI: 0 = every
 // epilogue of the C ABI; 1 = C has the type of the operands, no scales, no activation; 2 = C in a 16-bit type with a bias row
 // at most (rows_epilogue), any N; 3 = the lean epilogue (gemm_epilogue16_lean) with C in the operands' type.
-// ANYK: any K of whole 16-byte chunks, one tile (see head_load).  (The reference's own uneven-K shape: 8192 x 8192 x 8176,
+// ANYK: any K of whole dwords, one tile (see head_load).  (The reference's own uneven-K shape: 8192 x 8192 x 8176,
 // python/test/regression/test_performance.py:46.)
 template <typename V8, bool B_KMAJOR, bool XCD, int EPI = 0, bool ANYK = false, int BM = 256>
 __device__ __forceinline__ void gemm_wave128_tiles(const GemmArgs& p, int tile, const int tile_step, const unsigned lds0, const int tile_stop = -1) {
@@ -65,13 +65,13 @@ __device__ __forceinline__ void gemm_wave128_tiles(const GemmArgs& p, int tile, 
 
   // Sizes that are no whole tiles: the last tile of a row or column ends where the matrix does and covers part of its
   // neighbour once more (the same sums in the same order: both write the same bits), so that no load and no row needs a
-  // bound.  A row-major B is fetched in 16-byte chunks: there the last tile begins at one, and the epilogue leaves out the
+  // bound.  Where the rows of a row-major B begin on 16 bytes the last tile begins at such a chunk, and the epilogue leaves out the
   // up to seven columns of padding that it then ends in.
   // (Edges ran the eight-wave kernel, with bounds on every load and an epilogue of single elements, us: 3001 x 5003 x 1024 bf16
   // with a bias row 83 -> 39, 6420 x 6701 x 844 240 -> 106, 3738 x 7135 x 455 fp16 112 -> 61, 4095 x 4100 x 4100 bf16 162 -> 140;
   // a bias row on whole tiles, 4096^3 fp16 129 -> 108, is the epilogue alone.)
   const int num_m = (p.M + BM - 1) / BM, num_n = (p.N + BN - 1) / BN;
-  const int last_m0 = p.M - BM, last_n0 = (B_KMAJOR ? p.N : (p.N + 7) & ~7) - BN;
+  const int last_m0 = p.M - BM, last_n0 = (B_KMAJOR || ((p.ldb | (int64_t)(uintptr_t)p.B) & 15) ? p.N : (p.N + 7) & ~7) - BN;
   const int ntiles = num_m * num_n;
   const int tend = tile_stop < 0 ? ntiles : tile_stop;   // the walk ends before this tile
   // The tiles are computed as ONE stream of K steps: the loads of the last two steps of a tile already
@@ -258,9 +258,9 @@ __device__ __forceinline__ void gemm_wave128_tiles(const GemmArgs& p, int tile, 
     fB -= kstepB;
     if constexpr (PF) { pA -= ROWB; pB -= kstepB; }
     second_stage();
-    head_store(ta, lds0 + wave * (LA * 1024), lane, head);
+    head_store<LA, false, true>(ta, lds0 + wave * (LA * 1024), lane, head);
     if constexpr (B_KMAJOR) {
-      head_store(tb, lds0 + A_BYTES + wave * 8192, lane, head);
+      head_store<8, false, true>(tb, lds0 + A_BYTES + wave * 8192, lane, head);
     } else {
       const i32x4 zero = {0, 0, 0, 0};
 #pragma unroll
@@ -899,8 +899,8 @@ bool gemm_wave128_f8_192_ok(const GemmArgs& p, bool b_kmajor, int tile_m) {
 }
 
 bool gemm_wave128_ok(const GemmArgs& p, bool b_kmajor) {
-  // a whole tile at least, a pair of 128-byte K steps, 32-bit lane offsets
-  if (!(p.M >= 256 && p.N >= 256 && p.k_bytes % 16 == 0 && p.k_bytes >= 256)) return false;
+  // a whole tile at least, a pair of 128-byte K steps, rows of whole dwords, 32-bit lane offsets
+  if (!(p.M >= 256 && p.N >= 256 && p.k_bytes % 4 == 0 && p.k_bytes >= 256)) return false;
   if (p.lda * 8 + p.k_bytes >= (1ll << 31)) return false;
   return b_kmajor ? p.ldb * 8 + p.k_bytes < (1ll << 31) : (int64_t)p.K * p.ldb + 512 < (1ll << 31);
 }
