@@ -1713,7 +1713,7 @@ def test_whoever_is_told_to_bring_a_workspace_finds_sums_in_it(gpu, dtype, kmajo
         assert not ws[:need // 4].isnan().any() and ws[need // 4:].isnan().all(), (M, N, K, need)
 
 
-@pytest.mark.parametrize("tile", [None, 6, 8, 9, 10])
+@pytest.mark.parametrize("tile", [None, 6, 8, 9, 10, 13])
 @pytest.mark.parametrize("kmajor", [False, True])
 @pytest.mark.parametrize("M,N,K,pad,at", [
     (300, 258, 130, 0, 0), (256, 256, 8, 0, 2), (129, 10, 70, 2, 0), (67, 8, 64, 2, 2), (257, 262, 192, 0, 4), (384, 266, 1028, 0, 0), (513, 500, 1090, 6, 2),
@@ -1761,3 +1761,23 @@ def test_large_products_of_rows_on_dwords(gpu, M, N, K, kmajor):
     a, b = (torch.randint(-1, 2, shape, device=gpu, generator=g).to(torch.bfloat16) for shape in ((M, K), (N, K) if kmajor else (K, N)))
     b = b.t() if kmajor else b
     assert torch.equal(triton_amd.matmul(a, b, out_dtype=torch.float32), a.float() @ b.float())
+
+
+@pytest.mark.parametrize("dtype", ["fp16", "bf16", "e4m3"])
+def test_rings_of_two_stages_at_their_edges_are_bit_exact(gpu, dtype, monkeypatch):
+    test_ring_kernels_at_the_edges_of_their_ring_are_bit_exact(gpu, dtype, 13, monkeypatch)
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "e4m3"])
+@pytest.mark.parametrize("M,N,K", [(3200, 3072, 192), (1408, 6784, 64), (3840, 5376, 448), (4991, 1664, 512), (4733, 3160, 128), (2177, 2176, 2048)])
+def test_more_tiles_than_cus_of_a_short_k_on_two_workgroups_a_cu(gpu, dtype, M, N, K):
+    # what the default takes for them; whole numbers, an addend row, rows of C beside 16-byte boundaries
+    g = torch.Generator(device=gpu).manual_seed(M + N + K)
+    tdt = torch.bfloat16 if dtype == "bf16" else torch.float8_e4m3fn
+    a, b = (torch.randint(-1, 2, shape, device=gpu, generator=g).to(tdt) for shape in ((M, K), (N, K)))
+    want = a.float() @ b.float().t()
+    row = torch.randint(-8, 9, (N,), device=gpu, generator=g).to(torch.bfloat16)
+    for tb in (b.t(), b.t().contiguous()) if dtype == "bf16" else (b.t(),):
+        assert torch.equal(triton_amd.matmul(a, tb, out_dtype=torch.float32), want)
+        assert torch.equal(triton_amd.matmul(a, tb, out_dtype=torch.bfloat16), want.bfloat16())
+        assert torch.equal(triton_amd.matmul(a, tb, out_dtype=torch.bfloat16, add=row), (want + row.float()).bfloat16())

@@ -416,3 +416,8 @@ def test_less_workspace_than_a_split_wants_means_the_plain_call(gpu, fmt):
                                   None if null else ws.data_ptr(), size, stream)
         assert rc == 0 and bits_equal(to_np(c), ref), (size, null)
         assert bool((ws == 0xA5).all()) == (size < need or null), (size, null)
+
+
+@pytest.mark.parametrize("fmt", ["mxfp4", "mxfp8"])
+def test_rings_of_two_stages_at_their_edges_are_bit_exact(gpu, monkeypatch, fmt):
+    test_ring_kernels_at_the_edges_of_their_ring_are_bit_exact(gpu, monkeypatch, fmt, 13)

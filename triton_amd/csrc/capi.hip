@@ -198,6 +198,20 @@ double ring_rounds_us(int M, int N, int steps, int cus, int shape) {
   return 1.2 + (rounds > 1 ? t.whole * rounds + (1.0 - t.whole) * tiles / cus : 1.0) * (t.round_us + steps * t.step_us * (rounds > 1 ? 1.0 : 1.04));
 }
 
+// Ring tiles of 128x128 in two stages, two workgroups on a CU (more tiles than CUs only): while one waits for its first steps or stores, the other
+// multiplies, which four stages with a CU to themselves pay for in every tile.  us, before / so: bf16 K-major 3200 x 3072 x 192 19.6 / 11.4, 3456 x 1664 x 256
+// 11.1 / 8.2, row-major B 1408 x 6784 x 192 19.4 / 11.9, 3840 x 5376 x 448 37.7 / 27.0, 8064 x 2048 x 576 32.4 / 26.5; e4m3 1536 x 4224 x 640 13.0 / 10.8, 4352 x 5888
+// x 384 28.5 / 25.0; MXFP4 6400 x 4224 x 768 34.3 / 24.2, 2432 x 4992 x 1280 22.4 / 16.9, MXFP8 4224 x 4992 x 384 30.1 / 18.6.  A long K hides the waits anyway, and
+// two stages less of the latency: K-major 3712 x 4736 x 1920 63.7 / 77.4, e4m3 5376 x 2304 x 2048 26.0 / 33.6, MXFP8 3584 x 3968 x 4352 60.7 / 89.2; up to a round of tiles
+// a workgroup is alone either way: 1024 x 3712 x 768 9.5 / 10.2.  (150 products of 200 .. 3000 tiles and 2 .. 40 steps: within 6 % rms, block-scaled 12.)
+// `apart`: rows that do not begin on 128-byte lines (K-major bf16 2048 x 7808 x 984 37.8 / 44.0).  `epilogue`: us a round for what C takes beyond plain stores.
+double pairs_us(int M, int N, int steps, int cus, bool mx, bool apart, double epilogue = 0.0) {
+  const long tiles = (long)((M + 127) / 128) * ((N + 127) / 128), rounds = (tiles + cus - 1) / cus;
+  if (tiles <= cus) return 1e30;
+  const double k = (apart ? 1.5 : 1.0) * steps;
+  return mx ? 1.2 + (double)rounds * (1.9 + 0.6 * k) : 1.2 + (0.8 * rounds + 0.2 * tiles / cus) * (2.0 + epilogue + 0.45 * k);
+}
+
 // The same for the kernels of 256-column tiles with `rows` rows of C each (gemm_wave128.hip; edges: the eight-wave kernel, for
 // what that one does not take).  A K step of a 256-row tile is bound by its 64 KiB of operands and by power: with idle CUs it is
 // somewhat shorter, and several rounds are dealt evenly, so that an unfilled last round is spread over all of them.  180 products
@@ -250,7 +264,8 @@ Cut best_cut(int M, int N, int steps, int cus, int tile, int ring, bool is8) {
 // workgroups on a CU where a ring leaves room for one.  Measured over 16 .. 1280 tiles and K bytes of 16 .. 2048, this kernel / ring or
 // 256x256 tiles, us: 2688 x 2688 x 64 fp16 8.2 / 11.5, x 192 11.5 / 13.2, x 256 12.4 / 13.0; e4m3 x 384 10.6 / 12.6, x 512 12.3 / 12.7; row-major B, x 256
 // 12.0 / 13.6; edges cost it more (2659 x 2656 x 64 9.4 / 11.4, x 192 12.2 / 13.0).  Up to half as many tiles, whole ones only (1792 x 1920 x 64 6.0 / 7.1, 1763 x 1888
-// 1.06).  Not where one round of 256x256 tiles fills the CUs (3840 x 4096 x 16 1.1).
+// 1.06).  Not where one round of 256x256 tiles fills the CUs (3840 x 4096 x 16 1.1).  With more tiles than CUs the ring of two stages (pairs_us) takes what
+// it takes of them, that kernel / ring: fp16 3840 x 1792 x 256 11.1 / 8.2, row-major B 1642 x 3586 x 128 14.8 / 10.2, 1950 x 4480 x 64 10.0 / 10.3.
 bool short_k(int M, int N, int k_bytes, bool b_kmajor, int cus) {
   const long tiles = (long)((M + 127) / 128) * ((N + 127) / 128), tiles256 = (long)((M + 255) / 256) * ((N + 255) / 256);
   if (tiles256 <= cus && tiles256 * 10 >= cus * 9) return false;
@@ -477,10 +492,15 @@ PartChoice part_choice(const GemmArgs& p, const TileChoice& c, int es, bool b_km
   const long tiles256 = (long)((M + 255) / 256) * ((N + 255) / 256);
   const bool partial = knobs().tile_m == UNSET && knobs().mixed_rows == UNSET && (M % (c.tile_m ? c.tile_m : 256) != 0 || N % 256 != 0) &&
                        p.activation == MI355_ACT_NONE && (tiles256 > cus || tiles256 * 2 <= cus) && p.k_bytes <= (tiles256 > cus || !b_kmajor ? 384 : 320);
-  if (!by_knob && (tile != 6 || partial) && !p.aux && p.c_vec_ok && short_k(M, N, p.k_bytes, b_kmajor, cus)) r.tile = 1;   // (its addends and odd rows of C cost more)
+  const bool pairs_ok = !by_knob && knobs().tile_m == UNSET && knobs().mixed_rows == UNSET && ring_ok(es, b_kmajor);
+  if (!by_knob && (tile != 6 || partial) && !p.aux && p.c_vec_ok && short_k(M, N, p.k_bytes, b_kmajor, cus)) {   // (its addends and odd rows of C cost more)
+    if (pairs_ok && (long)((M + 127) / 128) * ((N + 127) / 128) > cus) r.ring = 4;
+    else r.tile = 1;
+  }
   else if (tile == 1 && by_knob) r.ring = 0;
   else if (tile >= 8 && tile <= 10) r.ring = tile - 8;
   else if (tile == 12 && b_kmajor) r.ring = 3;
+  else if (tile == 13) r.ring = 4;
   else if (tile == 11) r.tile = 1;   // the one-barrier-per-step kernel on 128x128 tiles
   else if (tile == 1 || (!by_knob && knobs().tile_m == UNSET && knobs().mixed_rows == UNSET)) {
     const int rows = tile == 6 && c.tile_m ? c.tile_m : 256;
@@ -492,6 +512,15 @@ PartChoice part_choice(const GemmArgs& p, const TileChoice& c, int es, bool b_km
     if (plan_us < (tile == 6 ? 0.92 : 1.0) * other) r.ring = plan.shape;   // (pitches move the rings by up to 15 %: 1664 x 6912 x 2112 bf16, 702 tiles, 53 us for the estimate's 47)
     const Cut cut = best_cut(M, N, steps, cus, tile, r.ring, is8);
     if (cut.us < (tile == 1 ? 0.88 : 0.92) * std::min(plan_us, other)) r.cut = cut;
+    // (an addend: fp16 3799 x 2304 x 512 23.2 / 23.7, row-major B 3840 x 6016 x 64, on the eight-wave kernel, 35.9 / 25.0; rows of C that are no whole groups of four:
+    // K-major 1468 x 4405 x 128 13.2 / 10.7; both, 2176 x 4234 x 256 18.3 / 19.3)
+    const double epilogue = (p.aux ? 2.2 : 0.0) + (p.c_vec_ok ? 0.0 : 2.0);
+    const double added = p.aux && tile != 1 ? (tile == 6 ? 2.8 : 6.5) * (double)(((long)((M + rows - 1) / rows) * ((N + 255) / 256) + cus - 1) / cus) : 0.0;
+    const double rings = plan_us + epilogue * (double)((M + 127) / 128) * ((N + 127) / 128) / cus;
+    if (pairs_ok && pairs_us(M, N, steps, cus, false, (p.lda | p.ldb) % 128 != 0, epilogue) < 0.97 * std::min({rings, other + added, r.cut.us})) {
+      r.ring = 4;
+      r.cut = {M, N, 1e30};
+    }
   }
   return r;
 }
@@ -1345,7 +1374,7 @@ static int mx_impl(const uint8_t* A, const uint8_t* sA, const uint8_t* B, const 
     const int steps = (p.k_bytes + 127) / 128;
     int shape = -1, splits = 1;
     if (knobs().tile != UNSET) {
-      if (knobs().tile >= 8 && knobs().tile <= 10) shape = knobs().tile - 8;
+      if ((knobs().tile >= 8 && knobs().tile <= 10) || knobs().tile == 13) shape = knobs().tile == 13 ? 4 : knobs().tile - 8;
     } else {
       // (less room than mi355_mx_gemm_workspace asks for: the plain call)
       if (workspace) splits = mx_splits(M, N, p.k_bytes, cus);
@@ -1360,7 +1389,8 @@ static int mx_impl(const uint8_t* A, const uint8_t* sA, const uint8_t* B, const 
         const double fill = rounds > 1 ? 1.0 : (double)tiles / cus, share = rows == 256 ? 1.0 : rows == 192 ? 0.78 : 0.64;
         other = kLaunchUs + (double)rounds * share * (8.0 + 1.5 * steps * (0.7 + 0.3 * fill));
       }
-      if (plan.us < other) shape = plan.shape;
+      if (splits <= 1 && pairs_us(M, N, steps, cus, true, (p.lda | p.ldb) % 128 != 0) < 0.97 * std::min(plan.us, other)) shape = 4;
+      else if (plan.us < other) shape = plan.shape;
       else splits = 1;
     }
     if (shape >= 0) {

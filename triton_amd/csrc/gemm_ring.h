@@ -232,8 +232,10 @@ __device__ __forceinline__ void ring_pin(f32x4& c) {
 template <int NS, int L>
 __device__ __forceinline__ void ring_drain_wait(int left) {
 #if MI355_DEVICE_PASS
-  static_assert(NS == 4 || NS == 8, "the ladders of these depths");
-  if constexpr (NS == 4)
+  static_assert(NS == 2 || NS == 4 || NS == 8, "the ladders of these depths");
+  if constexpr (NS == 2)
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  else if constexpr (NS == 4)
     asm volatile("s_cmp_lt_i32 %0, 4\n\ts_cbranch_scc1 ring_three_%=\n\ts_waitcnt vmcnt(%1)\n\ts_branch ring_done_%=\n"
                  "ring_three_%=:\n\ts_cmp_lt_i32 %0, 3\n\ts_cbranch_scc1 ring_all_%=\n\ts_waitcnt vmcnt(%2)\n\ts_branch ring_done_%=\n"
                  "ring_all_%=:\n\ts_waitcnt vmcnt(0)\nring_done_%=:" :: "s"(left), "i"(2 * L), "i"(L) : "memory", "scc");
@@ -454,15 +456,19 @@ __device__ __forceinline__ void gemm_ring_tile(const GemmArgs& p, const int pm, 
     const int kfull = p.k_bytes - tail;                       // bytes of K before the tail
     const int krows = p.K - kfull / E::kElemBytes;            // (a row-major B may end before the padded rows of A do)
     // The chunk that a row ends inside is read as the row's last 16 bytes and moved down: of K-contiguous rows at k_bytes, of rows of a
-    // row-major B at N (past_row: bytes that the lane's chunk of load q reaches beyond).
-    auto cut_chunk = [&](i32x4 v, int chunk) { return MX || E::kElemBytes != 2 || chunk * 16 + 16 <= tail ? v : bytes_down(v, -tail & 15); };
-    auto past_row = [&](int q) {
-      if (!open_rows) return 0;
+    // row-major B at N (past: bytes that the lane's chunk of load q reaches beyond).
+    int past[LB];
+#pragma unroll
+    for (int q = 0; q < LB; q++) past[q] = 0;
+    if (!B_KMAJOR && open_rows) {
       constexpr int CPR = BN / 8, RPI = 64 / CPR;
-      const int pc = lane % CPR, k = (wave * LB + q) * RPI + lane / CPR;
-      const int chunk = min((((pc >> 1) ^ xor_of(k)) << 1) | (pc & 1), (p.N + 7) / 8 - 1 - n0 / 8);
-      return max(0, (n0 + chunk * 8 + 8 - p.N) * 2);
-    };
+#pragma unroll
+      for (int q = 0; q < LB; q++) {
+        const int pc = lane % CPR, k = (wave * LB + q) * RPI + lane / CPR;
+        const int chunk = min((((pc >> 1) ^ xor_of(k)) << 1) | (pc & 1), (p.N + 7) / 8 - 1 - n0 / 8);
+        past[q] = max(0, (n0 + chunk * 8 + 8 - p.N) * 2);
+      }
+    }
     const char* kA = tileA + kfull;
     const char* kB = B_KMAJOR ? tileB + kfull : tileB + (int64_t)(kfull / 2) * p.ldb;
 #pragma unroll
@@ -470,24 +476,39 @@ __device__ __forceinline__ void gemm_ring_tile(const GemmArgs& p, const int pm, 
 #pragma unroll
     for (int q = 0; q < LB; q++) {
       if constexpr (B_KMAJOR) load16_sbase<0>(tb[q], kB, voffB[q] + q * 1024 - rowB[q] * 16 + min(rowB[q] * 16, tail - 16));
-      else load16_sbase<0>(tb[q], kB, voffB[q] + q * 1024 - (unsigned)(rowB[q] - min(rowB[q], krows - 1)) * (unsigned)p.ldb - (unsigned)past_row(q));
+      else load16_sbase<0>(tb[q], kB, voffB[q] + q * 1024 - (unsigned)(rowB[q] - min(rowB[q], krows - 1)) * (unsigned)p.ldb - (unsigned)past[q]);
     }
     int ts = 0;   // (block-scaled: K is a multiple of 128 elements, so an MXFP4 tail is four blocks - one dword of scales - and there is no other)
     const int bs = wave % BLOCKS;
     if constexpr (MX) load4_sbase(ts, scale_base(bs) + kfull / RING_ROW * 4 * SD, scale_rows(bs));
     fill(true);
     const i32x4 zero = {0, 0, 0, 0};
+    // (landed, all of them: from here on branches may move them)
+#pragma unroll
+    for (int q = 0; q < LA; q++) lds_use(ta[q]);
+#pragma unroll
+    for (int q = 0; q < LB; q++) lds_use(tb[q]);
+    if constexpr (!MX && E::kElemBytes == 2) {
+      if (tail & 15) {
+#pragma unroll
+        for (int q = 0; q < LA; q++) ta[q] = chunkA[q] * 16 + 16 <= tail ? ta[q] : bytes_down(ta[q], -tail & 15);
+        if constexpr (B_KMAJOR) {
+#pragma unroll
+          for (int q = 0; q < LB; q++) tb[q] = rowB[q] * 16 + 16 <= tail ? tb[q] : bytes_down(tb[q], -tail & 15);
+        }
+      }
+      if (!B_KMAJOR && open_rows) {
+#pragma unroll
+        for (int q = 0; q < LB; q++) tb[q] = past[q] > 0 ? bytes_down(tb[q], -2 * p.N & 15) : tb[q];
+      }
+    }
 #pragma unroll
     for (int q = 0; q < LA; q++) {
-      lds_use(ta[q]);
-      *(LDS_PTR(i32x4))(uintptr_t)(lds0 + (wave * LA + q) * 1024 + lane * 16) = chunkA[q] * 16 < tail ? cut_chunk(ta[q], chunkA[q]) : zero;
+      *(LDS_PTR(i32x4))(uintptr_t)(lds0 + (wave * LA + q) * 1024 + lane * 16) = chunkA[q] * 16 < tail ? ta[q] : zero;
     }
 #pragma unroll
     for (int q = 0; q < LB; q++) {
-      lds_use(tb[q]);
       const bool in = B_KMAJOR ? rowB[q] * 16 < tail : rowB[q] < krows;
-      if constexpr (B_KMAJOR) tb[q] = cut_chunk(tb[q], rowB[q]);
-      else if (past_row(q) > 0) tb[q] = bytes_down(tb[q], -2 * p.N & 15);
       *(LDS_PTR(i32x4))(uintptr_t)(lds0 + A_BYTES + (wave * LB + q) * 1024 + lane * 16) = in ? tb[q] : zero;
     }
     if constexpr (MX) {

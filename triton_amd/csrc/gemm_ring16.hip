@@ -8,6 +8,7 @@ template <typename E, bool KM>
 int launch(const GemmArgs& p, int shape, int splits, int chunk_bytes, hipStream_t stream) {
   switch (shape) {
     case 0: return launch_gemm_ring<E, 128, 128, 2, KM, 4>(p, splits, chunk_bytes, stream);
+    case 4: return launch_gemm_ring<E, 128, 128, 2, KM, 2>(p, splits, chunk_bytes, stream);
     case 1: return launch_gemm_ring<E, 128, 64, 2, KM, 4>(p, splits, chunk_bytes, stream);
     case 3:
       if constexpr (KM) return launch_gemm_ring<E, 64, 32, 2, true, 8>(p, splits, chunk_bytes, stream);

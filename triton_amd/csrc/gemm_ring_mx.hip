@@ -9,6 +9,7 @@ template <typename E>
 int launch(const GemmArgs& p, int shape, int splits, int chunk_bytes, hipStream_t stream) {
   switch (shape) {
     case 0: return launch_gemm_ring<E, 128, 128, 2, true, 4>(p, splits, chunk_bytes, stream);
+    case 4: return launch_gemm_ring<E, 128, 128, 2, true, 2>(p, splits, chunk_bytes, stream);
     case 1: return launch_gemm_ring<E, 128, 64, 2, true, 4>(p, splits, chunk_bytes, stream);
     default: return launch_gemm_ring<E, 64, 64, 2, true, 4>(p, splits, chunk_bytes, stream);
   }

@@ -167,7 +167,7 @@ int gemm_masked_grouped_launch(const GroupedTable& ga, bool bf16, hipStream_t st
 int gemm16_grouped_launch(const GroupedArgs& ga, bool bf16, int nprog, int nprog_big, hipStream_t stream);
 int gemm16_launch(const GemmArgs& p, bool bf16, bool b_kmajor, int tile, hipStream_t stream);
 int gemm8_launch(const GemmArgs& p, bool e5m2, bool b_kmajor, int tile, hipStream_t stream);
-// ring kernels (gemm_ring.h); shape: 0 = tiles of 128x128, 1 = 128x64, 2 = 64x64; chunk_bytes of K per split, whole 128-byte steps
+// ring kernels (gemm_ring.h); shape: 0 = tiles of 128x128, 1 = 128x64, 2 = 64x64, 4 = 128x128 in two stages; chunk_bytes of K per split, whole 128-byte steps
 int gemm_ring16_launch(const GemmArgs& p, bool bf16, bool b_kmajor, int shape, int splits, int chunk_bytes, hipStream_t stream);
 int gemm_ring8_launch(const GemmArgs& p, bool e5m2, int shape, int splits, int chunk_bytes, hipStream_t stream);
 int gemm32_launch(const GemmArgs& p, int tile, hipStream_t stream);   // fp32 operands, K-major B; tile as for gemm16_launch
