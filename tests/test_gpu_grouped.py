@@ -254,3 +254,18 @@ def test_groups_checked_in_native_code_are_the_python_function_s(gpu, monkeypatc
     with Dispatch():
         triton_amd.matmul(a[0], b[0])
     assert Dispatch.seen > 0
+
+
+@pytest.mark.parametrize("nprog", [0, 7])
+@pytest.mark.parametrize("sizes", [
+    [(m, 256, 3072) for m in (1, 130, 65, 300)],                          # 64x64 tiles
+    [(m, 1024, 1280) for m in (18, 1615, 32, 112, 371, 524)],             # 128x128 tiles
+    [(m, 2304, 256) for m in (314, 305, 626, 369, 35, 1464, 1, 1154)],    # of those, two workgroups on a CU
+    [(728, 1320, 1120), (1128, 1064, 192), (360, 136, 128), (112, 592, 1192), (1, 8, 8), (1900, 1608, 552)]])
+def test_every_shape_of_tiles_is_bit_exact_on_integers(gpu, sizes, nprog):
+    # several tiles a program, K steps fewer than stages, partial tiles.  Whole numbers up to 4096: exact in fp32, rounded once
+    g = torch.Generator(device=gpu).manual_seed(len(sizes))
+    a = [torch.randint(-1, 2, (m, k), device=gpu, generator=g).bfloat16() for m, n, k in sizes]
+    b = [torch.randint(-1, 2, (k, n), device=gpu, generator=g).bfloat16() for m, n, k in sizes]
+    for x, y, c in zip(a, b, triton_amd.group_gemm_fn(a, b, num_programs=nprog)):
+        assert torch.equal(c, (x.float() @ y.float()).bfloat16()), (x.shape, y.shape)

@@ -212,6 +212,39 @@ double pairs_us(int M, int N, int steps, int cus, bool mx, bool apart, double ep
   return mx ? 1.2 + (double)rounds * (1.9 + 0.6 * k) : 1.2 + (0.8 * rounds + 0.2 * tiles / cus) * (2.0 + epilogue + 0.45 * k);
 }
 
+// A group on ring tiles of one shape (0, 2 or 4), its problems in `order`, the longest K first.  us: all tiles' time spread over the CUs, or what the CU
+// with the most tiles of the first problems has, or one tile of the longest K (60 drawn groups of 2 .. 16 problems: within 13 % rms; the shape chosen by it is
+// within 1 % of the best of the three in the geometric mean).
+// chunk: the order of the tiles.  An eighth of them for each XCD, one after the other, keeps the operands in its L2; but where the first eighth has the tiles of
+// the longest K, one XCD works when the others are done: then runs of `chunk` tiles are dealt to the XCDs in turn.  us, eighths / runs: ten problems
+// of 64 .. 1792 rows and K of 64 .. 2048 22.4 / 17.2 (64x64), 64 .. 1600 23.3 / 16.9, 25.3 / 16.3 (128x128); one K for all, 2304 -> 256 24.5 / 26.9, 1024 -> 1280 14.5 / 17.0;
+// no more tiles than CUs, K of 256 .. 1792 7.3 / 7.6.
+struct GroupPlan { double us; int chunk; int64_t tiles; };
+GroupPlan group_plan(const int32_t* sizes, const int* order, int n, int shape, int cus) {
+  static const struct { int edge, slots, chunk; double base, tile_us, step_us, most, lone_us, lone_step_us; } kShapes[3] = {
+      {128, 1, 8, 1.5, 4.5, 0.49, 0.82, 1.35, 0.33}, {64, 1, 16, 3.5, 0.78, 0.227, 0.68, 0.6, 0.128}, {128, 2, 8, 2.6, 2.3, 0.58, 0.89, 1.0, 0.65}};
+  const auto& t = kShapes[shape / 2];
+  auto steps = [&](int i) { return (sizes[3 * order[i] + 2] + 63) / 64; };
+  auto count = [&](int i) {
+    const int32_t* s = sizes + 3 * order[i];
+    return (int64_t)((s[0] + t.edge - 1) / t.edge) * ((s[1] + t.edge - 1) / t.edge);
+  };
+  double sum = 0.0, longest = t.lone_us + t.lone_step_us * steps(0);
+  int64_t tiles = 0;
+  for (int i = 0; i < n; i++) {
+    const double us = t.tile_us + t.step_us * steps(i);
+    tiles += count(i);
+    sum += (double)count(i) * us;
+    longest = std::max(longest, t.most * us * (double)((tiles + t.slots * cus - 1) / (t.slots * cus)));
+  }
+  double first = 0.0, left = (double)tiles / 8;
+  for (int i = 0; i < n && left > 0.0; i++) {
+    first += std::min((double)count(i), left) * (t.tile_us + t.step_us * steps(i));
+    left -= (double)count(i);
+  }
+  return {t.base + std::max(sum / cus, longest), tiles > cus && first > 1.15 * sum / 8 ? t.chunk : 0, tiles};
+}
+
 // The same for the kernels of 256-column tiles with `rows` rows of C each (gemm_wave128.hip; edges: the eight-wave kernel, for
 // what that one does not take).  A K step of a 256-row tile is bound by its 64 KiB of operands and by power: with idle CUs it is
 // somewhat shorter, and several rounds are dealt evenly, so that an unfilled last round is spread over all of them.  180 products
@@ -1189,7 +1222,6 @@ int mi355_grouped_gemm_host(const void* const* a, const void* const* b, void* co
   for (int g0 = 0; g0 < group_size; g0 += G) {
     const int count = std::min(G, group_size - g0);
     int order[G], n = 0, odd[G], nodd = 0;
-    double cost64[G], cost128[G], sum64 = 0, sum128 = 0, sum = 0, top64 = 0, top128 = 0, top = 0;
     bool whole = true;
     long tiles256 = 0;
     for (int i = 0; i < count; i++) {
@@ -1199,13 +1231,6 @@ int mi355_grouped_gemm_host(const void* const* a, const void* const* b, void* co
         odd[nodd++] = i;
         continue;
       }
-      // us of one tile and of all, on either tile size (the figures of ring_plan with several rounds under way)
-      const int steps = (s[2] + 63) / 64;
-      const double one128 = 2.5 + 0.5 * steps, one64 = 0.6 + 0.195 * steps;
-      cost128[i] = one128 * ((s[0] + 127) / 128) * ((s[1] + 127) / 128);
-      cost64[i] = one64 * ((s[0] + 63) / 64) * ((s[1] + 63) / 64);
-      sum128 += cost128[i]; sum64 += cost64[i]; sum += std::min(cost128[i], cost64[i]);
-      top128 = std::max(top128, one128); top64 = std::max(top64, one64); top = std::max(top, cost64[i] <= cost128[i] ? one64 : one128);
       tiles256 += (long)((s[0] + 255) / 256) * ((s[1] + 255) / 256);
       whole = whole && s[0] % 256 == 0 && s[1] % 256 == 0 && s[2] % 128 == 0 && s[2] >= knob(knobs().grouped_wave128_min_k, 512) && l[1] % 256 == 0 &&
               (int64_t)l[0] * 16 + s[2] * 2 < (1ll << 31) && (int64_t)s[2] * l[1] * 2 + 512 < (1ll << 31);
@@ -1247,23 +1272,27 @@ int mi355_grouped_gemm_host(const void* const* a, const void* const* b, void* co
       ga.total_tiles = (int)tiles256;
       rc = gemm_wave128_grouped_table_launch(ga, bf16, num_programs > 0 ? std::min(num_programs, cus) : cus, stream);
     } else {
-      // every problem on the tile size that costs it less, unless larger tiles leave CUs idle; the longest tiles first, so
-      // that the last ones to be started are short
-      const double t64 = std::max(sum64 / cus, top64), t128 = std::max(sum128 / cus, top128), tmix = std::max(sum / cus, top);
-      const int pick = t64 <= t128 && t64 <= tmix ? 64 : t128 <= tmix ? 128 : 0;
+      // the longest tiles first, so that the last ones to be started are short
       std::stable_sort(order, order + n, [&](int x, int y) { return sizes[3 * (g0 + x) + 2] > sizes[3 * (g0 + y) + 2]; });
-      int64_t tiles = 0;
+      GroupPlan plan{1e30, 0, 0};
+      int shape = 0;
+      for (int candidate : {2, 0, 4}) {
+        const GroupPlan x = group_plan(sizes + 3 * g0, order, n, candidate, cus);
+        if (x.us < plan.us) { plan = x; shape = candidate; }
+      }
+      if (plan.tiles > INT_MAX / 2) return MI355_ESHAPE;
+      const int edge = shape == 2 ? 64 : 128;
+      int tiles = 0;
       for (int at = 0; at < n; at++) {
-        const int i = order[at], edge = pick ? pick : cost64[i] <= cost128[i] ? 64 : 128;
-        put(ga, at, i);
-        ga.first_tile[at] = (int)tiles;
-        if (edge == 64) ga.small_tiles |= 1ull << at;
-        tiles += (int64_t)((ga.sizes[3 * at] + edge - 1) / edge) * ((ga.sizes[3 * at + 1] + edge - 1) / edge);
-        if (tiles > INT_MAX / 2) return MI355_ESHAPE;
+        put(ga, at, order[at]);
+        ga.first_tile[at] = tiles;
+        tiles += ((ga.sizes[3 * at] + edge - 1) / edge) * ((ga.sizes[3 * at + 1] + edge - 1) / edge);
       }
       for (int at = n; at < G; at++) ga.first_tile[at] = INT_MAX;
-      ga.total_tiles = (int)tiles;
-      rc = gemm_ring_grouped_launch(ga, bf16, num_programs > 0 ? (int)std::min<int64_t>(num_programs, tiles) : (int)tiles, stream);
+      ga.total_tiles = tiles;
+      ga.chunk = plan.chunk;
+      ga.padded_tiles = plan.chunk > 0 ? (tiles + 8 * plan.chunk - 1) / (8 * plan.chunk) * (8 * plan.chunk) : tiles;
+      rc = gemm_ring_grouped_launch(ga, bf16, shape, num_programs > 0 ? std::min(num_programs, tiles) : ga.padded_tiles, stream);
     }
     if (rc) return rc;
   }

@@ -18,20 +18,27 @@ int launch(const GemmArgs& p, int shape, int splits, int chunk_bytes, hipStream_
 }
 
 // Grouped GEMM (python/tutorials/08-grouped-gemm.py:64-140: row-major A, B and C of one type) with the problem table as a
-// kernel argument: program b takes the tiles b, b + gridDim.x, ... of all problems, numbered problem after problem, each
-// problem on tiles of 128x128 or of 64x64 as the host chose for it.  Problems have rows of whole 16-byte chunks (A and B).
+// kernel argument: program b takes the tiles b, b + gridDim.x, ... of all problems, numbered problem after problem, in the
+// order that group_plan chose.
+// Problems have rows of whole 16-byte chunks (A and B).
 // Bound by the launch for small groups: with the tables copied to the device (five copies) and three launches of which one
-// works, the group 1024^3, 512^3, 256^3, 128^3 took 112 us a call, 25 of them on 85 tiles of 128x128; now 11 us, one launch of
-// 340 tiles of 64x64.  Experts 2440 -> 600 with 20 .. 334 rows each, four of them: 126 -> 14 us; 1664 -> 3712 with 30 .. 1758 rows,
-// three: 156 -> 50.
-template <typename E>
+// works, the group 1024^3, 512^3, 256^3, 128^3 took 112 us a call, 25 of them on 85 tiles of 128x128; now 8, one launch of
+// 340 tiles of 64x64.  Larger ones run on 128x128 tiles, in four stages or, more of them than CUs, in two with two
+// workgroups on a CU (group_plan): us on 64x64 / 128x128 / those pairs, eleven experts 2304 -> 256 of 35 .. 1464 rows 35.0 / 33.4 / 24.5,
+// 272 -> 3248 18.0 / 28.7 / 39.9, 1024 -> 1280 19.4 / 14.5 / 18.2.  (Small and large tiles in one launch, each problem on what costs it less:
+// never far ahead, 20.4 for 15.2 where its 64x64 tiles had 128x128 ones' LDS and a CU to themselves.)
+template <typename E, int EDGE, int NS>
 __global__ __launch_bounds__(256, 1) void gemm_ring_grouped_kernel(GroupedTable ga) {
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   const unsigned lds0 = lds_addr((LDS_PTR(char))smem);
   const int nprog = gridDim.x;
   // one table entry per lane: the problem of a tile is a comparison away, whatever the number of problems
   const int first = ga.first_tile[threadIdx.x & 63];
-  for (int t = xcd_remap(blockIdx.x, nprog); t < ga.total_tiles; t += nprog) {
+  // chunk: the tiles in runs of so many, dealt to the XCDs in turn; 0: an XCD takes an eighth of them, one after the other
+  const int c = ga.chunk;
+  for (int u = c > 0 ? (int)blockIdx.x : xcd_remap(blockIdx.x, nprog); u < ga.padded_tiles; u += nprog) {
+    const int t = c > 0 ? (u / 8 / c * 8 + u % 8) * c + u / 8 % c : u;
+    if (t >= ga.total_tiles) continue;
     const int gi = __builtin_amdgcn_readfirstlane((int)__popcll(__ballot(first <= t)) - 1);
     const int tile = t - ga.first_tile[gi];
     GemmArgs p{};
@@ -41,33 +48,36 @@ __global__ __launch_bounds__(256, 1) void gemm_ring_grouped_kernel(GroupedTable 
     p.lda = (int64_t)ga.lds[gi * 3] * 2; p.ldb = (int64_t)ga.lds[gi * 3 + 1] * 2; p.ldc = ga.lds[gi * 3 + 2];
     p.scn = 1; p.out_dtype = ga.out_dtype;
     p.c_vec_ok = p.ldc % 4 == 0 && (uintptr_t)p.C % 16 == 0;
-    const int edge = (ga.small_tiles >> gi) & 1 ? 64 : 128;
     int pm, pn;
-    grouped_tile(tile, (p.M + edge - 1) / edge, (p.N + edge - 1) / edge, 8, pm, pn);
-    if (edge == 64) gemm_ring_tile<E, 64, 64, 2, false, 4>(p, pm, pn, lds0);
-    else gemm_ring_tile<E, 128, 128, 2, false, 4>(p, pm, pn, lds0);
+    grouped_tile(tile, (p.M + EDGE - 1) / EDGE, (p.N + EDGE - 1) / EDGE, 8, pm, pn);
+    gemm_ring_tile<E, EDGE, EDGE, 2, false, NS>(p, pm, pn, lds0);
     wait_vmcnt<0>();   // (the stores: the next tile counts its loads)
     block_barrier();   // the next tile's loads overwrite the stages
   }
 }
 
-template <typename E>
+template <typename E, int EDGE, int NS>
 int launch_grouped(const GroupedTable& ga, int nprog, hipStream_t stream) {
-  constexpr int most = 4 * (128 + 128) * RING_ROW;
+  constexpr int smem = NS * 2 * EDGE * RING_ROW;
   static bool attr_set = false;
   if (!attr_set) {
-    hipError_t e = hipFuncSetAttribute((const void*)gemm_ring_grouped_kernel<E>, hipFuncAttributeMaxDynamicSharedMemorySize, most);
+    hipError_t e = hipFuncSetAttribute((const void*)gemm_ring_grouped_kernel<E, EDGE, NS>, hipFuncAttributeMaxDynamicSharedMemorySize, smem);
     if (e != hipSuccess) return (int)e;
     attr_set = true;
   }
-  const uint64_t all = ga.group_size == 64 ? ~0ull : (1ull << ga.group_size) - 1;
-  gemm_ring_grouped_kernel<E><<<dim3(nprog), dim3(256), ga.small_tiles == all ? most / 2 : most, stream>>>(ga);
+  gemm_ring_grouped_kernel<E, EDGE, NS><<<dim3(nprog), dim3(256), smem, stream>>>(ga);
   return (int)hipGetLastError();
+}
+
+template <typename E>
+int launch_grouped(const GroupedTable& ga, int shape, int nprog, hipStream_t stream) {
+  if (shape == 2) return launch_grouped<E, 64, 4>(ga, nprog, stream);
+  return shape == 4 ? launch_grouped<E, 128, 2>(ga, nprog, stream) : launch_grouped<E, 128, 4>(ga, nprog, stream);
 }
 }  // namespace
 
-int gemm_ring_grouped_launch(const GroupedTable& ga, bool bf16, int nprog, hipStream_t stream) {
-  return bf16 ? launch_grouped<Ring16<bf16x8>>(ga, nprog, stream) : launch_grouped<Ring16<f16x8>>(ga, nprog, stream);
+int gemm_ring_grouped_launch(const GroupedTable& ga, bool bf16, int shape, int nprog, hipStream_t stream) {
+  return bf16 ? launch_grouped<Ring16<bf16x8>>(ga, shape, nprog, stream) : launch_grouped<Ring16<f16x8>>(ga, shape, nprog, stream);
 }
 
 int gemm_ring16_launch(const GemmArgs& p, bool bf16, bool b_kmajor, int shape, int splits, int chunk_bytes, hipStream_t stream) {
