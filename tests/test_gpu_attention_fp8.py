@@ -97,3 +97,27 @@ def test_fp8_forward_needs_transposed_v_and_has_no_backward(gpu):
     t = torch.zeros(1, 1, 128, 64, device=gpu, dtype=torch.float8_e5m2)
     with pytest.raises(AssertionError):
         triton_amd.attention(t, t, t, False, 0.5)          # v with D contiguous
+
+
+@pytest.mark.parametrize("fmt", ["e5m2", "e4m3"])
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("variant,shape", [(6, (1, 2, 128, 64)), (6, (2, 3, 640, 64)), (6, (1, 2, 128, 128)), (6, (1, 3, 896, 128)), (7, (1, 2, 256, 64)),
+                                           (7, (1, 3, 1280, 64)), (8, (1, 2, 128, 64)), (8, (1, 3, 640, 64)), (8, (1, 2, 384, 128))])
+def test_groups_of_waves_along_the_keys_agree_with_one(gpu, fmt, causal, variant, shape, monkeypatch):
+    # scores that no block's maximum exceeds the first one's by 2^4 of: every group rounds the same P, and only the order of the fp32 sums differs.
+    # Rows of a block that begin and end beside a group's blocks, fewer blocks than groups.  With larger scores: as far from 64 bits as one group is
+    (q, k, v), (tq, tk, tv) = _fp8_inputs(sum(shape), shape, fmt, gpu)
+    tk = tk.contiguous()
+    for scale, same in ((shape[-1] ** -0.5, True), (shape[-1] ** 0.5, False)):
+        set_knob(monkeypatch, "MI355_ATTN_FWD_VARIANT", "1")
+        one = triton_amd.attention(tq, tk, tv, causal, scale).float()
+        set_knob(monkeypatch, "MI355_ATTN_FWD_VARIANT", str(variant))
+        got = triton_amd.attention(tq, tk, tv, causal, scale).float()
+        if same:
+            assert (got != one).float().mean() < 1e-3 and (got - one).norm() < 5e-3 * one.norm()
+        s = torch.from_numpy(q).to(gpu).double() @ torch.from_numpy(k).to(gpu).double().transpose(2, 3) * scale
+        if causal:
+            s.masked_fill_(torch.ones_like(s, dtype=torch.bool).triu(1), float("-inf"))
+        want = torch.softmax(s, -1) @ torch.from_numpy(v).to(gpu).double()
+        err = [((x.double() - want).norm() / want.norm()).item() for x in (one, got)]
+        assert err[1] <= 1.05 * err[0], err

@@ -33,17 +33,22 @@ __device__ __forceinline__ f32x16 mfma_f8(i32x8 a, i32x8 b, f32x16 c) {
 // missing columns are zeros that never exist in memory - the Q fragments are zero-filled in registers, the K / V^T
 // tiles in LDS are zeroed once and only the chunks present are ever loaded, and only the first d_real columns of O are
 // stored.  Zero columns add nothing to the scores and give zero columns of O: what a HEAD_DIM d_real kernel computes.
-template <int FMT, int D, int NW, bool PAD = false>
+// KW > 1: groups of waves along the keys, as in attn_fwd.hip: every group takes each KW-th block of 64 keys for the same rows, and their
+// maxima, sums and accumulators meet in LDS, for launches of fewer blocks than CUs, which last as long as one block's walk
+// over the keys.  P is rounded to two or three bits of fraction, so that another maximum under it would be another result altogether:
+// every group starts from the maximum of the row's first 64 keys, as a single one does.
+template <int FMT, int D, int NW, bool PAD = false, int KW = 1>
 __global__ __launch_bounds__(NW * 64, NW == 4 && D <= 128 ? 2 : 1) void attn_fwd8_kernel(AttnArgs p) {
-  static_assert(!PAD || D == 64, "the padded form is the 64-column one");
-  constexpr int BM = NW * 32, BN = 64;
+  static_assert(!PAD || (D == 64 && KW == 1), "the padded form is the 64-column one");
+  constexpr int QW = NW / KW;          // waves along the query rows
+  constexpr int BM = QW * 32, BN = 64;
   constexpr int KSQ = D / 64;          // MFMA k-steps of S^T
   constexpr int DT = D / 32;           // 32-row tiles of O^T
   constexpr int KTILE = BN * D;        // K tile: 64 rows of D bytes
   constexpr int VTILE = D * BN;        // V^T tile: D rows of 64 bytes
-  constexpr int STAGE = KTILE + VTILE;
+  constexpr int BLOCK = KTILE + VTILE, STAGE = KW * BLOCK;
   constexpr int KCH = D / 16;          // 16-byte chunks per K row
-  constexpr int KINST = KTILE / 1024 / NW, VINST = VTILE / 1024 / NW;
+  constexpr int KINST = KTILE / 1024 / QW, VINST = VTILE / 1024 / QW;
   static_assert(KINST >= 1 && VINST >= 1, "tiles too small for this wave count");
 
   extern __shared__ __attribute__((aligned(1024))) char smem[];
@@ -52,12 +57,13 @@ __global__ __launch_bounds__(NW * 64, NW == 4 && D <= 128 ? 2 : 1) void attn_fwd
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l32 = lane & 31, g = lane >> 5;
+  const int kw = wave / QW, qw = wave % QW;   // the wave's group along the keys, its 32 rows
 
   const int nqb = (p.N + BM - 1) / BM;
   int hz, z, h, qb;
   attn_block(p, nqb, hz, z, h, qb);
   if (p.causal) qb = nqb - 1 - qb;   // longest first
-  const int m0 = qb * BM, row0 = m0 + wave * 32;
+  const int m0 = qb * BM, row0 = m0 + qw * 32;
 
   const char* qbase = p.q + (int64_t)z * p.sq[0] + (int64_t)h * p.sq[1];
   const char* kbase = p.k + (int64_t)z * p.sk[0] + (int64_t)h * p.sk[1];
@@ -94,14 +100,14 @@ __global__ __launch_bounds__(NW * 64, NW == 4 && D <= 128 ? 2 : 1) void attn_fwd
   bool presentK[KINST], presentV[VINST];
 #pragma unroll
   for (int i = 0; i < KINST; i++) {
-    const int r = (i * NW + wave) * (1024 / D) + lane / KCH;
+    const int r = (i * QW + qw) * (1024 / D) + lane / KCH;
     const int chunk = (lane % KCH) ^ kswz8(r);
     offK[i] = (unsigned)(r * kpitch) + (chunk << 4);
     presentK[i] = !PAD || chunk * 16 < p.d_real;
   }
 #pragma unroll
   for (int i = 0; i < VINST; i++) {
-    const int r = (i * NW + wave) * 16 + lane / 4;   // d row
+    const int r = (i * QW + qw) * 16 + lane / 4;   // d row
     offV[i] = (unsigned)(r * vpitch) + (((lane % 4) ^ vswz8(r)) << 4);
     presentV[i] = !PAD || r < p.d_real;
   }
@@ -111,15 +117,15 @@ __global__ __launch_bounds__(NW * 64, NW == 4 && D <= 128 ? 2 : 1) void attn_fwd
     __syncthreads();
   }
   auto issue_kv = [&](int j, int stage) {
-    const unsigned kd = lds_base + stage * STAGE, vd = kd + KTILE;
-    const char* ksrc = kbase + (int64_t)j * BN * kpitch;
-    const char* vsrc = vbase + (int64_t)j * BN;
+    const unsigned kd = lds_base + stage * STAGE + kw * BLOCK, vd = kd + KTILE;
+    const char* ksrc = kbase + (int64_t)(j * KW + kw) * BN * kpitch;   // (N is a multiple of KW blocks: the host's rule)
+    const char* vsrc = vbase + (int64_t)(j * KW + kw) * BN;
 #pragma unroll
     for (int i = 0; i < KINST; i++)
-      if (presentK[i]) async_copy16_sbase(ksrc, offK[i], kd + (i * NW + wave) * 1024);
+      if (presentK[i]) async_copy16_sbase(ksrc, offK[i], kd + (i * QW + qw) * 1024);
 #pragma unroll
     for (int i = 0; i < VINST; i++)
-      if (presentV[i]) async_copy16_sbase(vsrc, offV[i], vd + (i * NW + wave) * 1024);
+      if (presentV[i]) async_copy16_sbase(vsrc, offV[i], vd + (i * QW + qw) * 1024);
   };
 
   // per-lane LDS offsets.  K operand of tile row l32 = 8a + 4b + e is key row 16b + 4a + e
@@ -148,50 +154,75 @@ __global__ __launch_bounds__(NW * 64, NW == 4 && D <= 128 ? 2 : 1) void attn_fwd
   constexpr float RESCALE_LOG2 = 4.f;
 
   const int kv_end_blk = p.causal ? min(p.N, m0 + BM) : p.N;
-  const int nsteps = (kv_end_blk + BN - 1) / BN;
-  const int wave_last = p.causal ? (row0 + 31) / BN : nsteps - 1;
-  const int wave_first_masked = p.causal ? row0 / BN : nsteps;
+  const int nsteps = (kv_end_blk + BN * KW - 1) / (BN * KW);
+  const int wave_last = p.causal ? (row0 + 31) / BN : nsteps * KW - 1;
+  const int wave_first_masked = p.causal ? row0 / BN : nsteps * KW;
 
   issue_kv(0, 0);
   wait_all();
   __syncthreads();
 
+  // S^T = K Q^T for the two 32-key tiles of the block at LDS address `base`
+  auto scores = [&](f32x16 (&s)[2], const unsigned base) {
+    i32x4 kf[2][KSQ][2];
+    static_for<2>([&](auto A_) {
+      constexpr int a = decltype(A_)::value;
+      static_for<KSQ>([&](auto KS_) {
+        constexpr int ks = decltype(KS_)::value;
+        kf[a][ks][0] = lds_read_b128<a * 32 * D>(base + ka[ks][0]);
+        kf[a][ks][1] = lds_read_b128<a * 32 * D>(base + ka[ks][1]);
+      });
+    });
+    static_for<2>([&](auto A_) {
+      constexpr int a = decltype(A_)::value;
+      lds_wait<(1 - a) * 2 * KSQ>();
+      static_for<KSQ>([&](auto KS_) {
+        constexpr int ks = decltype(KS_)::value;
+        lds_use(kf[a][ks][0]);
+        lds_use(kf[a][ks][1]);
+        i32x8 kop = __builtin_shufflevector(kf[a][ks][0], kf[a][ks][1], 0, 1, 2, 3, 4, 5, 6, 7);
+        if constexpr (ks == 0) {
+          f32x16 zero;
+#pragma unroll
+          for (int r = 0; r < 16; r++) zero[r] = 0.f;
+          s[a] = mfma_f8<FMT>(kop, qf[0], zero);
+        } else {
+          s[a] = mfma_f8<FMT>(kop, qf[ks], s[a]);
+        }
+      });
+    });
+  };
+  // masks the scores of block `blk` and returns the row's largest
+  auto row_max = [&](f32x16 (&s)[2], const int blk) {
+    if (blk >= wave_first_masked) {
+      const int qrow = row0 + l32;
+#pragma unroll
+      for (int a = 0; a < 2; a++)
+#pragma unroll
+        for (int r = 0; r < 16; r++)
+          if (blk * BN + a * 32 + g * 16 + r > qrow) s[a][r] = -INFINITY;
+    }
+    float mx = s[0][0];
+#pragma unroll
+    for (int a = 0; a < 2; a++)
+#pragma unroll
+      for (int r = 0; r < 16; r++) mx = fmaxf(mx, s[a][r]);
+    return pair_max(mx);
+  };
+  if (KW > 1 && kw > 0) {   // (block 0 is the first group's, in the first stage)
+    f32x16 s[2];
+    scores(s, lds0);
+    m_i = row_max(s, 0) * qk_scale;
+  }
+
   auto step = [&](const int j, auto STAGE_) {
     constexpr int SOFF = decltype(STAGE_)::value * STAGE;
     if (j + 1 < nsteps) issue_kv(j + 1, decltype(STAGE_)::value ^ 1);
-    if (j <= wave_last && row0 < p.N) {
-      const unsigned base = lds0 + SOFF;
-      // ---- S^T = K Q^T for the two 32-key tiles
+    const int blk = j * KW + kw;
+    if (blk <= wave_last && row0 < p.N) {
+      const unsigned base = lds0 + SOFF + kw * BLOCK;
       f32x16 s[2];
-      {
-        i32x4 kf[2][KSQ][2];
-        static_for<2>([&](auto A_) {
-          constexpr int a = decltype(A_)::value;
-          static_for<KSQ>([&](auto KS_) {
-            constexpr int ks = decltype(KS_)::value;
-            kf[a][ks][0] = lds_read_b128<a * 32 * D>(base + ka[ks][0]);
-            kf[a][ks][1] = lds_read_b128<a * 32 * D>(base + ka[ks][1]);
-          });
-        });
-        static_for<2>([&](auto A_) {
-          constexpr int a = decltype(A_)::value;
-          lds_wait<(1 - a) * 2 * KSQ>();
-          static_for<KSQ>([&](auto KS_) {
-            constexpr int ks = decltype(KS_)::value;
-            lds_use(kf[a][ks][0]);
-            lds_use(kf[a][ks][1]);
-            i32x8 kop = __builtin_shufflevector(kf[a][ks][0], kf[a][ks][1], 0, 1, 2, 3, 4, 5, 6, 7);
-            if constexpr (ks == 0) {
-              f32x16 zero;
-#pragma unroll
-              for (int r = 0; r < 16; r++) zero[r] = 0.f;
-              s[a] = mfma_f8<FMT>(kop, qf[0], zero);
-            } else {
-              s[a] = mfma_f8<FMT>(kop, qf[ks], s[a]);
-            }
-          });
-        });
-      }
+      scores(s, base);
       // V^T operands of the first O^T tiles while the softmax runs
       i32x4 vf[DT][2];
       static_for<DT>([&](auto C_) {
@@ -200,20 +231,7 @@ __global__ __launch_bounds__(NW * 64, NW == 4 && D <= 128 ? 2 : 1) void attn_fwd
         vf[c][1] = lds_read_b128<c * 32 * 64>(base + va[1]);
       });
       // ---- online softmax; register r of tile a is key 32a + 16g + r of this lane's query row
-      if (j >= wave_first_masked) {
-        const int qrow = row0 + l32;
-#pragma unroll
-        for (int a = 0; a < 2; a++)
-#pragma unroll
-          for (int r = 0; r < 16; r++)
-            if (j * BN + a * 32 + g * 16 + r > qrow) s[a][r] = -INFINITY;
-      }
-      float mx = s[0][0];
-#pragma unroll
-      for (int a = 0; a < 2; a++)
-#pragma unroll
-        for (int r = 0; r < 16; r++) mx = fmaxf(mx, s[a][r]);
-      mx = pair_max(mx);
+      const float mx = row_max(s, blk);
       const float m_new = fmaxf(m_i, mx * qk_scale);
       if (__builtin_amdgcn_ballot_w64(m_new > m_i + RESCALE_LOG2) != 0) {
         const float alpha = fast_exp2(m_i - m_new);
@@ -259,6 +277,43 @@ __global__ __launch_bounds__(NW * 64, NW == 4 && D <= 128 ? 2 : 1) void attn_fwd
     if (j + 1 < nsteps) step(j + 1, std::integral_constant<int, 1>{});
   }
 
+  // ---- the groups' partial results into the first group's waves (the K/V stages are free)
+  if constexpr (KW > 1) {
+    constexpr int PER = DT * 16 + 2;   // floats per lane: accumulator, maximum, sum
+    LDS_PTR(float) const part = (LDS_PTR(float))lds;
+    if (kw > 0) {
+      LDS_PTR(float) to = part + ((kw - 1) * QW + qw) * (PER * 64) + lane;
+#pragma unroll
+      for (int c = 0; c < DT; c++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) to[(c * 16 + r) * 64] = oacc[c][r];
+      to[(PER - 2) * 64] = m_i;
+      to[(PER - 1) * 64] = l_i;
+    }
+    __syncthreads();
+    if (kw > 0) return;
+    float top = m_i;
+#pragma unroll
+    for (int w = 1; w < KW; w++) top = fmaxf(top, part[((w - 1) * QW + qw) * (PER * 64) + (PER - 2) * 64 + lane]);
+    const float own = fast_exp2(m_i - top);
+    l_i *= own;
+#pragma unroll
+    for (int c = 0; c < DT; c++)
+#pragma unroll
+      for (int r = 0; r < 16; r++) oacc[c][r] *= own;
+#pragma unroll
+    for (int w = 1; w < KW; w++) {
+      LDS_PTR(float) from = part + ((w - 1) * QW + qw) * (PER * 64) + lane;
+      const float f = fast_exp2(from[(PER - 2) * 64] - top);
+      l_i += f * from[(PER - 1) * 64];
+#pragma unroll
+      for (int c = 0; c < DT; c++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) oacc[c][r] += f * from[(c * 16 + r) * 64];
+    }
+    m_i = top;
+  }
+
   // ---- epilogue: O = acc / l rounded to the fp8 type, M = m + log2(l)
   {
     const float l = pair_sum(l_i);
@@ -286,25 +341,31 @@ __global__ __launch_bounds__(NW * 64, NW == 4 && D <= 128 ? 2 : 1) void attn_fwd
   }
 }
 
-template <int FMT, int D, int NW, bool PAD = false>
+template <int FMT, int D, int NW, bool PAD = false, int KW = 1>
 static int launch_fwd8(const AttnArgs& p, hipStream_t stream) {
-  constexpr int BM = NW * 32;
-  constexpr int smem = 2 * 2 * 64 * D;
+  constexpr int BM = NW / KW * 32;
+  constexpr int smem = std::max(2 * 2 * 64 * D * KW, (KW - 1) * (NW / KW) * (D / 32 * 16 + 2) * 256);   // stages, or the partial results
   static bool attr_set = false;
   if (!attr_set) {
-    hipError_t e = hipFuncSetAttribute((const void*)attn_fwd8_kernel<FMT, D, NW, PAD>,
+    hipError_t e = hipFuncSetAttribute((const void*)attn_fwd8_kernel<FMT, D, NW, PAD, KW>,
                                        hipFuncAttributeMaxDynamicSharedMemorySize, smem);
     if (e != hipSuccess) return (int)e;
     attr_set = true;
   }
   const int nqb = (p.N + BM - 1) / BM;
-  attn_fwd8_kernel<FMT, D, NW, PAD><<<dim3(nqb * p.Z * p.H), dim3(NW * 64), smem, stream>>>(deal_blocks(p, nqb));
+  attn_fwd8_kernel<FMT, D, NW, PAD, KW><<<dim3(nqb * p.Z * p.H), dim3(NW * 64), smem, stream>>>(deal_blocks(p, nqb));
   return (int)hipGetLastError();
 }
 
 template <int FMT>
 static int launch_fwd8_fmt(const AttnArgs& p, hipStream_t stream) {
-  // variant 2: eight waves (256 query rows per K/V stream), head_dim 128 only
+  // variant 2: eight waves (256 query rows per K/V stream), head_dim 128 only; groups along the keys: 6 = 64 rows and two, 8 = 128 rows and
+  // two, 7 = 32 rows and four (head_dim 64, N a multiple of 256)
+  if (p.d_real == p.D && p.D == 128 && p.variant == 6) return launch_fwd8<FMT, 128, 4, false, 2>(p, stream);
+  if (p.d_real == p.D && p.D == 128 && p.variant == 8) return launch_fwd8<FMT, 128, 8, false, 2>(p, stream);
+  if (p.d_real == p.D && p.D == 64 && p.variant == 6) return launch_fwd8<FMT, 64, 4, false, 2>(p, stream);
+  if (p.d_real == p.D && p.D == 64 && p.variant == 8) return launch_fwd8<FMT, 64, 8, false, 2>(p, stream);
+  if (p.d_real == p.D && p.D == 64 && p.variant == 7 && p.N % 256 == 0) return launch_fwd8<FMT, 64, 4, false, 4>(p, stream);
   if (p.D == 256) return launch_fwd8<FMT, 256, 4>(p, stream);   // (one workgroup per CU: 128 accumulator registers per lane)
   if (p.D == 128) return p.variant == 2 ? launch_fwd8<FMT, 128, 8>(p, stream) : launch_fwd8<FMT, 128, 4>(p, stream);
   if (p.d_real < p.D) return launch_fwd8<FMT, 64, 4, true>(p, stream);    // head dims 16 / 32

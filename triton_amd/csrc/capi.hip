@@ -1579,6 +1579,28 @@ static int attn_fwd_variant(const AttnArgs& p, int cus) {
   return 2;
 }
 
+// The same for fp8: 1 = 128 rows a workgroup (eight waves along 256 rows are 6 to 12 % slower), and as above 8, 6 and 7 = groups along the keys.
+// us, e5m2, 1 / 6 / 8 / 7; rows per CU in brackets.  The groups' sums differ from the one's as their running maxima do (P has two bits of fraction):
+// by up to 2.2 % of the result without a mask at 4096 keys, 1 % with it at 6144, which is why longer rows without a mask stay.
+static int attn_fwd8_variant(const AttnArgs& p, int cus) {
+  if (p.D == 256 || p.d_real < p.D || p.N < 256 || (!p.causal && p.N > 4096)) return 1;
+  const int64_t rows = (int64_t)p.Z * p.H * p.N;
+  if (p.D == 64) {
+    // mask: 2 x 3840 [30] 37.6 / 22.0 / 31.8 / 15.1, 4 x 6144 [96] 59.6 / 34.7 / 49.1 / 29.2, 8 x 3328 [104] 34.3 / 21.2 / 28.6 / 20.8, 37 x 256 [37] 6.3 / 5.4 /
+    // 6.3 / 5.8; none: 4 x 4096 [64] 41.7 / 24.8 / 34.4 / 22.9, 27 x 1536 [162] 25.9 / 21.1 / 25.1 / 28.1
+    if (p.N % 256 == 0 && p.N >= 512 && rows <= (p.causal ? 96ll : 64ll) * cus) return 7;
+    // mask: 17 x 2432 [162] 27.7 / 19.9 / 23.9, 83 x 512 [166] 9.3 / 8.5 / 9.3, 71 x 1024 [284] 16.3 / 15.8 / 16.2, 143 x 640 [358] 13.7 / 14.3 / 14.7, 61 x
+    // 2048 [488] 38.3 / 37.2 / 35.5; none: 39 x 1152 [176] 20.8 / 17.3 / 19.9, 78 x 256 [78] 6.2 / 6.4 / 6.4, 211 x 384 [316] 13.0 / 13.4 / 14.5
+    if (rows <= 64ll * cus || (rows <= (p.causal ? 200ll : 180ll) * cus && p.N >= (p.causal ? 256 : 640)) || (p.causal && rows <= 300ll * cus && p.N >= 1024)) return 6;
+    return p.causal && rows <= 560ll * cus && p.N >= 1536 ? 8 : 1;
+  }
+  // mask: 2 x 2560 [20] 32.7 / 21.4 / 27.3, 63 x 384 [94] 9.5 / 8.5 / 9.6, 6 x 4992 [117] 59.9 / 40.7 / 48.2, 61 x 640 [152] 13.5 / 14.6 / 14.0, 35 x 2048
+  // [280] 33.4 / 35.8 / 39.8; none: 5 x 2944 [58] 38.1 / 25.3 / 31.5, 31 x 640 [78] 11.9 / 12.2 / 11.6, 6 x 3968 [93] 51.2 / 44.3 / 41.4, 18 x 1664 [117]
+  // 24.3 / 22.8 / 21.6, 17 x 2944 [196] 58.9 / 67.7 / 64.7
+  if (rows <= 64ll * cus || (p.causal && rows <= 128ll * cus && p.N >= 384)) return 6;
+  return !p.causal && rows <= 128ll * cus && p.N >= 1024 ? 8 : 1;
+}
+
 int mi355_attn_fwd(const void* q, const void* k, const void* v, void* o, float* Mlse,
                    int Z, int H, int N_CTX, int D,
                    const int64_t* sq, const int64_t* sk, const int64_t* sv, const int64_t* so,
@@ -1599,7 +1621,7 @@ int mi355_attn_fwd(const void* q, const void* k, const void* v, void* o, float* 
       return MI355_ESTRIDE;
     p.q = (const char*)q; p.k = (const char*)k; p.v = (const char*)v; p.o = (char*)o; p.lse = Mlse;
     p.sm_scale = sm_scale; p.causal = causal != 0;
-    p.variant = knob(knobs().attn_fwd_variant, 1);  // fp8: four waves, two workgroups per CU (eight waves measured 6-12 % slower)
+    p.variant = knob(knobs().attn_fwd_variant, attn_fwd8_variant(p, device_info().cus > 0 ? device_info().cus : 256));
     return attn_fwd8_launch(p, dtype == MI355_F8E5M2, (hipStream_t)stream_);
   }
   int rc = attn_common(p, Z, H, N_CTX, D, dtype);
