@@ -93,7 +93,7 @@ enum {
  * Same arguments as the kernel: three pointers, M N K, six strides (any strides are accepted;
  * the tiled MFMA kernels need a unit stride on one axis of each operand and rows that start on 16-byte boundaries -
  * either layout of B for every type; K a multiple of 16 bytes, N any size when a row-major B's pitch covers N rounded up
- * to 16 bytes -, anything else runs a slower MFMA kernel of 64x64 tiles with masked element loads), plus ACTIVATION.  in_dtype is the type of A and B
+ * to 16 bytes; fp16 and bf16: rows of whole dwords, an even K of 8 and more and an even N of a row-major B, do too -, anything else runs a slower MFMA kernel of 64x64 tiles with masked element loads), plus ACTIVATION.  in_dtype is the type of A and B
  * (they must match, python/triton/language/semantic.py:1355): fp16, bf16, fp8e4nv, fp8e5 or fp32.  fp32 operands are
  * multiplied exactly on the fp32 MFMAs (the `ieee` input precision of `tl.dot`, semantic.py:1322-1410; what the
  * reference's CPU path computes, python/triton/runtime/interpreter.py:542-549) when A's rows and B's columns are
@@ -125,7 +125,7 @@ int mi355_gemm(const void* A, const void* B, void* C,
  * take ceil(tiles / programs) tiles each as one stream of K steps)
  * (a kernel that does not exist for the dtype or shape falls back to the nearest one).  group_m: the
  * reference's GROUP_SIZE_M (:265-273), 0 = default 8.  Operands without 16-byte rows run the
- * masked any-stride kernel whatever `tile` says.
+ * masked any-stride kernel whatever `tile` says, 16-bit ones with rows of whole dwords the ring or the four-wave kernels.
  */
 int mi355_gemm_tuned(const void* A, const void* B, void* C,
                      int M, int N, int K,
@@ -158,8 +158,8 @@ int mi355_gemm_splitk(const void* A, const void* B, void* C,
                       int activation, int splits, void* workspace, size_t workspace_bytes, void* stream);
 
 /* mi355_gemm_epilogue with a workspace, for products that gain from one: operands whose rows are not whole 16-byte chunks
- * (K or N not a multiple of the vector width, odd pitches, unaligned bases) are copied into padded rows first - one
- * launch for both, zeros beyond K, where the reference masks its loads (python/tutorials/03-matrix-multiplication.py:297-298) -
+ * (K or N not a multiple of the vector width, odd pitches, unaligned bases) and not 16-bit rows of whole dwords that run as fast in place are
+ * copied into padded rows first - one launch for both, zeros beyond K, where the reference masks its loads (python/tutorials/03-matrix-multiplication.py:297-298) -
  * and few tiles with a long K are split as by mi355_gemm_splitk.  mi355_gemm_workspace says how many bytes such a product
  * wants (0: none, the plain call); give mi355_gemm_ws that many, 256-byte aligned, contents irrelevant, used until the
  * launches of the call have run.  workspace_bytes = 0 and softmax = 1 run as mi355_gemm_epilogue.
@@ -288,7 +288,7 @@ int mi355_grouped_gemm(const void* d_a_ptrs, const void* d_b_ptrs, const void* d
 
 /* The same from tables in HOST memory, read before the call returns (they travel as a kernel argument, so nothing is copied
  * to the device first): `a`, `b`, `c` are arrays of device addresses, `sizes` and `lds` as above.  One launch for up to 64
- * problems, with tile sizes chosen per problem; problems without 16-byte rows, or whose rows of A or B overlap (a row stride below
+ * problems, with one tile size chosen for the group; problems without 16-byte rows, or whose rows of A or B overlap (a row stride below
  * the row's length, 0 for one row repeated), share a second launch.
  * num_programs > 0 caps the workgroups of a launch.
  */

@@ -306,7 +306,7 @@ bool short_k(int M, int N, int k_bytes, bool b_kmajor, int cus) {
   return M % 128 == 0 && N % 128 == 0 && k_bytes <= 256 && tiles * 2 > cus;
 }
 
-// Operands as the ring kernels want them, on top of what every tile kernel asks (16-byte chunks): 16-bit with either layout
+// Operands as the ring kernels want them, on top of what every tile kernel asks (16-byte chunks, or dword_rows): 16-bit with either layout
 // of B, fp8 with a K-major one.
 bool ring_ok(int elem_bytes, bool b_kmajor) { return elem_bytes == 2 || (elem_bytes == 1 && b_kmajor); }
 
@@ -880,7 +880,7 @@ static bool rowfused(int M, int N, int K, int in_dtype) {
 }
 
 // ---- mi355_gemm_ws: how a product with a workspace runs.  Operands whose rows the MFMA kernels cannot load (rows that are not
-// whole 16-byte chunks) are first copied into rows of a padded pitch, both in one launch, zeros behind K; few tiles with a
+// whole 16-byte chunks nor, in 16 bits, whole dwords) or only at more than the copies' cost are first copied into rows of a padded pitch, both in one launch, zeros behind K; few tiles with a
 // long K are split.  The any-stride kernel stays where the copies would cost more than they gain.
 namespace {
 

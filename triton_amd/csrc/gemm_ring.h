@@ -483,12 +483,12 @@ __device__ __forceinline__ void gemm_ring_tile(const GemmArgs& p, const int pm, 
     if constexpr (MX) load4_sbase(ts, scale_base(bs) + kfull / RING_ROW * 4 * SD, scale_rows(bs));
     fill(true);
     const i32x4 zero = {0, 0, 0, 0};
-    // (landed, all of them: from here on branches may move them)
-#pragma unroll
-    for (int q = 0; q < LA; q++) lds_use(ta[q]);
-#pragma unroll
-    for (int q = 0; q < LB; q++) lds_use(tb[q]);
     if constexpr (!MX && E::kElemBytes == 2) {
+      // (landed, all of them: from here on branches may move them)
+#pragma unroll
+      for (int q = 0; q < LA; q++) lds_use(ta[q]);
+#pragma unroll
+      for (int q = 0; q < LB; q++) lds_use(tb[q]);
       if (tail & 15) {
 #pragma unroll
         for (int q = 0; q < LA; q++) ta[q] = chunkA[q] * 16 + 16 <= tail ? ta[q] : bytes_down(ta[q], -tail & 15);
@@ -504,10 +504,12 @@ __device__ __forceinline__ void gemm_ring_tile(const GemmArgs& p, const int pm, 
     }
 #pragma unroll
     for (int q = 0; q < LA; q++) {
+      lds_use(ta[q]);
       *(LDS_PTR(i32x4))(uintptr_t)(lds0 + (wave * LA + q) * 1024 + lane * 16) = chunkA[q] * 16 < tail ? ta[q] : zero;
     }
 #pragma unroll
     for (int q = 0; q < LB; q++) {
+      lds_use(tb[q]);
       const bool in = B_KMAJOR ? rowB[q] * 16 < tail : rowB[q] < krows;
       *(LDS_PTR(i32x4))(uintptr_t)(lds0 + A_BYTES + (wave * LB + q) * 1024 + lane * 16) = in ? tb[q] : zero;
     }
