@@ -202,12 +202,12 @@ double ring_rounds_us(int M, int N, int steps, int cus, int shape) {
 // multiplies, which four stages with a CU to themselves pay for in every tile.  us, before / so: bf16 K-major 3200 x 3072 x 192 19.6 / 11.4, 3456 x 1664 x 256
 // 11.1 / 8.2, row-major B 1408 x 6784 x 192 19.4 / 11.9, 3840 x 5376 x 448 37.7 / 27.0, 8064 x 2048 x 576 32.4 / 26.5; e4m3 1536 x 4224 x 640 13.0 / 10.8, 4352 x 5888
 // x 384 28.5 / 25.0; MXFP4 6400 x 4224 x 768 34.3 / 24.2, 2432 x 4992 x 1280 22.4 / 16.9, MXFP8 4224 x 4992 x 384 30.1 / 18.6.  A long K hides the waits anyway, and
-// two stages less of the latency: K-major 3712 x 4736 x 1920 63.7 / 77.4, e4m3 5376 x 2304 x 2048 26.0 / 33.6, MXFP8 3584 x 3968 x 4352 60.7 / 89.2; up to a round of tiles
+// two stages less of the latency: K-major 3712 x 4736 x 1920 63.7 / 77.4, e4m3 5376 x 2304 x 2048 26.0 / 33.6, MXFP8 3584 x 3968 x 4352 60.7 / 89.2, 3543 x 5760 x 4736 117 / 125 (block-scaled products of more than sixteen steps are left out); up to a round of tiles
 // a workgroup is alone either way: 1024 x 3712 x 768 9.5 / 10.2.  (150 products of 200 .. 3000 tiles and 2 .. 40 steps: within 6 % rms, block-scaled 12.)
 // `apart`: rows that do not begin on 128-byte lines (K-major bf16 2048 x 7808 x 984 37.8 / 44.0).  `epilogue`: us a round for what C takes beyond plain stores.
 double pairs_us(int M, int N, int steps, int cus, bool mx, bool apart, double epilogue = 0.0) {
   const long tiles = (long)((M + 127) / 128) * ((N + 127) / 128), rounds = (tiles + cus - 1) / cus;
-  if (tiles <= cus) return 1e30;
+  if (tiles <= cus || (mx && steps > 16)) return 1e30;
   const double k = (apart ? 1.5 : 1.0) * steps;
   return mx ? 1.2 + (double)rounds * (1.9 + 0.6 * k) : 1.2 + (0.8 * rounds + 0.2 * tiles / cus) * (2.0 + epilogue + 0.45 * k);
 }
