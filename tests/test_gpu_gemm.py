@@ -1763,6 +1763,30 @@ def test_large_products_of_rows_on_dwords(gpu, M, N, K, kmajor):
     assert torch.equal(triton_amd.matmul(a, b, out_dtype=torch.float32), a.float() @ b.float())
 
 
+@pytest.mark.parametrize("tile", [8, 9, 10, 12, 13])
+@pytest.mark.parametrize("kmajor", [False, True])
+def test_each_cause_of_rows_on_dwords_has_the_ring_kernels_of_its_own(gpu, monkeypatch, tile, kmajor):
+    # whole chunks but for one thing: the end of K, a pitch, a base.  NaN between and around the rows, whole numbers: exact, with and without splits
+    set_knob(monkeypatch, "MI355_GEMM_TILE", tile)
+    lib, stream, M, N = _lib.load(), torch.cuda.current_stream().cuda_stream, 200, 136
+    g = torch.Generator(device=gpu).manual_seed(tile)
+    for K, columns, pad_a, pad_b, at_a, at_b in ((512, N, 0, 0, 0, 0), (514, N, 6, 6 if kmajor else 0, 0, 0), (512, N, 2, 0, 0, 0), (512, N, 0, 4, 0, 0),
+                                                 (512, N, 0, 0, 2, 0), (512, N, 0, 0, 0, 6), (512, N - 2, 0, 2, 0, 4)):
+        def operand(rows, cols, pad, at):
+            room = torch.full((at + rows * (cols + pad) + 8,), float("nan"), device=gpu, dtype=torch.bfloat16)
+            x = room[at:at + rows * (cols + pad)].view(rows, cols + pad)[:, :cols]
+            return x.copy_(torch.randint(-1, 2, (rows, cols), device=gpu, generator=g))
+
+        a, b = operand(M, K, pad_a, at_a), operand(*((columns, K) if kmajor else (K, columns)), pad_b, at_b)
+        bt = b.t() if kmajor else b
+        want, ws = a.float() @ bt.float(), torch.full((2 * M * N,), float("nan"), device=gpu)
+        for splits in (1, 2):
+            c = torch.full((M, columns), float("nan"), device=gpu)
+            rc = lib.mi355_gemm_splitk(a.data_ptr(), b.data_ptr(), c.data_ptr(), M, columns, K, a.stride(0), 1, *bt.stride(), columns, 1, _lib.BF16, _lib.F32,
+                                       None, None, _lib.ACT_NONE, splits, ws.data_ptr(), 8 * M * N, stream)
+            assert rc == 0 and torch.equal(c, want), (K, columns, pad_a, pad_b, at_a, at_b, splits)
+
+
 @pytest.mark.parametrize("dtype", ["fp16", "bf16", "e4m3"])
 def test_rings_of_two_stages_at_their_edges_are_bit_exact(gpu, dtype, monkeypatch):
     test_ring_kernels_at_the_edges_of_their_ring_are_bit_exact(gpu, dtype, 13, monkeypatch)

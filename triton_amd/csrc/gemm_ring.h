@@ -253,12 +253,12 @@ constexpr int ring_stage_bytes() { return (BM + BN) * (RING_ROW + 4 * E::kScaleD
 
 // Tile (pm, pn) of the product p with the ring of NS stages at LDS address lds0 (NS * (BM + BN) * 128 bytes).  A has whole
 // 16-byte chunks along K (k_bytes in all) and a K-major B too; a row-major B (16-bit types) has p.K rows of whole 16-byte chunks: in
-// the last chunk's place of A's rows there may be zeros beyond K.  16-bit types: dwords instead of chunks will do (8 elements at least),
-// for the rows' begin as for their length - a direct load moves 16 bytes from any dword on, as fast as from rows of 16-byte but not 128-byte
+// the last chunk's place of A's rows there may be zeros beyond K.  DWORDS (16-bit types): dwords instead of chunks will do (8 elements at
+// least), for the rows' begin as for their length - a direct load moves 16 bytes from any dword on, as fast as from rows of 16-byte but not 128-byte
 // pitch (bf16 2048^3, rows of 2048 / 2056 / 2050 elements 18.6 / 24.5 / 24.4 us, 1024^3 8.1 / 8.2 / 8.3).  Block-scaled: both operands K-major, K a
 // multiple of 128 elements, scale rows that begin on dwords.  Every wave's
 // fragments are in registers when the last step's MFMAs begin, so a caller that runs another tile needs one barrier first.
-template <typename E, int BM, int BN, int WN, bool B_KMAJOR, int NS>
+template <typename E, int BM, int BN, int WN, bool B_KMAJOR, int NS, bool DWORDS = false>
 __device__ __forceinline__ void gemm_ring_tile(const GemmArgs& p, const int pm, const int pn, const unsigned lds0) {
 #if MI355_DEVICE_PASS
   using Op = typename E::Operand;
@@ -266,6 +266,7 @@ __device__ __forceinline__ void gemm_ring_tile(const GemmArgs& p, const int pm, 
   constexpr int SD = E::kScaleDwords;
   constexpr bool MX = SD > 0;
   static_assert(B_KMAJOR || (E::kElemBytes == 2 && BN >= 64), "row-major B: 16-bit types, pieces of 128 bytes and more");
+  static_assert(!DWORDS || E::kElemBytes == 2, "rows on dwords: 16-bit types");
   static_assert((BM == 64 || BM == 128) && (BN == 32 || BN == 64 || BN == 128), "tile sizes");
   constexpr int NW = 2 * WN, TM = BM / 2, TN = BN / WN, MT = TM / 16, NT = TN / 16;
   constexpr int A_BYTES = BM * RING_ROW, S_BYTES = (BM + BN) * RING_ROW, STAGE = ring_stage_bytes<E, BM, BN>();
@@ -281,7 +282,7 @@ __device__ __forceinline__ void gemm_ring_tile(const GemmArgs& p, const int pm, 
   // (a step that a row-major B ends inside is a tail too, a whole one where A's padding fills it: B has no rows to load there)
   // (and so is one that holds the last row of a row-major B whose rows end inside a chunk: nothing may be read behind that row)
   const int rest = p.k_bytes % RING_ROW;
-  const bool open_rows = !B_KMAJOR && p.N % 8 != 0 && ((p.ldb | (int64_t)(uintptr_t)p.B) & 15) != 0;
+  const bool open_rows = DWORDS && !B_KMAJOR && p.N % 8 != 0 && ((p.ldb | (int64_t)(uintptr_t)p.B) & 15) != 0;
   const int tail = !B_KMAJOR && rest == 0 && (open_rows || p.K * E::kElemBytes < p.k_bytes) ? RING_ROW : rest;
   const int steps = (p.k_bytes + RING_ROW - 1) / RING_ROW;
   constexpr int KROWS = RING_ROW / 2;                        // k rows of a row-major B per step
@@ -460,7 +461,7 @@ __device__ __forceinline__ void gemm_ring_tile(const GemmArgs& p, const int pm, 
     int past[LB];
 #pragma unroll
     for (int q = 0; q < LB; q++) past[q] = 0;
-    if (!B_KMAJOR && open_rows) {
+    if (open_rows) {
       constexpr int CPR = BN / 8, RPI = 64 / CPR;
 #pragma unroll
       for (int q = 0; q < LB; q++) {
@@ -483,7 +484,7 @@ __device__ __forceinline__ void gemm_ring_tile(const GemmArgs& p, const int pm, 
     if constexpr (MX) load4_sbase(ts, scale_base(bs) + kfull / RING_ROW * 4 * SD, scale_rows(bs));
     fill(true);
     const i32x4 zero = {0, 0, 0, 0};
-    if constexpr (!MX && E::kElemBytes == 2) {
+    if constexpr (DWORDS) {
       // (landed, all of them: from here on branches may move them)
 #pragma unroll
       for (int q = 0; q < LA; q++) lds_use(ta[q]);
@@ -497,7 +498,7 @@ __device__ __forceinline__ void gemm_ring_tile(const GemmArgs& p, const int pm, 
           for (int q = 0; q < LB; q++) tb[q] = rowB[q] * 16 + 16 <= tail ? tb[q] : bytes_down(tb[q], -tail & 15);
         }
       }
-      if (!B_KMAJOR && open_rows) {
+      if (open_rows) {
 #pragma unroll
         for (int q = 0; q < LB; q++) tb[q] = past[q] > 0 ? bytes_down(tb[q], -2 * p.N & 15) : tb[q];
       }
@@ -591,7 +592,7 @@ __device__ __forceinline__ void gemm_ring_tile(const GemmArgs& p, const int pm, 
 
 // Splits of K: workgroup z * tiles + t multiplies the K bytes [z * chunk, z * chunk + chunk) of tile t into slice z of the
 // workspace (chunk: whole K steps; 0 = no split).
-template <typename E, int BM, int BN, int WN, bool B_KMAJOR, int NS>
+template <typename E, int BM, int BN, int WN, bool B_KMAJOR, int NS, bool DWORDS>
 __global__ __launch_bounds__(128 * WN, 1) void gemm_ring_kernel(GemmArgs p, int chunk_bytes) {
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   const int num_m = (p.M + BM - 1) / BM, num_n = (p.N + BN - 1) / BN, tiles = num_m * num_n;
@@ -611,21 +612,21 @@ __global__ __launch_bounds__(128 * WN, 1) void gemm_ring_kernel(GemmArgs p, int 
   }
   int pm, pn;
   grouped_tile(xcd_remap(t, tiles), num_m, num_n, p.group_m, pm, pn);
-  gemm_ring_tile<E, BM, BN, WN, B_KMAJOR, NS>(p, pm, pn, lds_addr((LDS_PTR(char))smem));
+  gemm_ring_tile<E, BM, BN, WN, B_KMAJOR, NS, DWORDS>(p, pm, pn, lds_addr((LDS_PTR(char))smem));
 }
 
-template <typename E, int BM, int BN, int WN, bool B_KMAJOR, int NS>
+template <typename E, int BM, int BN, int WN, bool B_KMAJOR, int NS, bool DWORDS = false>
 static int launch_gemm_ring(const GemmArgs& p, int splits, int chunk_bytes, hipStream_t stream) {
   constexpr int smem = NS * ring_stage_bytes<E, BM, BN>();
   static_assert(smem <= 160 * 1024, "LDS ring does not fit");
   static bool attr_set = false;  // benign race: setting the attribute twice is harmless
   if (!attr_set) {
-    hipError_t e = hipFuncSetAttribute((const void*)gemm_ring_kernel<E, BM, BN, WN, B_KMAJOR, NS>, hipFuncAttributeMaxDynamicSharedMemorySize, smem);
+    hipError_t e = hipFuncSetAttribute((const void*)gemm_ring_kernel<E, BM, BN, WN, B_KMAJOR, NS, DWORDS>, hipFuncAttributeMaxDynamicSharedMemorySize, smem);
     if (e != hipSuccess) return (int)e;
     attr_set = true;
   }
   const int tiles = ((p.M + BM - 1) / BM) * ((p.N + BN - 1) / BN);
-  gemm_ring_kernel<E, BM, BN, WN, B_KMAJOR, NS><<<dim3(tiles * splits), dim3(128 * WN), smem, stream>>>(p, splits > 1 ? chunk_bytes : 0);
+  gemm_ring_kernel<E, BM, BN, WN, B_KMAJOR, NS, DWORDS><<<dim3(tiles * splits), dim3(128 * WN), smem, stream>>>(p, splits > 1 ? chunk_bytes : 0);
   return (int)hipGetLastError();
 }
 

@@ -4,17 +4,25 @@
 namespace mi355 {
 
 namespace {
-template <typename E, bool KM>
+template <typename E, bool KM, bool DWORDS>
 int launch(const GemmArgs& p, int shape, int splits, int chunk_bytes, hipStream_t stream) {
   switch (shape) {
-    case 0: return launch_gemm_ring<E, 128, 128, 2, KM, 4>(p, splits, chunk_bytes, stream);
-    case 4: return launch_gemm_ring<E, 128, 128, 2, KM, 2>(p, splits, chunk_bytes, stream);
-    case 1: return launch_gemm_ring<E, 128, 64, 2, KM, 4>(p, splits, chunk_bytes, stream);
+    case 0: return launch_gemm_ring<E, 128, 128, 2, KM, 4, DWORDS>(p, splits, chunk_bytes, stream);
+    case 4: return launch_gemm_ring<E, 128, 128, 2, KM, 2, DWORDS>(p, splits, chunk_bytes, stream);
+    case 1: return launch_gemm_ring<E, 128, 64, 2, KM, 4, DWORDS>(p, splits, chunk_bytes, stream);
     case 3:
-      if constexpr (KM) return launch_gemm_ring<E, 64, 32, 2, true, 8>(p, splits, chunk_bytes, stream);
+      if constexpr (KM) return launch_gemm_ring<E, 64, 32, 2, true, 8, DWORDS>(p, splits, chunk_bytes, stream);
       return (int)hipErrorInvalidValue;
-    default: return launch_gemm_ring<E, 64, 64, 2, KM, 4>(p, splits, chunk_bytes, stream);
+    default: return launch_gemm_ring<E, 64, 64, 2, KM, 4, DWORDS>(p, splits, chunk_bytes, stream);
   }
+}
+
+// Rows on dwords have kernels of their own: what the ends of their rows take in the prologue made the launches of whole chunks next to a
+// row-major B 1 to 2 % longer.  us, one kernel for both / two: fp16 256^3 4.09 / 4.00, 512^3 4.59 / 4.52, 768 x 2944 x 384 7.95 / 7.75, 2048 x 512 x 4096 16.9 / 16.7.
+template <typename E, bool KM>
+int launch(const GemmArgs& p, int shape, int splits, int chunk_bytes, hipStream_t stream) {
+  const bool chunks = ((p.k_bytes | p.lda | p.ldb | (int64_t)(uintptr_t)p.A | (int64_t)(uintptr_t)p.B) & 15) == 0;
+  return chunks ? launch<E, KM, false>(p, shape, splits, chunk_bytes, stream) : launch<E, KM, true>(p, shape, splits, chunk_bytes, stream);
 }
 
 // Grouped GEMM (python/tutorials/08-grouped-gemm.py:64-140: row-major A, B and C of one type) with the problem table as a
