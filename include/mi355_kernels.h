@@ -288,7 +288,7 @@ int mi355_grouped_gemm(const void* d_a_ptrs, const void* d_b_ptrs, const void* d
 
 /* The same from tables in HOST memory, read before the call returns (they travel as a kernel argument, so nothing is copied
  * to the device first): `a`, `b`, `c` are arrays of device addresses, `sizes` and `lds` as above.  One launch for up to 64
- * problems, with one tile size chosen for the group; problems without 16-byte rows, or whose rows of A or B overlap (a row stride below
+ * problems, with tile sizes chosen for the group; problems without 16-byte rows, or whose rows of A or B overlap (a row stride below
  * the row's length, 0 for one row repeated), share a second launch.
  * num_programs > 0 caps the workgroups of a launch.
  */

@@ -256,6 +256,23 @@ def test_groups_checked_in_native_code_are_the_python_function_s(gpu, monkeypatc
     assert Dispatch.seen > 0
 
 
+@pytest.mark.parametrize("run", [None, 0, 1, 16])
+@pytest.mark.parametrize("shape", [0, 2, 4, 5])
+def test_every_form_of_a_group_in_every_order_is_bit_exact_on_integers(gpu, monkeypatch, shape, run):
+    # tiles of either size, in two stages, of both sizes in one launch; eighths for the XCDs, runs of one and of sixteen tiles, the form's own choice; one
+    # tile and more than CUs, partial tiles, several tiles a program.  Whole numbers up to 4096: exact in fp32, rounded once
+    set_knob(monkeypatch, "MI355_GROUPED_SHAPE", shape)
+    if run is not None:
+        set_knob(monkeypatch, "MI355_GROUPED_RUN", run)
+    for sizes in ([(1, 8, 8)], [(1800, 1800, 136), (40, 72, 1032), (300, 1104, 520), (65, 640, 64), (1, 8, 2048), (129, 136, 8)]):
+        g = torch.Generator(device=gpu).manual_seed(shape)
+        a = [torch.randint(-1, 2, (m, k), device=gpu, generator=g).half() for m, n, k in sizes]
+        b = [torch.randint(-1, 2, (k, n), device=gpu, generator=g).half() for m, n, k in sizes]
+        for nprog in (0, 1, 100):
+            for x, y, c in zip(a, b, triton_amd.group_gemm_fn(a, b, num_programs=nprog)):
+                assert torch.equal(c, (x.float() @ y.float()).half()), (x.shape, y.shape, nprog)
+
+
 @pytest.mark.parametrize("nprog", [0, 7])
 @pytest.mark.parametrize("sizes", [
     [(m, 256, 3072) for m in (1, 130, 65, 300)],                          # 64x64 tiles

@@ -53,7 +53,7 @@ const DeviceInfo& device_info() {
 // UNSET = the variable is absent or empty and the call site's own default applies.
 constexpr int UNSET = INT_MIN;
 struct Knobs {
-  int force_strided, group_m, tile, programs, skinny, grouped_big_min, grouped_wave128_min_k, grouped_chunk,
+  int force_strided, group_m, tile, programs, skinny, grouped_big_min, grouped_wave128_min_k, grouped_chunk, grouped_shape, grouped_run,
       attn_fwd_variant, attn_bwd_groups, attn_programs, lean_epilogue, tile_m, rowfused_max_mk, mixed_rows, splitk;
 };
 Knobs g_knobs;
@@ -78,6 +78,8 @@ void load_knobs() {
   k.grouped_big_min = read_env("MI355_GROUPED_BIG_MIN", 1);
   k.grouped_wave128_min_k = read_env("MI355_GROUPED_WAVE128_MIN_K", 0);
   k.grouped_chunk = read_env("MI355_GROUPED_CHUNK", 1);
+  k.grouped_shape = read_env("MI355_GROUPED_SHAPE", 0);   // of group_plan: 0, 2, 4 or 5 (others: its choice)
+  k.grouped_run = read_env("MI355_GROUPED_RUN", 0);       // tiles that an XCD takes at a time (0: an eighth of all)
   k.attn_fwd_variant = read_env("MI355_ATTN_FWD_VARIANT", 0);
   k.attn_bwd_groups = read_env("MI355_ATTN_BWD_GROUPS", 0);   // dQ groups + 16 * dK/dV groups
   k.attn_programs = read_env("MI355_ATTN_PROGRAMS", 1);
@@ -212,37 +214,70 @@ double pairs_us(int M, int N, int steps, int cus, bool mx, bool apart, double ep
   return mx ? 1.2 + (double)rounds * (1.9 + 0.6 * k) : 1.2 + (0.8 * rounds + 0.2 * tiles / cus) * (2.0 + epilogue + 0.45 * k);
 }
 
-// A group on ring tiles of one shape (0, 2 or 4), its problems in `order`, the longest K first.  us: all tiles' time spread over the CUs, or what the CU
-// with the most tiles of the first problems has, or one tile of the longest K (60 drawn groups of 2 .. 16 problems: within 13 % rms; the shape chosen by it is
-// within 1 % of the best of the three in the geometric mean).
-// chunk: the order of the tiles.  An eighth of them for each XCD, one after the other, keeps the operands in its L2; but where the first eighth has the tiles of
-// the longest K, one XCD works when the others are done: then runs of `chunk` tiles are dealt to the XCDs in turn.  us, eighths / runs: ten problems
-// of 64 .. 1792 rows and K of 64 .. 2048 22.4 / 17.2 (64x64), 64 .. 1600 23.3 / 16.9, 25.3 / 16.3 (128x128); one K for all, 2304 -> 256 24.5 / 26.9, 1024 -> 1280 14.5 / 17.0;
-// no more tiles than CUs, K of 256 .. 1792 7.3 / 7.6.
-struct GroupPlan { double us; int chunk; int64_t tiles; };
-GroupPlan group_plan(const int32_t* sizes, const int* order, int n, int shape, int cus) {
-  static const struct { int edge, slots, chunk; double base, tile_us, step_us, most, lone_us, lone_step_us; } kShapes[3] = {
-      {128, 1, 8, 1.5, 4.5, 0.49, 0.82, 1.35, 0.33}, {64, 1, 16, 3.5, 0.78, 0.227, 0.68, 0.6, 0.128}, {128, 2, 8, 2.6, 2.3, 0.58, 0.89, 1.0, 0.65}};
-  const auto& t = kShapes[shape / 2];
-  auto steps = [&](int i) { return (sizes[3 * order[i] + 2] + 63) / 64; };
-  auto count = [&](int i) {
-    const int32_t* s = sizes + 3 * order[i];
-    return (int64_t)((s[0] + t.edge - 1) / t.edge) * ((s[1] + t.edge - 1) / t.edge);
-  };
-  double sum = 0.0, longest = t.lone_us + t.lone_step_us * steps(0);
-  int64_t tiles = 0;
+// A group on the ring kernels, its problems in `order`, the longest K first: which tiles (0 = 128x128, 2 = 64x64, 4 = 128x128 in two stages, 5 = each
+// problem on 0 or 2 by its cost) and in which order.
+// chunk: an eighth of the tiles for each XCD, one after the other (0), keeps the operands in its L2; but where the first eighth has the tiles of
+// the longest K, one XCD works when the others are done: then runs of `chunk` tiles are dealt to the XCDs in turn.
+// us, eighths | runs, of shapes 2 / 0 / 4 / 5: twelve problems of 80 .. 1904 rows and K of 88 .. 1832 27.5 / 31.5 / 25.7 / 31.6 | 14.3 / 18.8 / 24.0 / 19.0,
+// seven of 192 .. 2048, K of 128 .. 2048 40.3 / 30.9 / 30.2 / 31.8 | 24.5 / 21.5 / 27.5 / 21.7; twelve of 64 .. 1792, K of 64 .. 768 11.1 / 10.9 / 12.8 / 9.0 |
+// 10.8 / 11.2 / 13.0 / 9.3; seven 512 -> 4096 31.2 / 28.8 / 23.0 / 29.7 | 31.2 / 29.3 / 23.7 / 29.0; seven of 20 .. 1110 x 872 x 664 15.1 / 11.7 / 13.1 / 11.9 | 17.7 / 12.9
+// / 14.4 / 13.0; nine of 21 .. 1686 x 448 x 1088 10.5 / 12.7 / 15.9 / 12.8 | 12.0 / 13.1 / 17.3 / 13.1.
+// The estimate of each (1360 drawn groups of 2 .. 16 problems: within 9 to 12 % rms) is base + the largest of one tile of the longest K (`lone`) and, w : 1 - w, of what
+// the CU with the most tiles of the first problems has (most, `slots` workgroups a CU) and all tiles' time spread over the CUs, or over those of the first XCD;
+// `runs`: what their misses in the L2 cost.  Another form than the one of least cost, in eighths, has to be estimated 5 % shorter: of those groups
+// three are then more than 2 % slower than by cost alone, none more than 4 %, and in the geometric mean they are 1.18 times as fast (12, 17 % and 1.18 without that
+// margin); the best of the eight forms is 1.4 % ahead of the one taken.
+struct GroupPlan { int shape, chunk; uint64_t small_tiles; };   // small_tiles: the problems on 64x64, a bit for each of `order`
+GroupPlan group_plan(const int32_t* sizes, const int* order, int n, int cus, int forced) {
+  struct Tile { double us, step_us; };
+  static const struct { int shape, slots, chunk; double base; Tile large, small; double most, w, lone, lone_step, runs; } kForms[4] = {
+      {2, 2, 16, 3.06, {0.0, 0.0}, {0.97, 0.258}, 0.72, 0.376, 0.64, 0.13, 1.11}, {0, 1, 8, 3.2, {3.92, 0.594}, {0.0, 0.0}, 0.68, 0.541, 2.02, 0.31, 1.09},
+      {4, 2, 8, 2.36, {2.14, 0.634}, {0.0, 0.0}, 1.24, 0.559, 2.96, 0.2, 1.11}, {5, 1, 8, 3.52, {3.63, 0.565}, {1.2, 0.235}, 0.77, 0.55, 0.0, 0.15, 1.08}};
+  // Which shape costs least: all tiles' time (at the rates of ring_plan with several rounds under way) over the CUs, one tile at least.
+  double steps[GroupedTable::kMax], tiles64[GroupedTable::kMax], tiles128[GroupedTable::kMax];
+  double all[3] = {0.0, 0.0, 0.0}, top[3] = {0.0, 0.0, 0.0};   // on 64x64, on 128x128, each on the better one
+  uint64_t better64 = 0;
   for (int i = 0; i < n; i++) {
-    const double us = t.tile_us + t.step_us * steps(i);
-    tiles += count(i);
-    sum += (double)count(i) * us;
-    longest = std::max(longest, t.most * us * (double)((tiles + t.slots * cus - 1) / (t.slots * cus)));
+    const int32_t* s = sizes + 3 * order[i];
+    steps[i] = (s[2] + 63) / 64;
+    tiles64[i] = (double)((s[0] + 63) / 64) * ((s[1] + 63) / 64);
+    tiles128[i] = (double)((s[0] + 127) / 128) * ((s[1] + 127) / 128);
+    const double one64 = 0.6 + 0.195 * steps[i], one128 = 2.5 + 0.5 * steps[i], us64 = one64 * tiles64[i], us128 = one128 * tiles128[i];
+    const bool small = us64 <= us128;
+    if (small) better64 |= 1ull << i;
+    all[0] += us64; all[1] += us128; all[2] += small ? us64 : us128;
+    top[0] = std::max(top[0], one64); top[1] = std::max(top[1], one128); top[2] = std::max(top[2], small ? one64 : one128);
   }
-  double first = 0.0, left = (double)tiles / 8;
-  for (int i = 0; i < n && left > 0.0; i++) {
-    first += std::min((double)count(i), left) * (t.tile_us + t.step_us * steps(i));
-    left -= (double)count(i);
+  for (int e = 0; e < 3; e++) all[e] = std::max(all[e] / cus, top[e]);
+  const int least = all[0] <= all[1] && all[0] <= all[2] ? 2 : all[1] <= all[2] ? 0 : 5;
+  auto small_of = [&](int shape) { return shape == 2 ? ~0ull : shape == 5 ? better64 : 0ull; };
+
+  GroupPlan best{least, 0, small_of(least)};
+  double best_us = 1e30, least_us = 1e30;
+  for (const auto& f : kForms) {
+    if (forced >= 0 && f.shape != forced) continue;
+    const uint64_t small = small_of(f.shape);
+    const double slots = f.slots * cus;
+    double eighth = 0.0, tiles = 0.0, sum = 0.0, most = 0.0, first = 0.0;
+    for (int i = 0; i < n; i++) eighth += small >> i & 1 ? tiles64[i] : tiles128[i];
+    eighth *= 0.125;
+    for (int i = 0; i < n; i++) {
+      const bool s = small >> i & 1;
+      const double us = s ? f.small.us + f.small.step_us * steps[i] : f.large.us + f.large.step_us * steps[i], count = s ? tiles64[i] : tiles128[i];
+      first += us * std::max(0.0, std::min(count, eighth - tiles));
+      tiles += count;
+      sum += count * us;
+      most = std::max(most, f.most * us * (double)((int64_t)((tiles - 1.0) / slots) + 1));
+    }
+    const double lone = f.lone + f.lone_step * steps[0];
+    auto blend = [&](double spread) { return std::max(lone, f.w * most + (1.0 - f.w) * spread / cus); };
+    const double eighths = f.base + blend(std::max(sum, 8 * first)), runs = f.base + f.runs * blend(sum);
+    if (f.shape == least) least_us = eighths;
+    // (both tile sizes in eighths where one of them costs less: estimated shorter, but 17.2 -> 20.7 and 22.5 -> 26.3)
+    if (eighths < best_us && (f.shape != 5 || least == 5 || forced >= 0)) { best = {f.shape, 0, small}; best_us = eighths; }
+    if (runs < best_us) { best = {f.shape, f.chunk, small}; best_us = runs; }
   }
-  return {t.base + std::max(sum / cus, longest), tiles > cus && first > 1.15 * sum / 8 ? t.chunk : 0, tiles};
+  return best_us < 0.95 * least_us ? best : GroupPlan{least, 0, small_of(least)};
 }
 
 // The same for the kernels of 256-column tiles with `rows` rows of C each (gemm_wave128.hip; edges: the eight-wave kernel, for
@@ -1274,25 +1309,23 @@ int mi355_grouped_gemm_host(const void* const* a, const void* const* b, void* co
     } else {
       // the longest tiles first, so that the last ones to be started are short
       std::stable_sort(order, order + n, [&](int x, int y) { return sizes[3 * (g0 + x) + 2] > sizes[3 * (g0 + y) + 2]; });
-      GroupPlan plan{1e30, 0, 0};
-      int shape = 0;
-      for (int candidate : {2, 0, 4}) {
-        const GroupPlan x = group_plan(sizes + 3 * g0, order, n, candidate, cus);
-        if (x.us < plan.us) { plan = x; shape = candidate; }
-      }
-      if (plan.tiles > INT_MAX / 2) return MI355_ESHAPE;
-      const int edge = shape == 2 ? 64 : 128;
-      int tiles = 0;
+      const int forced = knobs().grouped_shape;
+      GroupPlan plan = group_plan(sizes + 3 * g0, order, n, cus, forced == 0 || forced == 2 || forced == 4 || forced == 5 ? forced : -1);
+      plan.chunk = std::min(knob(knobs().grouped_run, plan.chunk), 1024);
+      int64_t tiles = 0;
       for (int at = 0; at < n; at++) {
         put(ga, at, order[at]);
-        ga.first_tile[at] = tiles;
-        tiles += ((ga.sizes[3 * at] + edge - 1) / edge) * ((ga.sizes[3 * at + 1] + edge - 1) / edge);
+        ga.first_tile[at] = (int)tiles;
+        const int edge = plan.small_tiles >> at & 1 ? 64 : 128;
+        tiles += (int64_t)((ga.sizes[3 * at] + edge - 1) / edge) * ((ga.sizes[3 * at + 1] + edge - 1) / edge);
+        if (tiles > INT_MAX / 2) return MI355_ESHAPE;
       }
       for (int at = n; at < G; at++) ga.first_tile[at] = INT_MAX;
-      ga.total_tiles = tiles;
+      ga.total_tiles = (int)tiles;
+      ga.small_tiles = plan.small_tiles;
       ga.chunk = plan.chunk;
-      ga.padded_tiles = plan.chunk > 0 ? (tiles + 8 * plan.chunk - 1) / (8 * plan.chunk) * (8 * plan.chunk) : tiles;
-      rc = gemm_ring_grouped_launch(ga, bf16, shape, num_programs > 0 ? std::min(num_programs, tiles) : ga.padded_tiles, stream);
+      ga.padded_tiles = plan.chunk > 0 ? (ga.total_tiles + 8 * plan.chunk - 1) / (8 * plan.chunk) * (8 * plan.chunk) : ga.total_tiles;
+      rc = gemm_ring_grouped_launch(ga, bf16, plan.shape, num_programs > 0 ? std::min(num_programs, ga.total_tiles) : ga.padded_tiles, stream);
     }
     if (rc) return rc;
   }

@@ -33,8 +33,8 @@ int launch(const GemmArgs& p, int shape, int splits, int chunk_bytes, hipStream_
 // works, the group 1024^3, 512^3, 256^3, 128^3 took 112 us a call, 25 of them on 85 tiles of 128x128; now 8, one launch of
 // 340 tiles of 64x64.  Larger ones run on 128x128 tiles, in four stages or, more of them than CUs, in two with two
 // workgroups on a CU (group_plan): us on 64x64 / 128x128 / those pairs, eleven experts 2304 -> 256 of 35 .. 1464 rows 35.0 / 33.4 / 24.5,
-// 272 -> 3248 18.0 / 28.7 / 39.9, 1024 -> 1280 19.4 / 14.5 / 18.2.  (Small and large tiles in one launch, each problem on what costs it less:
-// never far ahead, 20.4 for 15.2 where its 64x64 tiles had 128x128 ones' LDS and a CU to themselves.)
+// 272 -> 3248 18.0 / 28.7 / 39.9, 1024 -> 1280 19.4 / 14.5 / 18.2.  EDGE 0: both sizes in one launch, each problem on what costs it less, the 64x64
+// tiles with the LDS of 128x128 ones and a CU to themselves: six problems of 64 .. 1984 x 72 .. 1448 and K of 96 .. 1552 17.3 / 16.1 / 20.7 / 13.4.
 template <typename E, int EDGE, int NS>
 __global__ __launch_bounds__(256, 1) void gemm_ring_grouped_kernel(GroupedTable ga) {
   extern __shared__ __attribute__((aligned(1024))) char smem[];
@@ -57,8 +57,11 @@ __global__ __launch_bounds__(256, 1) void gemm_ring_grouped_kernel(GroupedTable 
     p.scn = 1; p.out_dtype = ga.out_dtype;
     p.c_vec_ok = p.ldc % 4 == 0 && (uintptr_t)p.C % 16 == 0;
     int pm, pn;
-    grouped_tile(tile, (p.M + EDGE - 1) / EDGE, (p.N + EDGE - 1) / EDGE, 8, pm, pn);
-    gemm_ring_tile<E, EDGE, EDGE, 2, false, NS>(p, pm, pn, lds0);
+    const int edge = EDGE > 0 ? EDGE : (ga.small_tiles >> gi) & 1 ? 64 : 128;
+    grouped_tile(tile, (p.M + edge - 1) / edge, (p.N + edge - 1) / edge, 8, pm, pn);
+    if constexpr (EDGE > 0) gemm_ring_tile<E, EDGE, EDGE, 2, false, NS>(p, pm, pn, lds0);
+    else if (edge == 64) gemm_ring_tile<E, 64, 64, 2, false, NS>(p, pm, pn, lds0);
+    else gemm_ring_tile<E, 128, 128, 2, false, NS>(p, pm, pn, lds0);
     wait_vmcnt<0>();   // (the stores: the next tile counts its loads)
     block_barrier();   // the next tile's loads overwrite the stages
   }
@@ -66,7 +69,7 @@ __global__ __launch_bounds__(256, 1) void gemm_ring_grouped_kernel(GroupedTable 
 
 template <typename E, int EDGE, int NS>
 int launch_grouped(const GroupedTable& ga, int nprog, hipStream_t stream) {
-  constexpr int smem = NS * 2 * EDGE * RING_ROW;
+  constexpr int smem = NS * 2 * (EDGE > 0 ? EDGE : 128) * RING_ROW;
   static bool attr_set = false;
   if (!attr_set) {
     hipError_t e = hipFuncSetAttribute((const void*)gemm_ring_grouped_kernel<E, EDGE, NS>, hipFuncAttributeMaxDynamicSharedMemorySize, smem);
@@ -80,6 +83,7 @@ int launch_grouped(const GroupedTable& ga, int nprog, hipStream_t stream) {
 template <typename E>
 int launch_grouped(const GroupedTable& ga, int shape, int nprog, hipStream_t stream) {
   if (shape == 2) return launch_grouped<E, 64, 4>(ga, nprog, stream);
+  if (shape == 5) return launch_grouped<E, 0, 4>(ga, nprog, stream);
   return shape == 4 ? launch_grouped<E, 128, 2>(ga, nprog, stream) : launch_grouped<E, 128, 4>(ga, nprog, stream);
 }
 }  // namespace

@@ -152,6 +152,7 @@ struct GroupedTable {
   int sizes[kMax * 3];
   int lds[kMax * 3];
   int first_tile[kMax];    // ring and masked kernels: number of the problem's first tile (past the last problem: 2^31 - 1)
+  uint64_t small_tiles;    // ring kernel of both tile sizes: problems on tiles of 64x64, bit per problem (the others: 128x128)
   int group_size;
   int out_dtype;
   int total_tiles;
@@ -161,7 +162,7 @@ struct GroupedTable {
 static_assert(sizeof(GroupedTable) <= 3584, "a kernel's arguments are at most 4 KiB");
 
 int gemm_wave128_grouped_table_launch(const GroupedTable& ga, bool bf16, int nprog, hipStream_t stream);   // whole 256x256 tiles, K as in grouped_plan
-int gemm_ring_grouped_launch(const GroupedTable& ga, bool bf16, int shape, int nprog, hipStream_t stream);   // shape: 0, 2 or 4 of the ring kernels
+int gemm_ring_grouped_launch(const GroupedTable& ga, bool bf16, int shape, int nprog, hipStream_t stream);   // shape: 0, 2 or 4 of the ring kernels, 5 = each problem on 0 or 2
 int gemm_masked_grouped_launch(const GroupedTable& ga, bool bf16, hipStream_t stream);   // tiles of 64x64, any row strides
 
 int gemm16_grouped_launch(const GroupedArgs& ga, bool bf16, int nprog, int nprog_big, hipStream_t stream);
