@@ -1,0 +1,59 @@
+"""Which kernels calls run, read from a trace of their launches: the choices whose reasons stand beside the rules of capi.hip."""
+import re
+
+import pytest
+import torch
+
+import triton_amd
+from util import set_knob
+
+pytestmark = pytest.mark.gpu
+
+
+def launches(call):
+    """[(kernel, its numeric template arguments)] of a call's launches."""
+    call()   # (the first one sets attributes)
+    torch.cuda.synchronize()
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as trace:
+        call()
+        torch.cuda.synchronize()
+    found = []
+    for event in trace.events():
+        kernel = re.search(r"mi355.*?(?<![a-z_])([a-z][a-z0-9_]*_kernel)", event.name)
+        if kernel is None:
+            continue
+        rest = event.name[kernel.end():]
+        numbers = re.findall(r"L[ib](\d+)E", rest) if event.name.startswith("_Z") else re.findall(r"\b(\d+|true|false)\b", rest.rsplit(">(", 1)[0])
+        found.append((kernel.group(1), tuple({"true": 1, "false": 0}.get(n) if n in ("true", "false") else int(n) for n in numbers)))
+    assert found, [event.name for event in trace.events()]
+    return found
+
+
+def whole(gpu, *shape):
+    return torch.randint(-1, 2, shape, device=gpu, generator=torch.Generator(device=gpu).manual_seed(sum(shape)))
+
+
+def product(gpu, dtype, M, N, K, kmajor, add=False):
+    """The launches of a product of whole numbers, which has to be exact."""
+    tdt = {"bf16": torch.bfloat16, "e4m3": torch.float8_e4m3fn}[dtype]
+    a, b = whole(gpu, M, K).to(tdt), (whole(gpu, N, K) if kmajor else whole(gpu, K, N)).to(tdt)
+    bt, row, got = b.t() if kmajor else b, whole(gpu, N).to(torch.bfloat16) if add else None, []
+    names = launches(lambda: got.append(triton_amd.matmul(a, bt, out_dtype=torch.bfloat16, **({"add": row} if add else {}))))
+    want = a.float() @ bt.float()
+    want = (want + row.float() if add else want).bfloat16()
+    assert all(torch.equal(c, want) for c in got)
+    return names
+
+
+def two_stages(names):
+    # (template arguments of the ring kernels: the operands' type, then BM, BN, WN, K-major B, stages, rows on dwords)
+    return [numbers[-6:-3] + numbers[-2:-1] for name, numbers in names if name == "gemm_ring_kernel"] == [(128, 128, 2, 2)]
+
+
+@pytest.mark.parametrize("dtype,M,N,K,kmajor,ring", [
+    ("e4m3", 2560, 3712, 64, True, False), ("e4m3", 2432, 3456, 192, True, False), ("e4m3", 4096, 1664, 320, True, False), ("e4m3", 3200, 2176, 128, True, False),
+    ("bf16", 2944, 3456, 32, False, False), ("bf16", 1950, 4480, 64, False, False), ("bf16", 2304, 2432, 32, True, False),
+    ("e4m3", 2432, 3456, 256, True, True), ("bf16", 2304, 2432, 128, True, True), ("bf16", 1642, 3586, 128, True, True)])
+def test_half_filled_steps_of_a_short_k_stay_on_the_kernel_of_64_byte_steps(gpu, dtype, M, N, K, kmajor, ring):
+    names = product(gpu, dtype, M, N, K, kmajor)
+    assert two_stages(names) if ring else [name for name, _ in names] == ["gemm_kernel"], names

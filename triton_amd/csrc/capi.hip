@@ -341,6 +341,18 @@ bool short_k(int M, int N, int k_bytes, bool b_kmajor, int cus) {
   return M % 128 == 0 && N % 128 == 0 && k_bytes <= 256 && tiles * 2 > cus;
 }
 
+// Which of those products of more tiles than CUs stay on that kernel: its steps are 64 bytes long, the rings' 128, so that where half of the last one would be empty, or
+// there are few anyway, it is ahead - with whole columns of tiles, since edges there cost it more.  us, that kernel / rings of two stages, by K bytes: e4m3 5120 x 3712 x 64
+// 13.1 / 16.8, 4096 x 2304 x 64 9.1 / 11.1, 2432 x 3456 x 192 9.9 / 11.2, 4096 x 1664 x 320 8.6 / 9.7, 2944 x 5888 x 128 15.0 / 16.0; fp16 768 x 6400 x 64 6.3 / 6.7; the
+// time ratio, 100 products of each type, e4m3 64 0.84, 128 0.97, 192 0.92, 256 1.04, 320 0.91, 384 1.04; row-major B 64 0.90, 128 0.99, 192 0.93, 256 1.06, 320 0.98; K-major 64
+// 0.90, 128 1.02, 144 1.03, 192 0.95, 256 1.09, 320 1.0.  Other N: e4m3 64 0.92 above two rounds, else 1.04 and more.
+bool one_barrier_ahead(int M, int N, int k_bytes, bool is8, bool b_kmajor, int cus) {
+  const long tiles = (long)((M + 127) / 128) * ((N + 127) / 128);
+  if (N % 128 != 0) return is8 && k_bytes <= 64 && tiles > 2 * cus;
+  if (is8) return k_bytes <= 192 || (k_bytes > 256 && k_bytes <= 320);
+  return b_kmajor ? k_bytes <= 64 || (k_bytes > 160 && k_bytes <= 192) : k_bytes <= 192;
+}
+
 // Operands as the ring kernels want them, on top of what every tile kernel asks (16-byte chunks, or dword_rows): 16-bit with either layout
 // of B, fp8 with a K-major one.
 bool ring_ok(int elem_bytes, bool b_kmajor) { return elem_bytes == 2 || (elem_bytes == 1 && b_kmajor); }
@@ -562,7 +574,7 @@ PartChoice part_choice(const GemmArgs& p, const TileChoice& c, int es, bool b_km
                        p.activation == MI355_ACT_NONE && (tiles256 > cus || tiles256 * 2 <= cus) && p.k_bytes <= (tiles256 > cus || !b_kmajor ? 384 : 320);
   const bool pairs_ok = !by_knob && knobs().tile_m == UNSET && knobs().mixed_rows == UNSET && ring_ok(es, b_kmajor);
   if (!by_knob && (tile != 6 || partial) && !p.aux && p.c_vec_ok && short_k(M, N, p.k_bytes, b_kmajor, cus)) {   // (its addends and odd rows of C cost more)
-    if (pairs_ok && (long)((M + 127) / 128) * ((N + 127) / 128) > cus) r.ring = 4;
+    if (pairs_ok && (long)((M + 127) / 128) * ((N + 127) / 128) > cus && !one_barrier_ahead(M, N, p.k_bytes, is8, b_kmajor, cus)) r.ring = 4;
     else r.tile = 1;
   }
   else if (tile == 1 && by_knob) r.ring = 0;
