@@ -57,3 +57,9 @@ def two_stages(names):
 def test_half_filled_steps_of_a_short_k_stay_on_the_kernel_of_64_byte_steps(gpu, dtype, M, N, K, kmajor, ring):
     names = product(gpu, dtype, M, N, K, kmajor)
     assert two_stages(names) if ring else [name for name, _ in names] == ["gemm_kernel"], names
+
+
+@pytest.mark.parametrize("dtype,M,N,K,ring", [("e4m3", 1344, 6144, 2944, False), ("e4m3", 4782, 1792, 2944, False), ("bf16", 2304, 3648, 384, False), ("bf16", 3085, 2804, 704, False),
+                                              ("e4m3", 1536, 4224, 640, True), ("bf16", 3456, 1664, 256, True)])
+def test_two_stage_rings_are_taken_where_they_gain(gpu, dtype, M, N, K, ring):
+    assert two_stages(product(gpu, dtype, M, N, K, True)) == ring

@@ -593,11 +593,16 @@ PartChoice part_choice(const GemmArgs& p, const TileChoice& c, int es, bool b_km
     const Cut cut = best_cut(M, N, steps, cus, tile, r.ring, is8);
     if (cut.us < (tile == 1 ? 0.88 : 0.92) * std::min(plan_us, other)) r.cut = cut;
     // (an addend: fp16 3799 x 2304 x 512 23.2 / 23.7, row-major B 3840 x 6016 x 64, on the eight-wave kernel, 35.9 / 25.0; rows of C that are no whole groups of four:
-    // K-major 1468 x 4405 x 128 13.2 / 10.7; both, 2176 x 4234 x 256 18.3 / 19.3)
-    const double epilogue = (p.aux ? 2.2 : 0.0) + (p.c_vec_ok ? 0.0 : 2.0);
+    // K-major 1468 x 4405 x 128 13.2 / 10.7; both, 2176 x 4234 x 256 18.3 / 19.3; rows that do not begin on 16 bytes, K-major 3085 x 2804 x 704 21.5 / 23.8, 4204 x 2012 x 640 21.3 / 22.8)
+    const double epilogue = (p.aux ? 2.2 : 0.0) + (p.c_vec_ok && p.ldc % 8 == 0 ? 0.0 : 2.0);
     const double added = p.aux && tile != 1 ? (tile == 6 ? 2.8 : 6.5) * (double)(((long)((M + rows - 1) / rows) * ((N + 255) / 256) + cus - 1) / cus) : 0.0;
+    // What the two-stage rings are compared with is shorter than `other` says on 192 and 128 rows (0.91 .. 0.97 and 0.83 .. 0.95 of it, 60 products: K-major 2304 x 3648 x 384
+    // 14.6 / 16.7), and for two steps on the eight-wave fp8 kernel with whole columns of tiles (1920 x 7680 x 64 10.5 / 12.9, 4608 x 3584 x 64 10.8 / 13.4); fp8 of more
+    // than twenty steps is not worth the risk of either estimate (1344 x 6144 x 2944 33.8 / 39.7).  1472 drawn products that could run on either are 1.043 times as fast
+    // as without these rings, seven of them more than 5 % slower and none 10 % (17 without these factors).
+    const double shorter = tile == 6 ? (rows == 192 ? 0.95 : rows == 128 ? 0.9 : 1.0) : is8 && steps <= 2 && N % 256 == 0 ? 0.75 : 1.0;
     const double rings = plan_us + epilogue * (double)((M + 127) / 128) * ((N + 127) / 128) / cus;
-    if (pairs_ok && pairs_us(M, N, steps, cus, false, (p.lda | p.ldb) % 128 != 0, epilogue) < 0.97 * std::min({rings, other + added, r.cut.us})) {
+    if (pairs_ok && !(is8 && steps > 20) && pairs_us(M, N, steps, cus, false, (p.lda | p.ldb) % 128 != 0, epilogue) < 0.97 * std::min({rings, shorter * other + added, r.cut.us})) {
       r.ring = 4;
       r.cut = {M, N, 1e30};
     }
