@@ -63,3 +63,10 @@ def test_half_filled_steps_of_a_short_k_stay_on_the_kernel_of_64_byte_steps(gpu,
                                               ("e4m3", 1536, 4224, 640, True), ("bf16", 3456, 1664, 256, True)])
 def test_two_stage_rings_are_taken_where_they_gain(gpu, dtype, M, N, K, ring):
     assert two_stages(product(gpu, dtype, M, N, K, True)) == ring
+
+
+@pytest.mark.parametrize("M,N,K,kmajor,copied", [
+    (2154, 5428, 6548, True, True), (7454, 2496, 4234, True, True), (4390, 1838, 1838, False, True), (7258, 1110, 120, False, False),
+    (1024, 1030, 1026, True, False), (771, 2608, 1460, True, False), (1646, 6920, 214, True, False), (4095, 4100, 4100, False, False)])
+def test_rows_on_dwords_are_copied_where_that_is_shorter(gpu, M, N, K, kmajor, copied):
+    assert any(name == "repack_kernel" for name, _ in product(gpu, "bf16", M, N, K, kmajor)) == copied

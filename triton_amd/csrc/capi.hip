@@ -1017,12 +1017,14 @@ GemmRoute gemm_route(const void* A, const void* B, int M, int N, int K, int64_t 
   const bool one_barrier = !ring_ok(es, r.kmajor) && K >= (in_dtype == MI355_F8E4M3 ? 65 : 256);
   const double other = one_barrier ? 5.3 + 0.34 * (double)rounds128 * ((K + 63) / 64) : ring;
   const double any = std::min(other, tiles256_us(tiles256, 256, steps, cus, M < 256 || N < 256, es == 1));
-  // What rows that do not begin on 128-byte lines add to a kernel's time, a line being fetched in two pieces, against the copies: 70 drawn products of
-  // such rows either way, and these in the probe of both, bf16, us, pitch a multiple of 128 bytes / 4 bytes more: 256x256 tiles, row-major B 4096^3 103 / 109, 8192^3
-  // 747 / 790, K-major 101 / 112, 721 / 830; ring tiles 1024^3 8.1 / 8.3, 2048^3 18.6 / 24.4, 1024 x 4096 x 4096 32 / 39.  Ring tiles: 0.4 of a step for each
-  // operand, so that a short K stays (copied / in place: 684 x 1113 x 1554 15.4 / 8.3, 2732 x 426 x 972 15.3 / 9.7, 1349 x 5067 x 276 26 / 21) and a long one is copied
-  // (1282 x 604 x 6798 31.2 / 34.3, 3246 x 818 x 4286 41.4 / 45.9).  256-row tiles: 0.08 of their time, K-major 0.11 (5506 x 7021 x 2926 219 / 242, 2472 x 4042 x 1030
-  // 40.1 / 36.3), and a K that is not whole pairs of steps runs on no others (1581 x 7168 x 5428 146 / 169).
+  // What rows that do not begin on 128-byte lines add to a kernel's time, a line being fetched in two pieces, against the copies.  In the probe of both, bf16, us, pitch
+  // a multiple of 128 bytes / 4 bytes more: 256x256 tiles, row-major B 4096^3 103 / 109, 8192^3 747 / 790, K-major 101 / 112, 721 / 830; ring tiles 1024^3 8.1 / 8.3, 2048^3
+  // 18.6 / 24.4, 1024 x 4096 x 4096 32 / 39.  Ring tiles: 0.4 of a step for each operand, below 24 steps 0.24 (copied / in place: 684 x 1113 x 1554 15.4 / 8.3, 2732 x 426 x 972
+  // 15.3 / 9.7, 771 x 2608 x 1460 21 / 13.8, 1349 x 5067 x 276 26 / 21; a long K is copied, 1282 x 604 x 6798 31.2 / 34.3).  256-row tiles: 0.08 of their time, K-major
+  // 0.11 (5506 x 7021 x 2926 219 / 242, 2472 x 4042 x 1030 40.1 / 36.3); a K that is not whole pairs of steps runs on no others (1581 x 7168 x 5428 146 / 169), nor as one stream
+  // over several rounds, and with 24 steps and more and both operands so a round that they leave unfilled costs up to half of that again (2154 x 5428 x 6548, 198
+  // tiles, 175 / 215, 7454 x 2496 x 4234, 300, 199 / 240; row-major B 4390 x 1838 x 1838, 144, 59 / 73).  2387 drawn products of such rows are 1.30 times as fast as all
+  // copied, eight of them more than 5 % slower and none 10 % (without that term 18, ten of them by up to 23 %).
   const bool loose_a = a_line && !a_ok, loose_b = b_line && !(r.kmajor ? bk_ok : bn_ok);
   bool loose = false;
   if (loose_a || loose_b) {
@@ -1033,13 +1035,17 @@ GemmRoute gemm_route(const void* A, const void* B, int M, int N, int K, int64_t 
       const int s = auto_splits(M, N, (int64_t)K * es, in_dtype, r.kmajor, true, cus), shape = ring_plan(M, N, steps, cus, s, s).shape;
       const int bm = shape == 2 ? 64 : 128, bn = shape == 0 ? 128 : 64;
       const double rounds = std::max(1.0, (double)((M + bm - 1) / bm) * ((N + bn - 1) / bn) * s / cus);
-      lines = (loose_a + loose_b) * 0.4 * (shape == 0 ? 0.42 : shape == 1 ? 0.265 : 0.165) * ((steps + s - 1) / s) * rounds;
+      lines = (loose_a + loose_b) * (steps < 24 && !launch ? 0.24 : 0.4) * (shape == 0 ? 0.42 : shape == 1 ? 0.265 : 0.165) * ((steps + s - 1) / s) * rounds;
     } else {
       const double here = M >= 256 && N >= 256 ? std::min(any, best_cut(M, N, steps, cus, 6, -1, false).us) : any;
       double other_rows = here;
       if (K * es % 256 != 0)
         for (int h : {192, 128}) other_rows = std::min(other_rows, tiles256_us((long)((M + h - 1) / h) * ((N + 255) / 256), h, steps, cus, false, false));
-      lines = (loose_a + loose_b) * (r.kmajor ? 0.11 : 0.08) * here + here - other_rows;
+      auto blocks = [](int n) { return n > 256 && n % 256 <= 64 ? n / 256 : (n + 255) / 256; };   // (up to 64 rows or columns more are a call of their own: best_cut)
+      const long tiles = (long)blocks(M) * blocks(N);
+      const double filled = (double)tiles / (double)((tiles + cus - 1) / cus * cus);
+      const double idle = steps >= 24 && K * es % 256 != 0 && loose_a && loose_b ? (r.kmajor ? 0.5 : 0.3) * std::max(0.0, 0.9 - filled) * any : 0.0;
+      lines = (loose_a + loose_b) * ((r.kmajor ? 0.11 : 0.08) * here + idle) + here - other_rows;
     }
     loose = lines <= copies;
   }
