@@ -70,3 +70,12 @@ def test_two_stage_rings_are_taken_where_they_gain(gpu, dtype, M, N, K, ring):
     (1024, 1030, 1026, True, False), (771, 2608, 1460, True, False), (1646, 6920, 214, True, False), (4095, 4100, 4100, False, False)])
 def test_rows_on_dwords_are_copied_where_that_is_shorter(gpu, M, N, K, kmajor, copied):
     assert any(name == "repack_kernel" for name, _ in product(gpu, "bf16", M, N, K, kmajor)) == copied
+
+
+@pytest.mark.parametrize("tile", [8, 9, 10, 13])
+@pytest.mark.parametrize("kmajor", [False, True])
+@pytest.mark.parametrize("M,N,K", [(256, 258, 8), (130, 254, 46)])
+def test_a_tile_that_is_asked_for_runs_rows_on_dwords_of_any_k(gpu, monkeypatch, tile, kmajor, M, N, K):
+    set_knob(monkeypatch, "MI355_GEMM_TILE", tile)
+    K -= K % 4   # (46: 44, no whole chunks)
+    assert [name for name, _ in product(gpu, "bf16", M, N, K, kmajor, add=True)] == ["gemm_ring_kernel"]

@@ -717,7 +717,7 @@ static int gemm_impl(const void* A, const void* B, void* C, int M, int N, int K,
   // Rows of 16-bit elements that begin on dwords: the ring and the four-wave kernels' (`loose`), where no kernel of 16-byte chunks takes the operands
   const bool chunks = a_ok && (b_kmajor16 || b_nmajor);
   const DwordRows rows = dword_rows(A, B, M, N, K, sam, sak, sbk, sbn, es, behind);
-  const bool loose = !chunks && rows.a && (rows.bk || rows.bn) && (k_rows > 0 || !any_stride_ahead(M, N, K, aux != nullptr, device_info().cus > 0 ? device_info().cus : 256));
+  const bool loose = !chunks && rows.a && (rows.bk || rows.bn) && (k_rows > 0 || tile_arg >= 0 || knobs().tile != UNSET || !any_stride_ahead(M, N, K, aux != nullptr, device_info().cus > 0 ? device_info().cus : 256));
   const bool b_kmajor = loose ? rows.bk : b_kmajor16;
   // the tile copies address 256 rows of an operand with 32-bit byte offsets from a 64-bit tile base
   const bool pitch_ok = (int64_t)sam * es < (1 << 23) && (b_kmajor ? (int64_t)sbn * es < (1 << 23) : (int64_t)sbk * es < (1 << 26));
