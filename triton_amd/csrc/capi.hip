@@ -224,9 +224,9 @@ double pairs_us(int M, int N, int steps, int cus, bool mx, bool apart, double ep
 // / 14.4 / 13.0; nine of 21 .. 1686 x 448 x 1088 10.5 / 12.7 / 15.9 / 12.8 | 12.0 / 13.1 / 17.3 / 13.1.
 // The estimate of each (1360 drawn groups of 2 .. 16 problems: within 9 to 12 % rms) is base + the largest of one tile of the longest K (`lone`) and, w : 1 - w, of what
 // the CU with the most tiles of the first problems has (most, `slots` workgroups a CU) and all tiles' time spread over the CUs, or over those of the first XCD;
-// `runs`: what their misses in the L2 cost.  Another form than the one of least cost, in eighths, has to be estimated 5 % shorter: of those groups
-// three are then more than 2 % slower than by cost alone, none more than 4 %, and in the geometric mean they are 1.18 times as fast (12, 17 % and 1.18 without that
-// margin); the best of the eight forms is 1.4 % ahead of the one taken.
+// `runs`: what their misses in the L2 cost.  Another form than the one of least cost, in eighths, has to be estimated 2 % shorter: of 1000 other drawn groups 17 are then
+// more than 2 % slower than by cost alone, six more than 5 % and one more than 10, and in the geometric mean they are 1.184 times as fast (5 %: the same 17, 1.182, but 85
+// for 70 groups more than 2 % behind a choice by a coarser estimate of three forms; no margin: 23, nine and one, 1.185); the best of the eight forms is 1 % ahead of the one taken.
 struct GroupPlan { int shape, chunk; uint64_t small_tiles; };   // small_tiles: the problems on 64x64, a bit for each of `order`
 GroupPlan group_plan(const int32_t* sizes, const int* order, int n, int cus, int forced) {
   struct Tile { double us, step_us; };
@@ -277,7 +277,7 @@ GroupPlan group_plan(const int32_t* sizes, const int* order, int n, int cus, int
     if (eighths < best_us && (f.shape != 5 || least == 5 || forced >= 0)) { best = {f.shape, 0, small}; best_us = eighths; }
     if (runs < best_us) { best = {f.shape, f.chunk, small}; best_us = runs; }
   }
-  return best_us < 0.95 * least_us ? best : GroupPlan{least, 0, small_of(least)};
+  return best_us < 0.98 * least_us ? best : GroupPlan{least, 0, small_of(least)};
 }
 
 // The same for the kernels of 256-column tiles with `rows` rows of C each (gemm_wave128.hip; edges: the eight-wave kernel, for
