@@ -79,3 +79,23 @@ def test_a_tile_that_is_asked_for_runs_rows_on_dwords_of_any_k(gpu, monkeypatch,
     set_knob(monkeypatch, "MI355_GEMM_TILE", tile)
     K -= K % 4   # (46: 44, no whole chunks)
     assert [name for name, _ in product(gpu, "bf16", M, N, K, kmajor, add=True)] == ["gemm_ring_kernel"]
+
+
+def attention_launches(gpu, dtype, H, N, D, backward):
+    g = torch.Generator(device=gpu).manual_seed(N)
+    q, k, v = (torch.randn(1, H, N, D, device=gpu, generator=g).half().requires_grad_(backward) for _ in range(3))
+    if dtype == "e5m2":
+        q, k, v = (t.to(torch.float8_e5m2) for t in (q, k, v))
+        v = v.view(torch.uint8).permute(0, 1, 3, 2).contiguous().permute(0, 1, 3, 2).view(torch.float8_e5m2)
+    if not backward:
+        return dict(launches(lambda: triton_amd.attention(q, k, v, True, D ** -0.5)))
+    o = triton_amd.attention(q, k, v, True, D ** -0.5)
+    return dict(launches(lambda: torch.autograd.grad(o, (q, k, v), o.detach(), retain_graph=True)))
+
+
+# groups in dQ and in dK/dV, the last template argument of either
+@pytest.mark.parametrize("H,N,D,groups", [(8, 5248, 64, (2, 2)), (16, 2560, 64, (2, 2)), (16, 4096, 64, (2, 1)), (24, 1536, 64, (2, 1)), (36, 1024, 64, (2, 1)), (24, 4096, 64, (1, 1)),
+                                          (6, 5504, 128, (2, 2)), (13, 2560, 128, (2, 2)), (18, 2048, 128, (1, 1)), (12, 3328, 128, (1, 1))])
+def test_groups_of_the_backward_beyond_one_round_of_cus(gpu, H, N, D, groups):
+    names = attention_launches(gpu, "fp16", H, N, D, True)
+    assert (names["attn_bwd_dq_kernel"][-1], names["attn_bwd_dkdv_kernel"][-1]) == groups

@@ -1730,7 +1730,15 @@ static int attn_bwd_variant(const AttnArgs& p, int cus) {
   // 55.6, 48 x 384 29.0 / 33.1, 12 x 3712 169 / 176
   if (!p.causal) return 1 + 16;
   if (p.N >= (p.D == 64 ? 768 : 1024) && blocks <= cus) return 2 + 32;
-  return p.D == 64 && p.N >= 2560 && blocks * 4 <= cus * 5ll ? 2 + 32 : 1 + 16;
+  // Beyond that round one group each / two in dQ / two in both, the longer the rows the further; head_dim 128: 6 x 5504 219 / 203 / 181, 9 x 4096 174 / 170 / 164,
+  // 13 x 2560 112 / 111 / 107, 14 x 2560 114 / 115 / 114, 12 x 3328 148 / 155 / 156, 18 x 2048 95 / 99 / 101
+  if (p.D == 128) return p.N >= 2560 && blocks * 8 <= cus * 9ll ? 2 + 32 : 1 + 16;
+  // head_dim 64: 14 x 2560 77 / 68 / 65, 16 x 2560 79 / 70 / 70, 14 x 3072 93 / 85 / 85, 8 x 5248 147 / 131 / 125, 7 x 6528 189 / 171 / 168, 9 x 5248 154 / 141 / 142
+  if (p.N >= 2560 && blocks * 20 <= cus * (p.N >= 5120 ? 28ll : 25ll)) return 2 + 32;
+  // 36 x 1024 39.3 / 38.3, 40 x 1024 39.9 / 40.5, 29 x 1280 45.2 / 42.0, 36 x 1280 48.3 / 48.2, 24 x 1536 51.8 / 46.7, 32 x 1536 55.8 / 54.2, 43 x 1536 72.6 / 73.0, 20 x
+  // 2048 65 / 60, 32 x 2048 80.6 / 80.1, 38 x 2048 99 / 100, 16 x 4096 143 / 138, 12 x 6528 264 / 256, 24 x 4096 206 / 208
+  const int64_t tenths = p.N >= 4096 ? 24 : p.N >= 2048 ? 20 : p.N >= 1536 ? 15 : p.N >= 1024 ? 12 : 0;
+  return blocks * 10 <= cus * tenths ? 2 + 16 : 1 + 16;
 }
 
 static int attn_bwd(const void* q, const void* k, const void* v, const void* o, const void* d_o,
