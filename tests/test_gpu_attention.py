@@ -472,3 +472,31 @@ def test_dealt_causal_blocks_are_every_block_once(gpu, monkeypatch, dtype, H, N,
     for h in range(H):
         for a, b in zip(whole, call(slice(h, h + 1))):
             assert torch.equal(a[:, h:h + 1], b), h
+
+
+@pytest.mark.parametrize("form", ["fp8 6", "fp8 8", "fp8 7", "backward 34", "backward 18", "backward 68"])
+@pytest.mark.parametrize("H,N,D", [(24, 1536, 64), (27, 768, 64), (72, 640, 128)])   # (heads that eight XCDs share evenly, unevenly, one by one but for the last)
+def test_dealt_causal_blocks_of_groups_of_waves_are_every_block_once(gpu, monkeypatch, form, H, N, D):
+    # as above where the waves of a block are groups along the keys or the query rows: blocks of 32 and 64 rows, so that fewer heads are dealt
+    kind, variant = form.split()
+    if variant in ("7", "68") and (D != 64 or N % 256 != 0):
+        pytest.skip("four groups: head_dim 64, whole steps of 256 keys")
+    set_knob(monkeypatch, "MI355_ATTN_FWD_VARIANT", variant if kind == "fp8" else "1")
+    set_knob(monkeypatch, "MI355_ATTN_BWD_GROUPS", variant if kind == "backward" else str(1 + 16))
+    g = torch.Generator(device=gpu).manual_seed(N)
+    q, k, v, do = (torch.randn(1, H, N, D, device=gpu, generator=g).half() for _ in range(4))
+    if kind == "fp8":
+        q, k, v = (t.to(torch.float8_e5m2) for t in (q, k, v))
+        v = v.view(torch.uint8).permute(0, 1, 3, 2).contiguous().permute(0, 1, 3, 2).view(torch.float8_e5m2)
+
+    def call(h):
+        ts = [t[:, h] for t in (q, k, v)]
+        if kind == "fp8":
+            return [triton_amd.attention(*ts, True, D ** -0.5).view(torch.uint8)]
+        ts = [t.contiguous().requires_grad_() for t in ts]
+        return torch.autograd.grad(triton_amd.attention(*ts, True, D ** -0.5), ts, do[:, h].contiguous())
+
+    whole = call(slice(0, H))
+    for h in range(H):
+        for a, b in zip(whole, call(slice(h, h + 1))):
+            assert torch.equal(a[:, h:h + 1], b), h

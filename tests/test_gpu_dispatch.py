@@ -99,3 +99,9 @@ def attention_launches(gpu, dtype, H, N, D, backward):
 def test_groups_of_the_backward_beyond_one_round_of_cus(gpu, H, N, D, groups):
     names = attention_launches(gpu, "fp16", H, N, D, True)
     assert (names["attn_bwd_dq_kernel"][-1], names["attn_bwd_dkdv_kernel"][-1]) == groups
+
+
+@pytest.mark.parametrize("H,N,D", [(216, 896, 128), (60, 1024, 128), (154, 1280, 128), (54, 768, 128)])
+def test_short_causal_heads_of_128_columns_run_on_blocks_of_128_rows(gpu, H, N, D):
+    name, numbers = list(attention_launches(gpu, "fp16", H, N, D, False).items())[0]
+    assert name == "attn_fwd_kernel" and numbers == (D, 1, 4, 0, 1)   # (D, tiles and waves, padded, groups)

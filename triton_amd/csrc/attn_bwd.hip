@@ -421,7 +421,7 @@ static int launch_dq(const AttnArgs& p, hipStream_t stream) {
     attr_set = true;
   }
   int nqb = (p.N + BM - 1) / BM;
-  attn_bwd_dq_kernel<V8, D, QT, NW, PAD, KW><<<dim3(nqb * p.Z * p.H), dim3(NW * 64), smem, stream>>>(deal_blocks(p, nqb));
+  attn_bwd_dq_kernel<V8, D, QT, NW, PAD, KW><<<dim3(nqb * p.Z * p.H), dim3(NW * 64), smem, stream>>>(deal_blocks(p, nqb, 2));
   return (int)hipGetLastError();
 }
 

@@ -646,7 +646,7 @@ static int launch_dkdv(const AttnArgs& p, hipStream_t stream) {
     attr_set = true;
   }
   int nkb = (p.N + BN - 1) / BN;
-  attn_bwd_dkdv_kernel<V8, D, NW, PAD, KW><<<dim3(nkb * p.Z * p.H), dim3(NW * 64), smem, stream>>>(deal_blocks(p, nkb));
+  attn_bwd_dkdv_kernel<V8, D, NW, PAD, KW><<<dim3(nkb * p.Z * p.H), dim3(NW * 64), smem, stream>>>(deal_blocks(p, nkb, 2));
   return (int)hipGetLastError();
 }
 

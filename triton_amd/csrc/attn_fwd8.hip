@@ -353,7 +353,7 @@ static int launch_fwd8(const AttnArgs& p, hipStream_t stream) {
     attr_set = true;
   }
   const int nqb = (p.N + BM - 1) / BM;
-  attn_fwd8_kernel<FMT, D, NW, PAD, KW><<<dim3(nqb * p.Z * p.H), dim3(NW * 64), smem, stream>>>(deal_blocks(p, nqb));
+  attn_fwd8_kernel<FMT, D, NW, PAD, KW><<<dim3(nqb * p.Z * p.H), dim3(NW * 64), smem, stream>>>(deal_blocks(p, nqb, 1));
   return (int)hipGetLastError();
 }
 

@@ -747,7 +747,7 @@ static int launch_fwd_pipe(const AttnArgs& p, hipStream_t stream) {
     attr_set = true;
   }
   const int nqb = p.N / BM;
-  attn_fwd_pipe_kernel<S, BF><<<dim3(nqb * p.Z * p.H), dim3(256), smem, stream>>>(deal_blocks(p, nqb));
+  attn_fwd_pipe_kernel<S, BF><<<dim3(nqb * p.Z * p.H), dim3(256), smem, stream>>>(deal_blocks(p, nqb, 2));
   return (int)hipGetLastError();
 }
 

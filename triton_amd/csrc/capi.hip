@@ -1547,6 +1547,7 @@ static int attn_common(AttnArgs& p, int Z, int H, int N_CTX, int D, int dtype) {
   if (!device_info().gfx950) return MI355_EDEVICE;
   // 16 / 32: the 64-column kernels, which pad with zeros on the fly (loads, LDS tiles and stores know d_real)
   p.Z = Z; p.H = H; p.N = N_CTX; p.D = small ? 64 : D; p.d_real = D;
+  p.cus = std::min(device_info().cus > 0 ? device_info().cus : 256, 32767);
   return MI355_OK;
 }
 
@@ -1604,6 +1605,8 @@ static int attn_fwd_variant(const AttnArgs& p, int cus) {
   if (!p.causal) return rows <= 128ll * cus && p.N > 128 ? 8 : dflt;
   // Under the mask, with the blocks dealt by length (deal_blocks).  us, 6 / 8 / 1 / 2 / 4:
   if (p.D == 64) {
+    // (one round of blocks of 256 rows, 104 x 384 9.2 / 8.9 on 1 / 2; 86 x 512 10.7 / 12.4)
+    if (p.N > 256 && p.N <= 384 && rows > 128ll * cus && (int64_t)p.Z * p.H * 2 <= cus) return 2;
     // short rows: 48 x 640 9.4 / 10.3 / 11.1 / 12.6 / 14.6, 77 x 512 14.3 / 11.0 / 10.9 / 13.1 / 14.8, 256 x 512 26.6 / 21.9 / 18.9 / 19.1 / 22.7
     if (p.N < 1024) return rows <= 128ll * cus ? 6 : 1;
     // 14 x 2688 26.1 / 29.8 / 34.2 / 44.6 / 48.0, 24 x 2048 25.7 / 25.8 / 28.8 / 37.3 / 39.8, 25 x 2304 35.2 / 32.3 / 34.2 / 41.3 / 44.3
@@ -1621,6 +1624,10 @@ static int attn_fwd_variant(const AttnArgs& p, int cus) {
   // 125 x 512 39.3 / 26.1 / 21.4 / 20.7 / 22.0
   const int64_t heads = (int64_t)p.Z * p.H, nb = (p.N + 255) / 256, blocks = heads * nb, blocks128 = heads * ((p.N + 127) / 128);
   if (p.N <= 640) return blocks128 <= cus ? (p.N >= 512 ? 8 : 1) : p.N > 256 && blocks <= cus ? 2 : 1;
+  // More than a round of blocks of 128 rows in short heads, where what two rounds by length even out (deal_blocks) is most of a head: 1 / 2 / 4 / 8: 54 x 768 20.0 / 22.5 / 25.9 / 21.5, 60 x 1024
+  // 27.6 / 29.7 / 33.2 / 29.4, 54 x 1152 30.2 / 30.8 / 52.6 / 31.8, 128 x 896 39.2 / 40.7 / 46.9 / 52.8, 216 x 896 60.7 / 77.8 / 87.7 / 82.9, 154 x 1280 79 / 83 / 106 / 99
+  // (few rounds of longer ones stay: 40 x 1024 23.7 on 1, 21.6 on 8, 35 x 1280 28.9 / 25.7)
+  if (p.N <= 1280 && blocks128 * 10 > cus * (p.N < 1024 ? 12ll : 16ll)) return 1;
   // 32 x 2048 60.8 / 44.4 / 47.9 / 52.4 / 56.4, 10 x 4736 92.8 / 74.2 / 88.3 / 98.7 / 106
   if (rows <= 256ll * cus) return 8;
   // 16 x 5248 168 / 139 / 135 / 143 / 175, 30 x 2944 116 / 88.7 / 78.5 / 80.1 / 110; 20 x 5632 237 / 178 / 181 / 166 / 236, 39 x 2560 161 / 92 / 84 / 75 / 112
@@ -1677,7 +1684,7 @@ int mi355_attn_fwd(const void* q, const void* k, const void* v, void* o, float* 
       return MI355_ESTRIDE;
     p.q = (const char*)q; p.k = (const char*)k; p.v = (const char*)v; p.o = (char*)o; p.lse = Mlse;
     p.sm_scale = sm_scale; p.causal = causal != 0;
-    p.variant = knob(knobs().attn_fwd_variant, attn_fwd8_variant(p, device_info().cus > 0 ? device_info().cus : 256));
+    p.variant = knob(knobs().attn_fwd_variant, attn_fwd8_variant(p, p.cus));
     return attn_fwd8_launch(p, dtype == MI355_F8E5M2, (hipStream_t)stream_);
   }
   int rc = attn_common(p, Z, H, N_CTX, D, dtype);
@@ -1692,8 +1699,8 @@ int mi355_attn_fwd(const void* q, const void* k, const void* v, void* o, float* 
   // eight waves (256 query rows) per K/V stream halve the L2 -> LDS traffic.  Under the causal mask
   // their row ranges are uneven, which the persistent form (4) evens out by pairing long and short
   // query blocks per program; without a mask the one-item-per-workgroup form (2) is the faster one.
-  p.variant = knob(knobs().attn_fwd_variant, attn_fwd_variant(p, device_info().cus > 0 ? device_info().cus : 256));
-  p.num_programs = knob(knobs().attn_programs, device_info().cus > 0 ? device_info().cus : 256);
+  p.variant = knob(knobs().attn_fwd_variant, attn_fwd_variant(p, p.cus));
+  p.num_programs = std::min(knob(knobs().attn_programs, p.cus), 32767);
   // 5: four waves of 64 query rows, 16x16x32 MFMAs, software pipelined inside the wave (head_dim 128)
   if (p.variant == 5 && attn_fwd_pipe_ok(p)) return attn_fwd_pipe_launch(p, dtype == MI355_BF16, (hipStream_t)stream_);
   return attn_fwd_launch(p, dtype == MI355_BF16, (hipStream_t)stream_);
@@ -1758,7 +1765,7 @@ static int attn_bwd(const void* q, const void* k, const void* v, const void* o, 
   p.o = (char*)const_cast<void*>(o); p.lse = const_cast<float*>(Mlse); p.delta = delta;
   p.dq = (char*)dq; p.dk = (char*)dk; p.dv = (char*)dv;
   p.sm_scale = sm_scale; p.causal = causal != 0;
-  p.variant = knob(knobs().attn_bwd_groups, attn_bwd_variant(p, device_info().cus > 0 ? device_info().cus : 256));
+  p.variant = knob(knobs().attn_bwd_groups, attn_bwd_variant(p, p.cus));
   return attn_bwd_launch(p, dtype == MI355_BF16, (hipStream_t)stream_);
 }
 

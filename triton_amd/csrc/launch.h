@@ -93,7 +93,8 @@ struct AttnArgs {
   int Z, H, N;
   float sm_scale;
   int64_t sq[4], sk[4], sv[4], so[4];  // element strides
-  int num_programs;  // persistent forward: CUs to fill (0 = one workgroup per item)
+  int16_t num_programs;  // persistent forward: CUs to fill (0 = one workgroup per item)
+  int16_t cus;       // of the device (deal_blocks)
   int16_t causal;
   int16_t variant;  // tiling variant (tuning knob)
   int16_t D;
@@ -108,17 +109,18 @@ static_assert(sizeof(AttnArgs) <= 256, "two cache lines");
 // A launch of `nblk` blocks of rows for every head.  Under the mask the blocks of a head are of different lengths.  Most heads
 // still go one by one, each XCD through heads of its own, so that the blocks that run together share one head's rows in
 // their L2; the last ones go by length over all of them, the longest first, so that the launch ends with short blocks on
-// every CU and no XCD is left with more than another.  That part is four rounds of an XCD's 32 CUs and the heads that
-// eight XCDs do not share evenly.  us, forward and backward, heads in turn / the last two by length / four rounds / all:
-// bf16 10 x 6400 x 128 622 / 496 / 495 / 495 (a head and a quarter for each XCD in turn), fp16 24 x 3072 x 128 336 / 299
-// / 307 / 306, bf16 32 x 4096 x 64 378 / 377 / 347 / 347, 256 x 512 x 128 196 / 195 / 176 / 176, 128 x 4096 x 128 2366 /
-// 2356 / 2353 / 2420 (16 heads at a time in an XCD's L2).  Launches of one block a CU have nothing to even out and keep
-// their heads together (forward, 27 x 1024 x 128 19.1 / - / - / 20.7).
-inline AttnArgs deal_blocks(AttnArgs p, int nblk) {
+// every CU and no XCD is left with more than another.  That part is four rounds of an XCD's CUs and the heads that
+// eight XCDs do not share evenly - two rounds of short heads of 16-bit rows of 128 columns and more, of which its L2 holds few.  us, heads in turn / two rounds / four:
+// head_dim 64, backward 256 x 512 83 / 75 / 68, 64 x 2048 173 / 164 / 149, 32 x 4096 294 / 294 / 265, forward 154 x 1024 41.3 / 41.1 / 35.8; head_dim 128,
+// backward 256 x 384 91 / 87 / 98, 330 x 384 108 / 103 / 124, 216 x 640 146 / 139 / 162, 154 x 896 175 / 161 / 184, but 216 x 512 144 / 126 / 117, 154 x 1024 230 / 214 / 209, 32 x 4096 485 / 485 / 466,
+// forward 256 x 256 16.2 / 14.8 / 15.7, 330 x 384 31.3 / 29.9 / 32.4, 216 x 640 42.3 / 39.7 / 42.4, 105 x 3072 317 / 295 / 267; heads that the XCDs do not share
+// evenly, 10 x 6400 backward 503 / 360 / 365.  All of them by length: 128 x 4096 x 128, forward and backward, 2366 / 2353 (four) / 2420 (16 heads at a time
+// in an XCD's L2).  Launches of one block a CU have nothing to even out and keep their heads together (forward, 27 x 1024 x 128 19.1, all by length 20.7).
+inline AttnArgs deal_blocks(AttnArgs p, int nblk, int elem_bytes) {
   const int64_t heads = (int64_t)p.Z * p.H, blocks = heads * nblk;
   int64_t one_by_one = heads;
-  if (p.causal && blocks > 256) {
-    const int64_t tail = (128 + nblk - 1) / nblk;
+  if (p.causal && blocks > p.cus) {
+    const int64_t tail = ((p.D * elem_bytes >= 256 && p.N < 1024 && p.N != 512 ? 2 : 4) * p.cus / 8 + nblk - 1) / nblk;
     one_by_one = heads / 8 > tail ? (heads / 8 - tail) * 8 : 0;
   }
   p.head_blocks = (int)(one_by_one * nblk);
