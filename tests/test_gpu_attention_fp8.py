@@ -121,3 +121,21 @@ def test_groups_of_waves_along_the_keys_agree_with_one(gpu, fmt, causal, variant
         want = torch.softmax(s, -1) @ torch.from_numpy(v).to(gpu).double()
         err = [((x.double() - want).norm() / want.norm()).item() for x in (one, got)]
         assert err[1] <= 1.05 * err[0], err
+
+
+@pytest.mark.parametrize("D,N,variant", [(64, 8192, 7), (64, 8192, 6), (128, 6144, 6)])
+def test_groups_of_waves_are_no_further_from_64_bits_on_long_causal_rows(gpu, D, N, variant, monkeypatch):
+    # scores three times as wide as unit ones: the running maxima rise long after the first block, P is rounded against others in every group, and the
+    # results differ by about 5 % - but each group's maxima rise less often, so that its P keeps no fewer bits: seen 0.95 .. 0.97 of one group's error, 1.0003 with unit scores
+    g = torch.Generator(device=gpu).manual_seed(N)
+    for wide in (1.0, 3.0):
+        q, k, v = ((torch.randn(1, 1, N, D, device=gpu, generator=g) * s).to(torch.float8_e5m2) for s in (wide, 1.0, 1.0))
+        tv = v.view(torch.uint8).permute(0, 1, 3, 2).contiguous().permute(0, 1, 3, 2).view(torch.float8_e5m2)
+        rows = torch.arange(0, N, 8, device=gpu)
+        s = (q[0, 0, rows].double() @ k[0, 0].double().t()) * D ** -0.5
+        s.masked_fill_(torch.arange(N, device=gpu)[None, :] > rows[:, None], float("-inf"))
+        want, err = torch.softmax(s, -1) @ v[0, 0].double(), []
+        for form in (1, variant):
+            set_knob(monkeypatch, "MI355_ATTN_FWD_VARIANT", str(form))
+            err.append((triton_amd.attention(q, k, tv, True, D ** -0.5)[0, 0, rows].double() - want).norm().item())
+        assert err[1] <= 1.01 * err[0], err

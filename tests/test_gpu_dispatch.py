@@ -105,3 +105,9 @@ def test_groups_of_the_backward_beyond_one_round_of_cus(gpu, H, N, D, groups):
 def test_short_causal_heads_of_128_columns_run_on_blocks_of_128_rows(gpu, H, N, D):
     name, numbers = list(attention_launches(gpu, "fp16", H, N, D, False).items())[0]
     assert name == "attn_fwd_kernel" and numbers == (D, 1, 4, 0, 1)   # (D, tiles and waves, padded, groups)
+
+
+@pytest.mark.parametrize("H,N,groups", [(40, 512, 2), (24, 768, 2), (24, 1024, 2), (16, 1536, 2), (16, 1024, 4), (4, 6144, 4)])
+def test_groups_of_the_fp8_forward_in_short_heads(gpu, H, N, groups):
+    name, numbers = list(attention_launches(gpu, "e5m2", H, N, 64, False).items())[0]
+    assert name == "attn_fwd8_kernel" and numbers[-1] == groups

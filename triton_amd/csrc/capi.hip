@@ -1650,8 +1650,9 @@ static int attn_fwd8_variant(const AttnArgs& p, int cus) {
   const int64_t rows = (int64_t)p.Z * p.H * p.N;
   if (p.D == 64) {
     // mask: 2 x 3840 [30] 37.6 / 22.0 / 31.8 / 15.1, 4 x 6144 [96] 59.6 / 34.7 / 49.1 / 29.2, 8 x 3328 [104] 34.3 / 21.2 / 28.6 / 20.8, 37 x 256 [37] 6.3 / 5.4 /
-    // 6.3 / 5.8; none: 4 x 4096 [64] 41.7 / 24.8 / 34.4 / 22.9, 27 x 1536 [162] 25.9 / 21.1 / 25.1 / 28.1
-    if (p.N % 256 == 0 && p.N >= 512 && rows <= (p.causal ? 96ll : 64ll) * cus) return 7;
+    // 6.3 / 5.8; none: 4 x 4096 [64] 41.7 / 24.8 / 34.4 / 22.9, 27 x 1536 [162] 25.9 / 21.1 / 25.1 / 28.1; short rows, mask: 40 x 512 [80] 7.6 / 5.7 / 7.2 / 8.5, 24 x 768
+    // [72] 9.8 / 6.9 / 8.9 / 8.3, 16 x 1536 [96] 16.7 / 10.6 / 14.6 / 12.0, 16 x 1024 [64] 12.0 / 8.0 / 10.7 / 6.6; none: 24 x 512 [48] 7.2 / 5.5 / 7.0 / 6.1, 16 x 768 [48] 9.5 / 6.7 / 8.8 / 7.1
+    if (p.N % 256 == 0 && p.N >= 512 && rows <= (p.N < 2048 ? p.causal ? 64ll : 32ll : p.causal ? 96ll : 64ll) * cus) return 7;
     // mask: 17 x 2432 [162] 27.7 / 19.9 / 23.9, 83 x 512 [166] 9.3 / 8.5 / 9.3, 71 x 1024 [284] 16.3 / 15.8 / 16.2, 143 x 640 [358] 13.7 / 14.3 / 14.7, 61 x
     // 2048 [488] 38.3 / 37.2 / 35.5; none: 39 x 1152 [176] 20.8 / 17.3 / 19.9, 78 x 256 [78] 6.2 / 6.4 / 6.4, 211 x 384 [316] 13.0 / 13.4 / 14.5
     if (rows <= 64ll * cus || (rows <= (p.causal ? 200ll : 180ll) * cus && p.N >= (p.causal ? 256 : 640)) || (p.causal && rows <= 300ll * cus && p.N >= 1024)) return 6;
