@@ -1805,3 +1805,31 @@ def test_more_tiles_than_cus_of_a_short_k_on_two_workgroups_a_cu(gpu, dtype, M, 
         assert torch.equal(triton_amd.matmul(a, tb, out_dtype=torch.float32), want)
         assert torch.equal(triton_amd.matmul(a, tb, out_dtype=torch.bfloat16), want.bfloat16())
         assert torch.equal(triton_amd.matmul(a, tb, out_dtype=torch.bfloat16, add=row), (want + row.float()).bfloat16())
+
+
+@pytest.mark.parametrize("kmajor", [False, True])
+@pytest.mark.parametrize("M,N,K,knob,value", [
+    (2048, 4098, 4096, "MI355_GEMM_TILE", "6"), (2050, 1026, 512, "MI355_GEMM_TILE", "6"), (4096, 5122, 256, "MI355_GEMM_PROGRAMS", "96"),   # several tiles a program as one stream
+    (768, 1026, 512, "MI355_GEMM_TILE_M", "192"), (770, 514, 384, "MI355_GEMM_TILE_M", "192"), (640, 770, 512, "MI355_GEMM_TILE_M", "128"),
+    (768 + 192, 1024, 512, "MI355_GEMM_MIXED_ROWS", "768"), (256 + 384, 512, 1024, "MI355_GEMM_MIXED_ROWS", "256")])
+def test_rows_on_dwords_of_whole_steps_run_every_four_wave_kernel(gpu, monkeypatch, M, N, K, knob, value, kmajor):
+    # a K of whole pairs of 128-byte steps: the kernels without a head, with pitches 2 mod 8 elements and bases 4 bytes off.  NaN around the rows, whole numbers: exact
+    set_knob(monkeypatch, knob, value)
+    g = torch.Generator(device=gpu).manual_seed(M + N)
+
+    def operand(rows, cols):
+        pitch = cols + 2 + (-cols % 8) + (0 if cols % 8 else 8)
+        room = torch.full((2 + rows * pitch + 8,), float("nan"), device=gpu, dtype=torch.bfloat16)
+        x = room[2:2 + rows * pitch].view(rows, pitch)[:, :cols]
+        return x.copy_(torch.randint(-1, 2, (rows, cols), device=gpu, generator=g))
+
+    a, b = operand(M, K), operand(N, K) if kmajor else operand(K, N)
+    bt = b.t() if kmajor else b
+    assert a.stride(0) % 8 == 2 and b.stride(0) % 8 == 2
+    lib, stream = _lib.load(), torch.cuda.current_stream().cuda_stream
+    for row in (None, torch.randint(-8, 9, (N,), device=gpu, generator=g).to(torch.bfloat16)):
+        want = (a.float() @ bt.float() + (0 if row is None else row.float())).bfloat16()
+        c = torch.full((M, N), float("nan"), device=gpu, dtype=torch.bfloat16)
+        rc = lib.mi355_gemm_epilogue(a.data_ptr(), b.data_ptr(), c.data_ptr(), M, N, K, a.stride(0), 1, *bt.stride(), N, 1, _lib.BF16, _lib.BF16, None, None,
+                                     None if row is None else row.data_ptr(), 0, 1, _lib.BF16, _lib.ACT_NONE, 0, stream)
+        assert rc == 0 and torch.equal(c, want), row is None
