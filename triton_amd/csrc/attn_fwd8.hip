@@ -35,8 +35,8 @@ __device__ __forceinline__ f32x16 mfma_f8(i32x8 a, i32x8 b, f32x16 c) {
 // stored.  Zero columns add nothing to the scores and give zero columns of O: what a HEAD_DIM d_real kernel computes.
 // KW > 1: groups of waves along the keys, as in attn_fwd.hip: every group takes each KW-th block of 64 keys for the same rows, and their
 // maxima, sums and accumulators meet in LDS, for launches of fewer blocks than CUs, which last as long as one block's walk
-// over the keys.  P is rounded to two or three bits of fraction, so that another maximum under it would be another result altogether:
-// every group starts from the maximum of the row's first 64 keys, as a single one does.
+// over the keys.  P is rounded to two or three bits of fraction, and another maximum under it is another rounding:
+// every group starts from the maximum of the row's first 64 keys, as a single one does, and rounds as that one does until a later maximum passes it by 2^4.
 template <int FMT, int D, int NW, bool PAD = false, int KW = 1>
 __global__ __launch_bounds__(NW * 64, NW == 4 && D <= 128 ? 2 : 1) void attn_fwd8_kernel(AttnArgs p) {
   static_assert(!PAD || (D == 64 && KW == 1), "the padded form is the 64-column one");

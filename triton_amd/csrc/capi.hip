@@ -332,8 +332,8 @@ Cut best_cut(int M, int N, int steps, int cus, int tile, int ring, bool is8) {
 // workgroups on a CU where a ring leaves room for one.  Measured over 16 .. 1280 tiles and K bytes of 16 .. 2048, this kernel / ring or
 // 256x256 tiles, us: 2688 x 2688 x 64 fp16 8.2 / 11.5, x 192 11.5 / 13.2, x 256 12.4 / 13.0; e4m3 x 384 10.6 / 12.6, x 512 12.3 / 12.7; row-major B, x 256
 // 12.0 / 13.6; edges cost it more (2659 x 2656 x 64 9.4 / 11.4, x 192 12.2 / 13.0).  Up to half as many tiles, whole ones only (1792 x 1920 x 64 6.0 / 7.1, 1763 x 1888
-// 1.06).  Not where one round of 256x256 tiles fills the CUs (3840 x 4096 x 16 1.1).  With more tiles than CUs the ring of two stages (pairs_us) takes what
-// it takes of them, that kernel / ring: fp16 3840 x 1792 x 256 11.1 / 8.2, row-major B 1642 x 3586 x 128 14.8 / 10.2, 1950 x 4480 x 64 10.0 / 10.3.
+// 1.06).  Not where one round of 256x256 tiles fills the CUs (3840 x 4096 x 16 1.1).  With more tiles than CUs the rings of two stages take them, that kernel /
+// ring: fp16 3840 x 1792 x 256 11.1 / 8.2, row-major B 1642 x 3586 x 128 14.8 / 10.2, but where one_barrier_ahead says otherwise.
 bool short_k(int M, int N, int k_bytes, bool b_kmajor, int cus) {
   const long tiles = (long)((M + 127) / 128) * ((N + 127) / 128), tiles256 = (long)((M + 255) / 256) * ((N + 255) / 256);
   if (tiles256 <= cus && tiles256 * 10 >= cus * 9) return false;
@@ -1643,8 +1643,10 @@ static int attn_fwd_variant(const AttnArgs& p, int cus) {
 }
 
 // The same for fp8: 1 = 128 rows a workgroup (eight waves along 256 rows are 6 to 12 % slower), and as above 8, 6 and 7 = groups along the keys.
-// us, e5m2, 1 / 6 / 8 / 7; rows per CU in brackets.  The groups' sums differ from the one's as their running maxima do (P has two bits of fraction):
-// by up to 2.2 % of the result without a mask at 4096 keys, 1 % with it at 6144, which is why longer rows without a mask stay.
+// us, e5m2, 1 / 6 / 8 / 7; rows per CU in brackets.  The groups' sums differ from the one's as their running maxima do (P has two bits of fraction): with
+// unit scores by up to 2.2 % of the result without a mask at 4096 keys, with it 1 % at 6144 and 1.3 % at 24576, with scores three times as wide 4 to 6 %.  They are as close to
+// 64 bits as the one's or closer, with the mask 0.998 .. 1.0003 of its error at 1024 .. 32768 keys with unit scores and 0.93 .. 0.98 with the wide ones, whose maxima rise less
+// often within a group.  So the mask has no limit of length; longer rows without one stay on one group, which was not measured against 64 bits there.
 static int attn_fwd8_variant(const AttnArgs& p, int cus) {
   if (p.D == 256 || p.d_real < p.D || p.N < 256 || (!p.causal && p.N > 4096)) return 1;
   const int64_t rows = (int64_t)p.Z * p.H * p.N;
